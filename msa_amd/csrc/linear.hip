@@ -7,11 +7,11 @@
 //   k = unit * 32 J + 32 j + 8 g   (one load instruction covers 64 contiguous bytes of each of 16 rows),
 // and the same bytes of x row n (J = 4, or 2 when the RMSNorm is folded in).  The contraction order
 // inside a unit is permuted the same way on both operands, which a dot product does not see.  A workgroup owns R row groups and splits
-// K over its wavefronts; partial sums meet in LDS and are added in wavefront order (deterministic).
+// K over its wavefronts; partial sums meet in LDS and are added in wavefront order (deterministic).  Matrices of more than 3 MB
+// with rows of more than 512 elements take the form of rows_ring.h instead.
 #include <algorithm>
-#include <type_traits>
 
-#include "common.h"
+#include "rows_ring.h"
 
 namespace {
 
@@ -188,183 +188,47 @@ __global__ __launch_bounds__(kMaxWaves * 64) void skinny_linear_kernel(
   }
 }
 
-// Streaming form for matrices with many row groups per compute unit (gate/up, LM head): a workgroup stays for the
-// whole launch.  Wavefront w owns the K slice [32 F w, 32 F (w + 1)) for every row group the workgroup visits and
-// keeps its x operands for that slice (with the RMSNorm weight folded in) in registers, so the activations are read
-// once per workgroup instead of once per row group, and far fewer workgroups have to be dispatched.  Work items are
-// pairs of row groups (32 weight rows), or single row groups for the silu epilogue (8 gate rows and the same 8 up
-// rows: the finer grain matters because a launch lasts as long as its busiest compute unit), dealt round robin;
-// a step is one row group: its F weight vectors per lane are prefetched one step ahead, the partial sums meet in
-// a ring of four LDS buffers behind one barrier per step, and all threads share the work of adding them up (a fixed
-// tree) and storing the row group.  Launched with 16 wavefronts.
-template <int F, int kEpi, bool kNorm>
-__global__ __launch_bounds__(kMaxWaves * 64) void skinny_stream_kernel(
-    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const bf16_t* __restrict__ residual,
-    const bf16_t* __restrict__ norm_w, float eps, bf16_t* __restrict__ y, int32_t M, int32_t N, int32_t K,
-    int64_t y_row_stride, int32_t n_items) {
-  extern __shared__ __align__(16) float part[];   // [4][waves][64][4] partial sums, then [waves][16] sums of squares
-  const int tid = threadIdx.x, lane = tid & 63, waves = blockDim.x >> 6;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n_l = lane & 15, g = lane >> 4;
-  const int row_bytes = K * 2;
-  const int slice_off = wave * (F * 64);           // byte offset of this wavefront's K slice inside a row
-  const int voff = n_l * row_bytes + g * 16;
-  float* row_ssq = part + 4 * waves * 256;
-
-  // activations of the slice, once
-  const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<char*>(reinterpret_cast<const char*>(x)), 0, M * row_bytes, 0x00020000);
-  u32x4_t xf[F];
-#pragma unroll
-  for (int f = 0; f < F; ++f) xf[f] = __builtin_amdgcn_raw_buffer_load_b128(rs_x, voff, slice_off + f * 64, 0);
-
-  // this workgroup's items: blockIdx.x, blockIdx.x + gridDim.x, ...; an item is a pair of row groups (two steps), or
-  // a single row group for the silu epilogue, whose groups are complete in themselves (8 gate rows + 8 up rows)
-  constexpr int kPer = kEpi == kEpiSiluMul ? 1 : 2;
-  const int my_items = n_items > (int)blockIdx.x ? (n_items - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x : 0;
-  const int n_steps = kPer * my_items;
-  auto group_of = [&](int s) {
-    return kPer == 1 ? (int)blockIdx.x + s * (int)gridDim.x : 2 * ((int)blockIdx.x + (s >> 1) * (int)gridDim.x) + (s & 1);
+// What rows_ring.h's kernel does with a product.
+template <int kEpi>
+struct RingEnd {
+  struct Args {
+    const bf16_t* residual;
+    bf16_t* y;
+    int64_t y_row_stride;
   };
-  // Three register stages of weight operands, always indexed by compile-time constants: a step's loads are issued
-  // two steps ahead.  Every step issues its prefetch (an empty one past the end) and the step count is padded to a
-  // multiple of three, so the loop body is straight-line as far as memory instructions go and the wait counts the
-  // compiler derives are exact; with one stage less, the wait for a step's operands also covered the output store
-  // of the step before, i.e. a store round trip per step.
-  constexpr int kStages = 3;
-  u32x4_t fw[kStages][F];
-  auto load_w = [&](auto slot_tag, int s) {
-    constexpr int slot = decltype(slot_tag)::value;
-    const int gid = group_of(s);
-    // rows <= 0 for the missing second group of an odd tail and for the step past the last one (the prefetch is
-    // issued unconditionally so that the wait counts in the loop stay exact): an empty extent reads zeros and
-    // touches no memory.  The clamp compiles to a vector instruction; read-first-lane brings the extent back into a
-    // scalar register so that the descriptor stays scalar and the loads need no per-lane descriptor loop.
-    const int rows = s < n_steps ? min(16, N - gid * 16) : 0;
-    const int extent = __builtin_amdgcn_readfirstlane(max(0, rows) * row_bytes);
-    const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(reinterpret_cast<const char*>(w)) + (int64_t)gid * 16 * row_bytes, 0, extent, 0x00020000);
-#pragma unroll
-    for (int f = 0; f < F; ++f) fw[slot][f] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, voff, slice_off + f * 64, 0);
-  };
-  load_w(std::integral_constant<int, 0>{}, 0);
-  load_w(std::integral_constant<int, 1>{}, 1);
-
-  if constexpr (kNorm) {
-    // RMSNorm folded in: the operand is bf16(x * norm_w); the row scale rsqrt(mean(x^2) + eps) commutes with the
-    // product and is applied to the fp32 sums when a row group is stored
-    const __amdgpu_buffer_rsrc_t rs_g = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(reinterpret_cast<const char*>(norm_w)), 0, row_bytes, 0x00020000);
-    float ssq = 0.f;
-#pragma unroll
-    for (int f = 0; f < F; ++f) {
-      const u32x4_t gf = __builtin_amdgcn_raw_buffer_load_b128(rs_g, g * 16, slice_off + f * 64, 0);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const float lo = bf16lo(xf[f][c]), hi = bf16hi(xf[f][c]);
-        ssq += lo * lo + hi * hi;
-        xf[f][c] = pack_rne(lo * bf16lo(gf[c]), hi * bf16hi(gf[c]));
-      }
-    }
-    ssq += __shfl_xor(ssq, 16);
-    ssq += __shfl_xor(ssq, 32);
-    if (g == 0) row_ssq[wave * 16 + n_l] = ssq;       // visible to everyone behind the first step's barrier
+  bf16_t add;
+  __device__ __forceinline__ void begin(const Args&, int) {}
+  __device__ __forceinline__ void load(const Args& a, int m, int n, bool mine, bool, int) {
+    if (kEpi == kEpiResidual && mine) add = a.residual[(int64_t)m * a.y_row_stride + n];
   }
-
-  // Adding up a step's partial sums is shared by all 1024 threads, so that no wavefront falls behind the others at
-  // the next barrier: eight threads own a pair of neighbouring outputs (row o_m of x, columns o_n, o_n + 1 of the
-  // row group); each adds the partials of two wavefronts and the eight meet by three DPP exchanges (a fixed tree:
-  // results are reproducible).  A wavefront thus holds one output row of the group, and its store covers the row's
-  // 32 contiguous bytes in one instruction (a full memory sector; narrower pieces cost a read-modify-write).
-  const int pair = tid >> 3, sub = tid & 7;
-  const int o_m = pair >> 3, o_n = (pair & 7) * 2;
-  const int o_idx = ((o_m >> 2) * 16 + o_n) * 4 + (o_m & 3);          // float index of (o_m, o_n) in a partial row
-  float inv = 1.f;                                                  // RMSNorm scale of row o_m
-  bool have_inv = !kNorm;
-  auto sum_parts = [&](int s, float& v0, float& v1) {
-    const float* base = part + ((s & 3) * waves + 2 * sub) * 256 + o_idx;
-    v0 = base[0] + base[256];
-    v1 = base[4] + base[256 + 4];
-#pragma unroll
-    for (int x = 1; x < 8; x <<= 1) {
-      v0 += __shfl_xor(v0, x);
-      v1 += __shfl_xor(v1, x);
-    }
-  };
-  const bool pair_store = ((y_row_stride & 1) == 0) && ((reinterpret_cast<uintptr_t>(y) & 3) == 0);
-  auto store_pair = [&](int n, float a, float b) {          // columns n, n + 1 of row o_m
-    bf16_t* at = y + (int64_t)o_m * y_row_stride + n;
-    const int n_end = kEpi == kEpiSiluMul ? N / 2 : N;
-    if (pair_store && n + 1 < n_end) {
-      *reinterpret_cast<uint32_t*>(at) = (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
-    } else {
-      if (n < n_end) at[0] = f32_to_bf16(a);
-      if (n + 1 < n_end) at[1] = f32_to_bf16(b);
-    }
-  };
-
-  auto step = [&](int s, auto slot_tag) {
-    constexpr int slot = decltype(slot_tag)::value;
-    load_w(std::integral_constant<int, (slot + 2) % kStages>{}, s + 2);
-    floatx4_t acc = floatx4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int f = 0; f < F; ++f)
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(xf[f]), as_frag(fw[slot][f]), acc, 0, 0, 0);
-    // acc[e] is y[m = 4 g + e][16 gid + n_l] over this wavefront's K slice
-    *reinterpret_cast<floatx4_t*>(part + ((s & 3) * waves + wave) * 256 + lane * 4) = acc;
-    __syncthreads();
-    if (s >= n_steps) return;                        // padding step
-    if (!have_inv) {
-      float tot = 0.f;
-      for (int wv = 0; wv < waves; ++wv) tot += row_ssq[wv * 16 + o_m];
-      inv = rsqrtf(tot / (float)K + eps);
-      have_inv = true;
-    }
-    const int gid = group_of(s);
+  __device__ __forceinline__ void apply(const Args& a, int m, int n, float v, bool mine, bool, int) const {
     if constexpr (kEpi == kEpiSiluMul) {
-      // columns 0..7 of the group are gate rows, 8..15 the same up rows: the lanes 32 further on hold the up pair
-      float g0, g1;
-      sum_parts(s, g0, g1);
-      const float u0 = __shfl_xor(g0, 32), u1 = __shfl_xor(g1, 32);
-      if (sub != 0 || o_m >= M || o_n >= 8) return;
-      const float a0 = bf16_to_f32(f32_to_bf16(g0 * inv)), b0 = bf16_to_f32(f32_to_bf16(u0 * inv));
-      const float a1 = bf16_to_f32(f32_to_bf16(g1 * inv)), b1 = bf16_to_f32(f32_to_bf16(u1 * inv));
-      store_pair(gid * 8 + o_n, a0 / (1.f + __expf(-a0)) * b0, a1 / (1.f + __expf(-a1)) * b1);
-    } else {
-      float v0, v1;
-      sum_parts(s, v0, v1);
-      const int n = gid * 16 + o_n;
-      if (sub != 0 || o_m >= M) return;
-      v0 *= inv;
-      v1 *= inv;
-      if (kEpi == kEpiResidual) {
-        const bf16_t* r = residual + (int64_t)o_m * y_row_stride + n;
-        if (n < N) v0 = bf16_to_f32(f32_to_bf16(v0)) + bf16_to_f32(r[0]);
-        if (n + 1 < N) v1 = bf16_to_f32(f32_to_bf16(v1)) + bf16_to_f32(r[1]);
-      }
-      store_pair(n, v0, v1);
+      // a 16-row group holds gate rows in its first half and the same up rows in its second, 32 lanes on
+      const float gate = bf16_to_f32(f32_to_bf16(v)), up = bf16_to_f32(f32_to_bf16(__shfl_xor(v, 32)));
+      if (mine && (n & 8) == 0) a.y[(int64_t)m * a.y_row_stride + (n >> 4) * 8 + (n & 7)] = f32_to_bf16(gate / (1.f + __expf(-gate)) * up);
+    } else if (mine) {
+      if (kEpi == kEpiResidual) v = bf16_to_f32(f32_to_bf16(v)) + bf16_to_f32(add);
+      a.y[(int64_t)m * a.y_row_stride + n] = f32_to_bf16(v);
     }
-  };
-  for (int s = 0; s < n_steps; s += kStages) {
-    step(s, std::integral_constant<int, 0>{});
-    step(s + 1, std::integral_constant<int, 1>{});
-    step(s + 2, std::integral_constant<int, 2>{});
   }
-}
+};
 
-template <int F, int kEpi, bool kNorm>
-int launch_stream(const void* x, const void* w, const void* residual, const void* norm_w, float eps, void* y, int32_t M,
-                  int32_t N, int32_t K, int waves, int grid, int n_items, hipStream_t st) {
-  const size_t lds = (size_t)waves * (4 * 256 + 16) * sizeof(float);
-  const int64_t y_stride = kEpi == kEpiSiluMul ? N / 2 : N;
-  static std::atomic<int> lds_limit_raised{0};   // 16 wavefronts need 65 KB, just past the default dynamic LDS limit
-  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(skinny_stream_kernel<F, kEpi, kNorm>),
-                                  kMaxWaves * (4 * 256 + 16) * (int)sizeof(float)));
-  skinny_stream_kernel<F, kEpi, kNorm><<<grid, waves * 64, lds, st>>>(
-      static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), static_cast<const bf16_t*>(residual),
-      static_cast<const bf16_t*>(norm_w), eps, static_cast<bf16_t*>(y), M, N, K, y_stride, n_items);
-  MSA_LAUNCH_CHECK();
-  return MSA_OK;
+template <int kEpi>
+int launch_ring(const void* x, const void* w, const void* residual, const void* norm_w, float eps, void* y, int32_t M, int32_t N,
+                int32_t K, hipStream_t st) {
+  rows_ring::Args r{};
+  r.w = static_cast<const char*>(w);
+  r.x = static_cast<const char*>(x);
+  r.norm_w = static_cast<const char*>(norm_w);
+  r.xs = (int64_t)K * 2;
+  r.M = M;
+  r.N = r.n_b = N;
+  r.row_bytes = K * 2;
+  r.eps = eps;
+  const typename RingEnd<kEpi>::Args s{static_cast<const bf16_t*>(residual), static_cast<bf16_t*>(y), kEpi == kEpiSiluMul ? N / 2 : N};
+  const int granule = kEpi == kEpiSiluMul ? 16 : 1;
+  return norm_w ? rows_ring::launch<RingEnd<kEpi>, true>(r, s, granule, st)
+                : rows_ring::launch<RingEnd<kEpi>, false>(r, s, granule, st);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -454,16 +318,19 @@ __global__ __launch_bounds__(256) void skinny_tile_reduce_kernel(const float* __
 
 // The cut of the tiled form: up to 16 row groups per row block (fewer when the matrix has fewer than 256 groups), as
 // many K slices as keep the launch within one workgroup per compute unit (at most 16); used when it takes at least
-// 8 us less per compute unit than the plain form at ~34 GB/s (the second launch costs ~4 us).
+// 8 us less per compute unit than the plain form at ~34 GB/s (the second launch costs ~4 us), and the rows are many: up to eight
+// rows of activations are cheaper to read again than a second launch (2560 x 9728: 12.1 us in the form of rows_ring.h with one
+// row, 13.1 with eight, 16.4 with sixteen; 14.8 to 15.2 in this one).
+constexpr int kTileMinRows = 8;
 struct TilePlan {
   int n_slices, gpw, row_blocks;
   bool use;
 };
-TilePlan plan_tile(int32_t N, int32_t K) {
+TilePlan plan_tile(int32_t M, int32_t N, int32_t K) {
   TilePlan t{0, 0, 0, false};
   const int groups = (N + 15) / 16;
   const int steps = K / 32;
-  if (K % 32 != 0 || groups > 256) return t;
+  if (K % 32 != 0 || groups > 256 || M <= kTileMinRows) return t;
   t.gpw = std::min(kMaxWaves, (groups + 15) / 16);
   t.row_blocks = (groups + t.gpw - 1) / t.gpw;
   t.n_slices = std::min(std::min(kTileMaxSlices, steps), 256 / std::max(1, t.row_blocks));
@@ -511,22 +378,11 @@ extern "C" int msa_skinny_linear(const void* x, const void* w, const void* resid
   MSA_REQUIRE(norm_w == nullptr || eps > 0.f, "msa_skinny_linear: folded RMSNorm needs eps > 0");
   hipStream_t st = as_stream(stream);
 
-  // Many row groups per compute unit and a K that 16 wavefronts split into 5 MFMA steps each (K = 2560): the
-  // streaming kernel, one workgroup per compute unit at most, an equal number of items (32 rows) each.
-  if (K == 16 * 5 * 32) {
-    const int n_items = epilogue == kEpiSiluMul ? N / 16 : (N + 31) / 32;
-    const int iters = (n_items + 255) / 256;
-    const int grid = (n_items + iters - 1) / iters;
-    if (iters >= 2) {                                // with one item per workgroup the plain kernel does the same work
-#define MSA_STREAM(E_)                                                                                              \
-  (norm_w ? launch_stream<5, E_, true>(x, w, residual, norm_w, eps, y, M, N, K, kMaxWaves, grid, n_items, st)       \
-          : launch_stream<5, E_, false>(x, w, residual, norm_w, eps, y, M, N, K, kMaxWaves, grid, n_items, st))
-      switch (epilogue) {
-        case kEpiPlain: return MSA_STREAM(kEpiPlain);
-        case kEpiResidual: return MSA_STREAM(kEpiResidual);
-        case kEpiSiluMul: return MSA_STREAM(kEpiSiluMul);
-      }
-#undef MSA_STREAM
+  if (K > rows_ring::kMinK && (int64_t)N * K >= rows_ring::kMinWeights && (norm_w == nullptr || K <= rows_ring::kMaxResidentK)) {
+    switch (epilogue) {
+      case kEpiPlain: return launch_ring<kEpiPlain>(x, w, residual, norm_w, eps, y, M, N, K, st);
+      case kEpiResidual: return launch_ring<kEpiResidual>(x, w, residual, norm_w, eps, y, M, N, K, st);
+      case kEpiSiluMul: return launch_ring<kEpiSiluMul>(x, w, residual, norm_w, eps, y, M, N, K, st);
     }
   }
 
@@ -567,7 +423,7 @@ extern "C" int msa_skinny_linear(const void* x, const void* w, const void* resid
 
 extern "C" size_t msa_skinny_linear_workspace_bytes(int32_t M, int32_t N, int32_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const TilePlan t = plan_tile(N, K);
+  const TilePlan t = plan_tile(M, N, K);
   return t.use ? tile_workspace_bytes(t, N) : 0;
 }
 
@@ -579,7 +435,7 @@ extern "C" int msa_skinny_linear_ws(const void* x, const void* w, const void* re
                     (epilogue == kEpiResidual) == (residual != nullptr) && (int64_t)M * K * 2 < ((int64_t)1 << 31) &&
                     (int64_t)32 * K * 2 < ((int64_t)1 << 31) &&
                     (((uintptr_t)x | (uintptr_t)w | (uintptr_t)workspace) & 15) == 0;
-  const TilePlan t = fits ? plan_tile(N, K) : TilePlan{0, 0, 0, false};
+  const TilePlan t = fits ? plan_tile(M, N, K) : TilePlan{0, 0, 0, false};
   if (!fits || !t.use || workspace == nullptr || workspace_bytes < tile_workspace_bytes(t, N))
     return msa_skinny_linear(x, w, residual, norm_w, eps, epilogue, dtype, M, N, K, y, stream);   // it reports bad arguments
   hipStream_t st = as_stream(stream);

@@ -3,25 +3,31 @@
 // gated recurrence.  Like the skinny linear of the attention model a workgroup owns a few 16-row groups of the weights and
 // splits K over its wavefronts (16x16x32 MFMA: the 16 activation rows are exactly one operand); partial sums meet in LDS
 // and are added in wavefront order.  Everything behind the sums is element-wise in this model (dynamic tanh has no row
-// statistics), so a layer's chain of launches is one per weight matrix plus the state-space / attention step.
+// statistics), so a layer's chain of launches is one per weight matrix plus the state-space / attention step.  Large matrices take
+// the form of rows_ring.h with the same ends; this file's kernel is left with small ones, short rows and per-head products.
 #include <algorithm>
-#include <type_traits>
 
+#include "rows_ring.h"
 #include "seq_mfma.h"
 
 namespace {
 
 constexpr int kMaxWaves = 16;
 constexpr int kGruGroup = 16;
+// A workgroup of rows_ring.h takes 48 rows of the recurrence at least, which leaves compute units without work in small matrices
+// (4096 x 1024, 16 rows: 7.5 us against 6.8; 10240 x 2560: 13.8 against 17.5).
+constexpr int64_t kGruRingWeights = 8 << 20;
 
 // Units of 32 J elements of K (J 16-byte vectors per lane): shorter when three row groups share the registers.
 template <int R>
 constexpr int kVectors = R == 3 ? 2 : 4;
 
 // The element-wise end of product (m, n), `col` its column in the output.  What it reads besides the product is fetched by
-// `load`, which the kernels call before they multiply, so that it arrives with the weights instead of behind the sums.
+// `load`, which the kernels call before they multiply, so that it arrives with the weights instead of behind the sums; `begin`
+// fetches what the row alone tells.
 template <int EPI>
 struct Finish {
+  __device__ __forceinline__ void begin(const msa_rows_args&, int) {}
   __device__ __forceinline__ void load(const msa_rows_args& a, int m, int n) {}
   __device__ __forceinline__ void apply(const msa_rows_args& a, int m, int n, int64_t col, float v) const {
     if constexpr (EPI == MSA_ROWS_F32) {
@@ -39,10 +45,12 @@ template <>
 struct Finish<MSA_ROWS_MAMBA> {
   static constexpr int kTaps = 4;            // more taps than this are read when they are needed
   float keep[kTaps - 1], tap[kTaps], bias;
+  int32_t slot;
+  __device__ __forceinline__ void begin(const msa_rows_args& a, int m) { slot = m < a.M ? a.slot[m] : 0; }
   __device__ __forceinline__ void load(const msa_rows_args& a, int m, int n) {
     const int c = n - a.conv_lo;
     if (c < 0 || c >= a.conv_n) return;
-    const float* kp = a.conv_state + (int64_t)a.slot[m] * (a.conv_k - 1) * a.conv_n + c;
+    const float* kp = a.conv_state + (int64_t)slot * (a.conv_k - 1) * a.conv_n + c;
     const float* tp = a.taps + (int64_t)c * a.conv_k;
     bias = a.conv_bias ? a.conv_bias[c] : 0.f;
 #pragma unroll
@@ -54,7 +62,7 @@ struct Finish<MSA_ROWS_MAMBA> {
   __device__ __forceinline__ void apply(const msa_rows_args& a, int m, int n, int64_t col, float v) const {
     const int c = n - a.conv_lo;
     if (c >= 0 && c < a.conv_n) {
-      float* kp = a.conv_state + (int64_t)a.slot[m] * (a.conv_k - 1) * a.conv_n + c;
+      float* kp = a.conv_state + (int64_t)slot * (a.conv_k - 1) * a.conv_n + c;
       float y = bias;
       if (a.conv_k <= kTaps) {
 #pragma unroll
@@ -83,26 +91,30 @@ struct Finish<MSA_ROWS_MAMBA> {
 
 template <>
 struct Finish<MSA_ROWS_RESIDUAL> {
-  float x, gate, w, b, mix, before;
+  float x, bias, w, b, mix, before;
+  bf16_t gate;
+  int32_t slot;
+  __device__ __forceinline__ void begin(const msa_rows_args& a, int m) { slot = a.shift && m < a.M ? a.slot[m] : 0; }
   __device__ __forceinline__ void load(const msa_rows_args& a, int m, int n) {
     x = a.x_in[(int64_t)m * a.N + n];
-    gate = bf16_to_f32(static_cast<const bf16_t*>(a.gate)[m * a.gate_stride + n]) + a.gate_bias[n];
+    gate = static_cast<const bf16_t*>(a.gate)[m * a.gate_stride + n];
+    bias = a.gate_bias[n];
     if (!a.norm.w) return;
     w = a.norm.w[n];
     b = a.norm.b[n];
     if (!a.shift) return;
     mix = a.shift[n];
-    before = a.prev[(int64_t)a.slot[m] * a.N + n];
+    before = a.prev[(int64_t)slot * a.N + n];
   }
   __device__ __forceinline__ void apply(const msa_rows_args& a, int m, int n, int64_t, float v) const {
     const int64_t at = (int64_t)m * a.N + n;
-    const float y = x + sigmoid_f(gate) * v;
+    const float y = x + sigmoid_f(bf16_to_f32(gate) + bias) * v;
     a.x_out[at] = y;
     if (!a.norm.w) return;
     const float h = tanh_f(a.norm.alpha * y) * w + b;
     if (a.h) static_cast<bf16_t*>(a.h)[at] = f32_to_bf16(h);
     if (!a.shift) return;
-    a.prev[(int64_t)a.slot[m] * a.N + n] = h;
+    a.prev[(int64_t)slot * a.N + n] = h;
     static_cast<bf16_t*>(a.h_shift)[at] = f32_to_bf16(h + (before - h) * mix);
   }
 };
@@ -110,6 +122,7 @@ struct Finish<MSA_ROWS_RESIDUAL> {
 // A (gate, up) pair of neighbouring columns, in the lane of the even one.
 template <>
 struct Finish<MSA_ROWS_GLU> {
+  __device__ __forceinline__ void begin(const msa_rows_args&, int) {}
   __device__ __forceinline__ void load(const msa_rows_args& a, int m, int n) {}
   __device__ __forceinline__ void apply(const msa_rows_args& a, int m, int n, float gate, float up) const {
     if (n & 1) return;
@@ -145,7 +158,10 @@ __global__ __launch_bounds__(kMaxWaves * 64) void rows_linear_kernel(msa_rows_ar
   Finish<EPI> fin;                          // of this thread's first output
   {
     const int m = row_of(tid & 255), nr = 16 * (tid >> 8) + col_of(tid & 255);
-    if (tid < R * 256 && m < a.M && nr < rows_w) fin.load(a, m, n_base + nr);
+    if (tid < R * 256 && m < a.M && nr < rows_w) {
+      fin.begin(a, m);
+      fin.load(a, m, n_base + nr);
+    }
   }
 
   floatx4_t acc[R];
@@ -213,123 +229,79 @@ __global__ __launch_bounds__(kMaxWaves * 64) void rows_linear_kernel(msa_rows_ar
       const float v = total(r, i), up = __shfl_xor(v, 4);
       fin.apply(a, m, n, v, up);
     } else {
-      if (o != tid) fin.load(a, m, n);
+      if (o != tid) {
+        fin.begin(a, m);
+        fin.load(a, m, n);
+      }
       fin.apply(a, m, n, (int64_t)grp * a.N + n, total(r, i));
     }
   }
 }
 
-// Streaming form for matrices with many rows per compute unit (input projections, up, the head): a workgroup stays for the
-// whole launch.  Wavefront w owns the K slice [32 F w, 32 F (w + 1)) for every item the workgroup visits and keeps its
-// activations of that slice in registers, so they are read once per workgroup.  An item is up to 16 weight rows (as many as
-// make every workgroup's share equal), its F vectors per lane requested kStages - 1 items ahead; partial sums meet in two LDS
-// buffers behind one barrier per item, four threads add up an output.  A workgroup's items are contiguous, so it changes from
-// the first operand's rows to the second's at most once.
-constexpr int kPartStride = 260;            // floats per wavefront's partial block: the four adders of an output hit distinct banks
-
-template <int EPI, int F>
-__global__ __launch_bounds__(kMaxWaves * 64) void rows_stream_kernel(msa_rows_args a, int32_t rows_per_item, int32_t items_a,
-                                                                     int32_t items, int32_t per_wg) {
-  constexpr int kStages = F <= 5 ? 3 : 2;
-  __shared__ __align__(16) float part[2][kMaxWaves][kPartStride];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n_l = lane & 15, g = lane >> 4;
-  const int row_bytes = a.K * 2, slice = wave * (F * 64);
-  constexpr int kFar = 0x7ff00000;
-  const int i0 = blockIdx.x * per_wg, i1 = min(items, i0 + per_wg);
-  int at[F];                                // this lane's byte offsets in a row, or past every extent
-#pragma unroll
-  for (int f = 0; f < F; ++f) at[f] = slice + f * 64 + g * 16 < row_bytes ? slice + f * 64 + g * 16 : kFar;
-  auto base_of = [&](int item) { return item < items_a ? item * rows_per_item : a.n_b + (item - items_a) * rows_per_item; };
-  auto rows_of = [&](int item) {
-    if (item >= i1) return 0;
-    return min(rows_per_item, (item < items_a ? min(a.n_b, a.N) : a.N) - base_of(item));
-  };
-  u32x4_t xf[F];
-  auto load_x = [&](bool second) {
-    const int64_t xs = second ? a.x_b_stride : a.x_stride;
-    const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(static_cast<const char*>(second ? a.x_b : a.x)), 0, (int)((a.M - 1) * xs * 2 + row_bytes), 0x00020000);
-#pragma unroll
-    for (int f = 0; f < F; ++f) xf[f] = __builtin_amdgcn_raw_buffer_load_b128(rs_x, at[f] == kFar ? kFar : n_l * (int)(xs * 2) + at[f], 0, 0);
-  };
-  u32x4_t fw[kStages][F];
-  auto load_w = [&](auto slot_tag, int item) {
-    constexpr int slot = decltype(slot_tag)::value;
-    // an empty extent (behind the last item) reads zeros and touches no memory
-    const int extent = __builtin_amdgcn_readfirstlane(max(0, rows_of(item)) * row_bytes);
-    const int base = __builtin_amdgcn_readfirstlane(item < i1 ? base_of(item) : 0);
-    const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(static_cast<const char*>(a.w)) + (int64_t)base * row_bytes, 0, extent, 0x00020000);
-#pragma unroll
-    for (int f = 0; f < F; ++f)
-      fw[slot][f] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, at[f] == kFar ? kFar : n_l * row_bytes + at[f], 0, 0);
-  };
-  bool second = i0 >= items_a;
-  load_x(second);
-  load_w(std::integral_constant<int, 0>{}, i0);
-  if constexpr (kStages == 3) load_w(std::integral_constant<int, 1>{}, i0 + 1);
-  const int o = tid >> 2, quarter = tid & 3;
-  const int m = 4 * (o >> 6) + (o & 3), nr = (o >> 2) & 15;
-  auto step = [&](int item, auto slot_tag) {
-    constexpr int slot = decltype(slot_tag)::value;
-    load_w(std::integral_constant<int, (slot + kStages - 1) % kStages>{}, item + kStages - 1);
-    if (!second && item >= items_a && item < i1) {
-      second = true;
-      load_x(true);
-    }
-    const bool mine = quarter == 0 && m < a.M && nr < rows_of(item);
-    const int n = base_of(item) + nr;
-    Finish<EPI> fin;
+// What rows_ring.h's kernel does with a product: the same ends, and the minimal gated recurrence, whose three sums of a channel
+// are three consecutive items of a workgroup.
+template <int EPI>
+struct RingEnd {
+  using Args = msa_rows_args;
+  Finish<EPI> fin;
+  __device__ __forceinline__ void begin(const Args& a, int m) { fin.begin(a, m); }
+  __device__ __forceinline__ void load(const Args& a, int m, int n, bool mine, bool, int) {
     if (mine) fin.load(a, m, n);
-    floatx4_t acc = floatx4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int f = 0; f < F; ++f)
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xf[f]), __builtin_bit_cast(bf16x8_t, fw[slot][f]), acc, 0, 0, 0);
-    float(*buf)[kPartStride] = part[item & 1];
-    *reinterpret_cast<floatx4_t*>(&buf[wave][lane * 4]) = acc;
-    __syncthreads();
-    float v = (buf[4 * quarter][o] + buf[4 * quarter + 1][o]) + (buf[4 * quarter + 2][o] + buf[4 * quarter + 3][o]);
-    v += __shfl_xor(v, 1);
-    v += __shfl_xor(v, 2);
+  }
+  __device__ __forceinline__ void apply(const Args& a, int m, int n, float v, bool mine, bool, int) const {
     if constexpr (EPI == MSA_ROWS_GLU) {
-      const float up = __shfl_xor(v, 16);
+      const float up = __shfl_xor(v, 4);
       if (mine) fin.apply(a, m, n, v, up);
     } else if (mine) {
       fin.apply(a, m, n, n, v);
     }
-  };
-  for (int item = i0; item < i1; item += kStages) {       // whole rounds: items behind the last read zeros and store nothing
-    step(item, std::integral_constant<int, 0>{});
-    step(item + 1, std::integral_constant<int, 1>{});
-    if constexpr (kStages == 3) step(item + 2, std::integral_constant<int, 2>{});
   }
-}
+};
 
-template <int EPI, int F>
-int launch_stream(const msa_rows_args& a, hipStream_t st) {
-  const int cus = device_compute_units();
-  const int n_a = std::min(a.n_b, a.N), n_b = a.N - n_a;
-  const int iters = (a.N + 16 * cus - 1) / (16 * cus);
-  int rpi = std::min(16, std::max(1, (a.N + iters * cus - 1) / (iters * cus)));
-  if (EPI == MSA_ROWS_GLU) rpi = (rpi + 1) & ~1;                      // pairs stay together
-  auto split = [&] { return (n_a + rpi - 1) / rpi + (n_b + rpi - 1) / rpi; };   // the second operand's rows start an item of their own
-  while (rpi < 16 && split() > iters * cus) ++rpi;
-  const int items_a = (n_a + rpi - 1) / rpi, items = split();
-  const int per_wg = (items + cus - 1) / cus;
-  rows_stream_kernel<EPI, F><<<(items + per_wg - 1) / per_wg, kMaxWaves * 64, 0, st>>>(a, rpi, items_a, items, per_wg);
-  MSA_LAUNCH_CHECK();
-  return MSA_OK;
-}
+template <>
+struct RingEnd<MSA_ROWS_GRU> {
+  using Args = msa_rows_args;
+  float before = 0.f, zb = 0.f, ub = 0.f, z = 0.f, u = 0.f;
+  int32_t slot;
+  __device__ __forceinline__ void begin(const Args& a, int m) { slot = m < a.M ? a.slot[m] : 0; }
+  __device__ __forceinline__ static int channel(int n) { return n / (3 * kGruGroup) * kGruGroup + n % kGruGroup; }
+  __device__ __forceinline__ void load(const Args& a, int m, int n, bool mine, bool second, int item) {
+    const int c = channel(n);
+    if (second || !mine || item % 3 != 0 || c >= a.gru_n) return;
+    before = a.gru_state[(int64_t)slot * a.gru_n + c];
+    zb = a.z_bias[c];
+    ub = a.u_bias[c];
+  }
+  __device__ __forceinline__ void apply(const Args& a, int m, int n, float v, bool mine, bool second, int item) {
+    if (!mine) return;
+    if (second) {
+      static_cast<bf16_t*>(a.out)[m * a.out_stride + n] = f32_to_bf16(v);
+      return;
+    }
+    const int c = channel(n), part = item % 3;
+    if (c >= a.gru_n) return;
+    z = part == 0 ? sigmoid_f(v + zb) : z;
+    u = part == 1 ? v + ub : u;
+    if (part < 2) return;
+    const float S = (1.0f - z) * before + z * (u >= 0.f ? u + 0.5f : sigmoid_f(u));
+    a.gru_state[(int64_t)slot * a.gru_n + c] = S;
+    static_cast<bf16_t*>(a.out2)[(int64_t)m * a.gru_n + c] = f32_to_bf16(S * silu_f(v));
+  }
+};
+
 template <int EPI>
-int launch_stream(const msa_rows_args& a, hipStream_t st) {
-  const int f = (a.K + 511) / 512;
-  if (f <= 2) return launch_stream<EPI, 2>(a, st);
-  if (f <= 3) return launch_stream<EPI, 3>(a, st);
-  if (f <= 4) return launch_stream<EPI, 4>(a, st);
-  if constexpr (EPI == MSA_ROWS_MAMBA) return launch_stream<EPI, 5>(a, st);    // (its operands would not fit beside eight vectors)
-  else return f <= 5 ? launch_stream<EPI, 5>(a, st) : launch_stream<EPI, 8>(a, st);
+int launch_ring(const msa_rows_args& a, hipStream_t st) {
+  rows_ring::Args r{};
+  r.w = static_cast<const char*>(a.w);
+  r.x = static_cast<const char*>(a.x);
+  r.x_b = static_cast<const char*>(a.x_b);
+  r.xs = a.x_stride * 2;
+  r.xbs = a.x_b_stride * 2;
+  r.M = a.M;
+  r.N = a.N;
+  r.n_b = a.n_b;
+  r.row_bytes = a.K * 2;
+  return rows_ring::launch<RingEnd<EPI>>(r, a, EPI == MSA_ROWS_GRU ? 3 * kGruGroup : EPI == MSA_ROWS_GLU ? 2 : 1, st);
 }
 
 template <int EPI, int R>
@@ -396,12 +368,15 @@ extern "C" int msa_rows_linear(const msa_rows_args* args, int32_t epilogue, void
   for (int cand = waves; cand >= std::max(1, waves / 2); --cand)
     if (units % cand == 0) { waves = cand; break; }
   hipStream_t st = as_stream(stream);
-  // Many rows per compute unit: the streaming form.
-  if (a.groups == 1 && a.K > 512 && a.K <= 4096 && a.N >= 2 * 16 * device_compute_units()) {
-    if (epilogue == MSA_ROWS_PLAIN) return launch_stream<MSA_ROWS_PLAIN>(a, st);
-    if (epilogue == MSA_ROWS_F32) return launch_stream<MSA_ROWS_F32>(a, st);
-    if (epilogue == MSA_ROWS_GLU) return launch_stream<MSA_ROWS_GLU>(a, st);
-    if (epilogue == MSA_ROWS_MAMBA && a.K <= 2560) return launch_stream<MSA_ROWS_MAMBA>(a, st);
+  if (a.groups == 1 && a.K > rows_ring::kMinK && !(gru && (int64_t)a.N * a.K < kGruRingWeights) && (int64_t)a.N * a.K >= rows_ring::kMinWeights) {
+    switch (epilogue) {
+      case MSA_ROWS_PLAIN: return launch_ring<MSA_ROWS_PLAIN>(a, st);
+      case MSA_ROWS_F32: return launch_ring<MSA_ROWS_F32>(a, st);
+      case MSA_ROWS_RESIDUAL: return launch_ring<MSA_ROWS_RESIDUAL>(a, st);
+      case MSA_ROWS_MAMBA: return launch_ring<MSA_ROWS_MAMBA>(a, st);
+      case MSA_ROWS_GLU: return launch_ring<MSA_ROWS_GLU>(a, st);
+      case MSA_ROWS_GRU: return launch_ring<MSA_ROWS_GRU>(a, st);
+    }
   }
   switch (epilogue * 4 + R) {
     case MSA_ROWS_PLAIN * 4 + 1: return launch_rows<MSA_ROWS_PLAIN, 1>(a, waves, rows_per_wg, st);
