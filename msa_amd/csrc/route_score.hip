@@ -1109,6 +1109,103 @@ __global__ void decode_scores_kernel(const uint32_t* __restrict__ key, int64_t n
   }
 }
 
+// ------------------------------------------------------------------------------------------
+// fp32 banks of few chunks, or few query rows.  Tiles of 128 x 128 give a bank of 8000 chunks to 63 workgroups, each of which
+// multiplies 1024-deep products at a compute unit's fp32 rate alone (57 us a tile, also where half of its rows are padding).  Here
+// a workgroup owns 32 chunks and its four wavefronts a quarter of K each: a wavefront's share of the K_r rows stays in 128 of its
+// registers for the whole launch, the query rows come from L2 a 32-row block at a time, eight 16-byte vectors ahead of the MFMAs,
+// and the four partial blocks meet in LDS behind one barrier per block, where the rows' maximum is taken.  Both operands permute K
+// alike (lane half h holds the second 16 bytes of every 32).  Column maxima of a query wait in LDS and are merged into the key
+// plane at the end.  What bounds it: the matrix cores' fp32 rate (256 FLOP a cycle and compute unit) and, with few rows, the
+// first loads.
+// A whole routing call, us, against the tiles: 8192 chunks x 64 rows 38 against 82, x 256 rows 66 against 85; 1024 x 128 rows 37
+// against 81.
+// ------------------------------------------------------------------------------------------
+constexpr int kSplitK = 1024, kSplitWaves = 4, kSplitCols = 32, kSplitMaxBlocks = 32;
+
+template <bool kDocMax>
+__global__ __launch_bounds__(kSplitWaves * 64, 2) void score_split_kernel(const float* __restrict__ qs, const float* __restrict__ kr,
+                                                                        const uint32_t* __restrict__ row_bits,
+                                                                        uint32_t* __restrict__ out_key,
+                                                                        const int32_t* __restrict__ chunk_doc, int32_t M_rows,
+                                                                        int32_t C, int32_t blocks_per_query, int32_t n_docs,
+                                                                        int32_t blocks_per_wg) {
+  constexpr int kRow = kSplitK * (int)sizeof(float), kSlice = kRow / kSplitWaves, kSteps = kSlice / 32, kGroup = 8, kGroups = kSteps / kGroup;
+  static_assert(kGroups == 4, "a block starts in the first register buffer");
+  __shared__ float part[2][kSplitWaves][32 * kSplitCols];
+  __shared__ uint32_t best[kSplitMaxBlocks][kSplitCols];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, half = lane >> 5;
+  const int n0 = blockIdx.x * kSplitCols, blocks = M_rows >> 5;
+  const int b0 = blockIdx.y * blocks_per_wg, b1 = min(blocks, b0 + blocks_per_wg);
+  const __amdgpu_buffer_rsrc_t rs_k = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char*>(reinterpret_cast<const char*>(kr)) + (int64_t)n0 * kRow, 0, min(kSplitCols, C - n0) * kRow, 0x00020000);
+  const int off = l32 * kRow + wave * kSlice + half * 16;
+  u32x4_t k[kSteps], q[2][kGroup];
+  auto load_q = [&](auto buf_tag, int blk, int group) {
+    constexpr int buf = decltype(buf_tag)::value;
+    // a block past the range reads zeros through an empty extent
+    const int base = __builtin_amdgcn_readfirstlane(blk < b1 ? blk : b0), extent = __builtin_amdgcn_readfirstlane(blk < b1 ? 32 * kRow : 0);
+    const __amdgpu_buffer_rsrc_t rs_q = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(reinterpret_cast<const char*>(qs)) + (int64_t)base * 32 * kRow, 0, extent, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < kGroup; ++i) q[buf][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_q, off, (group * kGroup + i) * 32, 0);
+  };
+  load_q(std::integral_constant<int, 0>{}, b0, 0);
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i) k[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_k, off, i * 32, 0);
+  const int q0 = b0 / blocks_per_query;
+  for (int i = tid; i < kSplitMaxBlocks * kSplitCols; i += kSplitWaves * 64) best[i / kSplitCols][i % kSplitCols] = 0u;
+  int query = q0, in_query = b0 - q0 * blocks_per_query;
+  for (int blk = b0; blk < b1; ++blk) {
+    const uint32_t bits = row_bits[blk];                 // all rows of a block are scored, or none (presum_queries_kernel)
+    floatx16_t acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+    auto group = [&](auto g_tag) {
+      constexpr int g = decltype(g_tag)::value;
+      if constexpr (g + 1 < kGroups) load_q(std::integral_constant<int, (g + 1) & 1>{}, blk, g + 1);
+      else load_q(std::integral_constant<int, 0>{}, blk + 1, 0);
+#pragma unroll
+      for (int i = 0; i < kGroup; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          acc = Mma<float>::mma(__uint_as_float(q[g & 1][i][c]), __uint_as_float(k[g * kGroup + i][c]), acc);
+    };
+    group(std::integral_constant<int, 0>{});
+    group(std::integral_constant<int, 1>{});
+    group(std::integral_constant<int, 2>{});
+    group(std::integral_constant<int, 3>{});
+    // acc[e] is (row 8 * (e / 4) + 4 * half + e % 4, column l32) over this wavefront's quarter of K
+    float(*p)[32 * kSplitCols] = part[blk & 1];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) p[wave][(8 * (e >> 2) + 4 * half + (e & 3)) * kSplitCols + l32] = acc[e];
+    __syncthreads();
+    float top = -INFINITY;                               // of four rows; the other half of the wavefront has four more
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = ((tid >> 5) * 4 + r) * kSplitCols + l32;
+      top = fmaxf(top, (p[0][i] + p[1][i]) + (p[2][i] + p[3][i]));
+    }
+    top = fmaxf(top, __shfl_xor(top, 32));
+    if (bits != 0 && half == 0) atomicMax(&best[query - q0][l32], f32_to_key(top));
+    if (++in_query == blocks_per_query) {
+      in_query = 0;
+      ++query;
+    }
+  }
+  __syncthreads();
+  const int queries = b1 > b0 ? (b1 - 1) / blocks_per_query - q0 + 1 : 0;
+  for (int i = tid; i < queries * kSplitCols; i += kSplitWaves * 64) {
+    const int n = n0 + i % kSplitCols;
+    const uint32_t key = best[i / kSplitCols][i % kSplitCols];
+    if (n >= C || key == 0) continue;
+    const int64_t row = q0 + i / kSplitCols;
+    if constexpr (kDocMax) atomicMax(&out_key[row * n_docs + chunk_doc[n]], key);
+    else atomicMax(&out_key[row * C + n], key);
+  }
+}
+
 // Optional timing of the scoring kernel alone: event pairs recorded around its launch.  The lock makes the record
 // list safe against concurrent callers; while timing is off a launch only reads one atomic flag.
 struct KernelTimer {
@@ -1166,6 +1263,27 @@ int launch_gemm(const void* qs, const void* kr, const uint32_t* row_bits, uint32
   kern<<<grid, WAVES_M * WAVES_N * 64, lds, st>>>(static_cast<const T*>(qs), static_cast<const T*>(kr), row_bits, out_key,
                                                   chunk_doc, M_rows, C, K, blocks_per_query, tiles_m, tiles_n, m_group,
                                                   n_docs);
+  MSA_LAUNCH_CHECK();
+  if (slot >= 0) MSA_HIP(hipEventRecord(g_timer.stop[slot], st));
+  return MSA_OK;
+}
+
+// As many workgroups along the query blocks as give every compute unit two, at most kSplitMaxBlocks blocks each.
+template <bool kDocMax>
+int launch_split(const void* qs, const void* kr, const uint32_t* row_bits, uint32_t* out_key, const int32_t* chunk_doc,
+                 int32_t M_rows, int32_t C, int32_t blocks_per_query, int32_t n_docs, hipStream_t st) {
+  const int cols = (C + kSplitCols - 1) / kSplitCols, blocks = M_rows / 32;
+  const int want = std::min(blocks, std::max((blocks + kSplitMaxBlocks - 1) / kSplitMaxBlocks, 2 * compute_units() / cols));
+  const int per_wg = (blocks + want - 1) / want;
+  const dim3 grid((unsigned)cols, (unsigned)((blocks + per_wg - 1) / per_wg));
+  int slot = -1;
+  if (g_timer.on.load(std::memory_order_acquire)) {
+    std::lock_guard<std::mutex> lock(g_timer.mu);
+    if (g_timer.n < g_timer.cap) slot = g_timer.n++;
+  }
+  if (slot >= 0) MSA_HIP(hipEventRecord(g_timer.start[slot], st));
+  score_split_kernel<kDocMax><<<grid, kSplitWaves * 64, 0, st>>>(static_cast<const float*>(qs), static_cast<const float*>(kr), row_bits,
+                                                                 out_key, chunk_doc, M_rows, C, blocks_per_query, n_docs, per_wg);
   MSA_LAUNCH_CHECK();
   if (slot >= 0) MSA_HIP(hipEventRecord(g_timer.stop[slot], st));
   return MSA_OK;
@@ -1237,6 +1355,11 @@ template <bool kDocMax>
 int launch_gemm_for(int32_t dtype, const void* qs, const void* kr, const uint32_t* row_bits, uint32_t* out_key,
                     const int32_t* chunk_doc, int32_t M_rows, int32_t C, int32_t K, int32_t bpq, int32_t n_docs,
                     hipStream_t st, const GatherJob* job, bool* job_taken, uint32_t* sched) {
+  // The line between the fp32 forms: above it the tiles' reuse of both operands is worth more than the even split (16384 chunks x
+  // 128 rows: 61 us in the split form, 84 in tiles; x 256 rows 95 and 88; 65536 x 128: 190 and 151), except that the tiles pad up
+  // to 64 rows to 128 (65536 x 64: 123 and 142).
+  if (dtype != MSA_BF16 && K == kSplitK && (M_rows <= 64 || (int64_t)C * M_rows <= (int64_t)1 << 21))
+    return launch_split<kDocMax>(qs, kr, row_bits, out_key, chunk_doc, M_rows, C, bpq, n_docs, st);
   if (dtype != MSA_BF16)
     return launch_gemm<float, 128, 128, 2, 2, 1, kDocMax, false>(qs, kr, row_bits, out_key, chunk_doc, M_rows, C, K, bpq, n_docs, st);
   if (M_rows <= 64)

@@ -1,0 +1,87 @@
+"""Routing over small banks: the fp32 form that splits K over a workgroup's wavefronts at its edges (chunks that are no multiple of 32,
+row blocks shared out over workgroups, queries without a scored token, per-chunk scores) against float64, single candidate lists,
+and the gather's plan with documents that many samples share."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import closed_form as cf
+
+pytestmark = pytest.mark.gpu
+
+
+def make(doc_chunks, B, S, seed, host=False):
+    from msa_amd import ops
+    g = torch.Generator().manual_seed(seed)
+    off = np.concatenate([[0], np.cumsum(doc_chunks)])
+    C = int(off[-1])
+    kr = torch.nn.functional.normalize(torch.randn((C, 8, 128), generator=g), dim=-1)
+    q = torch.randn((B, S, 32, 128), generator=g)
+    bank = ops.Bank(1, off.tolist(), [7 * i + 1 for i in range(len(doc_chunks))], 8, 128, torch.float32)
+    kv = [torch.randn((C, 8, 128), generator=g).pin_memory() for _ in range(2)] if host else [None, None]
+    bank.set_layer(0, kr.cuda(), *kv)
+    return bank, kr, q, off, kv
+
+
+# (largest document, documents, queries, tokens): 1 chunk; 31 to 33 and their neighbours; more row blocks than a workgroup keeps (1 x
+# 1200 tokens: 38 blocks); blocks of many queries; the line to the tiles (chunks x rows = 2^21) from both sides
+@pytest.mark.parametrize("top,docs,B,S", [(1, 1, 1, 1), (1, 31, 2, 33), (1, 32, 1, 64), (1, 33, 3, 70), (9, 40, 1, 1200), (5, 300, 40, 5), (17, 800, 2, 130),
+                                          (16, 2100, 1, 65), (16, 2100, 1, 128), (16, 2040, 1, 128)])
+def test_split_scores(top, docs, B, S):
+    from msa_amd import ops
+    rng = np.random.default_rng(docs)
+    doc_chunks = rng.integers(1, top + 1, size=docs).tolist()
+    bank, kr, q, off, _ = make(doc_chunks, B, S, docs + S)
+    mask = torch.ones((B, S), dtype=torch.bool)
+    if B > 1:
+        mask[1, : (S + 1) // 2] = False
+        mask[B - 1, :] = False                           # no scored token at all
+        mask[B - 1, S - 1] = B == 2
+    want = cf.chunk_scores(q, mask, kr)
+    got = ops.chunk_scores(bank, 0, q.cuda(), mask.cuda()).cpu().double()
+    seen = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(got), seen)
+    # 1024 products of unit vectors in fp32: 1e-5 of the largest score
+    assert (got - want)[seen].abs().max() <= 1e-5 * want[seen].abs().max()
+    per_doc = torch.stack([want[:, off[d]:off[d + 1]].amax(1) for d in range(docs)], 1)
+    k = min(16, docs)
+    scores, doc, gid = (t.cpu() for t in ops.route_topk(bank, 0, q.cuda(), mask.cuda(), topk=k))
+    for b in range(B):
+        if not mask[b].any():
+            assert torch.isinf(scores[b]).all()
+            continue
+        assert (scores[b].double() - per_doc[b].topk(k).values).abs().max() <= 1e-5 * per_doc[b].abs().max()
+        assert (per_doc[b][doc[b].long()] - scores[b].double()).abs().max() <= 1e-5 * per_doc[b].abs().max()
+        assert torch.equal(gid[b], 7 * doc[b].long() + 1) and len(set(doc[b].tolist())) == k
+
+
+@pytest.mark.parametrize("B,k", [(1, 1), (3, 16), (33, 17), (20, 33), (32, 64), (70, 64)])
+def test_gather_plan_of_shared_documents(B, k):
+    """Few documents for many picks: nearly all are shared, some repeat within a sample, some are out of range."""
+    from msa_amd import ops
+    rng = np.random.default_rng(B * k)
+    doc_chunks = rng.integers(1, 6, size=80).tolist()
+    bank, _, _, off, kv = make(doc_chunks, 1, 1, B, host=True)
+    sel = torch.from_numpy(rng.integers(-2, 83, size=(B, k)).astype(np.int32))
+    keep = [sorted({d for d in row if 0 <= d < 80}) for row in sel.tolist()]
+    want = [torch.cat([t[off[d]:off[d + 1]] for row in keep for d in row] + [t[:0]]) for t in kv]
+    n = want[0].shape[0]
+    k_out, v_out, cu = ops.gather_kv_device(bank, 0, sel.cuda(), max(1, n))
+    assert cu.tolist() == np.concatenate([[0], np.cumsum([sum(doc_chunks[d] for d in row) for row in keep])]).tolist()
+    assert torch.equal(k_out[:n].cpu(), want[0]) and torch.equal(v_out[:n].cpu(), want[1])
+
+
+@pytest.mark.parametrize("dtype,L", [(torch.float32, 1), (torch.float32, 200), (torch.bfloat16, 255)])
+def test_single_pass_decode_attention(dtype, L):
+    """Contexts that are not split: the output comes from the first launch; a sample without keys yields zeros."""
+    from msa_amd import ops
+    g = torch.Generator().manual_seed(L)
+    q, k, v = (torch.randn(s, generator=g).to(dtype) for s in ((3, 32, 128), (3 * L, 8, 128), (3 * L, 8, 128)))
+    lens = torch.tensor([L, 0, max(1, L // 2)], dtype=torch.int32)
+    out = ops.sparse_attn(q.cuda(), k.cuda(), v.cuda(), (torch.arange(3) * L).cuda(), lens.cuda(), L).cpu().double()
+    assert (out[1] == 0).all()
+    for b in (0, 2):
+        kk, vv = (t[b * L:b * L + int(lens[b])].double().repeat_interleave(4, dim=1) for t in (k, v))
+        p = torch.softmax((q[b].double()[None] * kk).sum(-1) * 128 ** -0.5, dim=0)
+        want = (p[..., None] * vv).sum(0)
+        assert (out[b] - want).abs().max() <= (1e-5 if dtype == torch.float32 else 1e-2) * want.abs().max()
