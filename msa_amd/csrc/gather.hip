@@ -121,7 +121,7 @@ extern "C" int msa_gather_kv(const msa_bank* bank, int32_t layer, const int32_t*
 // ------------------------------------------------------------------------------------------
 namespace {
 
-constexpr int kPlanWaves = 4;
+constexpr int kPlanWaves = 16;
 using msa_gather::kPlanInts;
 using msa_gather::kDedupMaxEntries;
 using msa_gather::kCopyRowLanes;
