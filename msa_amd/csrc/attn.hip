@@ -195,7 +195,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
     const T* __restrict__ q, const int32_t* __restrict__ cu_q, const T* __restrict__ k, const T* __restrict__ v,
     const int64_t* __restrict__ kv_off, const int32_t* __restrict__ kv_len, int32_t B, int32_t Hq, int32_t Hkv,
     float scale_log2e, int32_t causal, int32_t n_split, int32_t split_keys, float* __restrict__ part_ml,
-    float* __restrict__ part_acc) {
+    float* __restrict__ part_acc, T* __restrict__ out) {
   __shared__ float sm_m[kAttnWaves][G], sm_l[kAttnWaves][G];
   __shared__ float sm_acc[kAttnWaves][G][kHeadDim];
 
@@ -283,6 +283,12 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
       at += sm_acc[w][h][d] * a;
     }
     const int64_t o = ((int64_t)row * Hq + g * G + h) * n_split + split;
+    if (n_split == 1) {                                  // nothing to merge: the output itself (a launch of 4 us less)
+      const float y = lt > 0.f ? at / lt : 0.f;          // a row that sees no key yields zeros
+      if constexpr (sizeof(T) == 2) out[o * kHeadDim + d] = f32_to_bf16(y);
+      else out[o * kHeadDim + d] = y;
+      continue;
+    }
     part_acc[o * kHeadDim + d] = at;
     if (d == 0) { part_ml[o * 2] = mn; part_ml[o * 2 + 1] = lt; }
   }
@@ -493,7 +499,7 @@ int launch_attn(const void* q, const int32_t* cu_q, const void* k, const void* v
   case GG:                                                                                                         \
     attn_partial_kernel<T, GG, WW><<<grid, WW * 64, 0, st>>>(                                                      \
         static_cast<const T*>(q), cu_q, static_cast<const T*>(k), static_cast<const T*>(v), kv_off, kv_len, B, Hq, \
-        Hkv, sl2, causal, n_split, 0, part_ml, part_acc);                                                          \
+        Hkv, sl2, causal, n_split, 0, part_ml, part_acc, static_cast<T*>(out));                                                          \
     break;
   switch (G) {
     MSA_ATTN_CASE(1, 4)
@@ -506,6 +512,7 @@ int launch_attn(const void* q, const int32_t* cu_q, const void* k, const void* v
   }
 #undef MSA_ATTN_CASE
   MSA_LAUNCH_CHECK();
+  if (n_split == 1) return MSA_OK;
   attn_combine_kernel<T><<<(unsigned)((int64_t)total_q * Hq), kHeadDim, 0, st>>>(part_ml, part_acc, n_split,
                                                                                  static_cast<T*>(out));
   MSA_LAUNCH_CHECK();

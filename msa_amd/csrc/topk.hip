@@ -71,8 +71,35 @@ __device__ __forceinline__ uint64_t wave_merge_desc(uint64_t best, uint64_t batc
 // sorted and merged 64 at a time, so the bitonic network runs a few times per wavefront, not once per batch.
 constexpr int kLoadsPerLane = 4;
 
+// Where a query's result goes, and what turns a key into a score and a document into its global id.
+struct TopkOut {
+  const int64_t* doc_global_id;
+  float mul;
+  float* scores;
+  int32_t* doc;
+  int64_t* doc_global;           // optional
+};
+// The first topk lanes of a sorted list, written as query b's result.
+__device__ __forceinline__ void write_topk(const TopkOut& out, int b, int32_t topk, int lane, uint64_t best) {
+  if (lane >= topk) return;
+  const int64_t o = (int64_t)b * topk + lane;
+  if (best == 0) {
+    out.scores[o] = -INFINITY;
+    out.doc[o] = -1;
+    if (out.doc_global) out.doc_global[o] = -1;
+  } else {
+    const uint32_t k = (uint32_t)(best >> 32);
+    const int32_t d = (int32_t)(0xffffffffu - (uint32_t)best);
+    out.scores[o] = k == 0 ? -INFINITY : key_to_f32(k) * out.mul;
+    out.doc[o] = d;
+    if (out.doc_global) out.doc_global[o] = out.doc_global_id[d];
+  }
+}
+
+// A bank of one workgroup's documents has one list per query: its result is written here (a launch of 4 us less), otherwise the
+// lists go to merge_topk_kernel.
 __global__ __launch_bounds__(kWaves * 64) void doc_topk_kernel(const uint32_t* __restrict__ doc_key, int32_t n_docs,
-                                                               int32_t topk, uint64_t* __restrict__ cand) {
+                                                               int32_t topk, uint64_t* __restrict__ cand, TopkOut out) {
   __shared__ uint64_t pend[kWaves][128];
   __shared__ uint64_t lists[kWaves][64];
   const int b = blockIdx.y;
@@ -124,17 +151,15 @@ __global__ __launch_bounds__(kWaves * 64) void doc_topk_kernel(const uint32_t* _
   if (wave == 0) {
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) best = wave_merge_desc(best, lists[w][lane], lane);
-    cand[((int64_t)b * gridDim.x + blockIdx.x) * kTopkMax + lane] = best;
+    if (gridDim.x == 1) write_topk(out, b, topk, lane, best);
+    else cand[((int64_t)b * gridDim.x + blockIdx.x) * kTopkMax + lane] = best;
   }
 }
 
 constexpr int kMergeWaves = 4;
 
 __global__ __launch_bounds__(kMergeWaves * 64) void merge_topk_kernel(const uint64_t* __restrict__ cand, int32_t blocks,
-                                                                      const int64_t* __restrict__ doc_global_id, float mul,
-                                                                      int32_t topk, float* __restrict__ scores_out,
-                                                                      int32_t* __restrict__ doc_out,
-                                                                      int64_t* __restrict__ doc_global_out) {
+                                                                      int32_t topk, TopkOut out) {
   __shared__ uint64_t lists[kMergeWaves][64];
   const int b = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint64_t best = 0;
@@ -152,20 +177,18 @@ __global__ __launch_bounds__(kMergeWaves * 64) void merge_topk_kernel(const uint
   if (wave != 0) return;
 #pragma unroll
   for (int w = 1; w < kMergeWaves; ++w) best = wave_merge_desc(best, lists[w][lane], lane);
-  if (lane < topk) {
-    const int64_t o = (int64_t)b * topk + lane;
-    if (best == 0) {
-      scores_out[o] = -INFINITY;
-      doc_out[o] = -1;
-      if (doc_global_out) doc_global_out[o] = -1;
-    } else {
-      const uint32_t k = (uint32_t)(best >> 32);
-      const int32_t d = (int32_t)(0xffffffffu - (uint32_t)best);
-      scores_out[o] = k == 0 ? -INFINITY : key_to_f32(k) * mul;
-      doc_out[o] = d;
-      if (doc_global_out) doc_global_out[o] = doc_global_id[d];
-    }
-  }
+  write_topk(out, b, topk, lane, best);
+}
+
+// The top-k of every query's keys [B, n_docs].
+int launch_topk(const uint32_t* key, const msa_bank* bank, const RouteWorkspace& w, uint64_t* cand, int32_t B, int32_t topk,
+                const TopkOut& out, hipStream_t st) {
+  doc_topk_kernel<<<dim3((unsigned)w.topk_blocks, (unsigned)B), kWaves * 64, 0, st>>>(key, (int32_t)bank->n_docs, topk, cand, out);
+  MSA_LAUNCH_CHECK();
+  if (w.topk_blocks == 1) return MSA_OK;
+  merge_topk_kernel<<<B, kMergeWaves * 64, 0, st>>>(cand, w.topk_blocks, topk, out);
+  MSA_LAUNCH_CHECK();
+  return MSA_OK;
 }
 
 }  // namespace
@@ -187,13 +210,7 @@ int route_topk_impl(const msa_bank* bank, int32_t layer, const void* q, const ui
   char* ws = static_cast<char*>(workspace);
   const uint32_t* key = reinterpret_cast<const uint32_t*>(ws + w.off_key);
   uint64_t* cand = reinterpret_cast<uint64_t*>(ws + w.off_cand);
-  dim3 grid((unsigned)w.topk_blocks, (unsigned)B);
-  doc_topk_kernel<<<grid, kWaves * 64, 0, st>>>(key, (int32_t)bank->n_docs, topk, cand);
-  MSA_LAUNCH_CHECK();
-  merge_topk_kernel<<<B, kMergeWaves * 64, 0, st>>>(cand, w.topk_blocks, bank->doc_global_id_dev, mul, topk, scores_out, doc_out,
-                                      doc_global_out);
-  MSA_LAUNCH_CHECK();
-  return MSA_OK;
+  return launch_topk(key, bank, w, cand, B, topk, TopkOut{bank->doc_global_id_dev, mul, scores_out, doc_out, doc_global_out}, st);
 }
 
 // keys of the per-chunk scores [B, C] -> keys of each document's mean over its chunks [B, n_docs]; a query whose
@@ -242,13 +259,7 @@ extern "C" int msa_route_topk_reduce(const msa_bank* bank, int32_t layer, const 
     key = doc_key;
   }
   uint64_t* cand = reinterpret_cast<uint64_t*>(ws + w.off_cand);
-  dim3 grid((unsigned)w.topk_blocks, (unsigned)B);
-  doc_topk_kernel<<<grid, kWaves * 64, 0, st>>>(key, (int32_t)bank->n_docs, topk, cand);
-  MSA_LAUNCH_CHECK();
-  merge_topk_kernel<<<B, kMergeWaves * 64, 0, st>>>(cand, w.topk_blocks, bank->doc_global_id_dev, mul, topk, scores_out, doc_out,
-                                      doc_global_out);
-  MSA_LAUNCH_CHECK();
-  return MSA_OK;
+  return launch_topk(key, bank, w, cand, B, topk, TopkOut{bank->doc_global_id_dev, mul, scores_out, doc_out, doc_global_out}, st);
 }
 
 extern "C" int msa_route_topk(const msa_bank* bank, int32_t layer, const void* q, const uint8_t* qmask_u8, int32_t B,
