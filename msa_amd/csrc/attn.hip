@@ -24,17 +24,10 @@ __device__ __forceinline__ uint4 ld16_stream(const void* p) {
   return make_uint4(w.x, w.y, w.z, w.w);
 }
 
-template <typename T>
-__device__ __forceinline__ void ld8(const T* p, float (&x)[8]) {
-  if constexpr (sizeof(T) == 2) {
-    const uint4 w = ld16_stream(p);
-    x[0] = bf16lo(w.x); x[1] = bf16hi(w.x); x[2] = bf16lo(w.y); x[3] = bf16hi(w.y);
-    x[4] = bf16lo(w.z); x[5] = bf16hi(w.z); x[6] = bf16lo(w.w); x[7] = bf16hi(w.w);
-  } else {
-    const uint4 a = ld16_stream(p), b = ld16_stream(p + 4);
-    x[0] = __uint_as_float(a.x); x[1] = __uint_as_float(a.y); x[2] = __uint_as_float(a.z); x[3] = __uint_as_float(a.w);
-    x[4] = __uint_as_float(b.x); x[5] = __uint_as_float(b.y); x[6] = __uint_as_float(b.z); x[7] = __uint_as_float(b.w);
-  }
+__device__ __forceinline__ void ld8(const float* p, float (&x)[8]) {
+  const uint4 a = ld16_stream(p), b = ld16_stream(p + 4);
+  x[0] = __uint_as_float(a.x); x[1] = __uint_as_float(a.y); x[2] = __uint_as_float(a.z); x[3] = __uint_as_float(a.w);
+  x[4] = __uint_as_float(b.x); x[5] = __uint_as_float(b.y); x[6] = __uint_as_float(b.z); x[7] = __uint_as_float(b.w);
 }
 
 // Finds the sample owning query row `row` in cu_q (B is small: linear scan is fine and uniform).
@@ -42,6 +35,11 @@ __device__ __forceinline__ int find_sample(const int32_t* cu_q, int B, int row) 
   int b = 0;
   while (b + 1 < B && cu_q[b + 1] <= row) ++b;
   return b;
+}
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
 }
 
 // sum over the 16 lanes of a DPP row (the lanes sharing one key); every lane gets the total
@@ -58,8 +56,8 @@ __device__ __forceinline__ float row16_allsum(float d) {
 // batch are issued before any arithmetic (bytes in flight), scores are reduced over the 16 lanes of a key with
 // DPP row rotations, and the running softmax is rescaled once per batch.  `lane_off` is the element offset of
 // key 0's slice for this lane.
-template <typename T, int G>
-__device__ __forceinline__ void attend_keys(const T* __restrict__ k, const T* __restrict__ v, int64_t lane_off,
+template <int G>
+__device__ __forceinline__ void attend_keys(const float* __restrict__ k, const float* __restrict__ v, int64_t lane_off,
                                             int row_elems, int first, int key1, int stride, const float (&qv)[G][8],
                                             float (&m)[G], float (&l)[G], float (&acc)[G][8]) {
   constexpr int kBatch = 4;
@@ -71,8 +69,8 @@ __device__ __forceinline__ void attend_keys(const T* __restrict__ k, const T* __
       const int kk = kb + u * stride;
       ok[u] = kk < key1;
       const int64_t off = lane_off + (int64_t)(ok[u] ? kk : kb) * row_elems;   // clamp: always in range
-      ld8<T>(k + off, kx[u]);
-      ld8<T>(v + off, vx[u]);
+      ld8(k + off, kx[u]);
+      ld8(v + off, vx[u]);
     }
 #pragma unroll
     for (int h = 0; h < G; ++h) {
@@ -105,97 +103,251 @@ __device__ __forceinline__ void attend_keys(const T* __restrict__ k, const T* __
   }
 }
 
-// bf16 form on packed operands: q.k with v_dot2c_f32_bf16 (two products per instruction, K is never unpacked; q
-// stays un-scaled in bf16 and the fp32 dot is scaled afterwards), and p.v over PAIRS of keys: the two keys'
-// values of one dim are interleaved with v_perm_b32 and the two probabilities rounded to bf16 (as flash
-// attention does before its second product).  qp[h][c] holds dims 8 j + 2 c, 8 j + 2 c + 1 of head h.
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
-  union { uint32_t u; bf16x2_t v; } x, y;
-  x.u = a; y.u = b;
-  return __builtin_amdgcn_fdot2_f32_bf16(x.v, y.v, c, false);
+// ------------------------------------------------------------------------------------------------
+// bf16 single rows: keys and values of one KV head through a ring in LDS, products on the matrix cores.
+//
+// A workgroup has four wavefronts, each with 8 KB for a step's 32 keys and 8 KB for their values, and every fourth step, so that
+// nothing waits for another wavefront until the end.  K is requested again as soon as its products are read, under the softmax, V
+// behind the second product: 8 to 16 KB a wavefront are in flight, and two workgroups a compute unit cover each other's ends.  Rows
+// of 256 bytes arrive by direct-to-LDS loads, four whole rows an instruction, non-temporal (a decode step reads every cache row
+// once), their 16-byte units XORed with the row against bank conflicts.  S^T = K Q^T (16 keys x 16 heads, of which G exist) leaves
+// the scores where P^T is wanted as the operand of O^T = V^T P^T; V^T comes by transposing LDS reads.  What bounds it is HBM for long
+// contexts (8 KV heads: 16 samples of 32768 keys 353 us, 6.1 TB/s; 16 of 2194 to 4388 keys 52.3 -> 47.9 us; one of 4388 17.5 -> 11.9)
+// and the chain lengths - first step - sums - combining launch for short ones (one sample of 256 keys 9.5 -> 8.8 us): the form
+// before held K and V in registers and took packed dot products on the vector units, 350 instructions per 8 KB.
+// ------------------------------------------------------------------------------------------------
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
+typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+constexpr int kRingWaves = 4, kRingKeys = 32, kRowBytes = kHeadDim * 2, kSlab = kRingKeys * kRowBytes;
+constexpr int kParts = kRingWaves + 1, kSumStride = kHeadDim + 4;      // a wavefront each, and the new token's
+[[maybe_unused]] constexpr int kNonTemporal = 2;
+constexpr int kRingLds = kRingWaves * 2 * kSlab;
+constexpr int wait_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }   // vmcnt(n) alone
+
+__device__ __forceinline__ uint32_t lds_offset(const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
+// 16 bytes of LDS that no ring writes: the compiler's own accesses would wait for what the rings have in flight.
+__device__ __forceinline__ uint4 lds_read16(const uint4* p) {
+  u32x4_t v;
+  asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(lds_offset(p)) : "memory");
+  return make_uint4(v.x, v.y, v.z, v.w);
 }
-__device__ __forceinline__ uint32_t pack_pair_rne(float lo, float hi) {
-  typedef float f32x2_t __attribute__((ext_vector_type(2)));
-  union { bf16x2_t b; uint32_t u; } c;
-  c.b = __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t);
-  return c.u;
+__device__ __forceinline__ void lds_write16(uint4* p, uint4 v) {
+  asm volatile("ds_write_b128 %0, %1" : : "v"(lds_offset(p)), "v"(u32x4_t{v.x, v.y, v.z, v.w}) : "memory");
 }
 
-template <int G>
-__device__ __forceinline__ void attend_keys_bf16(const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
-                                                 int64_t lane_off, int row_elems, int first, int key1, int stride,
-                                                 const uint32_t (&qp)[G][4], float scale_log2e, float (&m)[G],
-                                                 float (&l)[G], float (&acc)[G][8]) {
-  constexpr int kBatch = 4;
-  for (int kb = first; kb < key1; kb += stride * kBatch) {
-    uint4 kx[kBatch], vx[kBatch];
-    bool ok[kBatch];
+// What one wavefront (or the new token) knows of its keys, per head: reference maximum, sum, un-normalised output.  A wavefront's
+// lie where its ring was, the new token's behind the rings.
+struct HeadSums {
+  float m[kMaxG], l[kMaxG], o[kMaxG][kSumStride];
+};
+static_assert(sizeof(HeadSums) <= 2 * kSlab, "sums take a ring's place");
+__device__ __forceinline__ HeadSums& sums_of(char* lds, int part) { return *reinterpret_cast<HeadSums*>(lds + part * 2 * kSlab); }
+
+// Keys key0 .. key1 (`k` / `v`: the head's columns of key 0, `row_bytes` between keys).  `start` requests this wavefront's first
+// step; `run` leaves its sums where its ring was.
+struct Ring {
+  const bf16_t *k, *v;
+  char *kt, *vt;
+  int row_bytes, key0, key1, steps, wave, off[4];
+  __device__ __forceinline__ Ring(const bf16_t* k_, const bf16_t* v_, int row_bytes_, int key0_, int key1_, int wave_, int lane, char* lds)
+      : k(k_), v(v_), kt(lds + wave_ * 2 * kSlab), vt(kt + kSlab), row_bytes(row_bytes_), key0(key0_), key1(key1_),
+        steps(key1_ > key0_ ? (key1_ - key0_ + kRingKeys - 1) / kRingKeys : 0), wave(wave_) {
+    // lane's place in four rows: row lane / 16, where unit (lane % 16) ^ row lies; rows 4 i .. further on change the unit's high bits
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int kk = kb + u * stride;
-      ok[u] = kk < key1;
-      const int64_t off = lane_off + (int64_t)(ok[u] ? kk : kb) * row_elems;   // clamp: always in range
-      kx[u] = ld16_stream(k + off);
-      vx[u] = ld16_stream(v + off);
-    }
-    // scores of all heads first: they only need K, so the arithmetic starts while V is still arriving
-    float s[G][kBatch];
+    for (int i = 0; i < 4; ++i) off[i] = (4 * i + (lane >> 4)) * row_bytes + (((lane & 15) ^ (4 * i + (lane >> 4))) * 16);
+  }
+  __device__ __forceinline__ void request(const bf16_t* src, char* dst, int step) const {
+    const int64_t at = (int64_t)(key0 + (step < steps ? step : 0) * kRingKeys) * row_bytes;
+    const int rows = __builtin_amdgcn_readfirstlane(step < steps ? min(kRingKeys, key1 - key0 - step * kRingKeys) : 0);
+    const int extent = rows > 0 ? (rows - 1) * row_bytes + kRowBytes : 0;       // rows behind the range read as zeros
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(src) + at), 0, extent, 0x00020000);
 #pragma unroll
-    for (int h = 0; h < G; ++h)
+    for (int i = 0; i < 8; ++i) MSA_LOAD_TO_LDS(rs, dst + i * 1024, off[i & 3], (i >> 2) * 16 * row_bytes, kNonTemporal);
+  }
+  __device__ __forceinline__ void start() const {
+    request(k, kt, wave);
+    request(v, vt, wave);
+  }
+  __device__ __forceinline__ void run(int lane, int G, const bf16x8_t (&qf)[4], float scale_log2e, char* lds) const;
+};
+
+__device__ __forceinline__ void Ring::run(int lane, int G, const bf16x8_t (&qf)[4], float scale_log2e, char* lds) const {
+  const int l16 = lane & 15, g = lane >> 4;
+  // V^T operands: eight bytes of row 4 g + l16 / 4 (and of the row 16 further on): lanes 4 r .. 4 r + 3 of 16 name the pieces of
+  // row r, column block c's 32 bytes of it being units 2 c and 2 c + 1
+  uint32_t v_at[8];
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        float d = dot2_bf16(qp[h][0], kx[u].x, 0.f);
-        d = dot2_bf16(qp[h][1], kx[u].y, d);
-        d = dot2_bf16(qp[h][2], kx[u].z, d);
-        d = dot2_bf16(qp[h][3], kx[u].w, d);
-        d = row16_allsum(d);
-        s[h][u] = ok[u] ? d * scale_log2e : -INFINITY;
-      }
-    // the two keys of a pair, one dim per 32-bit word: vlo[pr][c] = (v_2pr[2c], v_2pr+1[2c]), vhi the odd dims
-    uint32_t vlo[kBatch / 2][4], vhi[kBatch / 2][4];
+  for (int c = 0; c < 8; ++c) {
+    const int row = 4 * g + (l16 >> 2);
+    v_at[c] = lds_offset(vt) + row * kRowBytes + (l16 & 1) * 8 + (((2 * c + ((l16 & 3) >> 1)) ^ row) * 16);
+  }
+  // A second pass without the weights' low parts, if there are NaN: a low part of zero or below against an infinite value makes one
+  // where the weight itself leaves the infinity.
+  floatx4_t o[8];
+  float m, l;                            // of head l16: m the same in its four lanes, l each lane's own keys
+  for (bool low_part = true;;) {
 #pragma unroll
-    for (int pr = 0; pr < kBatch / 2; ++pr) {
-      const uint32_t a[4] = {vx[2 * pr].x, vx[2 * pr].y, vx[2 * pr].z, vx[2 * pr].w};
-      const uint32_t b[4] = {vx[2 * pr + 1].x, vx[2 * pr + 1].y, vx[2 * pr + 1].z, vx[2 * pr + 1].w};
+    for (int c = 0; c < 8; ++c) o[c] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    m = -INFINITY;
+    l = 0.f;
+    for (int step = wave; step < steps; step += kRingWaves) {
+      __builtin_amdgcn_s_waitcnt(wait_vm(8));                // K: only V is younger
+      asm volatile("" ::: "memory");
+      floatx4_t sc[2] = {floatx4_t{0.f, 0.f, 0.f, 0.f}, floatx4_t{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        vlo[pr][c] = __builtin_amdgcn_perm(b[c], a[c], 0x05040100u);
-        vhi[pr][c] = __builtin_amdgcn_perm(b[c], a[c], 0x07060302u);
-      }
-    }
+      for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float mb = m[h];
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) mb = fmaxf(mb, s[h][u]);
-      const float alpha = fast_exp2(m[h] - mb);          // mb is finite: the batch's first key is always valid
-      float psum = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc[h][i] *= alpha;
-#pragma unroll
-      for (int pr = 0; pr < kBatch / 2; ++pr) {
-        const float p0 = fast_exp2(s[h][2 * pr] - mb), p1 = fast_exp2(s[h][2 * pr + 1] - mb);
-        psum += p0 + p1;
-        const uint32_t pp = pack_pair_rne(p0, p1);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          acc[h][2 * c] = dot2_bf16(vlo[pr][c], pp, acc[h][2 * c]);
-          acc[h][2 * c + 1] = dot2_bf16(vhi[pr][c], pp, acc[h][2 * c + 1]);
+        for (int t = 0; t < 2; ++t) {
+          const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(kt + (16 * t + l16) * kRowBytes + ((4 * kk + g) ^ l16) * 16);
+          sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[kk], sc[t], 0, 0, 0);
         }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // K may be requested again
+      request(k, kt, step + kRingWaves);
+      // sc[t][e] is head l16's score of key 16 t + 4 g + e
+      const int valid = key1 - key0 - step * kRingKeys;
+      float x[2][4], mx = m;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[t][e] = 16 * t + 4 * g + e < valid ? sc[t][e] * scale_log2e : -INFINITY;
+          mx = fmaxf(mx, x[t][e]);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      if (__any(mx > m)) {
+        const float alpha = mx == -INFINITY ? 1.f : fast_exp2(m - mx);
+        l *= alpha;
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[c][e] *= alpha;
+        m = mx;
       }
-      l[h] = l[h] * alpha + psum;
-      m[h] = mb;
+      const float ref = m == -INFINITY ? 0.f : m;            // (scores of -inf alone: every weight is 0)
+      // weights as a high and a low bf16 part: rounded once, they depend on which keys share a reference maximum
+      uint32_t ph[4], pl[4];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+          const float p0 = fast_exp2(x[t][e] - ref), p1 = fast_exp2(x[t][e + 1] - ref);
+          l += p0 + p1;
+          const uint32_t hi = pack_bf16x2(p0, p1);
+          ph[2 * t + e / 2] = hi;
+          pl[2 * t + e / 2] = pack_bf16x2(p0 - bf16lo(hi), p1 - bf16hi(hi));
+        }
+      const bf16x8_t hi8 = __builtin_bit_cast(bf16x8_t, make_uint4(ph[0], ph[1], ph[2], ph[3]));
+      const bf16x8_t lo8 = __builtin_bit_cast(bf16x8_t, make_uint4(pl[0], pl[1], pl[2], pl[3]));
+      __builtin_amdgcn_s_waitcnt(wait_vm(8));                // V: only the next K is younger
+      asm volatile("" ::: "memory");
+      // (the transposing reads are written out, wait included: in front of its own the compiler waits for the next K too, 4 us in 50)
+      u32x2_t vr[16];
+      asm volatile(
+          "ds_read_b64_tr_b16 %0, %16\n\tds_read_b64_tr_b16 %1, %16 offset:4096\n\t"
+          "ds_read_b64_tr_b16 %2, %17\n\tds_read_b64_tr_b16 %3, %17 offset:4096\n\t"
+          "ds_read_b64_tr_b16 %4, %18\n\tds_read_b64_tr_b16 %5, %18 offset:4096\n\t"
+          "ds_read_b64_tr_b16 %6, %19\n\tds_read_b64_tr_b16 %7, %19 offset:4096\n\t"
+          "ds_read_b64_tr_b16 %8, %20\n\tds_read_b64_tr_b16 %9, %20 offset:4096\n\t"
+          "ds_read_b64_tr_b16 %10, %21\n\tds_read_b64_tr_b16 %11, %21 offset:4096\n\t"
+          "ds_read_b64_tr_b16 %12, %22\n\tds_read_b64_tr_b16 %13, %22 offset:4096\n\t"
+          "ds_read_b64_tr_b16 %14, %23\n\tds_read_b64_tr_b16 %15, %23 offset:4096\n\t"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&v"(vr[0]), "=&v"(vr[1]), "=&v"(vr[2]), "=&v"(vr[3]), "=&v"(vr[4]), "=&v"(vr[5]), "=&v"(vr[6]), "=&v"(vr[7]),
+            "=&v"(vr[8]), "=&v"(vr[9]), "=&v"(vr[10]), "=&v"(vr[11]), "=&v"(vr[12]), "=&v"(vr[13]), "=&v"(vr[14]), "=&v"(vr[15])
+          : "v"(v_at[0]), "v"(v_at[1]), "v"(v_at[2]), "v"(v_at[3]), "v"(v_at[4]), "v"(v_at[5]), "v"(v_at[6]), "v"(v_at[7])
+          : "memory");
+      request(v, vt, step + kRingWaves);                     // (V has been read)
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, make_uint4(vr[2 * c].x, vr[2 * c].y, vr[2 * c + 1].x, vr[2 * c + 1].y));
+        o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, hi8, o[c], 0, 0, 0);
+        if (low_part) o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, lo8, o[c], 0, 0, 0);
+      }
     }
+    __builtin_amdgcn_s_waitcnt(wait_vm(0));                  // nothing may still be writing LDS when the sums go there
+    asm volatile("" ::: "memory");
+    bool nan = false;
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) nan |= o[c][e] != o[c][e];
+    if (!low_part || !__any(nan)) break;
+    low_part = false;
+    start();
+  }
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (l16 >= G) return;
+  HeadSums& out = sums_of(lds, wave);
+#pragma unroll
+  for (int c = 0; c < 8; ++c) *reinterpret_cast<floatx4_t*>(&out.o[l16][16 * c + 4 * g]) = o[c];
+  if (g == 0) {
+    out.m[l16] = m;
+    out.l[l16] = l;
   }
 }
 
-template <typename T, int G, int kAttnWaves>
+// Folds the first `parts` sums of a head; thread (h, d).
+__device__ __forceinline__ void fold_sums(char* lds, int parts, int h, int d, float& m, float& l, float& o) {
+  m = -INFINITY;
+  for (int w = 0; w < parts; ++w) m = fmaxf(m, sums_of(lds, w).m[h]);
+  l = o = 0.f;
+  for (int w = 0; w < parts; ++w) {
+    const HeadSums& s = sums_of(lds, w);
+    const float a = s.m[h] == -INFINITY ? 0.f : fast_exp2(s.m[h] - m);
+    l += s.l[h] * a;
+    o += s.o[h][d] * a;
+  }
+}
+
+// bf16 rows: workgroup (row, KV head, split) as in attn_partial_kernel below.
+__global__ __launch_bounds__(kRingWaves * 64) void attn_ring_kernel(
+    const bf16_t* __restrict__ q, const int32_t* __restrict__ cu_q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
+    const int64_t* __restrict__ kv_off, const int32_t* __restrict__ kv_len, int32_t B, int32_t Hq, int32_t Hkv, float scale_log2e,
+    int32_t causal, int32_t n_split, float* __restrict__ part_ml, float* __restrict__ part_acc, bf16_t* __restrict__ out) {
+  extern __shared__ __align__(16) char lds[];
+  const int row = blockIdx.x, g = blockIdx.y, split = blockIdx.z, G = Hq / Hkv;
+  const int b = cu_q ? find_sample(cu_q, B, row) : row;
+  const int q_first = cu_q ? cu_q[b] : row, sq = cu_q ? cu_q[b + 1] - q_first : 1;
+  const int L = kv_len[b], visible = causal ? max(0, L - sq + (row - q_first) + 1) : L;
+  // balanced splits of this sample's own length (the host only knows an upper bound of it)
+  const int per_split = (L + n_split - 1) / n_split, key0 = split * per_split, key1 = min(visible, key0 + per_split);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t at = kv_off[b] * Hkv * kHeadDim + g * kHeadDim;
+  const Ring ring(k + at, v + at, Hkv * kRowBytes, key0, key1, wave, lane, lds);
+  bf16x8_t qf[4];
+  const uint4* q16 = reinterpret_cast<const uint4*>(q + ((int64_t)row * Hq + g * G) * kHeadDim);
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk)                           // lane l16 holds head l16, zeros behind the last
+    qf[kk] = __builtin_bit_cast(bf16x8_t, (lane & 15) < G ? q16[(lane & 15) * 16 + 4 * kk + (lane >> 4)] : make_uint4(0, 0, 0, 0));
+  asm volatile("" ::: "memory");                           // (the ring counts what is younger)
+  ring.start();
+  ring.run(lane, G, qf, scale_log2e, lds);
+  __syncthreads();
+  for (int idx = tid; idx < G * kHeadDim; idx += kRingWaves * 64) {
+    const int h = idx / kHeadDim, d = idx % kHeadDim;
+    float mn, lt, at_d;
+    fold_sums(lds, kRingWaves, h, d, mn, lt, at_d);
+    const int64_t o = ((int64_t)row * Hq + g * G + h) * n_split + split;
+    if (n_split == 1) {                                    // nothing to merge: the output itself (a launch of 4 us less)
+      out[o * kHeadDim + d] = f32_to_bf16(lt > 0.f ? at_d / lt : 0.f);          // a row that sees no key yields zeros
+      continue;
+    }
+    part_acc[o * kHeadDim + d] = at_d;
+    if (d == 0) { part_ml[o * 2] = mn; part_ml[o * 2 + 1] = lt; }
+  }
+}
+
+// fp32 rows.
+template <int G, int kAttnWaves>
 __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
-    const T* __restrict__ q, const int32_t* __restrict__ cu_q, const T* __restrict__ k, const T* __restrict__ v,
+    const float* __restrict__ q, const int32_t* __restrict__ cu_q, const float* __restrict__ k, const float* __restrict__ v,
     const int64_t* __restrict__ kv_off, const int32_t* __restrict__ kv_len, int32_t B, int32_t Hq, int32_t Hkv,
-    float scale_log2e, int32_t causal, int32_t n_split, int32_t split_keys, float* __restrict__ part_ml,
-    float* __restrict__ part_acc, T* __restrict__ out) {
+    float scale_log2e, int32_t causal, int32_t n_split, float* __restrict__ part_ml,
+    float* __restrict__ part_acc, float* __restrict__ out) {
   __shared__ float sm_m[kAttnWaves][G], sm_l[kAttnWaves][G];
   __shared__ float sm_acc[kAttnWaves][G][kHeadDim];
 
@@ -206,7 +358,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
   const int L = kv_len[b];
   const int visible = causal ? max(0, L - sq + (row - q_first) + 1) : L;
   // balanced splits of this sample's own length (the host only knows an upper bound of it)
-  const int per_split = split_keys > 0 ? split_keys : (L + n_split - 1) / n_split;
+  const int per_split = (L + n_split - 1) / n_split;
   const int key0 = split * per_split;
   const int key1 = min(visible, key0 + per_split);
 
@@ -223,27 +375,15 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
     for (int i = 0; i < 8; ++i) acc[h][i] = 0.f;
   }
   const int64_t lane_off = base * row_elems + g * kHeadDim + 8 * j;     // this lane's slice of key 0
-  const T* q_lane = q + ((int64_t)row * Hq + g * G) * kHeadDim + 8 * j;
-  // the packed form pays off once several heads share the loads (its dependent dot2 / DPP chains need the
-  // other heads' work to hide behind): measured 61 vs 65 us at G = 4, 88 vs 112 at G = 8, but 65 vs 55 at G = 1
-  if constexpr (sizeof(T) == 2 && G >= 4) {
-    uint32_t qp[G][4];
+  const float* q_lane = q + ((int64_t)row * Hq + g * G) * kHeadDim + 8 * j;
+  float qv[G][8];
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      const uint4 w = *reinterpret_cast<const uint4*>(q_lane + h * kHeadDim);
-      qp[h][0] = w.x; qp[h][1] = w.y; qp[h][2] = w.z; qp[h][3] = w.w;
-    }
-    attend_keys_bf16<G>(k, v, lane_off, row_elems, key0 + wave * 4 + slot, key1, kAttnWaves * 4, qp, scale_log2e, m, l, acc);
-  } else {
-    float qv[G][8];
+  for (int h = 0; h < G; ++h) {
+    ld8(q_lane + h * kHeadDim, qv[h]);
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      ld8<T>(q_lane + h * kHeadDim, qv[h]);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) qv[h][i] *= scale_log2e;      // scores in log2 units: exp2f below
-    }
-    attend_keys<T, G>(k, v, lane_off, row_elems, key0 + wave * 4 + slot, key1, kAttnWaves * 4, qv, m, l, acc);
+    for (int i = 0; i < 8; ++i) qv[h][i] *= scale_log2e;      // scores in log2 units: exp2f below
   }
+  attend_keys<G>(k, v, lane_off, row_elems, key0 + wave * 4 + slot, key1, kAttnWaves * 4, qv, m, l, acc);
 
   // merge the 4 key slots of the wavefront (lanes differing in bits 4 and 5)
 #pragma unroll
@@ -285,8 +425,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
     const int64_t o = ((int64_t)row * Hq + g * G + h) * n_split + split;
     if (n_split == 1) {                                  // nothing to merge: the output itself (a launch of 4 us less)
       const float y = lt > 0.f ? at / lt : 0.f;          // a row that sees no key yields zeros
-      if constexpr (sizeof(T) == 2) out[o * kHeadDim + d] = f32_to_bf16(y);
-      else out[o * kHeadDim + d] = y;
+      out[o * kHeadDim + d] = y;
       continue;
     }
     part_acc[o * kHeadDim + d] = at;
@@ -297,209 +436,183 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
 // ------------------------------------------------------------------------------------------------
 // Decode step with the q / k RMSNorm, the rotary embedding and the cache append folded into the attention launch
 // (bf16, one new token per sample, groups of 4 or 8 query heads).  Row b of `qkv` is the fused projection output
-// [Hq q heads | Hkv k heads | Hkv v heads].  Every workgroup (sample, KV head, split) normalises and rotates the q
-// heads of its group (16 lanes per head, 8 dims per lane, the same arithmetic as the stand-alone kernel) and shares
-// them through LDS; the workgroup of the last split also prepares the new token's k / v row of its KV head, writes it
-// to the cache at [b][kv_len[b]] and feeds it to its running softmax as one more key.  kv_len is only read here: the
-// combine kernel that follows advances it.  A full cache drops the new row (and the token then does not see itself).
+// [Hq q heads | Hkv k heads | Hkv v heads].  A workgroup normalises and rotates the q heads of its group (16 lanes per head, 8 dims
+// per lane, the same arithmetic as the stand-alone kernel) and shares them through LDS; the workgroup with a sample's last keys
+// also prepares the new token's k / v row of its KV head, writes it to the cache at [b][kv_len[b]] and folds it in as one more
+// key.  kv_len is only read here: the combine kernel that follows advances it.  A full cache drops the new row (and the token
+// then does not see itself).
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ float row16_ror8(float v) {  // value of the lane 8 places away in the 16-lane row
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false));
 }
 
-// RMSNorm over the head's 128 dims (fp32) times the norm weight, then half-split rotary with the table row
-// cos_row / sin_row; `src` and `w` point at this lane's 8 elements; returns them packed to bf16.
-__device__ __forceinline__ uint4 norm_rope_8(const bf16_t* src, const bf16_t* w, float eps, const float* cos_row,
-                                             const float* sin_row, int j) {
-  const uint4 xr = *reinterpret_cast<const uint4*>(src), wr = *reinterpret_cast<const uint4*>(w);
-  const uint32_t xs[4] = {xr.x, xr.y, xr.z, xr.w}, ws[4] = {wr.x, wr.y, wr.z, wr.w};
-  float x[8], wt[8];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    x[2 * c] = bf16lo(xs[c]); x[2 * c + 1] = bf16hi(xs[c]);
-    wt[2 * c] = bf16lo(ws[c]); wt[2 * c + 1] = bf16hi(ws[c]);
+// RMSNorm over a head's 128 dims (fp32) times the norm weight, then half-split rotary, 16 lanes a head and 8 dims a lane.  What it
+// takes from memory is requested apart from what is done with it: the ring's requests go between the two.
+struct NormRope {
+  uint4 x, w;
+  float cs[8], sn[8];
+  __device__ __forceinline__ void load(const bf16_t* src, const bf16_t* weight) {            // this lane's 8 elements
+    x = *reinterpret_cast<const uint4*>(src);
+    w = *reinterpret_cast<const uint4*>(weight);
   }
-  float ssq = 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) ssq += x[i] * x[i];
-  const float inv = rsqrtf(row16_allsum(ssq) * (1.0f / kHeadDim) + eps);
-  const int f = 8 * (j & 7);                    // frequency index of this lane's first element
-  float out[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float y = x[i] * inv * wt[i];
-    const float other = row16_ror8(y);          // the paired dim (d + 64 for j < 8, d - 64 for j >= 8)
-    const float c = cos_row[f + i], sn = sin_row[f + i];
-    out[i] = j < 8 ? y * c - other * sn : y * c + other * sn;
+  __device__ __forceinline__ void load_rotary(const float* cos_row, const float* sin_row, int j) {
+    ld8(cos_row + 8 * (j & 7), cs);
+    ld8(sin_row + 8 * (j & 7), sn);
   }
-  uint4 r;
-  r.x = pack_bf16x2(out[0], out[1]); r.y = pack_bf16x2(out[2], out[3]);
-  r.z = pack_bf16x2(out[4], out[5]); r.w = pack_bf16x2(out[6], out[7]);
-  return r;
-}
+  __device__ __forceinline__ uint4 result(float eps, int j) const {
+    const uint32_t xs[4] = {x.x, x.y, x.z, x.w}, ws[4] = {w.x, w.y, w.z, w.w};
+    float v[8], wt[8], ssq = 0.f, out[8];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      v[2 * c] = bf16lo(xs[c]); v[2 * c + 1] = bf16hi(xs[c]);
+      wt[2 * c] = bf16lo(ws[c]); wt[2 * c + 1] = bf16hi(ws[c]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ssq += v[i] * v[i];
+    const float inv = rsqrtf(row16_allsum(ssq) * (1.0f / kHeadDim) + eps);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float y = v[i] * inv * wt[i];
+      const float other = row16_ror8(y);        // the paired dim (d + 64 for j < 8, d - 64 for j >= 8)
+      out[i] = j < 8 ? y * cs[i] - other * sn[i] : y * cs[i] + other * sn[i];
+    }
+    return make_uint4(pack_bf16x2(out[0], out[1]), pack_bf16x2(out[2], out[3]), pack_bf16x2(out[4], out[5]), pack_bf16x2(out[6], out[7]));
+  }
+};
 
-template <int G>
-__global__ __launch_bounds__(8 * 64) void attn_decode_fused_kernel(
+__global__ __launch_bounds__(kRingWaves * 64) void attn_decode_fused_kernel(
     const bf16_t* __restrict__ qkv, int64_t row_stride, int32_t Hq, int32_t Hkv, const int64_t* __restrict__ pos,
     const bf16_t* __restrict__ qw, const bf16_t* __restrict__ kw, float eps, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, int32_t rope_rows, bf16_t* __restrict__ kcache, bf16_t* __restrict__ vcache,
     int32_t Lcap, const int32_t* __restrict__ kv_len, float scale_log2e, int32_t n_split,
     float* __restrict__ part_ml, float* __restrict__ part_acc) {
-  constexpr int kW = 8;
-  __shared__ float sm_m[kW][G], sm_l[kW][G];
-  __shared__ float sm_acc[kW][G][kHeadDim];
-  __shared__ uint4 sm_q[G][16];
+  extern __shared__ __align__(16) char lds[];
+  HeadSums& new_token = sums_of(lds, kRingWaves);
+  uint4* sm_q = reinterpret_cast<uint4*>(lds + kRingLds + sizeof(HeadSums));        // [G][16]
+  const int b = blockIdx.x, g = blockIdx.y, split = blockIdx.z, G = Hq / Hkv;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15, hq = tid >> 4;                  // 16 lanes a head: the group's q heads, and behind them the new key
+  const bf16_t* row = qkv + (int64_t)b * row_stride + 8 * j;
+  NormRope head;
+  head.load(row + (int64_t)(hq < G ? g * G + hq : Hq + g) * kHeadDim, (hq < G ? qw : kw) + 8 * j);
+  const uint4 v_new = *reinterpret_cast<const uint4*>(row + (int64_t)(Hq + Hkv + g) * kHeadDim);
+  const int64_t p = min((int64_t)max((int64_t)0, pos[b]), (int64_t)rope_rows - 1);
+  head.load_rotary(cos_t + p * 64, sin_t + p * 64, j);
 
-  const int b = blockIdx.x, g = blockIdx.y, split = blockIdx.z;
   const int L_old = kv_len[b];
   const bool has_new = L_old < Lcap;
-  const int per_split = (L_old + n_split - 1) / n_split;
-  const int key0 = split * per_split;
-  const int key1 = min(L_old, key0 + per_split);
+  const int per_split = (L_old + n_split - 1) / n_split, key0 = split * per_split, key1 = min(L_old, key0 + per_split);
+  const int64_t column = ((int64_t)b * Lcap * Hkv + g) * kHeadDim;
+  const Ring ring(kcache + column, vcache + column, Hkv * kRowBytes, key0, key1, wave, lane, lds);
+  asm volatile("" ::: "memory");                           // (the requests above stay above: loads return in order)
+  ring.start();                                            // in flight under the queries' preparation
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int slot = lane >> 4, j = lane & 15;
-  const int row_elems = Hkv * kHeadDim;
-  const int64_t p = min((int64_t)max((int64_t)0, pos[b]), (int64_t)rope_rows - 1);
-  const float* cos_row = cos_t + p * 64;
-  const float* sin_row = sin_t + p * 64;
-  const bf16_t* row = qkv + (int64_t)b * row_stride;
-
-  // q heads of the group: head 4 wave + slot (wavefront 0, and wavefront 1 when G = 8)
-  const int hq = wave * 4 + slot;
-  if (hq < G) sm_q[hq][j] = norm_rope_8(row + (int64_t)(g * G + hq) * kHeadDim + 8 * j, qw + 8 * j, eps, cos_row, sin_row, j);
-  // the new token's key / value of this KV head: the last wavefront's first key slot, in the last split only
-  const bool owner = split == n_split - 1 && wave == kW - 1 && slot == 0 && has_new;
-  uint4 k_new = make_uint4(0, 0, 0, 0), v_new = k_new;
+  const uint4 prepared = head.result(eps, j);
+  if (hq < G) lds_write16(sm_q + hq * 16 + j, prepared);
+  // the new token: the first 16 lanes of the last wavefront of the last split
+  const bool takes_new = has_new && split == n_split - 1, owner = takes_new && wave == kRingWaves - 1 && lane < 16;
   if (owner) {
-    k_new = norm_rope_8(row + (int64_t)(Hq + g) * kHeadDim + 8 * j, kw + 8 * j, eps, cos_row, sin_row, j);
-    v_new = *reinterpret_cast<const uint4*>(row + (int64_t)(Hq + Hkv + g) * kHeadDim + 8 * j);
     const int64_t at = (((int64_t)b * Lcap + L_old) * Hkv + g) * kHeadDim + 8 * j;
-    *reinterpret_cast<uint4*>(kcache + at) = k_new;
+    *reinterpret_cast<uint4*>(kcache + at) = prepared;
     *reinterpret_cast<uint4*>(vcache + at) = v_new;
   }
-  __syncthreads();
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");         // (a full fence would wait for the ring)
 
-  float m[G], l[G], acc[G][8];
-  uint32_t qp[G][4];
+  bf16x8_t qf[4];
 #pragma unroll
-  for (int h = 0; h < G; ++h) {
-    m[h] = -INFINITY; l[h] = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[h][i] = 0.f;
-    const uint4 w = sm_q[h][j];
-    qp[h][0] = w.x; qp[h][1] = w.y; qp[h][2] = w.z; qp[h][3] = w.w;
+  for (int kk = 0; kk < 4; ++kk) {
+    const uint4 u = lds_read16(sm_q + (j < G ? j : 0) * 16 + 4 * kk + (lane >> 4));
+    qf[kk] = __builtin_bit_cast(bf16x8_t, j < G ? u : make_uint4(0, 0, 0, 0));
   }
-  const int64_t lane_off = (int64_t)b * Lcap * row_elems + g * kHeadDim + 8 * j;     // this lane's slice of key 0
-  attend_keys_bf16<G>(kcache, vcache, lane_off, row_elems, key0 + wave * 4 + slot, key1, kW * 4, qp, scale_log2e, m, l, acc);
+  ring.run(lane, G, qf, scale_log2e, lds);
   if (owner) {
-    // one more key, straight from registers; the probability is rounded to bf16 as in the paired products above
+    // one more key, straight from registers: its weight against itself is 1
     const uint32_t vs[4] = {v_new.x, v_new.y, v_new.z, v_new.w};
-#pragma unroll
     for (int h = 0; h < G; ++h) {
-      float d = dot2_bf16(qp[h][0], k_new.x, 0.f);
-      d = dot2_bf16(qp[h][1], k_new.y, d);
-      d = dot2_bf16(qp[h][2], k_new.z, d);
-      d = dot2_bf16(qp[h][3], k_new.w, d);
-      const float sc = row16_allsum(d) * scale_log2e;
-      const float mb = fmaxf(m[h], sc);
-      const float alpha = fast_exp2(m[h] - mb), pr = fast_exp2(sc - mb);
-      const float prb = bf16lo(pack_pair_rne(pr, 0.f));
+      const uint4 q4 = lds_read16(sm_q + h * 16 + j);
+      float d = dot2_bf16(q4.x, prepared.x, 0.f);
+      d = dot2_bf16(q4.y, prepared.y, d);
+      d = dot2_bf16(q4.z, prepared.z, d);
+      d = dot2_bf16(q4.w, prepared.w, d);
+      d = row16_allsum(d);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        acc[h][2 * c] = acc[h][2 * c] * alpha + prb * bf16lo(vs[c]);
-        acc[h][2 * c + 1] = acc[h][2 * c + 1] * alpha + prb * bf16hi(vs[c]);
+        new_token.o[h][8 * j + 2 * c] = bf16lo(vs[c]);
+        new_token.o[h][8 * j + 2 * c + 1] = bf16hi(vs[c]);
       }
-      l[h] = l[h] * alpha + pr;
-      m[h] = mb;
-    }
-  }
-
-  // merge the 4 key slots of the wavefront (lanes differing in bits 4 and 5)
-#pragma unroll
-  for (int h = 0; h < G; ++h) {
-#pragma unroll
-    for (int x = 16; x <= 32; x <<= 1) {
-      const float mo = __shfl_xor(m[h], x), lo = __shfl_xor(l[h], x);
-      const float mn = fmaxf(m[h], mo);
-      const float a = mn == -INFINITY ? 0.f : fast_exp2(m[h] - mn), bo = mn == -INFINITY ? 0.f : fast_exp2(mo - mn);
-      l[h] = l[h] * a + lo * bo;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc[h][i] = acc[h][i] * a + __shfl_xor(acc[h][i], x) * bo;
-      m[h] = mn;
-    }
-  }
-  if (slot == 0) {
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      if (j == 0) { sm_m[wave][h] = m[h]; sm_l[wave][h] = l[h]; }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) sm_acc[wave][h][8 * j + i] = acc[h][i];
+      if (j == 0) {
+        new_token.m[h] = d * scale_log2e;
+        new_token.l[h] = 1.f;
+      }
     }
   }
   __syncthreads();
-  for (int idx = tid; idx < G * kHeadDim; idx += kW * 64) {
+  for (int idx = tid; idx < G * kHeadDim; idx += kRingWaves * 64) {
     const int h = idx / kHeadDim, d = idx % kHeadDim;
-    float mn = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kW; ++w) mn = fmaxf(mn, sm_m[w][h]);
-    float lt = 0.f, at = 0.f;
-#pragma unroll
-    for (int w = 0; w < kW; ++w) {
-      const float a = mn == -INFINITY ? 0.f : fast_exp2(sm_m[w][h] - mn);
-      lt += sm_l[w][h] * a;
-      at += sm_acc[w][h][d] * a;
-    }
+    float mn, lt, at_d;
+    fold_sums(lds, takes_new ? kParts : kRingWaves, h, d, mn, lt, at_d);
     const int64_t o = ((int64_t)b * Hq + g * G + h) * n_split + split;
-    part_acc[o * kHeadDim + d] = at;
+    part_acc[o * kHeadDim + d] = at_d;
     if (d == 0) { part_ml[o * 2] = mn; part_ml[o * 2 + 1] = lt; }
   }
 }
 
-// One workgroup of 128 threads per (query row, head): merge the splits and normalise.
-// With `bump_len` (decode step whose attention kernel appended the new token's K / V row itself) the workgroup of
-// head 0 of row b also advances bump_len[b], unless the cache was full and the row was dropped.
+// One workgroup of 128 threads per (query row, head): merges the row's partials and normalises.  The partials are requested sixteen
+// at a time (one after the other, each waited for the one before: 32 of them took 16 us).  With `kv_len` (decode: rows = samples)
+// the workgroup of head 0 also advances the sample's cache length, unless the cache was full and the new row was dropped.
 template <typename T>
 __global__ __launch_bounds__(kHeadDim) void attn_combine_kernel(const float* __restrict__ part_ml,
                                                                 const float* __restrict__ part_acc, int32_t n_split,
-                                                                T* __restrict__ out, int32_t* __restrict__ bump_len = nullptr,
+                                                                T* __restrict__ out, int32_t* __restrict__ kv_len = nullptr,
                                                                 int32_t Lcap = 0, int32_t Hq = 1) {
+  constexpr int kBatch = 16;
   const int64_t rh = blockIdx.x;   // row * Hq + head
   const int d = threadIdx.x;
-  if (bump_len != nullptr && d == 0 && rh % Hq == 0) {
-    const int64_t b = rh / Hq;
-    const int32_t len = bump_len[b];
-    if (len < Lcap) bump_len[b] = len + 1;
+  if (kv_len != nullptr && d == 0 && rh % Hq == 0) {
+    const int32_t len = kv_len[rh / Hq];
+    if (len < Lcap) kv_len[rh / Hq] = len + 1;
   }
-  float mn = -INFINITY;
-  for (int s = 0; s < n_split; ++s) mn = fmaxf(mn, part_ml[(rh * n_split + s) * 2]);
-  float lt = 0.f, at = 0.f;
-  for (int s = 0; s < n_split; ++s) {
-    const float ms = part_ml[(rh * n_split + s) * 2];
-    const float a = ms == -INFINITY ? 0.f : fast_exp2(ms - mn);
-    lt += part_ml[(rh * n_split + s) * 2 + 1] * a;
-    at += part_acc[(rh * n_split + s) * kHeadDim + d] * a;
+  float mn = -INFINITY, lt = 0.f, at = 0.f;
+  for (int s0 = 0; s0 < n_split; s0 += kBatch) {
+    float ms[kBatch], ls[kBatch], as[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int64_t p = rh * n_split + min(s0 + i, n_split - 1);
+      ms[i] = part_ml[p * 2];
+      ls[i] = part_ml[p * 2 + 1];
+      as[i] = part_acc[p * kHeadDim + d];
+    }
+    float mb = mn;
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) mb = s0 + i < n_split ? fmaxf(mb, ms[i]) : mb;
+    const float keep = mn == -INFINITY ? 0.f : fast_exp2(mn - mb);
+    lt *= keep;
+    at *= keep;
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const float a = s0 + i < n_split && ms[i] != -INFINITY ? fast_exp2(ms[i] - mb) : 0.f;
+      lt += ls[i] * a;
+      at += as[i] * a;
+    }
+    mn = mb;
   }
   const float o = lt > 0.f ? at / lt : 0.f;     // a row that sees no key yields zeros
   if constexpr (sizeof(T) == 2) out[rh * kHeadDim + d] = f32_to_bf16(o);
   else out[rh * kHeadDim + d] = o;
 }
 
-template <typename T>
-int launch_attn(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
-                const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
-                int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st) {
+int launch_attn_f32(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
+                    const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
+                    int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st) {
   const int n_split = plan.n_split;
   const int G = Hq / Hkv;
   dim3 grid((unsigned)total_q, (unsigned)Hkv, (unsigned)n_split);
   const float sl2 = scale * 1.4426950408889634f;
-  // Wavefronts per workgroup: the VALU work grows with the group size, and one 8-wavefront workgroup per
-  // compute unit measured better for G >= 4 than two of 4 (61 vs 64 us on the decode shape).
 #define MSA_ATTN_CASE(GG, WW)                                                                                      \
   case GG:                                                                                                         \
-    attn_partial_kernel<T, GG, WW><<<grid, WW * 64, 0, st>>>(                                                      \
-        static_cast<const T*>(q), cu_q, static_cast<const T*>(k), static_cast<const T*>(v), kv_off, kv_len, B, Hq, \
-        Hkv, sl2, causal, n_split, 0, part_ml, part_acc, static_cast<T*>(out));                                                          \
+    attn_partial_kernel<GG, WW><<<grid, WW * 64, 0, st>>>(                                                         \
+        static_cast<const float*>(q), cu_q, static_cast<const float*>(k), static_cast<const float*>(v), kv_off,    \
+        kv_len, B, Hq, Hkv, sl2, causal, n_split, part_ml, part_acc, static_cast<float*>(out));                    \
     break;
   switch (G) {
     MSA_ATTN_CASE(1, 4)
@@ -513,8 +626,32 @@ int launch_attn(const void* q, const int32_t* cu_q, const void* k, const void* v
 #undef MSA_ATTN_CASE
   MSA_LAUNCH_CHECK();
   if (n_split == 1) return MSA_OK;
-  attn_combine_kernel<T><<<(unsigned)((int64_t)total_q * Hq), kHeadDim, 0, st>>>(part_ml, part_acc, n_split,
-                                                                                 static_cast<T*>(out));
+  attn_combine_kernel<float><<<(unsigned)((int64_t)total_q * Hq), kHeadDim, 0, st>>>(part_ml, part_acc, n_split,
+                                                                                     static_cast<float*>(out));
+  MSA_LAUNCH_CHECK();
+  return MSA_OK;
+}
+
+constexpr int kFusedLds = kRingLds + (int)sizeof(HeadSums) + kMaxG * 16 * (int)sizeof(uint4);
+static_assert(2 * kFusedLds <= 160 * 1024, "two workgroups a compute unit");
+
+int launch_attn_bf16(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
+                     const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
+                     int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st) {
+  const int n_split = plan.n_split, G = Hq / Hkv;
+  if (G != 1 && G != 2 && G != 4 && G != 8) {
+    msa_set_error("msa_sparse_attn: GQA group size %d unsupported (1, 2, 4, 8)", G);
+    return MSA_EINVAL;
+  }
+  static std::atomic<int> lds_limit_raised{0};
+  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(attn_ring_kernel), kRingLds));
+  attn_ring_kernel<<<dim3((unsigned)total_q, (unsigned)Hkv, (unsigned)n_split), kRingWaves * 64, kRingLds, st>>>(
+      static_cast<const bf16_t*>(q), cu_q, static_cast<const bf16_t*>(k), static_cast<const bf16_t*>(v), kv_off, kv_len, B, Hq, Hkv,
+      scale * 1.4426950408889634f, causal, n_split, part_ml, part_acc, static_cast<bf16_t*>(out));
+  MSA_LAUNCH_CHECK();
+  if (n_split == 1) return MSA_OK;
+  attn_combine_kernel<bf16_t><<<(unsigned)((int64_t)total_q * Hq), kHeadDim, 0, st>>>(part_ml, part_acc, n_split,
+                                                                                      static_cast<bf16_t*>(out));
   MSA_LAUNCH_CHECK();
   return MSA_OK;
 }
@@ -523,8 +660,8 @@ int launch_attn(const void* q, const int32_t* cu_q, const void* k, const void* v
 
 extern "C" size_t msa_attn_workspace_bytes(int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D, int32_t max_kv) {
   if (total_q <= 0 || Hq <= 0 || Hkv <= 0 || D <= 0 || max_kv <= 0) return 0;
-  // sized for whichever of the two kernels splits the keys further
-  const int splits = std::max(plan_splits(total_q, Hkv, max_kv).n_split, plan_splits_valu(total_q, Hkv, max_kv).n_split);
+  // sized for whichever of the kernels has more partials
+  const int splits = std::max(plan_splits(total_q, Hkv, max_kv).n_split, plan_splits_rows(total_q, Hkv, max_kv, MSA_BF16).n_split);
   const size_t n = (size_t)total_q * Hq * splits;
   return align_up(n * 2 * sizeof(float), 256) + align_up(n * D * sizeof(float), 256);
 }
@@ -545,7 +682,7 @@ extern "C" int msa_sparse_attn(const void* q, const int32_t* cu_q, const void* k
               "msa_sparse_attn: q, k, v and out must be 16-byte aligned");
   MSA_REQUIRE((int64_t)total_q * Hq < (int64_t)1 << 31 && total_q < 65536 * 32, "msa_sparse_attn: too many rows");
   const bool mfma = dtype == MSA_BF16 && max_sq >= 8;
-  const SplitPlan plan = mfma ? plan_splits(total_q, Hkv, max_kv) : plan_splits_valu(total_q, Hkv, max_kv);
+  const SplitPlan plan = mfma ? plan_splits(total_q, Hkv, max_kv) : plan_splits_rows(total_q, Hkv, max_kv, dtype);
   const int n_split = plan.n_split;
   MSA_REQUIRE(n_split <= 65535, "msa_sparse_attn: max_kv=%d too large", max_kv);
   const size_t need = msa_attn_workspace_bytes(total_q, Hq, Hkv, D, max_kv);
@@ -569,10 +706,10 @@ extern "C" int msa_sparse_attn(const void* q, const int32_t* cu_q, const void* k
     return MSA_OK;
   }
   if (dtype == MSA_BF16)
-    return launch_attn<bf16_t>(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml,
+    return launch_attn_bf16(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml,
                                part_acc, st);
-  return launch_attn<float>(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml,
-                            part_acc, st);
+  return launch_attn_f32(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml,
+                         part_acc, st);
 }
 
 extern "C" int msa_decode_attn_fused(const void* qkv, int64_t row_stride, const int64_t* positions, const void* q_norm_w,
@@ -589,26 +726,22 @@ extern "C" int msa_decode_attn_fused(const void* qkv, int64_t row_stride, const 
   MSA_REQUIRE((((uintptr_t)qkv | (uintptr_t)q_norm_w | (uintptr_t)k_norm_w | (uintptr_t)kcache | (uintptr_t)vcache) & 15) == 0,
               "msa_decode_attn_fused: pointers must be 16-byte aligned");
   MSA_REQUIRE(Lcap > 0 && rope_rows > 0 && eps > 0.f && scale > 0.f, "msa_decode_attn_fused: bad scalar argument");
-  const SplitPlan plan = plan_splits_valu(B, Hkv, Lcap);
-  const int n_split = plan.n_split;
   const size_t need = msa_attn_workspace_bytes(B, Hq, Hkv, D, Lcap);
   if (need > workspace_bytes) {
     msa_set_error("msa_decode_attn_fused: workspace of %zu bytes, need %zu", workspace_bytes, need);
     return MSA_ESIZE;
   }
+  const int n_split = plan_splits_rows(B, Hkv, Lcap, MSA_BF16).n_split;
   const size_t n = (size_t)B * Hq * n_split;
   float* part_ml = static_cast<float*>(workspace);
   float* part_acc = reinterpret_cast<float*>(static_cast<char*>(workspace) + align_up(n * 2 * sizeof(float), 256));
   hipStream_t st = as_stream(stream);
-  dim3 grid((unsigned)B, (unsigned)Hkv, (unsigned)n_split);
-  const float sl2 = scale * 1.4426950408889634f;
-#define MSA_FUSED_CASE(GG)                                                                                           \
-  attn_decode_fused_kernel<GG><<<grid, 8 * 64, 0, st>>>(                                                            \
-      static_cast<const bf16_t*>(qkv), row_stride, Hq, Hkv, positions, static_cast<const bf16_t*>(q_norm_w),         \
-      static_cast<const bf16_t*>(k_norm_w), eps, rope_cos, rope_sin, rope_rows, static_cast<bf16_t*>(kcache),        \
-      static_cast<bf16_t*>(vcache), Lcap, kv_len, sl2, n_split, part_ml, part_acc)
-  if (Hq / Hkv == 4) MSA_FUSED_CASE(4); else MSA_FUSED_CASE(8);
-#undef MSA_FUSED_CASE
+  static std::atomic<int> lds_limit_raised{0};
+  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(attn_decode_fused_kernel), kFusedLds));
+  attn_decode_fused_kernel<<<dim3((unsigned)B, (unsigned)Hkv, (unsigned)n_split), kRingWaves * 64, kFusedLds, st>>>(
+      static_cast<const bf16_t*>(qkv), row_stride, Hq, Hkv, positions, static_cast<const bf16_t*>(q_norm_w),
+      static_cast<const bf16_t*>(k_norm_w), eps, rope_cos, rope_sin, rope_rows, static_cast<bf16_t*>(kcache),
+      static_cast<bf16_t*>(vcache), Lcap, kv_len, scale * 1.4426950408889634f, n_split, part_ml, part_acc);
   MSA_LAUNCH_CHECK();
   attn_combine_kernel<bf16_t><<<(unsigned)((int64_t)B * Hq), kHeadDim, 0, st>>>(part_ml, part_acc, n_split,
                                                                                 static_cast<bf16_t*>(out), kv_len, Lcap, Hq);

@@ -1,4 +1,4 @@
-// Shared between attn.hip (split-KV VALU kernel, combine) and flash_attn.hip (MFMA kernels).
+// Shared between attn.hip (single rows, combine) and flash_attn.hip (MFMA kernels).
 #pragma once
 #include <algorithm>
 
@@ -25,10 +25,10 @@ static inline SplitPlan plan_splits_for(int64_t total_q, int32_t Hkv, int32_t ma
 static inline SplitPlan plan_splits(int64_t total_q, int32_t Hkv, int32_t max_kv) {
   return plan_splits_for(total_q, Hkv, max_kv, 1024);
 }
-// VALU split kernel (decode): one workgroup per compute unit measured best (fewer, longer key streams); the
-// kernel itself divides each sample's own length evenly over n_split.
-static inline SplitPlan plan_splits_valu(int64_t total_q, int32_t Hkv, int32_t max_kv) {
-  return plan_splits_for(total_q, Hkv, max_kv, 256);
+// Single rows (decode): fp32 one workgroup per compute unit (fewer, longer key streams), bf16 the two whose rings fit (one sample
+// of 4388 keys 11.9 us, 17.5 as one per unit); the kernels divide each sample's own length evenly over n_split.
+static inline SplitPlan plan_splits_rows(int64_t total_q, int32_t Hkv, int32_t max_kv, int32_t dtype) {
+  return plan_splits_for(total_q, Hkv, max_kv, dtype == MSA_BF16 ? 512 : 256);
 }
 
 // flash_attn.hip: bf16 partial pass over split `blockIdx.z` of the keys; writes un-normalised

@@ -85,3 +85,28 @@ def test_single_pass_decode_attention(dtype, L):
         p = torch.softmax((q[b].double()[None] * kk).sum(-1) * 128 ** -0.5, dim=0)
         want = (p[..., None] * vv).sum(0)
         assert (out[b] - want).abs().max() <= (1e-5 if dtype == torch.float32 else 1e-2) * want.abs().max()
+
+
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+def test_decode_attention_through_the_ring(G):
+    """bf16 rows at the edges of a step's 32 keys, a round of four steps and a split, cut out of one block of keys, whose other rows
+    are NaN.  Bound: the output's rounding (half a unit of eight bits, 2^-8 of it) and the weights' (two bf16 parts, 2^-16 of the sum
+    of |p v|, twice for the fp32 sums; one part, 2^-8 of it, for the sample with an infinite value)."""
+    from msa_amd import ops
+    lens = [1, 31, 32, 33, 127, 128, 129, 0, 255, 257, 1030, 2100]
+    g = torch.Generator().manual_seed(G)
+    q = (2 * torch.randn((len(lens), 2 * G, 128), generator=g)).bfloat16()
+    off = [2 * b + sum(lens[:b]) for b in range(len(lens))]
+    k, v = (torch.full((off[-1] + lens[-1] + 2, 2, 128), float("nan"), dtype=torch.bfloat16) for _ in range(2))
+    for o, n in zip(off, lens):
+        k[o:o + n], v[o:o + n] = (torch.randn((n, 2, 128), generator=g).bfloat16() for _ in range(2))
+    v[off[4] + 100, 0, 5] = float("inf")
+    out = ops.sparse_attn(q.cuda(), k.cuda(), v.cuda(), torch.tensor(off).cuda(), torch.tensor(lens, dtype=torch.int32).cuda(), max(lens)).cpu().double()
+    for b, (o, n) in enumerate(zip(off, lens)):
+        kk, vv = (t[o:o + n].double().repeat_interleave(G, dim=1) for t in (k, v))
+        p = torch.softmax((q[b].double()[None] * kk).sum(-1) * 128 ** -0.5, dim=0)
+        want = (p[..., None] * vv).sum(0)
+        fin = torch.isfinite(want)
+        assert torch.equal(out[b][~fin], want[~fin])
+        bound = want.abs() * 2 ** -8 + (p[..., None] * vv.abs()).sum(0) * (2 ** -8 if b == 4 else 2 ** -15)
+        assert ((out[b] - want).abs() <= bound)[fin].all()
