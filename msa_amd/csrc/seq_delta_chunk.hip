@@ -10,7 +10,8 @@
 //   (2) StateWalk      a workgroup per (sequence, head, 16 or 32 value columns) walks over the chunks: U, o and S
 //   (3) msa_seq_head_norm_gate
 // (1) is bound by memory and arithmetic, (2) by the latency of its chain, so they share launches: one launch prepares a segment of
-// chunks while it walks over the segment before.  Segments also bound the workspace (two of them).
+// chunks while it walks over the segment before.  Segments also bound the workspace (two of them), though not so far that a launch
+// is short: one costs some 20 us beyond its chunks (states, first loads, walks that fill the chip in front of the preparation).
 //
 // Decays differ by channel, so L and A are products of operands that carry them: within blocks of 16 tokens everything is
 // relative to the block's start (rows, exponents <= 0) and its end (columns, exponents <= 0), and whole blocks' decays between
@@ -786,7 +787,10 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(ChunkArgs walk, Chu
   }
 }
 
-constexpr int64_t kMaxSegment = (int64_t)88 << 20;        // bytes: two segments stay in the memory-side cache
+// Bytes: 22 chunks of four sequences of 32 heads of 128 x 128.  (88 MB, of which two lie in the memory-side cache, is worth less than
+// long launches: 6001 tokens of five sequences take 470 us a layer then, 320 so, 357 with 176 MB, 322 with 704; one sequence of 8192
+// 410 either way.)
+constexpr int64_t kMaxSegment = (int64_t)352 << 20;
 constexpr int kSegments = 6, kLeastChunks = 22;           // segments of a long portion, chunks that are worth a launch
 
 int64_t unit_bytes(int32_t D, int32_t E) {
