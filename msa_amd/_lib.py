@@ -192,7 +192,7 @@ def load() -> C.CDLL:
 
 def load_seq() -> C.CDLL:
     """The same for the library of the recurrent / latent-attention layers."""
-    return _open(SEQ_LIB_PATH, {**SEQ_SIGNATURES, **{n: SIGNATURES[n] for n in SEQ_SHARED}})
+    return _libs.get(SEQ_LIB_PATH) or _open(SEQ_LIB_PATH, {**SEQ_SIGNATURES, **{n: SIGNATURES[n] for n in SEQ_SHARED}})
 
 
 def check(code: int, where: str, lib: Optional[C.CDLL] = None) -> None:

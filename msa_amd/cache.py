@@ -158,10 +158,10 @@ class SequenceStateCache:
         if not self._free:
             self._resize(2 * self.slots, self.capacity)
         slot = self._free.pop(0)
-        for spec, held in zip(self.specs, self.tensors):
-            for name, s in spec.items():
-                if not s.per_token:
-                    held[name][slot].zero_()
+        # in one launch: a model's six to thirty states took 4 us each, several times what clearing them costs
+        fixed = [held[name][slot] for spec, held in zip(self.specs, self.tensors) for name, s in spec.items() if not s.per_token]
+        if fixed:
+            torch._foreach_zero_(fixed)
         self.slot_of[key], self.length[key] = slot, 0
         return slot
 

@@ -19,7 +19,8 @@ MODES = {"cosine": MODE_COSINE, "scaled_dot": MODE_SCALED_DOT}
 
 
 def _stream(stream: Optional[torch.cuda.Stream] = None) -> int:
-    return (stream or torch.cuda.current_stream()).cuda_stream
+    # (current_stream() takes 9 us a call)
+    return stream.cuda_stream if stream is not None else torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _need_cuda(*ts):

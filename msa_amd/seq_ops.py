@@ -6,6 +6,7 @@ import ctypes as C
 from dataclasses import dataclass
 from typing import Optional, Sequence
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -20,7 +21,7 @@ def _check(code: int, where: str) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())     # (current_stream() takes 9 us a call)
 
 
 def _cuda(*ts):
@@ -50,11 +51,30 @@ def _f32(n: int, *ts):
             raise ValueError(f"expected {n} contiguous fp32 values on the device, got {t.dtype} {tuple(t.shape)}")
 
 
+def upload(device, arrays) -> list:
+    """Host arrays (int32 or int64) on the device, in one copy that nothing waits for: out of pinned memory, which the allocator
+    gives out again only once the copy has ended.  (From pageable memory every array is a copy of its own, behind which the host
+    waits for all work in front of it.)"""
+    device = torch.device(device)
+    places, words = [], 0
+    for a in arrays:
+        places.append(words)
+        words += (a.nbytes + 7) // 8
+    host = torch.empty(words, dtype=torch.int64, pin_memory=device.type == "cuda")
+    to = host.numpy()
+    for a, at in zip(arrays, places):
+        to[at:at + (a.nbytes + 7) // 8].view(a.dtype)[:len(a)] = a
+    dev = host.to(device, non_blocking=True)
+    return [dev[at:at + (a.nbytes + 7) // 8].view(torch.int32 if a.dtype == np.int32 else torch.int64)[:len(a)]
+            for a, at in zip(arrays, places)]
+
+
 class StepBatch:
     """Device-side description of a step's rows (``msa_seq_batch``): ``counts[s]`` new tokens of the sequence in
-    ``slots[s]`` that has already been fed ``positions[s]`` tokens."""
+    ``slots[s]`` that has already been fed ``positions[s]`` tokens.  ``extra`` int64 arrays go to the device with it
+    (``self.extra``)."""
 
-    def __init__(self, counts: Sequence[int], slots: Sequence[int], positions: Sequence[int], device):
+    def __init__(self, counts: Sequence[int], slots: Sequence[int], positions: Sequence[int], device, extra=()):
         n = len(counts)
         if not n or min(counts) < 1 or len(set(slots)) != n:
             raise ValueError("a step needs at least one token per sequence and one slot each")
@@ -63,12 +83,11 @@ class StepBatch:
         host = [0]
         for c in counts:
             host.append(host[-1] + c)
-        cu = list(host)
-        ints = torch.tensor(cu + list(slots), dtype=torch.int32).to(device)
-        self.cu, self.slot = ints[:n + 1], ints[n + 1:]
-        self.pos = torch.tensor(list(positions), dtype=torch.int64).to(device)
-        self.row_seq = (torch.zeros(self.rows, dtype=torch.int32, device=device) if n == 1 else
-                        torch.repeat_interleave(torch.arange(n, dtype=torch.int32), torch.tensor(self.counts)).to(device))
+        many = [] if n == 1 else [np.repeat(np.arange(n, dtype=np.int32), self.counts)]
+        self.cu, self.slot, self.pos, *rest = upload(device, [np.asarray(host, np.int32), np.asarray(self.slots, np.int32),
+                                                              np.asarray(self.positions, np.int64), *many, *extra])
+        self.row_seq = rest.pop(0) if many else torch.zeros(self.rows, dtype=torch.int32, device=device)
+        self.extra = rest
         self.c = _lib.SeqBatch(ptr(self.cu), ptr(self.row_seq), ptr(self.slot), ptr(self.pos), n, self.rows, self.max_rows, 0)
         self.ref = C.byref(self.c)
         self.max_keys = max(p + c for p, c in zip(positions, counts))     # longest sequence at the end of the step

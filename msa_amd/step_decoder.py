@@ -10,6 +10,7 @@ from __future__ import annotations
 
 from typing import Dict, Hashable, List, Optional, Sequence, Tuple, Union
 
+import numpy as np
 import torch
 import torch.nn.functional as F
 
@@ -128,23 +129,21 @@ class StepDecoder:
         for key, _, _ in entries:
             if key not in cache.slot_of:
                 cache.open(key)
-        counts = [len(t) for _, t, _ in entries]
-        batch = seq_ops.StepBatch(counts, [cache.slot_of[k] for k, _, _ in entries], [cache.length[k] for k, _, _ in entries],
-                                  self.device)
-        tokens = torch.cat([t for _, t, _ in entries]).to(self.device)
-        rows, at = [], 0
+        counts, rows, at = [len(t) for _, t, _ in entries], [], 0
         for (_, ts, want) in entries:
             rows += [at + w for w in want]
             at += len(ts)
-        logits = self.forward_rows(tokens, batch, cache, rows)
+        batch = seq_ops.StepBatch(counts, [cache.slot_of[k] for k, _, _ in entries], [cache.length[k] for k, _, _ in entries],
+                                  self.device, (np.concatenate([t.numpy() for _, t, _ in entries]), np.asarray(rows, np.int64)))
+        logits = self.forward_rows(batch.extra[0], batch, cache, rows, index=batch.extra[1])
         for key, ts, _ in entries:
             cache.advance(key, len(ts))
         return logits
 
     def forward_rows(self, tokens: torch.Tensor, batch: seq_ops.StepBatch, cache: SequenceStateCache, rows: List[int],
-                     trace: Optional[list] = None) -> Optional[torch.Tensor]:
+                     trace: Optional[list] = None, index: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
         """Logits of ``rows`` of a step whose states are reserved.  ``trace`` (a list) receives a copy of the residual stream
-        after every layer run."""
+        after every layer run.  ``index``: ``rows`` on the device (they are copied there if it is missing)."""
         if self.fused_decode and batch.max_rows == 1 and batch.rows <= seq_ops.MAX_ROWS:
             h = self._decode_rows(tokens, batch, cache, trace)
         else:
@@ -152,7 +151,7 @@ class StepDecoder:
         if not rows:
             return None
         if rows != list(range(batch.rows)):
-            h = h[rows[0]:rows[0] + 1] if len(rows) == 1 else h[torch.tensor(rows, device=h.device)]
+            h = h[rows[0]:rows[0] + 1] if len(rows) == 1 else h[torch.tensor(rows, device=h.device) if index is None else index]
         cap = getattr(self.config, "logit_softcap", None) or 0.0
         if self.fused_decode and len(rows) <= seq_ops.MAX_ROWS:
             return seq_ops.rows_linear_f32(h, self.head, cap)
