@@ -253,6 +253,19 @@ typedef struct {
 } msa_rows_args;
 int msa_rows_linear(const msa_rows_args* args, int32_t epilogue, void* stream);
 
+/* The same with msa_seq_rms_residual in front: args->x holds y, x_out = x_in + rms_norm(y) * w (fp32 [M, K]) and the product's
+ * operand is x_out in bf16.  Formed on the way for few rows where x_out is not x_in and the epilogue is PLAIN, MAMBA or GLU,
+ * otherwise in a launch of its own through `h` (bf16 [M, K], whose contents are undefined afterwards).  One operand, groups = 1. */
+typedef struct {
+  const float* x_in;
+  float* x_out;
+  const float* w;
+  void* h;
+  float eps;
+  int32_t reserved;
+} msa_rows_post;
+int msa_rows_linear_post(const msa_rows_args* args, int32_t epilogue, const msa_rows_post* post, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

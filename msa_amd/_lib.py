@@ -101,6 +101,11 @@ class RowsArgs(C.Structure):
                 ("slot", _vp), ("glu_limit", _f32), ("glu_alpha", _f32), ("glu_shift", _f32), ("reserved4", _i32)]
 
 
+class RowsPost(C.Structure):
+    """``msa_rows_post``."""
+    _fields_ = [("x_in", _vp), ("x_out", _vp), ("w", _vp), ("h", _vp), ("eps", _f32), ("reserved", _i32)]
+
+
 class QKRopeArgs(C.Structure):
     """``msa_qk_rope_args``."""
     _fields_ = [("q", _vp), ("k", _vp), ("v", _vp), ("q_stride", _i64), ("k_stride", _i64), ("v_stride", _i64), ("q_norm", _vp),
@@ -157,6 +162,7 @@ SEQ_SIGNATURES = {
     "msa_seq_rms_residual": (C.c_int, [_vp, _vp, _i64, _vp, _f32, _vp, _vp, _vp, _i32, _i32, _i32, _vp]),
     "msa_seq_clamped_glu": (C.c_int, [_vp, _i64, _i32, _i32, _i32, _f32, _f32, _f32, _vp, _vp]),
     "msa_rows_linear": (C.c_int, [C.POINTER(RowsArgs), _i32, _vp]),
+    "msa_rows_linear_post": (C.c_int, [C.POINTER(RowsArgs), _i32, C.POINTER(RowsPost), _vp]),
 }
 # entry points of include/msa_amd.h that libmsa_seq.so holds too (the error text is per library)
 SEQ_SHARED = ("msa_last_error", "msa_abi_version", "msa_greedy_sample")

@@ -227,8 +227,8 @@ int launch_ring(const void* x, const void* w, const void* residual, const void* 
   r.eps = eps;
   const typename RingEnd<kEpi>::Args s{static_cast<const bf16_t*>(residual), static_cast<bf16_t*>(y), kEpi == kEpiSiluMul ? N / 2 : N};
   const int granule = kEpi == kEpiSiluMul ? 16 : 1;
-  return norm_w ? rows_ring::launch<RingEnd<kEpi>, true>(r, s, granule, st)
-                : rows_ring::launch<RingEnd<kEpi>, false>(r, s, granule, st);
+  return norm_w ? rows_ring::launch<RingEnd<kEpi>, rows_ring::kNormed>(r, s, granule, st)
+                : rows_ring::launch<RingEnd<kEpi>>(r, s, granule, st);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -40,8 +40,15 @@ constexpr int kMinK = 512, kMinRows = 4;
 constexpr int64_t kMinWeights = 3 << 19;
 constexpr int kFar = 0x7ff00000;                   // past every extent, whatever is added: reads zeros, touches no memory
 // slots of a wavefront's ring
-constexpr int slots(bool norm) { return norm ? 3 : 2; }
-constexpr int lds_bytes(bool norm) { return 2 * kWaves * kPlane * 4 + kWaves * slots(norm) * kUnitSlab + (norm ? kWaves * 16 * 4 : 0); }
+// What happens to the activations in front of the products: nothing, an RMSNorm, or a residual step with the norm of its own (one
+// launch less, but all workgroups read its fp32 operands: seq_rows.hip has the line).
+enum { kPlain, kNormed, kPost };
+constexpr int kMaxPost = 3;                        // units per wavefront that the residual step takes: what its registers hold
+constexpr int slots(int pro) { return pro ? 3 : 2; }
+constexpr int lds_bytes(int pro) {
+  return 2 * kWaves * kPlane * 4 + kWaves * slots(pro) * kUnitSlab + (pro ? kWaves * 16 * 4 : 0) + (pro == kPost ? kWaves * 1024 : 0);
+}
+static_assert(kMaxPost * 2 * kUnitBytes <= 1024, "one request for a wavefront's part of the residual step's weights");
 constexpr int kNonTemporal = 2;                    // a step reads a weight once
 
 // vmcnt(n), the other counters not waited for
@@ -53,8 +60,17 @@ __device__ __forceinline__ float quad_xor(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kPerm, 0xf, 0xf, false));
 }
 
+__device__ __forceinline__ uint32_t lds_offset(const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
+__device__ __forceinline__ u32x4_t lds_read16(uint32_t at) {
+  u32x4_t v;
+  asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(at) : "memory");
+  return v;
+}
+
 struct Args {
   const char *w, *x, *x_b, *norm_w;
+  const float *post_x, *post_w;                    // kPost: the operand is post_x + rms_norm(x) * post_w, which one workgroup
+  float* post_out;                                 // leaves in post_out (rows of K)
   int64_t xs, xbs;                                 // bytes between activation rows
   int32_t M, N, n_b, row_bytes;                    // weight rows from n_b on multiply x_b
   int32_t wgs_a, granule, qa, ra, qb, rb;  // workgroup i < wgs_a: its share of the granules of the rows before n_b
@@ -65,10 +81,10 @@ struct Args {
 // item's products, `apply(s, m, n, v, mine, second, item)` behind them, in every lane: four neighbouring lanes hold output
 // (m, n), neighbouring columns are four lanes apart, `mine` in the first lane of each output that exists.  `load` must not wait
 // for what it requests: loads return in order, so that would wait for the weights in front of it.
-template <class Epi, int NU, bool kNorm>
+template <class Epi, int NU, int kPro>
 __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename Epi::Args s) {
-  constexpr bool kResident = NU > 0;
-  constexpr int kSlots = slots(kNorm);
+  constexpr bool kResident = NU > 0, kNorm = kPro == kNormed;
+  constexpr int kSlots = slots(kPro);
   extern __shared__ __align__(16) char lds[];
   float(*part)[kWaves][kPlane] = reinterpret_cast<float(*)[kWaves][kPlane]>(lds);
   float* row_ssq = reinterpret_cast<float*>(lds + 2 * kWaves * kPlane * 4 + kWaves * kSlots * kUnitSlab);
@@ -153,7 +169,24 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
         gw[u][h] = __builtin_amdgcn_raw_buffer_load_b128(rs_g, x_col + so < row_bytes ? x_col : kFar, so, 0);
       }
   }
-  epi.load(s, m, r0 + nr, quarter == 0 && m < a.M && r0 + nr < r1, second, 0);
+  // The residual step's other operands: the fp32 rows into registers, the weights, alike for all rows, through LDS
+  u32x4_t px[kPro == kPost ? NU : 1][2][2];
+  char* post_lds = lds + lds_bytes(kNormed) + wave * 1024;
+  if constexpr (kPro == kPost) {
+    const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.post_w), 0, 2 * row_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs_p = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.post_x), 0, a.M * 2 * row_bytes, 0x00020000);
+    MSA_LOAD_TO_LDS(rs_w, post_lds, (lane >> 4) * (2 * kUnitBytes * kWaves) + wave * 2 * kUnitBytes + (lane & 15) * 16, 0, 0);
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int so = u * (kUnitBytes * kWaves) + h * 64, at = x_col + so < row_bytes ? n_l * 2 * row_bytes + 2 * x_col : kFar;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) px[u][h][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_p, at + 16 * i, 2 * so, 0);
+      }
+  }
+  constexpr bool kLate = kPro == kPost && NU == kMaxPost;    // (no registers for it in front of the residual step)
+  if (!kLate) epi.load(s, m, r0 + nr, quarter == 0 && m < a.M && r0 + nr < r1, second, 0);
   asm volatile("" ::: "memory");                             // (not to be sunk behind the requests)
   point();
 #pragma unroll
@@ -183,6 +216,54 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
     ssq += __shfl_xor(ssq, 32);
     if (g == 0) row_ssq[wave * 16 + n_l] = ssq;              // read behind the first barrier
   }
+  if constexpr (kPro == kPost) {
+    // x + rms_norm(y) * w as the operand, the sums as in the launch of its own.  (LDS by hand: the compiler would wait for the ring
+    // in front of it.  The weights have arrived with what was requested behind them.)
+    float ssq = 0.f;
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float lo = bf16lo(xf[u][h][c]), hi = bf16hi(xf[u][h][c]);
+          ssq += lo * lo + hi * hi;
+        }
+    ssq += __shfl_xor(ssq, 16);
+    ssq += __shfl_xor(ssq, 32);
+    const uint32_t row_at = lds_offset(row_ssq + n_l * 16);
+    asm volatile("ds_write_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::"v"(row_at + 4 * wave), "v"(ssq) : "memory");
+    float total = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const u32x4_t p = lds_read16(row_at + 16 * i);
+      total += (__uint_as_float(p[0]) + __uint_as_float(p[1])) + (__uint_as_float(p[2]) + __uint_as_float(p[3]));
+    }
+    const float post_inv = 1.0f / sqrtf(total / (float)(row_bytes / 2) + a.eps);
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int so = u * (kUnitBytes * kWaves) + h * 64;
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const u32x4_t w = lds_read16(lds_offset(post_lds) + u * 2 * kUnitBytes + h * 128 + g * 32 + i * 16);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const uint32_t y = xf[u][h][2 * i + (c >> 1)];
+            v[4 * i + c] = __uint_as_float(px[u][h][i][c]) + (c & 1 ? bf16hi(y) : bf16lo(y)) * post_inv * __uint_as_float(w[c]);
+          }
+        }
+        if (wg == 0 && n_l < a.M && x_col + so < row_bytes) {
+          float4* to = reinterpret_cast<float4*>(a.post_out + (int64_t)n_l * (row_bytes / 2) + (x_col + so) / 2);
+          to[0] = make_float4(v[0], v[1], v[2], v[3]);
+          to[1] = make_float4(v[4], v[5], v[6], v[7]);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) xf[u][h][c] = pack_bf16x2(v[2 * c], v[2 * c + 1]);
+      }
+  }
 
   float inv = 1.f;
   if constexpr (kResident) {
@@ -197,7 +278,7 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
     auto round = [&](u32x4_t (&x)[2], int next, bool wraps, bool first) {
       __builtin_amdgcn_s_waitcnt(wait_vm((kResident ? 2 : 4) * (kSlots - 1)));
       asm volatile("" ::: "memory");
-      if (first && item > 0) epi.load(s, m, n, mine, second, item);
+      if (first && (kLate || item > 0)) epi.load(s, m, n, mine, second, item);
       acc = multiply(x, acc);
       if (wraps) {
         ++req_item;
@@ -257,29 +338,31 @@ static inline int plan(Args& a, int granule) {
   return wa + wb;
 }
 
-template <class Epi, int NU, bool kNorm>
+template <class Epi, int NU, int kPro>
 int start(const Args& a, const typename Epi::Args& s, int wgs, hipStream_t st) {
   static std::atomic<int> lds_limit_raised{0};
-  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(rows_ring_kernel<Epi, NU, kNorm>), lds_bytes(kNorm)));
-  rows_ring_kernel<Epi, NU, kNorm><<<wgs, kWaves * 64, lds_bytes(kNorm), st>>>(a, s);
+  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(rows_ring_kernel<Epi, NU, kPro>), lds_bytes(kPro)));
+  rows_ring_kernel<Epi, NU, kPro><<<wgs, kWaves * 64, lds_bytes(kPro), st>>>(a, s);
   MSA_LAUNCH_CHECK();
   return MSA_OK;
 }
 
-template <class Epi, bool kNorm = false>
+template <class Epi, int kPro = kPlain>
 int launch(Args a, const typename Epi::Args& s, int granule, hipStream_t st) {
   const int wgs = plan(a, granule);
   const int units = (a.row_bytes + kUnitBytes * kWaves - 1) / (kUnitBytes * kWaves);
-  if (units <= 1) return start<Epi, 1, kNorm>(a, s, wgs, st);
-  if (units <= 2) return start<Epi, 2, kNorm>(a, s, wgs, st);
-  if (units <= 3) return start<Epi, 3, kNorm>(a, s, wgs, st);
-  if (units <= 4) return start<Epi, 4, kNorm>(a, s, wgs, st);
-  if (units <= kMaxResident) return start<Epi, kMaxResident, kNorm>(a, s, wgs, st);
-  if constexpr (kNorm) {
-    msa_set_error("rows_ring: a folded norm takes rows of at most %d bytes, not %d", kMaxResident * kUnitBytes * kWaves, a.row_bytes);
+  if (units <= 1) return start<Epi, 1, kPro>(a, s, wgs, st);
+  if (units <= 2) return start<Epi, 2, kPro>(a, s, wgs, st);
+  if (units <= 3) return start<Epi, 3, kPro>(a, s, wgs, st);
+  if constexpr (kPro != kPost) {
+    if (units <= 4) return start<Epi, 4, kPro>(a, s, wgs, st);
+    if (units <= kMaxResident) return start<Epi, kMaxResident, kPro>(a, s, wgs, st);
+  }
+  if constexpr (kPro != kPlain) {
+    msa_set_error("rows_ring: a folded norm takes rows of at most %d bytes, not %d", (kPro == kPost ? kMaxPost : kMaxResident) * kUnitBytes * kWaves, a.row_bytes);
     return MSA_EINVAL;
   } else {
-    return start<Epi, 0, false>(a, s, wgs, st);
+    return start<Epi, 0, kPlain>(a, s, wgs, st);
   }
 }
 

@@ -289,9 +289,20 @@ struct RingEnd<MSA_ROWS_GRU> {
   }
 };
 
-template <int EPI>
-int launch_ring(const msa_rows_args& a, hipStream_t st) {
+// The weight ring's part of the calls (see kMinWeights).
+bool takes_ring(const msa_rows_args& a, int32_t epilogue) {
+  return a.groups == 1 && a.K > rows_ring::kMinK && (int64_t)a.N * a.K >= (epilogue == MSA_ROWS_GRU ? kGruRingWeights : rows_ring::kMinWeights);
+}
+
+template <int EPI, int kPro = rows_ring::kPlain>
+int launch_ring(const msa_rows_args& a, hipStream_t st, const msa_rows_post* post = nullptr) {
   rows_ring::Args r{};
+  if (post) {
+    r.post_x = post->x_in;
+    r.post_w = post->w;
+    r.post_out = post->x_out;
+    r.eps = post->eps;
+  }
   r.w = static_cast<const char*>(a.w);
   r.x = static_cast<const char*>(a.x);
   r.x_b = static_cast<const char*>(a.x_b);
@@ -301,7 +312,7 @@ int launch_ring(const msa_rows_args& a, hipStream_t st) {
   r.N = a.N;
   r.n_b = a.n_b;
   r.row_bytes = a.K * 2;
-  return rows_ring::launch<RingEnd<EPI>>(r, a, EPI == MSA_ROWS_GRU ? 3 * kGruGroup : EPI == MSA_ROWS_GLU ? 2 : 1, st);
+  return rows_ring::launch<RingEnd<EPI>, kPro>(r, a, EPI == MSA_ROWS_GRU ? 3 * kGruGroup : EPI == MSA_ROWS_GLU ? 2 : 1, st);
 }
 
 template <int EPI, int R>
@@ -314,9 +325,8 @@ int launch_rows(const msa_rows_args& a, int waves, int rows_per_wg, hipStream_t 
 
 }  // namespace
 
-extern "C" int msa_rows_linear(const msa_rows_args* args, int32_t epilogue, void* stream) {
-  MSA_REQUIRE(args != nullptr, "msa_rows_linear: null arguments");
-  msa_rows_args a = *args;
+namespace {
+int rows_entry(const msa_rows_args& a, int32_t epilogue, const msa_rows_post* post, void* stream) {
   MSA_REQUIRE(a.x && a.w && a.M > 0 && a.M <= 16 && a.N > 0 && a.K > 0 && a.K % 8 == 0 && a.groups > 0 && a.groups <= 65535,
               "msa_rows_linear: M=%d (1..16) N=%d K=%d (a multiple of 8) groups=%d", a.M, a.N, a.K, a.groups);
   MSA_REQUIRE(a.x_stride >= (int64_t)a.K * a.groups && a.x_stride % 8 == 0 && a.x_stride * 32 < ((int64_t)1 << 30) &&
@@ -368,7 +378,14 @@ extern "C" int msa_rows_linear(const msa_rows_args* args, int32_t epilogue, void
   for (int cand = waves; cand >= std::max(1, waves / 2); --cand)
     if (units % cand == 0) { waves = cand; break; }
   hipStream_t st = as_stream(stream);
-  if (a.groups == 1 && a.K > rows_ring::kMinK && !(gru && (int64_t)a.N * a.K < kGruRingWeights) && (int64_t)a.N * a.K >= rows_ring::kMinWeights) {
+  if (takes_ring(a, epilogue)) {
+    if (post) {
+      switch (epilogue) {
+        case MSA_ROWS_PLAIN: return launch_ring<MSA_ROWS_PLAIN, rows_ring::kPost>(a, st, post);
+        case MSA_ROWS_MAMBA: return launch_ring<MSA_ROWS_MAMBA, rows_ring::kPost>(a, st, post);
+        case MSA_ROWS_GLU: return launch_ring<MSA_ROWS_GLU, rows_ring::kPost>(a, st, post);
+      }
+    }
     switch (epilogue) {
       case MSA_ROWS_PLAIN: return launch_ring<MSA_ROWS_PLAIN>(a, st);
       case MSA_ROWS_F32: return launch_ring<MSA_ROWS_F32>(a, st);
@@ -393,4 +410,31 @@ extern "C" int msa_rows_linear(const msa_rows_args* args, int32_t epilogue, void
   }
   msa_set_error("msa_rows_linear: no kernel for epilogue %d with %d row groups", epilogue, R);
   return MSA_EINVAL;
+}
+}  // namespace
+
+extern "C" int msa_rows_linear(const msa_rows_args* args, int32_t epilogue, void* stream) {
+  MSA_REQUIRE(args != nullptr, "msa_rows_linear: null arguments");
+  return rows_entry(*args, epilogue, nullptr, stream);
+}
+
+// The residual step is folded where its operands are few: every workgroup reads all of them, six bytes an element where the product
+// alone reads two.  Up to 8192 elements that is worth less than a launch (with the product, us, folded against separate: 1 row of
+// 1024 7.6 / 8.4 and 6.8 / 7.7, 8 rows 7.9 / 8.6 and 7.5 / 7.9, 4 of 2048 11.2 / 11.1, 2 of 2560 21.6 / 22.0 and 11.5 / 12.1), beyond
+// it is not (4 of 2560 12.5 / 12.3, 16 of 1024 9.1 / 8.9, 16 of 2560 28.0 / 22.7).  The separate launch also works in place and takes
+// rows that the ring's registers do not hold.
+constexpr int kMaxPostElements = 8192;
+extern "C" int msa_rows_linear_post(const msa_rows_args* args, int32_t epilogue, const msa_rows_post* post, void* stream) {
+  MSA_REQUIRE(args && post && post->x_in && post->x_out && post->w && post->h && post->eps >= 0.f, "msa_rows_linear_post: null arguments");
+  msa_rows_args a = *args;
+  MSA_REQUIRE(a.x && a.M > 0 && a.M <= 16 && a.K > 0 && a.groups == 1 && a.x_stride >= a.K && a.n_b >= a.N,
+              "msa_rows_linear_post: M=%d (1..16) K=%d groups=%d n_b=%d", a.M, a.K, a.groups, a.n_b);
+  const bool folds = (epilogue == MSA_ROWS_PLAIN || epilogue == MSA_ROWS_MAMBA || epilogue == MSA_ROWS_GLU) && takes_ring(a, epilogue) && a.M * (int64_t)a.K <= kMaxPostElements && a.K % 8 == 0 &&
+                     a.K <= rows_ring::kMaxPost * rows_ring::kWaves * rows_ring::kUnitBytes / 2 && post->x_in != post->x_out &&
+                     (((uintptr_t)post->x_in | (uintptr_t)post->x_out | (uintptr_t)post->w) & 15) == 0;
+  if (folds) return rows_entry(a, epilogue, post, stream);
+  if (const int rc = msa_seq_rms_residual(post->x_in, a.x, a.x_stride, post->w, post->eps, post->x_out, nullptr, post->h, MSA_BF16, a.M, a.K, stream); rc != MSA_OK) return rc;
+  a.x = post->h;
+  a.x_stride = a.K;
+  return rows_entry(a, epilogue, nullptr, stream);
 }

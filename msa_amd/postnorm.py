@@ -2,9 +2,8 @@
 clamped gated feed-forwards: the Sugizen architecture.
 
 The residual stream is fp32 and is itself (in the activations' type) what every sublayer reads.  Behind an output projection
-stands one fused step, residual + norm + the next operand (``seq_ops.rms_residual``); it needs a row's statistics, so that also
-when decoding it is a launch of its own.  The decode form folds the convolution into the mixer's input projection and the gated
-unit into the feed-forward's.
+stands one fused step, residual + norm + the next operand (``seq_ops.rms_residual``).  The decode form folds it into the product
+that reads it (``seq_ops.PostRows``), the convolution into the mixer's input projection and the gated unit into the feed-forward's.
 """
 from __future__ import annotations
 
@@ -32,7 +31,10 @@ class PostNormForCausalLM(StepDecoder):
         return seq_ops.rms_residual(x, self.dtype, y, w, self.config.norm_eps, self.final_norm if last else None, out=x)
 
     def _start(self, tokens):
-        x = self._embed(tokens)
+        e = self.embed[tokens]
+        x = e.to(F32)
+        if self.layers and e.dtype == self.dtype != F32:     # (the stream in the activations' type is the row itself)
+            return x, e
         _, h = seq_ops.rms_residual(x, self.dtype, eps=self.config.norm_eps, next_w=None if self.layers else self.final_norm)
         return x, h
 
@@ -55,6 +57,19 @@ class PostNormForCausalLM(StepDecoder):
 
     def _decode_rows(self, tokens, batch, cache, trace=None):
         """One token for each of up to 16 sequences (bf16)."""
-        return self._layers(tokens, trace,
-                            lambda r, l, h: l.mixer.decode(l.mixer.w_in, h, None, self.run_state(cache, r), batch)[0], seq_ops.rows_linear,
-                            lambda l, h: seq_ops.rows_glu(h, l.w_gate_up, l.mlp.limit))
+        decode = lambda r, l, h: l.mixer.decode(l.mixer.w_in, h, None, self.run_state(cache, r), batch)[0]
+        glu = lambda l, h: seq_ops.rows_glu(h, l.w_gate_up, l.mlp.limit)
+        if trace is not None or not self.layers:
+            return self._layers(tokens, trace, decode, seq_ops.rows_linear, glu)
+        x, h = self._start(tokens)
+        y = w = None
+        for r, layer in enumerate(self.layers):
+            parts = [(lambda h: decode(r, layer, h), layer.w_o, layer.norm1)]
+            if layer.mlp is not None:
+                parts.append((lambda h: glu(layer, h), layer.w_down, layer.norm2))
+            for part, w_out, norm in parts:
+                if y is not None:
+                    h = seq_ops.PostRows(x, y, w, self.config.norm_eps)
+                    x = h.out
+                y, w = seq_ops.rows_linear(part(h), w_out), norm
+        return self._residual(x, y, w, True)[1]

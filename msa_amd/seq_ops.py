@@ -444,7 +444,23 @@ def kv_attn(q: torch.Tensor, k_cache, v_cache, scale: float, batch: StepBatch, c
     return out
 
 
+class PostRows:
+    """The operand ``x + rms_norm(y) * w`` of :func:`rms_residual` for up to 16 rows, which the product that takes it forms on the
+    way; the sum itself is then in ``out``."""
+
+    def __init__(self, x, y, w, eps: float):
+        _dense(x)
+        _f32(x.shape[1], w)
+        if x.dtype != torch.float32 or y.dtype != torch.bfloat16 or y.shape != x.shape:
+            raise ValueError("PostRows: fp32 stream and bf16 sublayer output [M, W]")
+        self.y, self.shape, self.device = y, y.shape, y.device
+        self.out, self.keep = torch.empty_like(x), (x, torch.empty(y.shape, dtype=y.dtype, device=y.device))
+        self.c = _lib.RowsPost(ptr(x), ptr(self.out), ptr(w), ptr(self.keep[1]), eps, 0)
+
+
 def _rows_args(x, w, groups: int = 1, x_b=None, n_b: Optional[int] = None) -> _lib.RowsArgs:
+    post = x if isinstance(x, PostRows) else None
+    x = x if post is None else post.y
     M = x.shape[0]
     K = w.shape[1]
     N = w.shape[0] // groups
@@ -458,10 +474,14 @@ def _rows_args(x, w, groups: int = 1, x_b=None, n_b: Optional[int] = None) -> _l
     a.n_b = N if n_b is None else n_b
     if x_b is not None:
         a.x_b, a.x_b_stride = ptr(x_b), _rows(x_b)
+    a.post = post
     return a
 
 
 def _run_rows(a: _lib.RowsArgs, epilogue: int) -> None:
+    if a.post is not None:
+        _check(_lib.load_seq().msa_rows_linear_post(C.byref(a), epilogue, C.byref(a.post.c), _stream()), "msa_rows_linear_post")
+        return
     _check(_lib.load_seq().msa_rows_linear(C.byref(a), epilogue, _stream()), "msa_rows_linear")
 
 
