@@ -231,7 +231,10 @@ struct SplitArgs {
 };
 
 // DP / EP: D and E padded to 64, 128 or 256.
-template <int DP, int EP>
+// kOnce: every cache row is read by one row of the step and one tile of heads.  Its values, whole lines, are then read non-temporal,
+// which leaves the caches to the keys, whose lines take two requests (8 key heads of 128, 16 sequences behind up to 4096 tokens: 50.1
+// -> 34.4 us, one 8.7 -> 7.5, 16 behind up to 500 10.4 -> 8.6; with the keys through LDS as well, as whole lines: 36.4, 8.1, 9.0).
+template <int DP, int EP, bool kOnce>
 __global__ __launch_bounds__(256) void kv_split_kernel(SplitArgs p, msa_seq_batch b) {
   constexpr int kVS = EP + 8, kUnits = EP / 8, kVP = kStepKeys * kUnits / 64, kK = DP / 32, kC = EP / 16;
   constexpr int kOS = EP + 4;                                    // row stride of the sums at the end
@@ -274,7 +277,7 @@ __global__ __launch_bounds__(256) void kv_split_kernel(SplitArgs p, msa_seq_batc
 #pragma unroll
       for (int kk = 0; kk < kK; ++kk) r.k[t][kk] = __builtin_amdgcn_raw_buffer_load_b128(rk, k_at[kk] == kOutside ? kOutside : k_at[kk] + 16 * t * krow, 0, 0);
 #pragma unroll
-    for (int i = 0; i < kVP; ++i) r.v[i] = __builtin_amdgcn_raw_buffer_load_b128(rv, v_at[i], 0, 0);
+    for (int i = 0; i < kVP; ++i) r.v[i] = __builtin_amdgcn_raw_buffer_load_b128(rv, v_at[i], 0, kOnce ? 2 : 0);
   };
   fetch(cur, first);
   bf16x8_t qf[kK];
@@ -446,7 +449,9 @@ template <int DP, int EP>
 int launch_split(const SplitArgs& p, const msa_seq_batch& b, hipStream_t st) {
   const msa_kv_attn_args& a = p.a;
   const int tiles = (a.H / a.G + kHeadTile - 1) / kHeadTile;
-  kv_split_kernel<DP, EP><<<dim3(p.n_split, a.G * tiles, b.rows), 256, 0, st>>>(p, b);
+  const dim3 grid(p.n_split, a.G * tiles, b.rows);
+  if (b.max_rows == 1 && tiles == 1) kv_split_kernel<DP, EP, true><<<grid, 256, 0, st>>>(p, b);
+  else kv_split_kernel<DP, EP, false><<<grid, 256, 0, st>>>(p, b);
   MSA_LAUNCH_CHECK();
   if (p.n_split > 1) {
     const int64_t items = (int64_t)b.rows * a.H;
