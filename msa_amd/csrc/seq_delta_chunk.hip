@@ -787,10 +787,11 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(ChunkArgs walk, Chu
   }
 }
 
-// Bytes: 22 chunks of four sequences of 32 heads of 128 x 128.  (88 MB, of which two lie in the memory-side cache, is worth less than
-// long launches: 6001 tokens of five sequences take 470 us a layer then, 320 so, 357 with 176 MB, 322 with 704; one sequence of 8192
-// 410 either way.)
-constexpr int64_t kMaxSegment = (int64_t)352 << 20;
+// Bytes of a sequence, of up to four: 23 chunks of 32 heads of 128 x 128.  (88 MB for all of them, of which two lie in the memory-side
+// cache, is worth less than long launches: 6001 tokens of five sequences take 470 us a layer then, 320 so, 357 with 176 MB, 322 with
+// 704; two sequences of 4096 are through in 425 with 88, 415 with 176 and 411 with 352.)
+constexpr int64_t kMaxSegment = (int64_t)88 << 20;
+constexpr int kMaxSegments = 4;
 constexpr int kSegments = 6, kLeastChunks = 22;           // segments of a long portion, chunks that are worth a launch
 
 int64_t unit_bytes(int32_t D, int32_t E) {
@@ -804,7 +805,7 @@ int64_t unit_bytes(int32_t D, int32_t E) {
 // Chunks of a segment: enough to be worth a launch, few enough to overlap, at most what the workspace holds.
 int segment(const msa_delta_args& a, int32_t max_rows, int32_t n_seq) {
   const int64_t chunks = (max_rows + kC - 1) / kC, per = unit_bytes(a.D, a.E) * a.H * n_seq;
-  const int64_t most = std::max<int64_t>(1, kMaxSegment / per), want = std::max<int64_t>(kLeastChunks, (chunks + kSegments - 1) / kSegments);
+  const int64_t most = std::max<int64_t>(1, kMaxSegment * std::min(n_seq, kMaxSegments) / per), want = std::max<int64_t>(kLeastChunks, (chunks + kSegments - 1) / kSegments);
   const int64_t parts = (chunks + std::min(most, want) - 1) / std::min(most, want);
   return (int)((chunks + parts - 1) / parts);
 }
