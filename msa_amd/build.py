@@ -63,6 +63,9 @@ CONTRACTS = {
     "route_score.hip": [("score_scan4_kernel", {"max_compiler_vgpr": 127, "no_agpr": True})],
     "flash_attn.hip": [("flash_attn_kernel", {}), ("flash_wide_kernel", {"max_compiler_vgpr": 55, "no_agpr": True})],
 }
+#  * rows_ring_kernel (rows_ring.h): what it requests into LDS in front of its loop is read by asm statements, for which
+#    the compiler does not wait.  The first request has to be waited for in front of the first LDS read.
+LDS_WAITS = {"linear.hip": "rows_ring_kernel", "seq_rows.hip": "rows_ring_kernel"}
 
 
 def _device_asm(src: str, extra=()) -> str:
@@ -123,14 +126,36 @@ def check_kernel_contracts(asm: str, kernel_substring: str, max_compiler_vgpr=No
     return problems
 
 
+def check_lds_waits(asm: str, kernel_substring: str):
+    """Violations in the kernels whose symbol contains `kernel_substring`: an LDS read that no wait covering the kernel's first
+    direct-to-LDS load precedes.  Loads return in order, so a wait for all but n operations covers it once n buffer loads are
+    younger (other operations may stand in branches and count for nothing)."""
+    problems, found = [], 0
+    for m in re.finditer(r"^(\S*%s\S*):(.*?)s_endpgm" % re.escape(kernel_substring), asm, flags=re.S | re.M):
+        found += 1
+        younger, covered = None, False
+        for line in m.group(2).split("\n"):
+            code = line.split(";")[0].strip()
+            wait = re.search(r"vmcnt\((\d+)\)", code)
+            if wait and younger is not None:
+                covered |= int(wait.group(1)) <= younger
+            elif code.startswith("buffer_load"):
+                younger = younger + 1 if younger is not None else 0 if code.endswith(" lds") else None
+            elif code.startswith("ds_read"):
+                if not covered:
+                    problems.append(f"{m.group(1)}: LDS is read before the first load into it has been waited for: {code}")
+                break
+    return problems if found else [f"no kernel matching {kernel_substring!r} in the assembly"]
+
+
 def _check_contracts(src: str) -> None:
-    rules = CONTRACTS.get(os.path.basename(src))
-    if not rules:
-        return
+    name = os.path.basename(src)
     asm = _device_asm(src)
     problems = []
-    for kernel, kw in rules:
+    for kernel, kw in CONTRACTS.get(name, ()):
         problems += check_kernel_contracts(asm, kernel, **kw)
+    if name in LDS_WAITS:
+        problems += check_lds_waits(asm, LDS_WAITS[name])
     if problems:
         raise RuntimeError("inline-asm contract broken in %s:\n  %s" % (src, "\n  ".join(problems[:20])))
 
@@ -168,8 +193,9 @@ def build(jobs: int = 8) -> str:
     for gen, inc in (("gen_scan_asm.py", "scan_asm.inc"), ("gen_flash_asm.py", "flash_asm.inc")):
         if subprocess.run([sys.executable, os.path.join(CSRC, gen), "--check"]).returncode != 0:
             raise RuntimeError(f"csrc/{inc} is not what csrc/{gen} generates: run the generator")
-    with ThreadPoolExecutor(max_workers=min(jobs, len(srcs) + len(CONTRACTS))) as ex:
-        checks = [ex.submit(_check_contracts, s) for s in srcs if os.path.basename(s) in CONTRACTS]
+    checked = [s for s in srcs if os.path.basename(s) in {**CONTRACTS, **LDS_WAITS}]
+    with ThreadPoolExecutor(max_workers=min(jobs, len(srcs) + len(checked))) as ex:
+        checks = [ex.submit(_check_contracts, s) for s in checked]
         objs = dict(zip(srcs, ex.map(_compile, srcs)))
         for c in checks:
             c.result()

@@ -218,7 +218,8 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
   }
   if constexpr (kPro == kPost) {
     // x + rms_norm(y) * w as the operand, the sums as in the launch of its own.  (LDS by hand: the compiler would wait for the ring
-    // in front of it.  The weights have arrived with what was requested behind them.)
+    // in front of it, and nor does it wait for the weights: what the ring has requested by now, 2 kSlots loads, is all that may be
+    // outstanding when they are read.  The build checks that.)
     float ssq = 0.f;
 #pragma unroll
     for (int u = 0; u < NU; ++u)
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
     ssq += __shfl_xor(ssq, 16);
     ssq += __shfl_xor(ssq, 32);
     const uint32_t row_at = lds_offset(row_ssq + n_l * 16);
-    asm volatile("ds_write_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::"v"(row_at + 4 * wave), "v"(ssq) : "memory");
+    asm volatile("ds_write_b32 %0, %1\n\ts_waitcnt vmcnt(%2) lgkmcnt(0)\n\ts_barrier" ::"v"(row_at + 4 * wave), "v"(ssq), "n"(2 * kSlots) : "memory");
     float total = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

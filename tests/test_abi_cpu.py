@@ -219,3 +219,45 @@ def test_build_guard_covers_the_wide_flash_kernel():
     assert "flash_wide_kernel" in names and "flash_attn_kernel" in names
     rules = dict(build.CONTRACTS["flash_attn.hip"])["flash_wide_kernel"]
     assert rules == {"max_compiler_vgpr": 55, "no_agpr": True}
+
+
+RING = """
+_ZN9rows_ring16rows_ring_kernelIXLi1ELi2EEEv:
+	buffer_load_dwordx4 v[2:5], v1, s[0:3], 0 offen
+	buffer_load_dwordx4 v1, s[0:3], s4 offen lds
+	buffer_load_dwordx4 v[6:9], v1, s[0:3], 0 offen
+	global_load_dword v10, v[11:12], off
+	buffer_load_dwordx4 v1, s[0:3], s4 offen nt lds
+	s_waitcnt vmcnt(%d)
+	ds_read_b128 v[12:15], v1
+	s_endpgm
+"""
+
+
+def test_build_guard_wants_a_wait_in_front_of_the_first_lds_read():
+    """Two buffer loads are certainly younger than the first load into LDS: vmcnt(2) covers it, vmcnt(3), with a load that may stand
+    in a branch, does not."""
+    from msa_amd import build as B
+    assert B.check_lds_waits(RING % 2, "rows_ring_kernel") == []
+    assert len(B.check_lds_waits(RING % 3, "rows_ring_kernel")) == 1
+    assert len(B.check_lds_waits(RING.replace("s_waitcnt vmcnt(%d)", "s_waitcnt lgkmcnt(0)"), "rows_ring_kernel")) == 1
+    assert B.check_lds_waits(RING % 2, "no_such_kernel") != []
+
+
+def test_residual_step_waits_for_its_weights():
+    """The folded residual step reads its weights from LDS behind a wait; without it (in a copy of the header, compiled only) all
+    nine kernels are reported: three epilogues, one to three units."""
+    from msa_amd import build as B
+    assert B.check_lds_waits(B._device_asm(os.path.join(B.CSRC, "seq_rows.hip")), "rows_ring_kernel") == []
+    header, source = (open(os.path.join(B.CSRC, f)).read() for f in ("rows_ring.h", "seq_rows.hip"))
+    assert header.count("s_waitcnt vmcnt(%2) lgkmcnt(0)") == 1
+    names = [os.path.join(B.CSRC, f) for f in ("_guard_ring.h", "_guard_rows.hip")]
+    try:
+        open(names[0], "w").write(header.replace("s_waitcnt vmcnt(%2) lgkmcnt(0)", "s_waitcnt lgkmcnt(0)"))
+        open(names[1], "w").write(source.replace('"rows_ring.h"', '"_guard_ring.h"'))
+        problems = B.check_lds_waits(B._device_asm(names[1]), "rows_ring_kernel")
+    finally:
+        for n in names:
+            if os.path.exists(n):
+                os.remove(n)
+    assert len(problems) == 9 and all("Li2EEEv" in p for p in problems), problems

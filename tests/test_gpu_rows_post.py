@@ -40,6 +40,27 @@ def test_post_operand(form, M, K, N):
     assert torch.equal(got, product(post.out.bfloat16(), s2)) and torch.equal(s1, s2)
 
 
+@pytest.mark.parametrize("form", ["plain", "glu", "conv"])
+@pytest.mark.parametrize("M,K,N", [(1, 1024, 4096), (3, 2048, 4100), (1, 3072, 6144)])
+def test_post_operand_with_cold_weights(form, M, K, N):
+    """The norm's weights come from memory (a gigabyte has been written since they were), the sublayer's output from a near cache:
+    the product is again the one of the sum's bf16 rows, bit for bit, from every workgroup."""
+    from msa_amd import seq_ops
+    x, y, w, g = operands(M, K, K + N)
+    m = (torch.randn((N, K), generator=g) * K ** -0.5).bfloat16().cuda()
+    taps, state = torch.randn((N, 4), generator=g).cuda(), torch.zeros((M, 3, N), device="cuda")
+    slot = torch.arange(M, dtype=torch.int32).cuda()
+    product = {"plain": lambda h: seq_ops.rows_linear(h, m), "glu": lambda h: seq_ops.rows_glu(h, m, 7.0),
+               "conv": lambda h: seq_ops.rows_conv(h, m, None, None, 0, taps, None, state.clone(), slot)}[form]
+    flush = torch.empty(1 << 28, device="cuda")
+    for i in range(4):
+        flush.fill_(float(i))
+        x.mul_(1.0), y.mul_(1.0)
+        post = seq_ops.PostRows(x, y, w, 1e-5)
+        got = product(post)
+        assert torch.equal(got, product(post.out.bfloat16())), i
+
+
 def test_post_operand_refuses_what_the_residual_step_refuses():
     from msa_amd import seq_ops
     x, y, w, _ = operands(2, 1024, 1)
