@@ -590,9 +590,10 @@ __global__ __launch_bounds__(kHeadDim) void attn_combine_kernel(const float* __r
     at *= keep;
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      const float a = s0 + i < n_split && ms[i] != -INFINITY ? fast_exp2(ms[i] - mb) : 0.f;
-      lt += ls[i] * a;
-      at += as[i] * a;
+      const bool in = s0 + i < n_split;                  // (an infinity in the last partial would be NaN in the places behind it)
+      const float a = ms[i] != -INFINITY ? fast_exp2(ms[i] - mb) : 0.f;
+      lt += in ? ls[i] * a : 0.f;
+      at += in ? as[i] * a : 0.f;
     }
     mn = mb;
   }

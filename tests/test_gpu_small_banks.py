@@ -110,3 +110,28 @@ def test_decode_attention_through_the_ring(G):
         assert torch.equal(out[b][~fin], want[~fin])
         bound = want.abs() * 2 ** -8 + (p[..., None] * vv.abs()).sum(0) * (2 ** -8 if b == 4 else 2 ** -15)
         assert ((out[b] - want).abs() <= bound)[fin].all()
+
+
+def _attention(q, k, v):
+    p = torch.softmax((q.double()[:, None] * k.double()[None]).sum(-1) * 128 ** -0.5, dim=1)       # [rows, keys, heads]
+    return (p[..., None] * v.double()[None]).sum(1)
+
+
+@pytest.mark.parametrize("dtype,sq,L", [(torch.bfloat16, 1, 700), (torch.bfloat16, 1, 4400), (torch.float32, 1, 700), (torch.float32, 1, 4400),
+                                        (torch.bfloat16, 12, 100), (torch.bfloat16, 12, 700), (torch.bfloat16, 12, 4400)])
+def test_infinite_values_in_the_last_split(dtype, sq, L):
+    """One sample, one infinite value among its last keys: splits of 256 keys or more, none of them sixteen or a multiple, single
+    rows and query blocks (the last key but one: a tile's last row also stands in for those behind it).  The head's column is
+    infinite and nothing else changes.  Bounds as for single passes above."""
+    from msa_amd import ops
+    g = torch.Generator().manual_seed(L + sq)
+    q, k, v = (torch.randn(s, generator=g).to(dtype) for s in ((sq, 8, 128), (L, 2, 128), (L, 2, 128)))
+    v[L - (1 if sq == 1 else 2), 1, 7] = float("inf")
+    cu = torch.tensor([0, sq], dtype=torch.int32).cuda() if sq > 1 else None
+    out = ops.sparse_attn(q.cuda(), k.cuda(), v.cuda(), torch.zeros(1, dtype=torch.int64).cuda(), torch.tensor([L], dtype=torch.int32).cuda(), L, cu_q=cu,
+                          max_sq=sq, causal=False).cpu().double()
+    want = _attention(q, k.repeat_interleave(4, dim=1), v.repeat_interleave(4, dim=1))
+    assert torch.isinf(want[:, 4:, 7]).all() and torch.equal(torch.isfinite(out), torch.isfinite(want))
+    fin = torch.isfinite(want)
+    assert (out[~fin] == want[~fin]).all()
+    assert (out - want)[fin].abs().max() <= (1e-5 if dtype == torch.float32 else 1e-2) * want[fin].abs().max()
