@@ -170,9 +170,18 @@ struct Ring {
     request(k, kt, wave);
     request(v, vt, wave);
   }
+  template <int kWeightParts>
   __device__ __forceinline__ void run(int lane, int G, const bf16x8_t (&qf)[4], float scale_log2e, char* lds) const;
 };
 
+// Two bf16 values with zeros in the place of infinities and NaN.
+__device__ __forceinline__ uint32_t finite_pair(uint32_t w) {
+  return ((w & 0x7f80u) == 0x7f80u ? 0u : w & 0xffffu) | ((w & 0x7f800000u) == 0x7f800000u ? 0u : w & 0xffff0000u);
+}
+
+// The weights go to the matrix cores as kWeightParts bf16 parts, the first the weight rounded, the others what is left of it: one
+// alone would depend on which keys share a reference maximum, two hold 16 bits of the weight, three all 24.
+template <int kWeightParts>
 __device__ __forceinline__ void Ring::run(int lane, int G, const bf16x8_t (&qf)[4], float scale_log2e, char* lds) const {
   const int l16 = lane & 15, g = lane >> 4;
   // V^T operands: eight bytes of row 4 g + l16 / 4 (and of the row 16 further on): lanes 4 r .. 4 r + 3 of 16 name the pieces of
@@ -183,11 +192,11 @@ __device__ __forceinline__ void Ring::run(int lane, int G, const bf16x8_t (&qf)[
     const int row = 4 * g + (l16 >> 2);
     v_at[c] = lds_offset(vt) + row * kRowBytes + (l16 & 1) * 8 + (((2 * c + ((l16 & 3) >> 1)) ^ row) * 16);
   }
-  // A second pass without the weights' low parts, if there are NaN: a low part of zero or below against an infinite value makes one
-  // where the weight itself leaves the infinity.
+  // A second pass, if there are NaN, in which the weights' low parts see finite values alone: a low part of zero or below against an
+  // infinite value makes NaN where the weight itself leaves the infinity.
   floatx4_t o[8];
   float m, l;                            // of head l16: m the same in its four lanes, l each lane's own keys
-  for (bool low_part = true;;) {
+  for (bool finite_only = false;;) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) o[c] = floatx4_t{0.f, 0.f, 0.f, 0.f};
     m = -INFINITY;
@@ -227,20 +236,20 @@ __device__ __forceinline__ void Ring::run(int lane, int G, const bf16x8_t (&qf)[
         m = mx;
       }
       const float ref = m == -INFINITY ? 0.f : m;            // (scores of -inf alone: every weight is 0)
-      // weights as a high and a low bf16 part: rounded once, they depend on which keys share a reference maximum
-      uint32_t ph[4], pl[4];
+      uint32_t part[kWeightParts][4];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int e = 0; e < 4; e += 2) {
-          const float p0 = fast_exp2(x[t][e] - ref), p1 = fast_exp2(x[t][e + 1] - ref);
+          float p0 = fast_exp2(x[t][e] - ref), p1 = fast_exp2(x[t][e + 1] - ref);
           l += p0 + p1;
-          const uint32_t hi = pack_bf16x2(p0, p1);
-          ph[2 * t + e / 2] = hi;
-          pl[2 * t + e / 2] = pack_bf16x2(p0 - bf16lo(hi), p1 - bf16hi(hi));
+#pragma unroll
+          for (int i = 0; i < kWeightParts; ++i) {
+            const uint32_t w = part[i][2 * t + e / 2] = pack_bf16x2(p0, p1);
+            p0 -= bf16lo(w);
+            p1 -= bf16hi(w);
+          }
         }
-      const bf16x8_t hi8 = __builtin_bit_cast(bf16x8_t, make_uint4(ph[0], ph[1], ph[2], ph[3]));
-      const bf16x8_t lo8 = __builtin_bit_cast(bf16x8_t, make_uint4(pl[0], pl[1], pl[2], pl[3]));
       __builtin_amdgcn_s_waitcnt(wait_vm(8));                // V: only the next K is younger
       asm volatile("" ::: "memory");
       // (the transposing reads are written out, wait included: in front of its own the compiler waits for the next K too, 4 us in 50)
@@ -261,10 +270,17 @@ __device__ __forceinline__ void Ring::run(int lane, int G, const bf16x8_t (&qf)[
           : "memory");
       request(v, vt, step + kRingWaves);                     // (V has been read)
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, make_uint4(vr[2 * c].x, vr[2 * c].y, vr[2 * c + 1].x, vr[2 * c + 1].y));
-        o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, hi8, o[c], 0, 0, 0);
-        if (low_part) o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, lo8, o[c], 0, 0, 0);
+      for (int i = 0; i < kWeightParts; ++i) {
+        if (i == 1 && finite_only) {
+#pragma unroll
+          for (int c = 0; c < 16; ++c) vr[c] = u32x2_t{finite_pair(vr[c].x), finite_pair(vr[c].y)};
+        }
+        const bf16x8_t w8 = __builtin_bit_cast(bf16x8_t, make_uint4(part[i][0], part[i][1], part[i][2], part[i][3]));
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, make_uint4(vr[2 * c].x, vr[2 * c].y, vr[2 * c + 1].x, vr[2 * c + 1].y));
+          o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, w8, o[c], 0, 0, 0);
+        }
       }
     }
     __builtin_amdgcn_s_waitcnt(wait_vm(0));                  // nothing may still be writing LDS when the sums go there
@@ -274,8 +290,8 @@ __device__ __forceinline__ void Ring::run(int lane, int G, const bf16x8_t (&qf)[
     for (int c = 0; c < 8; ++c)
 #pragma unroll
       for (int e = 0; e < 4; ++e) nan |= o[c][e] != o[c][e];
-    if (!low_part || !__any(nan)) break;
-    low_part = false;
+    if (finite_only || !__any(nan)) break;
+    finite_only = true;
     start();
   }
   l += __shfl_xor(l, 16);
@@ -304,6 +320,7 @@ __device__ __forceinline__ void fold_sums(char* lds, int parts, int h, int d, fl
 }
 
 // bf16 rows: workgroup (row, KV head, split) as in attn_partial_kernel below.
+template <int kWeightParts>
 __global__ __launch_bounds__(kRingWaves * 64) void attn_ring_kernel(
     const bf16_t* __restrict__ q, const int32_t* __restrict__ cu_q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
     const int64_t* __restrict__ kv_off, const int32_t* __restrict__ kv_len, int32_t B, int32_t Hq, int32_t Hkv, float scale_log2e,
@@ -325,7 +342,7 @@ __global__ __launch_bounds__(kRingWaves * 64) void attn_ring_kernel(
     qf[kk] = __builtin_bit_cast(bf16x8_t, (lane & 15) < G ? q16[(lane & 15) * 16 + 4 * kk + (lane >> 4)] : make_uint4(0, 0, 0, 0));
   asm volatile("" ::: "memory");                           // (the ring counts what is younger)
   ring.start();
-  ring.run(lane, G, qf, scale_log2e, lds);
+  ring.run<kWeightParts>(lane, G, qf, scale_log2e, lds);
   __syncthreads();
   for (int idx = tid; idx < G * kHeadDim; idx += kRingWaves * 64) {
     const int h = idx / kHeadDim, d = idx % kHeadDim;
@@ -524,7 +541,7 @@ __global__ __launch_bounds__(kRingWaves * 64) void attn_decode_fused_kernel(
     const uint4 u = lds_read16(sm_q + (j < G ? j : 0) * 16 + 4 * kk + (lane >> 4));
     qf[kk] = __builtin_bit_cast(bf16x8_t, j < G ? u : make_uint4(0, 0, 0, 0));
   }
-  ring.run(lane, G, qf, scale_log2e, lds);
+  ring.run<2>(lane, G, qf, scale_log2e, lds);
   if (owner) {
     // one more key, straight from registers: its weight against itself is 1
     const uint32_t vs[4] = {v_new.x, v_new.y, v_new.z, v_new.w};
@@ -636,17 +653,14 @@ int launch_attn_f32(const void* q, const int32_t* cu_q, const void* k, const voi
 constexpr int kFusedLds = kRingLds + (int)sizeof(HeadSums) + kMaxG * 16 * (int)sizeof(uint4);
 static_assert(2 * kFusedLds <= 160 * 1024, "two workgroups a compute unit");
 
-int launch_attn_bf16(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
+template <int kWeightParts>
+int launch_attn_ring(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                      const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
                      int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st) {
-  const int n_split = plan.n_split, G = Hq / Hkv;
-  if (G != 1 && G != 2 && G != 4 && G != 8) {
-    msa_set_error("msa_sparse_attn: GQA group size %d unsupported (1, 2, 4, 8)", G);
-    return MSA_EINVAL;
-  }
+  const int n_split = plan.n_split;
   static std::atomic<int> lds_limit_raised{0};
-  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(attn_ring_kernel), kRingLds));
-  attn_ring_kernel<<<dim3((unsigned)total_q, (unsigned)Hkv, (unsigned)n_split), kRingWaves * 64, kRingLds, st>>>(
+  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(attn_ring_kernel<kWeightParts>), kRingLds));
+  attn_ring_kernel<kWeightParts><<<dim3((unsigned)total_q, (unsigned)Hkv, (unsigned)n_split), kRingWaves * 64, kRingLds, st>>>(
       static_cast<const bf16_t*>(q), cu_q, static_cast<const bf16_t*>(k), static_cast<const bf16_t*>(v), kv_off, kv_len, B, Hq, Hkv,
       scale * 1.4426950408889634f, causal, n_split, part_ml, part_acc, static_cast<bf16_t*>(out));
   MSA_LAUNCH_CHECK();
@@ -655,6 +669,19 @@ int launch_attn_bf16(const void* q, const int32_t* cu_q, const void* k, const vo
                                                                                       static_cast<bf16_t*>(out));
   MSA_LAUNCH_CHECK();
   return MSA_OK;
+}
+
+// Groups of one and two heads keep all of their weights' bits.
+int launch_attn_bf16(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
+                     const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
+                     int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st) {
+  const int G = Hq / Hkv;
+  if (G != 1 && G != 2 && G != 4 && G != 8) {
+    msa_set_error("msa_sparse_attn: GQA group size %d unsupported (1, 2, 4, 8)", G);
+    return MSA_EINVAL;
+  }
+  const auto launch = G <= 2 ? launch_attn_ring<3> : launch_attn_ring<2>;
+  return launch(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml, part_acc, st);
 }
 
 }  // namespace
