@@ -575,14 +575,13 @@ __global__ __launch_bounds__(kRingWaves * 64) void attn_decode_fused_kernel(
 }
 
 // One workgroup of 128 threads per (query row, head): merges the row's partials and normalises.  The partials are requested sixteen
-// at a time (one after the other, each waited for the one before: 32 of them took 16 us).  With `kv_len` (decode: rows = samples)
+// at a time (one after the other, each waited for the one before: 32 of them took 16 us), four at a time where there are no more.  With `kv_len` (decode: rows = samples)
 // the workgroup of head 0 also advances the sample's cache length, unless the cache was full and the new row was dropped.
-template <typename T>
+template <typename T, int kBatch>
 __global__ __launch_bounds__(kHeadDim) void attn_combine_kernel(const float* __restrict__ part_ml,
                                                                 const float* __restrict__ part_acc, int32_t n_split,
-                                                                T* __restrict__ out, int32_t* __restrict__ kv_len = nullptr,
-                                                                int32_t Lcap = 0, int32_t Hq = 1) {
-  constexpr int kBatch = 16;
+                                                                T* __restrict__ out, int32_t* __restrict__ kv_len,
+                                                                int32_t Lcap, int32_t Hq) {
   const int64_t rh = blockIdx.x;   // row * Hq + head
   const int d = threadIdx.x;
   if (kv_len != nullptr && d == 0 && rh % Hq == 0) {
@@ -619,6 +618,15 @@ __global__ __launch_bounds__(kHeadDim) void attn_combine_kernel(const float* __r
   else out[rh * kHeadDim + d] = o;
 }
 
+template <typename T>
+int launch_combine(const float* part_ml, const float* part_acc, int64_t rows, int32_t n_split, void* out, hipStream_t st,
+                   int32_t* kv_len = nullptr, int32_t Lcap = 0, int32_t Hq = 1) {
+  const auto kernel = n_split <= 4 ? attn_combine_kernel<T, 4> : attn_combine_kernel<T, 16>;
+  kernel<<<(unsigned)rows, kHeadDim, 0, st>>>(part_ml, part_acc, n_split, static_cast<T*>(out), kv_len, Lcap, Hq);
+  MSA_LAUNCH_CHECK();
+  return MSA_OK;
+}
+
 int launch_attn_f32(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                     const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
                     int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st) {
@@ -644,10 +652,7 @@ int launch_attn_f32(const void* q, const int32_t* cu_q, const void* k, const voi
 #undef MSA_ATTN_CASE
   MSA_LAUNCH_CHECK();
   if (n_split == 1) return MSA_OK;
-  attn_combine_kernel<float><<<(unsigned)((int64_t)total_q * Hq), kHeadDim, 0, st>>>(part_ml, part_acc, n_split,
-                                                                                     static_cast<float*>(out));
-  MSA_LAUNCH_CHECK();
-  return MSA_OK;
+  return launch_combine<float>(part_ml, part_acc, (int64_t)total_q * Hq, n_split, out, st);
 }
 
 constexpr int kFusedLds = kRingLds + (int)sizeof(HeadSums) + kMaxG * 16 * (int)sizeof(uint4);
@@ -665,10 +670,7 @@ int launch_attn_ring(const void* q, const int32_t* cu_q, const void* k, const vo
       scale * 1.4426950408889634f, causal, n_split, part_ml, part_acc, static_cast<bf16_t*>(out));
   MSA_LAUNCH_CHECK();
   if (n_split == 1) return MSA_OK;
-  attn_combine_kernel<bf16_t><<<(unsigned)((int64_t)total_q * Hq), kHeadDim, 0, st>>>(part_ml, part_acc, n_split,
-                                                                                      static_cast<bf16_t*>(out));
-  MSA_LAUNCH_CHECK();
-  return MSA_OK;
+  return launch_combine<bf16_t>(part_ml, part_acc, (int64_t)total_q * Hq, n_split, out, st);
 }
 
 // Groups of one and two heads keep all of their weights' bits.
@@ -728,10 +730,7 @@ extern "C" int msa_sparse_attn(const void* q, const int32_t* cu_q, const void* k
     int rc = flash_attn_split_launch(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, part_ml,
                                      part_acc, st);
     if (rc != MSA_OK) return rc;
-    attn_combine_kernel<bf16_t><<<(unsigned)((int64_t)total_q * Hq), kHeadDim, 0, st>>>(part_ml, part_acc, n_split,
-                                                                                      static_cast<bf16_t*>(out));
-    MSA_LAUNCH_CHECK();
-    return MSA_OK;
+    return launch_combine<bf16_t>(part_ml, part_acc, (int64_t)total_q * Hq, n_split, out, st);
   }
   if (dtype == MSA_BF16)
     return launch_attn_bf16(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml,
@@ -771,8 +770,5 @@ extern "C" int msa_decode_attn_fused(const void* qkv, int64_t row_stride, const 
       static_cast<const bf16_t*>(k_norm_w), eps, rope_cos, rope_sin, rope_rows, static_cast<bf16_t*>(kcache),
       static_cast<bf16_t*>(vcache), Lcap, kv_len, scale * 1.4426950408889634f, n_split, part_ml, part_acc);
   MSA_LAUNCH_CHECK();
-  attn_combine_kernel<bf16_t><<<(unsigned)((int64_t)B * Hq), kHeadDim, 0, st>>>(part_ml, part_acc, n_split,
-                                                                                static_cast<bf16_t*>(out), kv_len, Lcap, Hq);
-  MSA_LAUNCH_CHECK();
-  return MSA_OK;
+  return launch_combine<bf16_t>(part_ml, part_acc, (int64_t)B * Hq, n_split, out, st, kv_len, Lcap, Hq);
 }

@@ -25,10 +25,15 @@ static inline SplitPlan plan_splits_for(int64_t total_q, int32_t Hkv, int32_t ma
 static inline SplitPlan plan_splits(int64_t total_q, int32_t Hkv, int32_t max_kv) {
   return plan_splits_for(total_q, Hkv, max_kv, 1024);
 }
-// Single rows (decode): fp32 one workgroup per compute unit (fewer, longer key streams), bf16 the two whose rings fit (one sample
-// of 4388 keys 11.9 us, 17.5 as one per unit); the kernels divide each sample's own length evenly over n_split.
+// Single rows (decode): one workgroup per compute unit (fewer, longer key streams); the kernels divide each sample's own length
+// evenly over n_split.  The bf16 ring, of which two fit, is cut finer where that does not come out even and leaves 256 keys a split
+// or more (groups of four, us: 24 samples of 2200 to 4400 keys with 2 KV heads in 288 workgroups 28.2, in 528 23.6; but 16 of 256 to
+// 512 with 8, even in 256, 13.4 against 15.1 in 384).
 static inline SplitPlan plan_splits_rows(int64_t total_q, int32_t Hkv, int32_t max_kv, int32_t dtype) {
-  return plan_splits_for(total_q, Hkv, max_kv, dtype == MSA_BF16 ? 512 : 256);
+  constexpr int kUnits = 256;
+  const int64_t pairs = std::max<int64_t>(1, total_q * Hkv), finer = (2 * kUnits + pairs - 1) / pairs;
+  const bool even = (kUnits + pairs - 1) / pairs * pairs == kUnits;
+  return plan_splits_for(total_q, Hkv, max_kv, dtype == MSA_BF16 && !even && max_kv >= kMinSplitKeys * finer ? 2 * kUnits : kUnits);
 }
 
 // flash_attn.hip: bf16 partial pass over split `blockIdx.z` of the keys; writes un-normalised

@@ -164,3 +164,19 @@ def test_weights_of_one_and_two_heads_keep_their_bits(G, infinite):
     fin = torch.isfinite(want)
     assert torch.equal(out[~fin], want[~fin])
     assert ((out - want).abs() <= want.abs() * 2 ** -8 + size * 2 ** -20)[fin].all()
+
+
+@pytest.mark.parametrize("B,L", [(1, 300), (3, 1024), (3, 1100), (16, 1300), (24, 2815), (24, 2816), (48, 1500)])
+def test_split_plans_and_partials(B, L):
+    """2 to 18 partials a head, four and sixteen a batch of the combining kernel and their neighbours, in plans of one and of two
+    workgroups a compute unit (24 samples of 2 heads from 2816 keys on).  Bounds as in the test of the ring."""
+    from msa_amd import ops
+    g = torch.Generator().manual_seed(L)
+    q, k, v = (torch.randn(s, generator=g).bfloat16() for s in ((B, 8, 128), (B * L, 2, 128), (B * L, 2, 128)))
+    lens = torch.tensor([L - 7 * b for b in range(B)], dtype=torch.int32)
+    out = ops.sparse_attn(q.cuda(), k.cuda(), v.cuda(), (L * torch.arange(B)).cuda(), lens.cuda(), L).cpu().double()
+    for b in range(0, B, max(1, B // 4)):
+        kk, vv = (t[b * L:b * L + int(lens[b])].double().repeat_interleave(4, dim=1) for t in (k, v))
+        p = torch.softmax((q[b].double()[None] * kk).sum(-1) * 128 ** -0.5, dim=0)
+        want = (p[..., None] * vv).sum(0)
+        assert ((out[b] - want).abs() <= want.abs() * 2 ** -8 + (p[..., None] * vv.abs()).sum(0) * 2 ** -15).all()
