@@ -20,10 +20,16 @@ constexpr int kMaxG = 8;
 // should not displace anything in L2 (the whole decode step runs 3 % faster with the hint).
 typedef unsigned int u32x4_stream_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint4 ld16_stream(const void* p) {
-  const u32x4_stream_t w = __builtin_nontemporal_load(reinterpret_cast<const u32x4_stream_t*>(p));
+  // (memory, said outright: of a pointer that may be one of two the compiler makes flat loads, which also wait for LDS)
+  const u32x4_stream_t w = __builtin_nontemporal_load((const __attribute__((address_space(1))) u32x4_stream_t*)(uintptr_t)p);
   return make_uint4(w.x, w.y, w.z, w.w);
 }
 
+__device__ __forceinline__ void ld8(const bf16_t* p, float (&x)[8]) {
+  const uint4 w = ld16_stream(p);
+  x[0] = bf16lo(w.x); x[1] = bf16hi(w.x); x[2] = bf16lo(w.y); x[3] = bf16hi(w.y);
+  x[4] = bf16lo(w.z); x[5] = bf16hi(w.z); x[6] = bf16lo(w.w); x[7] = bf16hi(w.w);
+}
 __device__ __forceinline__ void ld8(const float* p, float (&x)[8]) {
   const uint4 a = ld16_stream(p), b = ld16_stream(p + 4);
   x[0] = __uint_as_float(a.x); x[1] = __uint_as_float(a.y); x[2] = __uint_as_float(a.z); x[3] = __uint_as_float(a.w);
@@ -51,13 +57,15 @@ __device__ __forceinline__ float row16_allsum(float d) {
   return d;
 }
 
+__device__ const uint4 kZeros[2] = {};
+
 // Streams keys first, first + stride, ... < key1 of one KV head through the running softmax state of this
 // lane (key slot = lane / 16, dims 8 j .. 8 j + 8).  Keys go in batches of kBatch steps: all K / V loads of a
 // batch are issued before any arithmetic (bytes in flight), scores are reduced over the 16 lanes of a key with
 // DPP row rotations, and the running softmax is rescaled once per batch.  `lane_off` is the element offset of
 // key 0's slice for this lane.
-template <int G>
-__device__ __forceinline__ void attend_keys(const float* __restrict__ k, const float* __restrict__ v, int64_t lane_off,
+template <typename T, int G>
+__device__ __forceinline__ void attend_keys(const T* __restrict__ k, const T* __restrict__ v, int64_t lane_off,
                                             int row_elems, int first, int key1, int stride, const float (&qv)[G][8],
                                             float (&m)[G], float (&l)[G], float (&acc)[G][8]) {
   constexpr int kBatch = 4;
@@ -70,7 +78,7 @@ __device__ __forceinline__ void attend_keys(const float* __restrict__ k, const f
       ok[u] = kk < key1;
       const int64_t off = lane_off + (int64_t)(ok[u] ? kk : kb) * row_elems;   // clamp: always in range
       ld8(k + off, kx[u]);
-      ld8(v + off, vx[u]);
+      ld8(ok[u] ? v + off : reinterpret_cast<const T*>(kZeros), vx[u]);   // (an infinite value with the weight zero would be NaN)
     }
 #pragma unroll
     for (int h = 0; h < G; ++h) {
@@ -358,13 +366,13 @@ __global__ __launch_bounds__(kRingWaves * 64) void attn_ring_kernel(
   }
 }
 
-// fp32 rows.
-template <int G, int kAttnWaves>
+// fp32 rows, and bf16 rows of groups of one and two heads where takes_ring says so.
+template <typename T, int G, int kAttnWaves>
 __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
-    const float* __restrict__ q, const int32_t* __restrict__ cu_q, const float* __restrict__ k, const float* __restrict__ v,
+    const T* __restrict__ q, const int32_t* __restrict__ cu_q, const T* __restrict__ k, const T* __restrict__ v,
     const int64_t* __restrict__ kv_off, const int32_t* __restrict__ kv_len, int32_t B, int32_t Hq, int32_t Hkv,
     float scale_log2e, int32_t causal, int32_t n_split, float* __restrict__ part_ml,
-    float* __restrict__ part_acc, float* __restrict__ out) {
+    float* __restrict__ part_acc, T* __restrict__ out) {
   __shared__ float sm_m[kAttnWaves][G], sm_l[kAttnWaves][G];
   __shared__ float sm_acc[kAttnWaves][G][kHeadDim];
 
@@ -392,7 +400,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
     for (int i = 0; i < 8; ++i) acc[h][i] = 0.f;
   }
   const int64_t lane_off = base * row_elems + g * kHeadDim + 8 * j;     // this lane's slice of key 0
-  const float* q_lane = q + ((int64_t)row * Hq + g * G) * kHeadDim + 8 * j;
+  const T* q_lane = q + ((int64_t)row * Hq + g * G) * kHeadDim + 8 * j;
   float qv[G][8];
 #pragma unroll
   for (int h = 0; h < G; ++h) {
@@ -400,7 +408,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) qv[h][i] *= scale_log2e;      // scores in log2 units: exp2f below
   }
-  attend_keys<G>(k, v, lane_off, row_elems, key0 + wave * 4 + slot, key1, kAttnWaves * 4, qv, m, l, acc);
+  attend_keys<T, G>(k, v, lane_off, row_elems, key0 + wave * 4 + slot, key1, kAttnWaves * 4, qv, m, l, acc);
 
   // merge the 4 key slots of the wavefront (lanes differing in bits 4 and 5)
 #pragma unroll
@@ -442,7 +450,8 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
     const int64_t o = ((int64_t)row * Hq + g * G + h) * n_split + split;
     if (n_split == 1) {                                  // nothing to merge: the output itself (a launch of 4 us less)
       const float y = lt > 0.f ? at / lt : 0.f;          // a row that sees no key yields zeros
-      out[o * kHeadDim + d] = y;
+      if constexpr (sizeof(T) == 2) out[o * kHeadDim + d] = f32_to_bf16(y);
+      else out[o * kHeadDim + d] = y;
       continue;
     }
     part_acc[o * kHeadDim + d] = at;
@@ -627,7 +636,8 @@ int launch_combine(const float* part_ml, const float* part_acc, int64_t rows, in
   return MSA_OK;
 }
 
-int launch_attn_f32(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
+template <typename T>
+int launch_attn(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                     const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
                     int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st) {
   const int n_split = plan.n_split;
@@ -636,23 +646,29 @@ int launch_attn_f32(const void* q, const int32_t* cu_q, const void* k, const voi
   const float sl2 = scale * 1.4426950408889634f;
 #define MSA_ATTN_CASE(GG, WW)                                                                                      \
   case GG:                                                                                                         \
-    attn_partial_kernel<GG, WW><<<grid, WW * 64, 0, st>>>(                                                         \
-        static_cast<const float*>(q), cu_q, static_cast<const float*>(k), static_cast<const float*>(v), kv_off,    \
-        kv_len, B, Hq, Hkv, sl2, causal, n_split, part_ml, part_acc, static_cast<float*>(out));                    \
-    break;
-  switch (G) {
-    MSA_ATTN_CASE(1, 4)
-    MSA_ATTN_CASE(2, 4)
-    MSA_ATTN_CASE(4, 8)
-    MSA_ATTN_CASE(8, 8)
-    default:
-      msa_set_error("msa_sparse_attn: GQA group size %d unsupported (1, 2, 4, 8)", G);
-      return MSA_EINVAL;
-  }
+    attn_partial_kernel<T, GG, WW><<<grid, WW * 64, 0, st>>>(                                                      \
+        static_cast<const T*>(q), cu_q, static_cast<const T*>(k), static_cast<const T*>(v), kv_off, kv_len, B, Hq, \
+        Hkv, sl2, causal, n_split, part_ml, part_acc, static_cast<T*>(out));                                       \
+    return MSA_OK;
+  const auto first = [&] {
+    switch (G) {
+      MSA_ATTN_CASE(1, 4)
+      MSA_ATTN_CASE(2, 4)
+    }
+    if constexpr (sizeof(T) == 4) {
+      switch (G) {
+        MSA_ATTN_CASE(4, 8)
+        MSA_ATTN_CASE(8, 8)
+      }
+    }
+    msa_set_error("msa_sparse_attn: GQA group size %d unsupported (1, 2, 4, 8)", G);
+    return MSA_EINVAL;
+  };
 #undef MSA_ATTN_CASE
+  if (const int rc = first(); rc != MSA_OK) return rc;
   MSA_LAUNCH_CHECK();
   if (n_split == 1) return MSA_OK;
-  return launch_combine<float>(part_ml, part_acc, (int64_t)total_q * Hq, n_split, out, st);
+  return launch_combine<T>(part_ml, part_acc, (int64_t)total_q * Hq, n_split, out, st);
 }
 
 constexpr int kFusedLds = kRingLds + (int)sizeof(HeadSums) + kMaxG * 16 * (int)sizeof(uint4);
@@ -673,16 +689,11 @@ int launch_attn_ring(const void* q, const int32_t* cu_q, const void* k, const vo
   return launch_combine<bf16_t>(part_ml, part_acc, (int64_t)total_q * Hq, n_split, out, st);
 }
 
-// Groups of one and two heads keep all of their weights' bits.
 int launch_attn_bf16(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
-                     const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
+                     const int32_t* kv_len, int32_t B, int32_t total_q, int32_t max_kv, int32_t Hq, int32_t Hkv, float scale,
                      int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st) {
   const int G = Hq / Hkv;
-  if (G != 1 && G != 2 && G != 4 && G != 8) {
-    msa_set_error("msa_sparse_attn: GQA group size %d unsupported (1, 2, 4, 8)", G);
-    return MSA_EINVAL;
-  }
-  const auto launch = G <= 2 ? launch_attn_ring<3> : launch_attn_ring<2>;
+  const auto launch = !takes_ring(total_q, Hkv, max_kv, G) ? launch_attn<bf16_t> : G <= 2 ? launch_attn_ring<3> : launch_attn_ring<2>;
   return launch(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml, part_acc, st);
 }
 
@@ -691,7 +702,7 @@ int launch_attn_bf16(const void* q, const int32_t* cu_q, const void* k, const vo
 extern "C" size_t msa_attn_workspace_bytes(int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D, int32_t max_kv) {
   if (total_q <= 0 || Hq <= 0 || Hkv <= 0 || D <= 0 || max_kv <= 0) return 0;
   // sized for whichever of the kernels has more partials
-  const int splits = std::max(plan_splits(total_q, Hkv, max_kv).n_split, plan_splits_rows(total_q, Hkv, max_kv, MSA_BF16).n_split);
+  const int splits = std::max(plan_splits(total_q, Hkv, max_kv).n_split, plan_splits_rows(total_q, Hkv, max_kv, true).n_split);
   const size_t n = (size_t)total_q * Hq * splits;
   return align_up(n * 2 * sizeof(float), 256) + align_up(n * D * sizeof(float), 256);
 }
@@ -712,7 +723,7 @@ extern "C" int msa_sparse_attn(const void* q, const int32_t* cu_q, const void* k
               "msa_sparse_attn: q, k, v and out must be 16-byte aligned");
   MSA_REQUIRE((int64_t)total_q * Hq < (int64_t)1 << 31 && total_q < 65536 * 32, "msa_sparse_attn: too many rows");
   const bool mfma = dtype == MSA_BF16 && max_sq >= 8;
-  const SplitPlan plan = mfma ? plan_splits(total_q, Hkv, max_kv) : plan_splits_rows(total_q, Hkv, max_kv, dtype);
+  const SplitPlan plan = mfma ? plan_splits(total_q, Hkv, max_kv) : plan_splits_rows(total_q, Hkv, max_kv, dtype == MSA_BF16 && takes_ring(total_q, Hkv, max_kv, Hq / Hkv));
   const int n_split = plan.n_split;
   MSA_REQUIRE(n_split <= 65535, "msa_sparse_attn: max_kv=%d too large", max_kv);
   const size_t need = msa_attn_workspace_bytes(total_q, Hq, Hkv, D, max_kv);
@@ -733,10 +744,10 @@ extern "C" int msa_sparse_attn(const void* q, const int32_t* cu_q, const void* k
     return launch_combine<bf16_t>(part_ml, part_acc, (int64_t)total_q * Hq, n_split, out, st);
   }
   if (dtype == MSA_BF16)
-    return launch_attn_bf16(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml,
-                               part_acc, st);
-  return launch_attn_f32(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml,
-                         part_acc, st);
+    return launch_attn_bf16(q, cu_q, k, v, kv_off, kv_len, B, total_q, max_kv, Hq, Hkv, scale, causal, plan, out, part_ml,
+                            part_acc, st);
+  return launch_attn<float>(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml,
+                            part_acc, st);
 }
 
 extern "C" int msa_decode_attn_fused(const void* qkv, int64_t row_stride, const int64_t* positions, const void* q_norm_w,
@@ -758,7 +769,7 @@ extern "C" int msa_decode_attn_fused(const void* qkv, int64_t row_stride, const 
     msa_set_error("msa_decode_attn_fused: workspace of %zu bytes, need %zu", workspace_bytes, need);
     return MSA_ESIZE;
   }
-  const int n_split = plan_splits_rows(B, Hkv, Lcap, MSA_BF16).n_split;
+  const int n_split = plan_splits_rows(B, Hkv, Lcap, true).n_split;
   const size_t n = (size_t)B * Hq * n_split;
   float* part_ml = static_cast<float*>(workspace);
   float* part_acc = reinterpret_cast<float*>(static_cast<char*>(workspace) + align_up(n * 2 * sizeof(float), 256));

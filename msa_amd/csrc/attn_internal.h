@@ -29,11 +29,21 @@ static inline SplitPlan plan_splits(int64_t total_q, int32_t Hkv, int32_t max_kv
 // evenly over n_split.  The bf16 ring, of which two fit, is cut finer where that does not come out even and leaves 256 keys a split
 // or more (groups of four, us: 24 samples of 2200 to 4400 keys with 2 KV heads in 288 workgroups 28.2, in 528 23.6; but 16 of 256 to
 // 512 with 8, even in 256, 13.4 against 15.1 in 384).
-static inline SplitPlan plan_splits_rows(int64_t total_q, int32_t Hkv, int32_t max_kv, int32_t dtype) {
+static inline SplitPlan plan_splits_rows(int64_t total_q, int32_t Hkv, int32_t max_kv, bool ring) {
   constexpr int kUnits = 256;
   const int64_t pairs = std::max<int64_t>(1, total_q * Hkv), finer = (2 * kUnits + pairs - 1) / pairs;
   const bool even = (kUnits + pairs - 1) / pairs * pairs == kUnits;
-  return plan_splits_for(total_q, Hkv, max_kv, dtype == MSA_BF16 && !even && max_kv >= kMinSplitKeys * finer ? 2 * kUnits : kUnits);
+  return plan_splits_for(total_q, Hkv, max_kv, ring && !even && max_kv >= kMinSplitKeys * finer ? 2 * kUnits : kUnits);
+}
+// The line between the two forms for bf16 rows with G query heads a KV head.  With four and eight the vector units do not keep up
+// with memory; with one they do, and with two nearly: there the ring's own start and end count.  It is ahead with two heads, unless
+// short rows fill the chip several times over, and with one where a wavefront has one step of 32 keys.  On the vector units and in the
+// ring, us, 8 KV heads: two heads, one sample of 4388 keys 16.7 / 11.8, 8 of 500 to 1000 13.1 / 11.2, 16 of 2194 to 4388 53.6 / 47.1;
+// one head, 16 of 32 to 64 keys 6.0 / 4.8, but of 128 to 256 7.8 / 8.6 and of 2194 to 4388 46.3 / 48.4.  64 samples of 64 to 128 keys
+// with 32 KV heads: two heads 24.9 / 29.9, one 22.2 / 29.5 (of 256 to 512 with two 76.9 / 84.4).
+static inline bool takes_ring(int64_t total_q, int32_t Hkv, int32_t max_kv, int G) {
+  const int64_t pairs = total_q * Hkv;
+  return G > 2 || (G == 2 ? pairs <= 512 || max_kv > 1024 : pairs <= 512 && max_kv <= 128);
 }
 
 // flash_attn.hip: bf16 partial pass over split `blockIdx.z` of the keys; writes un-normalised

@@ -180,3 +180,28 @@ def test_split_plans_and_partials(B, L):
         p = torch.softmax((q[b].double()[None] * kk).sum(-1) * 128 ** -0.5, dim=0)
         want = (p[..., None] * vv).sum(0)
         assert ((out[b] - want).abs() <= want.abs() * 2 ** -8 + (p[..., None] * vv.abs()).sum(0) * 2 ** -15).all()
+
+
+# both sides of each line between the ring and the vector units: 512 rows and heads, 128 keys with one head, 1024 with two
+@pytest.mark.parametrize("G,B,L", [(1, 4, 128), (1, 4, 129), (1, 256, 100), (1, 257, 100), (1, 3, 2100), (2, 5, 128), (2, 20, 2048), (2, 256, 90), (2, 257, 90),
+                                   (2, 257, 1024), (2, 257, 1025)])
+def test_small_groups_on_both_sides_of_the_line(G, B, L):
+    """Ragged samples out of one block of keys whose other rows are NaN, one of them empty, one with an infinite value in its last key.
+    Bounds as in the test of the ring."""
+    from msa_amd import ops
+    g = torch.Generator().manual_seed(B + L)
+    q = (2 * torch.randn((B, 2 * G, 128), generator=g)).bfloat16()
+    lens = [L, 0, *(1 + int(x) for x in torch.randint(0, L, (B - 2,), generator=g))]
+    k, v = (torch.full((B * (L + 1), 2, 128), float("nan"), dtype=torch.bfloat16) for _ in range(2))
+    off = [b * (L + 1) for b in range(B)]
+    for o, n in zip(off, lens):
+        k[o:o + n], v[o:o + n] = (torch.randn((n, 2, 128), generator=g).bfloat16() for _ in range(2))
+    v[off[2] + lens[2] - 1, 1, 9] = float("inf")
+    out = ops.sparse_attn(q.cuda(), k.cuda(), v.cuda(), torch.tensor(off).cuda(), torch.tensor(lens, dtype=torch.int32).cuda(), L).cpu().double()
+    for b, (o, n) in enumerate(zip(off, lens)):
+        kk, vv = (t[o:o + n].double().repeat_interleave(G, dim=1) for t in (k, v))
+        p = torch.softmax((q[b].double()[None] * kk).sum(-1) * 128 ** -0.5, dim=0)
+        want, size = (p[..., None] * vv).sum(0), (p[..., None] * vv.abs()).sum(0)
+        fin = torch.isfinite(want)
+        assert fin.all() == (b != 2) and torch.equal(out[b][~fin], want[~fin])
+        assert ((out[b] - want).abs() <= want.abs() * 2 ** -8 + size * 2 ** -15)[fin].all(), (b, n)
