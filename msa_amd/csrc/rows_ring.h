@@ -39,16 +39,16 @@ constexpr int kMaxResidentK = kMaxResident * kWaves * kUnitBytes / 2;
 constexpr int kMinK = 512, kMinRows = 4;
 constexpr int64_t kMinWeights = 3 << 19;
 constexpr int kFar = 0x7ff00000;                   // past every extent, whatever is added: reads zeros, touches no memory
-// slots of a wavefront's ring
 // What happens to the activations in front of the products: nothing, an RMSNorm, or a residual step with the norm of its own (one
 // launch less, but all workgroups read its fp32 operands: seq_rows.hip has the line).
 enum { kPlain, kNormed, kPost };
 constexpr int kMaxPost = 3;                        // units per wavefront that the residual step takes: what its registers hold
-constexpr int slots(int pro) { return pro ? 3 : 2; }
+constexpr int slots(int pro) { return pro ? 3 : 2; }              // of a wavefront's ring
 constexpr int lds_bytes(int pro) {
-  return 2 * kWaves * kPlane * 4 + kWaves * slots(pro) * kUnitSlab + (pro ? kWaves * 16 * 4 : 0) + (pro == kPost ? kWaves * 1024 : 0);
+  return 2 * kWaves * kPlane * 4 + kWaves * slots(pro) * kUnitSlab + (pro ? kWaves * 16 * 4 + kWaves * 1024 : 0);
 }
-static_assert(kMaxPost * 2 * kUnitBytes <= 1024, "one request for a wavefront's part of the residual step's weights");
+static_assert(kMaxPost * 2 * kUnitBytes <= 1024 && kMaxResident * kUnitBytes <= 1024, "one request for a wavefront's part of the norm's weights");
+static_assert(lds_bytes(kNormed) <= 160 * 1024);
 constexpr int kNonTemporal = 2;                    // a step reads a weight once
 
 // vmcnt(n), the other counters not waited for
@@ -158,24 +158,19 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
 #pragma unroll
     for (int u = 0; u < NU; ++u) load_x(xf[u], u);
   }
-  u32x4_t gw[kNorm ? NU : 1][2];
+  // The norm's weights, alike for all rows, through LDS (in registers, five units of them spill: 2560 x 5120 with one row took 13.9
+  // us instead of 8.8)
+  char* norm_lds = lds + lds_bytes(kPro) - (kWaves - wave) * 1024;
   if constexpr (kNorm) {
     const __amdgpu_buffer_rsrc_t rs_g = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.norm_w), 0, row_bytes, 0x00020000);
-#pragma unroll
-    for (int u = 0; u < NU; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int so = u * (kUnitBytes * kWaves) + h * 64;
-        gw[u][h] = __builtin_amdgcn_raw_buffer_load_b128(rs_g, x_col + so < row_bytes ? x_col : kFar, so, 0);
-      }
+    MSA_LOAD_TO_LDS(rs_g, norm_lds, (lane >> 3) * (kUnitBytes * kWaves) + wave * kUnitBytes + (lane & 7) * 16, 0, 0);
   }
-  // The residual step's other operands: the fp32 rows into registers, the weights, alike for all rows, through LDS
+  // The residual step's other operands: the fp32 rows into registers, the weights likewise
   u32x4_t px[kPro == kPost ? NU : 1][2][2];
-  char* post_lds = lds + lds_bytes(kNormed) + wave * 1024;
   if constexpr (kPro == kPost) {
     const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.post_w), 0, 2 * row_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rs_p = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.post_x), 0, a.M * 2 * row_bytes, 0x00020000);
-    MSA_LOAD_TO_LDS(rs_w, post_lds, (lane >> 4) * (2 * kUnitBytes * kWaves) + wave * 2 * kUnitBytes + (lane & 15) * 16, 0, 0);
+    MSA_LOAD_TO_LDS(rs_w, norm_lds, (lane >> 4) * (2 * kUnitBytes * kWaves) + wave * 2 * kUnitBytes + (lane & 15) * 16, 0, 0);
 #pragma unroll
     for (int u = 0; u < NU; ++u)
 #pragma unroll
@@ -199,27 +194,33 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
     if constexpr (!kResident) load_x(xf[i], i);              // (in the loop's order: it counts what is outstanding)
   }
   __builtin_amdgcn_sched_barrier(0);                         // (nothing is computed before everything is requested)
+  // What a norm reads of LDS it reads by hand: the compiler would wait for the ring in front of it, and nor does it wait for the
+  // weights: what the ring has requested by now, 2 kSlots loads, is all that may be outstanding then.  The build checks that.
   if constexpr (kNorm) {
     // RMSNorm folded in: the operand is bf16(x * norm_w); the row's factor commutes with the product and joins at the end
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kSlots) : "memory");
     float ssq = 0.f;
 #pragma unroll
-    for (int u = 0; u < NU; ++u)
+    for (int u = 0; u < NU; ++u) {
+      u32x4_t gw[2];
+      asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:64\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(gw[0]), "=&v"(gw[1]) : "v"(lds_offset(norm_lds) + u * kUnitBytes + g * 16) : "memory");
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const float lo = bf16lo(xf[u][h][c]), hi = bf16hi(xf[u][h][c]);
           ssq += lo * lo + hi * hi;
-          xf[u][h][c] = pack_bf16x2(lo * bf16lo(gw[u][h][c]), hi * bf16hi(gw[u][h][c]));
+          xf[u][h][c] = pack_bf16x2(lo * bf16lo(gw[h][c]), hi * bf16hi(gw[h][c]));
         }
+      asm volatile("" : "+v"(xf[u][0]), "+v"(xf[u][1]), "+v"(ssq));      // (one unit unpacked at a time)
+    }
     ssq += __shfl_xor(ssq, 16);
     ssq += __shfl_xor(ssq, 32);
     if (g == 0) row_ssq[wave * 16 + n_l] = ssq;              // read behind the first barrier
   }
   if constexpr (kPro == kPost) {
-    // x + rms_norm(y) * w as the operand, the sums as in the launch of its own.  (LDS by hand: the compiler would wait for the ring
-    // in front of it, and nor does it wait for the weights: what the ring has requested by now, 2 kSlots loads, is all that may be
-    // outstanding when they are read.  The build checks that.)
+    // x + rms_norm(y) * w as the operand, the sums as in the launch of its own
     float ssq = 0.f;
 #pragma unroll
     for (int u = 0; u < NU; ++u)
@@ -249,7 +250,7 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
         float v[8];
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          const u32x4_t w = lds_read16(lds_offset(post_lds) + u * 2 * kUnitBytes + h * 128 + g * 32 + i * 16);
+          const u32x4_t w = lds_read16(lds_offset(norm_lds) + u * 2 * kUnitBytes + h * 128 + g * 32 + i * 16);
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
             const uint32_t y = xf[u][h][2 * i + (c >> 1)];

@@ -261,3 +261,12 @@ def test_residual_step_waits_for_its_weights():
             if os.path.exists(n):
                 os.remove(n)
     assert len(problems) == 9 and all("Li2EEEv" in p for p in problems), problems
+
+
+def test_build_guard_covers_the_rings():
+    """The kernels that count what their rings have in flight are built without scratch and spills (the folded norm over five units
+    of K once had 17 spilled registers)."""
+    from msa_amd import build as B
+    for source, kernels in (("linear.hip", ["rows_ring_kernel"]), ("seq_rows.hip", ["rows_ring_kernel"]), ("attn.hip", ["attn_ring_kernel", "attn_decode_fused_kernel"])):
+        assert [k for k, _ in B.CONTRACTS[source]] == kernels
+    assert B.check_kernel_contracts(B._device_asm(os.path.join(B.CSRC, "linear.hip")), "rows_ring_kernel") == []
