@@ -318,10 +318,13 @@ __global__ __launch_bounds__(256) void skinny_tile_reduce_kernel(const float* __
 
 // The cut of the tiled form: up to 16 row groups per row block (fewer when the matrix has fewer than 256 groups), as
 // many K slices as keep the launch within one workgroup per compute unit (at most 16); used when it takes at least
-// 8 us less per compute unit than the plain form at ~34 GB/s (the second launch costs ~4 us), and the rows are many: up to eight
-// rows of activations are cheaper to read again than a second launch (2560 x 9728: 12.1 us in the form of rows_ring.h with one
-// row, 13.1 with eight, 16.4 with sixteen; 14.8 to 15.2 in this one).
-constexpr int kTileMinRows = 8;
+// 8 us less per compute unit than the plain form at ~34 GB/s (the second launch costs ~4 us), and the rows are many or the matrix is
+// long: up to eight rows of activations are cheaper to read again than a second launch (2560 x 9728: 12.1 us in the form of
+// rows_ring.h with one row, 13.1 with eight, 16.4 with sixteen; 14.8 to 15.2 in this one), but not for a few hundred rows of weights,
+// of which each workgroup there has four (1024 x 9728: 10.6 and 12.2 us with one and eight rows, 9.8 here; 512 x 8192 8.5 and 10.1, 7.5
+// and 7.7; 1024 x 6144 7.7 and 8.8, 8.5;
+// 2048 x 14336 15.8 and 16.9, 17.6).
+constexpr int kTileMinRows = 8, kTileLong = 7;
 struct TilePlan {
   int n_slices, gpw, row_blocks;
   bool use;
@@ -330,7 +333,7 @@ TilePlan plan_tile(int32_t M, int32_t N, int32_t K) {
   TilePlan t{0, 0, 0, false};
   const int groups = (N + 15) / 16;
   const int steps = K / 32;
-  if (K % 32 != 0 || groups > 256 || M <= kTileMinRows) return t;
+  if (K % 32 != 0 || groups > 256 || (M <= kTileMinRows && K <= (int64_t)kTileLong * N)) return t;
   t.gpw = std::min(kMaxWaves, (groups + 15) / 16);
   t.row_blocks = (groups + t.gpw - 1) / t.gpw;
   t.n_slices = std::min(std::min(kTileMaxSlices, steps), 256 / std::max(1, t.row_blocks));

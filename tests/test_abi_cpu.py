@@ -270,3 +270,14 @@ def test_build_guard_covers_the_rings():
     for source, kernels in (("linear.hip", ["rows_ring_kernel"]), ("seq_rows.hip", ["rows_ring_kernel"]), ("attn.hip", ["attn_ring_kernel", "attn_decode_fused_kernel"])):
         assert [k for k, _ in B.CONTRACTS[source]] == kernels
     assert B.check_kernel_contracts(B._device_asm(os.path.join(B.CSRC, "linear.hip")), "rows_ring_kernel") == []
+
+
+def test_scratch_of_the_decode_products():
+    """K is cut over workgroups, which takes scratch, for more than eight rows, and for fewer where the matrix is more than seven
+    times as long as it has rows."""
+    lib = _lib.load()
+    need = lambda M, N, K: lib.msa_skinny_linear_workspace_bytes(M, N, K)
+    for M, N, K in ((1, 1024, 9728), (8, 176, 14336), (5, 512, 8192), (3, 2032, 14336), (9, 2560, 9728), (16, 1024, 5120)):
+        assert need(M, N, K) > 0, (M, N, K)
+    for M, N, K in ((1, 2560, 9728), (8, 2560, 9728), (8, 1392, 9728), (3, 2048, 14336), (8, 1024, 5120), (16, 2560, 2560)):
+        assert need(M, N, K) == 0, (M, N, K)

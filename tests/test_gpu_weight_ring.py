@@ -107,9 +107,10 @@ def test_recurrence(n, W, more):
     assert torch.all(s1[1] == 0)
 
 
-@pytest.mark.parametrize("M,N,K", [(16, 1600, 5120), (3, 336, 5120), (8, 2560, 9728), (1, 6160, 640), (16, 2576, 1152)])
+@pytest.mark.parametrize("M,N,K", [(16, 1600, 5120), (3, 336, 5120), (8, 2560, 9728), (1, 6160, 640), (16, 2576, 1152), (1, 1040, 7296), (8, 176, 14336),
+                                   (5, 512, 8192)])
 def test_skinny_linear(M, N, K):
-    """Folded norm, silu-mul of whole 16-row groups, residual."""
+    """Folded norm, silu-mul of whole 16-row groups, residual; the last three cut K over workgroups for few rows, too."""
     r = Rand(N + K)
     (x, x_), (w, w_), (nw, nw_), (res, res_) = r(M, K, dtype=BF16, scale=3.0), r(N, K, dtype=BF16, scale=K ** -0.5), r(K, dtype=BF16, scale=0.1, add=1.0), r(M, N, dtype=BF16)
     close(ops.skinny_linear(x, w, residual=res), (x_ @ w_.T) + res_, BF16, 1e-2)
