@@ -7,8 +7,8 @@
 //   k = unit * 32 J + 32 j + 8 g   (one load instruction covers 64 contiguous bytes of each of 16 rows),
 // and the same bytes of x row n (J = 4, or 2 when the RMSNorm is folded in).  The contraction order
 // inside a unit is permuted the same way on both operands, which a dot product does not see.  A workgroup owns R row groups and splits
-// K over its wavefronts; partial sums meet in LDS and are added in wavefront order (deterministic).  Matrices of more than 3 MB
-// with rows of more than 512 elements take the form of rows_ring.h instead.
+// K over its wavefronts; partial sums meet in LDS and are added in wavefront order (deterministic).  Matrices of more than
+// some 10 MB take the form of rows_ring.h instead (takes_ring).
 #include <algorithm>
 
 #include "rows_ring.h"
@@ -186,6 +186,14 @@ __global__ __launch_bounds__(kMaxWaves * 64) void skinny_linear_kernel(
       y[(int64_t)m * y_row_stride + n] = f32_to_bf16(v);
     }
   }
+}
+
+// The line to the form of rows_ring.h (us here and there, one / sixteen rows): 3072 x 1280 3.7 / 4.6 and 4.5 / 5.1, 6144 x 1280 5.5 / 6.1
+// and 5.8 / 6.3, 4096 x 1024 3.6 / 4.3 and 3.9 / 4.3; 2560 x 2560 5.1 / 7.2 and 5.3 / 6.4, 2560 x 2048 4.7 / 5.9 and 4.5 / 5.4,
+// 9728 x 1024 7.4 / 8.4 and 6.3 / 6.7.
+constexpr int64_t kRingWeights = 5 << 20;
+bool takes_ring(int32_t M, int32_t N, int32_t K, bool norm) {
+  return K > rows_ring::kMinK && rows_ring::busy_weights(N, K) >= kRingWeights && (!norm || K <= rows_ring::kMaxResidentK);
 }
 
 // What rows_ring.h's kernel does with a product.
@@ -381,7 +389,7 @@ extern "C" int msa_skinny_linear(const void* x, const void* w, const void* resid
   MSA_REQUIRE(norm_w == nullptr || eps > 0.f, "msa_skinny_linear: folded RMSNorm needs eps > 0");
   hipStream_t st = as_stream(stream);
 
-  if (K > rows_ring::kMinK && (int64_t)N * K >= rows_ring::kMinWeights && (norm_w == nullptr || K <= rows_ring::kMaxResidentK)) {
+  if (takes_ring(M, N, K, norm_w != nullptr)) {
     switch (epilogue) {
       case kEpiPlain: return launch_ring<kEpiPlain>(x, w, residual, norm_w, eps, y, M, N, K, st);
       case kEpiResidual: return launch_ring<kEpiResidual>(x, w, residual, norm_w, eps, y, M, N, K, st);

@@ -34,10 +34,14 @@ constexpr int kWaves = 16, kUnitBytes = 128, kUnitSlab = 16 * kUnitBytes;
 constexpr int kPlane = 272;                        // floats between two wavefronts' partial blocks: four adders hit distinct banks
 constexpr int kMaxResident = 5;                    // units per wavefront whose activations stay in registers
 constexpr int kMaxResidentK = kMaxResident * kWaves * kUnitBytes / 2;
-// The line between the two forms: matrices of less than 3 MB are done within the launch's own time, and rows of up to 512 elements
-// leave half of the sixteen wavefronts without work.
+// The line between the two forms: small matrices are done within the launch's own time, rows of up to 512 elements leave half of the
+// sixteen wavefronts without work, and so do some longer ones in their last round: what counts is the weights times the share of the
+// wavefronts at work.  Each library's products have a line of their own.
 constexpr int kMinK = 512, kMinRows = 4;
-constexpr int64_t kMinWeights = 3 << 19;
+static inline int64_t busy_weights(int64_t N, int64_t K) {
+  const int64_t units = (K * 2 + kUnitBytes - 1) / kUnitBytes, rounds = (units + kWaves - 1) / kWaves;
+  return N * K * units / (rounds * kWaves);
+}
 constexpr int kFar = 0x7ff00000;                   // past every extent, whatever is added: reads zeros, touches no memory
 // What happens to the activations in front of the products: nothing, an RMSNorm, or a residual step with the norm of its own (one
 // launch less, but all workgroups read its fp32 operands: seq_rows.hip has the line).

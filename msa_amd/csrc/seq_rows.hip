@@ -289,9 +289,14 @@ struct RingEnd<MSA_ROWS_GRU> {
   }
 };
 
-// The weight ring's part of the calls (see kMinWeights).
+// The weight ring's part of the calls (us without and with it, one / sixteen rows: 2560 x 1536 4.2 / 5.2 and 4.5 / 5.2, 3072 x 1280 4.0 /
+// 4.9 and 4.6 / 5.1, 2048 x 1024 3.5 / 4.2 and 3.6 / 4.2; 4096 x 1024 4.1 / 4.6 and 4.0 / 4.3, 1024 x 3072 5.3 / 7.2 and 5.1 / 6.9; with
+// fp32 results 512 x 6144 7.0 and 7.4, 768 x 3584 5.3 and 5.6).  From 2048 elements on this file's kernel is short of wavefronts.
+constexpr int64_t kRingWeights = 3 << 20, kLongRingWeights = 3 << 19, kLongK = 2048;
 bool takes_ring(const msa_rows_args& a, int32_t epilogue) {
-  return a.groups == 1 && a.K > rows_ring::kMinK && (int64_t)a.N * a.K >= (epilogue == MSA_ROWS_GRU ? kGruRingWeights : rows_ring::kMinWeights);
+  if (a.groups != 1 || a.K <= rows_ring::kMinK) return false;
+  if (epilogue == MSA_ROWS_GRU) return (int64_t)a.N * a.K >= kGruRingWeights;
+  return rows_ring::busy_weights(a.N, a.K) >= kRingWeights || (epilogue != MSA_ROWS_F32 && a.K >= kLongK && (int64_t)a.N * a.K >= kLongRingWeights);
 }
 
 template <int EPI, int kPro = rows_ring::kPlain>

@@ -12,7 +12,8 @@ from seq_helpers import BF16, F32, Rand, batch, close
 pytestmark = pytest.mark.gpu
 # rows: 3 and 4 a workgroup, 16 and 17, several rounds; K: one unit over a multiple of the wavefronts' 1024, one short, 5 x 1024 (the
 # most that stays in registers), above it with an odd and an even number of rounds
-SHAPES = [(1, 1021, 2056), (16, 1100, 1528), (7, 4097, 1024), (16, 4360, 520), (2, 777, 5120), (3, 2600, 5128), (16, 300, 6152), (5, 4500, 7168), (1, 9000, 1016)]
+SHAPES = [(1, 1021, 2056), (16, 1100, 1528), (7, 4097, 1024), (16, 4360, 520), (2, 777, 5120), (3, 2600, 5128), (16, 300, 6152), (5, 4500, 7168), (1, 9000, 1016),
+          (2, 2049, 2056), (16, 3000, 1528), (9, 14300, 520)]
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
@@ -29,10 +30,10 @@ def test_plain_and_two_operands(M, N, K):
     close(seq_ops.rows_linear(wide[:, :K], w), x_ @ w_.T, BF16, 4e-3)
 
 
-def test_not_finite_weights_stay_in_their_rows():
+@pytest.mark.parametrize("N,K", [(1001, 1640), (1001, 3368), (3001, 1640)])
+def test_not_finite_weights_stay_in_their_rows(N, K):
     """A row of infinities or NaN changes its own column only, also where a workgroup's last rows and a row's last units are empty."""
     r = Rand(3)
-    N, K = 1001, 1640
     (x, x_), (w, w_) = r(5, K, dtype=BF16), r(N, K, dtype=BF16, scale=K ** -0.5)
     for n, v in ((0, float("nan")), (499, float("inf")), (1000, float("nan"))):
         w[n, K - 8:] = v
@@ -44,14 +45,14 @@ def test_not_finite_weights_stay_in_their_rows():
     close(got[:, keep.cuda()], (x_ @ w_.T)[:, keep], F32)
 
 
-@pytest.mark.parametrize("M,ff,K", [(16, 901, 1032), (1, 4100, 1024), (9, 130, 6152)])
+@pytest.mark.parametrize("M,ff,K", [(16, 901, 1032), (1, 4100, 1024), (9, 130, 6152), (16, 3101, 1032)])
 def test_gated_units(M, ff, K):
     r = Rand(ff)
     (x, x_), (g, g_), (u, u_) = r(M, K, dtype=BF16), r(ff, K, dtype=BF16, scale=1.5 * K ** -0.5), r(ff, K, dtype=BF16, scale=1.5 * K ** -0.5)
     close(seq_ops.rows_glu(x, seq_ops.interleave_pairs(g, u), 1.5), O.clamped_glu(x_ @ g_.T, x_ @ u_.T, 1.5), BF16)
 
 
-@pytest.mark.parametrize("M,N,K", [(16, 1100, 1536), (4, 600, 6144)])
+@pytest.mark.parametrize("M,N,K", [(16, 1100, 1536), (4, 600, 6144), (16, 2900, 1536)])
 def test_residual(M, N, K):
     r = Rand(N)
     (x, x_), (w, w_), (g, g_) = r(M, K, dtype=BF16), r(N, K, dtype=BF16, scale=K ** -0.5), r(M, N + 16, dtype=BF16)
@@ -68,10 +69,11 @@ def test_residual(M, N, K):
     close(prev, prev_, F32)
 
 
+@pytest.mark.parametrize("W", [1104, 2064])
 @pytest.mark.parametrize("taps_n", [1, 4, 5])
-def test_convolution(taps_n):
+def test_convolution(taps_n, W):
     r = Rand(taps_n)
-    W, lo, C, n_b, rows = 1104, 40, 1500, 1600, 333
+    lo, C, n_b, rows = 40, 1500, 1600, 333
     (w, _), (taps, _), (b, _) = r(n_b + rows, W, dtype=BF16, scale=1.6 * W ** -0.5), r(C, taps_n), r(C)
     s1, s2 = torch.zeros(4, taps_n - 1, C, device="cuda"), torch.zeros(4, taps_n - 1, C, device="cuda")
     for step in range(6):
@@ -108,9 +110,10 @@ def test_recurrence(n, W, more):
 
 
 @pytest.mark.parametrize("M,N,K", [(16, 1600, 5120), (3, 336, 5120), (8, 2560, 9728), (1, 6160, 640), (16, 2576, 1152), (1, 1040, 7296), (8, 176, 14336),
-                                   (5, 512, 8192)])
+                                   (5, 512, 8192), (3, 1040, 5120), (1, 14000, 640), (16, 9600, 1152)])
 def test_skinny_linear(M, N, K):
-    """Folded norm, silu-mul of whole 16-row groups, residual; the last three cut K over workgroups for few rows, too."""
+    """Folded norm, silu-mul of whole 16-row groups, residual; (1, 1040, 7296) to (5, 512, 8192) cut
+    K over workgroups."""
     r = Rand(N + K)
     (x, x_), (w, w_), (nw, nw_), (res, res_) = r(M, K, dtype=BF16, scale=3.0), r(N, K, dtype=BF16, scale=K ** -0.5), r(K, dtype=BF16, scale=0.1, add=1.0), r(M, N, dtype=BF16)
     close(ops.skinny_linear(x, w, residual=res), (x_ @ w_.T) + res_, BF16, 1e-2)
