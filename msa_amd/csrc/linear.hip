@@ -192,7 +192,12 @@ __global__ __launch_bounds__(kMaxWaves * 64) void skinny_linear_kernel(
 // and 5.8 / 6.3, 4096 x 1024 3.6 / 4.3 and 3.9 / 4.3; 2560 x 2560 5.1 / 7.2 and 5.3 / 6.4, 2560 x 2048 4.7 / 5.9 and 4.5 / 5.4,
 // 9728 x 1024 7.4 / 8.4 and 6.3 / 6.7.
 constexpr int64_t kRingWeights = 5 << 20;
-bool takes_ring(int32_t M, int32_t N, int32_t K, bool norm) {
+// Rows of more than kMaxResidentK are read once per sixteen rows of weights: 24 to 31 a workgroup cost as much as 32, which this file's
+// kernel reads once (sixteen rows of activations: 6144 x 9728 28.5 us here and 31.8 in the ring, 7168 x 5632 19.9 and 21.4; eight 25.3
+// and 26.2; but 8192 x 9728 34.3 and 35.2, 5632 x 9728 in 352 workgroups 38.2 and 31.5).
+constexpr int kTwiceRows = 12, kTwiceFrom = 6144, kTwiceTo = 8192;
+bool takes_ring(int32_t M, int32_t N, int32_t K, bool norm, int32_t epilogue) {
+  if (epilogue != kEpiSiluMul && K > rows_ring::kMaxResidentK && M >= kTwiceRows && N >= kTwiceFrom && N < kTwiceTo) return false;
   return K > rows_ring::kMinK && rows_ring::busy_weights(N, K) >= kRingWeights && (!norm || K <= rows_ring::kMaxResidentK);
 }
 
@@ -389,7 +394,7 @@ extern "C" int msa_skinny_linear(const void* x, const void* w, const void* resid
   MSA_REQUIRE(norm_w == nullptr || eps > 0.f, "msa_skinny_linear: folded RMSNorm needs eps > 0");
   hipStream_t st = as_stream(stream);
 
-  if (takes_ring(M, N, K, norm_w != nullptr)) {
+  if (takes_ring(M, N, K, norm_w != nullptr, epilogue)) {
     switch (epilogue) {
       case kEpiPlain: return launch_ring<kEpiPlain>(x, w, residual, norm_w, eps, y, M, N, K, st);
       case kEpiResidual: return launch_ring<kEpiResidual>(x, w, residual, norm_w, eps, y, M, N, K, st);

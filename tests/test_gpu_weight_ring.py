@@ -110,7 +110,8 @@ def test_recurrence(n, W, more):
 
 
 @pytest.mark.parametrize("M,N,K", [(16, 1600, 5120), (3, 336, 5120), (8, 2560, 9728), (1, 6160, 640), (16, 2576, 1152), (1, 1040, 7296), (8, 176, 14336),
-                                   (5, 512, 8192), (3, 1040, 5120), (1, 14000, 640), (16, 9600, 1152)])
+                                   (5, 512, 8192), (3, 1040, 5120), (1, 14000, 640), (16, 9600, 1152),
+                                   (12, 6144, 5248), (11, 8176, 5248), (16, 8192, 5248)])
 def test_skinny_linear(M, N, K):
     """Folded norm, silu-mul of whole 16-row groups, residual; (1, 1040, 7296) to (5, 512, 8192) cut
     K over workgroups."""
