@@ -24,9 +24,11 @@ constexpr int kVectors = R == 3 ? 2 : 4;
 
 // The element-wise end of product (m, n), `col` its column in the output.  What it reads besides the product is fetched by
 // `load`, which the kernels call before they multiply, so that it arrives with the weights instead of behind the sums; `begin`
-// fetches what the row alone tells.
+// fetches what the row alone tells, `touches` is whether column n takes any of it: in front of rows_linear_kernel's products nothing
+// may be fetched that is not used there, or it is waited for before the weights are requested (3232 x 640: 4.3 us instead of 4.0).
 template <int EPI>
 struct Finish {
+  __device__ __forceinline__ static bool touches(const msa_rows_args&, int) { return true; }
   __device__ __forceinline__ void begin(const msa_rows_args&, int) {}
   __device__ __forceinline__ void load(const msa_rows_args& a, int m, int n) {}
   __device__ __forceinline__ void apply(const msa_rows_args& a, int m, int n, int64_t col, float v) const {
@@ -46,6 +48,7 @@ struct Finish<MSA_ROWS_MAMBA> {
   static constexpr int kTaps = 4;            // more taps than this are read when they are needed
   float keep[kTaps - 1], tap[kTaps], bias;
   int32_t slot;
+  __device__ __forceinline__ static bool touches(const msa_rows_args& a, int n) { return n >= a.conv_lo && n - a.conv_lo < a.conv_n; }
   __device__ __forceinline__ void begin(const msa_rows_args& a, int m) { slot = m < a.M ? a.slot[m] : 0; }
   __device__ __forceinline__ void load(const msa_rows_args& a, int m, int n) {
     const int c = n - a.conv_lo;
@@ -94,6 +97,7 @@ struct Finish<MSA_ROWS_RESIDUAL> {
   float x, bias, w, b, mix, before;
   bf16_t gate;
   int32_t slot;
+  __device__ __forceinline__ static bool touches(const msa_rows_args&, int) { return true; }
   __device__ __forceinline__ void begin(const msa_rows_args& a, int m) { slot = a.shift && m < a.M ? a.slot[m] : 0; }
   __device__ __forceinline__ void load(const msa_rows_args& a, int m, int n) {
     x = a.x_in[(int64_t)m * a.N + n];
@@ -122,6 +126,7 @@ struct Finish<MSA_ROWS_RESIDUAL> {
 // A (gate, up) pair of neighbouring columns, in the lane of the even one.
 template <>
 struct Finish<MSA_ROWS_GLU> {
+  __device__ __forceinline__ static bool touches(const msa_rows_args&, int) { return false; }
   __device__ __forceinline__ void begin(const msa_rows_args&, int) {}
   __device__ __forceinline__ void load(const msa_rows_args& a, int m, int n) {}
   __device__ __forceinline__ void apply(const msa_rows_args& a, int m, int n, float gate, float up) const {
@@ -158,7 +163,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void rows_linear_kernel(msa_rows_ar
   Finish<EPI> fin;                          // of this thread's first output
   {
     const int m = row_of(tid & 255), nr = 16 * (tid >> 8) + col_of(tid & 255);
-    if (tid < R * 256 && m < a.M && nr < rows_w) {
+    if (tid < R * 256 && m < a.M && nr < rows_w && fin.touches(a, n_base + nr)) {
       fin.begin(a, m);
       fin.load(a, m, n_base + nr);
     }
@@ -229,7 +234,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void rows_linear_kernel(msa_rows_ar
       const float v = total(r, i), up = __shfl_xor(v, 4);
       fin.apply(a, m, n, v, up);
     } else {
-      if (o != tid) {
+      if (o != tid && fin.touches(a, n)) {
         fin.begin(a, m);
         fin.load(a, m, n);
       }
