@@ -1196,13 +1196,26 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void score_split_kernel(const 
   }
   __syncthreads();
   const int queries = b1 > b0 ? (b1 - 1) / blocks_per_query - q0 + 1 : 0;
-  for (int i = tid; i < queries * kSplitCols; i += kSplitWaves * 64) {
-    const int n = n0 + i % kSplitCols;
-    const uint32_t key = best[i / kSplitCols][i % kSplitCols];
-    if (n >= C || key == 0) continue;
+  for (int base = wave * 64; base < queries * kSplitCols; base += kSplitWaves * 64) {        // 32 lanes a query
+    const int i = base + lane, n = n0 + l32;
+    const bool in = i < queries * kSplitCols && n < C;
+    uint32_t key = in ? best[i / kSplitCols][l32] : 0u;
     const int64_t row = q0 + i / kSplitCols;
-    if constexpr (kDocMax) atomicMax(&out_key[row * n_docs + chunk_doc[n]], key);
-    else atomicMax(&out_key[row * C + n], key);
+    if constexpr (kDocMax) {
+      // a document's chunks are neighbours: the first of its columns here takes their maximum (one atomic each would queue up where a
+      // few long documents meet many row blocks: 500 chunks of 16 documents x 1000 rows 215 us instead of 41)
+      const int32_t doc = in ? chunk_doc[n] : -1;
+#pragma unroll
+      for (int o = 1; o < kSplitCols; o <<= 1) {
+        const uint32_t other = __shfl_down(key, o, kSplitCols);
+        const int32_t other_doc = __shfl_down(doc, o, kSplitCols);
+        if (l32 + o < kSplitCols && other_doc == doc) key = max(key, other);
+      }
+      const bool first = __shfl_up(doc, 1, kSplitCols) != doc || l32 == 0;
+      if (in && first && key != 0) atomicMax(&out_key[row * n_docs + doc], key);
+    } else {
+      if (in && key != 0) atomicMax(&out_key[row * C + n], key);
+    }
   }
 }
 

@@ -24,9 +24,11 @@ def make(doc_chunks, B, S, seed, host=False):
 
 
 # (largest document, documents, queries, tokens): 1 chunk; 31 to 33 and their neighbours; more row blocks than a workgroup keeps (1 x
-# 1200 tokens: 38 blocks); blocks of many queries; the line to the tiles (chunks x rows = 2^21) from both sides
+# 1200 tokens: 38 blocks); blocks of many queries; the line to the tiles (chunks x rows = 2^21) from both sides;
+# documents of more chunks than a workgroup has, of which it sees several
 @pytest.mark.parametrize("top,docs,B,S", [(1, 1, 1, 1), (1, 31, 2, 33), (1, 32, 1, 64), (1, 33, 3, 70), (9, 40, 1, 1200), (5, 300, 40, 5), (17, 800, 2, 130),
-                                          (16, 2100, 1, 65), (16, 2100, 1, 128), (16, 2040, 1, 128)])
+                                          (16, 2100, 1, 65), (16, 2100, 1, 128), (16, 2040, 1, 128),
+                                          (90, 12, 1, 1000), (40, 16, 3, 70), (33, 30, 2, 64)])
 def test_split_scores(top, docs, B, S):
     from msa_amd import ops
     rng = np.random.default_rng(docs)
