@@ -232,8 +232,9 @@ struct SplitArgs {
 
 // DP / EP: D and E padded to 64, 128 or 256.
 // kOnce: every cache row is read by one row of the step and one tile of heads.  Its values, whole lines, are then read non-temporal,
-// which leaves the caches to the keys, whose lines take two requests (8 key heads of 128, 16 sequences behind up to 4096 tokens: 50.1
-// -> 34.4 us, one 8.7 -> 7.5, 16 behind up to 500 10.4 -> 8.6; with the keys through LDS as well, as whole lines: 36.4, 8.1, 9.0).
+// which leaves the caches to the keys, whose lines take two requests, where there are enough of both for that to matter (8 key heads
+// of 128, us without and with, none of it in a cache before: 16 sequences behind 2048 to 4096 tokens 52 / 45, 4 of them 21.2 / 19.1,
+// 32 behind 128 to 256, 33 MB, 9.7 / 9.0; but 16 of these 7.5 / 7.9, 4 behind 500 to 1000 11.0 / 11.6, one behind 256 6.5 / 6.9).
 template <int DP, int EP, bool kOnce>
 __global__ __launch_bounds__(256) void kv_split_kernel(SplitArgs p, msa_seq_batch b) {
   constexpr int kVS = EP + 8, kUnits = EP / 8, kVP = kStepKeys * kUnits / 64, kK = DP / 32, kC = EP / 16;
@@ -437,9 +438,12 @@ __global__ __launch_bounds__(256) void kv_combine_kernel(SplitArgs p, int64_t it
   }
 }
 
+// The most keys a row sees.
+int64_t kv_span(const msa_kv_attn_args& a) { return std::max<int64_t>(1, a.chunk > 0 ? std::min<int64_t>(a.chunk, a.max_keys) : a.max_keys); }
+constexpr int64_t kOnceBytes = (int64_t)24 << 20;
 // Ranges per row: two workgroups per compute unit, at least two steps per wavefront.
 int kv_splits(const msa_kv_attn_args& a, int32_t rows) {
-  const int64_t span = std::max<int64_t>(1, a.chunk > 0 ? std::min<int64_t>(a.chunk, a.max_keys) : a.max_keys);
+  const int64_t span = kv_span(a);
   const int64_t steps = (span + kStepKeys - 1) / kStepKeys;
   const int64_t blocks = (int64_t)rows * a.G * ((a.H / a.G + kHeadTile - 1) / kHeadTile);
   return (int)std::min<int64_t>(std::min<int64_t>(kMaxSplits, (steps + 7) / 8), std::max<int64_t>(1, (2 * device_compute_units() + blocks - 1) / blocks));
@@ -450,7 +454,8 @@ int launch_split(const SplitArgs& p, const msa_seq_batch& b, hipStream_t st) {
   const msa_kv_attn_args& a = p.a;
   const int tiles = (a.H / a.G + kHeadTile - 1) / kHeadTile;
   const dim3 grid(p.n_split, a.G * tiles, b.rows);
-  if (b.max_rows == 1 && tiles == 1) kv_split_kernel<DP, EP, true><<<grid, 256, 0, st>>>(p, b);
+  const int64_t bytes = kv_span(a) * b.rows * a.G * (a.D + a.E) * 2;
+  if (b.max_rows == 1 && tiles == 1 && bytes >= kOnceBytes) kv_split_kernel<DP, EP, true><<<grid, 256, 0, st>>>(p, b);
   else kv_split_kernel<DP, EP, false><<<grid, 256, 0, st>>>(p, b);
   MSA_LAUNCH_CHECK();
   if (p.n_split > 1) {

@@ -354,6 +354,18 @@ def test_split_attention_long():
         close(seq_ops.kv_attn(q, k, c.v, 0.3, c.batch), want.reshape(3, -1), BF16)
 
 
+@pytest.mark.parametrize("longest", [1535, 1536])
+@pytest.mark.parametrize("H", [8, 24])
+def test_decode_attention_around_24_megabytes(H, longest):
+    """Four sequences of 16 KB a token: from 1536 tokens on their values are read non-temporal."""
+    G, D, E = 8, 128, 128
+    r = Rand(longest)
+    c = Cache(G, D, E, [longest - 1, 40, 700, 1200], [1] * 4, BF16, seed=H)
+    (q, q_), (g, g_) = r(4, H * D, dtype=BF16), r(4, H, dtype=BF16)
+    want = c.attend(q_.view(4, H, D), 0.1, 0) * O.sigmoid(g_)[:, :, None]
+    close(seq_ops.kv_attn(q.view(4, H, D), c.k, c.v, 0.1, c.batch, 0, g), want.reshape(4, -1), BF16)
+
+
 @pytest.mark.parametrize("chunk", [0, 5, 32, 100, 128, 300])
 @pytest.mark.parametrize("H,G,D,E", [(8, 2, 88, 104), (4, 4, 40, 24), (8, 1, 64, 128), (2, 1, 200, 136), (3, 3, 8, 8)], ids=str)
 def test_prefill_attention(H, G, D, E, chunk):
