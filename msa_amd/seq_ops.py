@@ -51,10 +51,10 @@ def _f32(n: int, *ts):
             raise ValueError(f"expected {n} contiguous fp32 values on the device, got {t.dtype} {tuple(t.shape)}")
 
 
-def upload(device, arrays) -> list:
-    """Host arrays (int32 or int64) on the device, in one copy that nothing waits for: out of pinned memory, which the allocator
-    gives out again only once the copy has ended.  (From pageable memory every array is a copy of its own, behind which the host
-    waits for all work in front of it.)"""
+def upload(device, arrays, wait: bool = True) -> list:
+    """Host arrays (int32 or int64) on the device, in one copy out of pinned memory, which the allocator gives out again only once
+    the copy has ended.  Without ``wait`` the host goes on at once and the result is only good for the current stream; with it the
+    copy has ended, behind all work in front of it, and any stream may read."""
     device = torch.device(device)
     places, words = [], 0
     for a in arrays:
@@ -64,7 +64,7 @@ def upload(device, arrays) -> list:
     to = host.numpy()
     for a, at in zip(arrays, places):
         to[at:at + (a.nbytes + 7) // 8].view(a.dtype)[:len(a)] = a
-    dev = host.to(device, non_blocking=True)
+    dev = host.to(device, non_blocking=not wait)
     return [dev[at:at + (a.nbytes + 7) // 8].view(torch.int32 if a.dtype == np.int32 else torch.int64)[:len(a)]
             for a, at in zip(arrays, places)]
 
@@ -72,9 +72,9 @@ def upload(device, arrays) -> list:
 class StepBatch:
     """Device-side description of a step's rows (``msa_seq_batch``): ``counts[s]`` new tokens of the sequence in
     ``slots[s]`` that has already been fed ``positions[s]`` tokens.  ``extra`` int64 arrays go to the device with it
-    (``self.extra``)."""
+    (``self.extra``).  ``wait`` as in :func:`upload`: without it the description is for the current stream alone."""
 
-    def __init__(self, counts: Sequence[int], slots: Sequence[int], positions: Sequence[int], device, extra=()):
+    def __init__(self, counts: Sequence[int], slots: Sequence[int], positions: Sequence[int], device, extra=(), wait: bool = True):
         n = len(counts)
         if not n or min(counts) < 1 or len(set(slots)) != n:
             raise ValueError("a step needs at least one token per sequence and one slot each")
@@ -83,10 +83,11 @@ class StepBatch:
         host = [0]
         for c in counts:
             host.append(host[-1] + c)
+        zeros = torch.zeros(self.rows, dtype=torch.int32, device=device) if n == 1 else None      # (in front of the copy, which may wait)
         many = [] if n == 1 else [np.repeat(np.arange(n, dtype=np.int32), self.counts)]
         self.cu, self.slot, self.pos, *rest = upload(device, [np.asarray(host, np.int32), np.asarray(self.slots, np.int32),
-                                                              np.asarray(self.positions, np.int64), *many, *extra])
-        self.row_seq = rest.pop(0) if many else torch.zeros(self.rows, dtype=torch.int32, device=device)
+                                                              np.asarray(self.positions, np.int64), *many, *extra], wait)
+        self.row_seq = rest.pop(0) if many else zeros
         self.extra = rest
         self.c = _lib.SeqBatch(ptr(self.cu), ptr(self.row_seq), ptr(self.slot), ptr(self.pos), n, self.rows, self.max_rows, 0)
         self.ref = C.byref(self.c)

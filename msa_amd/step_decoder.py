@@ -134,7 +134,7 @@ class StepDecoder:
             rows += [at + w for w in want]
             at += len(ts)
         batch = seq_ops.StepBatch(counts, [cache.slot_of[k] for k, _, _ in entries], [cache.length[k] for k, _, _ in entries],
-                                  self.device, (np.concatenate([t.numpy() for _, t, _ in entries]), np.asarray(rows, np.int64)))
+                                  self.device, (np.concatenate([t.numpy() for _, t, _ in entries]), np.asarray(rows, np.int64)), wait=False)
         logits = self.forward_rows(batch.extra[0], batch, cache, rows, index=batch.extra[1])
         for key, ts, _ in entries:
             cache.advance(key, len(ts))

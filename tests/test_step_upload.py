@@ -1,4 +1,4 @@
-"""A step's description goes to the device in one copy that nothing waits for: contents and lifetime."""
+"""A step's description goes to the device in one copy: contents, lifetime, and who may read it when."""
 import numpy as np
 import pytest
 import torch
@@ -13,6 +13,46 @@ def check(b, counts, slots, pos, extra):
     assert [e.tolist() for e in b.extra] == [list(e) for e in extra]
     assert b.cu.dtype == b.slot.dtype == b.row_seq.dtype == torch.int32 and b.pos.dtype == torch.int64
     assert all(t.data_ptr() % t.element_size() == 0 for t in (b.cu, b.slot, b.pos, b.row_seq, *b.extra))
+
+
+def test_only_a_step_does_not_wait(monkeypatch):
+    """A description is complete when it is handed out, for any stream; a model's own step, which reads it on the stream it was made
+    on, asks for no wait."""
+    asked, to = [], torch.Tensor.to
+
+    def spy(self, *a, **k):
+        if "non_blocking" in k:
+            asked.append(k["non_blocking"])
+        return to(self, *a, **k)
+    monkeypatch.setattr(torch.Tensor, "to", spy)
+    seq_ops.StepBatch([2, 1], [0, 1], [0, 0], "cpu")
+    assert asked == [False]
+    asked.clear()
+    seq_ops.StepBatch([2, 1], [0, 1], [0, 0], "cpu", wait=False)
+    assert asked == [True]
+    from types import SimpleNamespace
+    from msa_amd.step_decoder import StepDecoder
+    cache = SimpleNamespace(length={}, slot_of={}, reserve=lambda n: None, advance=lambda k, n: None)
+    cache.open = lambda k: (cache.length.setdefault(k, 0), cache.slot_of.setdefault(k, len(cache.slot_of)))
+    model = SimpleNamespace(config=SimpleNamespace(vocab=9), device="cpu", forward_rows=lambda tokens, batch, *a, **k: tokens)
+    asked.clear()
+    assert StepDecoder.step(model, cache, [("a", [1, 2], [1]), ("b", [3], [0])]).tolist() == [1, 2, 3] and asked == [True]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts", [[4], [2, 3, 1]])
+def test_other_streams_may_read_a_description(counts):
+    """Made on a stream with a long queue, read on another one at once."""
+    busy, other = torch.cuda.Stream(), torch.cuda.Stream()
+    a = torch.randn(8192, 8192, device="cuda")
+    torch.cuda.synchronize()
+    for i in range(3):
+        with torch.cuda.stream(busy):
+            for _ in range(4):
+                a = torch.mm(a, a) * 1e-4
+            b = seq_ops.StepBatch(counts, [i + s for s in range(len(counts))], [7 * i] * len(counts), "cuda")
+        with torch.cuda.stream(other):
+            check(b, counts, [i + s for s in range(len(counts))], [7 * i] * len(counts), ())
 
 
 @pytest.mark.parametrize("counts", [[1], [5], [3, 1], [2, 7, 1], [1] * 16])
@@ -30,6 +70,6 @@ def test_pinned_memory_outlives_the_copies():
     for _ in range(8):
         a = torch.mm(a, a) * 1e-4
     extra = [(np.full(1000, i, np.int64),) for i in range(40)]
-    batches = [seq_ops.StepBatch([2, 3], [i, i + 1], [i, 0], "cuda", extra[i]) for i in range(40)]
+    batches = [seq_ops.StepBatch([2, 3], [i, i + 1], [i, 0], "cuda", extra[i], wait=False) for i in range(40)]
     for i, b in enumerate(batches):
         check(b, [2, 3], [i, i + 1], [i, 0], extra[i])
