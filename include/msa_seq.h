@@ -178,6 +178,9 @@ typedef struct {
   int32_t reserved;
 } msa_delta_args;
 int msa_seq_delta_scan(const msa_delta_args* args, int32_t dtype, const msa_seq_batch* batch, void* stream);
+/* A chunked portion is prepared in segments, of which two are in the workspace: of up to 88 MB, for n_seq sequences of up to
+ * min(n_seq, 4) * 88 MB (or a chunk of all of them).  Two segments of 88 MB will do for several sequences as well, in up to 1.5
+ * times the time; anything smaller than what the portion takes then is refused. */
 size_t msa_seq_delta_chunked_workspace_bytes(const msa_delta_args* args, int32_t max_rows, int32_t n_seq);
 int msa_seq_delta_chunked(const msa_delta_args* args, const msa_seq_batch* batch, void* workspace, size_t workspace_bytes, void* stream);
 

@@ -802,12 +802,21 @@ int64_t unit_bytes(int32_t D, int32_t E) {
     default: return Layout<128>::bytes(E);
   }
 }
-// Chunks of a segment: enough to be worth a launch, few enough to overlap, at most what the workspace holds.
-int segment(const msa_delta_args& a, int32_t max_rows, int32_t n_seq) {
+// Chunks of a segment: enough to be worth a launch, few enough to overlap, at most `most_bytes`.
+int segment(const msa_delta_args& a, int32_t max_rows, int32_t n_seq, int64_t most_bytes) {
   const int64_t chunks = (max_rows + kC - 1) / kC, per = unit_bytes(a.D, a.E) * a.H * n_seq;
-  const int64_t most = std::max<int64_t>(1, kMaxSegment * std::min(n_seq, kMaxSegments) / per), want = std::max<int64_t>(kLeastChunks, (chunks + kSegments - 1) / kSegments);
+  const int64_t most = std::max<int64_t>(1, most_bytes / per), want = std::max<int64_t>(kLeastChunks, (chunks + kSegments - 1) / kSegments);
   const int64_t parts = (chunks + std::min(most, want) - 1) / std::min(most, want);
   return (int)((chunks + parts - 1) / parts);
+}
+
+int segment(const msa_delta_args& a, int32_t max_rows, int32_t n_seq) {
+  return segment(a, max_rows, n_seq, kMaxSegment * std::min(n_seq, kMaxSegments));
+}
+// Two segments where there are more than one.
+size_t workspace_bytes_of(const msa_delta_args& a, int32_t max_rows, int32_t n_seq, int seg) {
+  const int chunks = (max_rows + kC - 1) / kC;
+  return (size_t)unit_bytes(a.D, a.E) * a.H * n_seq * seg * (seg < chunks ? 2 : 1);
 }
 
 template <int DP, int CT>
@@ -842,8 +851,7 @@ int launch_chunked(const ChunkArgs& c, const msa_seq_batch& b, hipStream_t st) {
 
 extern "C" size_t msa_seq_delta_chunked_workspace_bytes(const msa_delta_args* args, int32_t max_rows, int32_t n_seq) {
   if (!args || max_rows <= 0 || n_seq <= 0 || args->H <= 0 || args->D <= 0 || args->D > 128 || args->E <= 0) return 0;
-  const int chunks = (max_rows + kC - 1) / kC, seg = segment(*args, max_rows, n_seq);
-  return (size_t)unit_bytes(args->D, args->E) * args->H * n_seq * seg * (seg < chunks ? 2 : 1);
+  return workspace_bytes_of(*args, max_rows, n_seq, segment(*args, max_rows, n_seq));
 }
 
 extern "C" int msa_seq_delta_chunked(const msa_delta_args* args, const msa_seq_batch* batch, void* workspace, size_t workspace_bytes, void* stream) {
@@ -857,11 +865,14 @@ extern "C" int msa_seq_delta_chunked(const msa_delta_args* args, const msa_seq_b
                   a.gate_stride >= (int64_t)a.H * a.E && a.qkv_stride % 8 == 0 && a.a_stride % 2 == 0 && a.qkv_stride < (1 << 21) && a.a_stride < (1 << 21) &&
                   (int64_t)a.H * a.E < (1 << 21) && (((uintptr_t)a.qkv | (uintptr_t)workspace) & 15) == 0 && ((uintptr_t)a.a & 3) == 0 && ((uintptr_t)a.dt_bias & 7) == 0,
               "msa_seq_delta_chunked: strides or alignment");
-  if (workspace_bytes < msa_seq_delta_chunked_workspace_bytes(args, batch->max_rows, batch->n_seq)) {
+  // A smaller workspace is taken down to two segments of one sequence's size.
+  int seg = segment(a, batch->max_rows, batch->n_seq);
+  if (workspace_bytes < workspace_bytes_of(a, batch->max_rows, batch->n_seq, seg)) seg = segment(a, batch->max_rows, batch->n_seq, kMaxSegment);
+  if (workspace_bytes < workspace_bytes_of(a, batch->max_rows, batch->n_seq, seg)) {
     msa_set_error("msa_seq_delta_chunked: workspace of %zu bytes is too small", workspace_bytes);
     return MSA_ESIZE;
   }
-  const ChunkArgs c{a, static_cast<char*>(workspace), unit_bytes(a.D, a.E), 0, segment(a, batch->max_rows, batch->n_seq)};
+  const ChunkArgs c{a, static_cast<char*>(workspace), unit_bytes(a.D, a.E), 0, seg};
   MSA_REQUIRE((int64_t)a.H * batch->n_seq * std::max<int64_t>(2 * c.seg, (a.E + 15) / 8) < ((int64_t)1 << 30), "msa_seq_delta_chunked: step too large");
   hipStream_t st = as_stream(stream);
   const int tiles = (a.D + 31) / 32;

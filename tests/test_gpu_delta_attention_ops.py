@@ -1,5 +1,7 @@
 """The kernels of the channel-wise delta rule, rotary chunk attention, clamped gated units and output-normed residuals against the
 plain float64 mechanisms of oracle/delta_attention_layers.py: each alone, in portions, in ragged batches, in fp32 and bf16."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -243,6 +245,35 @@ def test_delta_chunked_in_segments():
         states.append(state)
     close(outs[1], outs[0], BF16)
     close(states[1], states[0], F32, 2e-4)
+
+
+def test_delta_chunked_in_a_small_workspace():
+    """Several sequences in a workspace of two segments of 88 MB: the same results as in the one asked for, four times as large; less
+    is refused."""
+    H, G, D, E, lens = 32, 4, 128, 128, [3000, 1700, 2900, 64, 2500]
+    g = torch.Generator(device="cuda").manual_seed(3)
+    T, n = sum(lens), len(lens)
+    bf = lambda *s: torch.randn(s, generator=g, device="cuda").to(BF16)
+    qkv, a, b, gate = bf(T, 2 * G * D + H * E), bf(T, H * D), bf(T, H), bf(T, H * E)
+    A_log, bias, norm = torch.rand(H, device="cuda"), torch.randn(H * D, device="cuda") - 3, torch.ones(E, device="cuda")
+    bt, lib = batch(lens, list(range(n))), _lib.load_seq()
+
+    def run(size):
+        out, state = torch.empty((T, H * E), dtype=BF16, device="cuda"), torch.zeros(n, H, D, E, device="cuda")
+        c = _lib.DeltaArgs(*(t.data_ptr() for t in (qkv, a, b, gate)), *(t.stride(0) for t in (qkv, a, b, gate)),
+                           *(t.data_ptr() for t in (A_log, bias, norm, state, out)), H, G, D, E, 1e-5, 0)
+        need = lib.msa_seq_delta_chunked_workspace_bytes(C.byref(c), max(lens), n)
+        ws = torch.empty(need if size is None else size, dtype=torch.uint8, device="cuda")
+        rc = lib.msa_seq_delta_chunked(C.byref(c), bt.ref, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+        return rc, need, out, state, lib.msa_seq_delta_chunked_workspace_bytes(C.byref(c), 64, n)
+    rc, need, out, state, chunk = run(None)
+    chunks, most = -(-max(lens) // 64), (88 << 20) // chunk                  # (at least 22 chunks or a sixth of them are wanted: more than fit)
+    parts = -(-chunks // most)
+    small = 2 * chunk * -(-chunks // parts)
+    assert rc == 0 and most < 22 and small <= 2 * (88 << 20) and need > 2 * small
+    rc, _, out2, state2, _ = run(small)
+    assert rc == 0 and torch.equal(out, out2) and torch.equal(state, state2)
+    assert run(small - 16)[0] == -3 and b"workspace" in lib.msa_last_error()
 
 
 def test_delta_chunked_segments_of_a_ragged_batch():
