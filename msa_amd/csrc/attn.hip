@@ -36,6 +36,17 @@ __device__ __forceinline__ void ld8(const float* p, float (&x)[8]) {
   x[4] = __uint_as_float(b.x); x[5] = __uint_as_float(b.y); x[6] = __uint_as_float(b.z); x[7] = __uint_as_float(b.w);
 }
 
+// The same of any float: the rotary tables need not be aligned.
+__device__ __forceinline__ void ld8_any(const float* p, float (&x)[8]) {
+  typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));
+  const f32x4_any_t a = *reinterpret_cast<const f32x4_any_t*>(p), b = *reinterpret_cast<const f32x4_any_t*>(p + 4);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = a[i];
+    x[4 + i] = b[i];
+  }
+}
+
 // Finds the sample owning query row `row` in cu_q (B is small: linear scan is fine and uniform).
 __device__ __forceinline__ int find_sample(const int32_t* cu_q, int B, int row) {
   int b = 0;
@@ -482,8 +493,8 @@ struct NormRope {
     w = *reinterpret_cast<const uint4*>(weight);
   }
   __device__ __forceinline__ void load_rotary(const float* cos_row, const float* sin_row, int j) {
-    ld8(cos_row + 8 * (j & 7), cs);
-    ld8(sin_row + 8 * (j & 7), sn);
+    ld8_any(cos_row + 8 * (j & 7), cs);
+    ld8_any(sin_row + 8 * (j & 7), sn);
   }
   __device__ __forceinline__ uint4 result(float eps, int j) const {
     const uint32_t xs[4] = {x.x, x.y, x.z, x.w}, ws[4] = {w.x, w.y, w.z, w.w};

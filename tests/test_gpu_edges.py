@@ -250,6 +250,11 @@ def test_decode_attn_fused_equals_the_separate_launches(ops, Hq, Hkv):
     assert l2.cpu().tolist() == l1.cpu().tolist() == [min(n + 1, Lcap) for n in lens]
     assert torch.equal(kc2, kc1) and torch.equal(vc2, vc1)
     assert cf.rel_err(got.cpu(), want.cpu()) < 2e-3
+    # rotary tables that begin at any float
+    odd = [torch.cat([t.new_zeros(1), t.flatten()])[1:].view_as(t) for t in rope]
+    kc3, vc3, l3 = kc0.clone(), vc0.clone(), torch.tensor(lens, dtype=torch.int32).cuda()
+    assert all(t.data_ptr() % 16 == 4 for t in odd)
+    assert torch.equal(ops.decode_attn_fused(qkv, Hq, Hkv, D, pos, qw, kw, 1e-6, odd, kc3, vc3, l3), got) and torch.equal(kc3, kc2)
     # and against the oracle from the raw projection output (sample 5: a long row; sample 0: the token alone)
     for b in (0, 5, 9):
         n = int(l2[b])
