@@ -429,17 +429,23 @@ extern "C" int msa_rows_linear(const msa_rows_args* args, int32_t epilogue, void
 }
 
 // The residual step is folded where its operands are few: every workgroup reads all of them, six bytes an element where the product
-// alone reads two.  Up to 8192 elements that is worth less than a launch (with the product, us, folded against separate: 1 row of
-// 1024 7.6 / 8.4 and 6.8 / 7.7, 8 rows 7.9 / 8.6 and 7.5 / 7.9, 4 of 2048 11.2 / 11.1, 2 of 2560 21.6 / 22.0 and 11.5 / 12.1), beyond
-// it is not (4 of 2560 12.5 / 12.3, 16 of 1024 9.1 / 8.9, 16 of 2560 28.0 / 22.7).  The separate launch also works in place and takes
-// rows that the ring's registers do not hold.
-constexpr int kMaxPostElements = 8192;
+// alone reads two, and waits for a second reduction.  That is worth less than a launch up to 8192 elements in rows of one unit a
+// wavefront, and in longer ones up to 6144 if the product is no short one itself (with the product, us, folded against separate: 1 and 8
+// rows of 1024 with 3104 x 1024 6.0 / 6.4 and 6.7 / 6.7, 3 of 2048 with 6144 x 2048 9.7 / 9.9, 2 of 2560 with 6144 x 2560 11.5 / 11.8; but
+// 3 of 2560 with 3104 x 2560 10.2 / 8.9, 4 of 2048 with 1024 x 2048 8.3 / 7.6, 5 of 1280 with 6144 x 1280 and the convolution 10.3 / 9.7,
+// 16 of 2560 28.0 / 22.7).  The separate launch also works in place and takes rows that the ring's registers do not hold.
+constexpr int kMaxPostElements = 8192, kMaxLongPostElements = 6144, kPostRow = rows_ring::kWaves * rows_ring::kUnitBytes / 2;
+constexpr int64_t kMinLongPostWeights = 12 << 20;
+bool worth_folding(const msa_rows_args& a) {
+  const int64_t elements = a.M * (int64_t)a.K;
+  return a.K <= kPostRow ? elements <= kMaxPostElements : elements <= kMaxLongPostElements && (int64_t)a.N * a.K >= kMinLongPostWeights;
+}
 extern "C" int msa_rows_linear_post(const msa_rows_args* args, int32_t epilogue, const msa_rows_post* post, void* stream) {
   MSA_REQUIRE(args && post && post->x_in && post->x_out && post->w && post->h && post->eps >= 0.f, "msa_rows_linear_post: null arguments");
   msa_rows_args a = *args;
   MSA_REQUIRE(a.x && a.M > 0 && a.M <= 16 && a.K > 0 && a.groups == 1 && a.x_stride >= a.K && a.n_b >= a.N,
               "msa_rows_linear_post: M=%d (1..16) K=%d groups=%d n_b=%d", a.M, a.K, a.groups, a.n_b);
-  const bool folds = (epilogue == MSA_ROWS_PLAIN || epilogue == MSA_ROWS_MAMBA || epilogue == MSA_ROWS_GLU) && takes_ring(a, epilogue) && a.M * (int64_t)a.K <= kMaxPostElements && a.K % 8 == 0 &&
+  const bool folds = (epilogue == MSA_ROWS_PLAIN || epilogue == MSA_ROWS_MAMBA || epilogue == MSA_ROWS_GLU) && takes_ring(a, epilogue) && worth_folding(a) && a.K % 8 == 0 &&
                      a.K <= rows_ring::kMaxPost * rows_ring::kWaves * rows_ring::kUnitBytes / 2 && post->x_in != post->x_out &&
                      (((uintptr_t)post->x_in | (uintptr_t)post->x_out | (uintptr_t)post->w) & 15) == 0;
   if (folds) return rows_entry(a, epilogue, post, stream);
