@@ -1,10 +1,11 @@
 // GQA attention of ragged query rows over per-sample KV ranges (decode and stage-2 prefill).
 //
-// Split-KV: workgroup (query row, KV head, split) streams its slice of K and V once and serves all
-// G query heads of that KV head from the same loads.  A wavefront takes 4 keys per step (16 lanes
-// per key, 8 head-dim elements per lane); every (key slot, dim slice) lane keeps an independent
-// online-softmax state (m, l, acc[G][8]) that is merged across slots, wavefronts and finally
-// splits (second kernel).  K / V rows are [Hkv, 128].
+// Split-KV: workgroup (query row, KV head, split) streams its slice of K and V once and serves all G query heads of that KV head from
+// the same loads; splits are merged by a second kernel.  K / V rows are [Hkv, 128].  Two forms: bf16 rows go through a ring in LDS and
+// the matrix cores (attn_ring_kernel, below), fp32 rows and some bf16 rows of one and two heads through the vector units
+// (attn_partial_kernel; takes_ring in attn_internal.h has the line).  In the latter a wavefront takes 4 keys per step (16 lanes per
+// key, 8 head-dim elements per lane); every (key slot, dim slice) lane keeps an online-softmax state (m, l, acc[G][8]) of its own that
+// is merged across slots and wavefronts.
 #include "attn_internal.h"
 
 namespace {
@@ -131,9 +132,9 @@ __device__ __forceinline__ void attend_keys(const T* __restrict__ k, const T* __
 // of 256 bytes arrive by direct-to-LDS loads, four whole rows an instruction, non-temporal (a decode step reads every cache row
 // once), their 16-byte units XORed with the row against bank conflicts.  S^T = K Q^T (16 keys x 16 heads, of which G exist) leaves
 // the scores where P^T is wanted as the operand of O^T = V^T P^T; V^T comes by transposing LDS reads.  What bounds it is HBM for long
-// contexts (8 KV heads: 16 samples of 32768 keys 353 us, 6.1 TB/s; 16 of 2194 to 4388 keys 52.3 -> 47.9 us; one of 4388 17.5 -> 11.9)
-// and the chain lengths - first step - sums - combining launch for short ones (one sample of 256 keys 9.5 -> 8.8 us): the form
-// before held K and V in registers and took packed dot products on the vector units, 350 instructions per 8 KB.
+// contexts (decode steps, 8 KV heads of four: 16 samples of 32768 keys 354 us, 6.1 TB/s; 16 of 2194 to 4388 keys 53.0 -> 47.8 us; one
+// of 4388 18.1 -> 12.6) and the chain lengths - first step - sums - combining launch for short ones (one sample of 256 keys 11.2 -> 9.7
+// us): the form before held K and V in registers and took packed dot products on the vector units, 350 instructions per 8 KB.
 // ------------------------------------------------------------------------------------------------
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
@@ -747,8 +748,8 @@ extern "C" int msa_sparse_attn(const void* q, const int32_t* cu_q, const void* k
   float* part_acc = reinterpret_cast<float*>(static_cast<char*>(workspace) + align_up(n * 2 * sizeof(float), 256));
   hipStream_t st = as_stream(stream);
   if (mfma) {
-    // bf16 query blocks: MFMA partial pass (K / V tiles through LDS) + the common combine; single rows
-    // (decode) stay on the split-KV kernel below, which keeps more loads in flight per wavefront
+    // bf16 query blocks: MFMA partial pass (K / V tiles through LDS, shared by a tile's rows) + the common combine; single rows
+    // (decode) share nothing between them and take the split-KV forms of this file
     int rc = flash_attn_split_launch(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, part_ml,
                                      part_acc, st);
     if (rc != MSA_OK) return rc;

@@ -11,7 +11,8 @@ from seq_helpers import BF16, F32, Rand, batch, close
 
 pytestmark = pytest.mark.gpu
 # rows: 3 and 4 a workgroup, 16 and 17, several rounds; K: one unit over a multiple of the wavefronts' 1024, one short, 5 x 1024 (the
-# most that stays in registers), above it with an odd and an even number of rounds
+# most that stays in registers), above it with an odd and an even number of rounds (some of the smaller matrices lie below the ring's
+# line and cover the form beside it)
 SHAPES = [(1, 1021, 2056), (16, 1100, 1528), (7, 4097, 1024), (16, 4360, 520), (2, 777, 5120), (3, 2600, 5128), (16, 300, 6152), (5, 4500, 7168), (1, 9000, 1016),
           (2, 2049, 2056), (16, 3000, 1528), (9, 14300, 520)]
 
