@@ -1,108 +1,134 @@
 #!/usr/bin/env python3
 """Writes ``scan_asm.inc``: the instruction-level K step of the large-tile routing scan (``score_scan4_kernel``).
 
-The scan's 256 x 256 tile is computed by four wavefronts, one per SIMD, 128 x 128 each: sixteen 32 x 32
-accumulators in the 256 accumulation registers a0-a255, operand fragments double-buffered in v128-v191.  One K step
-(64 elements of K: 64 MFMAs per wavefront) is one asm statement whose issue order is fixed here:
+The scan's 256 x 256 tile is computed by four wavefronts, one per SIMD, 128 x 128 each: 8 x 8 blocks of 16 x 16 in the 256
+accumulation registers a0-a255, eight fragments of each operand in v128-v191.  One K step (64 elements of K) is one asm statement
+whose issue order is fixed here: two sub-steps of 64 ``v_mfma_f32_16x16x32_bf16`` (the 32 x 32 x 16 form costs more power a FLOP: it
+passes an accumulator twice as often for the same products, and these loops run at the clock the power allows).
 
-* sub-step s (16 MFMAs on fragment slot s & 1) carries the eight LDS reads of sub-step s + 1 behind its first eight
-  MFMAs, one read per MFMA;
-* the eight 1 KB blocks of the K_r tile two steps ahead are requested during sub-step 0 and those of the query tile
-  two steps ahead during sub-step 3, one ``buffer_load_dwordx4 ... lds`` behind every second MFMA (the compute unit's
-  address unit takes about that long per load of four wavefronts), M0 set one instruction earlier;
-* the step's only wait for memory (everything but the eight newest loads) and the workgroup barrier sit at the start
-  of sub-step 3, the barrier behind that sub-step's first MFMA so that the matrix pipe runs while the wavefronts meet;
-  behind the barrier the stages this step has finished with are refilled and the first fragments of the next step
-  are read.
+* A sub-step walks over the four quadrants (half of the A fragments x half of the B fragments, sixteen MFMAs each) so that
+  neighbouring quadrants share a half and every half's last use comes a quadrant or two before its successor's first: the
+  fragments are single-buffered.  Each quadrant requests the four that the next but none needs (one read behind each of its MFMAs
+  1 - 4) and begins with the four that arrived last changing slowest, so that each wait covers one read and has had at least
+  sixteen MFMAs' time; the other operand goes to and fro, so that neighbouring MFMAs share an operand.
+* The eight 1 KB blocks of the K_r tile two steps ahead are requested during the first two quadrants and those of the query tile two
+  steps ahead during the last two, one ``buffer_load_dwordx4 ... lds`` behind every fourth MFMA (the compute unit's address unit
+  takes about that long per load of four wavefronts), M0 set one instruction earlier.
+* The step's only wait for memory (everything but the eight newest loads) and the workgroup barrier sit at the start of the last but
+  one quadrant, the barrier behind its first MFMA so that the matrix pipe runs while the wavefronts meet; behind the barrier the
+  stages this step has finished with are refilled and the first fragments of the next step are read.
 
 LDS: two stages of the query tile at 0 / 0x8000, three of the K_r tile at 0x10000 / 0x18000 / 0x20000, rows of 128
 bytes whose 16-byte units are XOR-swizzled by (row >> 1) & 7.
 
 Registers the statements own (the kernel's compiler-allocated code stays below v128 and uses no accumulation
-registers): v128-v159 / v160-v191 fragment slots (A0-A3, B0-B3), v192-v199 LDS addresses of the step, v200-v207
-per-lane LDS offsets of sub-steps 0-3 (A, then B), v208-v215 global offsets of the wavefront's eight 1 KB blocks,
-v216-v223 tile pool and prefetch values (see the kernel), v224-v239 the maxima of the sixteen accumulator blocks of
-the tile just finished (block (i, j) in v224 + 4 i + j; in the folding form the maxima over the four row blocks, column
-block j in v224 + j), v240-v247 scratch of the reduction and the fold, v248-v252 per-lane constants of the fold,
+registers): v128-v159 fragments A0-A7, v160-v191 B0-B7, v192-v197 LDS addresses of the step, v198-v201 per-lane LDS offsets of the
+two sub-steps (A, then B), v208-v215 global offsets of the wavefront's eight 1 KB blocks, v216-v223 tile pool and prefetch values
+(see the kernel), v224-v231 the maxima of the tile just finished (row block of 32 rows i and column group of 64 columns p in
+v224 + 2 i + p, lane l column 64 p + l; in the folding form the maxima over all rows, column group p in v224 + p), v232-v239 their
+parts before the lanes are joined, v240-v247 scratch of the reduction and the fold, v248-v252 per-lane constants of the fold,
 s76-s95 scratch.
 
-The reduction of a finished tile (per lane the maximum of each block's sixteen values: sixteen reads of accumulation
-registers and eight three-way maxima per block) rides in the first sub-step of the next tile's first K step, block
-(i, j) in front of the MFMA that overwrites it: with one wavefront per SIMD the matrix pipe runs under it.  When the
-wavefront's four row blocks belong to one query whose rows all count and the tile lies inside the bank, the fold of the
-column maxima over the chunks of a document (half-wave swap, order-preserving key, segmented max-scan over the 64
+The reduction of a finished tile (per lane the maximum of each block's four values, then of the blocks below it, then over the four
+lanes that hold a column: two half-wave swaps and a swap of rows of sixteen for four column blocks) rides in the first sub-step of
+the next tile's first K step, a block in front of the MFMA that overwrites it: with one wavefront per SIMD the matrix pipe runs
+under it.  When the wavefront's rows belong to one query and all count and the tile lies inside the bank, the fold of the
+column maxima over the chunks of a document (order-preserving key, segmented max-scan over the 64
 lanes by row moves, one atomic per document run) follows in the same statement, dealt out behind the MFMAs of
-sub-steps 1 and 2; its atomics are issued behind the step's wait so that the wait does not count them.
+the second sub-step; its atomics are issued behind the step's wait so that the wait does not count them.
 
 Run ``python gen_scan_asm.py`` after changing the schedule; the generated file is committed.
 """
 import os
 import sys
 
-F = [128, 160]
-VT = 192
-VADDR_A, VADDR_B = 200, 204
+FA, FB = 128, 160
+VT_A0, VT_B0, VT_A1, VT_B1, VT_AN, VT_BN = range(192, 198)
+VADDR = 198          # A of sub-steps 0 and 1, B of sub-steps 0 and 1
 VOFF = 208
 VMAX = 224
+VPART = 232
 VRED = 240           # 8 scratch registers; the fold's temporaries: pair p in v(240 + 4 p) .. v(243 + 4 p)
 V_LOWMASK, V_DISTBASE, V_L32P1, V_IS31, V_L15 = 248, 249, 250, 251, 252
-VDOC = 220           # documents of the wavefront's columns: pair p in v(220 + p)
+VDOC = 220           # documents of the wavefront's columns: group p in v(220 + p)
 S_HALF = "s[86:87]"  # lanes 32 - 63
 S_M0, S_AN, S_BN, S_BLD = "s92", "s93", "s94", "s95"
 B0, BEND = 0x10000, 0x28000
 
-# MFMA order inside a sub-step and the order in which the next sub-step's fragments are read (what is needed first)
-ORDER = [(0, 0), (0, 1), (1, 0), (1, 1), (0, 2), (0, 3), (1, 2), (1, 3),
-         (2, 0), (2, 1), (2, 2), (2, 3), (3, 0), (3, 1), (3, 2), (3, 3)]
-READS = [("a", 0), ("b", 0), ("b", 1), ("a", 1), ("b", 2), ("b", 3), ("a", 2), ("a", 3)]
+QUADS = [[(0, 0), (0, 1), (1, 1), (1, 0)], [(0, 1), (0, 0), (1, 0), (1, 1)]]      # (A half, B half) in the order of a sub-step
+# the fragments requested during a quadrant: operand, first index, address register
+READS = [[("b", 4, VT_B0), ("a", 4, VT_A0), ("a", 0, VT_A1), ("b", 4, VT_B1)],
+         [("b", 0, VT_B1), ("a", 4, VT_A1), ("a", 0, VT_AN), ("b", 0, VT_BN)]]
+BARRIER = (1, 2)
 
 
 def acc(i, j):
-    b = (i * 4 + j) * 16
-    return f"a[{b}:{b + 15}]"
+    b = (i * 8 + j) * 4
+    return f"a[{b}:{b + 3}]"
 
 
-def fa(slot, i):
-    b = F[slot] + i * 4
+def frag(kind, n):
+    b = (FA if kind == "a" else FB) + 4 * n
     return f"v[{b}:{b + 3}]"
 
 
-def fb(slot, j):
-    b = F[slot] + 16 + j * 4
-    return f"v[{b}:{b + 3}]"
-
-
-def reduce_block(i, j, joined=False):
-    """Per-lane maximum of accumulator block (i, j) into v(VMAX + 4 i + j); joined: into v(VMAX + j), over the row
-    blocks i as well.  Two halves of eight values, each a tree of depth three (a wavefront that is alone on its SIMD
-    waits out every dependent instruction)."""
-    b = (i * 4 + j) * 16
-    m = f"v{VMAX + j}" if joined else f"v{VMAX + i * 4 + j}"
-    r = [f"v{VRED + x}" for x in range(8)]
+def order(sub, q):
+    """The quadrant's sixteen blocks: the fragments that arrived last change slowest, the others go to and fro."""
+    ha, hb = QUADS[sub][q]
     out = []
-    for h in range(2):
-        out += [f"v_accvgpr_read_b32 {r[x]}, a{b + 8 * h + x}" for x in range(8)]
-        out.append(f"v_max3_f32 {r[0]}, {r[0]}, {r[1]}, {r[2]}")
-        out.append(f"v_max3_f32 {r[3]}, {r[3]}, {r[4]}, {r[5]}")
-        out.append(f"v_max3_f32 {r[0]}, {r[0]}, {r[3]}, {r[6]}")
-        if h == 0 and not (joined and i > 0):
-            out.append(f"v_max_f32 {m}, {r[0]}, {r[7]}")
-        else:
-            out.append(f"v_max3_f32 {m}, {m}, {r[0]}, {r[7]}")
+    for n in range(4):
+        for m in range(4):
+            x = m if n % 2 == 0 else 3 - m
+            out.append((4 * ha + n, 4 * hb + x) if q >= 2 else (4 * ha + x, 4 * hb + n))
     return out
 
 
+class Reduction:
+    """The maxima of a finished tile, a block at a time in the order of the first sub-step's quadrants."""
+
+    def __init__(self, joined):
+        self.joined, self.seen, self.flip = joined, set(), 0
+
+    def part(self, i, j):
+        # joined: one row of parts per column group, over all rows; otherwise one per row block of 32 inside the quadrant
+        return VPART + (4 * (j >> 2) if self.joined else 4 * ((i >> 1) & 1)) + (j & 3)
+
+    def block(self, i, j):
+        b = (i * 8 + j) * 4
+        r = [f"v{VRED + self.flip + x}" for x in range(4)]
+        self.flip ^= 4
+        m = f"v{self.part(i, j)}"
+        key = (j,) if self.joined else (i >> 1, j)
+        out = [f"v_accvgpr_read_b32 {r[x]}, a{b + x}" for x in range(4)]
+        out.append(f"v_max3_f32 {r[0]}, {r[0]}, {r[1]}, {r[2]}")
+        out.append(f"v_max3_f32 {m}, {m}, {r[0]}, {r[3]}" if key in self.seen else f"v_max_f32 {m}, {r[0]}, {r[3]}")
+        self.seen.add(key)
+        return out
+
+    def after(self, q):
+        """What a quadrant's parts allow: the lanes of a column group joined, lane l column l of the group."""
+        ha, hb = QUADS[0][q]
+        if self.joined:
+            groups = [(VPART + 4 * hb, VMAX + hb)] if q >= 2 else []
+        else:
+            groups = [(VPART, VMAX + 2 * (2 * ha) + hb), (VPART + 4, VMAX + 2 * (2 * ha + 1) + hb)]
+        out = []
+        for step in ("v_permlane32_swap_b32 {0}, {2}", "v_permlane32_swap_b32 {1}, {3}", "v_max_f32 {0}, {0}, {2}", "v_max_f32 {1}, {1}, {3}",
+                     "v_permlane16_swap_b32 {0}, {1}", "v_max_f32 {r}, {0}, {1}"):
+            for first, result in groups:
+                out.append(step.format(*(f"v{first + x}" for x in range(4)), r=f"v{result}"))
+        return out
+
+
 def fold_pair(p):
-    """Document fold of column blocks 2p / 2p + 1 (maxima over the rows in v(VMAX + 2p), v(VMAX + 2p + 1), documents of
+    """Document fold of column group p (maxima over the rows in v(VMAX + p), documents of
     the 64 columns in v(VDOC + p)): returns (instructions, the masked atomic).  [okey]: the query's row of keys."""
-    R, H, doc = f"v{VMAX + 2 * p}", f"v{VMAX + 2 * p + 1}", f"v{VDOC + p}"
+    R, doc = f"v{VMAX + p}", f"v{VDOC + p}"
     t0, t1, t2, t3 = (f"v{VRED + 4 * p + x}" for x in range(4))
     sc = f"s[{80 + 2 * p}:{81 + 2 * p}]"        # a condition
     shl, shh = f"s{76 + 2 * p}", f"s{77 + 2 * p}"   # run heads, one bit per lane
     sx = "s[88:89]"                             # exec saved around the atomic
     o = []
-    o.append(f"v_permlane32_swap_b32 {R}, {H}")            # lower 32 lanes: block 2p, upper 32: block 2p + 1
-    o.append(f"v_max_f32 {R}, {R}, {H}")
     o.append(f"v_ashrrev_i32 {t0}, 31, {R}")               # order-preserving key of the float
     o.append(f"v_or_b32 {t0}, 0x80000000, {t0}")
     o.append(f"v_xor_b32 {R}, {R}, {t0}")
@@ -189,78 +215,94 @@ def kstep(fresh, reduce=None):
     """One K step.  Operands: [sa] / [sb] LDS stage of the step's query / K_r tile (advanced to the next step's),
     [ra] / [rb] resources the loads of this step read, [k] their byte offset inside a row, [woff] wave * 8 KB.
     fresh: a tile's first step (the first sub-step multiplies into zero); reduce: it also reduces the accumulators the
-    previous tile left, "blocks" to one maximum per block, "fold" on to the key plane ([okey]: the query's keys)."""
+    previous tile left, "blocks" to one maximum per row block, "fold" on to the key plane ([okey]: the query's keys)."""
     out = []
     e = out.append
     fillers, atomics = [], []
+    red = Reduction(reduce == "fold") if reduce else None
     if reduce == "fold":
         (a0, at0), (a1, at1) = fold_pair(0), fold_pair(1)
         fillers = interleave(a0, a1)
         atomics = at0 + at1
-    per_slot = -(-len(fillers) // 32)
+    per_slot = -(-len(fillers) // 44)
     # The step's scalar and address arithmetic stands behind its first MFMAs, not in front of them (a wavefront that
     # is alone on its SIMD pays for every instruction the matrix pipe does not run under): `early` is what the first
-    # LDS read and the first tile load need, `later` the rest, three instructions per MFMA.
+    # LDS read and the first tile load need, `later` the rest, two instructions per MFMA.
     early = [f"s_mov_b32 {S_M0}, m0",
-             f"v_add_u32 v{VT}, %[sa], v{VADDR_A + 1}", f"v_add_u32 v{VT + 1}, %[sb], v{VADDR_B + 1}",
+             f"v_add_u32 v{VT_B0}, %[sb], v{VADDR + 2}", f"v_add_u32 v{VT_A0}, %[sa], v{VADDR}",
              f"s_sub_u32 {S_BLD}, %[sb], 0x8000", f"s_cmp_lt_u32 {S_BLD}, {B0:#x}",
              f"s_cselect_b32 {S_BLD}, {BEND - 0x8000:#x}, {S_BLD}", f"s_add_u32 {S_BLD}, {S_BLD}, %[woff]"]
-    later = [f"s_add_u32 {S_BN}, %[sb], 0x8000", f"s_cmp_eq_u32 {S_BN}, {BEND:#x}", f"s_cselect_b32 {S_BN}, {B0:#x}, {S_BN}",
-             f"s_xor_b32 {S_AN}, %[sa], 0x8000", f"v_add_u32 v{VT + 2}, %[sa], v{VADDR_A + 2}", f"v_add_u32 v{VT + 3}, %[sb], v{VADDR_B + 2}",
-             f"v_add_u32 v{VT + 4}, %[sa], v{VADDR_A + 3}", f"v_add_u32 v{VT + 5}, %[sb], v{VADDR_B + 3}", f"v_add_u32 v{VT + 6}, {S_AN}, v{VADDR_A}",
-             f"v_add_u32 v{VT + 7}, {S_BN}, v{VADDR_B}"]
+    later = [f"v_add_u32 v{VT_A1}, %[sa], v{VADDR + 1}", f"v_add_u32 v{VT_B1}, %[sb], v{VADDR + 3}",
+             f"s_add_u32 {S_BN}, %[sb], 0x8000", f"s_cmp_eq_u32 {S_BN}, {BEND:#x}", f"s_cselect_b32 {S_BN}, {B0:#x}, {S_BN}",
+             f"s_xor_b32 {S_AN}, %[sa], 0x8000", f"v_add_u32 v{VT_AN}, {S_AN}, v{VADDR}", f"v_add_u32 v{VT_BN}, {S_BN}, v{VADDR + 2}"]
     if reduce == "fold":
         later += ["s_mov_b32 s86, 0", "s_mov_b32 s87, -1"]
-    for sub in range(4):
-        slot, nslot = sub & 1, (sub & 1) ^ 1
-        va, vb = (VT + 2 * sub, VT + 2 * sub + 1) if sub < 3 else (VT + 6, VT + 7)
-        e("s_waitcnt vmcnt(8) lgkmcnt(0)" if sub == 3 else "s_waitcnt lgkmcnt(0)")
-        nload = 0
-        for n, (i, j) in enumerate(ORDER):
-            do_load = sub in (0, 3) and n % 2 == 1
-            if do_load:
-                if nload > 0:
-                    e("s_add_u32 m0, m0, 0x400")
-                elif sub == 0:
-                    e(f"s_mov_b32 m0, {S_BLD}")
-                else:
-                    e("s_add_u32 m0, %[sa], %[woff]")
-            c = "0" if (fresh and sub == 0) else acc(i, j)
-            if reduce and sub == 0:
-                out.extend(reduce_block(i, j, joined=reduce == "fold"))
-            e(f"v_mfma_f32_32x32x16_bf16 {acc(i, j)}, {fa(slot, i)}, {fb(slot, j)}, {c}")
-            if sub == 3 and n == 0:
-                e("s_barrier")
-            if sub == 0 and n == 0:
-                out.extend(early)
-            if sub == 0 and n >= 1:
-                for _ in range(3):
-                    if later:
-                        e(later.pop(0))
-            if sub in (1, 2):
-                for _ in range(per_slot):
-                    if fillers:
-                        e(fillers.pop(0))
-            if sub == 3 and n in (10, 12) and atomics:
-                for _ in range(3):
-                    e(atomics.pop(0))
-            rd = n if sub < 3 else n - 1
-            if 0 <= rd < 8:
-                kind, idx = READS[rd]
-                if kind == "a":
-                    e(f"ds_read_b128 {fa(nslot, idx)}, v{va} offset:{idx * 4096}")
-                else:
-                    e(f"ds_read_b128 {fb(nslot, idx)}, v{vb} offset:{idx * 4096}")
-            if do_load:
-                if sub == 0:
-                    e(f"buffer_load_dwordx4 v{VOFF + nload}, %[rb], %[k] offen nt lds")
-                else:
-                    e(f"buffer_load_dwordx4 v{VOFF + nload}, %[ra], %[k] offen lds")
-                nload += 1
+    pending = [("a", n) for n in range(4)] + [("b", n) for n in range(4)]      # reads in flight, oldest first: the step before left these
+    nload = 0
+    for sub in range(2):
+        for q in range(4):
+            kind, first, addr = READS[sub][q]
+            for n, (i, j) in enumerate(order(sub, q)):
+                if (sub, q) == BARRIER and n == 0:
+                    e("s_waitcnt vmcnt(8) lgkmcnt(0)")
+                    pending = []
+                need = max([pending.index(x) for x in (("a", i), ("b", j)) if x in pending], default=-1)
+                if need >= 0:
+                    pending = pending[need + 1:]
+                    e(f"s_waitcnt lgkmcnt({len(pending)})")
+                do_load = n % 4 == 3 and (sub, q) in ((0, 0), (0, 1), (1, 2), (1, 3))
+                if do_load:
+                    if nload % 8:
+                        e("s_add_u32 m0, m0, 0x400")
+                    elif sub == 0:
+                        e(f"s_mov_b32 m0, {S_BLD}")
+                    else:
+                        e("s_add_u32 m0, %[sa], %[woff]")
+                if red and sub == 0:
+                    out.extend(red.block(i, j))
+                c = "0" if (fresh and sub == 0) else acc(i, j)
+                e(f"v_mfma_f32_16x16x32_bf16 {acc(i, j)}, {frag('a', i)}, {frag('b', j)}, {c}")
+                if (sub, q) == BARRIER and n == 0:
+                    e("s_barrier")
+                if (sub, q, n) == (0, 0, 0):
+                    out.extend(early)
+                if (sub, q) == (0, 0) and n >= 4:
+                    for _ in range(2):
+                        if later:
+                            e(later.pop(0))
+                if sub == 1 and n > (4 if q == 2 else 0):
+                    for _ in range(per_slot):
+                        if fillers:
+                            e(fillers.pop(0))
+                if (sub, q) == (1, 3) and n in (10, 12) and atomics:
+                    assert not fillers
+                    for _ in range(3):
+                        e(atomics.pop(0))
+                if 1 <= n <= 4:
+                    idx = first + n - 1
+                    e(f"ds_read_b128 {frag(kind, idx)}, v{addr} offset:{idx * 2048}")
+                    pending.append((kind, idx))
+                if do_load:
+                    v = VOFF + nload % 8
+                    e(f"buffer_load_dwordx4 v{v}, %[rb], %[k] offen nt lds" if sub == 0 else f"buffer_load_dwordx4 v{v}, %[ra], %[k] offen lds")
+                    nload += 1
+            if red and sub == 0:
+                out.extend(red.after(q))
     e(f"s_mov_b32 %[sa], {S_AN}")
     e(f"s_mov_b32 %[sb], {S_BN}")
     e(f"s_mov_b32 m0, {S_M0}")
-    assert not fillers and not atomics and not later
+    assert not fillers and not atomics and not later and nload == 16 and pending[-4:] == [("b", n) for n in range(4)]
+    return fix_lane_move_hazards(out)
+
+
+def reduction():
+    """The reduction by itself, behind a workgroup's last tile (an MFMA's result may be read 18 wait states after its
+    issue at the earliest)."""
+    red, out = Reduction(False), ["s_nop 15", "s_nop 7"]
+    for q in range(4):
+        for i, j in order(0, q):
+            out += red.block(i, j)
+        out += red.after(q)
     return fix_lane_move_hazards(out)
 
 
@@ -275,14 +317,12 @@ def main():
     parts.append(define("MSA_SCAN4_KSTEP_FRESH", kstep(True)))
     parts.append(define("MSA_SCAN4_KSTEP_FRESH_REDUCE", kstep(True, "blocks")))
     parts.append(define("MSA_SCAN4_KSTEP_FRESH_FOLD", kstep(True, "fold")))
-    # the reduction by itself, behind a workgroup's last tile (an MFMA's result may be read 18 wait states after its
-    # issue at the earliest)
-    parts.append(define("MSA_SCAN4_REDUCE", ["s_nop 15", "s_nop 7"] + [l for (i, j) in ORDER for l in reduce_block(i, j)]))
-    parts.append(define("MSA_SCAN4_MAX_READ", [f"v_mov_b32 %{x}, v{VMAX + x}" for x in range(16)]))
-    # fragments of sub-step 0 out of the stages [sa] / [sb] into slot 0 (in front of the first step)
-    lines = [f"v_add_u32 v{VT + 6}, %[sa], v{VADDR_A}", f"v_add_u32 v{VT + 7}, %[sb], v{VADDR_B}"]
-    for kind, idx in READS:
-        lines.append(f"ds_read_b128 {fa(0, idx) if kind == 'a' else fb(0, idx)}, v{VT + 6 if kind == 'a' else VT + 7} offset:{idx * 4096}")
+    parts.append(define("MSA_SCAN4_REDUCE", reduction()))
+    parts.append(define("MSA_SCAN4_MAX_READ", [f"v_mov_b32 %{x}, v{VMAX + x}" for x in range(8)]))
+    # fragments of the first quadrant out of the stages [sa] / [sb] (in front of the first step)
+    lines = [f"v_add_u32 v{VT_AN}, %[sa], v{VADDR}", f"v_add_u32 v{VT_BN}, %[sb], v{VADDR + 2}"]
+    for kind, addr in (("a", VT_AN), ("b", VT_BN)):
+        lines += [f"ds_read_b128 {frag(kind, n)}, v{addr} offset:{n * 2048}" for n in range(4)]
     parts.append(define("MSA_SCAN4_FRAGS0", lines))
     # the wavefront's eight blocks of one operand tile into the LDS stage at [dst] (+ wave * 8 KB already added)
     for name, nt in (("MSA_SCAN4_LOAD8", ""), ("MSA_SCAN4_LOAD8_NT", " nt")):
@@ -293,7 +333,7 @@ def main():
                 lines += ["s_add_u32 m0, m0, 0x400", "s_nop 0"]
         lines.append(f"s_mov_b32 m0, {S_M0}")
         parts.append(define(name, lines))
-    parts.append(define("MSA_SCAN4_SET_ADDR", [f"v_mov_b32 v{VADDR_A + s}, %{s}" for s in range(8)]))
+    parts.append(define("MSA_SCAN4_SET_ADDR", [f"v_mov_b32 v{VADDR + s}, %{s}" for s in range(4)]))
     parts.append(define("MSA_SCAN4_SET_VOFF", [f"v_mov_b32 v{VOFF + s}, %{s}" for s in range(8)]))
     # the fold's per-lane constants from l32 = lane & 31 (operand 0)
     parts.append(define("MSA_SCAN4_SET_FOLD", [

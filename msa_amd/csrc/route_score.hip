@@ -787,15 +787,20 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void score_gemm_kernel(
 
 // ------------------------------------------------------------------------------------------
 // The MFMA-bound form (bf16, more than 128 query rows): 256 x 256 tile, four wavefronts (one per SIMD) of 128 x 128,
-// the sixteen 32 x 32 accumulators of a wavefront in the 256 accumulation registers, and the K step written at the
+// a wavefront's 8 x 8 blocks of 16 x 16 in the 256 accumulation registers, and the K step written at the
 // instruction level (scan_asm.inc, generated by gen_scan_asm.py, which describes the schedule and the registers the
 // asm statements own: v128 - v255 and a0 - a255; the compiler-allocated code of this kernel is held below v128 by the
 // register limit on its declaration and uses no accumulation registers, which the build checks).  One wavefront per
 // SIMD has nobody to cover a wait, so every wait the step contains is met long before it is reached: operand
 // fragments are read a sub-step ahead, the query and K_r tiles are requested two K steps ahead (LDS: two stages of the
 // query tile, three of the K_r tile, filled by buffer loads that write LDS directly), and the one barrier per step
-// stands behind an MFMA.  Per 128 x 128 wavefront tile a sub-step reads eight operand fragments for sixteen MFMAs,
-// against six for eight in a 2 x 4 layout of eight wavefronts.
+// stands behind an MFMA.  128 x 128 wavefront tiles read a third less from LDS per product than a 2 x 4 layout of eight
+// wavefronts.
+//
+// What bounds it is power: the clock falls until the chip is inside its budget, so what counts is energy per product.
+// v_mfma_f32_16x16x32_bf16 passes an accumulator half as often for the same products as v_mfma_f32_32x32x16_bf16: a loop of
+// nothing but MFMAs on random operands holds 2070 TFLOP/s with the first and 1800 with the second (2440 and 2480 on zeros), and
+// 1.605M chunks x 2048 query rows take 4.25 ms here, 4.66 with the 32 x 32 x 16 form (1.58 and 1.45 PFLOP/s).
 //
 // Persistent: one workgroup per compute unit walks its share of the tile list (scan_walk.h) as one sequence of K
 // steps, the loads two steps ahead across tile boundaries.  With a gather job attached the last workgroup of the
@@ -851,24 +856,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
   const int row_bytes = K * (int)sizeof(bf16_t);
   const int k_tiles = row_bytes / kRowBytes;
   {
-    // per-lane constants of the asm statements: LDS offsets of the operand fragments of sub-steps 0 - 3 (the rows of a
-    // wavefront's blocks are 32 apart, which leaves the swizzle term alone) and the global offsets of the lanes' 16
+    // per-lane constants of the asm statements: LDS offsets of the operand fragments of the two sub-steps (the rows of a
+    // wavefront's blocks are 16 apart, which leaves the swizzle term alone) and the global offsets of the lanes' 16
     // bytes in the wavefront's eight 1 KB blocks of a tile (lane l lands at byte 16 * l of its block, i.e. row l / 8,
     // unit slot l % 8, and fetches the unit that belongs there)
-    int aa[4], ab[4], vo[8];
+    int aa[2], ab[2], vo[8];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int sw = ((s * 2 + half) ^ ((l32 >> 1) & 7)) * 16;
-      aa[s] = (wm * 128 + l32) * 128 + sw;
-      ab[s] = (wn * 128 + l32) * 128 + sw;
+    for (int s = 0; s < 2; ++s) {
+      const int sw = ((s * 4 + (lane >> 4)) ^ (((lane & 15) >> 1) & 7)) * 16;
+      aa[s] = (wm * 128 + (lane & 15)) * 128 + sw;
+      ab[s] = (wn * 128 + (lane & 15)) * 128 + sw;
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int row = (wave * 8 + i) * 8 + (lane >> 3);
       vo[i] = row * row_bytes + (((lane & 7) ^ ((row >> 1) & 7)) * 16);
     }
-    asm volatile(MSA_SCAN4_SET_ADDR ::"v"(aa[0]), "v"(aa[1]), "v"(aa[2]), "v"(aa[3]), "v"(ab[0]), "v"(ab[1]), "v"(ab[2]), "v"(ab[3])
-                 : MSA_SCAN4_CLOBBERS);
+    asm volatile(MSA_SCAN4_SET_ADDR ::"v"(aa[0]), "v"(aa[1]), "v"(ab[0]), "v"(ab[1]) : MSA_SCAN4_CLOBBERS);
     asm volatile(MSA_SCAN4_SET_VOFF ::"v"(vo[0]), "v"(vo[1]), "v"(vo[2]), "v"(vo[3]), "v"(vo[4]), "v"(vo[5]), "v"(vo[6]), "v"(vo[7])
                  : MSA_SCAN4_CLOBBERS);
     // v222: byte offset of a lane's column in a run of 64 document ids; v223: the pool counter's increment
@@ -915,8 +919,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
   const bool drawer = wave == 0;
   const uint32_t zero_off = 0;
 
-  // ---- epilogue state: see score_gemm_kernel's epilogue, of which this is the 4 x 4 block form ----
-  // acc block (i, j), element e: row 8 * (e / 4) + 4 * half + e % 4 of row block i, column l32 of column block j.
+  // ---- epilogue state: see score_gemm_kernel's epilogue, of which this is the form with four row blocks ----
   const int n_queries = M_rows / (blocks_per_query * 32);
   typedef const __attribute__((address_space(4))) uint32_t* const_words_t;      // scalar loads
   const const_words_t row_bits_c = (const_words_t)row_bits;
@@ -942,12 +945,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
                    ::"s"(rsrc_docs), "s"(first) : MSA_SCAN4_CLOBBERS);
     }
   };
-  // One pair of column blocks (64 columns): after the half-wave swap the lower 32 lanes hold block 2p's column maxima
-  // and the upper 32 lanes block 2p + 1's; the segmented scan then leaves a document's maximum in the last lane of its
+  // One group of 64 columns, a column a lane: the segmented scan leaves a document's maximum in the last lane of its
   // run, which alone touches memory.
-  auto emit_pair = [&](int q, int n_first, float lo, float hi, int doc_raw) {
-    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
-    const float run = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+  auto emit_group = [&](int q, int n_first, float run, int doc_raw) {
     const int n = n_first + lane;
     const bool ok = n < C;
     const uint32_t key = ok ? f32_to_key(run) : 0u;
@@ -983,33 +983,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
   // repeat a scored one); a block whose mask word is zero belongs to a query without scored tokens or to the padding
   // past M_rows and is skipped.
   auto fold_tile = [&](int n0) {
-    float mx[16];
+    float mx[8];
     asm volatile(MSA_SCAN4_MAX_READ
-                 : "=v"(mx[0]), "=v"(mx[1]), "=v"(mx[2]), "=v"(mx[3]), "=v"(mx[4]), "=v"(mx[5]), "=v"(mx[6]), "=v"(mx[7]),
-                   "=v"(mx[8]), "=v"(mx[9]), "=v"(mx[10]), "=v"(mx[11]), "=v"(mx[12]), "=v"(mx[13]), "=v"(mx[14]), "=v"(mx[15]));
+                 : "=v"(mx[0]), "=v"(mx[1]), "=v"(mx[2]), "=v"(mx[3]), "=v"(mx[4]), "=v"(mx[5]), "=v"(mx[6]), "=v"(mx[7]));
     int doc0 = 0, doc1 = 0;
     if constexpr (kDocMax) asm volatile("v_mov_b32 %0, v220\n\tv_mov_b32 %1, v221" : "=v"(doc0), "=v"(doc1));
-    float run[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    float run[2] = {-INFINITY, -INFINITY};
     bool any = false;
     int run_q = q_first, r = r_first;
     auto emit = [&]() {
       if (!any || run_q >= n_queries) return;
-      emit_pair(run_q, n0 + wn * 128, run[0], run[1], doc0);
-      emit_pair(run_q, n0 + wn * 128 + 64, run[2], run[3], doc1);
+      emit_group(run_q, n0 + wn * 128, run[0], doc0);
+      emit_group(run_q, n0 + wn * 128 + 64, run[1], doc1);
     };
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (r == blocks_per_query) {                         // row block i opens the next query
         emit();
-#pragma unroll
-        for (int j = 0; j < 4; ++j) run[j] = -INFINITY;
+        run[0] = run[1] = -INFINITY;
         any = false; ++run_q; r = 0;
       }
       ++r;
       if (rbits[i] != 0) {
         any = true;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) run[j] = fmaxf(run[j], mx[i * 4 + j]);
+        run[0] = fmaxf(run[0], mx[2 * i]);
+        run[1] = fmaxf(run[1], mx[2 * i + 1]);
       }
     }
     emit();
