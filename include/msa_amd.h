@@ -327,8 +327,8 @@ int msa_qk_norm_rope(const void* q, const void* k, const void* v, int64_t q_row_
 /* Fused projection of a block of tokens (the encode path of stage 1 and the query prefill of stage 2): one bf16 GEMM
  * x[T, K] . w[N, K]^T over the concatenated weights of q_proj / k_proj / v_proj and, on router layers, router_k_proj
  * or router_q_proj (src/msa/memory_sparse_attention.py:125-127, 178, 263), with q_norm / k_norm and
- * apply_rotary_pos_emb (:129-133) applied to the q and k heads in the GEMM's epilogue, exactly as msa_qk_norm_rope
- * would to the bf16 projection output.  Rows of w, 128 per head: Hr_front router heads | Hq q heads | Hkv k heads |
+ * apply_rotary_pos_emb (:129-133) applied to the q and k heads in the GEMM's epilogue, as msa_qk_norm_rope
+ * would to the projection output (which is not rounded in between).  Rows of w, 128 per head: Hr_front router heads | Hq q heads | Hkv k heads |
  * Hkv v heads | Hr_back router heads (so one [rk | q | k | v | rq] matrix serves stage 1 with Hr_front = Hkv, stage 2
  * with a pointer 1024 rows in and Hr_back = Hq, and the decode step's q | k | v slice).  K a multiple of 64.
  * Outputs are dense: q_out [T, Hq, 128], k_out / v_out [T, Hkv, 128], r_out [T, Hr_front + Hr_back, 128]
@@ -340,6 +340,22 @@ int msa_qkv_proj(const void* x, int64_t T, int32_t K, const void* w, int32_t Hq,
                  int32_t Hr_back, const int64_t* positions, const void* q_norm_w, const void* k_norm_w, float eps,
                  const float* rope_cos, const float* rope_sin, int32_t rope_rows, void* q_out, void* k_out,
                  void* v_out, void* r_out, void* stream);
+/* Same with a workspace of msa_tile_workspace_bytes(T, K, 128 heads): the tiles that would leave compute units idle are multiplied in
+ * pieces of K.  The workspace need not be cleared; calls on different streams take different ones. */
+int msa_qkv_proj_ws(const void* x, int64_t T, int32_t K, const void* w, int32_t Hq, int32_t Hkv, int32_t Hr_front,
+                    int32_t Hr_back, const int64_t* positions, const void* q_norm_w, const void* k_norm_w, float eps,
+                    const float* rope_cos, const float* rope_sin, int32_t rope_rows, void* q_out, void* k_out,
+                    void* v_out, void* r_out, void* ws, size_t ws_bytes, void* stream);
+/* Products of a block of tokens, bf16 with fp32 sums: x [T, K] (rows ldx apart) . w [N, K]^T, w dense, K a multiple of 64, N of 8 (16),
+ * x / w / out 16-byte aligned, row strides multiples of 8.  mode: what becomes of the sums.
+ *   MSA_TILE_STORE     out [T, N] (rows ldo apart)
+ *   MSA_TILE_ADD       out += (the sum is rounded once)
+ *   MSA_TILE_SILU_MUL  out [T, N / 2] = silu(gate) * up, rows of w alternating in groups of eight gates and eight ups
+ * ws: msa_tile_workspace_bytes(T, K, N) bytes or NULL, as above. */
+enum { MSA_TILE_STORE = 0, MSA_TILE_ADD = 1, MSA_TILE_SILU_MUL = 2 };
+size_t msa_tile_workspace_bytes(int64_t T, int32_t K, int32_t N);
+int msa_tile_linear(const void* x, int64_t ldx, int64_t T, int32_t K, const void* w, int32_t N, int32_t mode, void* out,
+                    int64_t ldo, void* ws, size_t ws_bytes, void* stream);
 /* msa_qk_norm_rope for a decode step (one new token per sample, N = B) fused with msa_cache_append: the
  * normalised, rotated k row and the v row of sample b are written to kcache / vcache [b][kv_len[b]] and
  * kv_len[b] is incremented (src/msa/memory_sparse_attention.py:129-133 followed by the cache update at

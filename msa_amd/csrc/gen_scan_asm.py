@@ -1,5 +1,6 @@
 #!/usr/bin/env python3
-"""Writes ``scan_asm.inc``: the instruction-level K step of the large-tile routing scan (``score_scan4_kernel``).
+"""Writes ``scan_asm.inc``: the instruction-level K step of the large-tile routing scan (``score_scan4_kernel``), and
+``gemm_asm.inc``: the same step for the tiled products (``tile_gemm_kernel``).
 
 The scan's 256 x 256 tile is computed by four wavefronts, one per SIMD, 128 x 128 each: 8 x 8 blocks of 16 x 16 in the 256
 accumulation registers a0-a255, eight fragments of each operand in v128-v191.  One K step (64 elements of K) is one asm statement
@@ -37,7 +38,11 @@ column maxima over the chunks of a document (order-preserving key, segmented max
 lanes by row moves, one atomic per document run) follows in the same statement, dealt out behind the MFMAs of
 the second sub-step; its atomics are issued behind the step's wait so that the wait does not count them.
 
-Run ``python gen_scan_asm.py`` after changing the schedule; the generated file is committed.
+In the products the A operand is the weights and the B operand the tokens; each has row offsets of its own (v208-v215 the eight blocks
+of the A tile, v216-v223 those of the B tile), neither is read non-temporal, and a finished tile's accumulators are read behind its
+last step.
+
+Run ``python gen_scan_asm.py`` after changing the schedule; the generated files are committed.
 """
 import os
 import sys
@@ -46,6 +51,7 @@ FA, FB = 128, 160
 VT_A0, VT_B0, VT_A1, VT_B1, VT_AN, VT_BN = range(192, 198)
 VADDR = 198          # A of sub-steps 0 and 1, B of sub-steps 0 and 1
 VOFF = 208
+VOFF_B = 216         # of the products' B operand
 VMAX = 224
 VPART = 232
 VRED = 240           # 8 scratch registers; the fold's temporaries: pair p in v(240 + 4 p) .. v(243 + 4 p)
@@ -211,7 +217,7 @@ def fix_lane_move_hazards(lines):
     return out
 
 
-def kstep(fresh, reduce=None):
+def kstep(fresh, reduce=None, voff_b=VOFF, nt=" nt"):
     """One K step.  Operands: [sa] / [sb] LDS stage of the step's query / K_r tile (advanced to the next step's),
     [ra] / [rb] resources the loads of this step read, [k] their byte offset inside a row, [woff] wave * 8 KB.
     fresh: a tile's first step (the first sub-step multiplies into zero); reduce: it also reduces the accumulators the
@@ -283,8 +289,10 @@ def kstep(fresh, reduce=None):
                     e(f"ds_read_b128 {frag(kind, idx)}, v{addr} offset:{idx * 2048}")
                     pending.append((kind, idx))
                 if do_load:
-                    v = VOFF + nload % 8
-                    e(f"buffer_load_dwordx4 v{v}, %[rb], %[k] offen nt lds" if sub == 0 else f"buffer_load_dwordx4 v{v}, %[ra], %[k] offen lds")
+                    if sub == 0:
+                        e(f"buffer_load_dwordx4 v{voff_b + nload}, %[rb], %[k] offen{nt} lds")
+                    else:
+                        e(f"buffer_load_dwordx4 v{VOFF + nload - 8}, %[ra], %[k] offen lds")
                     nload += 1
             if red and sub == 0:
                 out.extend(red.after(q))
@@ -311,43 +319,88 @@ def define(name, lines):
     return f"#define {name} \\\n{body}\n"
 
 
-def main():
-    parts = ["// Generated by gen_scan_asm.py (the schedule and the register map are described there).  Do not edit.\n"]
-    parts.append(define("MSA_SCAN4_KSTEP", kstep(False)))
-    parts.append(define("MSA_SCAN4_KSTEP_FRESH", kstep(True)))
-    parts.append(define("MSA_SCAN4_KSTEP_FRESH_REDUCE", kstep(True, "blocks")))
-    parts.append(define("MSA_SCAN4_KSTEP_FRESH_FOLD", kstep(True, "fold")))
-    parts.append(define("MSA_SCAN4_REDUCE", reduction()))
-    parts.append(define("MSA_SCAN4_MAX_READ", [f"v_mov_b32 %{x}, v{VMAX + x}" for x in range(8)]))
-    # fragments of the first quadrant out of the stages [sa] / [sb] (in front of the first step)
+def frags0():
+    """Fragments of the first quadrant out of the stages [sa] / [sb] (in front of the first step)."""
     lines = [f"v_add_u32 v{VT_AN}, %[sa], v{VADDR}", f"v_add_u32 v{VT_BN}, %[sb], v{VADDR + 2}"]
     for kind, addr in (("a", VT_AN), ("b", VT_BN)):
         lines += [f"ds_read_b128 {frag(kind, n)}, v{addr} offset:{n * 2048}" for n in range(4)]
-    parts.append(define("MSA_SCAN4_FRAGS0", lines))
-    # the wavefront's eight blocks of one operand tile into the LDS stage at [dst] (+ wave * 8 KB already added)
-    for name, nt in (("MSA_SCAN4_LOAD8", ""), ("MSA_SCAN4_LOAD8_NT", " nt")):
-        lines = [f"s_mov_b32 {S_M0}, m0", "s_mov_b32 m0, %[dst]", "s_nop 4"]
-        for i in range(8):
-            lines.append(f"buffer_load_dwordx4 v{VOFF + i}, %[r], %[k] offen{nt} lds")
-            if i < 7:
-                lines += ["s_add_u32 m0, m0, 0x400", "s_nop 0"]
-        lines.append(f"s_mov_b32 m0, {S_M0}")
-        parts.append(define(name, lines))
-    parts.append(define("MSA_SCAN4_SET_ADDR", [f"v_mov_b32 v{VADDR + s}, %{s}" for s in range(4)]))
-    parts.append(define("MSA_SCAN4_SET_VOFF", [f"v_mov_b32 v{VOFF + s}, %{s}" for s in range(8)]))
-    # the fold's per-lane constants from l32 = lane & 31 (operand 0)
-    parts.append(define("MSA_SCAN4_SET_FOLD", [
-        f"v_lshlrev_b32 v{V_LOWMASK}, %0, 2", f"v_add_u32 v{V_LOWMASK}, -1, v{V_LOWMASK}",      # (2 << l32) - 1
-        f"v_add_u32 v{V_DISTBASE}, -31, %0", f"v_add_u32 v{V_L32P1}, 1, %0",
-        f"v_cmp_eq_u32 vcc, 31, %0", f"v_cndmask_b32 v{V_IS31}, 0, 1, vcc", f"v_and_b32 v{V_L15}, 15, %0"]))
+    return lines
+
+
+def load8(voff, nt=""):
+    """The wavefront's eight blocks of one operand tile into the LDS stage at [dst] (+ wave * 8 KB already added)."""
+    lines = [f"s_mov_b32 {S_M0}, m0", "s_mov_b32 m0, %[dst]", "s_nop 4"]
+    for i in range(8):
+        lines.append(f"buffer_load_dwordx4 v{voff + i}, %[r], %[k] offen{nt} lds")
+        if i < 7:
+            lines += ["s_add_u32 m0, m0, 0x400", "s_nop 0"]
+    return lines + [f"s_mov_b32 m0, {S_M0}"]
+
+
+def set_registers(first, count):
+    return [f"v_mov_b32 v{first + s}, %{s}" for s in range(count)]
+
+
+def clobbers(name):
     regs = [f"v{r}" for r in range(128, 256)] + [f"a{r}" for r in range(256)] + [f"s{r}" for r in range(76, 96)] + ["vcc", "scc", "memory"]
-    parts.append("#define MSA_SCAN4_CLOBBERS " + ", ".join(f'"{x}"' for x in regs) + "\n")
-    text = "\n".join(parts)
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "scan_asm.inc")
-    if len(sys.argv) > 1 and sys.argv[1] == "--check":
-        return 0 if open(path).read() == text else 1
-    open(path, "w").write(text)
-    return 0
+    return f"#define {name} " + ", ".join(f'"{x}"' for x in regs) + "\n"
+
+
+HEADER = "// Generated by gen_scan_asm.py (the schedule and the register map are described there).  Do not edit.\n"
+
+
+def scan_text():
+    return "\n".join([
+        HEADER,
+        define("MSA_SCAN4_KSTEP", kstep(False)),
+        define("MSA_SCAN4_KSTEP_FRESH", kstep(True)),
+        define("MSA_SCAN4_KSTEP_FRESH_REDUCE", kstep(True, "blocks")),
+        define("MSA_SCAN4_KSTEP_FRESH_FOLD", kstep(True, "fold")),
+        define("MSA_SCAN4_REDUCE", reduction()),
+        define("MSA_SCAN4_MAX_READ", [f"v_mov_b32 %{x}, v{VMAX + x}" for x in range(8)]),
+        define("MSA_SCAN4_FRAGS0", frags0()),
+        define("MSA_SCAN4_LOAD8", load8(VOFF)),
+        define("MSA_SCAN4_LOAD8_NT", load8(VOFF, " nt")),
+        define("MSA_SCAN4_SET_ADDR", set_registers(VADDR, 4)),
+        define("MSA_SCAN4_SET_VOFF", set_registers(VOFF, 8)),
+        # the fold's per-lane constants from l32 = lane & 31 (operand 0)
+        define("MSA_SCAN4_SET_FOLD", [
+            f"v_lshlrev_b32 v{V_LOWMASK}, %0, 2", f"v_add_u32 v{V_LOWMASK}, -1, v{V_LOWMASK}",      # (2 << l32) - 1
+            f"v_add_u32 v{V_DISTBASE}, -31, %0", f"v_add_u32 v{V_L32P1}, 1, %0",
+            f"v_cmp_eq_u32 vcc, 31, %0", f"v_cndmask_b32 v{V_IS31}, 0, 1, vcc", f"v_and_b32 v{V_L15}, 15, %0"]),
+        clobbers("MSA_SCAN4_CLOBBERS")])
+
+
+def gemm_text():
+    parts = [HEADER,
+             define("MSA_GEMM_KSTEP", kstep(False, voff_b=VOFF_B, nt="")),
+             define("MSA_GEMM_KSTEP_FRESH", kstep(True, voff_b=VOFF_B, nt="")),
+             define("MSA_GEMM_FRAGS0", frags0()),
+             define("MSA_GEMM_LOAD8_A", load8(VOFF)),
+             define("MSA_GEMM_LOAD8_B", load8(VOFF_B)),
+             define("MSA_GEMM_SET_ADDR", set_registers(VADDR, 4)),
+             define("MSA_GEMM_SET_VOFF_A", set_registers(VOFF, 8)),
+             define("MSA_GEMM_SET_VOFF_B", set_registers(VOFF_B, 8)),
+             # an MFMA's result may be read 18 wait states after its issue at the earliest
+             define("MSA_GEMM_SETTLE", ["s_nop 15", "s_nop 7"])]
+    # four of the eight row blocks of a column block, sixteen accumulators
+    for j in range(8):
+        for h in range(2):
+            parts.append(define(f"MSA_GEMM_ACC_{j}_{h}", [f"v_accvgpr_read_b32 %{4 * i + r}, a{((4 * h + i) * 8 + j) * 4 + r}"
+                                                          for i in range(4) for r in range(4)]))
+    parts.append(clobbers("MSA_GEMM_CLOBBERS"))
+    return "\n".join(parts)
+
+
+def main():
+    here, stale = os.path.dirname(os.path.abspath(__file__)), 0
+    for name, text in (("scan_asm.inc", scan_text()), ("gemm_asm.inc", gemm_text())):
+        path = os.path.join(here, name)
+        if len(sys.argv) > 1 and sys.argv[1] == "--check":
+            stale |= not os.path.exists(path) or open(path).read() != text
+        else:
+            open(path, "w").write(text)
+    return int(stale)
 
 
 if __name__ == "__main__":

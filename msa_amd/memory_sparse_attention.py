@@ -280,7 +280,7 @@ class MemorySparseAttention(nn.Module):
         dev = hidden_states.device
         out = ops.sparse_attn(q[0], k[0], v[0], cu[:-1].to(dev), torch.tensor(seg, dtype=torch.int32, device=dev),
                               max(seg), cu_q=cu.to(torch.int32).to(dev), max_sq=max(seg), scale=self.scaling, causal=True)
-        return self.o_proj(out.view(1, T, Hq * D)), None
+        return ops.linear(self.o_proj, out.view(1, T, Hq * D)), None
 
     # ------------------------------------------------------------------------------------------ stage 2
     def _stage2(self, hidden_states, doc_ids, attention_mask, q, k, v, cache, router_q=None):
@@ -352,7 +352,7 @@ class MemorySparseAttention(nn.Module):
         ck.update({"compacked_key_cache": kc, "compacked_value_cache": vc, "kv_lengths": kv_len, "kv_offsets": kv_off,
                    "kv_capacity": Lcap, "rows_free": self.decode_reserve})
         cache.record_kwargs(self.layer_idx, ck)
-        return self.o_proj(attn), None
+        return ops.linear(self.o_proj, attn), None
 
     # ------------------------------------------------------------------------------------------ decode
     def _generate(self, hidden_states, q, k, v, cache, attention_mask=None):
@@ -386,9 +386,9 @@ class MemorySparseAttention(nn.Module):
                                    ck["kv_capacity"], cu_q=cu_new, max_sq=max(n_host), scale=self.scaling, causal=True)
             attn = torch.zeros((B, S, Hq * D), device=q.device, dtype=q.dtype)
             attn[valid] = rows.view(-1, Hq * D)
-            return self.o_proj(attn), None
+            return ops.linear(self.o_proj, attn), None
         self._claim_rows(ck, 1)
         ops.cache_append(k[:, 0].contiguous(), v[:, 0].contiguous(), kc, vc, kv_len)
         out = ops.sparse_attn(q[:, 0].contiguous(), kc.view(-1, Hkv, D), vc.view(-1, Hkv, D), ck["kv_offsets"], kv_len,
                               ck["kv_capacity"], scale=self.scaling, causal=True)
-        return self.o_proj(out.view(B, 1, -1)), None
+        return ops.linear(self.o_proj, out.view(B, 1, -1)), None

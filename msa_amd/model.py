@@ -25,23 +25,46 @@ class MLP(nn.Module):
         self.up_proj = nn.Linear(config.hidden_size, config.intermediate_size, bias=False)
         self.down_proj = nn.Linear(config.intermediate_size, config.hidden_size, bias=False)
 
-        self._gate_up_weight = None
-        self._gate_up_interleaved = None
+        self._joined = {}
+
+    def _gate_up(self, interleaved: bool):
+        """Gate and up rows in one matrix, behind one another or as the silu-mul epilogues take them; made again when either weight
+        changes."""
+        parts = (self.gate_proj.weight, self.up_proj.weight)
+        key = tuple((w.data_ptr(), w._version, w.dtype, w.device) for w in parts)
+        if interleaved not in self._joined or self._joined[interleaved][0] != key:
+            gate, up = (w.detach() for w in parts)
+            self._joined[interleaved] = (key, ops.interleave_gate_up(gate, up) if interleaved else torch.cat([gate, up], dim=0).contiguous())
+        return self._joined[interleaved][1]
 
     def decode_rows(self, residual, norm_weight, eps):
         """``residual + down(silu(gate(n)) * up(n))`` with ``n = rmsnorm(residual)`` for up to 16 bf16 rows:
         two weight-streaming launches, the norm folded into the first, silu-mul into its epilogue, the residual
         add into the second."""
-        if self._gate_up_interleaved is None or self._gate_up_interleaved.device != residual.device:
-            self._gate_up_interleaved = ops.interleave_gate_up(self.gate_proj.weight, self.up_proj.weight)
-        act = ops.skinny_linear(residual, self._gate_up_interleaved, silu_mul=True, norm_weight=norm_weight, eps=eps)
+        act = ops.skinny_linear(residual, self._gate_up(True), silu_mul=True, norm_weight=norm_weight, eps=eps)
         return ops.skinny_linear(act, self.down_proj.weight, residual=residual)
+
+    def _activation(self, x):
+        gate, up = self.gate_proj.weight, self.up_proj.weight
+        if gate.shape[0] % 8 == 0 and x.is_contiguous() and ops.tile_linear_ok(x, gate, 2) and ops.tile_linear_ok(x, up, 2):
+            return ops.tile_linear(x.view(-1, x.shape[-1]), self._gate_up(True), silu_mul=True).view(*x.shape[:-1], -1)
+        return ops.silu_mul(F.linear(x, self._gate_up(False)))
+
+    def add_to(self, residual, x):
+        """``residual += self(x)`` (bf16 / fp32 on the GPU); a block of bf16 tokens has the add in the end of the second product, where the
+        sum is rounded once."""
+        if not ops.plain_module(self):
+            return residual.add_(self(x))
+        act = self._activation(x)
+        if ops.linear_ok(self.down_proj, act) and residual.is_contiguous() and residual.dtype == x.dtype and residual.shape == x.shape \
+                and residual.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and residual.requires_grad):
+            ops.tile_linear(act.view(-1, act.shape[-1]), self.down_proj.weight, out=residual.view(-1, x.shape[-1]), add=True)
+            return residual
+        return residual.add_(self.down_proj(act))
 
     def forward(self, x):
         if x.is_cuda and x.dtype in (torch.bfloat16, torch.float32):
-            if self._gate_up_weight is None or self._gate_up_weight.device != x.device:
-                self._gate_up_weight = torch.cat([self.gate_proj.weight, self.up_proj.weight], dim=0).contiguous()
-            return self.down_proj(ops.silu_mul(F.linear(x, self._gate_up_weight)))
+            return ops.linear(self.down_proj, self._activation(x))
         return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
 
 
@@ -65,7 +88,7 @@ class MSADecoderLayer(nn.Module):
             h, _ = self.self_attn(ops.rmsnorm(hidden_states, n1.weight, n1.variance_epsilon), doc_ids, attention_mask,
                                   position_embeddings, past_key_value, position_ids=position_ids)
             x = ops.rmsnorm(h.contiguous(), n2.weight, n2.variance_epsilon, residual=hidden_states)
-            return hidden_states.add_(self.mlp(x))
+            return self.mlp.add_to(hidden_states, x)
         h, _ = self.self_attn(self.input_layernorm(hidden_states), doc_ids, attention_mask, position_embeddings,
                               past_key_value)
         hidden_states = hidden_states + h

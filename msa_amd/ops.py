@@ -419,10 +419,79 @@ def qkv_proj(x: torch.Tensor, w: torch.Tensor, Hq: int, Hkv: int, positions: tor
     k = torch.empty((T, Hkv, D), dtype=x.dtype, device=dev)
     v = torch.empty((T, Hkv, D), dtype=x.dtype, device=dev)
     r = torch.empty((T, router_front + router_back, D), dtype=x.dtype, device=dev) if router_front + router_back else None
-    check(_lib.load().msa_qkv_proj(ptr(x), T, K, ptr(w), Hq, Hkv, router_front, router_back, ptr(positions), ptr(q_norm_w),
-                                   ptr(k_norm_w), eps, ptr(rope[0]), ptr(rope[1]), rope[0].shape[0], ptr(q), ptr(k), ptr(v),
-                                   ptr(r), _stream()), "msa_qkv_proj")
+    ws = _tile_workspace(T, K, heads * D, dev)
+    check(_lib.load().msa_qkv_proj_ws(ptr(x), T, K, ptr(w), Hq, Hkv, router_front, router_back, ptr(positions), ptr(q_norm_w),
+                                      ptr(k_norm_w), eps, ptr(rope[0]), ptr(rope[1]), rope[0].shape[0], ptr(q), ptr(k), ptr(v),
+                                      ptr(r), ptr(ws), 0 if ws is None else ws.numel(), _stream()), "msa_qkv_proj")
     return q, k, v, r
+
+
+def _tile_workspace(T: int, K: int, N: int, device) -> Optional[torch.Tensor]:
+    """Partial tiles of one call (from the allocator each time: calls on other streams have their own)."""
+    need = _lib.load().msa_tile_workspace_bytes(T, K, N)
+    return torch.empty(need, dtype=torch.uint8, device=device) if need else None
+
+
+TILE_STORE, TILE_ADD, TILE_SILU_MUL = range(3)
+
+
+def tile_linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, add: bool = False,
+                silu_mul: bool = False) -> torch.Tensor:
+    """``x @ w.T`` of a block of bf16 rows ``x [T, K]`` (unit column stride, K a multiple of 64) with a dense ``w [N, K]``, into ``out``
+    where given; ``add`` adds the product to ``out``; ``silu_mul`` takes ``w`` from ``interleave_gate_up`` and returns
+    ``silu(gate) * up`` of width ``N / 2``."""
+    _need_cuda(w)
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or x.stride(1) != 1 or not x.is_cuda:
+        raise ValueError("tile_linear: x [T, K] with unit column stride, w [N, K] contiguous, both on the device")
+    if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+        raise ValueError("tile_linear: x and w in bf16")
+    (T, K), N = x.shape, w.shape[0]
+    if add and (silu_mul or out is None):
+        raise ValueError("tile_linear: add needs out and excludes silu_mul")
+    width = N // 2 if silu_mul else N
+    if out is None:
+        out = torch.empty((T, width), dtype=x.dtype, device=x.device)
+    elif tuple(out.shape) != (T, width) or out.dtype != x.dtype or out.stride(1) != 1 or not out.is_cuda:
+        raise ValueError(f"tile_linear: out must be bf16 [{T}, {width}] on the device with unit column stride")
+    if not T:
+        return out
+    ws = _tile_workspace(T, K, N, x.device)
+    rows = lambda t: t.stride(0) if T > 1 else t.shape[1]
+    check(_lib.load().msa_tile_linear(ptr(x), rows(x), T, K, ptr(w), N, TILE_SILU_MUL if silu_mul else TILE_ADD if add else TILE_STORE,
+                                      ptr(out), rows(out), ptr(ws), 0 if ws is None else ws.numel(), _stream()), "msa_tile_linear")
+    return out
+
+
+TILE_MIN = 144          # tiles of 256 x 256 from which tile_linear is at least the vendor's equal
+
+
+def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1) -> bool:
+    """Whether ``x [..., K] @ w.T`` (``matrices`` of w's shape in one) is ``tile_linear``'s: operands as it takes them, no gradients asked for, and tiles enough to fill the
+    compute units.  Below ``TILE_MIN`` tiles the vendor's smaller ones win (us, vendor and here, K x N: 2560 x 2560 of 2048 tokens, 80
+    tiles, 31 and 43; of 4096, 160 tiles, 50 and 51; of 16384, 640 tiles, 233 and 161; 2560 x 19456 of 1000, 304 tiles, 102 and 90).
+    Depths under 1024 were not measured and stay where they were."""
+    T, K, N = x.numel() // max(x.shape[-1], 1), x.shape[-1], matrices * w.shape[0]
+    return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == K
+            and K % 64 == 0 and 1024 <= K <= 32768 and N % 8 == 0 and N < 1 << 20 and T < 1 << 22
+            and -(-T // 256) * -(-N // 256) >= TILE_MIN and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+
+
+def plain_module(module: torch.nn.Module) -> bool:
+    """Whether nothing but the module's own ``forward`` runs when it is called."""
+    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+
+
+def linear_ok(module: torch.nn.Module, x: torch.Tensor) -> bool:
+    return (type(module) is torch.nn.Linear and module.bias is None and x.is_contiguous() and tile_linear_ok(x, module.weight)
+            and plain_module(module))
+
+
+def linear(module: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``module(x)``, by ``tile_linear`` where that is the faster form."""
+    if linear_ok(module, x):
+        return tile_linear(x.view(-1, x.shape[-1]), module.weight).view(*x.shape[:-1], -1)
+    return module(x)
 
 
 def qk_norm_rope_append(qkv: torch.Tensor, Hq: int, Hkv: int, D: int, positions: torch.Tensor, q_norm_w, k_norm_w,
