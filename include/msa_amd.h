@@ -346,15 +346,21 @@ int msa_qkv_proj_ws(const void* x, int64_t T, int32_t K, const void* w, int32_t 
                     int32_t Hr_back, const int64_t* positions, const void* q_norm_w, const void* k_norm_w, float eps,
                     const float* rope_cos, const float* rope_sin, int32_t rope_rows, void* q_out, void* k_out,
                     void* v_out, void* r_out, void* ws, size_t ws_bytes, void* stream);
-/* Products of a block of tokens, bf16 with fp32 sums: x [T, K] (rows ldx apart) . w [N, K]^T, w dense, K a multiple of 64, N of 8 (16),
- * x / w / out 16-byte aligned, row strides multiples of 8.  mode: what becomes of the sums.
+/* Products of a block of tokens, bf16 with fp32 sums: x [T, K] (rows ldx apart) . w [N, K]^T, w dense, K a multiple of 64, N of 8 (16 where
+ * it is halved), x / w / out 16-byte aligned, row strides multiples of 8.  What becomes of the sums, each rounded once:
  *   MSA_TILE_STORE     out [T, N] (rows ldo apart)
- *   MSA_TILE_ADD       out += (the sum is rounded once)
+ *   MSA_TILE_ADD       out +=
  *   MSA_TILE_SILU_MUL  out [T, N / 2] = silu(gate) * up, rows of w alternating in groups of eight gates and eight ups
+ *   MSA_TILE_GLU       out [T, N / 2] = g sigmoid(alpha g) (u + shift), g = min(gate, limit), u = up within +- limit, rows of w alternating
+ *   MSA_TILE_GELU      out [T, N], the first gelu_n columns (a multiple of 8) through the tanh form of gelu
  * ws: msa_tile_workspace_bytes(T, K, N) bytes or NULL, as above. */
-enum { MSA_TILE_STORE = 0, MSA_TILE_ADD = 1, MSA_TILE_SILU_MUL = 2 };
+enum { MSA_TILE_STORE = 0, MSA_TILE_ADD = 1, MSA_TILE_SILU_MUL = 2, MSA_TILE_GLU = 4, MSA_TILE_GELU = 5 };
+typedef struct msa_tile_end {
+  int32_t mode, gelu_n;
+  float limit, alpha, shift;
+} msa_tile_end;
 size_t msa_tile_workspace_bytes(int64_t T, int32_t K, int32_t N);
-int msa_tile_linear(const void* x, int64_t ldx, int64_t T, int32_t K, const void* w, int32_t N, int32_t mode, void* out,
+int msa_tile_linear(const void* x, int64_t ldx, int64_t T, int32_t K, const void* w, int32_t N, const msa_tile_end* end, void* out,
                     int64_t ldo, void* ws, size_t ws_bytes, void* stream);
 /* msa_qk_norm_rope for a decode step (one new token per sample, N = B) fused with msa_cache_append: the
  * normalised, rotated k row and the v row of sample b are written to kcache / vcache [b][kv_len[b]] and

@@ -65,7 +65,7 @@ SIGNATURES = {
     "msa_qkv_proj_ws": (C.c_int, [_vp, _i64, _i32, _vp, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _f32, _vp, _vp, _i32, _vp, _vp, _vp,
                                   _vp, _vp, _sz, _vp]),
     "msa_tile_workspace_bytes": (_sz, [_i64, _i32, _i32]),
-    "msa_tile_linear": (C.c_int, [_vp, _i64, _i64, _i32, _vp, _i32, _i32, _vp, _i64, _vp, _sz, _vp]),
+    "msa_tile_linear": (C.c_int, [_vp, _i64, _i64, _i32, _vp, _i32, _vp, _vp, _i64, _vp, _sz, _vp]),
     "msa_qk_norm_rope_append": (C.c_int, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _f32, _vp, _vp, _i32, _i32, _i32,
                                           _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _vp]),
     "msa_rmsnorm": (C.c_int, [_vp, _vp, _vp, _i32, _i64, _i32, _f32, _vp, _vp]),
@@ -79,6 +79,14 @@ SIGNATURES = {
     "msa_sparse_attn": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _f32,
                                   _i32, _vp, _vp, _sz, _vp]),
 }
+
+
+class TileEnd(C.Structure):
+    """``msa_tile_end``."""
+    _fields_ = [("mode", _i32), ("gelu_n", _i32), ("limit", _f32), ("alpha", _f32), ("shift", _f32)]
+
+
+TILE_STORE, TILE_ADD, TILE_SILU_MUL, TILE_GLU, TILE_GELU = 0, 1, 2, 4, 5
 
 
 class SeqBatch(C.Structure):

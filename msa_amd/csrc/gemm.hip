@@ -14,6 +14,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "seq_common.h"
 
 namespace {
 
@@ -26,7 +27,8 @@ constexpr int kCompilerVgprs = 128;            // the compiler's share of the ve
 constexpr int kXcds = 8;
 constexpr int kPieceBytes = kTile * kTile * 4;
 
-enum { kStore = MSA_TILE_STORE, kAdd = MSA_TILE_ADD, kSiluMul = MSA_TILE_SILU_MUL, kHeads = 3 };
+enum { kStore = MSA_TILE_STORE, kAdd = MSA_TILE_ADD, kSiluMul = MSA_TILE_SILU_MUL, kHeads = 3, kGlu = MSA_TILE_GLU, kGelu = MSA_TILE_GELU };
+constexpr bool is_pair(int mode) { return mode == kSiluMul || mode == kGlu; }      // two weight rows an output
 
 struct TileArgs {
   const bf16_t* x;          // [T, K], rows ldx apart
@@ -39,6 +41,7 @@ struct TileArgs {
   int32_t split;            // K pieces of a tile of the last, incomplete round
   int32_t max_rem;          // tiles of that round in the XCD that has most of them
   int32_t stream;           // the output is larger than what the caches would keep for its reader: stored non-temporal
+  msa_tile_end end;
   // kHeads: w's heads are front plain heads | q | k | v | back plain heads
   const int64_t* pos;       // [T]
   const bf16_t* q_norm_w;   // [128]
@@ -99,15 +102,15 @@ __device__ inline bool item_at(const TileArgs& a, const Share& share, int xcd, i
 }
 
 // Output of a lane's value: row block i (of eight), register r, lane group g.
-//  kStore, kAdd, kHeads: weight row 32 (i / 2) + 8 g + 4 (i % 2) + r of the wavefront's 128
-//  kSiluMul:             output 32 (i / 4) + 8 g + 4 (i % 2) + r of its 64, gate in blocks with i / 2 even, up in the others; the weight's
-//                        rows are 8 gates, 8 ups, 8 gates, ...
+//  kStore, kAdd, kGelu, kHeads: weight row 32 (i / 2) + 8 g + 4 (i % 2) + r of the wavefront's 128
+//  kSiluMul, kGlu: output 32 (i / 4) + 8 g + 4 (i % 2) + r of its 64, gate in blocks with i / 2 even, up in the others; the weight's
+//                  rows are 8 gates, 8 ups, 8 gates, ... (kSiluMul) or gate, up, gate, ... (kGlu)
 template <int kMode>
 __host__ __device__ inline int weight_row(int lds_row) {
   const int wave_rows = lds_row & ~127, i = (lds_row >> 4) & 7, g = (lds_row >> 2) & 3, r = lds_row & 3;
-  if (kMode == kSiluMul) {
-    const int o = 32 * (i >> 2) + 8 * g + 4 * (i & 1) + r;
-    return wave_rows + 16 * (o >> 3) + (o & 7) + 8 * ((i >> 1) & 1);
+  if (is_pair(kMode)) {
+    const int o = 32 * (i >> 2) + 8 * g + 4 * (i & 1) + r, up = (i >> 1) & 1;
+    return wave_rows + (kMode == kGlu ? 2 * o + up : 16 * (o >> 3) + (o & 7) + 8 * up);
   }
   return wave_rows + 32 * (i >> 1) + 8 * g + 4 * (i & 1) + r;
 }
@@ -202,7 +205,7 @@ struct Finish {
   }
   // next: the token whose parts are requested (its table row), behind T there is none
   __device__ void finish(int token, float (&v)[32], Ahead& h, bool more, int next, int next_row) {
-    if constexpr (kMode == kStore || kMode == kAdd) {
+    if constexpr (kMode == kStore || kMode == kAdd || kMode == kGelu) {
       bf16_t* row = a.out + (int64_t)token * a.ldo + n0 + 8 * g;
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
@@ -213,9 +216,16 @@ struct Finish {
           for (int e = 0; e < 8; ++e) v[8 * m + e] += o[e];
           if (more) request(m, next, next_row, h);
         }
+        if constexpr (kMode == kGelu) {
+          if (n0 < a.end.gelu_n) {                 // (the same for all lanes)
+            const bool through = n0 + 32 * m + 8 * g < a.end.gelu_n;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[8 * m + e] = through ? gelu_tanh_f(v[8 * m + e]) : v[8 * m + e];
+          }
+        }
         if (m & 1) store_lines(row + 32 * (m - 1), a.ldo, token, a.T, a.N - (n0 + 32 * (m - 1) + 8 * g), pack8(v + 8 * m - 8), pack8(v + 8 * m), a.stream);
       }
-    } else if constexpr (kMode == kSiluMul) {
+    } else if constexpr (is_pair(kMode)) {
       const int n1 = n0 / 2;
       uint4 packed[2];
 #pragma unroll
@@ -224,7 +234,7 @@ struct Finish {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float gate = v[16 * m + e], up = v[16 * m + 8 + e];
-          o[e] = gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)) * up;
+          o[e] = kMode == kGlu ? clamped_glu_f(gate, up, a.end.limit, a.end.alpha, a.end.shift) : silu_f(gate) * up;
         }
         packed[m] = pack8(o);
       }
@@ -466,7 +476,7 @@ template <int kMode>
 int launch_tiles(TileArgs a, const Plan& p, hipStream_t st) {
   // Half of the memory-side cache: an output within it is still there for its reader (a 32771-token encoding block through two layers
   // takes 11.98 ms with all outputs non-temporal, 11.89 with none, 11.87 with the large ones).
-  a.stream = (int64_t)a.T * a.N * (kMode == kSiluMul ? 1 : 2) > (int64_t)128 << 20;
+  a.stream = (int64_t)a.T * a.N * (is_pair(kMode) ? 1 : 2) > (int64_t)128 << 20;
   a.tiles_t = p.tiles_t; a.tiles_n = p.tiles_n; a.group = p.group; a.split = p.split; a.max_rem = p.max_rem;
   auto kern = tile_gemm_kernel<kMode>;
   static std::atomic<int> lds_limit_raised{0}, resources_checked{0};
@@ -499,23 +509,29 @@ extern "C" size_t msa_tile_workspace_bytes(int64_t T, int32_t K, int32_t N) {
   return make_plan(T, K, N, true).bytes;
 }
 
-extern "C" int msa_tile_linear(const void* x, int64_t ldx, int64_t T, int32_t K, const void* w, int32_t N, int32_t mode, void* out,
+extern "C" int msa_tile_linear(const void* x, int64_t ldx, int64_t T, int32_t K, const void* w, int32_t N, const msa_tile_end* end, void* out,
                                int64_t ldo, void* ws, size_t ws_bytes, void* stream) {
-  MSA_REQUIRE(x && w && out, "msa_tile_linear: null pointer");
+  MSA_REQUIRE(x && w && out && end, "msa_tile_linear: null pointer");
   if (const int rc = check_operands("msa_tile_linear", x, T, ldx, w, K, N)) return rc;
-  MSA_REQUIRE(mode == MSA_TILE_STORE || mode == MSA_TILE_ADD || mode == MSA_TILE_SILU_MUL, "msa_tile_linear: mode %d", mode);
-  MSA_REQUIRE(N % (mode == MSA_TILE_SILU_MUL ? 16 : 8) == 0, "msa_tile_linear: N=%d", N);
-  MSA_REQUIRE(ldo >= (mode == MSA_TILE_SILU_MUL ? N / 2 : N) && ldo % 8 == 0 && ((uintptr_t)out & 15) == 0,
+  const int mode = end->mode;
+  MSA_REQUIRE(mode == kStore || mode == kAdd || mode == kGelu || is_pair(mode), "msa_tile_linear: mode %d", mode);
+  MSA_REQUIRE(N % (is_pair(mode) ? 16 : 8) == 0, "msa_tile_linear: N=%d", N);
+  MSA_REQUIRE(mode != kGelu || (end->gelu_n >= 0 && end->gelu_n <= N && end->gelu_n % 8 == 0), "msa_tile_linear: gelu_n=%d", end->gelu_n);
+  MSA_REQUIRE(ldo >= (is_pair(mode) ? N / 2 : N) && ldo % 8 == 0 && ((uintptr_t)out & 15) == 0,
               "msa_tile_linear: out must be 16-byte aligned, its row stride (%lld) a multiple of 8", (long long)ldo);
   TileArgs a{};
   a.x = static_cast<const bf16_t*>(x); a.w = static_cast<const bf16_t*>(w); a.out = static_cast<bf16_t*>(out);
-  a.ldx = ldx; a.ldo = ldo; a.T = (int32_t)T; a.K = K; a.N = N;
+  a.ldx = ldx; a.ldo = ldo; a.T = (int32_t)T; a.K = K; a.N = N; a.end = *end;
   Plan p = make_plan(T, K, N, ws != nullptr);
   if (p.bytes > ws_bytes || ((uintptr_t)ws & 15)) p = make_plan(T, K, N, false);
   a.pieces = static_cast<float*>(ws);
-  if (mode == MSA_TILE_STORE) return launch_tiles<kStore>(a, p, as_stream(stream));
-  if (mode == MSA_TILE_ADD) return launch_tiles<kAdd>(a, p, as_stream(stream));
-  return launch_tiles<kSiluMul>(a, p, as_stream(stream));
+  switch (mode) {
+    case kStore: return launch_tiles<kStore>(a, p, as_stream(stream));
+    case kAdd: return launch_tiles<kAdd>(a, p, as_stream(stream));
+    case kGelu: return launch_tiles<kGelu>(a, p, as_stream(stream));
+    case kGlu: return launch_tiles<kGlu>(a, p, as_stream(stream));
+    default: return launch_tiles<kSiluMul>(a, p, as_stream(stream));
+  }
 }
 
 extern "C" int msa_qkv_proj_ws(const void* x, int64_t T, int32_t K, const void* w, int32_t Hq, int32_t Hkv, int32_t Hr_front,

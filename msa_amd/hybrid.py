@@ -9,7 +9,6 @@ besides the state-space / attention step.
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 
 from . import seq_ops
 from .cache import SequenceStateCache
@@ -63,13 +62,12 @@ class HybridForCausalLM(StepDecoder):
             if h is None:
                 x, h, hs = seq_ops.residual_norm(x, batch, dt, **self._consumer(r, cache))
             after = {} if self._starts_pass(r + 1) else self._consumer(r + 1, cache)
-            y = F.linear(layer.mixer.mix(F.linear(hs, layer.mixer.w_in), state, batch), layer.w_o)
+            y = seq_ops.product(layer.mixer.mix(seq_ops.product(hs, layer.mixer.w_in), state, batch), layer.w_o)
             nxt = {"norm": layer.norm2} if layer.mlp is not None else after
-            x, h, hs = seq_ops.residual_norm(x, batch, dt, y, F.linear(h, layer.w_gate), layer.gate_b, **nxt)
+            x, h, hs = seq_ops.residual_norm(x, batch, dt, y, seq_ops.product(h, layer.w_gate), layer.gate_b, **nxt)
             if layer.mlp is not None:
-                up = F.linear(h, layer.w_up)
-                act = seq_ops.gelu_(up[:, :layer.mlp.ff])
-                x, h, hs = seq_ops.residual_norm(x, batch, dt, F.linear(act, layer.w_down), up[:, layer.n_up:], layer.gate2_b, **after)
+                up = seq_ops.product_gelu(h, layer.w_up, layer.mlp.ff)
+                x, h, hs = seq_ops.residual_norm(x, batch, dt, seq_ops.product(up[:, :layer.mlp.ff], layer.w_down), up[:, layer.n_up:], layer.gate2_b, **after)
             if trace is not None:
                 trace.append(x.clone())
         return h

@@ -432,23 +432,21 @@ def _tile_workspace(T: int, K: int, N: int, device) -> Optional[torch.Tensor]:
     return torch.empty(need, dtype=torch.uint8, device=device) if need else None
 
 
-TILE_STORE, TILE_ADD, TILE_SILU_MUL = range(3)
-
-
 def tile_linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, add: bool = False,
-                silu_mul: bool = False) -> torch.Tensor:
+                silu_mul: bool = False, glu: Optional[Tuple[float, float, float]] = None, gelu_n: int = 0) -> torch.Tensor:
     """``x @ w.T`` of a block of bf16 rows ``x [T, K]`` (unit column stride, K a multiple of 64) with a dense ``w [N, K]``, into ``out``
-    where given; ``add`` adds the product to ``out``; ``silu_mul`` takes ``w`` from ``interleave_gate_up`` and returns
-    ``silu(gate) * up`` of width ``N / 2``."""
+    where given.  At most one of: ``add`` adds the product to ``out``; ``silu_mul`` takes ``w`` from ``interleave_gate_up`` and returns
+    ``silu(gate) * up`` of width ``N / 2``; ``glu`` (limit, alpha, shift) takes rows in (gate, up) pairs and returns the clamped gated
+    unit; ``gelu_n`` puts the first columns through gelu."""
     _need_cuda(w)
     if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or x.stride(1) != 1 or not x.is_cuda:
         raise ValueError("tile_linear: x [T, K] with unit column stride, w [N, K] contiguous, both on the device")
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise ValueError("tile_linear: x and w in bf16")
+    if add + silu_mul + (glu is not None) + (gelu_n != 0) > 1 or (add and out is None):
+        raise ValueError("tile_linear: one of add (with out), silu_mul, glu and gelu_n")
     (T, K), N = x.shape, w.shape[0]
-    if add and (silu_mul or out is None):
-        raise ValueError("tile_linear: add needs out and excludes silu_mul")
-    width = N // 2 if silu_mul else N
+    width = N // 2 if silu_mul or glu is not None else N
     if out is None:
         out = torch.empty((T, width), dtype=x.dtype, device=x.device)
     elif tuple(out.shape) != (T, width) or out.dtype != x.dtype or out.stride(1) != 1 or not out.is_cuda:
@@ -456,9 +454,12 @@ def tile_linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
     if not T:
         return out
     ws = _tile_workspace(T, K, N, x.device)
+    mode = (_lib.TILE_ADD if add else _lib.TILE_SILU_MUL if silu_mul else _lib.TILE_GLU if glu is not None
+            else _lib.TILE_GELU if gelu_n else _lib.TILE_STORE)
+    end = _lib.TileEnd(mode, gelu_n, *(glu or (0.0, 0.0, 0.0)))
     rows = lambda t: t.stride(0) if T > 1 else t.shape[1]
-    check(_lib.load().msa_tile_linear(ptr(x), rows(x), T, K, ptr(w), N, TILE_SILU_MUL if silu_mul else TILE_ADD if add else TILE_STORE,
-                                      ptr(out), rows(out), ptr(ws), 0 if ws is None else ws.numel(), _stream()), "msa_tile_linear")
+    check(_lib.load().msa_tile_linear(ptr(x), rows(x), T, K, ptr(w), N, C.byref(end), ptr(out), rows(out), ptr(ws),
+                                      0 if ws is None else ws.numel(), _stream()), "msa_tile_linear")
     return out
 
 
@@ -470,8 +471,12 @@ def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1) -> bool:
     compute units.  Below ``TILE_MIN`` tiles the vendor's smaller ones win (us, vendor and here, K x N: 2560 x 2560 of 2048 tokens, 80
     tiles, 31 and 43; of 4096, 160 tiles, 50 and 51; of 16384, 640 tiles, 233 and 161; 2560 x 19456 of 1000, 304 tiles, 102 and 90).
     Depths under 1024 were not measured and stay where they were."""
-    T, K, N = x.numel() // max(x.shape[-1], 1), x.shape[-1], matrices * w.shape[0]
+    K, N = x.shape[-1], matrices * w.shape[0]
+    T = x.shape[0] if x.dim() == 2 else x.numel() // max(K, 1)
+    if (T + 255) * (N + 255) < TILE_MIN << 16:      # (most calls end here: steps of few tokens wait for the host)
+        return False
     return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == K
+            and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 21))
             and K % 64 == 0 and 1024 <= K <= 32768 and N % 8 == 0 and N < 1 << 20 and T < 1 << 22
             and -(-T // 256) * -(-N // 256) >= TILE_MIN and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))

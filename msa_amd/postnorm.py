@@ -7,8 +7,6 @@ that reads it (``seq_ops.PostRows``), the convolution into the mixer's input pro
 """
 from __future__ import annotations
 
-import torch.nn.functional as F
-
 from . import seq_ops
 from .config import PostNormConfig
 from .hybrid_layers import F32, PostNormLayer
@@ -52,8 +50,8 @@ class PostNormForCausalLM(StepDecoder):
     def _block_rows(self, tokens, batch, cache, trace=None):
         """Any rows: every element-wise step a kernel of its own between the products."""
         return self._layers(tokens, trace,
-                            lambda r, l, h: l.mixer.mix(F.linear(h, l.mixer.w_in), self.run_state(cache, r), batch), F.linear,
-                            lambda l, h: seq_ops.clamped_glu(F.linear(h, l.w_gate_up), l.mlp.limit))
+                            lambda r, l, h: l.mixer.mix(seq_ops.product(h, l.mixer.w_in), self.run_state(cache, r), batch), seq_ops.product,
+                            lambda l, h: seq_ops.product_glu(h, l.w_gate_up, l.mlp.limit))
 
     def _decode_rows(self, tokens, batch, cache, trace=None):
         """One token for each of up to 16 sequences (bf16)."""

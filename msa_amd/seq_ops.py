@@ -8,8 +8,9 @@ from typing import Optional, Sequence
 
 import numpy as np
 import torch
+import torch.nn.functional as F
 
-from . import _lib
+from . import _lib, ops
 from ._lib import dtype_code, ptr
 
 MAX_ROWS = 16           # rows of a step that the weight-streaming kernels take
@@ -185,6 +186,27 @@ def clamped_glu(gu: torch.Tensor, limit: float, alpha: float = GLU_ALPHA, shift:
     _check(_lib.load_seq().msa_seq_clamped_glu(ptr(gu), _rows(gu), dtype_code(gu.dtype), T, n, limit, alpha, shift, ptr(out), _stream()),
            "msa_seq_clamped_glu")
     return out
+
+
+def product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``x @ w.T`` of a step's rows."""
+    return ops.tile_linear(x, w) if ops.tile_linear_ok(x, w) else F.linear(x, w)
+
+
+def product_gelu(x: torch.Tensor, w: torch.Tensor, n: int) -> torch.Tensor:
+    """``x @ w.T``, its first ``n`` columns through gelu."""
+    if n % 8 == 0 and ops.tile_linear_ok(x, w):
+        return ops.tile_linear(x, w, gelu_n=n)
+    y = F.linear(x, w)
+    gelu_(y[:, :n])
+    return y
+
+
+def product_glu(x: torch.Tensor, w: torch.Tensor, limit: float, alpha: float = GLU_ALPHA, shift: float = GLU_SHIFT) -> torch.Tensor:
+    """``clamped_glu(x @ w.T)``."""
+    if w.shape[0] % 16 == 0 and ops.tile_linear_ok(x, w):
+        return ops.tile_linear(x, w, glu=(limit, alpha, shift))
+    return clamped_glu(F.linear(x, w), limit, alpha, shift)
 
 
 def gelu_(y: torch.Tensor) -> torch.Tensor:

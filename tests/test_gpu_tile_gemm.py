@@ -1,5 +1,5 @@
 """Products of a block of tokens (``ops.tile_linear``) against fp32: edges of the 256 x 256 tiles, one K tile and many, tiles multiplied in
-pieces, row strides, and every end (store, add, silu-mul; the heads' norm and rotary are tested with ``qkv_proj``).
+pieces, row strides, and every end (store, add, silu-mul, clamped unit, gelu; the heads' norm and rotary are tested with ``qkv_proj``).
 
 One rounding to bf16 leaves a relative error of up to 2^-9 a value, 1.7e-3 over many; the fp32 sums are far below it."""
 import pytest
@@ -63,6 +63,24 @@ def test_silu_mul(ops, T, K, N):
     up = (torch.randn((N // 2, K), device="cuda") * K ** -0.5).bfloat16()
     got = ops.tile_linear(x, ops.interleave_gate_up(gate, up), silu_mul=True)
     assert _err(got, torch.nn.functional.silu(want_gate) * (x.float() @ up.float().t())) < TOL
+
+
+@pytest.mark.parametrize("T,K,N", [(1, 64, 16), (129, 128, 272), (2100, 4096, 2592), (2048, 1024, 4096)])
+def test_glu(ops, T, K, N):
+    """Rows in (gate, up) pairs; sums up to 4 against a limit of 1.5, so that both are clamped."""
+    _say(f"glu T={T} K={K} N={N}")
+    x, w, want = _operands(T, K, N, 6)
+    got = ops.tile_linear(x, w, glu=(1.5, 1.702, 1.0))
+    gate, up = want[:, 0::2].clamp(max=1.5), want[:, 1::2].clamp(-1.5, 1.5)
+    assert _err(got, gate * torch.sigmoid(1.702 * gate) * (up + 1.0)) < TOL
+
+
+@pytest.mark.parametrize("T,K,N,n", [(1, 64, 8, 8), (129, 128, 264, 136), (257, 256, 512, 128), (2100, 4096, 2576, 1304), (2048, 1024, 4096, 3072)])
+def test_gelu(ops, T, K, N, n):
+    _say(f"gelu T={T} K={K} N={N} n={n}")
+    x, w, want = _operands(T, K, N, 7)
+    want[:, :n] = torch.nn.functional.gelu(want[:, :n], approximate="tanh")
+    assert _err(ops.tile_linear(x, w, gelu_n=n), want) < TOL
 
 
 def test_extreme_gates(ops):
