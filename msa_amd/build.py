@@ -55,7 +55,7 @@ def _compile(src: str) -> str:
 #  * score_scan4_kernel (route_score.hip): its asm statements own v128-v255 and all accumulation registers across
 #    statements.  The code the compiler generates for that kernel must therefore stay below v128, touch no
 #    accumulation register (the compiler would only do so to spill), and use no scratch memory.
-#  * tile_gemm_kernel (gemm.hip): the same registers.
+#  * tile_gemm_kernel (gemm.hip): the same registers; tile_flow_kernel: v24-v255 and all accumulation registers.
 #  * flash_wide_kernel (flash_attn.hip): likewise, its statements own v56-v255 and all accumulation registers.
 #  * flash_attn_kernel (flash_attn.hip): its direct-to-LDS loads are asm statements the compiler does not order
 #    against LDS reads; a spill would add vector-memory waits in the middle of that ring.  No scratch, no spills.
@@ -65,7 +65,7 @@ def _compile(src: str) -> str:
 # ---------------------------------------------------------------------------------------------------------------
 CONTRACTS = {
     "route_score.hip": [("score_scan4_kernel", {"max_compiler_vgpr": 127, "no_agpr": True})],
-    "gemm.hip": [("tile_gemm_kernel", {"max_compiler_vgpr": 127, "no_agpr": True})],
+    "gemm.hip": [("tile_gemm_kernel", {"max_compiler_vgpr": 127, "no_agpr": True}), ("tile_flow_kernel", {"max_compiler_vgpr": 23, "no_agpr": True})],
     "flash_attn.hip": [("flash_attn_kernel", {}), ("flash_wide_kernel", {"max_compiler_vgpr": 55, "no_agpr": True})],
     "linear.hip": [("rows_ring_kernel", {})],
     "seq_rows.hip": [("rows_ring_kernel", {})],
@@ -196,7 +196,7 @@ def build(jobs: int = 8) -> str:
     """Compiles every source (always, even if the libraries exist), checks the inline-asm contracts on the device
     assembly and links both shared libraries."""
     srcs = sources()
-    for gen, inc in (("gen_scan_asm.py", "{scan,gemm}_asm.inc"), ("gen_flash_asm.py", "flash_asm.inc")):
+    for gen, inc in (("gen_scan_asm.py", "scan_asm.inc"), ("gen_flash_asm.py", "flash_asm.inc")):
         if subprocess.run([sys.executable, os.path.join(CSRC, gen), "--check"]).returncode != 0:
             raise RuntimeError(f"csrc/{inc} is not what csrc/{gen} generates: run the generator")
     checked = [s for s in srcs if os.path.basename(s) in {**CONTRACTS, **LDS_WAITS}]

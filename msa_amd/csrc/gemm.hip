@@ -42,6 +42,7 @@ struct TileArgs {
   int32_t max_rem;          // tiles of that round in the XCD that has most of them
   int32_t stream;           // the output is larger than what the caches would keep for its reader: stored non-temporal
   msa_tile_end end;
+  float rate;               // -log2(e) alpha
   // kHeads: w's heads are front plain heads | q | k | v | back plain heads
   const int64_t* pos;       // [T]
   const bf16_t* q_norm_w;   // [128]
@@ -273,6 +274,48 @@ struct Finish {
   }
 };
 
+#if defined(__HIP_DEVICE_COMPILE__)
+// Per-lane constants of the asm statements: LDS offsets of the operand fragments of the two sub-steps, and the global offsets of the
+// lane's 16 bytes in the wavefront's eight 1 KB blocks of either tile (lane l lands at byte 16 l of its block, row l / 8, unit slot
+// l % 8, and fetches the unit that belongs there).
+template <int kMode>
+__device__ __forceinline__ void set_operand_registers(int lane, int wave, int ldw, int ldx) {
+  int v[4];
+#define MSA_GEMM_SET(TEXT) asm volatile(TEXT ::"v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]) : MSA_GEMM_CLOBBERS)
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int sw = ((s * 4 + (lane >> 4)) ^ (((lane & 15) >> 1) & 7)) * 16;
+    v[s] = ((wave >> 1) * 128 + (lane & 15)) * 128 + sw;
+    v[2 + s] = ((wave & 1) * 128 + (lane & 15)) * 128 + sw;
+  }
+  MSA_GEMM_SET(MSA_GEMM_SET_ADDR);
+  auto blocks = [&](int first, bool weights) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = (wave * 8 + first + i) * 8 + (lane >> 3);
+      v[i] = (weights ? weight_row<kMode>(row) * ldw : row * ldx) + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    }
+  };
+  blocks(0, true);
+  MSA_GEMM_SET(MSA_GEMM_SET_VOFF_A0);
+  blocks(4, true);
+  MSA_GEMM_SET(MSA_GEMM_SET_VOFF_A1);
+  blocks(0, false);
+  MSA_GEMM_SET(MSA_GEMM_SET_VOFF_B0);
+  blocks(4, false);
+  MSA_GEMM_SET(MSA_GEMM_SET_VOFF_B1);
+#undef MSA_GEMM_SET
+}
+
+// One resource per operand tile whose extent is the valid part of the tile: rows behind the last read as zero (the K displacement is
+// scalar and stays inside a row).  A tile that does not exist gets an empty extent.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rows(const bf16_t* base, int ld, int row_bytes, int tile, int rows, bool valid) {
+  const int n = min(kTile, rows - tile * kTile);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(base)) + (valid ? (int64_t)tile * kTile * ld : 0), 0,
+                                           valid ? (n - 1) * ld + row_bytes : 0, 0x00020000);
+}
+#endif
+
 template <int kMode>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_vgpr(kCompilerVgprs))) void tile_gemm_kernel(TileArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -285,39 +328,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_vgpr(kCompilerV
   Item cur, nxt{};
   if (!item_at(a, share, xcd, slot, per_xcd, k_tiles, 0, cur)) return;
   const int ldw = a.K * 2, ldx = (int)a.ldx * 2;
-  {
-    // LDS offsets of the operand fragments of the two sub-steps, and the global offsets of the lane's 16 bytes in the wavefront's
-    // eight 1 KB blocks of either tile (lane l lands at byte 16 l of its block, row l / 8, unit slot l % 8, and fetches the unit that
-    // belongs there)
-    int aa[2], ab[2], va[8], vb[8];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int sw = ((s * 4 + (lane >> 4)) ^ (((lane & 15) >> 1) & 7)) * 16;
-      aa[s] = (wm * 128 + (lane & 15)) * 128 + sw;
-      ab[s] = (wn * 128 + (lane & 15)) * 128 + sw;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int row = (wave * 8 + i) * 8 + (lane >> 3);
-      const int unit = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
-      va[i] = weight_row<kMode>(row) * ldw + unit;
-      vb[i] = row * ldx + unit;
-    }
-    asm volatile(MSA_GEMM_SET_ADDR ::"v"(aa[0]), "v"(aa[1]), "v"(ab[0]), "v"(ab[1]) : MSA_GEMM_CLOBBERS);
-    asm volatile(MSA_GEMM_SET_VOFF_A ::"v"(va[0]), "v"(va[1]), "v"(va[2]), "v"(va[3]), "v"(va[4]), "v"(va[5]), "v"(va[6]), "v"(va[7])
-                 : MSA_GEMM_CLOBBERS);
-    asm volatile(MSA_GEMM_SET_VOFF_B ::"v"(vb[0]), "v"(vb[1]), "v"(vb[2]), "v"(vb[3]), "v"(vb[4]), "v"(vb[5]), "v"(vb[6]), "v"(vb[7])
-                 : MSA_GEMM_CLOBBERS);
-  }
-  // One resource per operand tile whose extent is the valid part of the tile: rows behind N / T read as zero (the K displacement is
-  // scalar and stays inside a row).  A tile that does not exist gets an empty extent.
-  auto rows_of = [&](const bf16_t* base, int ld, int tile, int rows, bool valid) {
-    const int n = min(kTile, rows - tile * kTile);
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(base)) + (valid ? (int64_t)tile * kTile * ld : 0), 0,
-                                             valid ? (n - 1) * ld + a.K * 2 : 0, 0x00020000);
-  };
-  auto make_a = [&](const Item& it, bool valid) { return rows_of(a.w, ldw, it.tile_n, a.N, valid); };
-  auto make_b = [&](const Item& it, bool valid) { return rows_of(a.x, ldx, it.tile_t, a.T, valid); };
+  set_operand_registers<kMode>(lane, wave, ldw, ldx);
+  auto make_a = [&](const Item& it, bool valid) { return tile_rows(a.w, ldw, a.K * 2, it.tile_n, a.N, valid); };
+  auto make_b = [&](const Item& it, bool valid) { return tile_rows(a.x, ldx, a.K * 2, it.tile_t, a.T, valid); };
   const bool single = k_tiles == 1;              // the second K tile of every tile does not exist: zeros
   int n_item = 0;
   __amdgpu_buffer_rsrc_t ra_c = make_a(cur, true), rb_c = make_b(cur, true), ra_n, rb_n;
@@ -375,18 +388,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_vgpr(kCompilerV
                  "=v"(v[16 * H + 15]))
     if (cur.piece < 0) {
       Finish<kMode> f(a, cur.tile_n * kTile + wm * 128, lane);
-      int pos[8] = {};
-      if constexpr (kMode == kHeads) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) pos[j] = f.table_row(token0 + 16 * j);
-      }
+      auto table_row = [&](int j) { return kMode == kHeads ? f.table_row(token0 + 16 * j) : 0; };
       typename Finish<kMode>::Ahead ahead;
+      int row = table_row(0);
 #pragma unroll
-      for (int m = 0; m < 4; ++m) f.request(m, token0, pos[0], ahead);
+      for (int m = 0; m < 4; ++m) f.request(m, token0, row, ahead);
+      row = table_row(1);
 #define MSA_GEMM_COLUMN(J)                                                                       \
-  MSA_GEMM_READ(J, 0);                                                                           \
-  MSA_GEMM_READ(J, 1);                                                                           \
-  f.finish(token0 + 16 * J, v, ahead, J < 7, token0 + 16 * (J + 1), pos[(J + 1) & 7]);
+  {                                                                                              \
+    const int row2 = J < 6 ? table_row(J + 2) : 0;                                               \
+    MSA_GEMM_READ(J, 0);                                                                         \
+    MSA_GEMM_READ(J, 1);                                                                         \
+    f.finish(token0 + 16 * J, v, ahead, J < 7, token0 + 16 * (J + 1), row);                      \
+    row = row2;                                                                                  \
+  }
       MSA_GEMM_COLUMN(0) MSA_GEMM_COLUMN(1) MSA_GEMM_COLUMN(2) MSA_GEMM_COLUMN(3)
       MSA_GEMM_COLUMN(4) MSA_GEMM_COLUMN(5) MSA_GEMM_COLUMN(6) MSA_GEMM_COLUMN(7)
 #undef MSA_GEMM_COLUMN
@@ -401,6 +416,142 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_vgpr(kCompilerV
 #undef MSA_GEMM_COLUMN
     }
 #undef MSA_GEMM_READ
+    if (!more) break;
+    cur = nxt;
+    ra_c = ra_n; rb_c = rb_n;
+    plan_next();
+  }
+#undef MSA_GEMM_STEP
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+#endif
+}
+
+// The same walk for ends that need nothing but the sums: a finished tile is rounded to bf16 into 128 registers while the next tile's
+// first step overwrites its accumulators, and finished and stored, sixteen tokens a step, behind the MFMAs of the eight steps after that
+// (gen_scan_asm.py).  A wavefront is alone on its SIMD, so whatever it does between two tiles the matrix cores wait for: storing a
+// tile took it 5 us, gelu 10, against 57 us of steps at K = 2560 and 23 at K = 1024.  Whole calls, us, ends in registers and here: 32771 x
+// 2560 x 19456 stored 2392 and 2238, 6001 x 2560 x 19456 with the gated unit 434 and 415, 8192 x 1024 x 4096 with gelu 88 and 60.  (silu-mul:
+// 2257 and 2221, 11.99 and 12.00 ms for the block it is part of: its half output leaves little to hide, and power bounds the rest.)
+constexpr int kFlowVgprs = 24;                 // the compiler's share of the vector registers
+constexpr int kFlowSteps = 11;                 // an item of that many steps takes another tile's end: one packs, eight finish, the
+                                               // last two already load for the item behind
+constexpr int kFar = 0x7ff00000;               // behind every extent, whatever is added: nothing is stored
+
+template <int kMode, bool kStream>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_vgpr(kFlowVgprs))) void tile_flow_kernel(TileArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int per_xcd = gridDim.x / kXcds, xcd = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
+  const int k_tiles = a.K * 2 / kRowBytes;
+  const Share share = tile_share(a.tiles_t * a.tiles_n, per_xcd, xcd);
+  Item cur, nxt{};
+  if (!item_at(a, share, xcd, slot, per_xcd, k_tiles, 0, cur)) return;
+  const int ldw = a.K * 2, ldx = (int)a.ldx * 2;
+  set_operand_registers<kMode>(lane, wave, ldw, ldx);
+  if constexpr (kMode == kGelu) asm volatile(MSA_GEMM_SET_GELU ::: MSA_GEMM_FLOW_CLOBBERS);
+  auto make_a = [&](const Item& it, bool valid) { return tile_rows(a.w, ldw, a.K * 2, it.tile_n, a.N, valid); };
+  auto make_b = [&](const Item& it, bool valid) { return tile_rows(a.x, ldx, a.K * 2, it.tile_t, a.T, valid); };
+  // the output behind a tile's first token and column
+  constexpr int kCols = is_pair(kMode) ? kTile / 2 : kTile;
+  const int width = is_pair(kMode) ? a.N / 2 : a.N, ldo = (int)a.ldo * 2;
+  auto make_out = [&](const Item& it) {
+    const int rows = min(kTile, a.T - it.tile_t * kTile), at = it.tile_n * kCols;
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(a.out) + (int64_t)it.tile_t * kTile * ldo + at * 2, 0,
+                                             (rows - 1) * ldo + (width - at) * 2, 0x00020000);
+  };
+  // a lane's offsets in it: the columns of its group, tokens of the first eight of a column block in the lower lanes
+  int so0, so1;
+  auto set_offsets = [&](const Item& it) {
+    const bool low = (lane & 8) == 0;
+    const int col = wm * (kCols / 2) + 8 * (lane >> 4) + (low ? 0 : 32), at = it.tile_n * kCols + col;
+    const int row = (wn * 128 + (lane & 7)) * ldo + col * 2;
+    so0 = at < width ? row : kFar;
+    so1 = at + 64 < width ? row + 128 : kFar;
+  };
+
+  int n_item = 0;
+  __amdgpu_buffer_rsrc_t ra_c = make_a(cur, true), rb_c = make_b(cur, true), ra_n, rb_n, ro = make_out(cur);
+  bool more;
+  auto plan_next = [&]() {
+    more = item_at(a, share, xcd, slot, per_xcd, k_tiles, ++n_item, nxt);
+    ra_n = make_a(nxt, more);
+    rb_n = make_b(nxt, more);
+  };
+  plan_next();
+  const int woff = wave * 8192, row8 = 8 * ldo, row16 = 16 * ldo;
+  int sa = 0, sb = 0x10000;
+  {
+    const int k = cur.k0 * kRowBytes;
+    asm volatile(MSA_GEMM_LOAD8_B ::[dst] "s"(0x10000 + woff), [r] "s"(rb_c), [k] "s"(k) : MSA_GEMM_FLOW_CLOBBERS);
+    asm volatile(MSA_GEMM_LOAD8_A ::[dst] "s"(0 + woff), [r] "s"(ra_c), [k] "s"(k) : MSA_GEMM_FLOW_CLOBBERS);
+    asm volatile(MSA_GEMM_LOAD8_B ::[dst] "s"(0x18000 + woff), [r] "s"(rb_c), [k] "s"(k + kRowBytes) : MSA_GEMM_FLOW_CLOBBERS);
+    asm volatile(MSA_GEMM_LOAD8_A ::[dst] "s"(0x8000 + woff), [r] "s"(ra_c), [k] "s"(k + kRowBytes) : MSA_GEMM_FLOW_CLOBBERS);
+  }
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  asm volatile(MSA_GEMM_FRAGS0 ::[sa] "s"(sa), [sb] "s"(sb) : MSA_GEMM_FLOW_CLOBBERS);
+
+#define MSA_GEMM_STEP(TEXT, RA, RB, KOFF)                                                                    \
+  asm volatile(TEXT : [sa] "+s"(sa), [sb] "+s"(sb)                                                           \
+               : [ra] "s"(RA), [rb] "s"(RB), [k] "s"(KOFF), [woff] "s"(woff) : MSA_GEMM_FLOW_CLOBBERS)
+#define MSA_GEMM_ENDS                                                                                         \
+  [ro] "s"(ro), [row8] "s"(row8), [row16] "s"(row16), [so0] "v"(so0), [so1] "v"(so1), [limit] "s"(a.end.limit), [rate] "s"(a.rate), \
+      [shift] "s"(a.end.shift)
+#define MSA_GEMM_KSTEP_END(END, J, KOFF)                                                                     \
+  if constexpr (kStream)                                                                                     \
+    asm volatile(MSA_GEMM_KSTEP_##END##_##J(" nt") : [sa] "+s"(sa), [sb] "+s"(sb)                             \
+                 : [ra] "s"(ra_c), [rb] "s"(rb_c), [k] "s"(KOFF), [woff] "s"(woff), MSA_GEMM_ENDS : MSA_GEMM_FLOW_CLOBBERS); \
+  else                                                                                                       \
+    asm volatile(MSA_GEMM_KSTEP_##END##_##J("") : [sa] "+s"(sa), [sb] "+s"(sb)                                \
+                 : [ra] "s"(ra_c), [rb] "s"(rb_c), [k] "s"(KOFF), [woff] "s"(woff), MSA_GEMM_ENDS : MSA_GEMM_FLOW_CLOBBERS);
+#define MSA_GEMM_END(END, J)                                                                                 \
+  if constexpr (kStream) asm volatile(MSA_GEMM_END_##END##_##J(" nt") ::MSA_GEMM_ENDS : MSA_GEMM_FLOW_CLOBBERS); \
+  else asm volatile(MSA_GEMM_END_##END##_##J("") ::MSA_GEMM_ENDS : MSA_GEMM_FLOW_CLOBBERS);
+#define MSA_GEMM_EIGHT(DO, END, ...)                                                                         \
+  DO(END, 0 __VA_OPT__(, __VA_ARGS__ + 0 * kRowBytes)) DO(END, 1 __VA_OPT__(, __VA_ARGS__ + 1 * kRowBytes))  \
+  DO(END, 2 __VA_OPT__(, __VA_ARGS__ + 2 * kRowBytes)) DO(END, 3 __VA_OPT__(, __VA_ARGS__ + 3 * kRowBytes))  \
+  DO(END, 4 __VA_OPT__(, __VA_ARGS__ + 4 * kRowBytes)) DO(END, 5 __VA_OPT__(, __VA_ARGS__ + 5 * kRowBytes))  \
+  DO(END, 6 __VA_OPT__(, __VA_ARGS__ + 6 * kRowBytes)) DO(END, 7 __VA_OPT__(, __VA_ARGS__ + 7 * kRowBytes))
+#define MSA_GEMM_BY_MODE(DO, ...)                                                                            \
+  if constexpr (kMode == kStore) { MSA_GEMM_EIGHT(DO, STORE __VA_OPT__(, __VA_ARGS__)) }                     \
+  else if constexpr (kMode == kSiluMul) { MSA_GEMM_EIGHT(DO, SILU __VA_OPT__(, __VA_ARGS__)) }               \
+  else if constexpr (kMode == kGlu) { MSA_GEMM_EIGHT(DO, GLU __VA_OPT__(, __VA_ARGS__)) }                    \
+  else { MSA_GEMM_EIGHT(DO, GELU __VA_OPT__(, __VA_ARGS__)) }
+  // (gelu's columns end at a multiple of a wavefront's rows: a tile's part of the wavefront is through gelu or is not)
+  bool held = false, plain = false;              // a finished tile waits for its end (ro, so0, so1 are its); without gelu
+  for (;;) {
+    const int k_first = cur.k0 * kRowBytes, k_end = (cur.k0 + cur.nk) * kRowBytes, k_next = nxt.k0 * kRowBytes;
+    int k = k_first + 3 * kRowBytes;             // what the next step requests
+    if (held) {                                  // (cur.nk >= kFlowSteps)
+      MSA_GEMM_STEP(MSA_GEMM_KSTEP_FRESH_PACK, ra_c, rb_c, k_first + 2 * kRowBytes);
+      if (kMode == kGelu && plain) { MSA_GEMM_EIGHT(MSA_GEMM_KSTEP_END, STORE, k) }
+      else { MSA_GEMM_BY_MODE(MSA_GEMM_KSTEP_END, k) }
+      k += 8 * kRowBytes;
+    } else if (cur.nk > 2) {
+      MSA_GEMM_STEP(MSA_GEMM_KSTEP_FRESH, ra_c, rb_c, k_first + 2 * kRowBytes);
+    } else {
+      MSA_GEMM_STEP(MSA_GEMM_KSTEP_FRESH, ra_n, rb_n, k_next);
+    }
+    for (; k < k_end; k += kRowBytes) MSA_GEMM_STEP(MSA_GEMM_KSTEP, ra_c, rb_c, k);
+    if (cur.nk > 2) MSA_GEMM_STEP(MSA_GEMM_KSTEP, ra_n, rb_n, k_next);
+    MSA_GEMM_STEP(MSA_GEMM_KSTEP, ra_n, rb_n, k_next + kRowBytes);
+    held = cur.piece < 0 && more && nxt.nk >= kFlowSteps;
+    if (cur.piece >= 0) {
+      const int sp = __builtin_amdgcn_readfirstlane(wave * (kPieceBytes / 4));
+      const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(
+          reinterpret_cast<char*>(a.pieces) + (int64_t)cur.piece * kPieceBytes, 0, kPieceBytes, 0x00020000);
+      asm volatile(MSA_GEMM_PIECE ::[rp] "s"(to), [vp] "v"(lane * 16), [sp] "s"(sp) : MSA_GEMM_FLOW_CLOBBERS);
+    } else {
+      ro = make_out(cur);
+      set_offsets(cur);
+      plain = kMode == kGelu && cur.tile_n * kTile + wm * 128 >= a.end.gelu_n;
+      if (!held) {
+        asm volatile(MSA_GEMM_PACK ::: MSA_GEMM_FLOW_CLOBBERS);
+        if (kMode == kGelu && plain) { MSA_GEMM_EIGHT(MSA_GEMM_END, STORE) }
+        else { MSA_GEMM_BY_MODE(MSA_GEMM_END) }
+      }
+    }
     if (!more) break;
     cur = nxt;
     ra_c = ra_n; rb_c = rb_n;
@@ -472,25 +623,40 @@ Plan make_plan(int64_t T, int K, int N, bool may_split) {
   return p;
 }
 
+template <void (*kern)(TileArgs)>
+int launch_tile_kernel(const TileArgs& a, const Plan& p, hipStream_t st) {
+  static std::atomic<int> lds_limit_raised{0}, resources_checked{0};
+  if (const int rc = check_asm_kernel_resources(resources_checked, reinterpret_cast<const void*>(kern), "tile kernel", nullptr, nullptr)) return rc;
+  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(kern), kLdsBytes));
+  kern<<<p.grid, kThreads, kLdsBytes, st>>>(a);
+  MSA_LAUNCH_CHECK();
+  return MSA_OK;
+}
+
+template <int kMode>
+int launch_finish(const TileArgs& a, const Plan& p, hipStream_t st) {
+  tile_finish_kernel<kMode><<<kXcds * p.max_rem * 8, kThreads, 0, st>>>(a, p.grid / kXcds);
+  MSA_LAUNCH_CHECK();
+  return MSA_OK;
+}
+
 template <int kMode>
 int launch_tiles(TileArgs a, const Plan& p, hipStream_t st) {
   // Half of the memory-side cache: an output within it is still there for its reader (a 32771-token encoding block through two layers
   // takes 11.98 ms with all outputs non-temporal, 11.89 with none, 11.87 with the large ones).
   a.stream = (int64_t)a.T * a.N * (is_pair(kMode) ? 1 : 2) > (int64_t)128 << 20;
   a.tiles_t = p.tiles_t; a.tiles_n = p.tiles_n; a.group = p.group; a.split = p.split; a.max_rem = p.max_rem;
-  auto kern = tile_gemm_kernel<kMode>;
-  static std::atomic<int> lds_limit_raised{0}, resources_checked{0};
-  if (const int rc = check_asm_kernel_resources(resources_checked, reinterpret_cast<const void*>(kern), "tile_gemm_kernel", nullptr, nullptr))
-    return rc;
-  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(kern), kLdsBytes));
-  kern<<<p.grid, kThreads, kLdsBytes, st>>>(a);
-  MSA_LAUNCH_CHECK();
-  if (p.split > 1) {
-    const int per_xcd = p.grid / kXcds;
-    tile_finish_kernel<kMode><<<kXcds * p.max_rem * 8, kThreads, 0, st>>>(a, per_xcd);
-    MSA_LAUNCH_CHECK();
+  // An end under the next tile's steps wants tiles of kFlowSteps steps, and gelu's line between two wavefronts' rows.
+  constexpr bool kFlows = kMode != kAdd && kMode != kHeads;
+  if constexpr (kFlows) {
+    if (a.K >= 64 * kFlowSteps && a.ldo < ((int64_t)1 << 21) && (kMode != kGelu || a.end.gelu_n % 128 == 0)) {
+      a.rate = -1.4426950408889634f * a.end.alpha;
+      const int rc = a.stream ? launch_tile_kernel<tile_flow_kernel<kMode, true>>(a, p, st) : launch_tile_kernel<tile_flow_kernel<kMode, false>>(a, p, st);
+      return rc != MSA_OK || p.split == 1 ? rc : launch_finish<kMode>(a, p, st);
+    }
   }
-  return MSA_OK;
+  const int rc = launch_tile_kernel<tile_gemm_kernel<kMode>>(a, p, st);
+  return rc != MSA_OK || p.split == 1 ? rc : launch_finish<kMode>(a, p, st);
 }
 
 int check_operands(const char* name, const void* x, int64_t T, int64_t ldx, const void* w, int32_t K, int64_t N) {

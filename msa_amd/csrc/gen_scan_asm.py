@@ -42,7 +42,8 @@ In the products the A operand is the weights and the B operand the tokens; each 
 of the A tile, v216-v223 those of the B tile), neither is read non-temporal, and a finished tile's accumulators are read behind its
 last step.
 
-Run ``python gen_scan_asm.py`` after changing the schedule; the generated files are committed.
+Run ``python gen_scan_asm.py`` after changing the schedule; ``scan_asm.inc`` is committed, ``gemm_asm.inc`` (a copy of the step for every
+column of every end) is written by every build.
 """
 import os
 import sys
@@ -62,15 +63,27 @@ S_M0, S_AN, S_BN, S_BLD = "s92", "s93", "s94", "s95"
 B0, BEND = 0x10000, 0x28000
 
 QUADS = [[(0, 0), (0, 1), (1, 1), (1, 0)], [(0, 1), (0, 0), (1, 0), (1, 1)]]      # (A half, B half) in the order of a sub-step
-# the fragments requested during a quadrant: operand, first index, address register
-READS = [[("b", 4, VT_B0), ("a", 4, VT_A0), ("a", 0, VT_A1), ("b", 4, VT_B1)],
-         [("b", 0, VT_B1), ("a", 4, VT_A1), ("a", 0, VT_AN), ("b", 0, VT_BN)]]
+# the fragments requested during a quadrant (operand, half, address register)
+READS = [[("b", 1, VT_B0), ("a", 1, VT_A0), ("a", 0, VT_A1), ("b", 1, VT_B1)],
+         [("b", 0, VT_B1), ("a", 1, VT_A1), ("a", 0, VT_AN), ("b", 0, VT_BN)]]
 BARRIER = (1, 2)
 
 
-def acc(i, j):
-    b = (i * 8 + j) * 4
-    return f"a[{b}:{b + 3}]"
+class Tile:
+    """A wavefront's blocks (rows of A x rows of B, in sixteens) and what follows from them: LDS stages, loads of a wavefront."""
+
+    def __init__(self, a_blocks=8, b_blocks=8):
+        self.a, self.b = a_blocks, b_blocks
+        self.stage_a, self.stage_b = a_blocks * 4096, b_blocks * 4096
+        self.b0 = 2 * self.stage_a
+        self.b_end = self.b0 + 3 * self.stage_b
+
+    def acc(self, i, j):
+        b = (i * self.b + j) * 4
+        return f"a[{b}:{b + 3}]"
+
+
+SCAN = Tile()
 
 
 def frag(kind, n):
@@ -78,14 +91,16 @@ def frag(kind, n):
     return f"v[{b}:{b + 3}]"
 
 
-def order(sub, q):
-    """The quadrant's sixteen blocks: the fragments that arrived last change slowest, the others go to and fro."""
+def order(sub, q, tile=SCAN):
+    """The quadrant's blocks: the fragments that arrived last change slowest, the others go to and fro."""
     ha, hb = QUADS[sub][q]
+    na, nb = tile.a // 2, tile.b // 2
+    slow, fast = (na, nb) if q >= 2 else (nb, na)
     out = []
-    for n in range(4):
-        for m in range(4):
-            x = m if n % 2 == 0 else 3 - m
-            out.append((4 * ha + n, 4 * hb + x) if q >= 2 else (4 * ha + x, 4 * hb + n))
+    for n in range(slow):
+        for m in range(fast):
+            x = m if n % 2 == 0 else fast - 1 - m
+            out.append((na * ha + n, nb * hb + x) if q >= 2 else (na * ha + x, nb * hb + n))
     return out
 
 
@@ -217,66 +232,75 @@ def fix_lane_move_hazards(lines):
     return out
 
 
-def kstep(fresh, reduce=None, voff_b=VOFF, nt=" nt"):
-    """One K step.  Operands: [sa] / [sb] LDS stage of the step's query / K_r tile (advanced to the next step's),
-    [ra] / [rb] resources the loads of this step read, [k] their byte offset inside a row, [woff] wave * 8 KB.
+def kstep(fresh, reduce=None, tile=SCAN, voff_b=VOFF, nt=" nt", woff=("woff", "woff"), fillers=(), stores=(), early_fillers=()):
+    """One K step.  Operands: [sa] / [sb] LDS stage of the step's A / B tile (advanced to the next step's),
+    [ra] / [rb] resources the loads of this step read, [k] their byte offset inside a row, [woff] the wavefront's part of a stage.
     fresh: a tile's first step (the first sub-step multiplies into zero); reduce: it also reduces the accumulators the
-    previous tile left, "blocks" to one maximum per row block, "fold" on to the key plane ([okey]: the query's keys)."""
+    previous tile left, "blocks" to one maximum per row block, "fold" on to the key plane ([okey]: the query's keys).
+    fillers go behind the MFMAs, stores (of the tile before) behind the step's wait so that it does not count them;
+    early_fillers: a list per block in front of the MFMA that overwrites it."""
     out = []
     e = out.append
-    fillers, atomics = [], []
+    fillers, atomics, stores = list(fillers), [], list(stores)
     red = Reduction(reduce == "fold") if reduce else None
     if reduce == "fold":
         (a0, at0), (a1, at1) = fold_pair(0), fold_pair(1)
         fillers = interleave(a0, a1)
         atomics = at0 + at1
-    per_slot = -(-len(fillers) // 44)
+    blocks = tile.a * tile.b
+    per_slot = -(-len(fillers) // 44) if reduce else -(-len(fillers) // (blocks + blocks // 2 - 12)) if fillers else 0
     # The step's scalar and address arithmetic stands behind its first MFMAs, not in front of them (a wavefront that
     # is alone on its SIMD pays for every instruction the matrix pipe does not run under): `early` is what the first
     # LDS read and the first tile load need, `later` the rest, two instructions per MFMA.
     early = [f"s_mov_b32 {S_M0}, m0",
              f"v_add_u32 v{VT_B0}, %[sb], v{VADDR + 2}", f"v_add_u32 v{VT_A0}, %[sa], v{VADDR}",
-             f"s_sub_u32 {S_BLD}, %[sb], 0x8000", f"s_cmp_lt_u32 {S_BLD}, {B0:#x}",
-             f"s_cselect_b32 {S_BLD}, {BEND - 0x8000:#x}, {S_BLD}", f"s_add_u32 {S_BLD}, {S_BLD}, %[woff]"]
+             f"s_sub_u32 {S_BLD}, %[sb], {tile.stage_b:#x}", f"s_cmp_lt_u32 {S_BLD}, {tile.b0:#x}",
+             f"s_cselect_b32 {S_BLD}, {tile.b_end - tile.stage_b:#x}, {S_BLD}", f"s_add_u32 {S_BLD}, {S_BLD}, %[{woff[1]}]"]
     later = [f"v_add_u32 v{VT_A1}, %[sa], v{VADDR + 1}", f"v_add_u32 v{VT_B1}, %[sb], v{VADDR + 3}",
-             f"s_add_u32 {S_BN}, %[sb], 0x8000", f"s_cmp_eq_u32 {S_BN}, {BEND:#x}", f"s_cselect_b32 {S_BN}, {B0:#x}, {S_BN}",
-             f"s_xor_b32 {S_AN}, %[sa], 0x8000", f"v_add_u32 v{VT_AN}, {S_AN}, v{VADDR}", f"v_add_u32 v{VT_BN}, {S_BN}, v{VADDR + 2}"]
+             f"s_add_u32 {S_BN}, %[sb], {tile.stage_b:#x}", f"s_cmp_eq_u32 {S_BN}, {tile.b_end:#x}", f"s_cselect_b32 {S_BN}, {tile.b0:#x}, {S_BN}",
+             f"s_xor_b32 {S_AN}, %[sa], {tile.stage_a:#x}", f"v_add_u32 v{VT_AN}, {S_AN}, v{VADDR}", f"v_add_u32 v{VT_BN}, {S_BN}, v{VADDR + 2}"]
     if reduce == "fold":
         later += ["s_mov_b32 s86, 0", "s_mov_b32 s87, -1"]
-    pending = [("a", n) for n in range(4)] + [("b", n) for n in range(4)]      # reads in flight, oldest first: the step before left these
-    nload = 0
+    half = {"a": tile.a // 2, "b": tile.b // 2}
+    pending = [("a", n) for n in range(half["a"])] + [("b", n) for n in range(half["b"])]      # reads in flight, oldest first: the step before left these
+    quad = blocks // 4                                     # MFMAs of a quadrant
+    every = {0: 2 * quad // tile.b, 1: 2 * quad // tile.a}  # MFMAs between two tile loads of a sub-step's
+    nload = {0: 0, 1: 0}
+    read_from = 1 if quad > half["a"] else 0
     for sub in range(2):
         for q in range(4):
-            kind, first, addr = READS[sub][q]
-            for n, (i, j) in enumerate(order(sub, q)):
+            kind, which, addr = READS[sub][q]
+            for n, (i, j) in enumerate(order(sub, q, tile)):
                 if (sub, q) == BARRIER and n == 0:
-                    e("s_waitcnt vmcnt(8) lgkmcnt(0)")
+                    e(f"s_waitcnt vmcnt({tile.b}) lgkmcnt(0)")
                     pending = []
                 need = max([pending.index(x) for x in (("a", i), ("b", j)) if x in pending], default=-1)
                 if need >= 0:
                     pending = pending[need + 1:]
                     e(f"s_waitcnt lgkmcnt({len(pending)})")
-                do_load = n % 4 == 3 and (sub, q) in ((0, 0), (0, 1), (1, 2), (1, 3))
+                do_load = n % every[sub] == every[sub] - 1 and q // 2 == sub
                 if do_load:
-                    if nload % 8:
+                    if nload[sub]:
                         e("s_add_u32 m0, m0, 0x400")
                     elif sub == 0:
                         e(f"s_mov_b32 m0, {S_BLD}")
                     else:
-                        e("s_add_u32 m0, %[sa], %[woff]")
+                        e(f"s_add_u32 m0, %[sa], %[{woff[0]}]")
                 if red and sub == 0:
                     out.extend(red.block(i, j))
-                c = "0" if (fresh and sub == 0) else acc(i, j)
-                e(f"v_mfma_f32_16x16x32_bf16 {acc(i, j)}, {frag('a', i)}, {frag('b', j)}, {c}")
+                if early_fillers and sub == 0:
+                    out.extend(early_fillers[i][j])
+                c = "0" if (fresh and sub == 0) else tile.acc(i, j)
+                e(f"v_mfma_f32_16x16x32_bf16 {tile.acc(i, j)}, {frag('a', i)}, {frag('b', j)}, {c}")
                 if (sub, q) == BARRIER and n == 0:
                     e("s_barrier")
                 if (sub, q, n) == (0, 0, 0):
                     out.extend(early)
-                if (sub, q) == (0, 0) and n >= 4:
-                    for _ in range(2):
+                if (sub, q) == (0, 0) and n >= min(4, quad // 2):
+                    for _ in range(max(2, -(-len(later) // (quad - n)))):
                         if later:
                             e(later.pop(0))
-                if sub == 1 and n > (4 if q == 2 else 0):
+                if (sub == 1 and n > (4 if q == 2 else 0)) if reduce else ((sub, q) not in ((0, 0), (1, 3)) and not ((sub, q) == BARRIER and n < 2)):
                     for _ in range(per_slot):
                         if fillers:
                             e(fillers.pop(0))
@@ -284,22 +308,31 @@ def kstep(fresh, reduce=None, voff_b=VOFF, nt=" nt"):
                     assert not fillers
                     for _ in range(3):
                         e(atomics.pop(0))
-                if 1 <= n <= 4:
-                    idx = first + n - 1
+                if (sub, q) == (1, 3) and stores:
+                    assert not fillers
+                    if n % max(1, quad // len_stores) == 0:
+                        e(stores.pop(0))
+                elif (sub, q) == (1, 2):
+                    len_stores = max(1, len(stores))
+                if read_from <= n < read_from + half[kind]:
+                    idx = which * half[kind] + n - read_from
                     e(f"ds_read_b128 {frag(kind, idx)}, v{addr} offset:{idx * 2048}")
                     pending.append((kind, idx))
                 if do_load:
                     if sub == 0:
-                        e(f"buffer_load_dwordx4 v{voff_b + nload}, %[rb], %[k] offen{nt} lds")
+                        e(f"buffer_load_dwordx4 v{voff_b + nload[0]}, %[rb], %[k] offen{nt} lds")
                     else:
-                        e(f"buffer_load_dwordx4 v{VOFF + nload - 8}, %[ra], %[k] offen lds")
-                    nload += 1
+                        e(f"buffer_load_dwordx4 v{VOFF + nload[1]}, %[ra], %[k] offen lds")
+                    nload[sub] += 1
             if red and sub == 0:
                 out.extend(red.after(q))
     e(f"s_mov_b32 %[sa], {S_AN}")
     e(f"s_mov_b32 %[sb], {S_BN}")
     e(f"s_mov_b32 m0, {S_M0}")
-    assert not fillers and not atomics and not later and nload == 16 and pending[-4:] == [("b", n) for n in range(4)]
+    assert not fillers and not atomics and not later and not stores and nload == {0: tile.b, 1: tile.a}
+    scc = [l.split()[0] for l in out if l.startswith(("s_cmp", "s_cselect", "s_add_u32", "s_sub_u32", "s_xor", "s_or_b32", "s_and_save"))]
+    assert all(scc[n - 1].startswith("s_cmp") for n, l in enumerate(scc) if l == "s_cselect_b32")
+    assert pending[-half["b"]:] == [("b", n) for n in range(half["b"])]
     return fix_lane_move_hazards(out)
 
 
@@ -315,7 +348,8 @@ def reduction():
 
 
 def define(name, lines):
-    body = " \\\n".join(f'  "{l}\\n\\t"' for l in lines)
+    """(@NT in a line stands for the macro's parameter)"""
+    body = " \\\n".join(f'  "{l}\\n\\t"' for l in lines).replace("@NT", '" NT "')
     return f"#define {name} \\\n{body}\n"
 
 
@@ -341,8 +375,8 @@ def set_registers(first, count):
     return [f"v_mov_b32 v{first + s}, %{s}" for s in range(count)]
 
 
-def clobbers(name):
-    regs = [f"v{r}" for r in range(128, 256)] + [f"a{r}" for r in range(256)] + [f"s{r}" for r in range(76, 96)] + ["vcc", "scc", "memory"]
+def clobbers(name, first=128):
+    regs = [f"v{r}" for r in range(first, 256)] + [f"a{r}" for r in range(256)] + [f"s{r}" for r in range(76, 96)] + ["vcc", "scc", "memory"]
     return f"#define {name} " + ", ".join(f'"{x}"' for x in regs) + "\n"
 
 
@@ -371,36 +405,166 @@ def scan_text():
         clobbers("MSA_SCAN4_CLOBBERS")])
 
 
+# ---------------------------------------------------------------------------------------------------------------
+# The tiled products' ends under the next tile's steps (tile_flow_kernel).  A tile's first step rounds the accumulators of the tile
+# before to bf16, a block in front of the MFMA that overwrites it, into 128 held registers; each of the next eight steps finishes one
+# column block of them (128 weight rows x 16 tokens) behind its MFMAs and stores it.  Held registers of column j, row block i, pair of
+# rows p: number 16 j + 2 i + p.
+HOLD_LOW = 24                       # compiler code has the registers below
+TEMP = list(range(202, 208)) + list(range(248, 255))
+V_GELU = 255                        # a constant of gelu
+LOG2E = 1.4426950408889634
+S_LOW, S_ROW = "s[76:77]", "s78"    # lanes whose token is one of the first eight of its sixteen; byte offset of the column's rows
+
+
+def hold(n):
+    return HOLD_LOW + n if n < 128 - HOLD_LOW else 224 + n - (128 - HOLD_LOW)
+
+
+def hex_f32(x):
+    import struct
+    return f"{struct.unpack('<I', struct.pack('<f', x))[0]:#010x}"
+
+
+def pack_block(tile, i, j, t):
+    """Four accumulators, rounded, into two held registers; t: four scratch registers."""
+    b, h = (i * tile.b + j) * 4, 16 * j + 2 * i
+    return [f"v_accvgpr_read_b32 v{t[x]}, a{b + x}" for x in range(4)] + \
+           [f"v_cvt_pk_bf16_f32 v{hold(h + p)}, v{t[2 * p]}, v{t[2 * p + 1]}" for p in range(2)]
+
+
+def gelu_pair(r, t):
+    """The tanh form of gelu of the two values in r: z / (1 + 2^(z (a + b z^2)))."""
+    a, b = -1.5957691216057308 * LOG2E, -1.5957691216057308 * 0.044715 * LOG2E
+    lo, hi, u, w = t
+    return [f"v_lshlrev_b32 v{lo}, 16, v{r}", f"v_and_b32 v{hi}, 0xffff0000, v{r}",
+            f"v_mul_f32 v{u}, v{lo}, v{lo}", f"v_mul_f32 v{w}, v{hi}, v{hi}",
+            f"v_fmamk_f32 v{u}, v{u}, {hex_f32(b)}, v{V_GELU}", f"v_fmamk_f32 v{w}, v{w}, {hex_f32(b)}, v{V_GELU}",
+            f"v_mul_f32 v{u}, v{u}, v{lo}", f"v_mul_f32 v{w}, v{w}, v{hi}",
+            f"v_exp_f32 v{u}, v{u}", f"v_exp_f32 v{w}, v{w}", "s_nop 0",
+            f"v_add_f32 v{u}, 1.0, v{u}", f"v_add_f32 v{w}, 1.0, v{w}",
+            f"v_rcp_f32 v{u}, v{u}", f"v_rcp_f32 v{w}, v{w}", "s_nop 0",
+            f"v_mul_f32 v{lo}, v{lo}, v{u}", f"v_mul_f32 v{hi}, v{hi}, v{w}",
+            f"v_cvt_pk_bf16_f32 v{r}, v{lo}, v{hi}"]
+
+
+def gated_pair(mode, gate, up, t):
+    """The two gated units of the gates in one register and the ups in another, into the gates' register."""
+    g0, g1, e0, e1, u0, u1 = t
+    o = [f"v_lshlrev_b32 v{g0}, 16, v{gate}", f"v_and_b32 v{g1}, 0xffff0000, v{gate}",
+         f"v_lshlrev_b32 v{u0}, 16, v{up}", f"v_and_b32 v{u1}, 0xffff0000, v{up}"]
+    if mode == "glu":
+        o += [f"v_min_f32 v{g0}, %[limit], v{g0}", f"v_min_f32 v{g1}, %[limit], v{g1}",
+              f"v_max_f32_e64 v{u0}, -%[limit], v{u0}", f"v_max_f32_e64 v{u1}, -%[limit], v{u1}",
+              f"v_min_f32 v{u0}, %[limit], v{u0}", f"v_min_f32 v{u1}, %[limit], v{u1}",
+              f"v_mul_f32 v{e0}, %[rate], v{g0}", f"v_mul_f32 v{e1}, %[rate], v{g1}",
+              f"v_add_f32 v{u0}, %[shift], v{u0}", f"v_add_f32 v{u1}, %[shift], v{u1}"]
+    else:
+        o += [f"v_mul_f32 v{e0}, {hex_f32(-LOG2E)}, v{g0}", f"v_mul_f32 v{e1}, {hex_f32(-LOG2E)}, v{g1}"]
+    return o + [f"v_exp_f32 v{e0}, v{e0}", f"v_exp_f32 v{e1}, v{e1}", "s_nop 0",
+                f"v_add_f32 v{e0}, 1.0, v{e0}", f"v_add_f32 v{e1}, 1.0, v{e1}",
+                f"v_rcp_f32 v{e0}, v{e0}", f"v_rcp_f32 v{e1}, v{e1}", "s_nop 0",
+                f"v_mul_f32 v{g0}, v{g0}, v{e0}", f"v_mul_f32 v{g1}, v{g1}, v{e1}",
+                f"v_mul_f32 v{g0}, v{g0}, v{u0}", f"v_mul_f32 v{g1}, v{g1}, v{u1}",
+                f"v_cvt_pk_bf16_f32 v{gate}, v{g0}, v{g1}"]
+
+
+def whole_lines(p0, p1, at, so):
+    """Two 16-byte groups of every token, 32 columns apart: token t's lanes and those of token t + 8 change halves, so that a store
+    writes whole cache lines of eight tokens.  at: registers for the two stores' offsets.  (instructions, stores)"""
+    t = TEMP[2:6]
+    o = [f"v_add_u32 v{at[0]}, {S_ROW}, %[{so}]", f"v_add_u32 v{at[1]}, %[row8], v{at[0]}"]
+    o += [f"v_cndmask_b32_e64 v{t[k]}, v{p0 + k}, v{p1 + k}, {S_LOW}" for k in range(4)]
+    o += [f"v_mov_b32_dpp v{t[k]}, v{t[k]} row_ror:8 row_mask:0xf bank_mask:0xf" for k in range(4)]
+    o += [f"v_cndmask_b32_e64 v{p0 + k}, v{t[k]}, v{p0 + k}, {S_LOW}" for k in range(4)]
+    o += [f"v_cndmask_b32_e64 v{p1 + k}, v{p1 + k}, v{t[k]}, {S_LOW}" for k in range(4)]
+    return o, [f"buffer_store_dwordx4 v[{p}:{p + 3}], v{v}, %[ro], 0 offen@NT" for p, v in ((p0, at[0]), (p1, at[1]))]
+
+
+def finish_column(mode, j):
+    """(instructions, stores) of column block j."""
+    h = lambda n: hold(16 * j + n)
+    o, stores = [f"s_mov_b32 s76, 0x00ff00ff", "s_mov_b32 s77, 0x00ff00ff", f"s_mul_i32 {S_ROW}, %[row16], {j}"], []
+    if mode == "gelu":
+        for n in range(0, 16, 2):
+            o += interleave(gelu_pair(h(n), TEMP[0:4]), gelu_pair(h(n + 1), TEMP[6:10]))
+    if mode in ("silu", "glu"):
+        for m in range(2):
+            for n in range(0, 4, 2):
+                o += interleave(gated_pair(mode, h(8 * m + n), h(8 * m + 4 + n), TEMP[0:6]),
+                                gated_pair(mode, h(8 * m + n + 1), h(8 * m + 5 + n), TEMP[6:12]))
+        a, b = whole_lines(h(0), h(8), (TEMP[0], TEMP[1]), "so0")
+        return o + a, stores + b
+    for m, so, at in ((0, "so0", (TEMP[0], TEMP[1])), (2, "so1", (TEMP[6], TEMP[7]))):
+        a, b = whole_lines(h(4 * m), h(4 * m + 4), at, so)
+        o, stores = o + a, stores + b
+    return o, stores
+
+
+SETTLE = ["s_nop 15", "s_nop 7"]     # an MFMA's result may be read 18 wait states after its issue at the earliest
+
+
+def pack_all(tile):
+    return SETTLE + [x for i in range(tile.a) for j in range(tile.b) for x in pack_block(tile, i, j, TEMP[0:4] if j % 2 else TEMP[6:10])]
+
+
+def piece(tile):
+    """The accumulators as they are, 1 KB a block, to a partial tile ([rp], [vp] the lane's offset, [sp] the wavefront's)."""
+    out = SETTLE + ["s_mov_b32 s79, %[sp]"]
+    for n, (j, i) in enumerate((j, i) for j in range(tile.b) for i in range(tile.a)):
+        t = TEMP[2:6] if n % 2 else TEMP[6:10]
+        out += [f"v_accvgpr_read_b32 v{t[x]}, a{(i * tile.b + j) * 4 + x}" for x in range(4)]
+        out.append(f"buffer_store_dwordx4 v[{t[0]}:{t[3]}], %[vp], %[rp], s79 offen offset:{n % 4 * 1024}")
+        if n % 4 == 3:
+            out.append("s_add_u32 s79, s79, 0x1000")
+    return out
+
+
 def gemm_text():
+    tile = SCAN
+    step = lambda fresh, **kw: kstep(fresh, voff_b=VOFF_B, nt="", **kw)
     parts = [HEADER,
-             define("MSA_GEMM_KSTEP", kstep(False, voff_b=VOFF_B, nt="")),
-             define("MSA_GEMM_KSTEP_FRESH", kstep(True, voff_b=VOFF_B, nt="")),
+             define("MSA_GEMM_KSTEP", step(False)),
+             define("MSA_GEMM_KSTEP_FRESH", step(True)),
              define("MSA_GEMM_FRAGS0", frags0()),
              define("MSA_GEMM_LOAD8_A", load8(VOFF)),
              define("MSA_GEMM_LOAD8_B", load8(VOFF_B)),
              define("MSA_GEMM_SET_ADDR", set_registers(VADDR, 4)),
-             define("MSA_GEMM_SET_VOFF_A", set_registers(VOFF, 8)),
-             define("MSA_GEMM_SET_VOFF_B", set_registers(VOFF_B, 8)),
-             # an MFMA's result may be read 18 wait states after its issue at the earliest
-             define("MSA_GEMM_SETTLE", ["s_nop 15", "s_nop 7"])]
+             *(define(f"MSA_GEMM_SET_VOFF_{name}{h}", set_registers(first + 4 * h, 4)) for name, first in (("A", VOFF), ("B", VOFF_B)) for h in range(2)),
+             define("MSA_GEMM_SETTLE", SETTLE)]
     # four of the eight row blocks of a column block, sixteen accumulators
     for j in range(8):
         for h in range(2):
             parts.append(define(f"MSA_GEMM_ACC_{j}_{h}", [f"v_accvgpr_read_b32 %{4 * i + r}, a{((4 * h + i) * 8 + j) * 4 + r}"
                                                           for i in range(4) for r in range(4)]))
+    packs = [[pack_block(tile, i, j, TEMP[0:4] if j % 2 else TEMP[6:10]) for j in range(tile.b)] for i in range(tile.a)]
+    parts.append(define("MSA_GEMM_KSTEP_FRESH_PACK", step(True, early_fillers=packs)))
+    parts.append(define("MSA_GEMM_PACK", pack_all(tile)))
+    parts.append(define("MSA_GEMM_PIECE", piece(tile)))
+    parts.append(define("MSA_GEMM_SET_GELU", [f"v_mov_b32 v{V_GELU}, {hex_f32(-1.5957691216057308 * LOG2E)}"]))
+    for mode in ("store", "gelu", "silu", "glu"):
+        for j in range(tile.b):
+            work, stores = finish_column(mode, j)
+            parts.append(define(f"MSA_GEMM_KSTEP_{mode.upper()}_{j}(NT)", step(False, fillers=work, stores=stores)))
+            parts.append(define(f"MSA_GEMM_END_{mode.upper()}_{j}(NT)", fix_lane_move_hazards(work + stores)))
     parts.append(clobbers("MSA_GEMM_CLOBBERS"))
+    parts.append(clobbers("MSA_GEMM_FLOW_CLOBBERS", HOLD_LOW))
     return "\n".join(parts)
 
 
 def main():
-    here, stale = os.path.dirname(os.path.abspath(__file__)), 0
-    for name, text in (("scan_asm.inc", scan_text()), ("gemm_asm.inc", gemm_text())):
-        path = os.path.join(here, name)
-        if len(sys.argv) > 1 and sys.argv[1] == "--check":
-            stale |= not os.path.exists(path) or open(path).read() != text
-        else:
-            open(path, "w").write(text)
-    return int(stale)
+    """``scan_asm.inc`` (``--check``: is it what would be written?) and, always, ``gemm_asm.inc``, which every build writes again."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    path, text = os.path.join(here, "gemm_asm.inc"), gemm_text()
+    if not os.path.exists(path) or open(path).read() != text:
+        with open(path, "w") as f:
+            f.write(text)
+    path, text = os.path.join(here, "scan_asm.inc"), scan_text()
+    if len(sys.argv) > 1 and sys.argv[1] == "--check":
+        return 0 if open(path).read() == text else 1
+    with open(path, "w") as f:
+        f.write(text)
+    return 0
 
 
 if __name__ == "__main__":

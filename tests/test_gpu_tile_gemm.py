@@ -1,7 +1,9 @@
 """Products of a block of tokens (``ops.tile_linear``) against fp32: edges of the 256 x 256 tiles, one K tile and many, tiles multiplied in
 pieces, row strides, and every end (store, add, silu-mul, clamped unit, gelu; the heads' norm and rotary are tested with ``qkv_proj``).
 
-One rounding to bf16 leaves a relative error of up to 2^-9 a value, 1.7e-3 over many; the fp32 sums are far below it."""
+One rounding to bf16 leaves a relative error of up to 2^-9 a value, 1.7e-3 over many; the fp32 sums are far below it.  The gated ends and
+gelu may round the sums before and the result behind: three roundings for a gated unit, the gate's passed on by a factor of up to 1.3
+over many values, sqrt(1 + 1 + 1.3^2) of one."""
 import pytest
 import torch
 
@@ -9,6 +11,7 @@ from msa_amd._lib import MsaError
 
 pytestmark = pytest.mark.gpu
 TOL = 3e-3
+TOL_END = 4e-3
 
 
 def _say(msg):
@@ -34,8 +37,10 @@ def _err(got, want):
     return ((got.float() - want).norm() / want.norm()).item()
 
 
+# several tiles a workgroup, their ends under the next one's steps from K = 704 on: the last three
 # (2100 x 4096 x 2576: 99 tiles on 256 compute units, in pieces of K; 257 x 1024 x 16400: 130 tiles, whole)
-SHAPES = [(1, 64, 8), (255, 64, 256), (256, 128, 256), (257, 192, 264), (17, 320, 1000), (300, 4096, 2048), (2100, 4096, 2576), (257, 1024, 16400)]
+SHAPES = [(1, 64, 8), (255, 64, 256), (256, 128, 256), (257, 192, 264), (17, 320, 1000), (300, 4096, 2048), (2100, 4096, 2576), (257, 1024, 16400),
+          (6001, 704, 5144), (9000, 640, 4360), (5000, 1024, 6664)]
 
 
 @pytest.mark.parametrize("T,K,N", SHAPES)
@@ -56,31 +61,31 @@ def test_store_and_add(ops, T, K, N):
     assert bool((wide == 7.0).all())
 
 
-@pytest.mark.parametrize("T,K,N", [(1, 64, 16), (129, 128, 272), (513, 256, 1040), (2100, 4096, 2592), (2048, 1024, 4096)])
+@pytest.mark.parametrize("T,K,N", [(1, 64, 16), (129, 128, 272), (513, 256, 1040), (2100, 4096, 2592), (6001, 1024, 5136), (6001, 704, 5200)])
 def test_silu_mul(ops, T, K, N):
     _say(f"silu-mul T={T} K={K} N={N}")
     x, gate, want_gate = _operands(T, K, N // 2, 2)
     up = (torch.randn((N // 2, K), device="cuda") * K ** -0.5).bfloat16()
     got = ops.tile_linear(x, ops.interleave_gate_up(gate, up), silu_mul=True)
-    assert _err(got, torch.nn.functional.silu(want_gate) * (x.float() @ up.float().t())) < TOL
+    assert _err(got, torch.nn.functional.silu(want_gate) * (x.float() @ up.float().t())) < TOL_END
 
 
-@pytest.mark.parametrize("T,K,N", [(1, 64, 16), (129, 128, 272), (2100, 4096, 2592), (2048, 1024, 4096)])
+@pytest.mark.parametrize("T,K,N", [(1, 64, 16), (129, 128, 272), (2100, 4096, 2592), (6001, 1024, 5136), (6001, 704, 5200)])
 def test_glu(ops, T, K, N):
     """Rows in (gate, up) pairs; sums up to 4 against a limit of 1.5, so that both are clamped."""
     _say(f"glu T={T} K={K} N={N}")
     x, w, want = _operands(T, K, N, 6)
     got = ops.tile_linear(x, w, glu=(1.5, 1.702, 1.0))
     gate, up = want[:, 0::2].clamp(max=1.5), want[:, 1::2].clamp(-1.5, 1.5)
-    assert _err(got, gate * torch.sigmoid(1.702 * gate) * (up + 1.0)) < TOL
+    assert _err(got, gate * torch.sigmoid(1.702 * gate) * (up + 1.0)) < TOL_END
 
 
-@pytest.mark.parametrize("T,K,N,n", [(1, 64, 8, 8), (129, 128, 264, 136), (257, 256, 512, 128), (2100, 4096, 2576, 1304), (2048, 1024, 4096, 3072)])
+@pytest.mark.parametrize("T,K,N,n", [(1, 64, 8, 8), (129, 128, 264, 136), (257, 256, 512, 128), (2100, 4096, 2576, 1304), (6001, 1024, 5144, 3072), (6001, 704, 5200, 1408)])
 def test_gelu(ops, T, K, N, n):
     _say(f"gelu T={T} K={K} N={N} n={n}")
     x, w, want = _operands(T, K, N, 7)
     want[:, :n] = torch.nn.functional.gelu(want[:, :n], approximate="tanh")
-    assert _err(ops.tile_linear(x, w, gelu_n=n), want) < TOL
+    assert _err(ops.tile_linear(x, w, gelu_n=n), want) < TOL_END
 
 
 def test_extreme_gates(ops):
