@@ -435,7 +435,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_vgpr(kCompilerV
 constexpr int kFlowVgprs = 24;                 // the compiler's share of the vector registers
 constexpr int kFlowSteps = 11;                 // an item of that many steps takes another tile's end: one packs, eight finish, the
                                                // last two already load for the item behind
-constexpr int kFar = 0x7ff00000;               // behind every extent, whatever is added: nothing is stored
+[[maybe_unused]] constexpr int kFar = 0x7ff00000;               // behind every extent, whatever is added: nothing is stored
 
 template <int kMode, bool kStream>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_vgpr(kFlowVgprs))) void tile_flow_kernel(TileArgs a) {
