@@ -154,6 +154,74 @@ __global__ __launch_bounds__(1024) void gather_copy_kernel(const uint4* __restri
                                      (int)gridDim.y * groups, (int)threadIdx.x % kCopyRowLanes);
 }
 
+// A selection of up to 64 documents (samples of KW lanes each) in one launch: every wavefront plans it for itself, in registers, a
+// document a lane, and a document that several samples picked is read once and stored to all their rows.  The plan costs a wavefront
+// two dependent loads, a sort and a scan; as a launch of its own in front of the copy, and with a third for the repeated
+// documents, a lookup of 16 documents of 8 chunks took 25.1 us, here 22.4 (1 MB over the link takes 20; more workgroups change nothing).
+template <int KW>
+__global__ __launch_bounds__(kCopyThreads) void gather_few_kernel(const int32_t* __restrict__ doc_sel,
+                                                                  const int32_t* __restrict__ doc_chunk_off, int32_t n_docs, int32_t B,
+                                                                  int32_t k, int64_t capacity_rows, int32_t* __restrict__ cu_sel,
+                                                                  const uint4* __restrict__ k_src, const uint4* __restrict__ v_src,
+                                                                  int32_t row_vecs, uint4* __restrict__ k_dst, uint4* __restrict__ v_dst) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sample = lane / KW, pos = lane % KW;
+  int32_t d = msa_gather::kNoDoc;
+  if (sample < B && pos < k) {
+    const int32_t x = doc_sel[sample * k + pos];
+    if (x >= 0 && x < n_docs) d = x;
+  }
+#pragma unroll
+  for (int kk = 2; kk <= KW; kk <<= 1)           // ascending inside the sample's lanes
+#pragma unroll
+    for (int j = kk >> 1; j > 0; j >>= 1) {
+      const int32_t o = msa_gather::xor_lane(d, j);
+      const bool asc = kk == KW || (lane & kk) == 0, lower = (lane & j) == 0;
+      d = (lower == asc) ? min(d, o) : max(d, o);
+    }
+  const int32_t prev = __shfl_up(d, 1);
+  const bool keep = d != msa_gather::kNoDoc && (pos == 0 || prev != d);
+  const int32_t c0 = keep ? doc_chunk_off[d] : 0, n = keep ? doc_chunk_off[d + 1] - c0 : 0;
+  int32_t incl = n;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int32_t t = __shfl_up(incl, o);
+    if (lane >= o) incl += t;
+  }
+  const int32_t at = incl - n;
+  // rows past the output's capacity are never written: the prefix sums stop there too
+  if (blockIdx.x == 0 && blockIdx.y == 0 && wave == 0) {
+    if (lane == 0) cu_sel[0] = 0;
+    if (pos == KW - 1 && sample < B) cu_sel[sample + 1] = (int32_t)min((int64_t)incl, capacity_rows);
+  }
+  // the first lane that keeps the same document
+  const int32_t mine = keep ? d : -1 - lane;
+  int first = lane;
+  if (B > 1)
+    for (int e = B * KW - 1; e >= 0; --e)
+      if (__builtin_amdgcn_readlane(mine, e) == mine) first = e;
+  const uint64_t sources = __ballot(keep && first == lane);
+  // 128 lanes share a row: both wavefronts of a workgroup walk alike
+  const int row_lane = threadIdx.x;
+  int ordinal = 0;
+  for (uint64_t left = sources; left != 0; left &= left - 1, ++ordinal) {
+    if (ordinal % (int)gridDim.x != (int)blockIdx.x) continue;
+    const int e = __builtin_ctzll(left);
+    const int32_t src = __builtin_amdgcn_readlane(c0, e), rows = __builtin_amdgcn_readlane(n, e);
+    const uint64_t targets = __ballot(keep && first == e);
+    for (int r = blockIdx.y; r < rows; r += gridDim.y)
+      for (int off = row_lane; off < row_vecs; off += kCopyRowLanes) {
+        const uint4 a = k_src[(int64_t)(src + r) * row_vecs + off], b = v_src[(int64_t)(src + r) * row_vecs + off];
+        for (uint64_t t = targets; t != 0; t &= t - 1) {
+          const int64_t row = (int64_t)__builtin_amdgcn_readlane(at, __builtin_ctzll(t)) + r;
+          if (row >= capacity_rows) continue;
+          k_dst[row * row_vecs + off] = a;
+          v_dst[row * row_vecs + off] = b;
+        }
+      }
+  }
+}
+
 }  // namespace
 
 extern "C" size_t msa_gather_device_workspace_bytes(int32_t B, int32_t k) {
@@ -178,14 +246,23 @@ extern "C" int msa_gather_kv_device(const msa_bank* bank, int32_t layer, const i
   }
   hipStream_t st = as_stream(stream);
   int32_t* plan = static_cast<int32_t*>(workspace);
+  const int32_t row_vecs = (int32_t)((size_t)bank->Hkv * bank->D * elem_bytes(bank->dtype) / 16);
+  dim3 grid((unsigned)std::min(B * k, kCopyGridX), kCopyGridY);
+  const int lanes = k <= 16 ? 16 : k <= 32 ? 32 : 64;       // of a sample
+  if (B * lanes <= 64) {
+    const auto kernel = lanes == 16 ? gather_few_kernel<16> : lanes == 32 ? gather_few_kernel<32> : gather_few_kernel<64>;
+    kernel<<<grid, kCopyThreads, 0, st>>>(doc_sel, bank->doc_chunk_off_dev, (int32_t)bank->n_docs, B, k, out_capacity_chunks, cu_sel,
+                                          static_cast<const uint4*>(bank->k_host[layer]), static_cast<const uint4*>(bank->v_host[layer]),
+                                          row_vecs, static_cast<uint4*>(k_out), static_cast<uint4*>(v_out));
+    MSA_LAUNCH_CHECK();
+    return MSA_OK;
+  }
   const int32_t dedup = B > 1 && B * k <= kDedupMaxEntries ? 1 : 0;
   const int32_t cap32 = (int32_t)std::min<int64_t>(out_capacity_chunks, 0x7fffffff);
   const size_t lds = msa_gather::plan_lds_ints(B, k, dedup) * sizeof(int32_t);
   gather_plan_kernel<<<1, kPlanWaves * 64, lds, st>>>(doc_sel, bank->doc_chunk_off_dev, (int32_t)bank->n_docs, B, k,
                                                       cap32, dedup, cu_sel, plan);
   MSA_LAUNCH_CHECK();
-  const int32_t row_vecs = (int32_t)((size_t)bank->Hkv * bank->D * elem_bytes(bank->dtype) / 16);
-  dim3 grid((unsigned)std::min(B * k, kCopyGridX), kCopyGridY);
   gather_copy_kernel<false><<<grid, kCopyThreads, 0, st>>>(static_cast<const uint4*>(bank->k_host[layer]),
                                                   static_cast<const uint4*>(bank->v_host[layer]), plan, B * k, row_vecs,
                                                   out_capacity_chunks, static_cast<uint4*>(k_out),
