@@ -80,7 +80,9 @@ template <typename T, int G>
 __device__ __forceinline__ void attend_keys(const T* __restrict__ k, const T* __restrict__ v, int64_t lane_off,
                                             int row_elems, int first, int key1, int stride, const float (&qv)[G][8],
                                             float (&m)[G], float (&l)[G], float (&acc)[G][8]) {
-  constexpr int kBatch = 4;
+  // (fp32: with one head twice the bytes in flight are worth their registers, 16 samples of 3000 keys 98 -> 75 us; with four they cost
+  // a wavefront a SIMD, 16 of 4388 131 -> 158)
+  constexpr int kBatch = sizeof(T) == 4 && G == 1 ? 8 : 4;
   for (int kb = first; kb < key1; kb += stride * kBatch) {
     float kx[kBatch][8], vx[kBatch][8];
     bool ok[kBatch];
@@ -378,6 +380,32 @@ __global__ __launch_bounds__(kRingWaves * 64) void attn_ring_kernel(
   }
 }
 
+// The softmax states of two lanes kBit apart become their merger in both.
+template <int kBit>
+__device__ __forceinline__ void merge_slots(float& m, float& l, float (&acc)[8]) {
+  auto both = [](float x, float& lower, float& upper) {
+    const uint32_t u = __float_as_uint(x);
+    if constexpr (kBit == 16) {
+      const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+      lower = __uint_as_float(r[0]); upper = __uint_as_float(r[1]);
+    } else {
+      const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+      lower = __uint_as_float(r[0]); upper = __uint_as_float(r[1]);
+    }
+  };
+  float m0, m1, x0, x1;
+  both(m, m0, m1);
+  m = fmaxf(m0, m1);
+  const float a0 = m == -INFINITY ? 0.f : fast_exp2(m0 - m), a1 = m == -INFINITY ? 0.f : fast_exp2(m1 - m);
+  both(l, x0, x1);
+  l = x0 * a0 + x1 * a1;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    both(acc[i], x0, x1);
+    acc[i] = x0 * a0 + x1 * a1;
+  }
+}
+
 // fp32 rows, and bf16 rows of groups of one and two heads where takes_ring says so.
 template <typename T, int G, int kAttnWaves>
 __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
@@ -422,19 +450,11 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
   }
   attend_keys<T, G>(k, v, lane_off, row_elems, key0 + wave * 4 + slot, key1, kAttnWaves * 4, qv, m, l, acc);
 
-  // merge the 4 key slots of the wavefront (lanes differing in bits 4 and 5)
+  // merge the 4 key slots of the wavefront (lanes differing in bits 4 and 5): a swap leaves both lanes' values in both, without LDS
 #pragma unroll
   for (int h = 0; h < G; ++h) {
-#pragma unroll
-    for (int x = 16; x <= 32; x <<= 1) {
-      const float mo = __shfl_xor(m[h], x), lo = __shfl_xor(l[h], x);
-      const float mn = fmaxf(m[h], mo);
-      const float a = mn == -INFINITY ? 0.f : fast_exp2(m[h] - mn), bo = mn == -INFINITY ? 0.f : fast_exp2(mo - mn);
-      l[h] = l[h] * a + lo * bo;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc[h][i] = acc[h][i] * a + __shfl_xor(acc[h][i], x) * bo;
-      m[h] = mn;
-    }
+    merge_slots<16>(m[h], l[h], acc[h]);
+    merge_slots<32>(m[h], l[h], acc[h]);
   }
   if (slot == 0) {
 #pragma unroll
