@@ -1111,74 +1111,126 @@ __global__ void decode_scores_kernel(const uint32_t* __restrict__ key, int64_t n
 // fp32 banks of few chunks, or few query rows.  Tiles of 128 x 128 give a bank of 8000 chunks to 63 workgroups, each of which
 // multiplies 1024-deep products at a compute unit's fp32 rate alone (57 us a tile, also where half of its rows are padding).  Here
 // a workgroup owns 32 chunks and its four wavefronts a quarter of K each: a wavefront's share of the K_r rows stays in 128 of its
-// registers for the whole launch, the query rows come from L2 a 32-row block at a time, eight 16-byte vectors ahead of the MFMAs,
-// and the four partial blocks meet in LDS behind one barrier per block, where the rows' maximum is taken.  Both operands permute K
-// alike (lane half h holds the second 16 bytes of every 32).  Column maxima of a query wait in LDS and are merged into the key
-// plane at the end.  What bounds it: the matrix cores' fp32 rate (256 FLOP a cycle and compute unit) and, with few rows, the
-// first loads.
-// A whole routing call, us, against the tiles: 8192 chunks x 64 rows 38 against 82, x 256 rows 66 against 85; 1024 x 128 rows 37
-// against 81.
+// registers for the whole launch, the query rows follow a 32-row block at a time, and the four partial blocks meet in LDS behind one
+// barrier per block, where the rows' maximum is taken.  Column maxima of a query wait in LDS and are merged into the key plane at the end.
+// K_r and query rows come through a ring of stages of a cache line of 32 rows, direct loads of eight whole lines: an MFMA operand
+// loaded from memory touches 32 lines an instruction, 32 bytes each, and the address unit takes four times as long over it.  What
+// bounds it: the matrix cores' fp32 rate (256 FLOP a cycle and compute unit) and, with few rows, the launch and the first loads.
+// The kernel at 8000 chunks x 64 rows 21.0 -> 17.8 us (8 of them matrix cores); whole routing calls, us, operands from memory and
+// through the ring: 8000 x 64 30.7 and 26.4, 512 x 64 20.4 and 17.9, 64000 x 64 123 and 106, 128000 x 32 178 and 157, 8000 x 512 85 and 83.
 // ------------------------------------------------------------------------------------------
 constexpr int kSplitK = 1024, kSplitWaves = 4, kSplitCols = 32, kSplitMaxBlocks = 32;
+constexpr int kSplitSlab = 32 * 128;           // a stage of a wavefront's ring: 32 rows, a cache line (32 values of K) each
+constexpr int split_lds_bytes(int ring) {
+  return kSplitWaves * ring * kSplitSlab + (2 * kSplitWaves * 32 + kSplitMaxBlocks) * kSplitCols * 4;
+}
+static_assert(split_lds_bytes(6) <= 160 * 1024 && 2 * split_lds_bytes(2) <= 160 * 1024);
 
-template <bool kDocMax>
+// Four 1 KB blocks straight into LDS, as an asm statement so that the compiler does not drain what is in flight in front of its own LDS
+// reads; the kernel counts.  M0 is put back as it was.
+__device__ __forceinline__ void request_slab(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds_dst, const int (&at)[4], int soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t saved_m0;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 4\n\t"
+      "buffer_load_dwordx4 %2, %6, %7 offen lds\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
+      "buffer_load_dwordx4 %3, %6, %7 offen lds\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
+      "buffer_load_dwordx4 %4, %6, %7 offen lds\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
+      "buffer_load_dwordx4 %5, %6, %7 offen lds\n\ts_mov_b32 m0, %0"
+      : "=&s"(saved_m0) : "s"(lds_dst), "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "s"(rsrc), "s"(soff) : "scc", "memory");
+#endif
+}
+
+template <bool kDocMax, int kRing>
 __global__ __launch_bounds__(kSplitWaves * 64, 2) void score_split_kernel(const float* __restrict__ qs, const float* __restrict__ kr,
                                                                         const uint32_t* __restrict__ row_bits,
                                                                         uint32_t* __restrict__ out_key,
                                                                         const int32_t* __restrict__ chunk_doc, int32_t M_rows,
                                                                         int32_t C, int32_t blocks_per_query, int32_t n_docs,
                                                                         int32_t blocks_per_wg) {
-  constexpr int kRow = kSplitK * (int)sizeof(float), kSlice = kRow / kSplitWaves, kSteps = kSlice / 32, kGroup = 8, kGroups = kSteps / kGroup;
-  static_assert(kGroups == 4, "a block starts in the first register buffer");
-  __shared__ float part[2][kSplitWaves][32 * kSplitCols];
-  __shared__ uint32_t best[kSplitMaxBlocks][kSplitCols];
+  constexpr int kRow = kSplitK * (int)sizeof(float), kSlice = kRow / kSplitWaves, kStages = kSlice / 128;
+  static_assert(kStages == 8, "stages alternate between two register buffers");
+  extern __shared__ __align__(16) char lds[];
+  char* const shared = lds + kSplitWaves * kRing * kSplitSlab;
+  float(*part)[kSplitWaves][32 * kSplitCols] = reinterpret_cast<float(*)[kSplitWaves][32 * kSplitCols]>(shared);
+  uint32_t(*best)[kSplitCols] = reinterpret_cast<uint32_t(*)[kSplitCols]>(shared + 2 * kSplitWaves * 32 * kSplitCols * 4);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, half = lane >> 5;
   const int n0 = blockIdx.x * kSplitCols, blocks = M_rows >> 5;
   const int b0 = blockIdx.y * blocks_per_wg, b1 = min(blocks, b0 + blocks_per_wg);
-  const __amdgpu_buffer_rsrc_t rs_k = __builtin_amdgcn_make_buffer_rsrc(
+  char* const ring = lds + wave * kRing * kSplitSlab;
+  const uint32_t ring_at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)ring);
+  // a load's lanes take eight rows, eight 16-byte units each; unit u of row r lies at u ^ (r & 7)
+  int at[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) at[i] = (8 * i + (lane >> 3)) * kRow + wave * kSlice + (((lane & 7) ^ (lane >> 3)) * 16);
+  // what is requested next: stage `stage` of the K_r rows, then of one block of query rows after another (behind the last, zeros
+  // through an empty extent)
+  int stage = 0, req_blk = b0 - 1, req_slot = 0, slot = 0;
+  __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<char*>(reinterpret_cast<const char*>(kr)) + (int64_t)n0 * kRow, 0, min(kSplitCols, C - n0) * kRow, 0x00020000);
-  const int off = l32 * kRow + wave * kSlice + half * 16;
-  u32x4_t k[kSteps], q[2][kGroup];
-  auto load_q = [&](auto buf_tag, int blk, int group) {
-    constexpr int buf = decltype(buf_tag)::value;
-    // a block past the range reads zeros through an empty extent
-    const int base = __builtin_amdgcn_readfirstlane(blk < b1 ? blk : b0), extent = __builtin_amdgcn_readfirstlane(blk < b1 ? 32 * kRow : 0);
-    const __amdgpu_buffer_rsrc_t rs_q = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(reinterpret_cast<const char*>(qs)) + (int64_t)base * 32 * kRow, 0, extent, 0x00020000);
-#pragma unroll
-    for (int i = 0; i < kGroup; ++i) q[buf][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_q, off, (group * kGroup + i) * 32, 0);
+  auto request = [&]() {
+    request_slab(rs, ring_at + req_slot * kSplitSlab, at, stage * 128);
+    req_slot = req_slot + 1 == kRing ? 0 : req_slot + 1;
+    if (++stage == kStages) {
+      stage = 0;
+      ++req_blk;
+      rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(qs)) + (int64_t)min(req_blk, blocks - 1) * 32 * kRow,
+                                             0, req_blk < b1 ? 32 * kRow : 0, 0x00020000);
+    }
   };
-  load_q(std::integral_constant<int, 0>{}, b0, 0);
+  auto wait_for = [&](auto younger_tag) {        // all stages but the `younger` newest have arrived
+    constexpr int n = 4 * decltype(younger_tag)::value;
+    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
+    asm volatile("" ::: "memory");
+  };
+  int unit[4];
 #pragma unroll
-  for (int i = 0; i < kSteps; ++i) k[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_k, off, i * 32, 0);
+  for (int c = 0; c < 4; ++c) unit[c] = l32 * 128 + (((2 * c + half) ^ (l32 & 7)) * 16);
+  auto read = [&](u32x4_t* to) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) to[c] = *reinterpret_cast<const u32x4_t*>(ring + slot * kSplitSlab + unit[c]);
+    slot = slot + 1 == kRing ? 0 : slot + 1;
+  };
+  u32x4_t k[4 * kStages], q[2][4];
+#pragma unroll
+  for (int i = 0; i < kRing; ++i) request();
   const int q0 = b0 / blocks_per_query;
   for (int i = tid; i < kSplitMaxBlocks * kSplitCols; i += kSplitWaves * 64) best[i / kSplitCols][i % kSplitCols] = 0u;
+#pragma unroll
+  for (int i = 0; i < kStages; ++i) {
+    wait_for(std::integral_constant<int, kRing - 1>{});
+    read(k + 4 * i);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the slot may be requested again
+    request();
+  }
+  wait_for(std::integral_constant<int, kRing - 1>{});
+  read(q[0]);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  request();
   int query = q0, in_query = b0 - q0 * blocks_per_query;
   for (int blk = b0; blk < b1; ++blk) {
     const uint32_t bits = row_bits[blk];                 // all rows of a block are scored, or none (presum_queries_kernel)
     floatx16_t acc;
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-    auto group = [&](auto g_tag) {
-      constexpr int g = decltype(g_tag)::value;
-      if constexpr (g + 1 < kGroups) load_q(std::integral_constant<int, (g + 1) & 1>{}, blk, g + 1);
-      else load_q(std::integral_constant<int, 0>{}, blk + 1, 0);
 #pragma unroll
-      for (int i = 0; i < kGroup; ++i)
+    for (int i = 0; i < kStages; ++i) {                  // stage i's products beside the reads of the one behind it
+      wait_for(std::integral_constant<int, kRing - 1>{});
+      read(q[(i + 1) & 1]);
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-          acc = Mma<float>::mma(__uint_as_float(q[g & 1][i][c]), __uint_as_float(k[g * kGroup + i][c]), acc);
-    };
-    group(std::integral_constant<int, 0>{});
-    group(std::integral_constant<int, 1>{});
-    group(std::integral_constant<int, 2>{});
-    group(std::integral_constant<int, 3>{});
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          acc = Mma<float>::mma(__uint_as_float(q[i & 1][c][x]), __uint_as_float(k[4 * i + c][x]), acc);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      request();
+    }
     // acc[e] is (row 8 * (e / 4) + 4 * half + e % 4, column l32) over this wavefront's quarter of K
     float(*p)[32 * kSplitCols] = part[blk & 1];
 #pragma unroll
     for (int e = 0; e < 16; ++e) p[wave][(8 * (e >> 2) + 4 * half + (e & 3)) * kSplitCols + l32] = acc[e];
-    __syncthreads();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     float top = -INFINITY;                               // of four rows; the other half of the wavefront has four more
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -1192,6 +1244,7 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void score_split_kernel(const 
       ++query;
     }
   }
+  __builtin_amdgcn_s_waitcnt(0);                         // (nothing in flight when the workgroup ends)
   __syncthreads();
   const int queries = b1 > b0 ? (b1 - 1) / blocks_per_query - q0 + 1 : 0;
   for (int base = wave * 64; base < queries * kSplitCols; base += kSplitWaves * 64) {        // 32 lanes a query
@@ -1279,12 +1332,14 @@ int launch_gemm(const void* qs, const void* kr, const uint32_t* row_bits, uint32
   return MSA_OK;
 }
 
-// As many workgroups along the query blocks as give every compute unit two, at most kSplitMaxBlocks blocks each.
+// As many workgroups along the query blocks as give every compute unit two, at most kSplitMaxBlocks blocks each; one where that
+// alone fills three quarters of the units or more, so that K_r is read once (8000 chunks x 64 rows: 26.4 us, with two 30.8).
 template <bool kDocMax>
 int launch_split(const void* qs, const void* kr, const uint32_t* row_bits, uint32_t* out_key, const int32_t* chunk_doc,
                  int32_t M_rows, int32_t C, int32_t blocks_per_query, int32_t n_docs, hipStream_t st) {
   const int cols = (C + kSplitCols - 1) / kSplitCols, blocks = M_rows / 32;
-  const int want = std::min(blocks, std::max((blocks + kSplitMaxBlocks - 1) / kSplitMaxBlocks, 2 * compute_units() / cols));
+  const int each = cols <= compute_units() && cols * 4 >= 3 * compute_units() ? 1 : 2;
+  const int want = std::min(blocks, std::max((blocks + kSplitMaxBlocks - 1) / kSplitMaxBlocks, each * compute_units() / cols));
   const int per_wg = (blocks + want - 1) / want;
   const dim3 grid((unsigned)cols, (unsigned)((blocks + per_wg - 1) / per_wg));
   int slot = -1;
@@ -1293,8 +1348,14 @@ int launch_split(const void* qs, const void* kr, const uint32_t* row_bits, uint3
     if (g_timer.n < g_timer.cap) slot = g_timer.n++;
   }
   if (slot >= 0) MSA_HIP(hipEventRecord(g_timer.start[slot], st));
-  score_split_kernel<kDocMax><<<grid, kSplitWaves * 64, 0, st>>>(static_cast<const float*>(qs), static_cast<const float*>(kr), row_bits,
-                                                                 out_key, chunk_doc, M_rows, C, blocks_per_query, n_docs, per_wg);
+  // one workgroup a compute unit: the deep ring; more: two of them with two slots a wavefront
+  const bool one = (int64_t)grid.x * grid.y <= compute_units();
+  const auto kern = one ? score_split_kernel<kDocMax, 6> : score_split_kernel<kDocMax, 2>;
+  const int lds = split_lds_bytes(one ? 6 : 2);
+  static std::atomic<int> lds_limit_raised[2] = {{0}, {0}};
+  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised[one], reinterpret_cast<const void*>(kern), lds));
+  kern<<<grid, kSplitWaves * 64, lds, st>>>(static_cast<const float*>(qs), static_cast<const float*>(kr), row_bits,
+                                            out_key, chunk_doc, M_rows, C, blocks_per_query, n_docs, per_wg);
   MSA_LAUNCH_CHECK();
   if (slot >= 0) MSA_HIP(hipEventRecord(g_timer.stop[slot], st));
   return MSA_OK;
