@@ -399,6 +399,11 @@ int msa_greedy_sample(const void* logits, int32_t dtype, int32_t B, int64_t V, v
                       int64_t* pos, int64_t* out, int64_t out_stride, int64_t* col, int32_t max_new,
                       void* stream);
 
+/* Rows tokens[0 .. rows) of an embedding table [vocab, W] (W a multiple of 8, 16-byte aligned), in the table's type (out) and / or in fp32
+ * (out_f32).  wrap: negative tokens count from the table's end.  Any other token outside the table ends the program. */
+int msa_embed_rows(const int64_t* tokens, int64_t rows, const void* table, int64_t vocab, int32_t wrap, int32_t W, int32_t dtype, void* out,
+                   float* out_f32, void* stream);
+
 /* Linear layer for the few rows of a decode step: y[M, N] = x[M, K] . w[N, K]^T, bf16, M <= 16,
  * K a multiple of 128, w in torch.nn.Linear layout (the F.linear calls behind q/k/v/o_proj and the MLP at
  * src/msa/memory_sparse_attention.py:125-127, 405 when one token per sample is decoded).  The weight matrix is

@@ -46,6 +46,11 @@ typedef struct {
 int msa_seq_residual_norm(const float* x_in, const void* y, int64_t y_stride, const void* gate, int64_t gate_stride,
                           const float* gate_bias, float* x_out, int32_t dtype, int32_t W, const msa_dyn_tanh* norm,
                           void* h, const float* shift, float* prev, void* h_shift, const msa_seq_batch* batch, void* stream);
+/* The same of a step's first stream: x_out = rows `tokens` (int64 [rows]; negative ones count from the end, others outside the table end
+ * the program) of an embedding table [vocab, W] of `dtype`, in fp32. */
+int msa_seq_embed_norm(const int64_t* tokens, const void* table, int64_t vocab, float* x_out, int32_t dtype, int32_t W,
+                       const msa_dyn_tanh* norm, void* h, const float* shift, float* prev, void* h_shift, const msa_seq_batch* batch,
+                       void* stream);
 
 /* In place: the tanh form of gelu on columns [0, n) of `rows` rows. */
 int msa_seq_gelu(void* y, int64_t y_stride, int32_t dtype, int32_t rows, int32_t n, void* stream);
@@ -178,6 +183,14 @@ typedef struct {
   int32_t reserved;
 } msa_delta_args;
 int msa_seq_delta_scan(const msa_delta_args* args, int32_t dtype, const msa_seq_batch* batch, void* stream);
+/* One bf16 token a sequence, D and E up to 128, where a and gate (unused in args) are themselves products of a low rank: a[row] = w[0 .. H D)
+ * a_low[row], gate[row] = w[n_a .. n_a + H E) g_low[row], w dense [n_a + H E, rank], in fp32. */
+typedef struct {
+  const void *a_low, *g_low, *w;
+  int64_t a_stride, g_stride;
+  int32_t rank, n_a;
+} msa_delta_low;
+int msa_seq_delta_step(const msa_delta_args* args, const msa_delta_low* low, const msa_seq_batch* batch, void* stream);
 /* A chunked portion is prepared in segments, of which two are in the workspace: of up to 88 MB, for n_seq sequences of up to
  * min(n_seq, 4) * 88 MB (or a chunk of all of them).  Two segments of 88 MB will do for several sequences as well, in up to 1.5
  * times the time; anything smaller than what the portion takes then is refused. */

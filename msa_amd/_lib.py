@@ -72,6 +72,7 @@ SIGNATURES = {
     "msa_silu_mul": (C.c_int, [_vp, _i32, _i64, _i32, _vp, _vp]),
     "msa_decode_attn_fused": (C.c_int, [_vp, _i64, _vp, _vp, _vp, _f32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp,
                                         _i32, _vp, _f32, _vp, _vp, _sz, _vp]),
+    "msa_embed_rows": (C.c_int, [_vp, _i64, _vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp]),
     "msa_greedy_sample": (C.c_int, [_vp, _i32, _i32, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _i32, _vp]),
     "msa_skinny_linear": (C.c_int, [_vp, _vp, _vp, _vp, _f32, _i32, _i32, _i32, _i32, _i32, _vp, _vp]),
     "msa_skinny_linear_workspace_bytes": (_sz, [_i32, _i32, _i32]),
@@ -138,6 +139,11 @@ class DeltaArgs(C.Structure):
                 ("G", _i32), ("D", _i32), ("E", _i32), ("eps", _f32), ("reserved", _i32)]
 
 
+class DeltaLow(C.Structure):
+    """``msa_delta_low``."""
+    _fields_ = [("a_low", _vp), ("g_low", _vp), ("w", _vp), ("a_stride", _i64), ("g_stride", _i64), ("rank", _i32), ("n_a", _i32)]
+
+
 ROWS_PLAIN, ROWS_F32, ROWS_RESIDUAL, ROWS_MAMBA, ROWS_GRU, ROWS_GLU = range(6)
 _batch = C.POINTER(SeqBatch)
 
@@ -145,6 +151,7 @@ _batch = C.POINTER(SeqBatch)
 SEQ_SIGNATURES = {
     "msa_seq_residual_norm": (C.c_int, [_vp, _vp, _i64, _vp, _i64, _vp, _vp, _i32, _i32, C.POINTER(DynTanh), _vp, _vp, _vp, _vp,
                                         _batch, _vp]),
+    "msa_seq_embed_norm": (C.c_int, [_vp, _vp, _i64, _vp, _i32, _i32, C.POINTER(DynTanh), _vp, _vp, _vp, _vp, _batch, _vp]),
     "msa_seq_gelu": (C.c_int, [_vp, _i64, _i32, _i32, _i32, _vp]),
     "msa_seq_softcap": (C.c_int, [_vp, _i32, _i64, _f32, _vp, _vp]),
     "msa_seq_join": (C.c_int, [_vp, _vp, _i32, _i32, _i32, _vp, _vp]),
@@ -168,6 +175,7 @@ SEQ_SIGNATURES = {
     "msa_seq_kv_decode_workspace_bytes": (_sz, [C.POINTER(KVAttnArgs), _i32]),
     "msa_seq_kv_decode": (C.c_int, [C.POINTER(KVAttnArgs), _batch, _vp, _sz, _vp]),
     "msa_seq_delta_scan": (C.c_int, [C.POINTER(DeltaArgs), _i32, _batch, _vp]),
+    "msa_seq_delta_step": (C.c_int, [C.POINTER(DeltaArgs), C.POINTER(DeltaLow), _batch, _vp]),
     "msa_seq_delta_chunked_workspace_bytes": (_sz, [C.POINTER(DeltaArgs), _i32, _i32]),
     "msa_seq_delta_chunked": (C.c_int, [C.POINTER(DeltaArgs), _batch, _vp, _sz, _vp]),
     "msa_seq_head_norm_gate": (C.c_int, [_vp, _vp, _i64, _vp, _f32, _i32, _i32, _i32, _i32, _vp]),
@@ -177,7 +185,7 @@ SEQ_SIGNATURES = {
     "msa_rows_linear_post": (C.c_int, [C.POINTER(RowsArgs), _i32, C.POINTER(RowsPost), _vp]),
 }
 # entry points of include/msa_amd.h that libmsa_seq.so holds too (the error text is per library)
-SEQ_SHARED = ("msa_last_error", "msa_abi_version", "msa_greedy_sample")
+SEQ_SHARED = ("msa_last_error", "msa_abi_version", "msa_greedy_sample", "msa_embed_rows")
 
 
 class MsaError(RuntimeError):

@@ -126,6 +126,14 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 #define MSA_LOAD_TO_LDS(rsrc, lds_dst, voffset, soffset, aux) ((void)(rsrc), (void)(lds_dst), (void)(voffset), (void)(soffset))
 #endif
 
+// Row of an embedding table: negative tokens count from its end where `wrap` says so.  A token outside the table ends the program, as
+// torch's own lookup does.
+__device__ __forceinline__ int64_t embed_row(int64_t token, int64_t vocab, bool wrap) {
+  if (wrap && token < 0) token += vocab;
+  if (token < 0 || token >= vocab) __builtin_trap();
+  return token;
+}
+
 static inline hipStream_t as_stream(void* s) { return (hipStream_t)s; }
 static inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 static inline size_t elem_bytes(int dtype) { return dtype == MSA_F32 ? 4 : 2; }

@@ -270,6 +270,23 @@ __global__ void greedy_commit_kernel(const unsigned long long* __restrict__ part
   }
 }
 
+// Rows of an embedding table as they are and, wanted or not, in fp32.  A decode step's few rows are one launch's latency: torch's lookup
+// of 16 rows takes 9 us, and a conversion behind it 4 more, this 4.
+template <typename T>
+__global__ __launch_bounds__(256) void embed_rows_kernel(const int64_t* __restrict__ tokens, int64_t rows, const T* __restrict__ table,
+                                                         int64_t vocab, int32_t wrap, int32_t W, T* __restrict__ out,
+                                                         float* __restrict__ out_f32) {
+  for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+    const T* from = table + embed_row(tokens[r], vocab, wrap != 0) * W;
+    for (int i = (blockIdx.y * 256 + threadIdx.x) * 8; i < W; i += gridDim.y * 256 * 8) {
+      float x[8];
+      load8g<T>(from + i, x);
+      if (out) store8g<T>(out + r * W + i, x);
+      if (out_f32) store8g<float>(out_f32 + r * W + i, x);
+    }
+  }
+}
+
 }  // namespace
 
 static int qk_norm_rope_launch(const char* who, const void* q, const void* k, const void* v, int64_t q_row_stride,
@@ -379,6 +396,22 @@ extern "C" int msa_greedy_sample(const void* logits, int32_t dtype, int32_t B, i
   MSA_LAUNCH_CHECK();
   greedy_commit_kernel<<<(B + 63) / 64, 64, 0, st>>>(static_cast<const unsigned long long*>(scratch), B, tok, pos, out,
                                                      out_stride, col, max_new);
+  MSA_LAUNCH_CHECK();
+  return MSA_OK;
+}
+
+extern "C" int msa_embed_rows(const int64_t* tokens, int64_t rows, const void* table, int64_t vocab, int32_t wrap, int32_t W, int32_t dtype,
+                              void* out, float* out_f32, void* stream) {
+  MSA_REQUIRE(tokens && table && (out || out_f32), "msa_embed_rows: null pointer");
+  MSA_REQUIRE(dtype == MSA_BF16 || dtype == MSA_F32, "msa_embed_rows: dtype %d", dtype);
+  MSA_REQUIRE(rows > 0 && vocab > 0 && W > 0 && W % 8 == 0, "msa_embed_rows: rows=%lld vocab=%lld W=%d (a multiple of 8)", (long long)rows,
+              (long long)vocab, W);
+  MSA_REQUIRE((((uintptr_t)table | (uintptr_t)out | (uintptr_t)out_f32) & 15) == 0, "msa_embed_rows: 16-byte alignment");
+  const dim3 grid((unsigned)std::min<int64_t>(rows, 65536), (unsigned)std::min(4, (W + 2047) / 2048));
+  if (dtype == MSA_BF16)
+    embed_rows_kernel<bf16_t><<<grid, 256, 0, as_stream(stream)>>>(tokens, rows, (const bf16_t*)table, vocab, wrap, W, (bf16_t*)out, out_f32);
+  else
+    embed_rows_kernel<float><<<grid, 256, 0, as_stream(stream)>>>(tokens, rows, (const float*)table, vocab, wrap, W, (float*)out, out_f32);
   MSA_LAUNCH_CHECK();
   return MSA_OK;
 }

@@ -15,8 +15,25 @@ namespace {
 
 constexpr int kTok = 8;                  // tokens per stage
 
-template <typename T, int NI, int RW, int CW>
-__global__ __launch_bounds__(RW * CW * 64) void delta_scan_kernel(msa_delta_args a, msa_seq_batch b) {
+// One 16-byte chunk's products of a weight row and its operand.
+__device__ __forceinline__ float dot8(const uint4& w, const uint4& x, float s) {
+  s += bf16lo(w.x) * bf16lo(x.x); s += bf16hi(w.x) * bf16hi(x.x);
+  s += bf16lo(w.y) * bf16lo(x.y); s += bf16hi(w.y) * bf16hi(x.y);
+  s += bf16lo(w.z) * bf16lo(x.z); s += bf16hi(w.z) * bf16hi(x.z);
+  s += bf16lo(w.w) * bf16lo(x.w); s += bf16hi(w.w) * bf16hi(x.w);
+  return s;
+}
+
+template <int kCtrl>
+__device__ __forceinline__ float add_moved(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kCtrl, 0xf, 0xf, false));
+}
+
+// kLow: the decays' and the gate's operands come through a low rank (`low`), whose second product is formed here: the head's D + E weight
+// rows, sixteen lanes a row, requested in front of everything else and multiplied when the state is on its way too.  A launch of 16 heads of
+// 64 x 128 takes 9.0 us so, 7.6 without, behind a product of 4.1.
+template <typename T, int NI, int RW, int CW, bool kLow = false>
+__global__ __launch_bounds__(RW * CW * 64) void delta_scan_kernel(msa_delta_args a, msa_seq_batch b, msa_delta_low low = {}) {
   constexpr int kD = NI * RW, kCols = CW * 64, kWaves = RW * CW;
   __shared__ __align__(16) float ks[kTok][kD], qs[kTok][kD], gs[kTok][kD];
   __shared__ float beta[kTok], kq[kTok];
@@ -37,6 +54,22 @@ __global__ __launch_bounds__(RW * CW * 64) void delta_scan_kernel(msa_delta_args
   const T* ap = static_cast<const T*>(a.a) + (int64_t)lo * a.a_stride + (int64_t)head * a.D;
   const T* bp = static_cast<const T*>(a.b) + (int64_t)lo * a.b_stride + head;
   const T* gp = static_cast<const T*>(a.gate) + (int64_t)lo * a.gate_stride + (int64_t)head * a.E;
+  __shared__ float low_out[kLow ? kD + kCols : 1];
+  constexpr int kLowRows = RW * CW * 4, kTurns = kLow ? (kD + kCols + kLowRows - 1) / kLowRows : 1;      // weight rows at a time
+  [[maybe_unused]] uint4 lw[kTurns], lx[kTurns];
+  auto fetch_low = [&](int u) {                            // unit u of the lane's rows 0 .. kD (decays) .. kD + kCols (gate)
+#pragma unroll
+    for (int i = 0; i < kTurns; ++i) {
+      const int r = i * kLowRows + (tid >> 4);
+      const bool gate = r >= kD, in = u < low.rank / 8 && (gate ? r - kD < a.E : r < a.D);
+      const int64_t row = gate ? low.n_a + (int64_t)head * a.E + (r - kD) : (int64_t)head * a.D + r;
+      const bf16_t* x = gate ? static_cast<const bf16_t*>(low.g_low) + (int64_t)lo * low.g_stride
+                             : static_cast<const bf16_t*>(low.a_low) + (int64_t)lo * low.a_stride;
+      lw[i] = in ? reinterpret_cast<const uint4*>(low.w)[row * (low.rank / 8) + u] : make_uint4(0, 0, 0, 0);
+      lx[i] = in ? reinterpret_cast<const uint4*>(x)[u] : make_uint4(0, 0, 0, 0);
+    }
+  };
+  if constexpr (kLow) fetch_low(tid & 15);
   constexpr int kEach = (kD + 63) / 64, kMine = (kTok + kWaves - 1) / kWaves;    // values of a lane, tokens of a wavefront in a stage
   // What a stage reads is requested together, and the first one's in front of the state: loads arrive in the order they are made,
   // and the vectors are ready by the time the state is there.
@@ -55,7 +88,7 @@ __global__ __launch_bounds__(RW * CW * 64) void delta_scan_kernel(msa_delta_args
         const bool in = i < a.D;
         k[m][j] = in ? to_f32<T>(kp[t * a.qkv_stride + i]) : 0.f;
         q[m][j] = in ? to_f32<T>(qp[t * a.qkv_stride + i]) : 0.f;
-        x[m][j] = in ? to_f32<T>(ap[t * a.a_stride + i]) : 0.f;
+        if constexpr (!kLow) x[m][j] = in ? to_f32<T>(ap[t * a.a_stride + i]) : 0.f;
       }
       bv[m] = to_f32<T>(bp[t * a.b_stride]);
     }
@@ -64,10 +97,29 @@ __global__ __launch_bounds__(RW * CW * 64) void delta_scan_kernel(msa_delta_args
   };
   fetch(0);
   const float out_w = live && whole ? a.norm[col] : 0.f;
-  const float gate0 = live && whole ? to_f32<T>(gp[col]) : 0.f;   // of the first token, all there is when decoding
+  float gate0 = 0.f;                                     // of the first token, all there is when decoding
+  if constexpr (!kLow) gate0 = live && whole ? to_f32<T>(gp[col]) : 0.f;
   float S[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) S[i] = live && rw * NI + i < a.D ? st[(int64_t)i * a.E] : 0.f;
+  if constexpr (kLow) {
+    float sum[kTurns] = {};
+    for (int u0 = 0; u0 < low.rank / 8; u0 += 16) {
+      if (u0 > 0) fetch_low(u0 + (tid & 15));
+#pragma unroll
+      for (int i = 0; i < kTurns; ++i) sum[i] = dot8(lw[i], lx[i], sum[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < kTurns; ++i) {
+      const float v = add_moved<0x140>(add_moved<0x141>(add_moved<0x4E>(add_moved<0xB1>(sum[i]))));
+      const int r = i * kLowRows + (tid >> 4);
+      if ((tid & 15) == 0 && r < kD + kCols) low_out[r] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) x[0][j] = lane + 64 * j < kD ? low_out[lane + 64 * j] : 0.f;
+    gate0 = low_out[kD + cl];
+  }
   for (int t0 = 0; t0 < n_tok; t0 += kTok) {
     const int rows = min(kTok, n_tok - t0);
     if (t0 > 0) fetch(t0);
@@ -205,7 +257,37 @@ int launch_scan(const msa_delta_args& a, const msa_seq_batch& b, hipStream_t st)
   return MSA_OK;
 }
 
+template <int NI, int RW>
+void launch_step(const msa_delta_args& a, const msa_delta_low& low, const msa_seq_batch& b, hipStream_t st) {
+  const dim3 grid(1, a.H, b.n_seq);
+  if (a.E <= 64) delta_scan_kernel<bf16_t, NI, RW, 1, true><<<grid, RW * 64, 0, st>>>(a, b, low);
+  else delta_scan_kernel<bf16_t, NI, RW, 2, true><<<grid, RW * 128, 0, st>>>(a, b, low);
+}
+
 }  // namespace
+
+extern "C" int msa_seq_delta_step(const msa_delta_args* args, const msa_delta_low* low, const msa_seq_batch* batch, void* stream) {
+  MSA_CHECK_BATCH(batch, "msa_seq_delta_step");
+  MSA_REQUIRE(args && low && args->qkv && args->b && args->A_log && args->dt_bias && args->norm && args->state && args->out && low->a_low &&
+                  low->g_low && low->w, "msa_seq_delta_step: null pointer");
+  const msa_delta_args& a = *args;
+  MSA_REQUIRE(batch->max_rows == 1, "msa_seq_delta_step: one token a sequence, got %d", batch->max_rows);
+  MSA_REQUIRE(a.H > 0 && a.H <= 65535 && a.G > 0 && a.H % a.G == 0 && a.D > 0 && a.D <= 128 && a.E > 0 && a.E <= 128 && batch->n_seq <= 65535,
+              "msa_seq_delta_step: H=%d G=%d D=%d E=%d (both up to 128)", a.H, a.G, a.D, a.E);
+  MSA_REQUIRE(a.qkv_stride >= 2LL * a.G * a.D + (int64_t)a.H * a.E && a.b_stride >= a.H, "msa_seq_delta_step: strides");
+  MSA_REQUIRE(low->rank > 0 && low->rank % 8 == 0 && low->a_stride >= low->rank && low->g_stride >= low->rank && low->a_stride % 8 == 0 &&
+                  low->g_stride % 8 == 0 && low->n_a >= a.H * a.D &&
+                  (((uintptr_t)low->a_low | (uintptr_t)low->g_low | (uintptr_t)low->w) & 15) == 0,
+              "msa_seq_delta_step: rank=%d (a multiple of 8, 16-byte aligned rows)", low->rank);
+  hipStream_t st = as_stream(stream);
+  if (a.D <= 16) launch_step<4, 4>(a, *low, *batch, st);
+  else if (a.D <= 32) launch_step<8, 4>(a, *low, *batch, st);
+  else if (a.D <= 64) launch_step<16, 4>(a, *low, *batch, st);
+  else if ((int64_t)a.H * batch->n_seq <= device_compute_units() / 2) launch_step<16, 8>(a, *low, *batch, st);
+  else launch_step<32, 4>(a, *low, *batch, st);
+  MSA_LAUNCH_CHECK();
+  return MSA_OK;
+}
 
 extern "C" int msa_seq_delta_scan(const msa_delta_args* args, int32_t dtype, const msa_seq_batch* batch, void* stream) {
   MSA_CHECK_BATCH(batch, "msa_seq_delta_scan");

@@ -12,7 +12,10 @@
 namespace {
 
 struct ResNorm {
-  const float* x_in;
+  const float* x_in;          // or, with tokens, rows of an embedding table
+  const int64_t* tokens;
+  const void* table;
+  int64_t vocab;
   const void* y;
   const void* gate;
   const float* gate_bias;
@@ -41,7 +44,8 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResNorm a, msa_seq_b
   if (a.shift) load_vec<float, VEC>(a.shift + col, sh);
   struct Raw { float x[VEC], y[VEC], g[VEC]; };
   auto fetch = [&](int t, Raw& r) {
-    load_vec<float, VEC>(a.x_in + (int64_t)t * a.W + col, r.x);
+    if (a.tokens) load_vec<T, VEC>(static_cast<const T*>(a.table) + embed_row(a.tokens[t], a.vocab, true) * a.W + col, r.x);
+    else load_vec<float, VEC>(a.x_in + (int64_t)t * a.W + col, r.x);
     if (!a.y) return;
     load_vec<T, VEC>(static_cast<const T*>(a.y) + t * a.y_stride + col, r.y);
     load_vec<T, VEC>(static_cast<const T*>(a.gate) + t * a.gate_stride + col, r.g);
@@ -412,25 +416,19 @@ int grid_for(int64_t items) { return (int)std::min<int64_t>(std::max<int64_t>(1,
 
 }  // namespace
 
-extern "C" int msa_seq_residual_norm(const float* x_in, const void* y, int64_t y_stride, const void* gate, int64_t gate_stride,
-                                     const float* gate_bias, float* x_out, int32_t dtype, int32_t W, const msa_dyn_tanh* norm,
-                                     void* h, const float* shift, float* prev, void* h_shift, const msa_seq_batch* batch,
-                                     void* stream) {
-  MSA_CHECK_BATCH(batch, "msa_seq_residual_norm");
-  MSA_CHECK_DTYPE(dtype, "msa_seq_residual_norm");
-  MSA_REQUIRE(x_in && W > 0, "msa_seq_residual_norm: null stream or W=%d", W);
-  MSA_REQUIRE(!y || (gate && gate_bias && x_out && x_out != x_in && y_stride >= W && gate_stride >= W),
-              "msa_seq_residual_norm: a sublayer output needs its gate, strides of at least W and an x_out that is not x_in");
-  const bool with_norm = norm && norm->w;
-  MSA_REQUIRE(!with_norm || norm->b, "msa_seq_residual_norm: norm without b");
-  MSA_REQUIRE(!with_norm || h || shift, "msa_seq_residual_norm: norm without an output");
-  MSA_REQUIRE(!shift || (with_norm && prev && h_shift), "msa_seq_residual_norm: shift needs norm, prev and h_shift");
-  ResNorm a{x_in, y, gate, gate_bias, y ? x_out : nullptr, with_norm ? *norm : msa_dyn_tanh{}, with_norm ? h : nullptr,
-            shift, prev, h_shift, y_stride, gate_stride, W, 1};
+static int residual_norm(ResNorm a, int32_t dtype, const msa_seq_batch* batch, void* stream, const char* who) {
+  MSA_CHECK_BATCH(batch, who);
+  MSA_CHECK_DTYPE(dtype, who);
+  MSA_REQUIRE(a.W > 0, "%s: W=%d", who, a.W);
+  MSA_REQUIRE(!a.norm.w || a.norm.b, "%s: norm without b", who);
+  MSA_REQUIRE(!a.norm.w || a.h || a.shift, "%s: norm without an output", who);
+  MSA_REQUIRE(!a.shift || (a.norm.w && a.prev && a.h_shift), "%s: shift needs norm, prev and h_shift", who);
+  if (!a.norm.w) a.h = nullptr;
   a.rows_per_wg = batch->rows <= 256 ? 1 : 8;
-  const bool vec = vec_ok(4, {x_in, y, gate, gate_bias, x_out, a.norm.w, a.norm.b, h, shift, prev, h_shift}, {W, y_stride, gate_stride});
+  const bool vec = vec_ok(4, {a.x_in, a.table, a.y, a.gate, a.gate_bias, a.x_out, a.norm.w, a.norm.b, a.h, a.shift, a.prev, a.h_shift},
+                          {a.W, a.y_stride, a.gate_stride});
   const int V = vec ? 4 : 1;
-  const dim3 grid((batch->rows + a.rows_per_wg - 1) / a.rows_per_wg, (W + 256 * V - 1) / (256 * V));
+  const dim3 grid((batch->rows + a.rows_per_wg - 1) / a.rows_per_wg, (a.W + 256 * V - 1) / (256 * V));
   hipStream_t st = as_stream(stream);
   if (dtype == MSA_BF16) {
     if (vec) residual_norm_kernel<bf16_t, 4><<<grid, 256, 0, st>>>(a, *batch);
@@ -441,6 +439,25 @@ extern "C" int msa_seq_residual_norm(const float* x_in, const void* y, int64_t y
   }
   MSA_LAUNCH_CHECK();
   return MSA_OK;
+}
+
+extern "C" int msa_seq_residual_norm(const float* x_in, const void* y, int64_t y_stride, const void* gate, int64_t gate_stride,
+                                     const float* gate_bias, float* x_out, int32_t dtype, int32_t W, const msa_dyn_tanh* norm,
+                                     void* h, const float* shift, float* prev, void* h_shift, const msa_seq_batch* batch,
+                                     void* stream) {
+  MSA_REQUIRE(x_in, "msa_seq_residual_norm: null stream");
+  MSA_REQUIRE(!y || (gate && gate_bias && x_out && x_out != x_in && y_stride >= W && gate_stride >= W),
+              "msa_seq_residual_norm: a sublayer output needs its gate, strides of at least W and an x_out that is not x_in");
+  return residual_norm({x_in, nullptr, nullptr, 0, y, gate, gate_bias, y ? x_out : nullptr, norm ? *norm : msa_dyn_tanh{}, h, shift, prev,
+                        h_shift, y_stride, gate_stride, W, 1}, dtype, batch, stream, "msa_seq_residual_norm");
+}
+
+extern "C" int msa_seq_embed_norm(const int64_t* tokens, const void* table, int64_t vocab, float* x_out, int32_t dtype, int32_t W,
+                                  const msa_dyn_tanh* norm, void* h, const float* shift, float* prev, void* h_shift,
+                                  const msa_seq_batch* batch, void* stream) {
+  MSA_REQUIRE(tokens && table && vocab > 0 && x_out, "msa_seq_embed_norm: null pointer or vocab=%lld", (long long)vocab);
+  return residual_norm({nullptr, tokens, table, vocab, nullptr, nullptr, nullptr, x_out, norm ? *norm : msa_dyn_tanh{}, h, shift, prev,
+                        h_shift, 0, 0, W, 1}, dtype, batch, stream, "msa_seq_embed_norm");
 }
 
 extern "C" int msa_seq_gelu(void* y, int64_t y_stride, int32_t dtype, int32_t rows, int32_t n, void* stream) {

@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import torch
 
-from . import seq_ops
+from . import ops, seq_ops
 from .cache import SequenceStateCache
 from .config import HybridConfig
 from .hybrid_layers import HybridLayer, load_norm, norm_shapes
@@ -50,11 +50,18 @@ class HybridForCausalLM(StepDecoder):
         layer = self.layers[self.runs[r][0]]
         return {"norm": layer.norm1, "shift": layer.shift, "prev": cache.tensors[r]["shift"]}
 
+    def _start(self, tokens, batch, cache):
+        """The stream and what the first run reads of it (nothing yet where that projects the stream first)."""
+        consumer = None if not self.runs or self._starts_pass(0) else self._consumer(0, cache)
+        if consumer is None or self.embed.dtype != self.dtype or not ops.embed_ok(self.embed, tokens):
+            return self._embed(tokens), None, None
+        return seq_ops.embed_norm(tokens, self.embed, batch, **consumer)
+
     def _block_rows(self, tokens, batch, cache, trace=None):
         """Any rows: every element-wise step a kernel of its own between the products."""
         dt = self.dtype
-        x0 = x = self._embed(tokens)
-        h = hs = None
+        x, h, hs = self._start(tokens, batch, cache)
+        x0 = x
         for r, (i, t) in enumerate(self.runs):
             layer, state = self.layers[i], self.run_state(cache, r)
             if self._starts_pass(r):
@@ -75,9 +82,8 @@ class HybridForCausalLM(StepDecoder):
     def _decode_rows(self, tokens, batch, cache, trace=None):
         """One token for each of up to 16 sequences (bf16)."""
         loop = self.config.loop
-        x0 = self._embed(tokens)
+        x0, h, hs = self._start(tokens, batch, cache)
         x = x0.clone() if loop is not None and loop.start > 0 else x0
-        h = hs = None
         for r, (i, t) in enumerate(self.runs):
             layer, state = self.layers[i], self.run_state(cache, r)
             if self._starts_pass(r):

@@ -242,6 +242,11 @@ class ChannelDeltaMixer:
         n_b = self.w_in.shape[0]
         out = seq_ops.rows_conv(hs, w, h, n_b, 0, self.taps, None, state["conv"], batch.slot)
         a_low, g_low = self._low(out)
+        c = self.c
+        if c.heads * batch.n_seq <= seq_ops.DELTA_STEP_HEADS and c.dim <= 128 and c.vdim <= 128 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
+            return seq_ops.delta_step(out[:, :c.conv_channels], a_low, g_low, self.w_low, self.n_a, out[:, self.b_at:self.b_at + c.heads],
+                                      self.A_log, self.dt_bias, self.norm, self.eps, c.heads, c.kv_heads, c.dim, c.vdim, state["delta"],
+                                      batch), out[:, n_b:]
         low = seq_ops.rows_linear(a_low, self.w_low, x_b=g_low, n_b=self.n_a)
         return self._rule(out[:, :self.c.conv_channels], low[:, :self.n_a], low[:, self.n_a:], out, state, batch), out[:, n_b:]
 

@@ -121,7 +121,11 @@ class MSAModel(nn.Module):
         self.norm = RMSNorm(config.hidden_size, config.rms_norm_eps)
 
     def forward(self, input_ids, attention_mask, position_ids, past_key_values, doc_ids, final_norm: bool = True):
-        h = self.embed_tokens(input_ids)
+        e = self.embed_tokens
+        if (type(e) is nn.Embedding and e.max_norm is None and ops.plain_module(e) and ops.embed_ok(e.weight, input_ids)):
+            h = ops.embed_rows(e.weight, input_ids)
+        else:
+            h = e(input_ids)
         if past_key_values is not None and attention_mask is not None and input_ids.shape[1] > 1:
             past_key_values.meta["q_lens_host"] = attention_mask.sum(dim=1).tolist()   # one sync per forward, not per layer
             if h.is_cuda and position_ids is not None:

@@ -463,28 +463,48 @@ def tile_linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
     return out
 
 
-TILE_MIN = 144          # tiles of 256 x 256 from which tile_linear is at least the vendor's equal
+TILE_MIN = 144 << 16    # outputs (144 tiles of 256 x 256) from which tile_linear is at least the vendor's equal
+TILE_ROWS = 256         # no matrix of the models has outputs enough for fewer rows
 
 
 def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1) -> bool:
-    """Whether ``x [..., K] @ w.T`` (``matrices`` of w's shape in one) is ``tile_linear``'s: operands as it takes them, no gradients asked for, and tiles enough to fill the
-    compute units.  Below ``TILE_MIN`` tiles the vendor's smaller ones win (us, vendor and here, K x N: 2560 x 2560 of 2048 tokens, 80
-    tiles, 31 and 43; of 4096, 160 tiles, 50 and 51; of 16384, 640 tiles, 233 and 161; 2560 x 19456 of 1000, 304 tiles, 102 and 90).
-    Depths under 1024 were not measured and stay where they were."""
+    """Whether ``x [..., K] @ w.T`` (``matrices`` of w's shape in one) is ``tile_linear``'s: operands as it takes them, no gradients asked
+    for, and outputs enough to fill the compute units.  Below ``TILE_MIN`` the vendor's smaller tiles win (us, vendor and here, K x N: 2560 x 2560 of 2048 tokens, 80
+    tiles, 31 and 43; of 4096, 160 tiles, 50 and 51; of 16384, 640 tiles, 233 and 161; 2560 x 19456 of 1000, 304 tiles, 102 and 90), and
+    padding does not count (2560 x 12288 of 573 tokens, 107 tiles' outputs in 144, 45 and 61).  Depths under 1024 were not measured and
+    stay where they were."""
     K, N = x.shape[-1], matrices * w.shape[0]
     T = x.shape[0] if x.dim() == 2 else x.numel() // max(K, 1)
-    if (T + 255) * (N + 255) < TILE_MIN << 16:      # (most calls end here: steps of few tokens wait for the host)
+    if T * N < TILE_MIN:                            # (most calls end here: steps of few tokens wait for the host)
         return False
     return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == K
             and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 21))
             and K % 64 == 0 and 1024 <= K <= 32768 and N % 8 == 0 and N < 1 << 20 and T < 1 << 22
-            and -(-T // 256) * -(-N // 256) >= TILE_MIN and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
 
 
 def plain_module(module: torch.nn.Module) -> bool:
     """Whether nothing but the module's own ``forward`` runs when it is called."""
     return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+
+
+def embed_ok(table: torch.Tensor, tokens: torch.Tensor) -> bool:
+    """Whether ``embed_rows`` takes the lookup (torch's own takes the others)."""
+    return (table.is_cuda and tokens.device == table.device and table.dim() == 2 and table.dtype in (torch.bfloat16, torch.float32)
+            and tokens.dtype == torch.int64 and tokens.numel() > 0 and table.shape[1] % 8 == 0 and table.is_contiguous()
+            and tokens.is_contiguous() and table.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and table.requires_grad))
+
+
+def embed_rows(table: torch.Tensor, tokens: torch.Tensor, f32: bool = False, wrap: bool = False, lib=None):
+    """``table[tokens]`` and, with ``f32``, the same in fp32 (``(rows, rows in fp32)``).  ``wrap``: negative tokens count from the end."""
+    _need_cuda(table, tokens)
+    out = torch.empty((*tokens.shape, table.shape[1]), dtype=table.dtype, device=table.device)
+    wide = torch.empty(out.shape, dtype=torch.float32, device=table.device) if f32 else None
+    lib = lib or _lib.load()
+    check(lib.msa_embed_rows(ptr(tokens), tokens.numel(), ptr(table), table.shape[0], wrap, table.shape[1], dtype_code(table.dtype), ptr(out),
+                             ptr(wide), _stream()), "msa_embed_rows", lib)
+    return (out, wide) if f32 else out
 
 
 def linear_ok(module: torch.nn.Module, x: torch.Tensor) -> bool:

@@ -7,7 +7,7 @@ that reads it (``seq_ops.PostRows``), the convolution into the mixer's input pro
 """
 from __future__ import annotations
 
-from . import seq_ops
+from . import _lib, ops, seq_ops
 from .config import PostNormConfig
 from .hybrid_layers import F32, PostNormLayer
 from .step_decoder import StepDecoder
@@ -29,9 +29,13 @@ class PostNormForCausalLM(StepDecoder):
         return seq_ops.rms_residual(x, self.dtype, y, w, self.config.norm_eps, self.final_norm if last else None, out=x)
 
     def _start(self, tokens):
+        as_it_is = self.layers and self.embed.dtype == self.dtype != F32     # the stream in the activations' type is the row itself
+        if as_it_is and ops.embed_ok(self.embed, tokens):
+            e, x = ops.embed_rows(self.embed, tokens, f32=True, wrap=True, lib=_lib.load_seq())
+            return x, e
         e = self.embed[tokens]
         x = e.to(F32)
-        if self.layers and e.dtype == self.dtype != F32:     # (the stream in the activations' type is the row itself)
+        if as_it_is:
             return x, e
         _, h = seq_ops.rms_residual(x, self.dtype, eps=self.config.norm_eps, next_w=None if self.layers else self.final_norm)
         return x, h

@@ -152,6 +152,25 @@ def residual_norm(x: torch.Tensor, batch: StepBatch, dtype: torch.dtype, y=None,
     return (x if y is None else x_out), h, hs
 
 
+def embed_norm(tokens: torch.Tensor, table: torch.Tensor, batch: StepBatch, norm: DynTanhNorm, shift=None, prev=None):
+    """``(x, h, h_shift)`` of :func:`residual_norm` where the stream is ``table[tokens]``."""
+    _dense(tokens, table, prev)
+    (T, W), dtype = (batch.rows, table.shape[1]), table.dtype
+    _f32(W, norm.w, norm.b)
+    if tokens.dtype != torch.int64 or tokens.numel() != T:
+        raise ValueError("tokens must be int64 [rows]")
+    if shift is not None:
+        _f32(W, shift)
+        if prev.dtype != torch.float32 or prev.shape[1] != W or prev.shape[0] <= max(batch.slots):
+            raise ValueError("prev must be fp32 [slots, W]")
+    x = torch.empty((T, W), dtype=torch.float32, device=table.device)
+    h = torch.empty((T, W), dtype=dtype, device=table.device)
+    hs = torch.empty((T, W), dtype=dtype, device=table.device) if shift is not None else None
+    _check(_lib.load_seq().msa_seq_embed_norm(ptr(tokens), ptr(table), table.shape[0], ptr(x), dtype_code(dtype), W, C.byref(norm.c), ptr(h),
+                                              ptr(shift), ptr(prev), ptr(hs), batch.ref, _stream()), "msa_seq_embed_norm")
+    return x, h, hs
+
+
 def rms_residual(x: torch.Tensor, dtype: torch.dtype, y=None, w=None, eps: float = 0.0, next_w=None, out=None, want_h: bool = True):
     """``(x', h)``: ``x' = x + rms_norm(y) * w`` (``x`` itself without ``y``; into ``out``, which may be ``x``), and ``h = x'``, or
     ``rms_norm(x') * next_w``, in ``dtype``."""
@@ -190,12 +209,12 @@ def clamped_glu(gu: torch.Tensor, limit: float, alpha: float = GLU_ALPHA, shift:
 
 def product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x @ w.T`` of a step's rows."""
-    return ops.tile_linear(x, w) if ops.tile_linear_ok(x, w) else F.linear(x, w)
+    return ops.tile_linear(x, w) if x.shape[0] >= ops.TILE_ROWS and ops.tile_linear_ok(x, w) else F.linear(x, w)
 
 
 def product_gelu(x: torch.Tensor, w: torch.Tensor, n: int) -> torch.Tensor:
     """``x @ w.T``, its first ``n`` columns through gelu."""
-    if n % 8 == 0 and ops.tile_linear_ok(x, w):
+    if x.shape[0] >= ops.TILE_ROWS and n % 8 == 0 and ops.tile_linear_ok(x, w):
         return ops.tile_linear(x, w, gelu_n=n)
     y = F.linear(x, w)
     gelu_(y[:, :n])
@@ -204,7 +223,7 @@ def product_gelu(x: torch.Tensor, w: torch.Tensor, n: int) -> torch.Tensor:
 
 def product_glu(x: torch.Tensor, w: torch.Tensor, limit: float, alpha: float = GLU_ALPHA, shift: float = GLU_SHIFT) -> torch.Tensor:
     """``clamped_glu(x @ w.T)``."""
-    if w.shape[0] % 16 == 0 and ops.tile_linear_ok(x, w):
+    if x.shape[0] >= ops.TILE_ROWS and w.shape[0] % 16 == 0 and ops.tile_linear_ok(x, w):
         return ops.tile_linear(x, w, glu=(limit, alpha, shift))
     return clamped_glu(F.linear(x, w), limit, alpha, shift)
 
@@ -313,6 +332,34 @@ def delta(qkv, a, b, gate, A_log, dt_bias, norm, eps: float, H: int, G: int, D: 
         _check(lib.msa_seq_delta_chunked(C.byref(c), batch.ref, ptr(ws), ws.numel(), _stream()), "msa_seq_delta_chunked")
     else:
         _check(lib.msa_seq_delta_scan(C.byref(c), dtype_code(qkv.dtype), batch.ref, _stream()), "msa_seq_delta_scan")
+    return out
+
+
+# Heads of all sequences up to which a decode step forms the low rank's second product beside its state: a workgroup a head, one a
+# compute unit.  A whole step, us, product apart and here: 16 heads 188.7 and 186.1, 128 (1b) 214.2 and 210.0, 256 (1b) 240.0 and 232.9,
+# (4b) 448.1 and 441.4; 512 498 and 521 (its registers leave one workgroup a compute unit instead of two).
+DELTA_STEP_HEADS = 256
+
+
+def delta_step(qkv, a_low, g_low, w_low, n_a: int, b, A_log, dt_bias, norm, eps: float, H: int, G: int, D: int, E: int, state,
+               batch: StepBatch) -> torch.Tensor:
+    """:func:`delta` for one bf16 token a sequence, D and E up to 128, with ``a = a_low @ w_low[:H D].T`` and
+    ``gate = g_low @ w_low[n_a:].T`` formed in the same launch."""
+    T, R = batch.rows, w_low.shape[1]
+    _f32(H, A_log)
+    _f32(H * D, dt_bias)
+    _f32(E, norm)
+    _dense(state, w_low)
+    if state.dtype != torch.float32 or tuple(state.shape[1:]) != (H, D, E) or state.shape[0] <= max(batch.slots):
+        raise ValueError("state must be fp32 [slots, H, D, E]")
+    if qkv.shape != (T, 2 * G * D + H * E) or b.shape != (T, H) or a_low.shape != (T, R) or g_low.shape != (T, R) or \
+            w_low.shape[0] < n_a + H * E or n_a < H * D or not (qkv.dtype == b.dtype == a_low.dtype == g_low.dtype == w_low.dtype == torch.bfloat16):
+        raise ValueError("bf16 qkv [rows, 2 G D + H E], b [rows, H], a_low and g_low [rows, rank], w_low [n_a + H E, rank]")
+    out = torch.empty((T, H * E), dtype=qkv.dtype, device=qkv.device)
+    c = _lib.DeltaArgs(ptr(qkv), None, ptr(b), None, _rows(qkv), 0, _rows(b), 0, ptr(A_log), ptr(dt_bias), ptr(norm), ptr(state), ptr(out),
+                       H, G, D, E, eps, 0)
+    low = _lib.DeltaLow(ptr(a_low), ptr(g_low), ptr(w_low), _rows(a_low), _rows(g_low), R, n_a)
+    _check(_lib.load_seq().msa_seq_delta_step(C.byref(c), C.byref(low), batch.ref, _stream()), "msa_seq_delta_step")
     return out
 
 
