@@ -304,6 +304,12 @@ int msa_flash_attn_hint(const void* q, const int32_t* cu_q, const void* k, const
                         const int64_t* kv_off, const int32_t* kv_len, int32_t B, int32_t total_q,
                         int32_t Hq, int32_t Hkv, int32_t D, float scale, int32_t causal, void* out,
                         int32_t max_sq, void* stream);
+/* Causal attention of rows as a decoder of mixed layers has them: query rows q_stride elements apart, sample b's keys end with its own rows
+ * behind kv_pos[b] earlier ones.  sink [Hq] (or NULL): a member of every softmax of head h without a value; gate [rows, Hq] bf16, rows
+ * gate_stride apart (or NULL): outputs times its sigmoid.  out [rows, Hq, D] dense. */
+int msa_flash_attn_rows(const void* q, int64_t q_stride, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
+                        const int64_t* kv_pos, int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv, int32_t D,
+                        float scale, const float* sink, const void* gate, int64_t gate_stride, void* out, void* stream);
 /* msa_flash_attn has two forms of its kernel: 32 (token, head) columns per wavefront, two workgroups per compute unit,
  * and a wide one (64 columns per wavefront, one wavefront per SIMD, the tile step written at the instruction level)
  * that it picks when the call has at least 4096 columns.  form 0: by size (the default), 1: always the first,

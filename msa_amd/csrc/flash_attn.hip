@@ -112,6 +112,25 @@ __device__ __forceinline__ void load4_to_lds(u32x4_t rsrc, uint32_t lds_dst, int
 #endif
 }
 
+// What a call may have besides: query rows of a wider tensor, a sink per query head (a member of every softmax that has no value), outputs
+// times the sigmoid of a gate per row and head, and keys that end with the sample's own rows behind kv_pos earlier ones (without kv_len).
+struct RowOptions {
+  int64_t q_stride;          // elements between query rows
+  const float* sink;         // [Hq] or null
+  const bf16_t* gate;        // [rows, Hq], rows gate_stride apart, or null
+  int64_t gate_stride;
+  const int64_t* kv_pos;     // [B], used where kv_len is null
+};
+constexpr float kLog2e = 1.4426950408889634f;
+
+// What a column's sums are multiplied by: 1 / (their weights and the sink's, which is infinite behind a reference maximum of no key).
+__device__ __forceinline__ float column_factor(const RowOptions& x, float m, float l, int head, int64_t row, bool live) {
+  if (x.sink) l += fast_exp2(x.sink[head] * kLog2e - m);
+  float f = l > 0.f ? 1.0f / l : 0.f;              // a row that sees no key yields zeros
+  if (x.gate && live) f *= __builtin_amdgcn_rcpf(1.0f + fast_exp2(-kLog2e * bf16_to_f32(x.gate[row * x.gate_stride + head])));
+  return f;
+}
+
 // kSplit: blockIdx.z selects a range of split_keys keys; the un-normalised accumulators and the
 // (reference max, sum) pair of every column go to part_acc / part_ml for the combine kernel.
 template <int G, bool kSplit>
@@ -119,7 +138,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void flash_attn_kernel(
     const bf16_t* __restrict__ q, const int32_t* __restrict__ cu_q, const bf16_t* __restrict__ k,
     const bf16_t* __restrict__ v, const int64_t* __restrict__ kv_off, const int32_t* __restrict__ kv_len, int32_t B,
     int32_t Hq, int32_t Hkv, float scale_log2e, int32_t causal, bf16_t* __restrict__ out, int32_t n_split,
-    int32_t split_keys, float* __restrict__ part_ml, float* __restrict__ part_acc) {
+    int32_t split_keys, float* __restrict__ part_ml, float* __restrict__ part_acc, RowOptions opt) {
   constexpr int kTokPerWave = 32 / G;
   constexpr int kTokPerBlock = kWaves * kTokPerWave;
   constexpr int kLoads = kTileBytes / (kWaves * 64 * 16);     // load instructions per wavefront, tile and tensor
@@ -150,7 +169,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void flash_attn_kernel(
   const int q_first = cu_q ? cu_q[b] : b;
   const int sq = cu_q ? cu_q[b + 1] - q_first : 1;
   const int t0 = blk * kTokPerBlock;
-  const int L = kv_len[b];
+  const int L = kv_len ? kv_len[b] : (int)opt.kv_pos[b] + sq;
   const int64_t base = kv_off[b];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -173,7 +192,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void flash_attn_kernel(
   // dims 16 s + 8 half .. + 8 of its column's query row.
   bf16x8_t qf[8];
   {
-    const bf16_t* qrow = q + ((int64_t)(q_first + (col_ok ? tok : 0)) * Hq + head) * kHeadDim + 8 * half;
+    const bf16_t* qrow = q + (int64_t)(q_first + (col_ok ? tok : 0)) * opt.q_stride + head * kHeadDim + 8 * half;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       uint4 w = col_ok ? *reinterpret_cast<const uint4*>(qrow + 16 * s) : make_uint4(0, 0, 0, 0);
@@ -436,7 +455,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void flash_attn_kernel(
               make_float4(o[d][4 * e4], o[d][4 * e4 + 1], o[d][4 * e4 + 2], o[d][4 * e4 + 3]);
     }
   } else if (col_ok) {
-    const float inv = l > 0.f ? 1.0f / l : 0.f;        // a row that sees no key yields zeros
+    const float inv = column_factor(opt, m, l, head, q_first + tok, true);
     bf16_t* orow = out + ((int64_t)(q_first + tok) * Hq + head) * kHeadDim;
 #pragma unroll
     for (int d = 0; d < 4; ++d)
@@ -481,7 +500,7 @@ template <int G>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVgprs))) void flash_wide_kernel(
     const bf16_t* __restrict__ q, const int32_t* __restrict__ cu_q, const bf16_t* __restrict__ k,
     const bf16_t* __restrict__ v, const int64_t* __restrict__ kv_off, const int32_t* __restrict__ kv_len, int32_t B,
-    int32_t Hq, int32_t Hkv, float scale_log2e, int32_t causal, bf16_t* __restrict__ out, int32_t total_blocks) {
+    int32_t Hq, int32_t Hkv, float scale_log2e, int32_t causal, bf16_t* __restrict__ out, int32_t total_blocks, RowOptions opt) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int kTokPerWave = 64 / G;
   constexpr int kTokPerBlock = 4 * kTokPerWave;
@@ -539,7 +558,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVg
           blkout.q_first = first;
           blkout.sq = sq_b;
           blkout.t0 = blk * kTokPerBlock;
-          blkout.L = kv_len[cur_b];
+          blkout.L = kv_len ? kv_len[cur_b] : (int)opt.kv_pos[cur_b] + sq_b;
           blkout.base = kv_off[cur_b];
           const int last_tok = min(sq_b, blkout.t0 + kTokPerBlock) - 1;
           blkout.kmax = causal ? max(0, min(blkout.L, blkout.L - sq_b + last_tok + 1)) : blkout.L;
@@ -591,9 +610,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVg
   auto request_block = [&](const Block& nb) {
     {
       // the wavefront's 64 columns are 16 blocks of four rows; a buffer resource over the sample's query rows
-      const uintptr_t qa = reinterpret_cast<uintptr_t>(q) + (uintptr_t)nb.q_first * Hq * kRowBytes;
-      const u32x4_t rq = {(uint32_t)qa, (uint32_t)(qa >> 32) & 0xffffu, (uint32_t)min((int64_t)nb.sq * Hq * kRowBytes, (int64_t)0xffffff00),
-                          0x00020000u};
+      const uintptr_t qa = reinterpret_cast<uintptr_t>(q) + (uintptr_t)nb.q_first * opt.q_stride * 2;
+      const int64_t extent = (int64_t)(nb.sq - 1) * opt.q_stride * 2 + Hq * kRowBytes;
+      const u32x4_t rq = {(uint32_t)qa, (uint32_t)(qa >> 32) & 0xffffu, (uint32_t)min(extent, (int64_t)0xffffff00), 0x00020000u};
+      const int q_row = (int)opt.q_stride * 2;
       int lane_q = lane;
       asm volatile("" : "+v"(lane_q));
 #pragma unroll
@@ -605,7 +625,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVg
           const int tok = nb.t0 + wave * kTokPerWave + col / G;
           const int piece = (lane_q & 15) ^ (col & 15);
           // a column past the sample's rows reads from beyond the extent (nothing is fetched; the column is masked)
-          qo[jj] = tok < nb.sq ? (tok * Hq + g * G + col % G) * kRowBytes + piece * 16 : -16;
+          qo[jj] = tok < nb.sq ? tok * q_row + (g * G + col % G) * kRowBytes + piece * 16 : -16;
         }
         asm volatile(FLASHW_LOADQ4 ::[dst] "s"(ldsq + j4 * 4096), [r] "s"(rq), [o0] "v"(qo[0]), [o1] "v"(qo[1]),
                      [o2] "v"(qo[2]), [o3] "v"(qo[3])
@@ -716,7 +736,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVg
     FLASHW_ASM(FLASHW_DRAIN);
     float m0, m1, lsum[2];
     asm volatile(FLASHW_GET_ML : "=v"(m0), "=v"(m1), "=v"(lsum[0]), "=v"(lsum[1]));
-    (void)m0; (void)m1;
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
     int64_t orow_e[2];
@@ -746,8 +765,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVg
     float inv[2];
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
-      const float l = half_wave_sum(lsum[cb]);
-      inv[cb] = l > 0.f ? 1.0f / l : 0.f;        // a row that sees no key yields zeros
+      const int col = 32 * cb + (lane_e & 31);
+      inv[cb] = column_factor(opt, cb ? m1 : m0, half_wave_sum(lsum[cb]), g * G + col % G, cur.q_first + cur.t0 + wave * kTokPerWave + col / G,
+                              ok_e[cb]);
     }
     FLASHW_STORE(0, 0) FLASHW_STORE(0, 1) FLASHW_STORE(0, 2) FLASHW_STORE(0, 3)
     FLASHW_STORE(1, 0) FLASHW_STORE(1, 1) FLASHW_STORE(1, 2) FLASHW_STORE(1, 3)
@@ -762,7 +782,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVg
 template <int G>
 int flash_wide_launch_g(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                         const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
-                        int32_t causal, void* out, hipStream_t st) {
+                        int32_t causal, void* out, const RowOptions& opt, hipStream_t st) {
   constexpr int kTokPerBlock = 4 * 64 / G;
   const int64_t blocks = ((int64_t)total_q + kTokPerBlock - 1) / kTokPerBlock + B;   // upper bound over ragged samples
   MSA_REQUIRE(blocks < (int64_t)1 << 30, "flash attention: too many query rows");
@@ -776,7 +796,7 @@ int flash_wide_launch_g(const void* q, const int32_t* cu_q, const void* k, const
   MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(kern), kWideLdsBytes));
   kern<<<dim3((unsigned)(per_head * Hkv)), 256, kWideLdsBytes, st>>>(
       static_cast<const bf16_t*>(q), cu_q, static_cast<const bf16_t*>(k), static_cast<const bf16_t*>(v), kv_off, kv_len,
-      B, Hq, Hkv, scale * 1.4426950408889634f, causal, static_cast<bf16_t*>(out), (int32_t)blocks);
+      B, Hq, Hkv, scale * kLog2e, causal, static_cast<bf16_t*>(out), (int32_t)blocks, opt);
   MSA_LAUNCH_CHECK();
   return MSA_OK;
 }
@@ -798,7 +818,7 @@ std::atomic<int> g_flash_form{0};   // 0: by size, 1: the 32-column form, 2: the
 template <int G, bool kSplit>
 int flash_launch_g(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                    const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
-                   int32_t causal, void* out, SplitPlan plan, float* part_ml, float* part_acc, hipStream_t st) {
+                   int32_t causal, void* out, SplitPlan plan, float* part_ml, float* part_acc, const RowOptions& opt, hipStream_t st) {
   constexpr int kTokPerBlock = kWaves * 32 / G;
   const int64_t blocks = ((int64_t)total_q + kTokPerBlock - 1) / kTokPerBlock + B;   // upper bound over ragged samples
   MSA_REQUIRE(blocks * Hkv < (int64_t)1 << 31, "flash attention: too many query rows");
@@ -808,8 +828,8 @@ int flash_launch_g(const void* q, const int32_t* cu_q, const void* k, const void
   MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(kern), kLdsBytes));
   kern<<<grid, kWaves * 64, kLdsBytes, st>>>(static_cast<const bf16_t*>(q), cu_q, static_cast<const bf16_t*>(k),
                                              static_cast<const bf16_t*>(v), kv_off, kv_len, B, Hq, Hkv,
-                                             scale * 1.4426950408889634f, causal, static_cast<bf16_t*>(out),
-                                             kSplit ? plan.n_split : 1, kSplit ? plan.split_keys : 0, part_ml, part_acc);
+                                             scale * kLog2e, causal, static_cast<bf16_t*>(out),
+                                             kSplit ? plan.n_split : 1, kSplit ? plan.split_keys : 0, part_ml, part_acc, opt);
   MSA_LAUNCH_CHECK();
   return MSA_OK;
 }
@@ -829,10 +849,14 @@ int flash_launch(int G, Args... args) {
 }  // namespace
 
 namespace {
+bool wide_enough(int32_t total_q, int32_t Hq, int32_t Hkv) { return Hkv > 0 && (int64_t)total_q * (Hq / Hkv) >= 4096; }
+RowOptions dense_rows(int32_t Hq, int32_t D) { return {(int64_t)Hq * D, nullptr, nullptr, 0, nullptr}; }
+
 int flash_attn_entry(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                      const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D, float scale,
-                     int32_t causal, void* out, int32_t max_sq, void* stream) {
-  MSA_REQUIRE(q && k && v && kv_off && kv_len && out, "msa_flash_attn: null pointer");
+                     int32_t causal, void* out, int32_t max_sq, bool enough, const RowOptions& opt, void* stream) {
+  MSA_REQUIRE(q && k && v && kv_off && (kv_len || opt.kv_pos) && out, "msa_flash_attn: null pointer");
+  MSA_REQUIRE(opt.q_stride >= (int64_t)Hq * D && opt.q_stride % 8 == 0 && (!opt.gate || opt.gate_stride >= Hq), "msa_flash_attn: strides");
   MSA_REQUIRE(D == kHeadDim, "msa_flash_attn: head dim %d unsupported (need %d)", D, kHeadDim);
   MSA_REQUIRE(B > 0 && total_q > 0, "msa_flash_attn: bad sizes");
   MSA_REQUIRE(cu_q != nullptr || total_q == B, "msa_flash_attn: cu_q is required when total_q != B");
@@ -848,24 +872,39 @@ int flash_attn_entry(const void* q, const int32_t* cu_q, const void* k, const vo
   // the hardware hands out one by one)
   const int form = g_flash_form.load(std::memory_order_relaxed);
   const bool ragged = max_sq > 0 && (int64_t)max_sq * B > (int64_t)total_q + total_q / 4;
-  if (form == 2 || (form == 0 && (int64_t)total_q * G >= 4096 && !ragged))
-    return flash_wide_launch(G, q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, out, as_stream(stream));
+  if (form == 2 || (form == 0 && enough && !ragged))
+    return flash_wide_launch(G, q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, out, opt, as_stream(stream));
   return flash_launch<false>(G, q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale,
-                             causal, out, SplitPlan{1, 0}, (float*)nullptr, (float*)nullptr, as_stream(stream));
+                             causal, out, SplitPlan{1, 0}, (float*)nullptr, (float*)nullptr, opt, as_stream(stream));
 }
 }  // namespace
 
 extern "C" int msa_flash_attn(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                               const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D,
                               float scale, int32_t causal, void* out, void* stream) {
-  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, 0, stream);
+  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, 0, wide_enough(total_q, Hq, Hkv),
+                          dense_rows(Hq, D), stream);
 }
 
 extern "C" int msa_flash_attn_hint(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                                    const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D,
                                    float scale, int32_t causal, void* out, int32_t max_sq, void* stream) {
   MSA_REQUIRE(max_sq > 0, "msa_flash_attn_hint: max_sq must be the longest query block of the batch");
-  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, max_sq, stream);
+  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, max_sq, wide_enough(total_q, Hq, Hkv),
+                          dense_rows(Hq, D), stream);
+}
+
+extern "C" int msa_flash_attn_rows(const void* q, int64_t q_stride, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
+                                   const int64_t* kv_pos, int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv, int32_t D,
+                                   float scale, const float* sink, const void* gate, int64_t gate_stride, void* out, void* stream) {
+  MSA_REQUIRE(cu_q && kv_pos && max_sq > 0, "msa_flash_attn_rows: cu_q, kv_pos and max_sq are required");
+  MSA_REQUIRE((int64_t)max_sq * q_stride < (int64_t)1 << 30, "msa_flash_attn_rows: query rows too far apart");
+  // One and a half blocks of 256 columns a compute unit: us, 32-column form and wide, 32 query heads: 2048 rows, one a unit, 53 and 58, but
+  // behind 4000 keys 176 and 171; 4000 rows in eight samples 43 and 39; 8192 rows 531 and 490; 16 heads: 2048 rows 40 and 54, 6001
+  // 175 and 177, 8192 271 and 250.
+  const bool enough = (int64_t)total_q * Hq * 2 >= (int64_t)3 * 256 * device_compute_units();
+  return flash_attn_entry(q, cu_q, k, v, kv_off, nullptr, B, total_q, Hq, Hkv, D, scale, 1, out, max_sq, enough,
+                          {q_stride, sink, static_cast<const bf16_t*>(gate), gate_stride, kv_pos}, stream);
 }
 
 int flash_wide_kernel_resources(int* num_regs, int* scratch_bytes) {
@@ -884,5 +923,5 @@ int flash_attn_split_launch(const void* q, const int32_t* cu_q, const void* k, c
                             const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
                             int32_t causal, SplitPlan plan, float* part_ml, float* part_acc, hipStream_t st) {
   return flash_launch<true>(Hq / Hkv, q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq,
-                            Hkv, scale, causal, (void*)nullptr, plan, part_ml, part_acc, st);
+                            Hkv, scale, causal, (void*)nullptr, plan, part_ml, part_acc, dense_rows(Hq, kHeadDim), st);
 }

@@ -437,6 +437,18 @@ def flash_ok(dtype, D: int, E: int, scale: float) -> bool:
     return dtype == torch.bfloat16 and D % 8 == 0 and E % 8 == 0 and max(D, E) <= 256 and scale > 0
 
 
+FLASH_ROWS = 512        # of the longest portion
+
+
+def takes_flash_rows(q, k, v, H: int, G: int, D: int, E: int, chunk: int, batch: StepBatch) -> bool:
+    """Whether the attention model's prefill kernels take the call: heads of 128, dense keys and values, and no position behind the first
+    chunk (there it hides nothing).  Long portions gain (us, the general kernel and those, 16 heads of their own keys: 8192 rows 343 and
+    256, 2048 49 and 41, 2048 behind 4000 keys 132 and 111, 1000 27.3 and 26.0); shorter ones wait for the host, which has more to do."""
+    return (batch.max_rows >= FLASH_ROWS and D == E == 128 and H // G in (1, 2, 4, 8) and (not chunk or batch.max_keys <= chunk)
+            and _rows(k) == _rows(v) == G * D and _rows(q) % 8 == 0 and batch.max_rows * _rows(q) < 1 << 30
+            and not (q.data_ptr() | k.data_ptr() | v.data_ptr()) % 16)
+
+
 def flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv_off: torch.Tensor, sink: Optional[torch.Tensor], scale: float, H: int,
           batch: StepBatch, kv_heads: Optional[int] = None, chunk: int = 0, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Causal attention of ``q [rows, H D]`` over ``k [keys, G D]``, ``v [keys, G E]`` (``G = kv_heads``, H without); sequence ``s``
@@ -452,6 +464,11 @@ def flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv_off: torch.Tenso
     if gate is not None and (gate.shape != (batch.rows, H) or gate.dtype != q.dtype):
         raise ValueError("gate must be [rows, H] of the activations' type")
     out = torch.empty((batch.rows, H * E), dtype=q.dtype, device=q.device)
+    if takes_flash_rows(q, k, v, H, G, D, E, chunk, batch):
+        _lib.check(_lib.load().msa_flash_attn_rows(ptr(q), _rows(q), ptr(batch.cu), ptr(k), ptr(v), ptr(kv_off), ptr(batch.pos), batch.n_seq,
+                                                   batch.rows, batch.max_rows, H, G, D, scale, ptr(sink), ptr(gate),
+                                                   _rows(gate) if gate is not None else 0, ptr(out), _stream()), "msa_flash_attn_rows")
+        return out
     _check(_lib.load_seq().msa_seq_flash(ptr(q), _rows(q), ptr(k), _rows(k), ptr(v), _rows(v), ptr(kv_off), ptr(sink), scale,
                                          dtype_code(q.dtype), H, G, D, E, chunk, ptr(gate), _rows(gate) if gate is not None else 0, ptr(out),
                                          batch.ref, _stream()), "msa_seq_flash")
