@@ -368,6 +368,11 @@ typedef struct msa_tile_end {
 size_t msa_tile_workspace_bytes(int64_t T, int32_t K, int32_t N);
 int msa_tile_linear(const void* x, int64_t ldx, int64_t T, int32_t K, const void* w, int32_t N, const msa_tile_end* end, void* out,
                     int64_t ldo, void* ws, size_t ws_bytes, void* stream);
+/* Same for blocks of few tokens, in one launch of smaller tiles without a workspace: MSA_TILE_STORE, MSA_TILE_GLU or MSA_TILE_GELU.
+ * msa_block_linear_us: about what it takes. */
+float msa_block_linear_us(int64_t T, int32_t K, int32_t N);
+int msa_block_linear(const void* x, int64_t ldx, int64_t T, int32_t K, const void* w, int32_t N, const msa_tile_end* end, void* out,
+                     int64_t ldo, void* stream);
 /* msa_qk_norm_rope for a decode step (one new token per sample, N = B) fused with msa_cache_append: the
  * normalised, rotated k row and the v row of sample b are written to kcache / vcache [b][kv_len[b]] and
  * kv_len[b] is incremented (src/msa/memory_sparse_attention.py:129-133 followed by the cache update at

@@ -171,7 +171,7 @@ class LatentAttention:
         else:
             lat = torch.cat([cache[s, :e] for s, e in zip(batch.slots, ends)])
             off = [sum(ends[:i]) for i in range(batch.n_seq)]
-        return seq_ops.flash(q, F.linear(lat, self.uk), F.linear(lat, self.uv),
+        return seq_ops.flash(q, seq_ops.product(lat, self.uk), seq_ops.product(lat, self.uv),
                              torch.tensor(off, dtype=torch.int64).to(q.device), self.sink, c.scale, c.heads, batch)
 
     def decode(self, w, hs, h, state, batch):
@@ -236,7 +236,7 @@ class ChannelDeltaMixer:
     def mix(self, proj, state, batch):
         qkv = seq_ops.conv_silu(proj[:, :self.c.conv_channels], self.taps, None, state["conv"], batch)
         a_low, g_low = self._low(proj)
-        return self._rule(qkv, F.linear(a_low, self.w_low[:self.n_a]), F.linear(g_low, self.w_low[self.n_a:]), proj, state, batch)
+        return self._rule(qkv, seq_ops.product(a_low, self.w_low[:self.n_a]), seq_ops.product(g_low, self.w_low[self.n_a:]), proj, state, batch)
 
     def decode(self, w, hs, h, state, batch):
         n_b = self.w_in.shape[0]

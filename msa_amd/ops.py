@@ -484,6 +484,34 @@ def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1) -> bool:
             and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
 
 
+BLOCK_US, BLOCK_ROWS, BLOCK_DEPTH = 23.0, 2048, 128
+
+
+def block_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``x [T, K] @ w.T`` is ``block_linear``'s: operands as it takes them, no gradients asked for, and one of two cases.  The
+    host takes about 21 us to hand a product to the vendor's library and 7 to this, so up to ``BLOCK_ROWS`` rows, where a prompt waits for
+    the host, products of about that length are here also where the vendor's kernel alone is a little faster (us, the vendor's and here,
+    rows x K x N: 64 x 1024 x 1024 6.6 and 5.0, 1000 x 1024 x 6176 24.2 and 20.5, 2048 x 1024 x 4096 20.6 and 22; behind the line 300 x 2560 x 8192, 25.8
+    and 27.4).  Of more rows those of a depth up to ``BLOCK_DEPTH`` (6001 x 128 x 4096 25.9 and 18.5; 8192 x 256 x 2048 16.7 and 19.0)."""
+    (T, K), N = (x.shape if x.dim() == 2 else (0, 0)), w.shape[0]
+    return (T > 0 and w.dim() == 2 and x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] == K
+            and K % 64 == 0 and 64 <= K <= 32768 and N % 16 == 0 and 0 < N < 1 << 20 and T < 1 << 22 and (T <= BLOCK_ROWS or K <= BLOCK_DEPTH)
+            and _lib.load().msa_block_linear_us(T, K, N) <= BLOCK_US
+            and (x.is_contiguous() or (x.stride(1) == 1 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 21))
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.device == x.device
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+
+
+def block_linear(x: torch.Tensor, w: torch.Tensor, glu: Optional[Tuple[float, float, float]] = None, gelu_n: int = 0) -> torch.Tensor:
+    """``tile_linear`` of few rows (``x`` and ``w`` as ``block_linear_ok`` has them), with ``glu``, ``gelu_n`` or neither."""
+    (T, K), N = x.shape, w.shape[0]
+    out = torch.empty((T, N if glu is None else N // 2), dtype=x.dtype, device=x.device)
+    end = _lib.TileEnd(_lib.TILE_GLU if glu is not None else _lib.TILE_GELU if gelu_n else _lib.TILE_STORE, gelu_n, *(glu or (0.0, 0.0, 0.0)))
+    check(_lib.load().msa_block_linear(x.data_ptr(), x.stride(0) if T > 1 else K, T, K, w.data_ptr(), N, C.byref(end), out.data_ptr(),
+                                       out.shape[1], _stream()), "msa_block_linear")
+    return out
+
+
 def plain_module(module: torch.nn.Module) -> bool:
     """Whether nothing but the module's own ``forward`` runs when it is called."""
     return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)

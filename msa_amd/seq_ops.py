@@ -209,13 +209,17 @@ def clamped_glu(gu: torch.Tensor, limit: float, alpha: float = GLU_ALPHA, shift:
 
 def product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x @ w.T`` of a step's rows."""
-    return ops.tile_linear(x, w) if x.shape[0] >= ops.TILE_ROWS and ops.tile_linear_ok(x, w) else F.linear(x, w)
+    if x.shape[0] >= ops.TILE_ROWS and ops.tile_linear_ok(x, w):
+        return ops.tile_linear(x, w)
+    return ops.block_linear(x, w) if ops.block_linear_ok(x, w) else F.linear(x, w)
 
 
 def product_gelu(x: torch.Tensor, w: torch.Tensor, n: int) -> torch.Tensor:
     """``x @ w.T``, its first ``n`` columns through gelu."""
     if x.shape[0] >= ops.TILE_ROWS and n % 8 == 0 and ops.tile_linear_ok(x, w):
         return ops.tile_linear(x, w, gelu_n=n)
+    if n % 8 == 0 and ops.block_linear_ok(x, w):
+        return ops.block_linear(x, w, gelu_n=n)
     y = F.linear(x, w)
     gelu_(y[:, :n])
     return y
@@ -225,6 +229,8 @@ def product_glu(x: torch.Tensor, w: torch.Tensor, limit: float, alpha: float = G
     """``clamped_glu(x @ w.T)``."""
     if x.shape[0] >= ops.TILE_ROWS and w.shape[0] % 16 == 0 and ops.tile_linear_ok(x, w):
         return ops.tile_linear(x, w, glu=(limit, alpha, shift))
+    if ops.block_linear_ok(x, w):
+        return ops.block_linear(x, w, glu=(limit, alpha, shift))
     return clamped_glu(F.linear(x, w), limit, alpha, shift)
 
 
