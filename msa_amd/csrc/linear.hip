@@ -192,12 +192,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void skinny_linear_kernel(
 // and 5.8 / 6.3, 4096 x 1024 3.6 / 4.3 and 3.9 / 4.3; 2560 x 2560 5.1 / 7.2 and 5.3 / 6.4, 2560 x 2048 4.7 / 5.9 and 4.5 / 5.4,
 // 9728 x 1024 7.4 / 8.4 and 6.3 / 6.7.
 constexpr int64_t kRingWeights = 5 << 20;
-// Rows of more than kMaxResidentK are read once per sixteen rows of weights: 24 to 31 a workgroup cost as much as 32, which this file's
-// kernel reads once (sixteen rows of activations: 6144 x 9728 28.5 us here and 31.8 in the ring, 7168 x 5632 19.9 and 21.4; eight 25.3
-// and 26.2; but 8192 x 9728 34.3 and 35.2, 5632 x 9728 in 352 workgroups 38.2 and 31.5).
-constexpr int kTwiceRows = 12, kTwiceFrom = 6144, kTwiceTo = 8192;
-bool takes_ring(int32_t M, int32_t N, int32_t K, bool norm, int32_t epilogue) {
-  if (epilogue != kEpiSiluMul && K > rows_ring::kMaxResidentK && M >= kTwiceRows && N >= kTwiceFrom && N < kTwiceTo) return false;
+bool takes_ring(int32_t N, int32_t K, bool norm) {
   return K > rows_ring::kMinK && rows_ring::busy_weights(N, K) >= kRingWeights && (!norm || K <= rows_ring::kMaxResidentK);
 }
 
@@ -331,13 +326,13 @@ __global__ __launch_bounds__(256) void skinny_tile_reduce_kernel(const float* __
 
 // The cut of the tiled form: up to 16 row groups per row block (fewer when the matrix has fewer than 256 groups), as
 // many K slices as keep the launch within one workgroup per compute unit (at most 16); used when it takes at least
-// 8 us less per compute unit than the plain form at ~34 GB/s (the second launch costs ~4 us), and the rows are many or the matrix is
-// long: up to eight rows of activations are cheaper to read again than a second launch (2560 x 9728: 12.1 us in the form of
-// rows_ring.h with one row, 13.1 with eight, 16.4 with sixteen; 14.8 to 15.2 in this one), but not for a few hundred rows of weights,
-// of which each workgroup there has four (1024 x 9728: 10.6 and 12.2 us with one and eight rows, 9.8 here; 512 x 8192 8.5 and 10.1, 7.5
-// and 7.7; 1024 x 6144 7.7 and 8.8, 8.5;
-// 2048 x 14336 15.8 and 16.9, 17.6).
-constexpr int kTileMinRows = 8, kTileLong = 7;
+// 8 us less per compute unit than the plain form at ~34 GB/s (the second launch costs ~4 us).  The form of rows_ring.h reads the
+// activations again once a workgroup, which is cheaper than a second launch up to fourteen of them (us there and here, nine / twelve /
+// sixteen rows: 2048 x 6144 9.4 / 9.7 / 10.4 and 11.6, 2560 x 8192 11.8 / 12.5 / 13.4 and 14.2, 4096 x 9728 17.4 / 17.9 / 19.4 and 22,
+// 2560 x 9728 14.3 / 15.1 / 16.4 and 15.8) and with more where this form saves no more than some 11 us by that measure, but not for a few
+// hundred rows of weights, of which each workgroup there has four (1024 x 9728 11.1 / 11.1 / 11.5 and 9.8 to 10.0).
+constexpr int kTileMinRows = 8, kRingRows = 14, kTileLong = 7;
+constexpr double kTileSaves = 8.0, kTileSavesOfRing = 11.5;
 struct TilePlan {
   int n_slices, gpw, row_blocks;
   bool use;
@@ -346,14 +341,15 @@ TilePlan plan_tile(int32_t M, int32_t N, int32_t K) {
   TilePlan t{0, 0, 0, false};
   const int groups = (N + 15) / 16;
   const int steps = K / 32;
-  if (K % 32 != 0 || groups > 256 || (M <= kTileMinRows && K <= (int64_t)kTileLong * N)) return t;
+  const bool is_long = K > (int64_t)kTileLong * N, ring = !is_long && takes_ring(N, K, false);
+  if (K % 32 != 0 || groups > 256 || (!is_long && M <= (ring ? kRingRows : kTileMinRows))) return t;
   t.gpw = std::min(kMaxWaves, (groups + 15) / 16);
   t.row_blocks = (groups + t.gpw - 1) / t.gpw;
   t.n_slices = std::min(std::min(kTileMaxSlices, steps), 256 / std::max(1, t.row_blocks));
   if (t.n_slices < 2) return t;
   const double plain_bytes = (16.0 + 16.0) * K * 2;                             // one row group + all of x
   const double tiled_bytes = (16.0 * t.gpw + 16.0) * ((double)K / t.n_slices) * 2;
-  t.use = (plain_bytes - tiled_bytes) / 34e3 > 8.0;                             // bytes / (34 GB/s) in us
+  t.use = (plain_bytes - tiled_bytes) / 34e3 > (ring ? kTileSavesOfRing : kTileSaves);      // bytes / (34 GB/s) in us
   return t;
 }
 
@@ -394,7 +390,7 @@ extern "C" int msa_skinny_linear(const void* x, const void* w, const void* resid
   MSA_REQUIRE(norm_w == nullptr || eps > 0.f, "msa_skinny_linear: folded RMSNorm needs eps > 0");
   hipStream_t st = as_stream(stream);
 
-  if (takes_ring(M, N, K, norm_w != nullptr, epilogue)) {
+  if (takes_ring(N, K, norm_w != nullptr)) {
     switch (epilogue) {
       case kEpiPlain: return launch_ring<kEpiPlain>(x, w, residual, norm_w, eps, y, M, N, K, st);
       case kEpiResidual: return launch_ring<kEpiResidual>(x, w, residual, norm_w, eps, y, M, N, K, st);

@@ -6,8 +6,9 @@
 // wavefronts; a wavefront requests a unit of the 16 rows as two direct-to-LDS loads of eight whole lines each into a ring of
 // two slots of its own, so no wavefront waits for another's data, and the next unit is always in flight.  The 16-byte pieces of a
 // line are stored XORed with the row, which spreads the operand reads over the banks.  The 16 activation rows are one operand of
-// the 16x16x32 MFMA and stay in registers (up to K = 5120; longer rows are read again unit by unit); the wavefronts' partial
-// sums meet in LDS behind one barrier per 16 rows and are added in a fixed order.
+// the 16x16x32 MFMA and stay in registers up to K = 5120; longer rows pass the ring beside the weights, as whole lines.  The
+// wavefronts' partial sums meet in LDS behind one barrier per 16 rows (two for long rows, whose ring leaves no room to take planes
+// in turn) and are added in a fixed order.
 //
 // What bounds it is HBM where a workgroup has several rounds, and the launch, the first loads' latency and the activations (every
 // workgroup reads all of them from its L2) where it has one.
@@ -17,9 +18,11 @@
 // need no registers for what is in flight.  Measured in graphs over operands larger than the caches, launches included, against
 // the register forms before, us with 1 / 16 rows: 151936 x 2560 fp32 out 120 / 131 against 154 / 177 (6.5 / 5.9 TB/s); 151936 x
 // 1024 48 / 56 against 74 / 77; 19456 x 2560 gated units 17.6 / 18.9 against 23.8 / 26.5; 14944 x 2560 with convolution 15.3 /
-// 18.0 against 20.5 / 25.8; 2560 x 4096 6.5 / 8.0 against 7.3 / 9.6; 2560 x 9728 12.1 / 16.2 against 12.9 / 18.3; 4096 x 1024 4.0 /
-// 4.3 against 4.1 / 4.7.  A third slot changes nothing, except with a folded norm, whose arithmetic it hides (6144 x 2560: 9.3 /
-// 10.3 against 9.9 / 11.0 with two); an item of the loop must not wait for its own output's store or for what the epilogue reads.
+// 18.0 against 20.5 / 25.8; 2560 x 4096 6.5 / 8.0 against 7.3 / 9.6; 4096 x 1024 4.0 / 4.3 against 4.1 / 4.7.  A
+// third slot changes nothing, except with a folded norm, whose arithmetic it hides (6144 x 2560: 9.3 / 10.3 against 9.9 / 11.0 with
+// two).  Long rows of activations held the weights up when they were loaded as the operand wants them (us with 1 / 4 / 16 rows, then and
+// through the ring: 2560 x 9728 12.4 / 13.9 / 18.4 and 12.5 / 13.9 / 16.5, 5120 x 8192 19.9 / 20.7 / 27.2 and 20.3 / 20.3 / 21.9,
+// 1024 x 9728 10.8 / 11.1 / 15.0 and 10.9 / 10.9 / 11.3; three or four slots of weights instead were 5 to 20 % slower).  An item of the loop must not wait for its own output's store or for what the epilogue reads.
 #pragma once
 
 #include "common.h"
@@ -48,11 +51,15 @@ constexpr int kFar = 0x7ff00000;                   // past every extent, whateve
 enum { kPlain, kNormed, kPost };
 constexpr int kMaxPost = 3;                        // units per wavefront that the residual step takes: what its registers hold
 constexpr int slots(int pro) { return pro ? 3 : 2; }              // of a wavefront's ring
-constexpr int lds_bytes(int pro) {
-  return 2 * kWaves * kPlane * 4 + kWaves * slots(pro) * kUnitSlab + (pro ? kWaves * 16 * 4 + kWaves * 1024 : 0);
+// Rows too long for the registers (nu = 0): the activations' unit lies behind the weights' in its slot, and there is room for one plane
+// of partial sums instead of two in turn.
+constexpr int planes(int nu) { return nu == 0 ? 1 : 2; }
+constexpr int slab(int nu) { return nu == 0 ? 2 * kUnitSlab : kUnitSlab; }
+constexpr int lds_bytes(int pro, int nu) {
+  return planes(nu) * kWaves * kPlane * 4 + kWaves * slots(pro) * slab(nu) + (pro ? kWaves * 16 * 4 + kWaves * 1024 : 0);
 }
 static_assert(kMaxPost * 2 * kUnitBytes <= 1024 && kMaxResident * kUnitBytes <= 1024, "one request for a wavefront's part of the norm's weights");
-static_assert(lds_bytes(kNormed) <= 160 * 1024);
+static_assert(lds_bytes(kNormed, 1) <= 160 * 1024 && lds_bytes(kPlain, 0) <= 160 * 1024);
 constexpr int kNonTemporal = 2;                    // a step reads a weight once
 
 // vmcnt(n), the other counters not waited for
@@ -88,12 +95,12 @@ struct Args {
 template <class Epi, int NU, int kPro>
 __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename Epi::Args s) {
   constexpr bool kResident = NU > 0, kNorm = kPro == kNormed;
-  constexpr int kSlots = slots(kPro);
+  constexpr int kSlots = slots(kPro), kPlanes = planes(NU), kSlab = slab(NU);
   extern __shared__ __align__(16) char lds[];
   float(*part)[kWaves][kPlane] = reinterpret_cast<float(*)[kWaves][kPlane]>(lds);
-  float* row_ssq = reinterpret_cast<float*>(lds + 2 * kWaves * kPlane * 4 + kWaves * kSlots * kUnitSlab);
+  float* row_ssq = reinterpret_cast<float*>(lds + kPlanes * kWaves * kPlane * 4 + kWaves * kSlots * kSlab);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  char* ring = lds + 2 * kWaves * kPlane * 4 + wave * kSlots * kUnitSlab;
+  char* ring = lds + kPlanes * kWaves * kPlane * 4 + wave * kSlots * kSlab;
   const int wg = blockIdx.x, n_l = lane & 15, g = lane >> 4;
   const bool second = wg >= a.wgs_a;
   const int i = second ? wg - a.wgs_a : wg, q = second ? a.qb : a.qa, rem = second ? a.rb : a.ra;
@@ -109,6 +116,10 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
   // ---- requests: unit u of the rows from `base` on, into the next slot
   const int l_row = lane >> 3, col = wave * kUnitBytes + ((lane & 7) ^ (l_row & 7)) * 16;
   const int off0 = l_row * row_bytes + col, off1 = off0 + 8 * row_bytes;
+  const int64_t xs = second ? a.xbs : a.xs;
+  const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(second ? a.x_b : a.x), 0,
+                                                                        (int)((a.M - 1) * xs + row_bytes), 0x00020000);
+  const int xoff0 = l_row * (int)xs + col, xoff1 = xoff0 + 8 * (int)xs;      // of the activations, likewise
   int req_item = 0, slot_in = 0;
   __amdgpu_buffer_rsrc_t rs;
   auto point = [&]() {
@@ -119,20 +130,23 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
   };
   auto request = [&](int u) {
     const int so = u * (kUnitBytes * kWaves);
-    char* dst = ring + slot_in * kUnitSlab;
-    int v0 = off0, v1 = off1;
+    char* dst = ring + slot_in * kSlab;
+    int v0 = off0, v1 = off1, x0 = xoff0, x1 = xoff1;
     if (so + kUnitBytes * kWaves > row_bytes) {    // a row's last units can leave it
       const bool in = col + so < row_bytes;
       v0 = in ? off0 : kFar;
       v1 = in ? off1 : kFar;
+      x0 = in ? xoff0 : kFar;
+      x1 = in ? xoff1 : kFar;
     }
     MSA_LOAD_TO_LDS(rs, dst, v0, so, kNonTemporal);
     MSA_LOAD_TO_LDS(rs, dst + kUnitSlab / 2, v1, so, kNonTemporal);
+    if constexpr (!kResident) {
+      MSA_LOAD_TO_LDS(rs_x, dst + kUnitSlab, x0, so, 0);
+      MSA_LOAD_TO_LDS(rs_x, dst + kUnitSlab * 3 / 2, x1, so, 0);
+    }
     slot_in = slot_in + 1 == kSlots ? 0 : slot_in + 1;
   };
-  const int64_t xs = second ? a.xbs : a.xs;
-  const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(second ? a.x_b : a.x), 0,
-                                                                        (int)((a.M - 1) * xs + row_bytes), 0x00020000);
   const int x_col = wave * kUnitBytes + g * 16;
   auto load_x = [&](u32x4_t (&x)[2], int u) {
 #pragma unroll
@@ -143,9 +157,13 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
   };
   const int rd0 = n_l * kUnitBytes + ((g ^ (n_l & 7)) * 16), rd1 = n_l * kUnitBytes + (((g + 4) ^ (n_l & 7)) * 16);
   int slot_out = 0;
-  auto multiply = [&](const u32x4_t (&x)[2], floatx4_t acc) {
-    const char* src = ring + slot_out * kUnitSlab;
+  auto multiply = [&](u32x4_t (&x)[2], floatx4_t acc) {
+    const char* src = ring + slot_out * kSlab;
     const u32x4_t w0 = *reinterpret_cast<const u32x4_t*>(src + rd0), w1 = *reinterpret_cast<const u32x4_t*>(src + rd1);
+    if constexpr (!kResident) {
+      x[0] = *reinterpret_cast<const u32x4_t*>(src + kUnitSlab + rd0);
+      x[1] = *reinterpret_cast<const u32x4_t*>(src + kUnitSlab + rd1);
+    }
     slot_out = slot_out + 1 == kSlots ? 0 : slot_out + 1;
     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[0]), __builtin_bit_cast(bf16x8_t, w0), acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[1]), __builtin_bit_cast(bf16x8_t, w1), acc, 0, 0, 0);
@@ -164,7 +182,7 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
   }
   // The norm's weights, alike for all rows, through LDS (in registers, five units of them spill: 2560 x 5120 with one row took 13.9
   // us instead of 8.8)
-  char* norm_lds = lds + lds_bytes(kPro) - (kWaves - wave) * 1024;
+  char* norm_lds = lds + lds_bytes(kPro, NU) - (kWaves - wave) * 1024;
   if constexpr (kNorm) {
     const __amdgpu_buffer_rsrc_t rs_g = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.norm_w), 0, row_bytes, 0x00020000);
     MSA_LOAD_TO_LDS(rs_g, norm_lds, (lane >> 3) * (kUnitBytes * kWaves) + wave * kUnitBytes + (lane & 7) * 16, 0, 0);
@@ -195,7 +213,6 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
       point();
     }
     request(i % kX);
-    if constexpr (!kResident) load_x(xf[i], i);              // (in the loop's order: it counts what is outstanding)
   }
   __builtin_amdgcn_sched_barrier(0);                         // (nothing is computed before everything is requested)
   // What a norm reads of LDS it reads by hand: the compiler would wait for the ring in front of it, and nor does it wait for the
@@ -291,7 +308,6 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
         point();
       }
       request(next);
-      if constexpr (!kResident) load_x(x, next);
     };
     if constexpr (kResident) {
 #pragma unroll
@@ -304,7 +320,7 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
       }
     }
     // acc[e] is (m = 4 g + e, n_l) over this wavefront's share of K
-    float(*buf)[kPlane] = part[item & 1];
+    float(*buf)[kPlane] = part[kPlanes == 2 ? item & 1 : 0];
 #pragma unroll
     for (int e = 0; e < 4; ++e) buf[wave][e * 64 + lane] = acc[e];
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -319,6 +335,7 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
       }
       v *= inv;
     }
+    if (kPlanes == 1 && item + 1 < items) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");    // (the block is read by all)
     epi.apply(s, m, n, v, mine, second, item);
   }
   __builtin_amdgcn_s_waitcnt(wait_vm(0));                    // nothing may still be writing LDS when the workgroup ends
@@ -347,8 +364,8 @@ static inline int plan(Args& a, int granule) {
 template <class Epi, int NU, int kPro>
 int start(const Args& a, const typename Epi::Args& s, int wgs, hipStream_t st) {
   static std::atomic<int> lds_limit_raised{0};
-  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(rows_ring_kernel<Epi, NU, kPro>), lds_bytes(kPro)));
-  rows_ring_kernel<Epi, NU, kPro><<<wgs, kWaves * 64, lds_bytes(kPro), st>>>(a, s);
+  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(rows_ring_kernel<Epi, NU, kPro>), lds_bytes(kPro, NU)));
+  rows_ring_kernel<Epi, NU, kPro><<<wgs, kWaves * 64, lds_bytes(kPro, NU), st>>>(a, s);
   MSA_LAUNCH_CHECK();
   return MSA_OK;
 }
