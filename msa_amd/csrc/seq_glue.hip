@@ -29,9 +29,14 @@ struct ResNorm {
   int32_t W, rows_per_wg;
 };
 
+// Bound by memory; a thread's rows follow one another, so a launch wants as few of them a thread as it can have: one where rows do not
+// look at the one in front (which a workgroup's first row computes again), else one to four by the launch's size.  us without / with the
+// shift, then eight rows and as it is here: 300 x 1024 9.2 / 11.6 and 4.3 / 6.0, 1000 x 1024 12.5 / 15.2 and 6.5 / 8.4, 8192 x 1024 28.8 /
+// 37.9 and 27.2 / 35.0 (4.2 TB/s), 600 x 2560 13.3 / 17.3 and 8.1 / 10.7, 2500 x 2560 26.9 / 35.3 and 23.0 / 29.3, 6001 x 2560 56 / 72 and
+// 47 / 61.
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void residual_norm_kernel(ResNorm a, msa_seq_batch b) {
-  const int col = (blockIdx.y * 256 + threadIdx.x) * VEC;
+  const int col = (blockIdx.y * blockDim.x + threadIdx.x) * VEC;
   if (col >= a.W) return;
   const int t0 = blockIdx.x * a.rows_per_wg, t1 = min(b.rows, t0 + a.rows_per_wg);
   float gb[VEC] = {}, nw[VEC] = {}, nb[VEC] = {}, sh[VEC] = {};
@@ -424,18 +429,25 @@ static int residual_norm(ResNorm a, int32_t dtype, const msa_seq_batch* batch, v
   MSA_REQUIRE(!a.norm.w || a.h || a.shift, "%s: norm without an output", who);
   MSA_REQUIRE(!a.shift || (a.norm.w && a.prev && a.h_shift), "%s: shift needs norm, prev and h_shift", who);
   if (!a.norm.w) a.h = nullptr;
-  a.rows_per_wg = batch->rows <= 256 ? 1 : 8;
-  const bool vec = vec_ok(4, {a.x_in, a.table, a.y, a.gate, a.gate_bias, a.x_out, a.norm.w, a.norm.b, a.h, a.shift, a.prev, a.h_shift},
-                          {a.W, a.y_stride, a.gate_stride});
-  const int V = vec ? 4 : 1;
-  const dim3 grid((batch->rows + a.rows_per_wg - 1) / a.rows_per_wg, (a.W + 256 * V - 1) / (256 * V));
+  // With the shift (us with one / two / four rows, and four of eight columns a thread): 1000 x 1024 8.4 / 9.1 / 10.6 and 11.3, 2048 x 1024
+  // 12.4 / 11.7 / 12.9 and 14.1, 1200 x 2560 17.5 / 17.5 / 17.4 and 17.4, 4096 x 1024 23.0 / 22.1 / 20.5 and 20.3, 2500 x 2560 32.9 / 31.8 /
+  // 34.0 and 29.3, 8192 x 1024 40.9 / 37.6 / 38.3 and 35.0.
+  constexpr int64_t kOneRow = 3 << 19, kTwoRows = 3 << 20;
+  const int64_t elements = (int64_t)batch->rows * a.W;
+  a.rows_per_wg = !a.shift || elements <= kOneRow ? 1 : elements <= kTwoRows ? 2 : 4;
+  auto aligned = [&](int n) {
+    return vec_ok(n, {a.x_in, a.table, a.y, a.gate, a.gate_bias, a.x_out, a.norm.w, a.norm.b, a.h, a.shift, a.prev, a.h_shift}, {a.W, a.y_stride, a.gate_stride});
+  };
+  const int V = dtype == MSA_BF16 && a.rows_per_wg == 4 && aligned(8) ? 8 : aligned(4) ? 4 : 1, threads = V == 8 ? 128 : 256;
+  const dim3 grid((batch->rows + a.rows_per_wg - 1) / a.rows_per_wg, (a.W + threads * V - 1) / (threads * V));
   hipStream_t st = as_stream(stream);
   if (dtype == MSA_BF16) {
-    if (vec) residual_norm_kernel<bf16_t, 4><<<grid, 256, 0, st>>>(a, *batch);
-    else residual_norm_kernel<bf16_t, 1><<<grid, 256, 0, st>>>(a, *batch);
+    if (V == 8) residual_norm_kernel<bf16_t, 8><<<grid, threads, 0, st>>>(a, *batch);
+    else if (V == 4) residual_norm_kernel<bf16_t, 4><<<grid, threads, 0, st>>>(a, *batch);
+    else residual_norm_kernel<bf16_t, 1><<<grid, threads, 0, st>>>(a, *batch);
   } else {
-    if (vec) residual_norm_kernel<float, 4><<<grid, 256, 0, st>>>(a, *batch);
-    else residual_norm_kernel<float, 1><<<grid, 256, 0, st>>>(a, *batch);
+    if (V == 4) residual_norm_kernel<float, 4><<<grid, threads, 0, st>>>(a, *batch);
+    else residual_norm_kernel<float, 1><<<grid, threads, 0, st>>>(a, *batch);
   }
   MSA_LAUNCH_CHECK();
   return MSA_OK;
