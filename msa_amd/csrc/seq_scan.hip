@@ -44,17 +44,18 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(const T* __restrict__ in
     }
 }
 
-// The same for 2 <= K <= 5 and aligned rows: a thread owns eight channels and slides its window of K - 1 inputs along.
+// The same for 2 <= K <= 5 and aligned rows: a thread owns eight channels and slides its window of K - 1 inputs along.  The workgroup of
+// a sequence's first rows replaces the kept inputs, so no other may look at them: rows_per_wg >= K - 1.
 template <typename T, int K>
 __global__ __launch_bounds__(256) void conv_silu_vec_kernel(const T* __restrict__ in, int64_t in_stride, const float* __restrict__ taps,
                                                             const float* __restrict__ bias, int32_t C, float* __restrict__ state,
-                                                            T* __restrict__ out, int64_t out_stride, msa_seq_batch b) {
+                                                            T* __restrict__ out, int64_t out_stride, int32_t rows_per_wg, msa_seq_batch b) {
   const int c = (blockIdx.x * 256 + threadIdx.x) * 8;
   const int s = blockIdx.z;
   const int lo = b.cu[s], n = b.cu[s + 1] - lo;
-  const int t0 = blockIdx.y * kConvRows;
+  const int t0 = blockIdx.y * rows_per_wg;
   if (c >= C || t0 >= n) return;
-  const int t1 = min(n, t0 + kConvRows);
+  const int t1 = min(n, t0 + rows_per_wg);
   float* keep = state + (int64_t)b.slot[s] * (K - 1) * C + c;
   const T* src = in + (int64_t)lo * in_stride + c;
   float tp[K][8], bs[8] = {}, win[K - 1][8];
@@ -99,11 +100,18 @@ int launch_conv(const T* in, int64_t in_stride, const float* taps, const float* 
                 int64_t out_stride, const msa_seq_batch& b, hipStream_t st) {
   const int row_blocks = (b.max_rows + kConvRows - 1) / kConvRows;
   if (K >= 2 && K <= 5 && vec_ok(8, {in, bias, state, out}, {in_stride, out_stride, C})) {
-    const dim3 grid((C / 8 + 255) / 256, row_blocks, b.n_seq);
-    if (K == 2) conv_silu_vec_kernel<T, 2><<<grid, 256, 0, st>>>(in, in_stride, taps, bias, C, state, out, out_stride, b);
-    else if (K == 3) conv_silu_vec_kernel<T, 3><<<grid, 256, 0, st>>>(in, in_stride, taps, bias, C, state, out, out_stride, b);
-    else if (K == 4) conv_silu_vec_kernel<T, 4><<<grid, 256, 0, st>>>(in, in_stride, taps, bias, C, state, out, out_stride, b);
-    else conv_silu_vec_kernel<T, 5><<<grid, 256, 0, st>>>(in, in_stride, taps, bias, C, state, out, out_stride, b);
+    // Rows a thread: few where that is what fills the chip, many where the taps and the window before the first row are worth sharing.
+    // bf16, four taps, us with 4 / 8 / 12 / 16 / 32: 300 x 4096 6.2 / 6.8 / 7.5 / 8.4 / 12.1, 700 x 4096 8.1 / 7.9 / 8.9 / 9.9 / 14.3, 700 x
+    // 8192 10.7 / 10.7 / 9.7 / 10.8 / 14.9, 1500 x 8192 18.1 / 15.5 / 15.2 / 16.5 / 18.7, 3000 x 8192 35.3 / 30.7 / 28.0 / 25.8 / 28.1, 6001 x
+    // 8192 65.1 / 52.0 / 48.9 / 49.4 / 45.5 (4.3 TB/s).
+    const int64_t elements = (int64_t)b.rows * C;
+    int rows_per_wg = elements <= 2 << 20 ? 4 : elements <= 4 << 20 ? 8 : elements <= 16 << 20 ? 12 : elements <= 32 << 20 ? 16 : 32;
+    if (b.max_rows > 4 * 65535) rows_per_wg = std::max(rows_per_wg, kConvRows);      // (the grid's limit)
+    const dim3 grid((C / 8 + 255) / 256, (b.max_rows + rows_per_wg - 1) / rows_per_wg, b.n_seq);
+    if (K == 2) conv_silu_vec_kernel<T, 2><<<grid, 256, 0, st>>>(in, in_stride, taps, bias, C, state, out, out_stride, rows_per_wg, b);
+    else if (K == 3) conv_silu_vec_kernel<T, 3><<<grid, 256, 0, st>>>(in, in_stride, taps, bias, C, state, out, out_stride, rows_per_wg, b);
+    else if (K == 4) conv_silu_vec_kernel<T, 4><<<grid, 256, 0, st>>>(in, in_stride, taps, bias, C, state, out, out_stride, rows_per_wg, b);
+    else conv_silu_vec_kernel<T, 5><<<grid, 256, 0, st>>>(in, in_stride, taps, bias, C, state, out, out_stride, rows_per_wg, b);
   } else {
     conv_silu_kernel<T><<<dim3((C + 255) / 256, row_blocks, b.n_seq), 256, 0, st>>>(in, in_stride, taps, bias, C, K, state, out, out_stride, b);
   }
