@@ -331,25 +331,28 @@ __global__ __launch_bounds__(256) void skinny_tile_reduce_kernel(const float* __
 // sixteen rows: 2048 x 6144 9.4 / 9.7 / 10.4 and 11.6, 2560 x 8192 11.8 / 12.5 / 13.4 and 14.2, 4096 x 9728 17.4 / 17.9 / 19.4 and 22,
 // 2560 x 9728 14.3 / 15.1 / 16.4 and 15.8) and with more where this form saves no more than some 11 us by that measure, but not for a few
 // hundred rows of weights, of which each workgroup there has four (1024 x 9728 11.1 / 11.1 / 11.5 and 9.8 to 10.0).
+// Scratch is asked for wherever the cut form could run, the calls that rows_ring.h takes included.
 constexpr int kTileMinRows = 8, kRingRows = 14, kTileLong = 7;
 constexpr double kTileSaves = 8.0, kTileSavesOfRing = 11.5;
 struct TilePlan {
   int n_slices, gpw, row_blocks;
-  bool use;
+  bool use, ring;                        // worth it beside the plain form, but not beside rows_ring.h
 };
 TilePlan plan_tile(int32_t M, int32_t N, int32_t K) {
-  TilePlan t{0, 0, 0, false};
+  TilePlan t{0, 0, 0, false, false};
   const int groups = (N + 15) / 16;
   const int steps = K / 32;
-  const bool is_long = K > (int64_t)kTileLong * N, ring = !is_long && takes_ring(N, K, false);
-  if (K % 32 != 0 || groups > 256 || (!is_long && M <= (ring ? kRingRows : kTileMinRows))) return t;
+  const bool is_long = K > (int64_t)kTileLong * N;
+  if (K % 32 != 0 || groups > 256 || (!is_long && M <= kTileMinRows)) return t;
   t.gpw = std::min(kMaxWaves, (groups + 15) / 16);
   t.row_blocks = (groups + t.gpw - 1) / t.gpw;
   t.n_slices = std::min(std::min(kTileMaxSlices, steps), 256 / std::max(1, t.row_blocks));
   if (t.n_slices < 2) return t;
   const double plain_bytes = (16.0 + 16.0) * K * 2;                             // one row group + all of x
   const double tiled_bytes = (16.0 * t.gpw + 16.0) * ((double)K / t.n_slices) * 2;
-  t.use = (plain_bytes - tiled_bytes) / 34e3 > (ring ? kTileSavesOfRing : kTileSaves);      // bytes / (34 GB/s) in us
+  const double saves = (plain_bytes - tiled_bytes) / 34e3;                      // bytes / (34 GB/s) in us
+  t.use = saves > kTileSaves;
+  t.ring = !is_long && takes_ring(N, K, false) && (M <= kRingRows || saves <= kTileSavesOfRing);
   return t;
 }
 
@@ -447,8 +450,8 @@ extern "C" int msa_skinny_linear_ws(const void* x, const void* w, const void* re
                     (epilogue == kEpiResidual) == (residual != nullptr) && (int64_t)M * K * 2 < ((int64_t)1 << 31) &&
                     (int64_t)32 * K * 2 < ((int64_t)1 << 31) &&
                     (((uintptr_t)x | (uintptr_t)w | (uintptr_t)workspace) & 15) == 0;
-  const TilePlan t = fits ? plan_tile(M, N, K) : TilePlan{0, 0, 0, false};
-  if (!fits || !t.use || workspace == nullptr || workspace_bytes < tile_workspace_bytes(t, N))
+  const TilePlan t = fits ? plan_tile(M, N, K) : TilePlan{0, 0, 0, false, false};
+  if (!fits || !t.use || t.ring || workspace == nullptr || workspace_bytes < tile_workspace_bytes(t, N))
     return msa_skinny_linear(x, w, residual, norm_w, eps, epilogue, dtype, M, N, K, y, stream);   // it reports bad arguments
   hipStream_t st = as_stream(stream);
   const int groups = (N + 15) / 16;
