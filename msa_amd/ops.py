@@ -23,6 +23,12 @@ def _stream(stream: Optional[torch.cuda.Stream] = None) -> int:
     return stream.cuda_stream if stream is not None else torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
+def scratch(need: int, device) -> Optional[torch.Tensor]:
+    """Scratch of one call, from the allocator each time: calls on other streams and threads have their own, and inside a capture it
+    belongs to the graph, whose replays then share it with nothing."""
+    return torch.empty(need, dtype=torch.uint8, device=device) if need else None
+
+
 def _need_cuda(*ts):
     for t in ts:
         if t is not None and not t.is_cuda:
@@ -118,7 +124,6 @@ class Bank:
         self.max_doc_chunks = int((self.off_host[1:] - self.off_host[:-1]).max())
         self.n_layers, self.Hkv, self.D, self.dtype = n_layers, Hkv, D, dtype
         self._keep = {}
-        self._ws: Optional[torch.Tensor] = None
         h = C.c_void_p()
         check(lib.msa_bank_create(C.byref(h), n_layers, self.C, Hkv, D, dtype_code(dtype), ptr(self.off_host),
                                   ptr(self.gid_host), self.n_docs), "msa_bank_create")
@@ -144,9 +149,7 @@ class Bank:
         lib = _lib.load()
         need = (lib.msa_route_workspace_bytes(B, S, Hq, self.Hkv, self.D, self.C, self.n_docs, topk) if chunk_plane
                 else lib.msa_route_topk_workspace_bytes(B, S, Hq, self.Hkv, self.D, self.n_docs, topk))
-        if self._ws is None or self._ws.numel() < need or self._ws.device != torch.device(device):
-            self._ws = torch.empty(need, dtype=torch.uint8, device=device)
-        return self._ws
+        return scratch(need, device)
 
     def close(self):
         if getattr(self, "handle", None):
@@ -335,7 +338,6 @@ def cache_append_rows(k_new, v_new, cu_new, max_new: int, kcache, vcache, kv_len
                                             _stream()), "msa_cache_append_rows")
 
 
-_attn_ws = {}
 FLASH_MIN_ROWS = 16     # bf16 query blocks at least this long go to the MFMA flash kernel
 
 
@@ -358,13 +360,11 @@ def sparse_attn(q, k, v, kv_off, kv_len, max_kv: int, cu_q=None, max_sq: int = 1
                                       sc, int(causal), ptr(out), int(max_sq), _stream()), "msa_flash_attn")
         return out
     need = lib.msa_attn_workspace_bytes(total_q, Hq, Hkv, D, max_kv)
-    ws = _attn_ws.get(q.device)
-    if ws is None or ws.numel() < need:
-        ws = _attn_ws[q.device] = torch.empty(need, dtype=torch.uint8, device=q.device)
+    ws = scratch(need, q.device)
     out = torch.empty_like(q)
     check(lib.msa_sparse_attn(ptr(q), ptr(cu_q), ptr(k), ptr(v), ptr(kv_off), ptr(kv_len), B, total_q, max_sq, max_kv,
                               Hq, Hkv, D, dtype_code(q.dtype), D ** -0.5 if scale is None else scale, int(causal),
-                              ptr(out), ptr(ws), ws.numel(), _stream()), "msa_sparse_attn")
+                              ptr(out), ptr(ws), need, _stream()), "msa_sparse_attn")
     return out
 
 
@@ -419,17 +419,11 @@ def qkv_proj(x: torch.Tensor, w: torch.Tensor, Hq: int, Hkv: int, positions: tor
     k = torch.empty((T, Hkv, D), dtype=x.dtype, device=dev)
     v = torch.empty((T, Hkv, D), dtype=x.dtype, device=dev)
     r = torch.empty((T, router_front + router_back, D), dtype=x.dtype, device=dev) if router_front + router_back else None
-    ws = _tile_workspace(T, K, heads * D, dev)
+    ws = scratch(_lib.load().msa_tile_workspace_bytes(T, K, heads * D), dev)
     check(_lib.load().msa_qkv_proj_ws(ptr(x), T, K, ptr(w), Hq, Hkv, router_front, router_back, ptr(positions), ptr(q_norm_w),
                                       ptr(k_norm_w), eps, ptr(rope[0]), ptr(rope[1]), rope[0].shape[0], ptr(q), ptr(k), ptr(v),
                                       ptr(r), ptr(ws), 0 if ws is None else ws.numel(), _stream()), "msa_qkv_proj")
     return q, k, v, r
-
-
-def _tile_workspace(T: int, K: int, N: int, device) -> Optional[torch.Tensor]:
-    """Partial tiles of one call (from the allocator each time: calls on other streams have their own)."""
-    need = _lib.load().msa_tile_workspace_bytes(T, K, N)
-    return torch.empty(need, dtype=torch.uint8, device=device) if need else None
 
 
 def tile_linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, add: bool = False,
@@ -453,7 +447,7 @@ def tile_linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
         raise ValueError(f"tile_linear: out must be bf16 [{T}, {width}] on the device with unit column stride")
     if not T:
         return out
-    ws = _tile_workspace(T, K, N, x.device)
+    ws = scratch(_lib.load().msa_tile_workspace_bytes(T, K, N), x.device)
     mode = (_lib.TILE_ADD if add else _lib.TILE_SILU_MUL if silu_mul else _lib.TILE_GLU if glu is not None
             else _lib.TILE_GELU if gelu_n else _lib.TILE_STORE)
     end = _lib.TileEnd(mode, gelu_n, *(glu or (0.0, 0.0, 0.0)))
@@ -608,13 +602,11 @@ def decode_attn_fused(qkv: torch.Tensor, Hq: int, Hkv: int, D: int, positions: t
     Lcap = kcache.shape[1]
     lib = _lib.load()
     need = lib.msa_attn_workspace_bytes(B, Hq, Hkv, D, Lcap)
-    ws = _attn_ws.get(qkv.device)
-    if ws is None or ws.numel() < need:
-        ws = _attn_ws[qkv.device] = torch.empty(need, dtype=torch.uint8, device=qkv.device)
+    ws = scratch(need, qkv.device)
     out = torch.empty((B, Hq, D), dtype=qkv.dtype, device=qkv.device)
     check(lib.msa_decode_attn_fused(ptr(qkv), W, ptr(positions), ptr(q_norm_w), ptr(k_norm_w), eps, ptr(rope[0]),
                                     ptr(rope[1]), rope[0].shape[0], B, Hq, Hkv, D, ptr(kcache), ptr(vcache), Lcap,
-                                    ptr(kv_len), D ** -0.5 if scale is None else scale, ptr(out), ptr(ws), ws.numel(),
+                                    ptr(kv_len), D ** -0.5 if scale is None else scale, ptr(out), ptr(ws), need,
                                     _stream()), "msa_decode_attn_fused")
     return out
 
@@ -643,7 +635,6 @@ def greedy_sample(logits: torch.Tensor, tok: torch.Tensor, pos: Optional[torch.T
 
 
 SKINNY_MAX_ROWS = 16
-_linear_ws = {}
 
 
 def interleave_gate_up(gate_w: torch.Tensor, up_w: torch.Tensor) -> torch.Tensor:
@@ -676,11 +667,8 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Ten
         raise ValueError("skinny_linear: norm_weight must be a contiguous [K] tensor of x's dtype")
     lib = _lib.load()
     need = lib.msa_skinny_linear_workspace_bytes(M, N, K)
-    ws = _linear_ws.get(x.device)
-    if need and (ws is None or ws.numel() < need):
-        ws = _linear_ws[x.device] = torch.empty(need, dtype=torch.uint8, device=x.device)
+    ws = scratch(need, x.device)
     check(lib.msa_skinny_linear_ws(ptr(x), ptr(w), ptr(residual) if residual is not None else None,
                                    ptr(norm_weight) if norm_weight is not None else None, float(eps), epi,
-                                   dtype_code(x.dtype), M, N, K, ptr(out), ptr(ws) if need else None,
-                                   ws.numel() if need else 0, _stream()), "msa_skinny_linear_ws")
+                                   dtype_code(x.dtype), M, N, K, ptr(out), ptr(ws), need, _stream()), "msa_skinny_linear_ws")
     return out

@@ -114,14 +114,6 @@ class DynTanhNorm:
 
 
 _NO_NORM = _lib.DynTanh(None, None, 0.0, 0)
-_scratch = {}
-
-
-def _workspace(device, need: int) -> torch.Tensor:
-    ws = _scratch.get(device)
-    if ws is None or ws.numel() < need:
-        ws = _scratch[device] = torch.empty(max(need, 1), dtype=torch.uint8, device=device)
-    return ws
 
 
 def residual_norm(x: torch.Tensor, batch: StepBatch, dtype: torch.dtype, y=None, gate=None, gate_bias=None,
@@ -289,8 +281,9 @@ def ssd(xbc, z, dt_raw, dt_bias, A_log, D, H: int, P: int, N: int, G: int, state
     args = [ptr(xbc), _rows(xbc), ptr(z), _rows(z), ptr(dt_raw), _rows(dt_raw), ptr(dt_bias), ptr(A_log), ptr(D),
             dtype_code(xbc.dtype), H, P, N, G, ptr(state), ptr(v), batch.ref]
     if chunked:
-        ws = _workspace(xbc.device, lib.msa_seq_ssd_chunked_workspace_bytes(batch.max_rows, batch.n_seq, H, P, N))
-        _check(lib.msa_seq_ssd_chunked(*args, ptr(ws), ws.numel(), _stream()), "msa_seq_ssd_chunked")
+        need = lib.msa_seq_ssd_chunked_workspace_bytes(batch.max_rows, batch.n_seq, H, P, N)
+        ws = ops.scratch(need, xbc.device)
+        _check(lib.msa_seq_ssd_chunked(*args, ptr(ws), need, _stream()), "msa_seq_ssd_chunked")
     else:
         _check(lib.msa_seq_ssd_scan(*args, _stream()), "msa_seq_ssd_scan")
     return v
@@ -334,8 +327,9 @@ def delta(qkv, a, b, gate, A_log, dt_bias, norm, eps: float, H: int, G: int, D: 
                        ptr(state), ptr(out), H, G, D, E, eps, 0)
     lib = _lib.load_seq()
     if chunked:
-        ws = _workspace(qkv.device, lib.msa_seq_delta_chunked_workspace_bytes(C.byref(c), batch.max_rows, batch.n_seq))
-        _check(lib.msa_seq_delta_chunked(C.byref(c), batch.ref, ptr(ws), ws.numel(), _stream()), "msa_seq_delta_chunked")
+        need = lib.msa_seq_delta_chunked_workspace_bytes(C.byref(c), batch.max_rows, batch.n_seq)
+        ws = ops.scratch(need, qkv.device)
+        _check(lib.msa_seq_delta_chunked(C.byref(c), batch.ref, ptr(ws), need, _stream()), "msa_seq_delta_chunked")
     else:
         _check(lib.msa_seq_delta_scan(C.byref(c), dtype_code(qkv.dtype), batch.ref, _stream()), "msa_seq_delta_scan")
     return out
@@ -392,9 +386,9 @@ def min_gru(zug: torch.Tensor, z_bias, u_bias, n: int, state, batch: StepBatch) 
     out = torch.empty((batch.rows, n), dtype=zug.dtype, device=zug.device)
     lib = _lib.load_seq()
     need = lib.msa_seq_min_gru_workspace_bytes(batch.rows, batch.n_seq, batch.max_rows, n)
-    ws = _workspace(zug.device, need) if need else None
+    ws = ops.scratch(need, zug.device)
     _check(lib.msa_seq_min_gru(ptr(zug), _rows(zug), ptr(z_bias), ptr(u_bias), dtype_code(zug.dtype), n, ptr(state), ptr(out),
-                               batch.ref, ptr(ws), ws.numel() if ws is not None else 0, _stream()), "msa_seq_min_gru")
+                               batch.ref, ptr(ws), need, _stream()), "msa_seq_min_gru")
     return out
 
 
@@ -430,9 +424,10 @@ def latent_attn(q: torch.Tensor, cache: torch.Tensor, sink: torch.Tensor, scale:
     lib = _lib.load_seq()
     if q.dtype == torch.bfloat16 and rank % 8 == 0 and rank <= 512 and T <= 65535:
         keys = batch.max_keys if max_keys is None else max_keys
-        ws = _workspace(q.device, lib.msa_seq_latent_decode_workspace_bytes(T, H, rank, keys))
+        need = lib.msa_seq_latent_decode_workspace_bytes(T, H, rank, keys)
+        ws = ops.scratch(need, q.device)
         _check(lib.msa_seq_latent_decode(ptr(q), ptr(cache), Lcap, ptr(sink), scale, dtype_code(q.dtype), H, rank, keys, ptr(ctx),
-                                         batch.ref, ptr(ws), ws.numel(), _stream()), "msa_seq_latent_decode")
+                                         batch.ref, ptr(ws), need, _stream()), "msa_seq_latent_decode")
     else:
         _check(lib.msa_seq_latent_attn(ptr(q), ptr(cache), Lcap, ptr(sink), scale, dtype_code(q.dtype), H, rank, ptr(ctx), batch.ref,
                                        _stream()), "msa_seq_latent_attn")
@@ -530,8 +525,8 @@ def kv_attn(q: torch.Tensor, k_cache, v_cache, scale: float, batch: StepBatch, c
         split = flash_ok(q.dtype, D, E, scale) and T <= 65535
     if split:
         need = lib.msa_seq_kv_decode_workspace_bytes(C.byref(c), T)
-        ws = _workspace(q.device, need) if need else None
-        _check(lib.msa_seq_kv_decode(C.byref(c), batch.ref, ptr(ws), ws.numel() if need else 0, _stream()), "msa_seq_kv_decode")
+        ws = ops.scratch(need, q.device)
+        _check(lib.msa_seq_kv_decode(C.byref(c), batch.ref, ptr(ws), need, _stream()), "msa_seq_kv_decode")
     else:
         _check(lib.msa_seq_kv_attn(C.byref(c), dtype_code(q.dtype), batch.ref, _stream()), "msa_seq_kv_attn")
     return out
