@@ -53,8 +53,6 @@ class MLP(nn.Module):
     def add_to(self, residual, x):
         """``residual += self(x)`` (bf16 / fp32 on the GPU); a block of bf16 tokens has the add in the end of the second product, where the
         sum is rounded once."""
-        if not ops.plain_module(self):
-            return residual.add_(self(x))
         act = self._activation(x)
         if ops.linear_ok(self.down_proj, act) and residual.is_contiguous() and residual.dtype == x.dtype and residual.shape == x.shape \
                 and residual.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and residual.requires_grad):
@@ -88,7 +86,7 @@ class MSADecoderLayer(nn.Module):
             h, _ = self.self_attn(ops.rmsnorm(hidden_states, n1.weight, n1.variance_epsilon), doc_ids, attention_mask,
                                   position_embeddings, past_key_value, position_ids=position_ids)
             x = ops.rmsnorm(h.contiguous(), n2.weight, n2.variance_epsilon, residual=hidden_states)
-            return self.mlp.add_to(hidden_states, x)
+            return self.mlp.add_to(hidden_states, x) if ops.plain_module(self.mlp, MLP) else hidden_states.add_(self.mlp(x))
         h, _ = self.self_attn(self.input_layernorm(hidden_states), doc_ids, attention_mask, position_embeddings,
                               past_key_value)
         hidden_states = hidden_states + h
@@ -122,7 +120,8 @@ class MSAModel(nn.Module):
 
     def forward(self, input_ids, attention_mask, position_ids, past_key_values, doc_ids, final_norm: bool = True):
         e = self.embed_tokens
-        if (type(e) is nn.Embedding and e.max_norm is None and ops.plain_module(e) and ops.embed_ok(e.weight, input_ids)):
+        if type(e) is nn.Embedding and e.max_norm is None and type(e.weight) is nn.Parameter and ops.embed_ok(e.weight, input_ids) \
+                and ops.plain_module(e, nn.Embedding):
             h = ops.embed_rows(e.weight, input_ids)
         else:
             h = e(input_ids)

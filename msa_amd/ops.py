@@ -11,6 +11,7 @@ from dataclasses import dataclass
 from typing import List, Optional, Sequence, Tuple
 
 import torch
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import _lib
 from ._lib import MODE_COSINE, MODE_SCALED_DOT, check, dtype_code, ptr
@@ -506,9 +507,12 @@ def block_linear(x: torch.Tensor, w: torch.Tensor, glu: Optional[Tuple[float, fl
     return out
 
 
-def plain_module(module: torch.nn.Module) -> bool:
-    """Whether nothing but the module's own ``forward`` runs when it is called."""
-    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+def plain_module(module: torch.nn.Module, base: type) -> bool:
+    """Whether ``base``'s own ``forward`` and nothing else runs when the module is called: no forward of a subclass or of the instance, and
+    no hooks, the module's or global ones."""
+    return (getattr(type(module), "forward", None) is base.forward and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+            and not _has_any_global_hook())
 
 
 def embed_ok(table: torch.Tensor, tokens: torch.Tensor) -> bool:
@@ -530,8 +534,8 @@ def embed_rows(table: torch.Tensor, tokens: torch.Tensor, f32: bool = False, wra
 
 
 def linear_ok(module: torch.nn.Module, x: torch.Tensor) -> bool:
-    return (type(module) is torch.nn.Linear and module.bias is None and x.is_contiguous() and tile_linear_ok(x, module.weight)
-            and plain_module(module))
+    return (type(module) is torch.nn.Linear and module.bias is None and x.is_contiguous() and type(module.weight) is torch.nn.Parameter
+            and tile_linear_ok(x, module.weight) and plain_module(module, torch.nn.Linear))
 
 
 def linear(module: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:

@@ -445,8 +445,8 @@ def takes_flash_rows(q, k, v, H: int, G: int, D: int, E: int, chunk: int, batch:
     """Whether the attention model's prefill kernels take the call: bf16, heads of 128, dense keys and values, and no position behind the
     first chunk (there it hides nothing).  Long portions gain (us, the general kernel and those, 16 heads of their own keys: 8192 rows 343 and
     256, 2048 49 and 41, 2048 behind 4000 keys 132 and 111, 1000 27.3 and 26.0); shorter ones wait for the host, which has more to do."""
-    return (batch.max_rows >= FLASH_ROWS and q.dtype == k.dtype == v.dtype == torch.bfloat16 and D == E == 128 and H // G in (1, 2, 4, 8) and (not chunk or batch.max_keys <= chunk)
-            and _rows(k) == _rows(v) == G * D and _rows(q) % 8 == 0 and batch.max_rows * _rows(q) < 1 << 30
+    return (batch.max_rows >= FLASH_ROWS and q.dtype == k.dtype == v.dtype == torch.bfloat16 and D == E == 128 and H // G in (1, 2, 4, 8)
+            and (not chunk or batch.max_keys <= chunk) and _rows(k) == _rows(v) == G * D and _rows(q) % 8 == 0 and batch.max_rows * _rows(q) < 1 << 30
             and not (q.data_ptr() | k.data_ptr() | v.data_ptr()) % 16)
 
 

@@ -16,4 +16,95 @@ def test_prefill_attention_of_other_types(anywhere):
     ok = lambda q, k, v: seq_ops.takes_flash_rows(q, k, v, 4, 4, 128, 128, 0, batch)
     assert ok(q.bfloat16(), k.bfloat16(), k.bfloat16())
     for a, b, c in ((q, k, k), (q.half(), k.half(), k.half()), (q.bfloat16(), k, k), (q.bfloat16(), k.bfloat16(), k)):
-        assert not ok(a, b, c)                # (the general kernel refuses them)
+        assert not ok(a, b, c)
+
+
+class _Doubled(torch.nn.Linear):
+    def forward(self, x):
+        return 2 * super().forward(x)
+
+
+def test_modules_whose_call_is_not_their_class_s_own():
+    from torch.nn.modules import module as m
+    from msa_amd import ops
+    plain = lambda x: ops.plain_module(x, torch.nn.Linear)
+    lin = torch.nn.Linear(4, 4)
+    assert plain(lin) and not plain(_Doubled(4, 4)) and not plain(torch.nn.Identity()) and not plain(object())
+    for register in (lin.register_forward_hook, lin.register_forward_pre_hook, lin.register_full_backward_hook, m.register_module_forward_hook,
+                     m.register_module_forward_pre_hook, m.register_module_full_backward_hook):
+        h = register(lambda *a: None)
+        assert not plain(lin)
+        h.remove()
+        assert plain(lin)
+    lin.forward = lambda x: x
+    assert not plain(lin)
+    del lin.forward
+    assert plain(lin)
+
+
+@pytest.fixture
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    from msa_amd import ops
+    return ops
+
+
+@pytest.mark.gpu
+def test_an_mlp_with_a_call_of_its_own(gpu):
+    """A layer adds what calling its MLP gives: a subclass's, an instance's or another module's forward, and a hook's result."""
+    from torch.nn.modules import module as m
+    from msa_amd.config import MSAConfig
+    from msa_amd.model import MLP, MSADecoderLayer
+
+    class Attention(torch.nn.Module):
+        def forward(self, x, *a, **k):
+            return x * 0.5, None
+
+    class Tripled(MLP):
+        def forward(self, x):
+            return 3 * super().forward(x)
+
+    cfg = MSAConfig(hidden_size=1024, intermediate_size=3072, num_hidden_layers=1)
+    torch.manual_seed(0)
+    layer = MSADecoderLayer(cfg, 0)
+    layer.self_attn = Attention()
+    tripled = Tripled(cfg)
+    layer, tripled = layer.cuda().bfloat16().requires_grad_(False), tripled.cuda().bfloat16().requires_grad_(False)
+    tripled.load_state_dict(layer.mlp.state_dict())
+    own = layer.mlp
+    x = torch.randn((1, 9600, 1024), device="cuda").bfloat16()       # (the products of 9600 rows are tiled ones)
+
+    def added():
+        """What the layer adds behind its attention, and that times one over the plain MLP's output."""
+        h = x.clone()
+        y = layer(h, None, None, None, None)
+        return (y.float() - (x + gpu.rmsnorm(x, layer.input_layernorm.weight, 1e-6) * 0.5).float())
+    base = added()
+    assert gpu.linear_ok(own.down_proj, torch.empty((1, 9600, 3072), device="cuda").bfloat16())
+    # (rounding the stream to bf16 leaves 2^-9 of values some ten times the MLP's, three times over)
+    close = lambda got, times: ((got - times * base).norm() / base.norm()).item() < 0.06 * max(1, times)
+    layer.mlp = tripled
+    print("[routes] subclass", flush=True)
+    assert close(added(), 3)
+    layer.mlp = own
+    inner = own.forward
+    own.forward = lambda x: 2 * inner(x)
+    assert close(added(), 2)
+    del own.forward
+    assert close(added(), 1)
+    h = m.register_module_forward_hook(lambda mod, i, o: o * 0 if mod is own else None)
+    assert close(added(), 0)
+    h.remove()
+    layer.mlp = torch.nn.Identity()
+    n = gpu.rmsnorm(x + gpu.rmsnorm(x, layer.input_layernorm.weight, 1e-6) * 0.5, layer.post_attention_layernorm.weight, 1e-6).float()
+    assert ((added() - n).norm() / n.norm()).item() < 0.02
+
+
+@pytest.mark.gpu
+def test_linear_and_embedding_with_a_call_of_their_own(gpu):
+    lin = torch.nn.Linear(1024, 4096, bias=False).cuda().bfloat16().requires_grad_(False)
+    x = torch.randn((4096, 1024), device="cuda").bfloat16()
+    assert gpu.linear_ok(lin, x)
+    lin.forward = lambda x: x[:, :8]
+    assert not gpu.linear_ok(lin, x) and torch.equal(gpu.linear(lin, x), x[:, :8])
