@@ -29,9 +29,9 @@ class MLP(nn.Module):
 
     def _gate_up(self, interleaved: bool):
         """Gate and up rows in one matrix, behind one another or as the silu-mul epilogues take them; made again when either weight
-        changes."""
+        changes (one made in inference mode does not tell of changes in place)."""
         parts = (self.gate_proj.weight, self.up_proj.weight)
-        key = tuple((w.data_ptr(), w._version, w.dtype, w.device) for w in parts)
+        key = tuple((w.data_ptr(), None if w.is_inference() else w._version, w.dtype, w.device) for w in parts)
         if interleaved not in self._joined or self._joined[interleaved][0] != key:
             gate, up = (w.detach() for w in parts)
             self._joined[interleaved] = (key, ops.interleave_gate_up(gate, up) if interleaved else torch.cat([gate, up], dim=0).contiguous())

@@ -108,3 +108,23 @@ def test_linear_and_embedding_with_a_call_of_their_own(gpu):
     assert gpu.linear_ok(lin, x)
     lin.forward = lambda x: x[:, :8]
     assert not gpu.linear_ok(lin, x) and torch.equal(gpu.linear(lin, x), x[:, :8])
+
+
+@pytest.mark.parametrize("interleaved", [False, True])
+def test_joined_weights_follow_their_parts(interleaved):
+    """Also of a model made in inference mode, whose tensors have no version."""
+    from msa_amd import ops
+    from msa_amd.config import MSAConfig
+    from msa_amd.model import MLP
+    want = lambda m: (ops.interleave_gate_up if interleaved else lambda *w: torch.cat(w))(m.gate_proj.weight, m.up_proj.weight)
+    cfg = MSAConfig(hidden_size=64, intermediate_size=128)
+    with torch.inference_mode():
+        m = MLP(cfg)
+        assert torch.equal(m._gate_up(interleaved), want(m))
+    m = MLP(cfg).requires_grad_(False)
+    first = m._gate_up(interleaved)
+    assert torch.equal(first, want(m)) and m._gate_up(interleaved) is first
+    m.up_proj.weight.mul_(2)
+    assert torch.equal(m._gate_up(interleaved), want(m))
+    m.gate_proj.weight = torch.nn.Parameter(torch.randn(128, 64))
+    assert torch.equal(m._gate_up(interleaved), want(m))
