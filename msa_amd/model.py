@@ -32,10 +32,15 @@ class MLP(nn.Module):
         changes (one made in inference mode does not tell of changes in place)."""
         parts = (self.gate_proj.weight, self.up_proj.weight)
         key = tuple((w.data_ptr(), None if w.is_inference() else w._version, w.dtype, w.device) for w in parts)
-        if interleaved not in self._joined or self._joined[interleaved][0] != key:
+        held = self._joined.get(interleaved)
+        if held is None or held[0] != key:
             gate, up = (w.detach() for w in parts)
-            self._joined[interleaved] = (key, ops.interleave_gate_up(gate, up) if interleaved else torch.cat([gate, up], dim=0).contiguous())
-        return self._joined[interleaved][1]
+            made = ops.interleave_gate_up(gate, up) if interleaved else torch.cat([gate, up], dim=0).contiguous()
+            if held is not None and (held[1].shape, held[1].dtype, held[1].device) == (made.shape, made.dtype, made.device):
+                with torch.inference_mode():       # in place: a captured step reads this memory
+                    made = held[1].copy_(made)
+            self._joined[interleaved] = held = (key, made)
+        return held[1]
 
     def decode_rows(self, residual, norm_weight, eps):
         """``residual + down(silu(gate(n)) * up(n))`` with ``n = rmsnorm(residual)`` for up to 16 bf16 rows:

@@ -128,3 +128,7 @@ def test_joined_weights_follow_their_parts(interleaved):
     assert torch.equal(m._gate_up(interleaved), want(m))
     m.gate_proj.weight = torch.nn.Parameter(torch.randn(128, 64))
     assert torch.equal(m._gate_up(interleaved), want(m))
+    # a captured step goes on reading the memory that it was captured with
+    assert m._gate_up(interleaved).data_ptr() == first.data_ptr() and torch.equal(first, want(m))
+    m.double()
+    assert m._gate_up(interleaved).dtype == torch.float64 and torch.equal(m._gate_up(interleaved), want(m))
