@@ -60,7 +60,7 @@ class MLP(nn.Module):
         sum is rounded once."""
         act = self._activation(x)
         if ops.linear_ok(self.down_proj, act) and residual.is_contiguous() and residual.dtype == x.dtype and residual.shape == x.shape \
-                and residual.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and residual.requires_grad):
+                and residual.device == x.device and residual.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and residual.requires_grad):
             ops.tile_linear(act.view(-1, act.shape[-1]), self.down_proj.weight, out=residual.view(-1, x.shape[-1]), add=True)
             return residual
         return residual.add_(self.down_proj(act))

@@ -434,8 +434,8 @@ def tile_linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
     ``silu(gate) * up`` of width ``N / 2``; ``glu`` (limit, alpha, shift) takes rows in (gate, up) pairs and returns the clamped gated
     unit; ``gelu_n`` puts the first columns through gelu."""
     _need_cuda(w)
-    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or x.stride(1) != 1 or not x.is_cuda:
-        raise ValueError("tile_linear: x [T, K] with unit column stride, w [N, K] contiguous, both on the device")
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or x.stride(1) != 1 or not x.is_cuda or w.device != x.device:
+        raise ValueError("tile_linear: x [T, K] with unit column stride, w [N, K] contiguous, both on one device")
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise ValueError("tile_linear: x and w in bf16")
     if add + silu_mul + (glu is not None) + (gelu_n != 0) > 1 or (add and out is None):
@@ -444,8 +444,8 @@ def tile_linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
     width = N // 2 if silu_mul or glu is not None else N
     if out is None:
         out = torch.empty((T, width), dtype=x.dtype, device=x.device)
-    elif tuple(out.shape) != (T, width) or out.dtype != x.dtype or out.stride(1) != 1 or not out.is_cuda:
-        raise ValueError(f"tile_linear: out must be bf16 [{T}, {width}] on the device with unit column stride")
+    elif tuple(out.shape) != (T, width) or out.dtype != x.dtype or out.stride(1) != 1 or out.device != x.device:
+        raise ValueError(f"tile_linear: out must be bf16 [{T}, {width}] on x's device with unit column stride")
     if not T:
         return out
     ws = scratch(_lib.load().msa_tile_workspace_bytes(T, K, N), x.device)
@@ -475,7 +475,7 @@ def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1) -> bool:
     return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == K
             and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 21))
             and K % 64 == 0 and 1024 <= K <= 32768 and N % 8 == 0 and N < 1 << 20 and T < 1 << 22
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.device == x.device
             and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
 
 

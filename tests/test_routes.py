@@ -132,3 +132,28 @@ def test_joined_weights_follow_their_parts(interleaved):
     assert m._gate_up(interleaved).data_ptr() == first.data_ptr() and torch.equal(first, want(m))
     m.double()
     assert m._gate_up(interleaved).dtype == torch.float64 and torch.equal(m._gate_up(interleaved), want(m))
+
+
+class _On:
+    """What a route looks at of a dense bf16 matrix on some device."""
+    dtype, is_cuda, requires_grad = torch.bfloat16, True, False
+
+    def __init__(self, device, *shape):
+        self.device, self.shape = torch.device(device), shape
+
+    dim = lambda self: len(self.shape)
+    is_contiguous = lambda self: True
+    stride = lambda self, i: (self.shape[1], 1)[i]
+    data_ptr = lambda self: 4096
+
+
+def test_operands_of_different_devices(monkeypatch):
+    from msa_amd import ops
+    x, w = _On("cuda:0", 8192, 2048), _On("cuda:0", 4096, 2048)
+    assert ops.tile_linear_ok(x, w)
+    assert not ops.tile_linear_ok(x, _On("cuda:1", 4096, 2048))
+    monkeypatch.setattr(ops, "_need_cuda", lambda *a: None)
+    with pytest.raises(ValueError, match="device"):
+        ops.tile_linear(x, _On("cuda:1", 4096, 2048))
+    with pytest.raises(ValueError, match="device"):
+        ops.tile_linear(x, w, out=_On("cuda:1", 8192, 4096))
