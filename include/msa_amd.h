@@ -353,7 +353,8 @@ int msa_qkv_proj_ws(const void* x, int64_t T, int32_t K, const void* w, int32_t 
                     const float* rope_cos, const float* rope_sin, int32_t rope_rows, void* q_out, void* k_out,
                     void* v_out, void* r_out, void* ws, size_t ws_bytes, void* stream);
 /* Products of a block of tokens, bf16 with fp32 sums: x [T, K] (rows ldx apart) . w [N, K]^T, w dense, K a multiple of 64, N of 8 (16 where
- * it is halved), x / w / out 16-byte aligned, row strides multiples of 8.  What becomes of the sums, each rounded once:
+ * it is halved), x / w / out 16-byte aligned, row strides multiples of 8.  What becomes of the sums (results
+ * are rounded to bf16; the gated ends and gelu may take the sums as they would be in memory, rounded, but all of a call's alike):
  *   MSA_TILE_STORE     out [T, N] (rows ldo apart)
  *   MSA_TILE_ADD       out +=
  *   MSA_TILE_SILU_MUL  out [T, N / 2] = silu(gate) * up, rows of w alternating in groups of eight gates and eight ups

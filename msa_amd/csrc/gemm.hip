@@ -154,8 +154,11 @@ __device__ __forceinline__ float column_sum(float v) {
 }
 
 // Epilogue of a wavefront's 128 weight rows x 16 tokens (a column block): a lane has token `token` and the values v[4 i + r].
-template <int kMode>
+// kRounded: the gated ends and gelu take the sums rounded to bf16, as tile_flow_kernel does of the call's whole tiles: a token's result
+// does not depend on which tiles are cut into pieces.
+template <int kMode, bool kRounded = false>
 struct Finish {
+  static __device__ __forceinline__ float taken(float sum) { return kRounded ? bf16_to_f32(f32_to_bf16(sum)) : sum; }
   const TileArgs& a;
   int n0, g;                // first weight row of the wavefront, lane group
   // kHeads
@@ -221,7 +224,7 @@ struct Finish {
           if (n0 < a.end.gelu_n) {                 // (the same for all lanes)
             const bool through = n0 + 32 * m + 8 * g < a.end.gelu_n;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[8 * m + e] = through ? gelu_tanh_f(v[8 * m + e]) : v[8 * m + e];
+            for (int e = 0; e < 8; ++e) v[8 * m + e] = through ? gelu_tanh_f(taken(v[8 * m + e])) : v[8 * m + e];
           }
         }
         if (m & 1) store_lines(row + 32 * (m - 1), a.ldo, token, a.T, a.N - (n0 + 32 * (m - 1) + 8 * g), pack8(v + 8 * m - 8), pack8(v + 8 * m), a.stream);
@@ -234,7 +237,7 @@ struct Finish {
         float o[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const float gate = v[16 * m + e], up = v[16 * m + 8 + e];
+          const float gate = taken(v[16 * m + e]), up = taken(v[16 * m + 8 + e]);
           o[e] = kMode == kGlu ? clamped_glu_f(gate, up, a.end.limit, a.end.alpha, a.end.shift) : silu_f(gate) * up;
         }
         packed[m] = pack8(o);
@@ -430,8 +433,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_vgpr(kCompilerV
 // first step overwrites its accumulators, and finished and stored, sixteen tokens a step, behind the MFMAs of the eight steps after that
 // (gen_scan_asm.py).  A wavefront is alone on its SIMD, so whatever it does between two tiles the matrix cores wait for: storing a
 // tile took it 5 us, gelu 10, against 57 us of steps at K = 2560 and 23 at K = 1024.  Whole calls, us, ends in registers and here: 32771 x
-// 2560 x 19456 stored 2392 and 2238, 6001 x 2560 x 19456 with the gated unit 434 and 415, 8192 x 1024 x 4096 with gelu 88 and 60.  (silu-mul:
-// 2257 and 2221, 11.99 and 12.00 ms for the block it is part of: its half output leaves little to hide, and power bounds the rest.)
+// 2560 x 19456 stored 2392 and 2238, 6001 x 2560 x 19456 with the gated unit 434 and 415, 8192 x 1024 x 4096 with gelu 88 and 60, and
+// with silu-mul 2257 and 2221 (the encoding block around it 12.00 and 11.90 ms: its half output leaves less to hide).
 constexpr int kFlowVgprs = 24;                 // the compiler's share of the vector registers
 constexpr int kFlowSteps = 11;                 // an item of that many steps takes another tile's end: one packs, eight finish, the
                                                // last two already load for the item behind
@@ -564,7 +567,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_vgpr(kFlowVgprs
 
 // The tiles that were multiplied in pieces: a workgroup adds up a column block's pieces, in their order, for the four wavefronts that
 // would have finished it.
-template <int kMode>
+template <int kMode, bool kRounded>
 __global__ __launch_bounds__(kThreads) void tile_finish_kernel(TileArgs a, int per_xcd) {
   const int j = blockIdx.x & 7, xcd = (blockIdx.x >> 3) / a.max_rem, u = (blockIdx.x >> 3) % a.max_rem;
   const Share share = tile_share(a.tiles_t * a.tiles_n, per_xcd, xcd);
@@ -573,8 +576,8 @@ __global__ __launch_bounds__(kThreads) void tile_finish_kernel(TileArgs a, int p
   tile_at(a, share.first + share.rounds * per_xcd + u, tile_t, tile_n);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave >> 1, wn = wave & 1;
   const int token = tile_t * kTile + wn * 128 + 16 * j + (lane & 15);
-  Finish<kMode> f(a, tile_n * kTile + wm * 128, lane);
-  typename Finish<kMode>::Ahead ahead;
+  Finish<kMode, kRounded> f(a, tile_n * kTile + wm * 128, lane);
+  typename Finish<kMode, kRounded>::Ahead ahead;
 #pragma unroll
   for (int m = 0; m < 4; ++m) f.request(m, token, kMode == kHeads ? f.table_row(token) : 0, ahead);
   const float4* from = reinterpret_cast<const float4*>(a.pieces + (int64_t)(blockIdx.x >> 3) * a.split * (kTile * kTile)) + wave * 4096 + j * 512 + lane;
@@ -633,9 +636,9 @@ int launch_tile_kernel(const TileArgs& a, const Plan& p, hipStream_t st) {
   return MSA_OK;
 }
 
-template <int kMode>
+template <int kMode, bool kRounded>
 int launch_finish(const TileArgs& a, const Plan& p, hipStream_t st) {
-  tile_finish_kernel<kMode><<<kXcds * p.max_rem * 8, kThreads, 0, st>>>(a, p.grid / kXcds);
+  tile_finish_kernel<kMode, kRounded><<<kXcds * p.max_rem * 8, kThreads, 0, st>>>(a, p.grid / kXcds);
   MSA_LAUNCH_CHECK();
   return MSA_OK;
 }
@@ -652,11 +655,11 @@ int launch_tiles(TileArgs a, const Plan& p, hipStream_t st) {
     if (a.K >= 64 * kFlowSteps && a.ldo < ((int64_t)1 << 21) && (kMode != kGelu || a.end.gelu_n % 128 == 0)) {
       a.rate = -1.4426950408889634f * a.end.alpha;
       const int rc = a.stream ? launch_tile_kernel<tile_flow_kernel<kMode, true>>(a, p, st) : launch_tile_kernel<tile_flow_kernel<kMode, false>>(a, p, st);
-      return rc != MSA_OK || p.split == 1 ? rc : launch_finish<kMode>(a, p, st);
+      return rc != MSA_OK || p.split == 1 ? rc : launch_finish<kMode, kMode != kStore>(a, p, st);
     }
   }
   const int rc = launch_tile_kernel<tile_gemm_kernel<kMode>>(a, p, st);
-  return rc != MSA_OK || p.split == 1 ? rc : launch_finish<kMode>(a, p, st);
+  return rc != MSA_OK || p.split == 1 ? rc : launch_finish<kMode, false>(a, p, st);
 }
 
 int check_operands(const char* name, const void* x, int64_t T, int64_t ldx, const void* w, int32_t K, int64_t N) {
