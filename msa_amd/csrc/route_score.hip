@@ -1116,8 +1116,8 @@ __global__ void decode_scores_kernel(const uint32_t* __restrict__ key, int64_t n
 // K_r and query rows come through a ring of stages of a cache line of 32 rows, direct loads of eight whole lines: an MFMA operand
 // loaded from memory touches 32 lines an instruction, 32 bytes each, and the address unit takes four times as long over it.  What
 // bounds it: the matrix cores' fp32 rate (256 FLOP a cycle and compute unit) and, with few rows, the launch and the first loads.
-// The kernel at 8000 chunks x 64 rows 21.0 -> 17.8 us (8 of them matrix cores); whole routing calls, us, operands from memory and
-// through the ring: 8000 x 64 30.7 and 26.4, 512 x 64 20.4 and 17.9, 64000 x 64 123 and 106, 128000 x 32 178 and 157, 8000 x 512 85 and 83.
+// Whole routing calls, us, operands from memory and through the ring: 8000 chunks x 64 rows 30.7 and 26.4, 512 x 64 20.4 and 17.9,
+// 64000 x 64 123 and 106, 128000 x 32 178 and 157, 8000 x 512 85 and 83.
 // ------------------------------------------------------------------------------------------
 constexpr int kSplitK = 1024, kSplitWaves = 4, kSplitCols = 32, kSplitMaxBlocks = 32;
 constexpr int kSplitSlab = 32 * 128;           // a stage of a wavefront's ring: 32 rows, a cache line (32 values of K) each
@@ -1157,6 +1157,7 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void score_split_kernel(const 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, half = lane >> 5;
   const int n0 = blockIdx.x * kSplitCols, blocks = M_rows >> 5;
+  if (n0 >= C) return;                                   // (the grid's columns are a multiple of eight)
   const int b0 = blockIdx.y * blocks_per_wg, b1 = min(blocks, b0 + blocks_per_wg);
   char* const ring = lds + wave * kRing * kSplitSlab;
   const uint32_t ring_at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)ring);
@@ -1332,16 +1333,17 @@ int launch_gemm(const void* qs, const void* kr, const uint32_t* row_bits, uint32
   return MSA_OK;
 }
 
-// As many workgroups along the query blocks as give every compute unit two, at most kSplitMaxBlocks blocks each; one where that
-// alone fills three quarters of the units or more, so that K_r is read once (8000 chunks x 64 rows: 26.4 us, with two 30.8).
+// As many workgroups along the query blocks as give every compute unit two, at most kSplitMaxBlocks blocks each.  Those of a column come
+// a multiple of the XCDs behind one another, so that one L2 has its K_r rows for all of them; the columns that this adds end at once.  us a
+// call, one workgroup a column and two: 8000 chunks x 64 rows 24.4 and 23.1, x 256 54.2 and 48.9, 6112 x 64 25.4 and 24.0 (two of 250 or
+// 191 columns that meet in different L2s: 30.5, 55.1 and 27.4).
 template <bool kDocMax>
 int launch_split(const void* qs, const void* kr, const uint32_t* row_bits, uint32_t* out_key, const int32_t* chunk_doc,
                  int32_t M_rows, int32_t C, int32_t blocks_per_query, int32_t n_docs, hipStream_t st) {
   const int cols = (C + kSplitCols - 1) / kSplitCols, blocks = M_rows / 32;
-  const int each = cols <= compute_units() && cols * 4 >= 3 * compute_units() ? 1 : 2;
-  const int want = std::min(blocks, std::max((blocks + kSplitMaxBlocks - 1) / kSplitMaxBlocks, each * compute_units() / cols));
+  const int want = std::min(blocks, std::max((blocks + kSplitMaxBlocks - 1) / kSplitMaxBlocks, 2 * compute_units() / cols));
   const int per_wg = (blocks + want - 1) / want;
-  const dim3 grid((unsigned)cols, (unsigned)((blocks + per_wg - 1) / per_wg));
+  const dim3 grid((unsigned)((cols + 7) / 8 * 8), (unsigned)((blocks + per_wg - 1) / per_wg));
   int slot = -1;
   if (g_timer.on.load(std::memory_order_acquire)) {
     std::lock_guard<std::mutex> lock(g_timer.mu);
@@ -1349,7 +1351,7 @@ int launch_split(const void* qs, const void* kr, const uint32_t* row_bits, uint3
   }
   if (slot >= 0) MSA_HIP(hipEventRecord(g_timer.start[slot], st));
   // one workgroup a compute unit: the deep ring; more: two of them with two slots a wavefront
-  const bool one = (int64_t)grid.x * grid.y <= compute_units();
+  const bool one = (int64_t)cols * grid.y <= compute_units();
   const auto kern = one ? score_split_kernel<kDocMax, 6> : score_split_kernel<kDocMax, 2>;
   const int lds = split_lds_bytes(one ? 6 : 2);
   static std::atomic<int> lds_limit_raised[2] = {{0}, {0}};
