@@ -210,7 +210,7 @@ def product_gelu(x: torch.Tensor, w: torch.Tensor, n: int) -> torch.Tensor:
     """``x @ w.T``, its first ``n`` columns through gelu."""
     if x.shape[0] >= ops.TILE_ROWS and n % 8 == 0 and ops.tile_linear_ok(x, w):
         return ops.tile_linear(x, w, gelu_n=n)
-    if n % 8 == 0 and ops.block_linear_ok(x, w):
+    if n % 8 == 0 and ops.block_linear_ok(x, w, True):
         return ops.block_linear(x, w, gelu_n=n)
     y = F.linear(x, w)
     gelu_(y[:, :n])
@@ -221,7 +221,7 @@ def product_glu(x: torch.Tensor, w: torch.Tensor, limit: float, alpha: float = G
     """``clamped_glu(x @ w.T)``."""
     if x.shape[0] >= ops.TILE_ROWS and w.shape[0] % 16 == 0 and ops.tile_linear_ok(x, w):
         return ops.tile_linear(x, w, glu=(limit, alpha, shift))
-    if ops.block_linear_ok(x, w):
+    if ops.block_linear_ok(x, w, True):
         return ops.block_linear(x, w, glu=(limit, alpha, shift))
     return clamped_glu(F.linear(x, w), limit, alpha, shift)
 

@@ -89,3 +89,18 @@ def test_captured(ops):
         torch.cuda.synchronize()
         assert torch.equal(held, out)
     assert _err(out, want) < TOL
+
+
+def test_route_of_captured_calls(ops):
+    """A captured call pays for no host: the line is the kernels' own."""
+    shapes = {(64, 1024, 1024): True, (17, 1024, 6176): True, (1000, 2048, 1024): True, (32, 2560, 2560): False, (1500, 128, 4096): False,
+              (573, 1024, 8192): False}
+    operands = {s: _operands(*s, 5) for s in shapes}
+    assert all(ops.block_linear_ok(x, w) for x, w, _ in operands.values())
+    graph, took = torch.cuda.CUDAGraph(), {}
+    keep = torch.zeros(1, device="cuda")
+    with torch.cuda.graph(graph):
+        keep.add_(1)
+        for s, (x, w, _) in operands.items():
+            took[s] = ops.block_linear_ok(x, w)
+    assert took == shapes
