@@ -1,5 +1,6 @@
-// Document top-k over the per-document keys the scoring kernel's epilogue leaves: wavefront-level bitonic sorts, joined across the
-// workgroup's wavefronts through LDS, and a final per-query merge of the per-workgroup candidate lists.
+// Document top-k over the per-document keys the scoring kernel's epilogue leaves: wavefront-level bitonic sorts (of all documents, or, where
+// many lists are made, of those above a running k-th best), joined across the workgroup's wavefronts through LDS, and a final per-query
+// merge of the per-workgroup candidate lists.
 //
 // Candidates are 64-bit composites (score key << 32 | ~doc) so one unsigned compare orders by
 // score descending, then document index ascending; 0 is the empty slot.
@@ -10,7 +11,7 @@
 
 namespace {
 
-constexpr int kWaves = 16;
+constexpr int kWaves = 16, kFewWaves = 4;
 
 // Lane i receives the value of lane i ^ m: data-parallel moves inside a row of 16 lanes, swaps of rows and of half-waves beyond
 // it.  The sort networks below are chains of dependent exchanges, so this latency is what the top-k kernels spend their time on.
@@ -69,6 +70,7 @@ __device__ __forceinline__ uint64_t wave_merge_desc(uint64_t best, uint64_t batc
 }
 
 // The wavefronts' lists joined in pairs, then the pairs' and so on; the result in wavefront 0.
+template <int kWaves>
 __device__ __forceinline__ uint64_t join_lists(uint64_t best, uint64_t (*lists)[64], int lane, int wave) {
 #pragma unroll
   for (int s = 1; s < kWaves; s <<= 1) {
@@ -107,8 +109,8 @@ __device__ __forceinline__ void write_topk(const TopkOut& out, int b, int32_t to
 // The scoring kernel leaves one key per (query, document).  A workgroup of sixteen wavefronts takes 2048 documents of a query, 128
 // a wavefront: two sorts that run beside one another, a merge, and the lists joined in four rounds.  It is a chain of exchanges from the
 // first load to the last merge, so what counts is its length: a wavefront of four, with 512 documents and a queue of those above its
-// k-th best, sorted and merged four to five times one after the other.  A launch over 1000 documents 6.5 -> 6.0 us, over 88000 documents
-// of one query 12.0 -> 11.1, the join of their 43 lists 9.0 -> 6.5.
+// k-th best (doc_topk_queue_kernel), sorted and merged four to five times one after the other.  us, four wavefronts and sixteen: 1000
+// documents 5.8 and 5.4, 8 queries of 1000 7.1 and 5.7, 40000 documents 8.4 and 7.8; launch_topk has the line between them.
 // A bank of one workgroup's documents has one list per query: its result is written here (a launch of 4 us less), otherwise the
 // lists go to merge_topk_kernel.
 __global__ __launch_bounds__(kWaves * 64) void doc_topk_kernel(const uint32_t* __restrict__ doc_key, int32_t n_docs,
@@ -127,13 +129,68 @@ __global__ __launch_bounds__(kWaves * 64) void doc_topk_kernel(const uint32_t* _
   } else {
     best = wave_sort<true>(best, lane);
   }
-  best = join_lists(best, lists, lane, wave);
+  best = join_lists<kWaves>(best, lists, lane, wave);
   if (wave == 0) {
     if (gridDim.x == 1) write_topk(out, b, topk, lane, best);
     else cand[((int64_t)b * gridDim.x + blockIdx.x) * kTopkMax + lane] = best;
   }
 }
 
+// The same of four wavefronts, for launches of more lists than compute units, where the length of a chain counts less than the
+// exchanges of all: a wavefront walks over its share 256 documents at a time, drops by a ballot what does not reach its k-th best so far,
+// and sorts and merges the rest 64 at a time.
+__global__ __launch_bounds__(kFewWaves * 64) void doc_topk_queue_kernel(const uint32_t* __restrict__ doc_key, int32_t n_docs,
+                                                                        int32_t topk, uint64_t* __restrict__ cand, TopkOut out) {
+  constexpr int kLoads = 4;
+  __shared__ uint64_t pending[kFewWaves][128], lists[kFewWaves][64];
+  const int b = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t* key = doc_key + (int64_t)b * n_docs;
+  const int d_begin = blockIdx.x * kTopkDocsPerBlock, d_end = min(d_begin + kTopkDocsPerBlock, n_docs);
+  uint64_t* queue = pending[wave];
+  uint64_t best = 0, kth = 0;
+  int n = 0;
+  auto flush = [&](int from, int count) {        // `count` (<= 64) queued candidates
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    best = wave_merge_desc(best, wave_sort<false>(lane < count ? queue[from + lane] : 0, lane), lane);
+    kth = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(best >> 32), topk - 1) << 32) |
+          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)best, topk - 1);
+  };
+  for (int base = d_begin + wave * 64 * kLoads; base < d_end; base += kFewWaves * 64 * kLoads) {     // (the same in all lanes)
+    uint32_t k[kLoads];
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      const int d = base + u * 64 + lane;
+      k[u] = d < d_end ? __builtin_nontemporal_load(key + d) : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      const int d = base + u * 64 + lane;
+      const uint64_t v = d < d_end ? ((uint64_t)k[u] << 32) | (uint64_t)(0xffffffffu - (uint32_t)d) : 0;
+      const bool in = v > kth;
+      const uint64_t mask = __ballot(in);
+      if (mask == 0) continue;
+      if (in) queue[n + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0))] = v;
+      n += __builtin_popcountll(mask);
+      if (n >= 64) {
+        n -= 64;
+        flush(n, 64);
+      }
+    }
+  }
+  flush(0, n);
+  best = join_lists<kFewWaves>(best, lists, lane, wave);
+  if (wave == 0) {
+    if (gridDim.x == 1) write_topk(out, b, topk, lane, best);
+    else cand[((int64_t)b * gridDim.x + blockIdx.x) * kTopkMax + lane] = best;
+  }
+}
+
+// Four wavefronts a query where sixteen would have a list each at most: us with 2 / 5 / 10 lists 2.0 / 2.3 / 2.6 and 3.4 / 3.3 / 3.4, with
+// 20 / 43 / 98 3.9 / 5.9 / 11.7 and 3.8 / 4.5 / 6.9.
+template <int kWaves>
 __global__ __launch_bounds__(kWaves * 64) void merge_topk_kernel(const uint64_t* __restrict__ cand, int32_t blocks,
                                                                  int32_t topk, TopkOut out) {
   __shared__ uint64_t lists[kWaves][64];
@@ -148,17 +205,22 @@ __global__ __launch_bounds__(kWaves * 64) void merge_topk_kernel(const uint64_t*
     for (int u = 0; u < 4; ++u)
       if (i + u * kWaves < blocks) best = wave_merge_desc(best, x[u], lane);
   }
-  best = join_lists(best, lists, lane, wave);
+  best = join_lists<kWaves>(best, lists, lane, wave);
   if (wave == 0) write_topk(out, b, topk, lane, best);
 }
 
-// The top-k of every query's keys [B, n_docs].
+// The top-k of every query's keys [B, n_docs].  Sixteen wavefronts a list up to a list for every compute unit, four beyond that; us, four
+// and sixteen: 4 queries of 88000 documents (172 lists) 8.8 and 8.1, 2 of 200000 (196) 8.8 and 8.4; 64 of 9000 (320) 9.6 and 13.6, 8 of 88000
+// (344) 9.2 and 13.0, 16 of 88000 10.8 and 17.2, 64 of 200000 52 and 112.
 int launch_topk(const uint32_t* key, const msa_bank* bank, const RouteWorkspace& w, uint64_t* cand, int32_t B, int32_t topk,
                 const TopkOut& out, hipStream_t st) {
-  doc_topk_kernel<<<dim3((unsigned)w.topk_blocks, (unsigned)B), kWaves * 64, 0, st>>>(key, (int32_t)bank->n_docs, topk, cand, out);
+  const dim3 grid((unsigned)w.topk_blocks, (unsigned)B);
+  if ((int64_t)w.topk_blocks * B <= device_compute_units()) doc_topk_kernel<<<grid, kWaves * 64, 0, st>>>(key, (int32_t)bank->n_docs, topk, cand, out);
+  else doc_topk_queue_kernel<<<grid, kFewWaves * 64, 0, st>>>(key, (int32_t)bank->n_docs, topk, cand, out);
   MSA_LAUNCH_CHECK();
   if (w.topk_blocks == 1) return MSA_OK;
-  merge_topk_kernel<<<B, kWaves * 64, 0, st>>>(cand, w.topk_blocks, topk, out);
+  if (w.topk_blocks <= kWaves) merge_topk_kernel<kFewWaves><<<B, kFewWaves * 64, 0, st>>>(cand, w.topk_blocks, topk, out);
+  else merge_topk_kernel<kWaves><<<B, kWaves * 64, 0, st>>>(cand, w.topk_blocks, topk, out);
   MSA_LAUNCH_CHECK();
   return MSA_OK;
 }

@@ -66,6 +66,25 @@ def test_topk_of_every_list_length(ops, docs):
         assert torch.equal(got[0], want) and torch.equal(got[1], want)
 
 
+# lists of 2048 documents on 256 compute units: 258, 256 and 257 of them, up to two, four and eighteen a query
+@pytest.mark.parametrize("docs,B", [(2049, 129), (2048, 256), (100, 257), (7000, 65), (2048 * 17 + 1, 15)])
+def test_topk_of_many_lists(ops, docs, B):
+    """Scores as above, rising for one query and falling for the next."""
+    _say(f"topk docs={docs} B={B}")
+    kr = torch.zeros((docs, 8, 128), device="cuda")
+    r = torch.randperm(docs, generator=torch.Generator().manual_seed(docs)).cuda()
+    kr[:, 0, 0] = (r // 3).float() / (1 << 17)                       # three documents a score
+    bank = ops.Bank(1, torch.arange(docs + 1, dtype=torch.int32), torch.arange(docs) + 1, 8, 128, torch.float32)
+    bank.set_layer(0, kr)
+    q = torch.zeros((B, 1, 32, 128), device="cuda")
+    q[0::2, :, :4, 0], q[1::2, :, :4, 0] = 1.0, -1.0
+    for k in (1, 16, 64):
+        _, got, _ = ops.route_topk(bank, 0, q, None, mode="scaled_dot", topk=k)
+        for sign in (0, 1):
+            want = torch.sort(-(r // 3) if sign == 0 else r // 3, stable=True)[1][:k].to(torch.int32)
+            assert torch.equal(got[sign::2], want.expand(len(range(sign, B, 2)), -1))
+
+
 @pytest.mark.parametrize("B,k,capacity", [(1, 1, 100), (1, 64, 400), (2, 32, 400), (4, 16, 400), (3, 5, 400), (4, 16, 37), (1, 17, 3), (5, 16, 400)])
 def test_gather_of_few_documents(ops, B, k, capacity):
     """Against the rows themselves: documents of several samples, missing and repeated picks, rows behind the capacity."""
