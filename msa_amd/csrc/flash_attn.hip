@@ -899,11 +899,18 @@ extern "C" int msa_flash_attn_rows(const void* q, int64_t q_stride, const int32_
                                    float scale, const float* sink, const void* gate, int64_t gate_stride, void* out, void* stream) {
   MSA_REQUIRE(cu_q && kv_pos && max_sq > 0, "msa_flash_attn_rows: cu_q, kv_pos and max_sq are required");
   MSA_REQUIRE((int64_t)max_sq * q_stride < (int64_t)1 << 30, "msa_flash_attn_rows: query rows too far apart");
-  // One and a half blocks of 256 columns a compute unit: us, 32-column form and wide, 32 query heads: 2048 rows, one a unit, 53 and 58, but
-  // behind 4000 keys 176 and 171; 4000 rows in eight samples 43 and 39; 8192 rows 531 and 490; 16 heads: 2048 rows 40 and 54, 6001
-  // 175 and 177, 8192 271 and 250.
-  const bool enough = (int64_t)total_q * Hq * 2 >= (int64_t)3 * 256 * device_compute_units();
-  return flash_attn_entry(q, cu_q, k, v, kv_off, nullptr, B, total_q, Hq, Hkv, D, scale, 1, out, max_sq, enough,
+  // The wide form's workgroups take its blocks of 256 columns in turn, back and forth, so their work is even where all samples are as
+  // long, in full blocks, and a head's blocks fill an even number of turns; elsewhere it waits for the longest of them.  us, 32-column form
+  // and wide, 16 heads: 8192 rows 254 and 240, four samples of 2048 92 and 78, eight of 1024 60 and 54; 32: 4096 134 and 129, 8192 500 and
+  // 475, four of 1024 behind 4000 keys 287 and 270; but 16 heads: 4096 rows 92 and 102, two of 3500 112 and 168, four of 2500 126 and 181; 32:
+  // 6001 283 and 300, three of 3000 over 8 key heads 230 and 249, ten of 600 65 and 90, eight of 800 79 and 94, of 512 43 and 45.
+  const int G = Hkv > 0 ? Hq / Hkv : 0;
+  bool even = false;
+  if (G > 0 && G <= 8 && (int64_t)max_sq * B == total_q) {
+    const int64_t columns = (int64_t)max_sq * G, blocks = (columns + 255) / 256, turn = std::max(1, device_compute_units() / Hkv);
+    even = blocks >= 4 && 16 * (256 * blocks - columns) <= columns && B * blocks % (2 * turn) == 0;
+  }
+  return flash_attn_entry(q, cu_q, k, v, kv_off, nullptr, B, total_q, Hq, Hkv, D, scale, 1, out, max_sq, even,
                           {q_stride, sink, static_cast<const bf16_t*>(gate), gate_stride, kv_pos}, stream);
 }
 

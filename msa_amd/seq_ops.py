@@ -438,15 +438,17 @@ def flash_ok(dtype, D: int, E: int, scale: float) -> bool:
     return dtype == torch.bfloat16 and D % 8 == 0 and E % 8 == 0 and max(D, E) <= 256 and scale > 0
 
 
-FLASH_ROWS = 512        # of the longest portion
+FLASH_ROWS, FLASH_MEAN = 512, 256        # of the longest portion, of all
 
 
 def takes_flash_rows(q, k, v, H: int, G: int, D: int, E: int, chunk: int, batch: StepBatch) -> bool:
     """Whether the attention model's prefill kernels take the call: bf16, heads of 128, dense keys and values, and no position behind the
     first chunk (there it hides nothing).  Long portions gain (us, the general kernel and those, 16 heads of their own keys: 8192 rows 343 and
-    256, 2048 49 and 41, 2048 behind 4000 keys 132 and 111, 1000 27.3 and 26.0); shorter ones wait for the host, which has more to do."""
-    return (batch.max_rows >= FLASH_ROWS and q.dtype == k.dtype == v.dtype == torch.bfloat16 and D == E == 128 and H // G in (1, 2, 4, 8)
-            and (not chunk or batch.max_keys <= chunk) and _rows(k) == _rows(v) == G * D and _rows(q) % 8 == 0 and batch.max_rows * _rows(q) < 1 << 30
+    256, 2048 49 and 41, 2048 behind 4000 keys 132 and 111, 1000 27.3 and 26.0); shorter ones wait for the host, which has more to do.  Nor do
+    short ones beside a long one gain (32 heads, 513 rows and forty of 20: 22.4 and 28.6, twenty of 100 26.2 and 28.8; 700, 300, 100 and 900
+    35 and 34, 1500 and eight of 300 50 and 50)."""
+    return (batch.max_rows >= FLASH_ROWS and batch.rows >= FLASH_MEAN * batch.n_seq and q.dtype == k.dtype == v.dtype == torch.bfloat16
+            and D == E == 128 and H // G in (1, 2, 4, 8) and (not chunk or batch.max_keys <= chunk) and _rows(k) == _rows(v) == G * D and _rows(q) % 8 == 0 and batch.max_rows * _rows(q) < 1 << 30
             and not (q.data_ptr() | k.data_ptr() | v.data_ptr()) % 16)
 
 

@@ -70,3 +70,4 @@ def test_what_stays_with_the_general_kernel():
     assert not ok(599) and not ok(D=64) and not ok(b=seq_ops.StepBatch([300, 300], [0, 1], [0, 0], "cuda"))
     assert not ok(k=torch.zeros((600, 520), device="cuda").bfloat16()[:, :512])
     assert not ok(q=torch.zeros((600, 516), device="cuda").bfloat16()[:, :512])
+    assert not ok(b=seq_ops.StepBatch([560] + [1] * 40, list(range(41)), [0] * 41, "cuda"))     # one long portion among short ones
