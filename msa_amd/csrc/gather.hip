@@ -209,14 +209,23 @@ __global__ __launch_bounds__(kCopyThreads) void gather_few_kernel(const int32_t*
     const int e = __builtin_ctzll(left);
     const int32_t src = __builtin_amdgcn_readlane(c0, e), rows = __builtin_amdgcn_readlane(n, e);
     const uint64_t targets = __ballot(keep && first == e);
-    for (int r = blockIdx.y; r < rows; r += gridDim.y)
+    // two rows' loads in flight (documents of 200 chunks: 4 % less with one)
+    const int step = gridDim.y;
+    for (int r = blockIdx.y; r < rows; r += 2 * step)
       for (int off = row_lane; off < row_vecs; off += kCopyRowLanes) {
-        const uint4 a = k_src[(int64_t)(src + r) * row_vecs + off], b = v_src[(int64_t)(src + r) * row_vecs + off];
+        const bool two = r + step < rows;              // (the same in all lanes)
+        const int64_t from = (int64_t)(src + r) * row_vecs + off, behind = (int64_t)step * row_vecs;
+        const uint4 a = k_src[from], b = v_src[from];
+        uint4 a2 = a, b2 = b;
+        if (two) { a2 = k_src[from + behind]; b2 = v_src[from + behind]; }
         for (uint64_t t = targets; t != 0; t &= t - 1) {
           const int64_t row = (int64_t)__builtin_amdgcn_readlane(at, __builtin_ctzll(t)) + r;
           if (row >= capacity_rows) continue;
           k_dst[row * row_vecs + off] = a;
           v_dst[row * row_vecs + off] = b;
+          if (!two || row + step >= capacity_rows) continue;
+          k_dst[row * row_vecs + behind + off] = a2;
+          v_dst[row * row_vecs + behind + off] = b2;
         }
       }
   }
