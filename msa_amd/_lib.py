@@ -216,7 +216,7 @@ def _open(path: str, table) -> C.CDLL:
 
 def load() -> C.CDLL:
     """Loads the library and declares every entry point; raises if it is missing."""
-    return _open(LIB_PATH, SIGNATURES)
+    return _libs.get(LIB_PATH) or _open(LIB_PATH, SIGNATURES)
 
 
 def load_seq() -> C.CDLL:

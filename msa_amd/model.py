@@ -27,17 +27,20 @@ class MLP(nn.Module):
 
         self._joined = {}
 
-    def _gate_up(self, interleaved: bool):
+    def _gate_up(self, interleaved: bool, parts=None):
         """Gate and up rows in one matrix, behind one another or as the silu-mul epilogues take them; made again when either weight
         changes (one made in inference mode does not tell of changes in place)."""
-        parts = (self.gate_proj.weight, self.up_proj.weight)
-        key = tuple((w.data_ptr(), None if w.is_inference() else w._version, w.dtype, w.device) for w in parts)
+        gate, up = parts or (self.gate_proj.weight, self.up_proj.weight)
+        try:
+            key = (gate.data_ptr(), up.data_ptr(), gate._version, up._version, gate.dtype, gate.device)
+        except RuntimeError:                           # (it has no version either)
+            key = (gate.data_ptr(), up.data_ptr(), None, None, gate.dtype, gate.device)
         held = self._joined.get(interleaved)
         if held is None or held[0] != key:
-            gate, up = (w.detach() for w in parts)
+            gate, up = gate.detach(), up.detach()
             made = ops.interleave_gate_up(gate, up) if interleaved else torch.cat([gate, up], dim=0).contiguous()
             if held is not None and (held[1].shape, held[1].dtype, held[1].device) == (made.shape, made.dtype, made.device):
-                with torch.inference_mode():       # in place: a captured step reads this memory
+                with torch.inference_mode():           # in place: a captured step reads this memory
                     made = held[1].copy_(made)
             self._joined[interleaved] = held = (key, made)
         return held[1]
@@ -51,9 +54,9 @@ class MLP(nn.Module):
 
     def _activation(self, x):
         gate, up = self.gate_proj.weight, self.up_proj.weight
-        if gate.shape[0] % 8 == 0 and x.is_contiguous() and ops.tile_linear_ok(x, gate, 2) and ops.tile_linear_ok(x, up, 2):
-            return ops.tile_linear(x.view(-1, x.shape[-1]), self._gate_up(True), silu_mul=True).view(*x.shape[:-1], -1)
-        return ops.silu_mul(F.linear(x, self._gate_up(False)))
+        if ops.tile_linear_ok(x, gate, 2) and ops.tile_linear_ok(x, up, 2) and gate.shape[0] % 8 == 0 and x.is_contiguous():
+            return ops.tile_linear(x.view(-1, x.shape[-1]), self._gate_up(True, (gate, up)), silu_mul=True).view(*x.shape[:-1], -1)
+        return ops.silu_mul(F.linear(x, self._gate_up(False, (gate, up))))
 
     def add_to(self, residual, x):
         """``residual += self(x)`` (bf16 / fp32 on the GPU); a block of bf16 tokens has the add in the end of the second product, where the

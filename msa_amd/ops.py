@@ -24,10 +24,29 @@ def _stream(stream: Optional[torch.cuda.Stream] = None) -> int:
     return stream.cuda_stream if stream is not None else torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
-def scratch(need: int, device) -> Optional[torch.Tensor]:
+class _Scratch:
+    """Bytes of the caching allocator on the current stream, given back when the call that holds them returns (a tensor of them takes the
+    host 1.4 us, this 0.5)."""
+    __slots__ = ("at",)
+
+    def __init__(self, at: int):
+        self.at = at
+
+    def __del__(self, free=torch._C._cuda_cudaCachingAllocator_raw_delete):
+        free(self.at)
+
+    def data_ptr(self) -> int:
+        return self.at
+
+
+def scratch(need: int, device):
     """Scratch of one call, from the allocator each time: calls on other streams and threads have their own, and inside a capture it
     belongs to the graph, whose replays then share it with nothing."""
-    return torch.empty(need, dtype=torch.uint8, device=device) if need else None
+    if not need:
+        return None
+    if device.type != "cuda" or device.index != torch._C._cuda_getDevice():
+        return torch.empty(need, dtype=torch.uint8, device=device)
+    return _Scratch(torch._C._cuda_cudaCachingAllocator_raw_alloc(need, _stream()))
 
 
 def _need_cuda(*ts):
@@ -144,13 +163,15 @@ class Bank:
               "msa_bank_set_layer")
         self._keep[layer] = (kr, k_host, v_host)
 
-    def workspace(self, B: int, S: int, Hq: int, topk: int, device, chunk_plane: bool = False) -> torch.Tensor:
-        """Scratch for ``route_topk`` (pre-summed queries, row masks, one key per document, candidate lists);
+    def workspace_bytes(self, B: int, S: int, Hq: int, topk: int, chunk_plane: bool = False) -> int:
+        """Scratch of ``route_topk`` (pre-summed queries, row masks, one key per document, candidate lists);
         with ``chunk_plane`` also room for the ``[B, C]`` key plane ``chunk_scores`` needs."""
         lib = _lib.load()
-        need = (lib.msa_route_workspace_bytes(B, S, Hq, self.Hkv, self.D, self.C, self.n_docs, topk) if chunk_plane
+        return (lib.msa_route_workspace_bytes(B, S, Hq, self.Hkv, self.D, self.C, self.n_docs, topk) if chunk_plane
                 else lib.msa_route_topk_workspace_bytes(B, S, Hq, self.Hkv, self.D, self.n_docs, topk))
-        return scratch(need, device)
+
+    def workspace(self, B: int, S: int, Hq: int, topk: int, device, chunk_plane: bool = False) -> torch.Tensor:
+        return torch.empty(self.workspace_bytes(B, S, Hq, topk, chunk_plane), dtype=torch.uint8, device=device)
 
     def close(self):
         if getattr(self, "handle", None):
@@ -182,10 +203,11 @@ def chunk_scores(bank: Bank, layer: int, q: torch.Tensor, qmask: Optional[torch.
                  scale: float = 1.0) -> torch.Tensor:
     """fp32 ``[B, C]`` chunk scores (mean over heads, max over scored tokens)."""
     B, S, Hq, qm = _route_args(bank, q, qmask, mode)
-    ws = bank.workspace(B, S, Hq, 16, q.device, chunk_plane=True)
+    need = bank.workspace_bytes(B, S, Hq, 16, chunk_plane=True)
+    ws = scratch(need, q.device)
     out = torch.empty((B, bank.C), dtype=torch.float32, device=q.device)
     check(_lib.load().msa_chunk_scores(bank.handle, layer, ptr(q), ptr(qm), B, S, Hq, MODES[mode], scale, ptr(out),
-                                       ptr(ws), ws.numel(), _stream()), "msa_chunk_scores")
+                                       ptr(ws), need, _stream()), "msa_chunk_scores")
     return out
 
 
@@ -205,16 +227,16 @@ def route_topk(bank: Bank, layer: int, q: torch.Tensor, qmask: Optional[torch.Te
     scores = torch.empty((B, topk), dtype=torch.float32, device=q.device)
     doc = torch.empty((B, topk), dtype=torch.int32, device=q.device)
     gid = torch.empty((B, topk), dtype=torch.int64, device=q.device)
+    need = bank.workspace_bytes(B, S, Hq, topk, chunk_plane=chunk_reduce != "max")
+    ws = scratch(need, q.device)
     if query_reduce == "max" and chunk_reduce == "max":
-        ws = bank.workspace(B, S, Hq, topk, q.device)
         check(_lib.load().msa_route_topk(bank.handle, layer, ptr(q), ptr(qm), B, S, Hq, MODES[mode], scale, topk,
-                                         ptr(scores), ptr(doc), ptr(gid), ptr(ws), ws.numel(), _stream()),
+                                         ptr(scores), ptr(doc), ptr(gid), ptr(ws), need, _stream()),
               "msa_route_topk")
     else:
-        ws = bank.workspace(B, S, Hq, topk, q.device, chunk_plane=chunk_reduce != "max")
         check(_lib.load().msa_route_topk_reduce(bank.handle, layer, ptr(q), ptr(qm), B, S, Hq, MODES[mode], scale,
                                                 QUERY_REDUCE[query_reduce], CHUNK_REDUCE[chunk_reduce], topk, ptr(scores),
-                                                ptr(doc), ptr(gid), ptr(ws), ws.numel(), _stream()),
+                                                ptr(doc), ptr(gid), ptr(ws), need, _stream()),
               "msa_route_topk_reduce")
     return scores, doc, gid
 
@@ -256,9 +278,10 @@ def gather_kv_device(bank: Bank, layer: int, doc_sel: torch.Tensor, capacity_chu
     else:
         k_out, v_out = out
     cu = torch.empty(B + 1, dtype=torch.int32, device=dev)
-    ws = torch.empty(lib.msa_gather_device_workspace_bytes(B, k), dtype=torch.uint8, device=dev)
+    need = lib.msa_gather_device_workspace_bytes(B, k)
+    ws = scratch(need, dev)
     check(lib.msa_gather_kv_device(bank.handle, layer, ptr(doc_sel), B, k, ptr(k_out), ptr(v_out), capacity_chunks, ptr(cu),
-                                   ptr(ws), ws.numel(), _stream()), "msa_gather_kv_device")
+                                   ptr(ws), need, _stream()), "msa_gather_kv_device")
     return k_out, v_out, cu
 
 
@@ -275,7 +298,8 @@ def route_topk_gather(bank: Bank, layer: int, q: torch.Tensor, qmask: Optional[t
     gB, gk = gather_doc_sel.shape
     lib = _lib.load()
     dev = q.device
-    ws = bank.workspace(B, S, Hq, topk, dev)
+    need, gneed = bank.workspace_bytes(B, S, Hq, topk), lib.msa_gather_device_workspace_bytes(gB, gk)
+    ws, gws = scratch(need, dev), scratch(gneed, dev)
     scores = torch.empty((B, topk), dtype=torch.float32, device=dev)
     doc = torch.empty((B, topk), dtype=torch.int32, device=dev)
     gid = torch.empty((B, topk), dtype=torch.int64, device=dev)
@@ -285,10 +309,9 @@ def route_topk_gather(bank: Bank, layer: int, q: torch.Tensor, qmask: Optional[t
     else:
         k_out, v_out = out
     cu = torch.empty(gB + 1, dtype=torch.int32, device=dev)
-    gws = torch.empty(lib.msa_gather_device_workspace_bytes(gB, gk), dtype=torch.uint8, device=dev)
     check(lib.msa_route_topk_gather(bank.handle, layer, ptr(q), ptr(qm), B, S, Hq, MODES[mode], scale, topk, ptr(scores),
-                                    ptr(doc), ptr(gid), ptr(ws), ws.numel(), gather_layer, ptr(gather_doc_sel), gB, gk,
-                                    ptr(k_out), ptr(v_out), capacity_chunks, ptr(cu), ptr(gws), gws.numel(), _stream()),
+                                    ptr(doc), ptr(gid), ptr(ws), need, gather_layer, ptr(gather_doc_sel), gB, gk,
+                                    ptr(k_out), ptr(v_out), capacity_chunks, ptr(cu), ptr(gws), gneed, _stream()),
           "msa_route_topk_gather")
     return (scores, doc, gid), (k_out, v_out, cu)
 
@@ -420,10 +443,11 @@ def qkv_proj(x: torch.Tensor, w: torch.Tensor, Hq: int, Hkv: int, positions: tor
     k = torch.empty((T, Hkv, D), dtype=x.dtype, device=dev)
     v = torch.empty((T, Hkv, D), dtype=x.dtype, device=dev)
     r = torch.empty((T, router_front + router_back, D), dtype=x.dtype, device=dev) if router_front + router_back else None
-    ws = scratch(_lib.load().msa_tile_workspace_bytes(T, K, heads * D), dev)
+    need = _lib.load().msa_tile_workspace_bytes(T, K, heads * D)
+    ws = scratch(need, dev)
     check(_lib.load().msa_qkv_proj_ws(ptr(x), T, K, ptr(w), Hq, Hkv, router_front, router_back, ptr(positions), ptr(q_norm_w),
                                       ptr(k_norm_w), eps, ptr(rope[0]), ptr(rope[1]), rope[0].shape[0], ptr(q), ptr(k), ptr(v),
-                                      ptr(r), ptr(ws), 0 if ws is None else ws.numel(), _stream()), "msa_qkv_proj")
+                                      ptr(r), ptr(ws), need, _stream()), "msa_qkv_proj")
     return q, k, v, r
 
 
@@ -448,13 +472,14 @@ def tile_linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
         raise ValueError(f"tile_linear: out must be bf16 [{T}, {width}] on x's device with unit column stride")
     if not T:
         return out
-    ws = scratch(_lib.load().msa_tile_workspace_bytes(T, K, N), x.device)
+    need = _lib.load().msa_tile_workspace_bytes(T, K, N)
+    ws = scratch(need, x.device)
     mode = (_lib.TILE_ADD if add else _lib.TILE_SILU_MUL if silu_mul else _lib.TILE_GLU if glu is not None
             else _lib.TILE_GELU if gelu_n else _lib.TILE_STORE)
     end = _lib.TileEnd(mode, gelu_n, *(glu or (0.0, 0.0, 0.0)))
     rows = lambda t: t.stride(0) if T > 1 else t.shape[1]
-    check(_lib.load().msa_tile_linear(ptr(x), rows(x), T, K, ptr(w), N, C.byref(end), ptr(out), rows(out), ptr(ws),
-                                      0 if ws is None else ws.numel(), _stream()), "msa_tile_linear")
+    check(_lib.load().msa_tile_linear(ptr(x), rows(x), T, K, ptr(w), N, C.byref(end), ptr(out), rows(out), ptr(ws), need,
+                                      _stream()), "msa_tile_linear")
     return out
 
 
@@ -468,10 +493,11 @@ def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1) -> bool:
     tiles, 31 and 43; of 4096, 160 tiles, 50 and 51; of 16384, 640 tiles, 233 and 161; 2560 x 19456 of 1000, 304 tiles, 102 and 90), and
     padding does not count (2560 x 12288 of 573 tokens, 107 tiles' outputs in 144, 45 and 61).  Depths under 1024 were not measured and
     stay where they were."""
-    K, N = x.shape[-1], matrices * w.shape[0]
-    T = x.shape[0] if x.dim() == 2 else x.numel() // max(K, 1)
-    if T * N < TILE_MIN:                            # (most calls end here: steps of few tokens wait for the host)
+    N = matrices * w.shape[0]
+    K = x.shape[-1]
+    if x.numel() * N < TILE_MIN * K:                # (most calls end here: steps of few tokens wait for the host)
         return False
+    T = x.numel() // K
     return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == K
             and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 21))
             and K % 64 == 0 and 1024 <= K <= 32768 and N % 8 == 0 and N < 1 << 20 and T < 1 << 22
@@ -539,8 +565,9 @@ def embed_rows(table: torch.Tensor, tokens: torch.Tensor, f32: bool = False, wra
 
 
 def linear_ok(module: torch.nn.Module, x: torch.Tensor) -> bool:
-    return (type(module) is torch.nn.Linear and module.bias is None and x.is_contiguous() and type(module.weight) is torch.nn.Parameter
-            and tile_linear_ok(x, module.weight) and plain_module(module, torch.nn.Linear))
+    if type(module) is not torch.nn.Linear or not tile_linear_ok(x, module.weight):
+        return False
+    return module.bias is None and x.is_contiguous() and type(module.weight) is torch.nn.Parameter and plain_module(module, torch.nn.Linear)
 
 
 def linear(module: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:

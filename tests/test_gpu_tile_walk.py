@@ -51,7 +51,7 @@ def _call(ops, x, w, out, mode, gelu_n=0, glu=(0.0, 0.0, 0.0), pieces=True):
     from msa_amd import _lib
     (T, K), N = x.shape, w.shape[0]
     end = _lib.TileEnd(mode, gelu_n, *glu)
-    ws = ops.scratch(_lib.load().msa_tile_workspace_bytes(T, K, N), "cuda") if pieces else None
+    ws = torch.empty(_lib.load().msa_tile_workspace_bytes(T, K, N), dtype=torch.uint8, device="cuda") if pieces else None
     ops.check(_lib.load().msa_tile_linear(ops.ptr(x), K, T, K, ops.ptr(w), N, C.byref(end), ops.ptr(out), out.shape[1], ops.ptr(ws),
                                           0 if ws is None else ws.numel(), ops._stream()), "msa_tile_linear")
     return out
