@@ -62,7 +62,7 @@ class MLP(nn.Module):
         """``residual += self(x)`` (bf16 / fp32 on the GPU); a block of bf16 tokens has the add in the end of the second product, where the
         sum is rounded once."""
         act = self._activation(x)
-        if ops.linear_ok(self.down_proj, act) and residual.is_contiguous() and residual.dtype == x.dtype and residual.shape == x.shape \
+        if ops.linear_ok(self.down_proj, act, end=True) and residual.is_contiguous() and residual.dtype == x.dtype and residual.shape == x.shape \
                 and residual.device == x.device and residual.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and residual.requires_grad):
             ops.tile_linear(act.view(-1, act.shape[-1]), self.down_proj.weight, out=residual.view(-1, x.shape[-1]), add=True)
             return residual

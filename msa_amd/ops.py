@@ -51,10 +51,11 @@ def scratch(need: int, device):
 
 def _need_cuda(*ts):
     for t in ts:
-        if t is not None and not t.is_cuda:
+        if t is None or (t.is_cuda and t.is_contiguous()):
+            continue
+        if not t.is_cuda:
             raise ValueError("expected a device tensor (the HIP path has no CPU fallback)")
-        if t is not None and not t.is_contiguous():
-            raise ValueError("expected a contiguous tensor")
+        raise ValueError("expected a contiguous tensor")
 
 
 # ------------------------------------------------------------------------------ chunk table
@@ -387,7 +388,7 @@ def sparse_attn(q, k, v, kv_off, kv_len, max_kv: int, cu_q=None, max_sq: int = 1
     ws = scratch(need, q.device)
     out = torch.empty_like(q)
     check(lib.msa_sparse_attn(ptr(q), ptr(cu_q), ptr(k), ptr(v), ptr(kv_off), ptr(kv_len), B, total_q, max_sq, max_kv,
-                              Hq, Hkv, D, dtype_code(q.dtype), D ** -0.5 if scale is None else scale, int(causal),
+                              Hq, Hkv, D, dtype_code(q.dtype), sc, int(causal),
                               ptr(out), ptr(ws), need, _stream()), "msa_sparse_attn")
     return out
 
@@ -483,19 +484,22 @@ def tile_linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
     return out
 
 
-TILE_MIN = 144 << 16    # outputs (144 tiles of 256 x 256) from which tile_linear is at least the vendor's equal
+TILE_MIN = 144 << 16    # outputs (144 tiles of 256 x 256) from which tile_linear with an end is at least the equal of the vendor's two launches
+TILE_PLAIN = 256 << 16  # without one, where the vendor's tiles fit the columns
 TILE_ROWS = 256         # no matrix of the models has outputs enough for fewer rows
 
 
-def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1) -> bool:
-    """Whether ``x [..., K] @ w.T`` (``matrices`` of w's shape in one) is ``tile_linear``'s: operands as it takes them, no gradients asked
-    for, and outputs enough to fill the compute units.  Below ``TILE_MIN`` the vendor's smaller tiles win (us, vendor and here, K x N: 2560 x 2560 of 2048 tokens, 80
-    tiles, 31 and 43; of 4096, 160 tiles, 50 and 51; of 16384, 640 tiles, 233 and 161; 2560 x 19456 of 1000, 304 tiles, 102 and 90), and
-    padding does not count (2560 x 12288 of 573 tokens, 107 tiles' outputs in 144, 45 and 61).  Depths under 1024 were not measured and
-    stay where they were."""
+def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1, end: bool = True) -> bool:
+    """Whether ``x [..., K] @ w.T`` (``matrices`` of w's shape in one; with an ``end`` besides the store) is ``tile_linear``'s: operands as it
+    takes them, no gradients asked for, and outputs enough to fill the compute units.  us in a loop of 60 ms, the vendor's (and its second
+    launch) and here, rows x K x N: with an end 573 x 2560 x 19456 glu and 1600 x 1024 x 6144 glu level, 900 x 2560 x 19456 1.06 times, 6001 1.26
+    times the speed; without one and N no multiple of 256 1600 x 1024 x 6176 1.10, 900 x 2560 x 14944 1.17 times.  Where N is one, a single
+    round of tiles is behind the vendor's smaller ones (6001 x 9728 x 2560 199 and 217, 6001 x 4096 x 2560 86 and 93, 10000 x 3072 x 1024 53 and
+    63), and several are level or ahead (7000 x 2560 x 2560 1.14 times, 6001 x 4096 x 12288 1.28, but 4096 x 2560 x 6144 0.87).  Padding does not
+    count.  Depths under 1024 were not measured and stay where they were."""
     N = matrices * w.shape[0]
     K = x.shape[-1]
-    if x.numel() * N < TILE_MIN * K:                # (most calls end here: steps of few tokens wait for the host)
+    if x.numel() * N < (TILE_MIN if end or N % 256 else TILE_PLAIN) * K:      # (most calls end here: steps of few tokens wait for the host)
         return False
     T = x.numel() // K
     return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == K
@@ -564,8 +568,8 @@ def embed_rows(table: torch.Tensor, tokens: torch.Tensor, f32: bool = False, wra
     return (out, wide) if f32 else out
 
 
-def linear_ok(module: torch.nn.Module, x: torch.Tensor) -> bool:
-    if type(module) is not torch.nn.Linear or not tile_linear_ok(x, module.weight):
+def linear_ok(module: torch.nn.Module, x: torch.Tensor, end: bool = False) -> bool:
+    if type(module) is not torch.nn.Linear or not tile_linear_ok(x, module.weight, end=end):
         return False
     return module.bias is None and x.is_contiguous() and type(module.weight) is torch.nn.Parameter and plain_module(module, torch.nn.Linear)
 

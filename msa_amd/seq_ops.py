@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import ctypes as C
 from dataclasses import dataclass
+from functools import lru_cache
 from typing import Optional, Sequence
 
 import numpy as np
@@ -201,7 +202,7 @@ def clamped_glu(gu: torch.Tensor, limit: float, alpha: float = GLU_ALPHA, shift:
 
 def product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x @ w.T`` of a step's rows."""
-    if x.shape[0] >= ops.TILE_ROWS and ops.tile_linear_ok(x, w):
+    if x.shape[0] >= ops.TILE_ROWS and ops.tile_linear_ok(x, w, end=False):
         return ops.tile_linear(x, w)
     return ops.block_linear(x, w) if ops.block_linear_ok(x, w) else F.linear(x, w)
 
@@ -335,10 +336,12 @@ def delta(qkv, a, b, gate, A_log, dt_bias, norm, eps: float, H: int, G: int, D: 
     return out
 
 
-# Heads of all sequences up to which a decode step forms the low rank's second product beside its state: a workgroup a head, one a
-# compute unit.  A whole step, us, product apart and here: 16 heads 188.7 and 186.1, 128 (1b) 214.2 and 210.0, 256 (1b) 240.0 and 232.9,
-# (4b) 448.1 and 441.4; 512 498 and 521 (its registers leave one workgroup a compute unit instead of two).
-DELTA_STEP_HEADS = 256
+@lru_cache(maxsize=None)
+def delta_step_heads(device: torch.device) -> int:
+    """Heads of all sequences up to which a decode step forms the low rank's second product beside its state: a workgroup a head, one a
+    compute unit.  A whole step, us, product apart and here: 16 heads 188.7 and 186.1, 128 (1b) 214.2 and 210.0, 256 (1b) 240.0 and 232.9,
+    (4b) 448.1 and 441.4; 512 498 and 521 (its registers leave one workgroup a compute unit instead of two)."""
+    return torch.cuda.get_device_properties(device).multi_processor_count
 
 
 def delta_step(qkv, a_low, g_low, w_low, n_a: int, b, A_log, dt_bias, norm, eps: float, H: int, G: int, D: int, E: int, state,

@@ -81,7 +81,7 @@ def test_an_mlp_with_a_call_of_its_own(gpu):
         y = layer(h, None, None, None, None)
         return (y.float() - (x + gpu.rmsnorm(x, layer.input_layernorm.weight, 1e-6) * 0.5).float())
     base = added()
-    assert gpu.linear_ok(own.down_proj, torch.empty((1, 9600, 3072), device="cuda").bfloat16())
+    assert gpu.linear_ok(own.down_proj, torch.empty((1, 9600, 3072), device="cuda").bfloat16(), end=True)
     # (rounding the stream to bf16 leaves 2^-9 of values some ten times the MLP's, three times over)
     close = lambda got, times: ((got - times * base).norm() / base.norm()).item() < 0.06 * max(1, times)
     layer.mlp = tripled
@@ -151,10 +151,61 @@ class _On:
 def test_operands_of_different_devices(monkeypatch):
     from msa_amd import ops
     x, w = _On("cuda:0", 8192, 2048), _On("cuda:0", 4096, 2048)
-    assert ops.tile_linear_ok(x, w)
+    assert ops.tile_linear_ok(x, w) and ops.tile_linear_ok(x, w, end=False)
     assert not ops.tile_linear_ok(x, _On("cuda:1", 4096, 2048))
+    # without an end a round of whole tiles is the vendor's, unless its tiles do not fit the columns either
+    few = _On("cuda:0", 4000, 2048)
+    assert ops.tile_linear_ok(few, w) and not ops.tile_linear_ok(few, w, end=False)
+    assert ops.tile_linear_ok(few, _On("cuda:0", 3000, 2048), end=False)
     monkeypatch.setattr(ops, "_need_cuda", lambda *a: None)
     with pytest.raises(ValueError, match="device"):
         ops.tile_linear(x, _On("cuda:1", 4096, 2048))
     with pytest.raises(ValueError, match="device"):
         ops.tile_linear(x, w, out=_On("cuda:1", 8192, 4096))
+
+
+def _err(got, want):
+    return ((got.float() - want).norm() / want.norm()).item()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,K,N", [(2500, 1024, 8192), (2500, 1024, 5136), (1900, 1024, 4096)])
+def test_products_of_a_step(gpu, monkeypatch, T, K, N):
+    """The decoders' products against fp32 where the tiled form takes them (the first two; the third with the vendor's or the small tiles'):
+    one rounding to bf16, 1.7e-3 over many values; three for the gated unit and gelu, the gate's passed on by up to 1.3 (4e-3)."""
+    taken = []
+    inner = gpu.tile_linear
+    monkeypatch.setattr(gpu, "tile_linear", lambda x, w, **k: (taken.append(sorted(k)), inner(x, w, **k))[1])
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn((T, K + 32), generator=g, device="cuda").bfloat16()[:, 8:K + 8]
+    w = (torch.randn((N, K), generator=g, device="cuda") * K ** -0.5).bfloat16()
+    want = x.float() @ w.float().t()
+    assert _err(seq_ops.product(x, w), want) < 3e-3
+    n = N // 2 // 128 * 128 + 8
+    act = torch.nn.functional.gelu(want[:, :n], approximate="tanh")
+    got = seq_ops.product_gelu(x, w, n)
+    assert _err(got[:, :n], act) < 4e-3 and _err(got[:, n:], want[:, n:]) < 3e-3
+    gate, up = want[:, 0::2].clamp(max=1.5), want[:, 1::2].clamp(-1.5, 1.5)
+    got = seq_ops.product_glu(x, w, 1.5)
+    assert _err(got, gate * torch.sigmoid(seq_ops.GLU_ALPHA * gate) * (up + seq_ops.GLU_SHIFT)) < 4e-3
+    assert taken == ([[], ["gelu_n"], ["glu"]] if T * N >= gpu.TILE_MIN else [])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 300, 1400, 1700, 9300])
+def test_mlp(gpu, T):
+    """Both sides of the lines of the two products, before and after an update of a weight in place.  The activation and the output are
+    rounded to bf16, and the gate and up sums may be: four roundings, each of 1.7e-3 over many values."""
+    from msa_amd.config import MSAConfig
+    from msa_amd.model import MLP
+    print(f"[routes] mlp T={T}", flush=True)
+    torch.manual_seed(T)
+    m = MLP(MSAConfig(hidden_size=1024, intermediate_size=3072)).cuda().bfloat16().requires_grad_(False)
+    x, base = torch.randn((1, T, 1024), device="cuda").bfloat16(), torch.randn((1, T, 1024), device="cuda").bfloat16()
+    for _ in range(2):
+        gate, up, down = (p.weight.float() for p in (m.gate_proj, m.up_proj, m.down_proj))
+        want = (torch.nn.functional.silu(x.float() @ gate.t()) * (x.float() @ up.t())) @ down.t()
+        assert _err(m(x), want) < 5e-3
+        out = base.clone()
+        assert m.add_to(out, x).data_ptr() == out.data_ptr() and _err(out, base.float() + want) < 5e-3
+        m.up_proj.weight.mul_(-1.5)
