@@ -244,19 +244,20 @@ def extra_decode(dev):
 
 
 def extra_mfma_ceiling(dev):
-    """What the matrix cores sustain with nothing but MFMAs running (a register-only loop at the scoring kernel's
-    occupancy): the rate with operands that toggle is the ceiling the scoring kernel's fraction can be read against."""
+    """What the matrix cores sustain with nothing but MFMAs running (register-only loops): the rate with operands that toggle in the
+    scoring kernel's form, 16 x 16 x 32, is the ceiling its fraction can be read against."""
     from msa_amd import _lib
     lib = _lib.load()
     wgs, iters = 256 * 4, 20000
     sink = torch.empty(wgs * 512, dtype=torch.float32, device=dev)
     flops = C.c_double(0)
-    out = {"workload": f"register-only v_mfma_f32_32x32x16_bf16 loop, {wgs} workgroups x 8 wavefronts x {iters} x 8 MFMAs"}
+    out = {"workload": f"register-only v_mfma_f32_32x32x16_bf16 loop, {wgs} workgroups x 8 wavefronts x {iters} x 8 MFMAs "
+                       f"(16x16x32: x 32 MFMAs of half the products)"}
     # mode + 16 * extra: other VALU work per 8 MFMAs (what the attention kernel's softmax asks of the issue port)
     for mode, name in ((0, "zero_operands"), (2, "toggling_operands"), (16, "zero_operands_plus_24_fma"),
                        (32, "zero_operands_plus_48_fma"), (48, "zero_operands_plus_24_exp"), (64, "zero_operands_plus_48_exp"),
                        (80, "zero_operands_plus_24_cvt_pk_bf16"), (96, "zero_operands_plus_24_dot2c_bf16"),
-                       (112, "zero_operands_plus_24_max3")):
+                       (112, "zero_operands_plus_24_max3"), (256, "zero_operands_16x16x32"), (258, "toggling_operands_16x16x32")):
         ms = []
         for rep in range(3):
             a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)

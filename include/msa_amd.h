@@ -154,8 +154,8 @@ int msa_profile_enable(int32_t max_records);
 int msa_profile_collect(float* ms_host, int32_t cap, int32_t* n_out);
 
 /* Measurement aid (no counterpart in the reference): a register-only loop of v_mfma_f32_32x32x16_bf16, 8 wavefronts
- * per workgroup with a 4 x 2 grid of accumulators each (the scoring kernel's shape and occupancy), `iters`
- * iterations of 8 MFMAs per wavefront, enqueued on `stream`.  mode 0: zero operands; 1: operands of ones (every
+ * per workgroup with a 4 x 2 grid of accumulators each, `iters` iterations of 8 MFMAs per wavefront, enqueued on
+ * `stream`.  mode 0: zero operands; 1: operands of ones (every
  * sink[thread] then holds 128 * iters exactly); 2: operands whose signs and mantissas change every iteration, which is
  * what the shader clock under real data answers to.  sink: device float [workgroups * 512]; *flops_out (host, may be
  * null) receives the launch's floating-point operations.  The rate of mode 2 is the ceiling of this GPU's matrix
@@ -163,7 +163,9 @@ int msa_profile_collect(float* ms_host, int32_t cap, int32_t* n_out);
  * mode + 16 * extra adds other VALU work per iteration of 8 MFMAs, on registers of its own (sink is then not
  * defined): extra 1 / 2: 24 / 48 v_fma_f32; 3 / 4: 24 / 48 v_exp_f32; 5: 24 v_cvt_pk_bf16_f32; 6: 24 v_dot2c_f32_bf16;
  * 7: 24 v_max3_f32.  The rates tell what each instruction costs on the SIMD's issue port next to the products
- * (the budget of a kernel that does softmax arithmetic between them). */
+ * (the budget of a kernel that does softmax arithmetic between them).
+ * 256 + mode: the same operands in v_mfma_f32_16x16x32_bf16, 8 x 4 blocks a wavefront and 32 MFMAs an iteration, the routing scan's form
+ * (ones: 1024 * iters in every sink[thread]). */
 int msa_diag_mfma_loop(int32_t workgroups, int32_t iters, int32_t mode, float* sink, double* flops_out, void* stream);
 
 /* Measurement aid (no counterpart in the reference): loops that only read `bytes` of device memory at `src`, taken

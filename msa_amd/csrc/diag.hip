@@ -10,7 +10,8 @@ typedef float floatx16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 512;          // 8 wavefronts, two per SIMD: the scoring kernel's occupancy
-constexpr int kMfmasPerIter = 8;       // a 4 x 2 grid of 32 x 32 accumulators per wavefront, as in the scoring kernel
+constexpr int kMfmasPerIter = 8;       // a 4 x 2 grid of 32 x 32 accumulators per wavefront
+constexpr int kForm16 = 256;           // modes from here on: the 16 x 16 x 32 form
 
 // mode 0: zero operands; 1: all ones (the result is known exactly: 16 per MFMA); 2: operands whose mantissas and signs
 // change from one iteration to the next (what a GEMM on real data presents to the multipliers).
@@ -83,6 +84,49 @@ __global__ __launch_bounds__(kThreads) void mfma_loop_kernel(int32_t iters, int3
 #pragma unroll
     for (int i = 0; i < 24; ++i) s += x[i] * 1e-30f;
   }
+  sink[tid] = s;
+}
+
+// The same in 16 x 16 x 32 form, the routing scan's and the tiled products': 8 x 4 blocks of 16 x 16 a wavefront.
+constexpr int kMfmas16PerIter = 32;
+__global__ __launch_bounds__(kThreads) void mfma16_loop_kernel(int32_t iters, int32_t mode, float* __restrict__ sink) {
+  const uint32_t tid = blockIdx.x * kThreads + threadIdx.x;
+  u32x4_t a[8], b[4];
+  uint32_t seed = tid * 2654435761u + 12345u;
+  auto word = [&]() -> uint32_t {
+    if (mode == 0) return 0u;
+    if (mode == 1) return 0x3f803f80u;                       // two bf16 ones
+    seed = seed * 1664525u + 1013904223u;
+    return (seed & 0x807f807fu) | 0x3f803f80u;               // random sign and mantissa, exponent of 1.0
+  };
+#pragma unroll
+  for (int i = 0; i < 8; ++i) a[i] = u32x4_t{word(), word(), word(), word()};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) b[j] = u32x4_t{word(), word(), word(), word()};
+  const uint32_t flip = mode == 2 ? 0x00550055u : 0u;        // mantissa bits that toggle every iteration
+  typedef float floatx4_t __attribute__((ext_vector_type(4)));
+  floatx4_t acc[8][4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  for (int it = 0; it < iters; ++it) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[i]),
+                                                            __builtin_bit_cast(bf16x8_t, b[j]), acc[i][j], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[i] ^= flip;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b[j] ^= flip;
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s += acc[i][j][0];
   sink[tid] = s;
 }
 
@@ -180,9 +224,15 @@ extern "C" int msa_diag_read_stream(const void* src, int64_t bytes, void* dst, i
 extern "C" int msa_diag_mfma_loop(int32_t workgroups, int32_t iters, int32_t mode, float* sink, double* flops_out,
                                   void* stream) {
   MSA_REQUIRE(workgroups > 0 && workgroups <= 65536 && iters > 0 && iters <= (1 << 24), "msa_diag_mfma_loop: bad sizes");
+  hipStream_t st = as_stream(stream);
+  if (mode >= kForm16 && mode <= kForm16 + 2 && sink != nullptr) {
+    mfma16_loop_kernel<<<workgroups, kThreads, 0, st>>>(iters, mode - kForm16, sink);
+    MSA_LAUNCH_CHECK();
+    if (flops_out) *flops_out = (double)workgroups * (kThreads / 64) * (double)iters * kMfmas16PerIter * (2.0 * 16 * 16 * 32);
+    return MSA_OK;
+  }
   const int operands = mode & 15, extra = mode >> 4;          // mode = operands + 16 * extra VALU work
   MSA_REQUIRE(mode >= 0 && operands <= 2 && extra <= 7 && sink != nullptr, "msa_diag_mfma_loop: bad mode / null sink");
-  hipStream_t st = as_stream(stream);
   switch (extra) {
     case 0: mfma_loop_kernel<0><<<workgroups, kThreads, 0, st>>>(iters, operands, sink); break;
     case 1: mfma_loop_kernel<1><<<workgroups, kThreads, 0, st>>>(iters, operands, sink); break;

@@ -190,7 +190,8 @@ __global__ __launch_bounds__(kMaxWaves * 64) void skinny_linear_kernel(
 
 // The line to the form of rows_ring.h (us here and there, one / sixteen rows): 3072 x 1280 3.7 / 4.6 and 4.5 / 5.1, 6144 x 1280 5.5 / 6.1
 // and 5.8 / 6.3, 4096 x 1024 3.6 / 4.3 and 3.9 / 4.3; 2560 x 2560 5.1 / 7.2 and 5.3 / 6.4, 2560 x 2048 4.7 / 5.9 and 4.5 / 5.4,
-// 9728 x 1024 7.4 / 8.4 and 6.3 / 6.7.
+// 9728 x 1024 7.4 / 8.4 and 6.3 / 6.7.  Longer rows than kMaxResidentK have no line of their own: with sixteen
+// rows, plain and ring, 6144 x 9728 32.3 and 27.4, 7168 x 5632 22.6 and 19.4, 6400 x 8192 30.4 and 23.5, 8176 x 9728 37.6 and 31.8.
 constexpr int64_t kRingWeights = 5 << 20;
 bool takes_ring(int32_t N, int32_t K, bool norm) {
   return K > rows_ring::kMinK && rows_ring::busy_weights(N, K) >= kRingWeights && (!norm || K <= rows_ring::kMaxResidentK);

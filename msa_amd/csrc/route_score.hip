@@ -797,10 +797,11 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void score_gemm_kernel(
 // stands behind an MFMA.  128 x 128 wavefront tiles read a third less from LDS per product than a 2 x 4 layout of eight
 // wavefronts.
 //
-// What bounds it is power: the clock falls until the chip is inside its budget, so what counts is energy per product.
-// v_mfma_f32_16x16x32_bf16 passes an accumulator half as often for the same products as v_mfma_f32_32x32x16_bf16: a loop of
-// nothing but MFMAs on random operands holds 2070 TFLOP/s with the first and 1800 with the second (2440 and 2480 on zeros), and
-// 1.605M chunks x 2048 query rows take 4.25 ms here, 4.66 with the 32 x 32 x 16 form (1.58 and 1.45 PFLOP/s).
+// What bounds it is power: the clock falls until the chip is inside its budget (matrix cores busy 0.84 of the cycles at 1.5 - 1.75 GHz,
+// of 2.4), so what counts is energy per product.  v_mfma_f32_16x16x32_bf16 passes an accumulator half as often for the same products as
+// v_mfma_f32_32x32x16_bf16: 1.605M chunks x 2048 query rows take 4.25 ms here, 4.66 with the 32 x 32 x 16 form (1.58 and 1.45
+// PFLOP/s).  A loop of nothing but MFMAs (msa_diag_mfma_loop) shows part of that: 1953 TFLOP/s against 1886 with operands that
+// change; on zeros, which cost little power, the larger form is the faster one (2213 and 2449).
 //
 // Persistent: one workgroup per compute unit walks its share of the tile list (scan_walk.h) as one sequence of K
 // steps, the loads two steps ahead across tile boundaries.  With a gather job attached the last workgroup of the

@@ -624,6 +624,21 @@ def test_mfma_loop_diagnostic_counts_exactly():
 
 
 @pytest.mark.gpu
+def test_mfma_loop_of_small_blocks_counts_exactly():
+    """The 16 x 16 x 32 form: with operands of ones every MFMA adds 32 to each accumulator element, thirty-two accumulators a wavefront."""
+    from msa_amd import _lib
+    lib = _lib.load()
+    wgs, iters = 3, 50
+    sink = torch.zeros(wgs * 512, dtype=torch.float32, device="cuda")
+    flops = C.c_double(0)
+    st = torch.cuda.current_stream().cuda_stream
+    _lib.check(lib.msa_diag_mfma_loop(wgs, iters, 256 + 1, sink.data_ptr(), C.byref(flops), st), "msa_diag_mfma_loop")
+    torch.cuda.synchronize()
+    assert bool((sink == 32 * 32 * iters).all()) and flops.value == wgs * 8 * iters * 32 * 2 * 16 * 16 * 32
+    assert lib.msa_diag_mfma_loop(wgs, iters, 256 + 3, sink.data_ptr(), None, st) != 0
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("seed", [1, 2, 3])
 def test_route_topk_mid_size_banks_with_the_tile_pool(seed):
     """Random mid-size banks (130k - 300k chunks, 9 - 24 queries of 64 - 200 tokens, 4 or 8 KV heads, ragged masks, both
