@@ -499,7 +499,7 @@ def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1, end: boo
     count.  Depths under 1024 were not measured and stay where they were."""
     N = matrices * w.shape[0]
     K = x.shape[-1]
-    if x.numel() * N < (TILE_MIN if end or N % 256 else TILE_PLAIN) * K:      # (most calls end here: steps of few tokens wait for the host)
+    if x.numel() * N < (TILE_MIN if end or N % 256 else TILE_PLAIN) * max(K, 1):   # (most calls end here: steps of few tokens wait for the host)
         return False
     T = x.numel() // K
     return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == K

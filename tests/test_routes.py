@@ -164,6 +164,14 @@ def test_operands_of_different_devices(monkeypatch):
         ops.tile_linear(x, w, out=_On("cuda:1", 8192, 4096))
 
 
+@pytest.mark.parametrize("rows", [0, 1, 300])
+def test_products_of_no_depth(rows):
+    from msa_amd import ops
+    x, w = torch.zeros((rows, 0)), torch.zeros((5, 0))
+    assert not ops.tile_linear_ok(x, w) and not ops.tile_linear_ok(x[None], w, 2) and not ops.block_linear_ok(x, w)
+    assert seq_ops.product(x, w).shape == (rows, 5)
+
+
 def _err(got, want):
     return ((got.float() - want).norm() / want.norm()).item()
 
