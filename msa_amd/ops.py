@@ -46,7 +46,7 @@ def scratch(need: int, device):
         return None
     if device.type != "cuda" or device.index != torch._C._cuda_getDevice():
         return torch.empty(need, dtype=torch.uint8, device=device)
-    return _Scratch(torch._C._cuda_cudaCachingAllocator_raw_alloc(need, _stream()))
+    return _Scratch(torch._C._cuda_cudaCachingAllocator_raw_alloc(need, torch._C._cuda_getCurrentRawStream(device.index)))
 
 
 def _need_cuda(*ts):
@@ -515,19 +515,22 @@ CAPTURED_US, CAPTURED_ROWS, CAPTURED_DEPTH = 12.5, 1024, 2048
 
 def block_linear_ok(x: torch.Tensor, w: torch.Tensor, end: bool = False) -> bool:
     """Whether ``x [T, K] @ w.T`` (with an ``end``: behind which the vendor's product needs another launch) is ``block_linear``'s: operands
-    as it takes them, no gradients asked for, and about as fast there or faster.  The host takes about 21 us to hand a product to the vendor's library and 7 to this, so up to ``BLOCK_ROWS`` rows, where a prompt waits for
-    the host, products of about that length are here also where the vendor's kernel alone is a little faster (us, the vendor's and here,
-    rows x K x N: 64 x 1024 x 1024 6.6 and 5.0, 1000 x 1024 x 6176 24.2 and 20.5, 2048 x 1024 x 4096 20.6 and 22; behind the line 300 x 2560 x 8192, 25.8
-    and 27.4).  Of more rows those of a depth up to ``BLOCK_DEPTH`` (6001 x 128 x 4096 25.9 and 18.5; 8192 x 256 x 2048 16.7 and 19.0).  A captured
+    as it takes them, no gradients asked for, and about as fast there or faster.  The host takes about 21 us to hand a product to the
+    vendor's library and 7 to this, so up to ``BLOCK_ROWS`` rows, where a prompt waits for the host, products of about that length are here
+    also where the vendor's kernel alone is a little faster (us, the vendor's and here, rows x K x N: 64 x 1024 x 1024 6.6 and 5.0, 1000 x
+    1024 x 6176 24.2 and 20.5, 2048 x 1024 x 4096 20.6 and 22; behind the line 300 x 2560 x 8192, 25.8 and 27.4).  Of more rows those of a depth up to ``BLOCK_DEPTH`` (6001 x 128 x 4096 25.9 and 18.5; 8192 x 256 x 2048 16.7 and 19.0).  A captured
     call pays for no host: there the kernels alone decide (17 x 1024 x 6176 9.0 and 5.7, 64 x 1024 x 1024 7.0 and 5.4, 1000 x 2048 x 1024 11.8
     and 11.0; behind the lines 32 x 2560 x 2560 7.7 and 9.9, 17 x 4096 x 2560 11.8 and 13.8, 1500 x 128 x 4096 9.0 and 10.4, 573 x 1024 x 8192
     16.4 and 21.0)."""
     (T, K), N = (x.shape if x.dim() == 2 else (0, 0)), w.shape[0]
-    return (T > 0 and w.dim() == 2 and x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] == K
-            and K % 64 == 0 and 64 <= K <= 32768 and N % 16 == 0 and 0 < N < 1 << 20 and T < 1 << 22 and (T <= BLOCK_ROWS or K <= BLOCK_DEPTH)
-            and (_lib.load().msa_block_linear_us(T, K, N) <= BLOCK_US if end or not torch.cuda.is_current_stream_capturing() else
-                 T <= CAPTURED_ROWS and K <= CAPTURED_DEPTH and _lib.load().msa_block_linear_us(T, K, N) <= CAPTURED_US)
-            and (x.is_contiguous() or (x.stride(1) == 1 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 21))
+    if not (T > 0 and w.dim() == 2 and x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] == K
+            and K % 64 == 0 and 64 <= K <= 32768 and N % 16 == 0 and 0 < N < 1 << 20 and T < 1 << 22 and (T <= BLOCK_ROWS or K <= BLOCK_DEPTH)):
+        return False
+    us = _lib.load().msa_block_linear_us(T, K, N)
+    if us > BLOCK_US or (not end and (us > CAPTURED_US or T > CAPTURED_ROWS or K > CAPTURED_DEPTH)
+                         and torch.cuda.is_current_stream_capturing()):
+        return False
+    return ((x.is_contiguous() or (x.stride(1) == 1 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 21))
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.device == x.device
             and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
 
