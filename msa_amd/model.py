@@ -59,8 +59,8 @@ class MLP(nn.Module):
         return ops.silu_mul(F.linear(x, self._gate_up(False, (gate, up))))
 
     def add_to(self, residual, x):
-        """``residual += self(x)`` (bf16 / fp32 on the GPU); a block of bf16 tokens has the add in the end of the second product, where the
-        sum is rounded once."""
+        """``residual += self(x)`` (bf16 / fp32 on the GPU) where the module's call is this class's (``ops.plain_module``); a block of bf16
+        tokens has the add in the end of the second product, where the sum is rounded once."""
         act = self._activation(x)
         if ops.linear_ok(self.down_proj, act, end=True) and residual.is_contiguous() and residual.dtype == x.dtype and residual.shape == x.shape \
                 and residual.device == x.device and residual.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and residual.requires_grad):
