@@ -4,7 +4,7 @@
 // the same loads; splits are merged by a second kernel.  K / V rows are [Hkv, 128].  Two forms: bf16 rows go through a ring in LDS and
 // the matrix cores (attn_ring_kernel, below), fp32 rows and some bf16 rows of one and two heads through the vector units
 // (attn_partial_kernel; takes_ring in attn_internal.h has the line).  In the latter a wavefront takes 4 keys per step (16 lanes per
-// key, 8 head-dim elements per lane); every (key slot, dim slice) lane keeps an online-softmax state (m, l, acc[G][8]) of its own that
+// key, 8 head-dim elements per lane: dim_of); every (key slot, dim slice) lane keeps an online-softmax state (m, l, acc[G][8]) of its own that
 // is merged across slots and wavefronts.
 #include "attn_internal.h"
 
@@ -32,9 +32,17 @@ __device__ __forceinline__ void ld8(const bf16_t* p, float (&x)[8]) {
   x[4] = bf16lo(w.z); x[5] = bf16hi(w.z); x[6] = bf16lo(w.w); x[7] = bf16hi(w.w);
 }
 __device__ __forceinline__ void ld8(const float* p, float (&x)[8]) {
-  const uint4 a = ld16_stream(p), b = ld16_stream(p + 4);
+  const uint4 a = ld16_stream(p), b = ld16_stream(p + kHeadDim / 2);
   x[0] = __uint_as_float(a.x); x[1] = __uint_as_float(a.y); x[2] = __uint_as_float(a.z); x[3] = __uint_as_float(a.w);
   x[4] = __uint_as_float(b.x); x[5] = __uint_as_float(b.y); x[6] = __uint_as_float(b.z); x[7] = __uint_as_float(b.w);
+}
+
+// Lane j of the 16 that share a key holds eight of its dimensions, in the pieces of 16 bytes that it loads: neighbours in bf16; of an fp32
+// row four in either half, so that the lanes' pieces are whole cache lines (eight neighbours are two loads that touch every second piece:
+// with non-temporal loads a line came twice from memory, 16 samples of 2926 to 4388 keys 140 -> 105 us).
+template <typename T>
+__device__ __forceinline__ constexpr int dim_of(int j, int i) {
+  return sizeof(T) == 2 ? 8 * j + i : 4 * j + (i & 3) + (i >> 2) * (kHeadDim / 2);
 }
 
 // The same of any float: the rotary tables need not be aligned.
@@ -69,20 +77,17 @@ __device__ __forceinline__ float row16_allsum(float d) {
   return d;
 }
 
-__device__ const uint4 kZeros[2] = {};
+__device__ const uint4 kZeros[(kHeadDim / 2 + 4) / 4] = {};             // what ld8 reaches of a float
 
 // Streams keys first, first + stride, ... < key1 of one KV head through the running softmax state of this
 // lane (key slot = lane / 16, dims 8 j .. 8 j + 8).  Keys go in batches of kBatch steps: all K / V loads of a
 // batch are issued before any arithmetic (bytes in flight), scores are reduced over the 16 lanes of a key with
 // DPP row rotations, and the running softmax is rescaled once per batch.  `lane_off` is the element offset of
 // key 0's slice for this lane.
-template <typename T, int G>
+template <typename T, int G, int kBatch>
 __device__ __forceinline__ void attend_keys(const T* __restrict__ k, const T* __restrict__ v, int64_t lane_off,
                                             int row_elems, int first, int key1, int stride, const float (&qv)[G][8],
                                             float (&m)[G], float (&l)[G], float (&acc)[G][8]) {
-  // (fp32: with one head twice the bytes in flight are worth their registers, 16 samples of 3000 keys 98 -> 75 us; with four they cost
-  // a wavefront a SIMD, 16 of 4388 131 -> 158)
-  constexpr int kBatch = sizeof(T) == 4 && G == 1 ? 8 : 4;
   for (int kb = first; kb < key1; kb += stride * kBatch) {
     float kx[kBatch][8], vx[kBatch][8];
     bool ok[kBatch];
@@ -406,7 +411,8 @@ __device__ __forceinline__ void merge_slots(float& m, float& l, float (&acc)[8])
   }
 }
 
-// fp32 rows, and bf16 rows of groups of one and two heads where takes_ring says so.
+// fp32 rows, and bf16 rows of groups of one and two heads where takes_ring says so.  A workgroup serves G heads, of a group of G or of a
+// larger one whose rows are then read once a workgroup.
 template <typename T, int G, int kAttnWaves>
 __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
     const T* __restrict__ q, const int32_t* __restrict__ cu_q, const T* __restrict__ k, const T* __restrict__ v,
@@ -416,7 +422,10 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
   __shared__ float sm_m[kAttnWaves][G], sm_l[kAttnWaves][G];
   __shared__ float sm_acc[kAttnWaves][G][kHeadDim];
 
-  const int row = blockIdx.x, g = blockIdx.y, split = blockIdx.z;
+  // (fp32: with one head twice the bytes in flight are worth their registers, 16 samples of 3000 keys 98 -> 75 us; with four they cost
+  // a wavefront a SIMD, 16 of 4388 131 -> 158)
+  constexpr int kBatch = sizeof(T) == 4 && G == 1 && kAttnWaves <= 8 ? 8 : 4;
+  const int row = blockIdx.x, h0 = blockIdx.y * G, g = h0 / (Hq / Hkv), split = blockIdx.z;
   const int b = cu_q ? find_sample(cu_q, B, row) : row;
   const int q_first = cu_q ? cu_q[b] : row;
   const int sq = cu_q ? cu_q[b + 1] - q_first : 1;
@@ -439,8 +448,8 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[h][i] = 0.f;
   }
-  const int64_t lane_off = base * row_elems + g * kHeadDim + 8 * j;     // this lane's slice of key 0
-  const T* q_lane = q + ((int64_t)row * Hq + g * G) * kHeadDim + 8 * j;
+  const int64_t lane_off = base * row_elems + g * kHeadDim + dim_of<T>(j, 0);     // this lane's slice of key 0
+  const T* q_lane = q + ((int64_t)row * Hq + h0) * kHeadDim + dim_of<T>(j, 0);
   float qv[G][8];
 #pragma unroll
   for (int h = 0; h < G; ++h) {
@@ -448,7 +457,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) qv[h][i] *= scale_log2e;      // scores in log2 units: exp2f below
   }
-  attend_keys<T, G>(k, v, lane_off, row_elems, key0 + wave * 4 + slot, key1, kAttnWaves * 4, qv, m, l, acc);
+  attend_keys<T, G, kBatch>(k, v, lane_off, row_elems, key0 + wave * 4 + slot, key1, kAttnWaves * 4, qv, m, l, acc);
 
   // merge the 4 key slots of the wavefront (lanes differing in bits 4 and 5): a swap leaves both lanes' values in both, without LDS
 #pragma unroll
@@ -461,7 +470,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
     for (int h = 0; h < G; ++h) {
       if (j == 0) { sm_m[wave][h] = m[h]; sm_l[wave][h] = l[h]; }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) sm_acc[wave][h][8 * j + i] = acc[h][i];
+      for (int i = 0; i < 8; ++i) sm_acc[wave][h][dim_of<T>(j, i)] = acc[h][i];
     }
   }
   __syncthreads();
@@ -479,7 +488,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
       lt += sm_l[w][h] * a;
       at += sm_acc[w][h][d] * a;
     }
-    const int64_t o = ((int64_t)row * Hq + g * G + h) * n_split + split;
+    const int64_t o = ((int64_t)row * Hq + h0 + h) * n_split + split;
     if (n_split == 1) {                                  // nothing to merge: the output itself (a launch of 4 us less)
       const float y = lt > 0.f ? at / lt : 0.f;          // a row that sees no key yields zeros
       if constexpr (sizeof(T) == 2) out[o * kHeadDim + d] = f32_to_bf16(y);
@@ -668,13 +677,26 @@ int launch_combine(const float* part_ml, const float* part_acc, int64_t rows, in
   return MSA_OK;
 }
 
+// Heads a workgroup of fp32 rows where whole groups would leave most of the chip idle; 0: whole groups.  A group's workgroups read its rows
+// again, from the caches, which costs less than its heads one after another as long as the workgroups do not outnumber the compute units
+// (`head_splits`: with one head each; twice as many with two).  More than two splits are short already.  us, 8 KV heads of four, groups
+// / two heads / one: one row of 192 keys 11.4 / 9.0 / 8.1, 8 rows 12.5 / 8.6 / 7.3, 16 rows 13.5 / 9.5 / 12.2, 32 rows 15.3 / 15.4 /
+// 21.9; 2 rows of 400 keys in two splits 14.5 / 11.3 / 11.2, of 1000 in four 15.2 / 12.2 / 14.8, of 2000 in eight 16.2 / 15.6 / 25.3; 4 rows
+// of 2000 19.3 / 26.8 / 32.8.
+int spread_heads(int64_t head_splits, int G, int n_split) {
+  constexpr int kUnits = 256;
+  if (head_splits <= kUnits && n_split <= 2) return 1;
+  return G >= 2 && head_splits <= 2 * kUnits ? 2 : 0;
+}
+
 template <typename T>
 int launch_attn(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                     const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
                     int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st) {
   const int n_split = plan.n_split;
-  const int G = Hq / Hkv;
-  dim3 grid((unsigned)total_q, (unsigned)Hkv, (unsigned)n_split);
+  const int spread = sizeof(T) == 4 ? spread_heads((int64_t)total_q * Hq * n_split, Hq / Hkv, n_split) : 0;
+  const int G = spread ? spread : Hq / Hkv;
+  dim3 grid((unsigned)total_q, (unsigned)(Hq / G), (unsigned)n_split);
   const float sl2 = scale * 1.4426950408889634f;
 #define MSA_ATTN_CASE(GG, WW)                                                                                      \
   case GG:                                                                                                         \
@@ -683,6 +705,12 @@ int launch_attn(const void* q, const int32_t* cu_q, const void* k, const void* v
         Hkv, sl2, causal, n_split, part_ml, part_acc, static_cast<T*>(out));                                       \
     return MSA_OK;
   const auto first = [&] {
+    if constexpr (sizeof(T) == 4) {
+      if (spread) switch (G) {
+          MSA_ATTN_CASE(1, 8)
+          MSA_ATTN_CASE(2, 8)
+        }
+    }
     switch (G) {
       MSA_ATTN_CASE(1, 4)
       MSA_ATTN_CASE(2, 4)
