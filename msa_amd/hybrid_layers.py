@@ -166,13 +166,8 @@ class LatentAttention:
         if batch.max_rows <= self.ABSORB_ROWS or not seq_ops.flash_ok(q.dtype, c.dim, c.vdim, c.scale) or proj.stride(0) % 8:
             return self._absorbed(q, cache, batch)
         ends = [p + n for p, n in zip(batch.positions, batch.counts)]
-        if batch.n_seq == 1:
-            lat, off = cache[batch.slots[0], :ends[0]], [0]
-        else:
-            lat = torch.cat([cache[s, :e] for s, e in zip(batch.slots, ends)])
-            off = [sum(ends[:i]) for i in range(batch.n_seq)]
-        return seq_ops.flash(q, seq_ops.product(lat, self.uk), seq_ops.product(lat, self.uv),
-                             torch.tensor(off, dtype=torch.int64).to(q.device), self.sink, c.scale, c.heads, batch)
+        lat = cache[batch.slots[0], :ends[0]] if batch.n_seq == 1 else torch.cat([cache[s, :e] for s, e in zip(batch.slots, ends)])
+        return seq_ops.flash(q, seq_ops.product(lat, self.uk), seq_ops.product(lat, self.uv), batch.key_off, self.sink, c.scale, c.heads, batch)
 
     def decode(self, w, hs, h, state, batch):
         c, n_b = self.c, self.w_in.shape[0]

@@ -87,8 +87,11 @@ class StepBatch:
             host.append(host[-1] + c)
         zeros = torch.zeros(self.rows, dtype=torch.int32, device=device) if n == 1 else None      # (in front of the copy, which may wait)
         many = [] if n == 1 else [np.repeat(np.arange(n, dtype=np.int32), self.counts)]
-        self.cu, self.slot, self.pos, *rest = upload(device, [np.asarray(host, np.int32), np.asarray(self.slots, np.int32),
-                                                              np.asarray(self.positions, np.int64), *many, *extra], wait)
+        # where a sequence's keys begin if all keys up to the step's end lie one sequence behind the other (uploaded with the rest: a copy
+        # of its own inside a layer would hold the host up until the device is there)
+        ends = np.asarray(self.positions, np.int64) + np.asarray(self.counts, np.int64)
+        self.cu, self.slot, self.pos, self.key_off, *rest = upload(device, [np.asarray(host, np.int32), np.asarray(self.slots, np.int32),
+                                                                            np.asarray(self.positions, np.int64), np.cumsum(ends) - ends, *many, *extra], wait)
         self.row_seq = rest.pop(0) if many else zeros
         self.extra = rest
         self.c = _lib.SeqBatch(ptr(self.cu), ptr(self.row_seq), ptr(self.slot), ptr(self.pos), n, self.rows, self.max_rows, 0)

@@ -73,3 +73,12 @@ def test_pinned_memory_outlives_the_copies():
     batches = [seq_ops.StepBatch([2, 3], [i, i + 1], [i, 0], "cuda", extra[i], wait=False) for i in range(40)]
     for i, b in enumerate(batches):
         check(b, [2, 3], [i, i + 1], [i, 0], extra[i])
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_offsets_of_keys_one_sequence_behind_the_other(device):
+    for counts, pos in (([1], [0]), ([5], [7]), ([3, 1, 4], [0, 2 ** 33, 9]), ([1] * 16, list(range(16)))):
+        b = seq_ops.StepBatch(counts, list(range(len(counts))), pos, device)
+        ends = [p + c for p, c in zip(pos, counts)]
+        assert b.key_off.tolist() == [sum(ends[:s]) for s in range(len(counts))]
+        assert b.key_off.dtype == torch.int64 and b.key_off.device == b.pos.device and b.key_off.data_ptr() % 8 == 0
