@@ -644,16 +644,34 @@ int launch_finish(const TileArgs& a, const Plan& p, hipStream_t st) {
   return MSA_OK;
 }
 
+// An end under the next tile's steps wants tiles of kFlowSteps steps, and gelu's line between two wavefronts' rows.
+bool flows(const TileArgs& a, int mode) {
+  return mode != kAdd && mode != kHeads && a.K >= 64 * kFlowSteps && a.ldo < ((int64_t)1 << 21) && (mode != kGelu || a.end.gelu_n % 128 == 0);
+}
+
+// The columns that fill whole rounds, where the others are better off in block_gemm.hip's smaller tiles (N: none).  A few tiles behind the
+// last whole round take a launch most of another one, whole or in pieces: `last`, fitted to 16 to 128 such tiles, 1024 and 2560 deep (less: not measured).  us,
+// rows x K x N, all tiles and split: 8192 x 1024 x 6176 (32 columns' tiles a fourth round) 98 and 87, x 2304 52 and 42, 6001 x 1024 x 3072 50
+// and 43, 8192 x 2560 x 4608 165 and 153, x 12368 442 and 431; level or behind, and not split: 8192 x 1024 x 3072 54 and 58, 6001 x 1024 x
+// 6176 74 and 76, x 2560 x 8480 204 and 205, 1700 x 2560 x 19456 glu 143 and 147.  The ends round their sums alike in both kernels where the tiles' end flows.
+int whole_columns(const TileArgs& a, int mode) {
+  if ((mode != kStore && mode != kGelu && mode != kGlu) || (mode != kStore && !flows(a, mode)) || a.K < 1024) return a.N;
+  const int tiles_t = (a.T + kTile - 1) / kTile, tiles_n = (a.N + kTile - 1) / kTile;
+  const int units = std::max(kXcds * 2, device_compute_units() / kXcds * kXcds), rounds = (int)((int64_t)tiles_t * tiles_n / units);
+  const int columns = (int)((int64_t)rounds * units / tiles_t), behind = (int)((int64_t)tiles_t * tiles_n - (int64_t)rounds * units);
+  if (behind == 0 || columns < 1 || columns >= tiles_n) return a.N;
+  const float last = std::min(1.2f * (float)(a.K / 64), 6.f + 0.45f * (float)behind);
+  return 1.35f * msa_block_linear_us(a.T, a.K, a.N - columns * kTile) < last ? columns * kTile : a.N;
+}
+
 template <int kMode>
 int launch_tiles(TileArgs a, const Plan& p, hipStream_t st) {
   // Half of the memory-side cache: an output within it is still there for its reader (a 32771-token encoding block through two layers
   // takes 11.98 ms with all outputs non-temporal, 11.89 with none, 11.87 with the large ones).
   a.stream = (int64_t)a.T * a.N * (is_pair(kMode) ? 1 : 2) > (int64_t)128 << 20;
   a.tiles_t = p.tiles_t; a.tiles_n = p.tiles_n; a.group = p.group; a.split = p.split; a.max_rem = p.max_rem;
-  // An end under the next tile's steps wants tiles of kFlowSteps steps, and gelu's line between two wavefronts' rows.
-  constexpr bool kFlows = kMode != kAdd && kMode != kHeads;
-  if constexpr (kFlows) {
-    if (a.K >= 64 * kFlowSteps && a.ldo < ((int64_t)1 << 21) && (kMode != kGelu || a.end.gelu_n % 128 == 0)) {
+  if constexpr (kMode != kAdd && kMode != kHeads) {
+    if (flows(a, kMode)) {
       a.rate = -1.4426950408889634f * a.end.alpha;
       const int rc = a.stream ? launch_tile_kernel<tile_flow_kernel<kMode, true>>(a, p, st) : launch_tile_kernel<tile_flow_kernel<kMode, false>>(a, p, st);
       return rc != MSA_OK || p.split == 1 ? rc : launch_finish<kMode, kMode != kStore>(a, p, st);
@@ -692,8 +710,15 @@ extern "C" int msa_tile_linear(const void* x, int64_t ldx, int64_t T, int32_t K,
   TileArgs a{};
   a.x = static_cast<const bf16_t*>(x); a.w = static_cast<const bf16_t*>(w); a.out = static_cast<bf16_t*>(out);
   a.ldx = ldx; a.ldo = ldo; a.T = (int32_t)T; a.K = K; a.N = N; a.end = *end;
-  Plan p = make_plan(T, K, N, ws != nullptr);
-  if (p.bytes > ws_bytes || ((uintptr_t)ws & 15)) p = make_plan(T, K, N, false);
+  if (const int n = whole_columns(a, mode); n < N) {
+    a.N = n;
+    msa_tile_end rest = *end;
+    rest.gelu_n = std::max(0, end->gelu_n - n);
+    a.end.gelu_n = std::min(end->gelu_n, n);
+    if (const int rc = msa_block_linear(x, ldx, T, K, a.w + (int64_t)n * K, N - n, &rest, a.out + (mode == kGlu ? n / 2 : n), ldo, stream)) return rc;
+  }
+  Plan p = make_plan(T, K, a.N, ws != nullptr);
+  if (p.bytes > ws_bytes || ((uintptr_t)ws & 15)) p = make_plan(T, K, a.N, false);
   a.pieces = static_cast<float*>(ws);
   switch (mode) {
     case kStore: return launch_tiles<kStore>(a, p, as_stream(stream));
