@@ -71,6 +71,15 @@ __device__ __forceinline__ float quad_xor(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kPerm, 0xf, 0xf, false));
 }
 
+// The sum over the lanes 16, 32 and 48 away, in the order (own + 16) + (32 + 48).
+__device__ __forceinline__ float lanes_sum(float v) {
+  uint32_t u = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  u = __float_as_uint(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+  const auto t = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+}
+
 __device__ __forceinline__ uint32_t lds_offset(const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
 __device__ __forceinline__ u32x4_t lds_read16(uint32_t at) {
   u32x4_t v;
@@ -236,8 +245,7 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
         }
       asm volatile("" : "+v"(xf[u][0]), "+v"(xf[u][1]), "+v"(ssq));      // (one unit unpacked at a time)
     }
-    ssq += __shfl_xor(ssq, 16);
-    ssq += __shfl_xor(ssq, 32);
+    ssq = lanes_sum(ssq);
     if (g == 0) row_ssq[wave * 16 + n_l] = ssq;              // read behind the first barrier
   }
   if constexpr (kPro == kPost) {
@@ -252,15 +260,18 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
           const float lo = bf16lo(xf[u][h][c]), hi = bf16hi(xf[u][h][c]);
           ssq += lo * lo + hi * hi;
         }
-    ssq += __shfl_xor(ssq, 16);
-    ssq += __shfl_xor(ssq, 32);
+    ssq = lanes_sum(ssq);
     const uint32_t row_at = lds_offset(row_ssq + n_l * 16);
     asm volatile("ds_write_b32 %0, %1\n\ts_waitcnt vmcnt(%2) lgkmcnt(0)\n\ts_barrier" ::"v"(row_at + 4 * wave), "v"(ssq), "n"(2 * kSlots) : "memory");
+    u32x4_t p[4];
+    if constexpr (NU < kMaxPost)
+      asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:16\n\tds_read_b128 %2, %4 offset:32\n\tds_read_b128 %3, %4 offset:48\n\t"
+                   "s_waitcnt lgkmcnt(0)" : "=&v"(p[0]), "=&v"(p[1]), "=&v"(p[2]), "=&v"(p[3]) : "v"(row_at) : "memory");
     float total = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const u32x4_t p = lds_read16(row_at + 16 * i);
-      total += (__uint_as_float(p[0]) + __uint_as_float(p[1])) + (__uint_as_float(p[2]) + __uint_as_float(p[3]));
+      if constexpr (NU == kMaxPost) p[i] = lds_read16(row_at + 16 * i);                    // (no registers for all of them)
+      total += (__uint_as_float(p[i][0]) + __uint_as_float(p[i][1])) + (__uint_as_float(p[i][2]) + __uint_as_float(p[i][3]));
     }
     const float post_inv = 1.0f / sqrtf(total / (float)(row_bytes / 2) + a.eps);
 #pragma unroll
@@ -269,13 +280,17 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
       for (int h = 0; h < 2; ++h) {
         const int so = u * (kUnitBytes * kWaves) + h * 64;
         float v[8];
+        u32x4_t w[2];
+        const uint32_t w_at = lds_offset(norm_lds) + u * 2 * kUnitBytes + h * 128 + g * 32;
+        if constexpr (NU < kMaxPost)
+          asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:16\n\ts_waitcnt lgkmcnt(0)" : "=&v"(w[0]), "=&v"(w[1]) : "v"(w_at) : "memory");
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          const u32x4_t w = lds_read16(lds_offset(norm_lds) + u * 2 * kUnitBytes + h * 128 + g * 32 + i * 16);
+          if constexpr (NU == kMaxPost) w[i] = lds_read16(w_at + 16 * i);
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
             const uint32_t y = xf[u][h][2 * i + (c >> 1)];
-            v[4 * i + c] = __uint_as_float(px[u][h][i][c]) + (c & 1 ? bf16hi(y) : bf16lo(y)) * post_inv * __uint_as_float(w[c]);
+            v[4 * i + c] = __uint_as_float(px[u][h][i][c]) + (c & 1 ? bf16hi(y) : bf16lo(y)) * post_inv * __uint_as_float(w[i][c]);
           }
         }
         if (wg == 0 && n_l < a.M && x_col + so < row_bytes) {
