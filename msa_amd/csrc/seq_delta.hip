@@ -9,31 +9,14 @@
 // (norm and gate); otherwise head_norm_gate_kernel does.
 #include <algorithm>
 
-#include "seq_common.h"
+#include "seq_mfma.h"
 
 namespace {
 
 constexpr int kTok = 8;                  // tokens per stage
 
-// One 16-byte chunk's products of a weight row and its operand.
-__device__ __forceinline__ float dot8(const uint4& w, const uint4& x, float s) {
-  s += bf16lo(w.x) * bf16lo(x.x); s += bf16hi(w.x) * bf16hi(x.x);
-  s += bf16lo(w.y) * bf16lo(x.y); s += bf16hi(w.y) * bf16hi(x.y);
-  s += bf16lo(w.z) * bf16lo(x.z); s += bf16hi(w.z) * bf16hi(x.z);
-  s += bf16lo(w.w) * bf16lo(x.w); s += bf16hi(w.w) * bf16hi(x.w);
-  return s;
-}
-
-template <int kCtrl>
-__device__ __forceinline__ float add_moved(float v) {
-  return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kCtrl, 0xf, 0xf, false));
-}
-
-// kLow: the decays' and the gate's operands come through a low rank (`low`), whose second product is formed here: the head's D + E weight
-// rows, sixteen lanes a row, requested in front of everything else and multiplied when the state is on its way too.  A launch of 16 heads of
-// 64 x 128 takes 9.0 us so, 7.6 without, behind a product of 4.1.
-template <typename T, int NI, int RW, int CW, bool kLow = false>
-__global__ __launch_bounds__(RW * CW * 64) void delta_scan_kernel(msa_delta_args a, msa_seq_batch b, msa_delta_low low = {}) {
+template <typename T, int NI, int RW, int CW>
+__global__ __launch_bounds__(RW * CW * 64) void delta_scan_kernel(msa_delta_args a, msa_seq_batch b) {
   constexpr int kD = NI * RW, kCols = CW * 64, kWaves = RW * CW;
   __shared__ __align__(16) float ks[kTok][kD], qs[kTok][kD], gs[kTok][kD];
   __shared__ float beta[kTok], kq[kTok];
@@ -54,22 +37,6 @@ __global__ __launch_bounds__(RW * CW * 64) void delta_scan_kernel(msa_delta_args
   const T* ap = static_cast<const T*>(a.a) + (int64_t)lo * a.a_stride + (int64_t)head * a.D;
   const T* bp = static_cast<const T*>(a.b) + (int64_t)lo * a.b_stride + head;
   const T* gp = static_cast<const T*>(a.gate) + (int64_t)lo * a.gate_stride + (int64_t)head * a.E;
-  __shared__ float low_out[kLow ? kD + kCols : 1];
-  constexpr int kLowRows = RW * CW * 4, kTurns = kLow ? (kD + kCols + kLowRows - 1) / kLowRows : 1;      // weight rows at a time
-  [[maybe_unused]] uint4 lw[kTurns], lx[kTurns];
-  auto fetch_low = [&](int u) {                            // unit u of the lane's rows 0 .. kD (decays) .. kD + kCols (gate)
-#pragma unroll
-    for (int i = 0; i < kTurns; ++i) {
-      const int r = i * kLowRows + (tid >> 4);
-      const bool gate = r >= kD, in = u < low.rank / 8 && (gate ? r - kD < a.E : r < a.D);
-      const int64_t row = gate ? low.n_a + (int64_t)head * a.E + (r - kD) : (int64_t)head * a.D + r;
-      const bf16_t* x = gate ? static_cast<const bf16_t*>(low.g_low) + (int64_t)lo * low.g_stride
-                             : static_cast<const bf16_t*>(low.a_low) + (int64_t)lo * low.a_stride;
-      lw[i] = in ? reinterpret_cast<const uint4*>(low.w)[row * (low.rank / 8) + u] : make_uint4(0, 0, 0, 0);
-      lx[i] = in ? reinterpret_cast<const uint4*>(x)[u] : make_uint4(0, 0, 0, 0);
-    }
-  };
-  if constexpr (kLow) fetch_low(tid & 15);
   constexpr int kEach = (kD + 63) / 64, kMine = (kTok + kWaves - 1) / kWaves;    // values of a lane, tokens of a wavefront in a stage
   // What a stage reads is requested together, and the first one's in front of the state: loads arrive in the order they are made,
   // and the vectors are ready by the time the state is there.
@@ -88,7 +55,7 @@ __global__ __launch_bounds__(RW * CW * 64) void delta_scan_kernel(msa_delta_args
         const bool in = i < a.D;
         k[m][j] = in ? to_f32<T>(kp[t * a.qkv_stride + i]) : 0.f;
         q[m][j] = in ? to_f32<T>(qp[t * a.qkv_stride + i]) : 0.f;
-        if constexpr (!kLow) x[m][j] = in ? to_f32<T>(ap[t * a.a_stride + i]) : 0.f;
+        x[m][j] = in ? to_f32<T>(ap[t * a.a_stride + i]) : 0.f;
       }
       bv[m] = to_f32<T>(bp[t * a.b_stride]);
     }
@@ -97,29 +64,10 @@ __global__ __launch_bounds__(RW * CW * 64) void delta_scan_kernel(msa_delta_args
   };
   fetch(0);
   const float out_w = live && whole ? a.norm[col] : 0.f;
-  float gate0 = 0.f;                                     // of the first token, all there is when decoding
-  if constexpr (!kLow) gate0 = live && whole ? to_f32<T>(gp[col]) : 0.f;
+  const float gate0 = live && whole ? to_f32<T>(gp[col]) : 0.f;        // of the first token, all there is when decoding
   float S[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) S[i] = live && rw * NI + i < a.D ? st[(int64_t)i * a.E] : 0.f;
-  if constexpr (kLow) {
-    float sum[kTurns] = {};
-    for (int u0 = 0; u0 < low.rank / 8; u0 += 16) {
-      if (u0 > 0) fetch_low(u0 + (tid & 15));
-#pragma unroll
-      for (int i = 0; i < kTurns; ++i) sum[i] = dot8(lw[i], lx[i], sum[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < kTurns; ++i) {
-      const float v = add_moved<0x140>(add_moved<0x141>(add_moved<0x4E>(add_moved<0xB1>(sum[i]))));
-      const int r = i * kLowRows + (tid >> 4);
-      if ((tid & 15) == 0 && r < kD + kCols) low_out[r] = v;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kEach; ++j) x[0][j] = lane + 64 * j < kD ? low_out[lane + 64 * j] : 0.f;
-    gate0 = low_out[kD + cl];
-  }
   for (int t0 = 0; t0 < n_tok; t0 += kTok) {
     const int rows = min(kTok, n_tok - t0);
     if (t0 > 0) fetch(t0);
@@ -233,6 +181,189 @@ __global__ __launch_bounds__(RW * CW * 64) void delta_scan_kernel(msa_delta_args
     if (live && rw * NI + i < a.D) st[(int64_t)i * a.E] = S[i];
 }
 
+// ---- One token a sequence, the decays' and the gate's operands through a low rank whose second product is formed here.
+//
+// A workgroup owns (sequence, head).  What it reads is cold, the state and the head's D + E weight rows 3 us away, and everything else is a
+// chain of a few sums: what bounds it is how soon all of that is requested, so no load stands in a branch (what lies outside a buffer reads
+// zero) or waits for more than the slot's number, and the code is one token's.  As the scan above with the low rank in front of it, unrolled
+// for eight tokens, 3400 cycles lay between its first request and the state's.  us, so and now: 1 / 16 sequences of 16 heads of 64 x 128, rank
+// 64, 10.6 / 13.2 and 6.3 / 8.4; 1 / 8 of 32 heads of 128 x 128, rank 128, 13.2 / 19.0 and 8.1 / 12.0 (twice the wavefronts, 16 rows each, 8.4 /
+// 12.0).  Whole steps with the low rank's product a launch of its own and here: 16 sequences 478 and 464 (4b), 242 and 221 (1b), 4 412 and 389.
+template <int kCtrl>
+__device__ __forceinline__ float add_moved(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kCtrl, 0xf, 0xf, false));
+}
+// The sum over sixteen lanes, and over a wavefront, in every lane.
+__device__ __forceinline__ float row_sum(float v) { return add_moved<0x140>(add_moved<0x141>(add_moved<0x4E>(add_moved<0xB1>(v)))); }
+__device__ __forceinline__ float wave_sum(float v) {
+  uint32_t u = __float_as_uint(row_sum(v));
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  u = __float_as_uint(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+  const auto t = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+}
+// One 16-byte chunk's products of a weight row and its operand.
+__device__ __forceinline__ float dot8(const u32x4_t& w, const u32x4_t& x, float s) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    s += bf16lo(w[i]) * bf16lo(x[i]);
+    s += bf16hi(w[i]) * bf16hi(x[i]);
+  }
+  return s;
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t bytes_rsrc(const void* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+__device__ __forceinline__ float load_bf16(__amdgpu_buffer_rsrc_t rs, int at) { return bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(rs, at, 0, 0)); }
+__device__ __forceinline__ float load_f32(__amdgpu_buffer_rsrc_t rs, int at) { return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0)); }
+
+// NI state rows a thread, RW wavefronts' shares of the rows, CW wavefronts of 64 value columns.
+template <int NI, int RW, int CW>
+__global__ __launch_bounds__(RW * CW * 64) void delta_step_kernel(msa_delta_args a, msa_seq_batch b, msa_delta_low low) {
+  constexpr int kD = NI * RW, kCols = CW * 64, kRows = RW * CW * 4;                       // kRows: weight rows at a time, sixteen lanes each
+  constexpr int kEach = (kD + 63) / 64, kTurnsA = (kD + kRows - 1) / kRows, kTurnsG = (kCols + kRows - 1) / kRows;
+  __shared__ __align__(16) float ks[kD], qs[kD], gs[kD];
+  __shared__ float low_out[kD + kCols], beta_kq[2];
+  __shared__ float2 part[RW][kCols];
+  const int head = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), cw = wave % CW, rw = wave / CW, col = cw * 64 + lane;
+  // (as many rows as sequences, none with more than one: nothing to look up in front of the first loads)
+  const bool dense = b.rows == b.n_seq;
+  const int row = dense ? s : b.cu[s], kvh = head / (a.H / a.G);
+  if (!dense && b.cu[s + 1] == row) return;
+  float* const st = a.state + ((int64_t)b.slot[s] * a.H + head) * a.D * a.E;
+  const bf16_t* const qkv = static_cast<const bf16_t*>(a.qkv) + row * a.qkv_stride;
+
+  const __amdgpu_buffer_rsrc_t rs_w = bytes_rsrc(static_cast<const bf16_t*>(low.w) + (int64_t)head * a.D * low.rank, a.D * low.rank * 2);
+  const __amdgpu_buffer_rsrc_t rs_g = bytes_rsrc(static_cast<const bf16_t*>(low.w) + (low.n_a + (int64_t)head * a.E) * low.rank, a.E * low.rank * 2);
+  const __amdgpu_buffer_rsrc_t rs_xa = bytes_rsrc(static_cast<const bf16_t*>(low.a_low) + row * low.a_stride, low.rank * 2);
+  const __amdgpu_buffer_rsrc_t rs_xg = bytes_rsrc(static_cast<const bf16_t*>(low.g_low) + row * low.g_stride, low.rank * 2);
+  u32x4_t wa[kTurnsA], wg[kTurnsG], xa, xg;
+  auto fetch_low = [&](int unit) {
+    const int at = (tid >> 4) * low.rank * 2 + unit * 16, end = unit * 8 < low.rank ? 0 : kOutside;        // (a row's end, not the next row)
+    xa = __builtin_amdgcn_raw_buffer_load_b128(rs_xa, unit * 16, 0, 0);
+    xg = __builtin_amdgcn_raw_buffer_load_b128(rs_xg, unit * 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < kTurnsA; ++i) wa[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, at + end, i * kRows * low.rank * 2, 0);
+#pragma unroll
+    for (int i = 0; i < kTurnsG; ++i) wg[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_g, at + end, i * kRows * low.rank * 2, 0);
+  };
+  // ---- everything is requested
+  float k[kEach], q[kEach], bias = 0.f;
+  const __amdgpu_buffer_rsrc_t rs_q = bytes_rsrc(qkv + (int64_t)kvh * a.D, a.D * 2), rs_k = bytes_rsrc(qkv + (int64_t)(a.G + kvh) * a.D, a.D * 2);
+#pragma unroll
+  for (int j = 0; j < kEach; ++j) {                        // (every wavefront: cheaper than a branch)
+    k[j] = load_bf16(rs_k, (lane + 64 * j) * 2);
+    q[j] = load_bf16(rs_q, (lane + 64 * j) * 2);
+  }
+  const float v = load_bf16(bytes_rsrc(qkv + 2LL * a.G * a.D + (int64_t)head * a.E, a.E * 2), col * 2);
+  const float bv = load_bf16(bytes_rsrc(static_cast<const bf16_t*>(a.b) + row * a.b_stride + head, 2), 0);
+  fetch_low(tid & 15);
+  bias = load_f32(bytes_rsrc(a.dt_bias + (int64_t)head * a.D, a.D * 4), tid * 4);
+  const float out_w = load_f32(bytes_rsrc(a.norm, a.E * 4), col * 4);
+  const __amdgpu_buffer_rsrc_t rs_s = bytes_rsrc(st, a.D * a.E * 4);
+  const int s_at = col < a.E ? (rw * NI * a.E + col) * 4 : kOutside;
+  float S[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) S[i] = load_f32(rs_s, s_at + i * a.E * 4);
+  __builtin_amdgcn_sched_barrier(0);
+  const float rate = -expf(a.A_log[head]);
+
+  // ---- unit vectors, and the low rank's second product
+  if (wave == 0) {
+    float kk = 0.f, qq = 0.f, dot = 0.f;
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+      kk += k[j] * k[j];
+      qq += q[j] * q[j];
+      dot += k[j] * q[j];
+    }
+    const float ki = 1.0f / sqrtf(wave_sum(kk) + 1e-6f), qi = 1.0f / (sqrtf((float)a.D) * sqrtf(wave_sum(qq) + 1e-6f));
+    dot = wave_sum(dot);
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+      const int i = lane + 64 * j;
+      if (i < kD) {
+        ks[i] = k[j] * ki;
+        qs[i] = q[j] * qi;
+      }
+    }
+    if (lane == 0) {
+      beta_kq[0] = sigmoid_f(bv);
+      beta_kq[1] = dot * ki * qi;
+    }
+  }
+  float sum[kTurnsA + kTurnsG] = {};
+  for (int u0 = 0;;) {
+#pragma unroll
+    for (int i = 0; i < kTurnsA; ++i) sum[i] = dot8(wa[i], xa, sum[i]);
+#pragma unroll
+    for (int i = 0; i < kTurnsG; ++i) sum[kTurnsA + i] = dot8(wg[i], xg, sum[kTurnsA + i]);
+    if ((u0 += 16) >= low.rank / 8) break;
+    fetch_low(u0 + (tid & 15));
+  }
+#pragma unroll
+  for (int i = 0; i < kTurnsA + kTurnsG; ++i) {
+    const float x = row_sum(sum[i]);
+    const int r = (i < kTurnsA ? i : i - kTurnsA) * kRows + (tid >> 4);
+    if ((tid & 15) == 0 && r < (i < kTurnsA ? kD : kCols)) low_out[(i < kTurnsA ? 0 : kD) + r] = x;
+  }
+  __syncthreads();
+  if (tid < kD) gs[tid] = tid < a.D ? expf(rate * softplus_f(low_out[tid] + bias)) : 0.f;
+  __syncthreads();
+
+  // ---- the rule
+  float rec = 0.f, read = 0.f;
+#pragma unroll
+  for (int i = 0; i < NI; i += 4) {
+    const float4 g4 = *reinterpret_cast<const float4*>(&gs[rw * NI + i]);
+    const float4 k4 = *reinterpret_cast<const float4*>(&ks[rw * NI + i]);
+    const float4 q4 = *reinterpret_cast<const float4*>(&qs[rw * NI + i]);
+    S[i] *= g4.x; rec += S[i] * k4.x; read += S[i] * q4.x;
+    S[i + 1] *= g4.y; rec += S[i + 1] * k4.y; read += S[i + 1] * q4.y;
+    S[i + 2] *= g4.z; rec += S[i + 2] * k4.z; read += S[i + 2] * q4.z;
+    S[i + 3] *= g4.w; rec += S[i + 3] * k4.w; read += S[i + 3] * q4.w;
+  }
+  part[rw][col] = make_float2(rec, read);
+  __syncthreads();
+  rec = read = 0.f;
+#pragma unroll
+  for (int w = 0; w < RW; ++w) {
+    const float2 x = part[w][col];
+    rec += x.x;
+    read += x.y;
+  }
+  const float beta = beta_kq[0], kq = beta_kq[1], u = beta * (v - rec), o = read + kq * u;
+#pragma unroll
+  for (int i = 0; i < NI; i += 4) {
+    const float4 k4 = *reinterpret_cast<const float4*>(&ks[rw * NI + i]);
+    S[i] += k4.x * u;
+    S[i + 1] += k4.y * u;
+    S[i + 2] += k4.z * u;
+    S[i + 3] += k4.w * u;
+  }
+#pragma unroll
+  for (int i = 0; i < NI; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(S[i]), rs_s, s_at + i * a.E * 4, 0, 0);
+
+  // ---- norm and gate of the output: the columns' sums of squares by the first share's wavefronts
+  __shared__ float squares[CW];
+  const float ssq = wave_sum(col < a.E ? o * o : 0.f);
+  if (CW > 1) {
+    if (rw == 0 && lane == 0) squares[cw] = ssq;
+    __syncthreads();
+  }
+  if (rw == 0 && col < a.E) {
+    float total = ssq;
+    if (CW > 1) {
+      total = squares[0];
+#pragma unroll
+      for (int w = 1; w < CW; ++w) total += squares[w];
+    }
+    static_cast<bf16_t*>(a.out)[((int64_t)row * a.H + head) * a.E + col] =
+        f32_to_bf16(o * (1.0f / sqrtf(total / (float)a.E + a.eps)) * out_w * sigmoid_f(low_out[kD + col]));
+  }
+}
+
 // Value columns of a workgroup.
 int column_block(int32_t D, int32_t E) { return E <= 64 || D > 256 ? 64 : 128; }
 
@@ -259,9 +390,9 @@ int launch_scan(const msa_delta_args& a, const msa_seq_batch& b, hipStream_t st)
 
 template <int NI, int RW>
 void launch_step(const msa_delta_args& a, const msa_delta_low& low, const msa_seq_batch& b, hipStream_t st) {
-  const dim3 grid(1, a.H, b.n_seq);
-  if (a.E <= 64) delta_scan_kernel<bf16_t, NI, RW, 1, true><<<grid, RW * 64, 0, st>>>(a, b, low);
-  else delta_scan_kernel<bf16_t, NI, RW, 2, true><<<grid, RW * 128, 0, st>>>(a, b, low);
+  const dim3 grid(a.H, b.n_seq);
+  if (a.E <= 64) delta_step_kernel<NI, RW, 1><<<grid, RW * 64, 0, st>>>(a, b, low);
+  else delta_step_kernel<NI, RW, 2><<<grid, RW * 128, 0, st>>>(a, b, low);
 }
 
 }  // namespace
@@ -282,8 +413,7 @@ extern "C" int msa_seq_delta_step(const msa_delta_args* args, const msa_delta_lo
   hipStream_t st = as_stream(stream);
   if (a.D <= 16) launch_step<4, 4>(a, *low, *batch, st);
   else if (a.D <= 32) launch_step<8, 4>(a, *low, *batch, st);
-  else if (a.D <= 64) launch_step<16, 4>(a, *low, *batch, st);
-  else if ((int64_t)a.H * batch->n_seq <= device_compute_units() / 2) launch_step<16, 8>(a, *low, *batch, st);
+  else if (a.D <= 64) launch_step<8, 8>(a, *low, *batch, st);
   else launch_step<32, 4>(a, *low, *batch, st);
   MSA_LAUNCH_CHECK();
   return MSA_OK;

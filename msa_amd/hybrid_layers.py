@@ -238,8 +238,7 @@ class ChannelDeltaMixer:
         out = seq_ops.rows_conv(hs, w, h, n_b, 0, self.taps, None, state["conv"], batch.slot)
         a_low, g_low = self._low(out)
         c = self.c
-        if c.heads * batch.n_seq <= seq_ops.delta_step_heads(out.device) and c.dim <= 128 and c.vdim <= 128 and out.stride(0) % 8 == 0 \
-                and out.data_ptr() % 16 == 0:
+        if c.dim <= 128 and c.vdim <= 128 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
             return seq_ops.delta_step(out[:, :c.conv_channels], a_low, g_low, self.w_low, self.n_a, out[:, self.b_at:self.b_at + c.heads],
                                       self.A_log, self.dt_bias, self.norm, self.eps, c.heads, c.kv_heads, c.dim, c.vdim, state["delta"],
                                       batch), out[:, n_b:]

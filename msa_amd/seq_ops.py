@@ -340,13 +340,6 @@ def delta(qkv, a, b, gate, A_log, dt_bias, norm, eps: float, H: int, G: int, D: 
 
 
 @lru_cache(maxsize=None)
-def delta_step_heads(device: torch.device) -> int:
-    """Heads of all sequences up to which a decode step forms the low rank's second product beside its state: a workgroup a head, one a
-    compute unit.  A whole step, us, product apart and here: 16 heads 188.7 and 186.1, 128 (1b) 214.2 and 210.0, 256 (1b) 240.0 and 232.9,
-    (4b) 448.1 and 441.4; 512 498 and 521 (its registers leave one workgroup a compute unit instead of two)."""
-    return torch.cuda.get_device_properties(device).multi_processor_count
-
-
 def delta_step(qkv, a_low, g_low, w_low, n_a: int, b, A_log, dt_bias, norm, eps: float, H: int, G: int, D: int, E: int, state,
                batch: StepBatch) -> torch.Tensor:
     """:func:`delta` for one bf16 token a sequence, D and E up to 128, with ``a = a_low @ w_low[:H D].T`` and

@@ -49,7 +49,7 @@ def test_embed_norm_is_lookup_and_residual_norm(ops, dtype, counts, W):
 
 
 @pytest.mark.parametrize("B,H,G,D,E,R", [(1, 16, 16, 64, 128, 64), (16, 4, 2, 128, 128, 128), (3, 2, 1, 16, 8, 8), (2, 3, 3, 24, 40, 136),
-                                         (5, 4, 4, 128, 64, 264), (1, 1, 1, 1, 1, 16), (70, 2, 1, 100, 120, 48)])
+                                         (5, 4, 4, 128, 64, 264), (1, 1, 1, 1, 1, 16), (70, 2, 1, 100, 120, 48), (16, 32, 16, 128, 128, 128)])
 def test_delta_step_with_its_low_rank(ops, B, H, G, D, E, R):
     """Against the fp32 rule on the products in fp32: the output's own rounding to bf16 (2^-9), the state's sums in another order."""
     _say(f"delta_step B={B} H={H} G={G} D={D} E={E} R={R}")
