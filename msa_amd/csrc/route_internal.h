@@ -25,7 +25,7 @@ struct RouteWorkspace {
   int32_t M_rows;       // B * S_pad
   int32_t topk_blocks;  // candidate lists per query
   int32_t mask_words;   // words of the scored-row bitmask, padded to whole M tiles
-  size_t off_qs;        // pre-summed queries [M_rows, Hkv * D]
+  size_t off_qs;        // pre-summed queries [M_rows, Hkv * D] (with `parts` six bytes a value: three bf16 parts of fp32)
   size_t off_row_bits;  // scored-row bitmask, one uint32 per 32 rows
   size_t off_key;       // uint32 [B, n_docs] (routing) or [B, C] (chunk scores): order-preserving keys of the unscaled scores
   size_t off_cand;      // uint64 [B, topk_blocks, kTopkMax] sorted candidates
@@ -39,7 +39,7 @@ static inline int32_t topk_blocks_for(int64_t n_docs) {
 }
 
 RouteWorkspace route_workspace_layout(int32_t B, int32_t S, int32_t Hkv, int32_t D, int64_t plane_cols, int64_t n_docs,
-                                      int32_t dtype);
+                                      int32_t dtype, bool parts = false);
 
 // query_reduce: MSA_QUERY_*; extra_plane_cols: words per query reserved behind the key plane (the per-document keys
 // of the chunk-mean reduction).

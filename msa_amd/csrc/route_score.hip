@@ -38,7 +38,30 @@ constexpr int kSchedCounterWords = 32;
 constexpr int kSchedMaxWorkgroups = 1024;
 constexpr size_t kSchedBytes = (size_t)(kSchedCounterWords + kSchedMaxWorkgroups) * sizeof(uint32_t);
 
-template <typename TIn, typename TOut>
+// Eight fp32 values as three bf16 operands whose sum they are: the first cut off (infinities stay, a NaN's remainder is one), the others
+// rounded, 8 + 9 + 8 bits or more together.
+template <bool kInfinite>
+__device__ __forceinline__ void split_three(const float (&x)[8], uint4 (&part)[3]) {
+  uint32_t w[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t a = __float_as_uint(x[2 * i]), b = __float_as_uint(x[2 * i + 1]);
+    const float a1 = __uint_as_float(a & 0xffff0000u), b1 = __uint_as_float(b & 0xffff0000u);
+    const float ra = kInfinite && x[2 * i] == a1 ? 0.f : x[2 * i] - a1, rb = kInfinite && x[2 * i + 1] == b1 ? 0.f : x[2 * i + 1] - b1;
+    w[0][i] = __builtin_amdgcn_perm(b, a, 0x07060302);
+    w[1][i] = pack_bf16x2(ra, rb);
+    w[2][i] = pack_bf16x2(ra - bf16lo(w[1][i]), rb - bf16hi(w[1][i]));
+  }
+#pragma unroll
+  for (int p = 0; p < 3; ++p) part[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
+}
+// Where score_parts_kernel's operands of the queries lie: 32 rows x 16 values of K, a part each, in the order of a wavefront's lanes.
+constexpr int kPartBytes = 1024, kPartStep = 3 * kPartBytes;
+__device__ __forceinline__ int64_t part_at(int row, int k, int K) {
+  return ((int64_t)(row >> 5) * (K / 16) + k / 16) * kPartStep + (row & 31) * 16 + (k & 8) * 64;
+}
+
+template <typename TIn, typename TOut, bool kParts = false>
 __global__ void presum_queries_kernel(const TIn* __restrict__ q, const uint8_t* __restrict__ qmask, int32_t B,
                                       int32_t S, int32_t S_pad, int32_t Hq, int32_t Hkv, int32_t normalize,
                                       TOut* __restrict__ qs, uint32_t* __restrict__ row_bits, int32_t mask_words,
@@ -115,6 +138,14 @@ __global__ void presum_queries_kernel(const TIn* __restrict__ q, const uint8_t* 
         for (int i = 0; i < 8; ++i) acc[i] += x[u][i] * inv;
       }
     }
+  }
+  if constexpr (kParts) {
+    uint4 part[3];
+    split_three<true>(acc, part);
+    char* to = reinterpret_cast<char*>(qs) + part_at(row, g * kHeadDim + 8 * j, Hkv * kHeadDim);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) *reinterpret_cast<uint4*>(to + p * kPartBytes) = part[p];
+    return;
   }
   TOut* o = qs + ((int64_t)row * Hkv + g) * kHeadDim + 8 * j;
   if constexpr (sizeof(TOut) == 2) {
@@ -1142,6 +1173,34 @@ __device__ __forceinline__ void request_slab(__amdgpu_buffer_rsrc_t rsrc, uint32
 #endif
 }
 
+// The maxima `best` of `queries` queries from q0 on, in the columns from n0 on, into the key plane.
+template <bool kDocMax>
+__device__ __forceinline__ void merge_best(uint32_t (*best)[kSplitCols], int queries, int q0, int n0, int C, int n_docs, int wave, int waves,
+                                           uint32_t* __restrict__ out_key, int32_t own_doc) {
+  const int lane = threadIdx.x & 63, l32 = lane & 31;
+  for (int base = wave * 64; base < queries * kSplitCols; base += waves * 64) {              // 32 lanes a query
+    const int i = base + lane, n = n0 + l32;
+    const bool in = i < queries * kSplitCols && n < C;
+    uint32_t key = in ? best[i / kSplitCols][l32] : 0u;
+    const int64_t row = q0 + i / kSplitCols;
+    if constexpr (kDocMax) {
+      // a document's chunks are neighbours: the first of its columns here takes their maximum (one atomic each would queue up where a
+      // few long documents meet many row blocks: 500 chunks of 16 documents x 1000 rows 215 us instead of 41)
+      const int32_t doc = in ? own_doc : -1;
+#pragma unroll
+      for (int o = 1; o < kSplitCols; o <<= 1) {
+        const uint32_t other = __shfl_down(key, o, kSplitCols);
+        const int32_t other_doc = __shfl_down(doc, o, kSplitCols);
+        if (l32 + o < kSplitCols && other_doc == doc) key = max(key, other);
+      }
+      const bool first = __shfl_up(doc, 1, kSplitCols) != doc || l32 == 0;
+      if (in && first && key != 0) atomicMax(&out_key[row * n_docs + doc], key);
+    } else {
+      if (in && key != 0) atomicMax(&out_key[row * C + n], key);
+    }
+  }
+}
+
 template <bool kDocMax, int kRing>
 __global__ __launch_bounds__(kSplitWaves * 64, 2) void score_split_kernel(const float* __restrict__ qs, const float* __restrict__ kr,
                                                                         const uint32_t* __restrict__ row_bits,
@@ -1198,6 +1257,7 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void score_split_kernel(const 
 #pragma unroll
   for (int i = 0; i < kRing; ++i) request();
   const int q0 = b0 / blocks_per_query;
+  const int32_t own_doc = kDocMax ? chunk_doc[min(n0 + l32, C - 1)] : 0;
   for (int i = tid; i < kSplitMaxBlocks * kSplitCols; i += kSplitWaves * 64) best[i / kSplitCols][i % kSplitCols] = 0u;
 #pragma unroll
   for (int i = 0; i < kStages; ++i) {
@@ -1248,28 +1308,156 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void score_split_kernel(const 
   }
   __builtin_amdgcn_s_waitcnt(0);                         // (nothing in flight when the workgroup ends)
   __syncthreads();
-  const int queries = b1 > b0 ? (b1 - 1) / blocks_per_query - q0 + 1 : 0;
-  for (int base = wave * 64; base < queries * kSplitCols; base += kSplitWaves * 64) {        // 32 lanes a query
-    const int i = base + lane, n = n0 + l32;
-    const bool in = i < queries * kSplitCols && n < C;
-    uint32_t key = in ? best[i / kSplitCols][l32] : 0u;
-    const int64_t row = q0 + i / kSplitCols;
-    if constexpr (kDocMax) {
-      // a document's chunks are neighbours: the first of its columns here takes their maximum (one atomic each would queue up where a
-      // few long documents meet many row blocks: 500 chunks of 16 documents x 1000 rows 215 us instead of 41)
-      const int32_t doc = in ? chunk_doc[n] : -1;
+  merge_best<kDocMax>(best, b1 > b0 ? (b1 - 1) / blocks_per_query - q0 + 1 : 0, q0, n0, C, n_docs, wave, kSplitWaves, out_key, own_doc);
+}
+
+// ------------------------------------------------------------------------------------------
+// fp32 banks of up to 32 chunks a compute unit: the same split of the work, the products on the bf16 matrix cores.  An fp32 value is
+// three bf16 ones exactly, and of the nine products of two values the six largest carry 24 bits (what is left out is below 2^-24 of
+// the product): 192 cycles where the fp32 form takes 512.  Errors of 8000 chunks x 64 rows against float64, all scores: 5.8e-8 of
+// their norm, 1.7e-7 there.  Eight wavefronts hold an eighth of K each, of their 32 chunks in three parts in 96 registers; the
+// queries come as operands from the prologue (part_at), a kilobyte a load, four steps of K ahead.  The first parts' products and the
+// others' have sums of their own, so that small ones are not rounded away one by one.  What bounds it: K_r from memory with few rows
+// (8000 chunks x 64 rows 15.6 -> 13.5 us, the first block multiplied as it arrives; 13.9 with all four slabs requested at once), and
+// the operands' way from the L2 with many, 196 KB a block, which takes twice the 1.4 us that the products do (half of it would want
+// 64 chunks a workgroup, whose parts the registers do not hold).  An infinity among the values makes NaN where parts of different
+// sign meet, so a block with a NaN is multiplied again value by value.
+// ------------------------------------------------------------------------------------------
+constexpr int kPartsWaves = 8, kPartsSlabs = 4, kPartsMaxRows = 1024;
+constexpr int kPartsLds = kPartsWaves * kPartsSlabs * kSplitSlab + kSplitMaxBlocks * kSplitCols * 4;
+static_assert(kPartsLds <= 160 * 1024 && 2 * kPartsWaves * 32 * kSplitCols * 4 <= kPartsWaves * kPartsSlabs * kSplitSlab, "partial sums take the slabs' place");
+
+template <bool kDocMax>
+__global__ __launch_bounds__(kPartsWaves * 64) void score_parts_kernel(const char* __restrict__ qs, const float* __restrict__ kr,
+                                                                      const uint32_t* __restrict__ row_bits, uint32_t* __restrict__ out_key,
+                                                                      const int32_t* __restrict__ chunk_doc, int32_t M_rows, int32_t C,
+                                                                      int32_t blocks_per_query, int32_t n_docs, int32_t blocks_per_wg) {
+  typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 operand_t;
+  constexpr int kRow = kSplitK * (int)sizeof(float), kSlice = kRow / kPartsWaves, kSteps = kSplitK / kPartsWaves / 16, kAhead = 4;
+  static_assert(kSlice == kPartsSlabs * 128 && kSteps == 2 * kPartsSlabs && kSteps % kAhead == 0 && kPartsSlabs == 4, "a wavefront's share of K");
+  extern __shared__ __align__(16) char lds[];
+  float(*part)[kPartsWaves][32 * kSplitCols] = reinterpret_cast<float(*)[kPartsWaves][32 * kSplitCols]>(lds);
+  uint32_t(*best)[kSplitCols] = reinterpret_cast<uint32_t(*)[kSplitCols]>(lds + kPartsWaves * kPartsSlabs * kSplitSlab);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, half = lane >> 5;
+  const int n0 = blockIdx.x * kSplitCols, blocks = M_rows >> 5;
+  if (n0 >= C) return;                                   // (the grid's columns are a multiple of eight)
+  const int b0 = blockIdx.y * blocks_per_wg, b1 = min(blocks, b0 + blocks_per_wg);
+  const int32_t own_doc = kDocMax ? chunk_doc[min(n0 + l32, C - 1)] : 0;
+
+  // The first operands, then the chunks' rows, a slab of every wavefront before the next ones: the requests are taken up as fast as memory
+  // answers, and the last wavefront's first slab would come behind all of the others'.
+  const __amdgpu_buffer_rsrc_t rs_q = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(qs) + (int64_t)b0 * (kSplitK / 16) * kPartStep, 0,
+                                                                        (b1 - b0) * (kSplitK / 16) * kPartStep, 0x00020000);
+  u32x4_t q[kAhead][3];
+  auto request_q = [&](u32x4_t (&to)[3], int blk, int step) {          // (of a block behind the last: zeros)
 #pragma unroll
-      for (int o = 1; o < kSplitCols; o <<= 1) {
-        const uint32_t other = __shfl_down(key, o, kSplitCols);
-        const int32_t other_doc = __shfl_down(doc, o, kSplitCols);
-        if (l32 + o < kSplitCols && other_doc == doc) key = max(key, other);
+    for (int p = 0; p < 3; ++p)
+      to[p] = __builtin_amdgcn_raw_buffer_load_b128(rs_q, lane * 16 + ((blk - b0) * (kSplitK / 16) + wave * kSteps + step) * kPartStep + p * kPartBytes, 0, 0);
+  };
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) request_q(q[i], b0, i);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  char* const slabs = lds + wave * kPartsSlabs * kSplitSlab;
+  const uint32_t slabs_at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)slabs);
+  int at[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) at[i] = (8 * i + (lane >> 3)) * kRow + wave * kSlice + (((lane & 7) ^ (lane >> 3)) * 16);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char*>(reinterpret_cast<const char*>(kr)) + (int64_t)n0 * kRow, 0, min(kSplitCols, C - n0) * kRow, 0x00020000);
+  auto request_k = [&](int i) { request_slab(rs, slabs_at + i * kSplitSlab, at, i * 128); };
+  request_k(0);
+  __builtin_amdgcn_s_barrier();
+  request_k(1);
+  __builtin_amdgcn_s_barrier();
+  request_k(2);
+  const int q0 = b0 / blocks_per_query;
+  for (int i = tid; i < kSplitMaxBlocks * kSplitCols; i += kPartsWaves * 64) best[i / kSplitCols][i % kSplitCols] = 0u;
+
+  u32x4_t k[kSteps][3];
+  floatx16_t big, small;
+  auto clear = [&]() {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) big[e] = small[e] = 0.f;
+  };
+  auto multiply = [&](int i, int blk) {                  // a step of K; what is kAhead steps on takes its operands' registers
+    u32x4_t(&a)[3] = q[i % kAhead];
+    auto mul = [&](int x, int y, floatx16_t c) {
+      return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(operand_t, a[x]), __builtin_bit_cast(operand_t, k[i][y]), c, 0, 0, 0);
+    };
+    small = mul(0, 1, small);
+    big = mul(0, 0, big);
+    small = mul(1, 0, small);
+    small = mul(1, 1, small);
+    small = mul(0, 2, small);
+    small = mul(2, 0, small);
+    request_q(a, blk + (i + kAhead) / kSteps, (i + kAhead) % kSteps);
+  };
+  clear();
+  auto take = [&](auto slab) {                           // once what is younger than the slab alone is outstanding: other slabs, operands
+    constexpr int i = decltype(slab)::value, kOps = 6;
+    constexpr int kYounger = i == 0 ? 8 : i == 1 ? 8 + kOps : i == 2 ? 4 + 2 * kOps : 2 * kOps;
+    __builtin_amdgcn_s_waitcnt((kYounger & 15) | (kYounger >> 4 << 14) | (7 << 4) | (15 << 8));
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float x[8];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const u32x4_t w = *reinterpret_cast<const u32x4_t*>(slabs + i * kSplitSlab + l32 * 128 + (((4 * h + 2 * half + c) ^ (l32 & 7)) * 16));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[4 * c + e] = __uint_as_float(w[e]);
       }
-      const bool first = __shfl_up(doc, 1, kSplitCols) != doc || l32 == 0;
-      if (in && first && key != 0) atomicMax(&out_key[row * n_docs + doc], key);
-    } else {
-      if (in && key != 0) atomicMax(&out_key[row * C + n], key);
+      uint4 parts[3];
+      split_three<false>(x, parts);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) k[2 * i + h][p] = __builtin_bit_cast(u32x4_t, parts[p]);
+      multiply(2 * i + h, b0);
     }
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);                   // (the operands' requests are counted)
+  };
+  take(std::integral_constant<int, 0>{});
+  request_k(3);
+  take(std::integral_constant<int, 1>{});
+  take(std::integral_constant<int, 2>{});
+  take(std::integral_constant<int, 3>{});
+  __syncthreads();                                       // partial sums lie where the slabs were
+  // sum e is (row 8 * (e / 4) + 4 * half + e % 4, column l32) over this wavefront's eighth of K
+  for (int blk = b0; blk < b1; ++blk) {
+    if (blk > b0) {
+      clear();
+#pragma unroll
+      for (int i = 0; i < kSteps; ++i) multiply(i, blk);
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) part[(blk - b0) & 1][wave][(8 * (e >> 2) + 4 * half + (e & 3)) * kSplitCols + l32] = big[e] + small[e];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const uint32_t bits = row_bits[blk];                 // all rows of a block are scored, or none (presum_queries_kernel)
+    const float(*p)[32 * kSplitCols] = part[(blk - b0) & 1];
+    float top = -INFINITY;                               // of two rows; the other half of the wavefront has two more
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int row = (tid >> 5) * 2 + r, i = row * kSplitCols + l32;
+      float v = ((p[0][i] + p[1][i]) + (p[2][i] + p[3][i])) + ((p[4][i] + p[5][i]) + (p[6][i] + p[7][i]));
+      if (v != v && n0 + l32 < C) {
+        v = 0.f;
+        for (int x = 0; x < kSplitK; x += 8) {
+          const char* qp = qs + part_at(32 * blk + row, x, kSplitK);
+          for (int e = 0; e < 8; ++e) {
+            auto piece = [&](int n) { return bf16_to_f32(reinterpret_cast<const bf16_t*>(qp + n * kPartBytes)[e]); };
+            v += ((piece(0) + piece(1)) + piece(2)) * kr[(int64_t)(n0 + l32) * kSplitK + x + e];
+          }
+        }
+      }
+      top = fmaxf(top, v);
+    }
+    top = fmaxf(top, __shfl_xor(top, 32));
+    if (bits != 0 && half == 0) atomicMax(&best[blk / blocks_per_query - q0][l32], f32_to_key(top));
   }
+  __syncthreads();
+  merge_best<kDocMax>(best, b1 > b0 ? (b1 - 1) / blocks_per_query - q0 + 1 : 0, q0, n0, C, n_docs, wave, kPartsWaves, out_key, own_doc);
 }
 
 // Optional timing of the scoring kernel alone: event pairs recorded around its launch.  The lock makes the record
@@ -1338,13 +1526,21 @@ int launch_gemm(const void* qs, const void* kr, const uint32_t* row_bits, uint32
 // a multiple of the XCDs behind one another, so that one L2 has its K_r rows for all of them; the columns that this adds end at once.  us a
 // call, one workgroup a column and two: 8000 chunks x 64 rows 24.4 and 23.1, x 256 54.2 and 48.9, 6112 x 64 25.4 and 24.0 (two of 250 or
 // 191 columns that meet in different L2s: 30.5, 55.1 and 27.4).
-template <bool kDocMax>
-int launch_split(const void* qs, const void* kr, const uint32_t* row_bits, uint32_t* out_key, const int32_t* chunk_doc,
-                 int32_t M_rows, int32_t C, int32_t blocks_per_query, int32_t n_docs, hipStream_t st) {
+struct SplitGrid {
+  int cols, per_wg, x, y;       // columns, blocks a workgroup; the grid
+};
+SplitGrid split_grid(int32_t C, int32_t M_rows) {
   const int cols = (C + kSplitCols - 1) / kSplitCols, blocks = M_rows / 32;
   const int want = std::min(blocks, std::max((blocks + kSplitMaxBlocks - 1) / kSplitMaxBlocks, 2 * compute_units() / cols));
   const int per_wg = (blocks + want - 1) / want;
-  const dim3 grid((unsigned)((cols + 7) / 8 * 8), (unsigned)((blocks + per_wg - 1) / per_wg));
+  return {cols, per_wg, (cols + 7) / 8 * 8, (blocks + per_wg - 1) / per_wg};
+}
+template <bool kDocMax>
+int launch_split(const void* qs, const void* kr, const uint32_t* row_bits, uint32_t* out_key, const int32_t* chunk_doc,
+                 int32_t M_rows, int32_t C, int32_t blocks_per_query, int32_t n_docs, hipStream_t st) {
+  const SplitGrid plan = split_grid(C, M_rows);
+  const int cols = plan.cols, per_wg = plan.per_wg;
+  const dim3 grid((unsigned)plan.x, (unsigned)plan.y);
   int slot = -1;
   if (g_timer.on.load(std::memory_order_acquire)) {
     std::lock_guard<std::mutex> lock(g_timer.mu);
@@ -1359,6 +1555,48 @@ int launch_split(const void* qs, const void* kr, const uint32_t* row_bits, uint3
   MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised[one], reinterpret_cast<const void*>(kern), lds));
   kern<<<grid, kSplitWaves * 64, lds, st>>>(static_cast<const float*>(qs), static_cast<const float*>(kr), row_bits,
                                             out_key, chunk_doc, M_rows, C, blocks_per_query, n_docs, per_wg);
+  MSA_LAUNCH_CHECK();
+  if (slot >= 0) MSA_HIP(hipEventRecord(g_timer.stop[slot], st));
+  return MSA_OK;
+}
+
+// Up to one workgroup a compute unit, those of a column a multiple of the XCDs behind one another (the columns that this adds count: 85
+// columns in three rows of 88 leave five XCDs with a workgroup more than they have compute units).
+SplitGrid parts_grid(int32_t C, int32_t M_rows) {
+  const int cols = (C + kSplitCols - 1) / kSplitCols, blocks = M_rows / 32, x = (cols + 7) / 8 * 8;
+  const int want = std::min(blocks, std::max(1, compute_units() / x)), per_wg = (blocks + want - 1) / want;
+  return {cols, per_wg, x, (blocks + per_wg - 1) / per_wg};
+}
+// The line between the other fp32 forms: launch_gemm_for has its figures.
+bool split_ok(int32_t C, int32_t M_rows) { return M_rows <= 64 || (int64_t)C * M_rows <= (int64_t)1 << 21; }
+// Whether a call of fp32 queries takes score_parts_kernel.  A block costs a compute unit about 3.2 us there and 3.7 in score_split_kernel, which has
+// two workgroups a unit and starts 1.3 us later; parts of queries are written in pieces of 16 bytes, some 7.5 us for a thousand rows.  Whole
+// calls, us, score_split_kernel (from 2^21 on tiles) and here: chunks x rows 300 x 64 17.4 and 16.3, 2000 x 128 18.1 and 17.8, 3300 x 192 29.7
+// and 23.8, 5500 x 512 82.8 and 64.8, 8192 x 64 24.2 and 22.0, x 1024 144 and 115; not taken: 300 x 512 20.5 and 22.5, 2700 x 512 41.0 and 43.8,
+// 4200 x 384 47.5 and 51.6 (132 workgroups of twelve blocks).
+bool takes_parts(int32_t dtype, int64_t C, int32_t K, int32_t M_rows, int32_t query_reduce) {
+  const int units = compute_units();
+  if (dtype != MSA_F32 || K != kSplitK || M_rows > kPartsMaxRows || query_reduce != kQueryMax || C > (int64_t)kSplitCols * units) return false;
+  const SplitGrid here = parts_grid((int32_t)C, M_rows), there = split_grid((int32_t)C, M_rows);
+  if (here.x > units) return false;
+  if (!split_ok((int32_t)C, M_rows)) return true;
+  const int share = there.per_wg * ((there.x * there.y + units - 1) / units);
+  return 3.2f * (float)here.per_wg + 0.0075f * (float)M_rows < 3.7f * (float)share + 1.3f;
+}
+template <bool kDocMax>
+int launch_parts(const void* qs, const void* kr, const uint32_t* row_bits, uint32_t* out_key, const int32_t* chunk_doc,
+                 int32_t M_rows, int32_t C, int32_t blocks_per_query, int32_t n_docs, hipStream_t st) {
+  const SplitGrid grid = parts_grid(C, M_rows);
+  static std::atomic<int> lds_limit_raised{0};
+  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(score_parts_kernel<kDocMax>), kPartsLds));
+  int slot = -1;
+  if (g_timer.on.load(std::memory_order_acquire)) {
+    std::lock_guard<std::mutex> lock(g_timer.mu);
+    if (g_timer.n < g_timer.cap) slot = g_timer.n++;
+  }
+  if (slot >= 0) MSA_HIP(hipEventRecord(g_timer.start[slot], st));
+  score_parts_kernel<kDocMax><<<dim3((unsigned)grid.x, (unsigned)grid.y), kPartsWaves * 64, kPartsLds, st>>>(
+      static_cast<const char*>(qs), static_cast<const float*>(kr), row_bits, out_key, chunk_doc, M_rows, C, blocks_per_query, n_docs, grid.per_wg);
   MSA_LAUNCH_CHECK();
   if (slot >= 0) MSA_HIP(hipEventRecord(g_timer.stop[slot], st));
   return MSA_OK;
@@ -1433,7 +1671,7 @@ int launch_gemm_for(int32_t dtype, const void* qs, const void* kr, const uint32_
   // The line between the fp32 forms: above it the tiles' reuse of both operands is worth more than the even split (16384 chunks x
   // 128 rows: 61 us in the split form, 84 in tiles; x 256 rows 95 and 88; 65536 x 128: 190 and 151), except that the tiles pad up
   // to 64 rows to 128 (65536 x 64: 123 and 142).
-  if (dtype != MSA_BF16 && K == kSplitK && (M_rows <= 64 || (int64_t)C * M_rows <= (int64_t)1 << 21))
+  if (dtype != MSA_BF16 && K == kSplitK && split_ok(C, M_rows))
     return launch_split<kDocMax>(qs, kr, row_bits, out_key, chunk_doc, M_rows, C, bpq, n_docs, st);
   if (dtype != MSA_BF16)
     return launch_gemm<float, 128, 128, 2, 2, 1, kDocMax, false>(qs, kr, row_bits, out_key, chunk_doc, M_rows, C, K, bpq, n_docs, st);
@@ -1451,14 +1689,14 @@ int launch_gemm_for(int32_t dtype, const void* qs, const void* kr, const uint32_
 // ------------------------------------------------------------------------------------------
 
 RouteWorkspace route_workspace_layout(int32_t B, int32_t S, int32_t Hkv, int32_t D, int64_t plane_cols, int64_t n_docs,
-                                      int32_t dtype) {
+                                      int32_t dtype, bool parts) {
   RouteWorkspace w{};
   w.S_pad = (S + 31) / 32 * 32;
   w.M_rows = B * w.S_pad;
   const int64_t m_alloc = ((int64_t)w.M_rows + 255) / 256 * 256;   // every M tile may read whole mask words
   w.mask_words = (int32_t)(m_alloc / 32);
   size_t off = 0;
-  w.off_qs = off;       off = align_up(off + (size_t)w.M_rows * Hkv * D * elem_bytes(dtype), 256);
+  w.off_qs = off;       off = align_up(off + (size_t)w.M_rows * Hkv * D * (parts ? 3 * sizeof(bf16_t) : elem_bytes(dtype)), 256);
   w.off_row_bits = off; off = align_up(off + (size_t)w.mask_words * sizeof(uint32_t), 256);
   w.off_key = off;      off = align_up(off + (size_t)B * plane_cols * sizeof(uint32_t), 256);
   w.topk_blocks = topk_blocks_for(n_docs);
@@ -1468,6 +1706,11 @@ RouteWorkspace route_workspace_layout(int32_t B, int32_t S, int32_t Hkv, int32_t
   w.bytes = off;
   return w;
 }
+
+namespace {
+// Whether some bank's fp32 queries of these sizes come in parts.
+bool may_take_parts(int32_t B, int32_t S, int32_t Hkv, int32_t D) { return (int64_t)B * ((S + 31) / 32 * 32) <= kPartsMaxRows && Hkv * D == kSplitK; }
+}  // namespace
 
 // Host-side replay of the large-tile scan's tile order (scan_walk.h): every scoring workgroup walks its own tiles
 // with the cursor the kernel uses, then the workgroups draw the pool's tiles in turn from one counter.
@@ -1584,14 +1827,14 @@ extern "C" size_t msa_route_workspace_bytes(int32_t B, int32_t S, int32_t Hq, in
   (void)Hq; (void)topk;
   if (B <= 0 || S <= 0 || Hkv <= 0 || D <= 0 || C <= 0 || n_docs <= 0) return 0;
   // sized for fp32 queries so one workspace serves both dtypes, and for the per-chunk plane of msa_chunk_scores
-  return route_workspace_layout(B, S, Hkv, D, C + n_docs, n_docs, MSA_F32).bytes;
+  return route_workspace_layout(B, S, Hkv, D, C + n_docs, n_docs, MSA_F32, may_take_parts(B, S, Hkv, D)).bytes;
 }
 
 extern "C" size_t msa_route_topk_workspace_bytes(int32_t B, int32_t S, int32_t Hq, int32_t Hkv, int32_t D,
                                                  int64_t n_docs, int32_t topk) {
   (void)Hq; (void)topk;
   if (B <= 0 || S <= 0 || Hkv <= 0 || D <= 0 || n_docs <= 0) return 0;
-  return route_workspace_layout(B, S, Hkv, D, n_docs, n_docs, MSA_F32).bytes;
+  return route_workspace_layout(B, S, Hkv, D, n_docs, n_docs, MSA_F32, may_take_parts(B, S, Hkv, D)).bytes;
 }
 
 int route_scores_to_keys(const msa_bank* bank, int32_t layer, const void* q, const uint8_t* qmask_u8, int32_t B,
@@ -1621,8 +1864,9 @@ int route_scores_to_keys(const msa_bank* bank, int32_t layer, const void* q, con
   const int64_t plane_cols = doc_max ? bank->n_docs : bank->C;
   // a collapsed query (mean / last over its tokens) is one row: one row block per query
   const int32_t S_scan = query_reduce == kQueryMax ? S : 1;
-  const RouteWorkspace w = route_workspace_layout(B, S_scan, bank->Hkv, bank->D, plane_cols + extra_plane_cols, bank->n_docs,
-                                                  bank->dtype);
+  RouteWorkspace w = route_workspace_layout(B, S_scan, bank->Hkv, bank->D, plane_cols + extra_plane_cols, bank->n_docs, bank->dtype, true);
+  const bool parts = takes_parts(bank->dtype, bank->C, bank->Hkv * bank->D, w.M_rows, query_reduce) && w.bytes <= workspace_bytes;
+  if (!parts) w = route_workspace_layout(B, S_scan, bank->Hkv, bank->D, plane_cols + extra_plane_cols, bank->n_docs, bank->dtype, false);
   if (w.bytes > workspace_bytes) {
     msa_set_error("%s: workspace of %zu bytes, need %zu", who, workspace_bytes, w.bytes);
     return MSA_ESIZE;
@@ -1657,6 +1901,10 @@ int route_scores_to_keys(const msa_bank* bank, int32_t layer, const void* q, con
     presum_queries_kernel<bf16_t, bf16_t><<<w.M_rows, pthreads, 0, st>>>(
         static_cast<const bf16_t*>(q), qmask_u8, B, S, w.S_pad, Hq, bank->Hkv, normalize, static_cast<bf16_t*>(qs),
         row_bits, w.mask_words, key, clear_words, sched);
+  } else if (parts) {
+    presum_queries_kernel<float, float, true><<<w.M_rows, pthreads, 0, st>>>(
+        static_cast<const float*>(q), qmask_u8, B, S, w.S_pad, Hq, bank->Hkv, normalize, static_cast<float*>(qs),
+        row_bits, w.mask_words, key, clear_words, sched);
   } else {
     presum_queries_kernel<float, float><<<w.M_rows, pthreads, 0, st>>>(
         static_cast<const float*>(q), qmask_u8, B, S, w.S_pad, Hq, bank->Hkv, normalize, static_cast<float*>(qs),
@@ -1666,7 +1914,10 @@ int route_scores_to_keys(const msa_bank* bank, int32_t layer, const void* q, con
 
   const int32_t K = bank->Hkv * bank->D;
   const int32_t bpq = w.S_pad / 32;
-  const int rc = doc_max ? launch_gemm_for<true>(bank->dtype, qs, bank->kr_dev[layer], row_bits, key, bank->chunk_doc_dev,
+  const auto by_parts = doc_max ? launch_parts<true> : launch_parts<false>;
+  const int rc = parts ? by_parts(qs, bank->kr_dev[layer], row_bits, key, doc_max ? bank->chunk_doc_dev : nullptr, w.M_rows, (int32_t)bank->C, bpq,
+                                  (int32_t)bank->n_docs, st)
+                 : doc_max ? launch_gemm_for<true>(bank->dtype, qs, bank->kr_dev[layer], row_bits, key, bank->chunk_doc_dev,
                                                  w.M_rows, (int32_t)bank->C, K, bpq, (int32_t)bank->n_docs, st, job,
                                                  job_taken, sched)
                          : launch_gemm_for<false>(bank->dtype, qs, bank->kr_dev[layer], row_bits, key, nullptr, w.M_rows,
