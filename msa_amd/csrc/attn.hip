@@ -547,6 +547,9 @@ struct NormRope {
   }
 };
 
+// kPaired (up to 64 samples): the pieces of samples of different lengths dealt so that two beside one another are about as long as any two.
+constexpr int kDecodeUnits = 256;
+template <bool kPaired>
 __global__ __launch_bounds__(kRingWaves * 64) void attn_decode_fused_kernel(
     const bf16_t* __restrict__ qkv, int64_t row_stride, int32_t Hq, int32_t Hkv, const int64_t* __restrict__ pos,
     const bf16_t* __restrict__ qw, const bf16_t* __restrict__ kw, float eps, const float* __restrict__ cos_t,
@@ -556,17 +559,41 @@ __global__ __launch_bounds__(kRingWaves * 64) void attn_decode_fused_kernel(
   extern __shared__ __align__(16) char lds[];
   HeadSums& new_token = sums_of(lds, kRingWaves);
   uint4* sm_q = reinterpret_cast<uint4*>(lds + kRingLds + sizeof(HeadSums));        // [G][16]
-  const int b = blockIdx.x, g = blockIdx.y, split = blockIdx.z, G = Hq / Hkv;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), G = Hq / Hkv;
+  int b = blockIdx.x, g = blockIdx.y, split = blockIdx.z, L_old;
+  int64_t position;
+  if constexpr (kPaired) {
+    // Units in the order of the workgroups, the longest samples first in each of their rounds, the second round (of those a compute unit has
+    // two places for) backwards: whoever has a long piece gets a short one beside it.
+    const int B = gridDim.x, total = B * Hkv * n_split, second = min(2 * kDecodeUnits, total);
+    const int len = lane < B ? kv_len[lane] : 0;
+    const int64_t at = lane < B ? pos[lane] : 0;
+    int unit = b + B * (g + Hkv * split);
+    if (unit >= kDecodeUnits && unit < second) unit = kDecodeUnits + second - 1 - unit;
+    const int row_of = unit / B, place = unit - row_of * B;
+    split = row_of / Hkv;
+    g = row_of - split * Hkv;
+    // a sample's place by length; no two keys are equal, and those of absent lanes come last
+    const uint32_t key = (uint32_t)min(max(len, 0), (1 << 25) - 1) * 64 + (63 - lane);
+    int rank = 0;
+    for (int i0 = 0; i0 < B; i0 += 16)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) rank += (uint32_t)__builtin_amdgcn_readlane((int)key, i0 + i) > key;
+    b = __builtin_ctzll(__ballot(rank == place));
+    L_old = __builtin_amdgcn_readlane(len, b);
+    position = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)((uint64_t)at >> 32), b) << 32 | (uint32_t)__builtin_amdgcn_readlane((int)at, b));
+  } else {
+    L_old = kv_len[b];
+    position = pos[b];
+  }
   const int j = lane & 15, hq = tid >> 4;                  // 16 lanes a head: the group's q heads, and behind them the new key
   const bf16_t* row = qkv + (int64_t)b * row_stride + 8 * j;
   NormRope head;
   head.load(row + (int64_t)(hq < G ? g * G + hq : Hq + g) * kHeadDim, (hq < G ? qw : kw) + 8 * j);
   const uint4 v_new = *reinterpret_cast<const uint4*>(row + (int64_t)(Hq + Hkv + g) * kHeadDim);
-  const int64_t p = min((int64_t)max((int64_t)0, pos[b]), (int64_t)rope_rows - 1);
+  const int64_t p = min((int64_t)max((int64_t)0, position), (int64_t)rope_rows - 1);
   head.load_rotary(cos_t + p * 64, sin_t + p * 64, j);
 
-  const int L_old = kv_len[b];
   const bool has_new = L_old < Lcap;
   const int per_split = (L_old + n_split - 1) / n_split, key0 = split * per_split, key1 = min(L_old, key0 + per_split);
   const int64_t column = ((int64_t)b * Lcap * Hkv + g) * kHeadDim;
@@ -757,14 +784,33 @@ int launch_attn_bf16(const void* q, const int32_t* cu_q, const void* k, const vo
   return launch(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml, part_acc, st);
 }
 
+int rows_splits(int32_t total_q, int32_t Hkv, int32_t max_kv) {
+  return std::max(plan_splits(total_q, Hkv, max_kv).n_split, plan_splits_rows(total_q, Hkv, max_kv, true).n_split);
+}
+size_t partials_bytes(int32_t total_q, int32_t Hq, int32_t D, int splits) {
+  const size_t n = (size_t)total_q * Hq * splits;
+  return align_up(n * 2 * sizeof(float), 256) + align_up(n * D * sizeof(float), 256);
+}
+// Splits where decoding samples take the paired form: as many as two workgroups a compute unit hold; 0 where plan_splits_rows' form is ahead.
+// Finding a workgroup's sample costs 0.4 us, and a piece wants keys: 500 where one workgroup a unit comes out even, 160 where it does not.
+// Both launches, us, even splits and pairs (8 KV heads, all of one length and of half of it to all): 16 of 4388 keys 55.6 -> 52.7 and
+// 49.4 -> 43.9, of 2500 36.1 -> 34.3 and 31.3 -> 29.0, one of 4388 and fifteen of 500 34.0 -> 25.0, 15 of 2000 31.1 -> 27.9 and 26.6 -> 23.4,
+// 7 of 2000 21.4 -> 17.6 and 19.8 -> 16.8, 5 of 2000 17.4 -> 15.4; not taken: 16 of 1000 18.1 -> 18.5, 8 of 2000 18.0 -> 19.1, 5 of 1000 11.1 -> 11.9,
+// 3 of 4388 16.5 -> 17.9.
+int paired_splits(int32_t B, int32_t Hkv, int32_t Lcap) {
+  const int64_t pairs = (int64_t)B * Hkv;
+  if (B > 64 || pairs < 32 || pairs > 2 * kDecodeUnits) return 0;
+  const int n = (int)(2 * kDecodeUnits / pairs);
+  if (n * pairs < 400) return 0;                           // (too few places taken: 24 samples of 2000 43.3 -> 44.0)
+  return Lcap >= n * (kDecodeUnits % pairs == 0 ? 500 : 160) ? n : 0;
+}
+
 }  // namespace
 
 extern "C" size_t msa_attn_workspace_bytes(int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D, int32_t max_kv) {
   if (total_q <= 0 || Hq <= 0 || Hkv <= 0 || D <= 0 || max_kv <= 0) return 0;
   // sized for whichever of the kernels has more partials
-  const int splits = std::max(plan_splits(total_q, Hkv, max_kv).n_split, plan_splits_rows(total_q, Hkv, max_kv, true).n_split);
-  const size_t n = (size_t)total_q * Hq * splits;
-  return align_up(n * 2 * sizeof(float), 256) + align_up(n * D * sizeof(float), 256);
+  return partials_bytes(total_q, Hq, D, std::max(rows_splits(total_q, Hkv, max_kv), paired_splits(total_q, Hkv, max_kv)));
 }
 
 extern "C" int msa_sparse_attn(const void* q, const int32_t* cu_q, const void* k, const void* v,
@@ -786,7 +832,7 @@ extern "C" int msa_sparse_attn(const void* q, const int32_t* cu_q, const void* k
   const SplitPlan plan = mfma ? plan_splits(total_q, Hkv, max_kv) : plan_splits_rows(total_q, Hkv, max_kv, dtype == MSA_BF16 && takes_ring(total_q, Hkv, max_kv, Hq / Hkv));
   const int n_split = plan.n_split;
   MSA_REQUIRE(n_split <= 65535, "msa_sparse_attn: max_kv=%d too large", max_kv);
-  const size_t need = msa_attn_workspace_bytes(total_q, Hq, Hkv, D, max_kv);
+  const size_t need = partials_bytes(total_q, Hq, D, rows_splits(total_q, Hkv, max_kv));
   if (need > workspace_bytes) {
     msa_set_error("msa_sparse_attn: workspace of %zu bytes, need %zu", workspace_bytes, need);
     return MSA_ESIZE;
@@ -824,19 +870,22 @@ extern "C" int msa_decode_attn_fused(const void* qkv, int64_t row_stride, const 
   MSA_REQUIRE((((uintptr_t)qkv | (uintptr_t)q_norm_w | (uintptr_t)k_norm_w | (uintptr_t)kcache | (uintptr_t)vcache) & 15) == 0,
               "msa_decode_attn_fused: pointers must be 16-byte aligned");
   MSA_REQUIRE(Lcap > 0 && rope_rows > 0 && eps > 0.f && scale > 0.f, "msa_decode_attn_fused: bad scalar argument");
-  const size_t need = msa_attn_workspace_bytes(B, Hq, Hkv, D, Lcap);
+  const int paired = paired_splits(B, Hkv, Lcap);
+  const bool pairs = paired > 0 && partials_bytes(B, Hq, D, paired) <= workspace_bytes;
+  const size_t need = partials_bytes(B, Hq, D, rows_splits(B, Hkv, Lcap));
   if (need > workspace_bytes) {
     msa_set_error("msa_decode_attn_fused: workspace of %zu bytes, need %zu", workspace_bytes, need);
     return MSA_ESIZE;
   }
-  const int n_split = plan_splits_rows(B, Hkv, Lcap, true).n_split;
+  const int n_split = pairs ? paired : plan_splits_rows(B, Hkv, Lcap, true).n_split;
   const size_t n = (size_t)B * Hq * n_split;
   float* part_ml = static_cast<float*>(workspace);
   float* part_acc = reinterpret_cast<float*>(static_cast<char*>(workspace) + align_up(n * 2 * sizeof(float), 256));
   hipStream_t st = as_stream(stream);
-  static std::atomic<int> lds_limit_raised{0};
-  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(attn_decode_fused_kernel), kFusedLds));
-  attn_decode_fused_kernel<<<dim3((unsigned)B, (unsigned)Hkv, (unsigned)n_split), kRingWaves * 64, kFusedLds, st>>>(
+  static std::atomic<int> lds_limit_raised[2] = {{0}, {0}};
+  const auto kernel = pairs ? attn_decode_fused_kernel<true> : attn_decode_fused_kernel<false>;
+  MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised[pairs], reinterpret_cast<const void*>(kernel), kFusedLds));
+  kernel<<<dim3((unsigned)B, (unsigned)Hkv, (unsigned)n_split), kRingWaves * 64, kFusedLds, st>>>(
       static_cast<const bf16_t*>(qkv), row_stride, Hq, Hkv, positions, static_cast<const bf16_t*>(q_norm_w),
       static_cast<const bf16_t*>(k_norm_w), eps, rope_cos, rope_sin, rope_rows, static_cast<bf16_t*>(kcache),
       static_cast<bf16_t*>(vcache), Lcap, kv_len, scale * 1.4426950408889634f, n_split, part_ml, part_acc);
