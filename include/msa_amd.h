@@ -306,6 +306,11 @@ int msa_flash_attn_hint(const void* q, const int32_t* cu_q, const void* k, const
                         const int64_t* kv_off, const int32_t* kv_len, int32_t B, int32_t total_q,
                         int32_t Hq, int32_t Hkv, int32_t D, float scale, int32_t causal, void* out,
                         int32_t max_sq, void* stream);
+/* The same in the form that is the faster one for a batch of these sizes. */
+int msa_flash_attn_fit(const void* q, const int32_t* cu_q, const void* k, const void* v,
+                       const int64_t* kv_off, const int32_t* kv_len, int32_t B, int32_t total_q,
+                       int32_t Hq, int32_t Hkv, int32_t D, float scale, int32_t causal, void* out,
+                       int32_t max_sq, void* stream);
 /* Causal attention of rows as a decoder of mixed layers has them: query rows q_stride elements apart, sample b's keys end with its own rows
  * behind kv_pos[b] earlier ones.  sink [Hq] (or NULL): a member of every softmax of head h without a value; gate [rows, Hq] bf16, rows
  * gate_stride apart (or NULL): outputs times its sigmoid.  out [rows, Hq, D] dense. */

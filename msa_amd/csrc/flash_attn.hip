@@ -487,12 +487,33 @@ constexpr int kWideCompilerVgprs = 56;
                  "=v"((X)[7]), "=v"((X)[8]), "=v"((X)[9]), "=v"((X)[10]), "=v"((X)[11]), "=v"((X)[12]), "=v"((X)[13]), \
                  "=v"((X)[14]), "=v"((X)[15]))
 
+// How many of the first 32 or of all 64 lanes have a smaller key (of less than 2^31).  By rotations within rows of 16 lanes: taken through scalar
+// registers, lane by lane, two rankings took 1.2 us.
+template <int R>
+__device__ __forceinline__ void count_smaller(uint32_t row, uint32_t key, int& n) {
+  n += (int)((row - key) >> 31);
+  if constexpr (R % 4 == 3) __builtin_amdgcn_sched_barrier(0);           // (registers)
+  if constexpr (R < 15) count_smaller<R + 1>((uint32_t)__builtin_amdgcn_mov_dpp((int)row, 0x121, 0xf, 0xf, false), key, n);
+}
+__device__ __forceinline__ uint32_t lane_before(uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x138, 0xf, 0xf, false); }
+__device__ __forceinline__ int place_of(uint32_t key, bool all) {
+  int n = 0;
+#pragma unroll 1
+  for (int row = 0; row < (all ? 64 : 32); row += 16) count_smaller<0>(__shfl_xor(key, row), key, n);
+  return n;
+}
+
 // The launch is persistent: one workgroup per compute unit walks the token blocks of its KV head (workgroup w serves
 // head w % Hkv, so with eight heads a head keeps to one XCD and its K / V to that XCD's L2, and is the (w / Hkv)-th of
 // the n workgroups of the head).  A head's blocks are listed sample by sample, under the causal mask a sample's late
-// (long) blocks first, and dealt out in rounds of n that alternate direction: workgroup c takes position c of an even
-// round and n - 1 - c of an odd one, so the workgroup that drew the longest block of a round draws the shortest of the
-// next (a sample of 2 n causal blocks splits evenly), and the n workgroups stay on the same sample's K / V.
+// (long) blocks first, and dealt out in rounds of n, so that the n workgroups stay on the same sample's K / V: the
+// longest block of a round goes to the workgroup that has had least so far, and so on.  Every workgroup follows the
+// rounds for all of them, lane = workgroup and lane = position, which takes two rankings a round and no memory (above
+// 64 workgroups a head, several groups deal every second, third, .. position).  A round's lookup takes 0.8 us (code
+// that is cold each time) and 1.7 with rankings, a fixed order of back and forth 0.5, which however leaves the longest
+// of the workgroups 10 to 50 % behind the mean with ragged samples: 4 of 1000 to 2000 tokens 189 and 160 us, three of
+// 2700 to 3500 314 and 252, 16 of 2048 to 4096 1447 and 1405; two of 1780 and 2200, whose blocks fill two rounds, 84 and
+// 87: with `in_turn` the order is that one.
 // Blocks are pipelined: once a block's last product is issued its LDS rings are free, so the next block's first tiles
 // and its query rows (into 16 KB of LDS per wavefront behind the rings) are requested before the finished block's
 // output is scaled and stored, and the block after that is looked up while those loads are awaited.
@@ -500,13 +521,15 @@ template <int G>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVgprs))) void flash_wide_kernel(
     const bf16_t* __restrict__ q, const int32_t* __restrict__ cu_q, const bf16_t* __restrict__ k,
     const bf16_t* __restrict__ v, const int64_t* __restrict__ kv_off, const int32_t* __restrict__ kv_len, int32_t B,
-    int32_t Hq, int32_t Hkv, float scale_log2e, int32_t causal, bf16_t* __restrict__ out, int32_t total_blocks, RowOptions opt) {
+    int32_t Hq, int32_t Hkv, float scale_log2e, int32_t causal, bf16_t* __restrict__ out, int32_t in_turn, RowOptions opt) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int kTokPerWave = 64 / G;
   constexpr int kTokPerBlock = 4 * kTokPerWave;
   extern __shared__ __align__(16) char lds[];
 
-  const int g = blockIdx.x % Hkv, c_wg = blockIdx.x / Hkv, n_wg = gridDim.x / Hkv;
+  const int g = blockIdx.x % Hkv;
+  const int groups = (gridDim.x / Hkv + 63) / 64, c_all = blockIdx.x / Hkv, group = c_all % groups, c_wg = c_all / groups;
+  const int n_wg = (gridDim.x / Hkv - group + groups - 1) / groups;              // of this group
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row_elems = Hkv * kHeadDim;
   const int row_bytes = row_elems * 2;
@@ -542,34 +565,70 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVg
     int q_first, sq, t0, kmax, n_tiles, L;
     int64_t base;
   };
-  // (a workgroup's positions in the list only grow, so the search for a position's sample resumes where the last
-  // one ended: `cur_b` is a sample, `before` the number of blocks of the samples in front of it)
-  int cur_b = 0, before = 0;
-  auto find_block = [&](int& round, Block& blkout) -> bool {
-    for (; round * n_wg < total_blocks; ++round) {
-      const int pos = round * n_wg + ((round & 1) ? n_wg - 1 - c_wg : c_wg);
-      for (; cur_b < B; ++cur_b) {
-        const int first = cu_q ? cu_q[cur_b] : cur_b;
-        const int sq_b = cu_q ? cu_q[cur_b + 1] - first : 1;
-        const int nb = (sq_b + kTokPerBlock - 1) / kTokPerBlock;
-        if (pos - before < nb) {
-          int blk = pos - before;
-          if (causal) blk = nb - 1 - blk;
-          blkout.q_first = first;
-          blkout.sq = sq_b;
-          blkout.t0 = blk * kTokPerBlock;
-          blkout.L = kv_len ? kv_len[cur_b] : (int)opt.kv_pos[cur_b] + sq_b;
-          blkout.base = kv_off[cur_b];
-          const int last_tok = min(sq_b, blkout.t0 + kTokPerBlock) - 1;
-          blkout.kmax = causal ? max(0, min(blkout.L, blkout.L - sq_b + last_tok + 1)) : blkout.L;
-          blkout.n_tiles = (blkout.kmax + kKeysPerTile - 1) / kKeysPerTile;
-          ++round;
-          return true;
-        }
-        before += nb;
+  // (positions only grow, so a round's search for its samples resumes where the last one ended: `cur_b` is a sample,
+  // `before` the number of blocks of the samples in front of it)
+  int cur_b = 0, before = 0, round = 0;
+  uint32_t load = lane < n_wg ? 0u : 1u << 24;  // half tiles that workgroup `lane` has had, more than the one with fewest
+  auto find_block = [&](Block& blkout) -> bool {
+    const int n_all = gridDim.x / Hkv;
+    const int pos = in_turn ? round * n_all + ((round & 1) ? n_all - 1 - c_all : c_all) : (round * n_wg + lane) * groups + group;
+    const int last = in_turn ? pos : (round * n_wg + n_wg - 1) * groups + group;
+    ++round;
+    uint32_t cost = 0;
+    int first_of = 0, sq_of = 0, block = 0, keys_of = 0, base_lo = 0, base_hi = 0;           // of lane's position
+    for (; cur_b < B; ++cur_b) {
+      const int first = cu_q ? cu_q[cur_b] : cur_b;
+      const int sq_b = cu_q ? cu_q[cur_b + 1] - first : 1;
+      const int nb = (sq_b + kTokPerBlock - 1) / kTokPerBlock;
+      const int L = kv_len ? kv_len[cur_b] : (int)opt.kv_pos[cur_b] + sq_b;
+      const int64_t base = kv_off[cur_b];
+      if ((in_turn || lane < n_wg) && pos >= before && pos < before + nb) {
+        block = causal ? nb - 1 - (pos - before) : pos - before;
+        const int last_tok = min(sq_b, (block + 1) * kTokPerBlock) - 1;
+        const int kmax = causal ? max(0, min(L, L - sq_b + last_tok + 1)) : L;
+        cost = 3 + min(kmax / (kKeysPerTile / 2), 1 << 20);        // (a block's start and end take as long as a tile and a half)
+        first_of = first;
+        sq_of = sq_b;
+        keys_of = L;
+        base_lo = (int)base;
+        base_hi = (int)(base >> 32);
       }
+      if (before + nb > last) break;
+      before += nb;
     }
-    return false;
+    int at = 0;
+    if (!in_turn) {
+      // Places: of the blocks by length, of the workgroups by what they have had.  Both are often in order already (a sample's blocks, and the
+      // workgroups after them).
+      const uint32_t cost_key = ((1 << 21) - cost) * 64 + lane, load_key = load * 64 + lane;
+      const bool inner = lane > 0 && lane < n_wg;
+      const uint32_t cost_before = lane_before(cost_key), load_before = lane_before(load_key);
+      int cost_place = lane, load_place = lane;
+      uint32_t by_place = cost;                              // (lanes behind the workgroups have places of their own, behind these)
+      if (__any(inner && cost_before > cost_key)) {
+        cost_place = place_of(cost_key, n_wg > 32);
+        by_place = (uint32_t)__builtin_amdgcn_ds_permute((lane < n_wg ? cost_place : lane) * 4, (int)cost);
+      }
+      if (__any(inner && load_before > load_key)) {
+        load_place = !__any(inner && load_before < load_key) ? n_wg - 1 - lane : place_of(load_key, n_wg > 32);
+        by_place = (uint32_t)__builtin_amdgcn_ds_bpermute((lane < n_wg ? load_place : lane) * 4, (int)by_place);
+      }
+      const int own = __builtin_amdgcn_readlane(load_place, c_wg);
+      at = __builtin_ctzll(__ballot(cost_place == own));
+      const uint32_t fewest = (uint32_t)__builtin_amdgcn_readlane((int)load, __builtin_ctzll(__ballot(load_place == 0)));
+      load += by_place - (lane < n_wg ? fewest : 0u);
+    }
+    const bool found = __builtin_amdgcn_readlane((int)cost, at) != 0;
+    if (!found) return false;
+    blkout.q_first = __builtin_amdgcn_readlane(first_of, at);
+    blkout.sq = __builtin_amdgcn_readlane(sq_of, at);
+    blkout.t0 = __builtin_amdgcn_readlane(block, at) * kTokPerBlock;
+    blkout.L = __builtin_amdgcn_readlane(keys_of, at);
+    blkout.base = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane(base_hi, at) << 32 | (uint32_t)__builtin_amdgcn_readlane(base_lo, at));
+    const int last_tok = min(blkout.sq, blkout.t0 + kTokPerBlock) - 1;
+    blkout.kmax = causal ? max(0, min(blkout.L, blkout.L - blkout.sq + last_tok + 1)) : blkout.L;
+    blkout.n_tiles = (blkout.kmax + kKeysPerTile - 1) / kKeysPerTile;
+    return true;
   };
 
   // running positions of the K and V tile streams of the block whose tiles are being loaded
@@ -650,130 +709,131 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVg
     }
   };
 
-  int round = 0;
   Block cur{}, nxt{};
-  bool have = find_block(round, cur);
-  if (have) request_block(cur);
-  while (have) {
-    const bool have_next = find_block(round, nxt);      // scalar work under the loads' latency
-    const int n_tiles = cur.n_tiles;
-    int wave_min_limit;
-    {
-      int lane_c = lane;
-      asm volatile("" : "+v"(lane_c));
-      const int half = lane_c >> 5;
-      int limit[2];
+  for (bool have = false;; have = true) {
+    const bool have_next = find_block(nxt);      // scalar work under the loads' latency
+    if (have) {
+      const int n_tiles = cur.n_tiles;
+      int wave_min_limit;
+      {
+        int lane_c = lane;
+        asm volatile("" : "+v"(lane_c));
+        const int half = lane_c >> 5;
+        int limit[2];
 #pragma unroll
-      for (int cb = 0; cb < 2; ++cb) {
-        const int col = 32 * cb + (lane_c & 31);
-        const int tok = cur.t0 + wave * kTokPerWave + col / G;
-        limit[cb] = tok < cur.sq ? (causal ? max(0, cur.L - cur.sq + tok + 1) : cur.L) : 0;
+        for (int cb = 0; cb < 2; ++cb) {
+          const int col = 32 * cb + (lane_c & 31);
+          const int tok = cur.t0 + wave * kTokPerWave + col / G;
+          limit[cb] = tok < cur.sq ? (causal ? max(0, cur.L - cur.sq + tok + 1) : cur.L) : 0;
+        }
+        asm volatile(FLASHW_SET_LIMIT ::"v"(limit[0] - 4 * half), "v"(limit[1] - 4 * half) : FLASHW_CLOBBERS);
+        int wm = min(limit[0], limit[1]);
+#pragma unroll
+        for (int x = 32; x > 0; x >>= 1) wm = min(wm, __shfl_xor(wm, x));
+        wave_min_limit = __builtin_amdgcn_readfirstlane(wm);
       }
-      asm volatile(FLASHW_SET_LIMIT ::"v"(limit[0] - 4 * half), "v"(limit[1] - 4 * half) : FLASHW_CLOBBERS);
-      int wm = min(limit[0], limit[1]);
-#pragma unroll
-      for (int x = 32; x > 0; x >>= 1) wm = min(wm, __shfl_xor(wm, x));
-      wave_min_limit = __builtin_amdgcn_readfirstlane(wm);
-    }
-    // the block's query rows and first tiles have landed (and the last block's output stores are out)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    asm volatile(FLASHW_Q_FROM_LDS ::[qoff] "s"(ldsq) : FLASHW_CLOBBERS);
-    FLASHW_ASM(FLASHW_INIT);
+      // the block's query rows and first tiles have landed (and the last block's output stores are out)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      asm volatile(FLASHW_Q_FROM_LDS ::[qoff] "s"(ldsq) : FLASHW_CLOBBERS);
+      FLASHW_ASM(FLASHW_INIT);
 
-    if (n_tiles > 0) {
-      asm volatile("s_barrier" ::: "memory");
-      FLASHW_ASM(FLASHW_QK_FIRST);
-      // The statements repeat with period six (LDS slots and score buffers are immediates), so the loop over the
-      // tiles is unrolled by six; tile 0 (nothing to multiply by V yet) stands in front.
-      int t = 0, flag;
+      if (n_tiles > 0) {
+        asm volatile("s_barrier" ::: "memory");
+        FLASHW_ASM(FLASHW_QK_FIRST);
+        // The statements repeat with period six (LDS slots and score buffers are immediates), so the loop over the
+        // tiles is unrolled by six; tile 0 (nothing to multiply by V yet) stands in front.
+        int t = 0, flag;
 #define FLASHW_HALF_A(TEXT) asm volatile(TEXT : [flag] "=&s"(flag) : [c] "s"(scale_log2e) : FLASHW_CLOBBERS)
 #define FLASHW_STEP(A_TEXT, A_TEXT_M, B_TEXT, B_TEXT_LAST)                                                          \
-  {                                                                                                                 \
-    if ((t + 1) * kKeysPerTile > wave_min_limit) {                                                                  \
-      asm volatile(A_TEXT_M : [flag] "=&s"(flag) : [c] "s"(scale_log2e), [t64] "s"(t * kKeysPerTile) : FLASHW_CLOBBERS); \
-    } else {                                                                                                        \
-      FLASHW_HALF_A(A_TEXT);                                                                                        \
-    }                                                                                                               \
-    if (flag) FLASHW_ASM(FLASHW_RESCALE);                                                                           \
-    if (++t < n_tiles) {                                                                                            \
-      const u32x4_t rk = next_k();                                                                                  \
-      const u32x4_t rv = next_v();                                                                                  \
-      asm volatile(B_TEXT ::[c] "s"(scale_log2e), [rk] "s"(rk), [rv] "s"(rv), [ldsw] "s"(ldsw) : FLASHW_CLOBBERS);  \
-    } else {                                                                                                        \
-      asm volatile(B_TEXT_LAST ::[c] "s"(scale_log2e) : FLASHW_CLOBBERS);                                           \
-      break;                                                                                                        \
-    }                                                                                                               \
-  }
-      do {
-        FLASHW_STEP(FLASHW_A_FIRST, FLASHW_A_FIRST_M, FLASHW_B0, FLASHW_B0_LAST)
-        for (;;) {
-          FLASHW_STEP(FLASHW_A1, FLASHW_A1_M, FLASHW_B1, FLASHW_B1_LAST)
-          FLASHW_STEP(FLASHW_A2, FLASHW_A2_M, FLASHW_B2, FLASHW_B2_LAST)
-          FLASHW_STEP(FLASHW_A3, FLASHW_A3_M, FLASHW_B3, FLASHW_B3_LAST)
-          FLASHW_STEP(FLASHW_A4, FLASHW_A4_M, FLASHW_B4, FLASHW_B4_LAST)
-          FLASHW_STEP(FLASHW_A5, FLASHW_A5_M, FLASHW_B5, FLASHW_B5_LAST)
-          FLASHW_STEP(FLASHW_A0, FLASHW_A0_M, FLASHW_B0, FLASHW_B0_LAST)
-        }
-      } while (false);
+    {                                                                                                                 \
+      if ((t + 1) * kKeysPerTile > wave_min_limit) {                                                                  \
+        asm volatile(A_TEXT_M : [flag] "=&s"(flag) : [c] "s"(scale_log2e), [t64] "s"(t * kKeysPerTile) : FLASHW_CLOBBERS); \
+      } else {                                                                                                        \
+        FLASHW_HALF_A(A_TEXT);                                                                                        \
+      }                                                                                                               \
+      if (flag) FLASHW_ASM(FLASHW_RESCALE);                                                                           \
+      if (++t < n_tiles) {                                                                                            \
+        const u32x4_t rk = next_k();                                                                                  \
+        const u32x4_t rv = next_v();                                                                                  \
+        asm volatile(B_TEXT ::[c] "s"(scale_log2e), [rk] "s"(rk), [rv] "s"(rv), [ldsw] "s"(ldsw) : FLASHW_CLOBBERS);  \
+      } else {                                                                                                        \
+        asm volatile(B_TEXT_LAST ::[c] "s"(scale_log2e) : FLASHW_CLOBBERS);                                           \
+        break;                                                                                                        \
+      }                                                                                                               \
+    }
+        do {
+          FLASHW_STEP(FLASHW_A_FIRST, FLASHW_A_FIRST_M, FLASHW_B0, FLASHW_B0_LAST)
+          for (;;) {
+            FLASHW_STEP(FLASHW_A1, FLASHW_A1_M, FLASHW_B1, FLASHW_B1_LAST)
+            FLASHW_STEP(FLASHW_A2, FLASHW_A2_M, FLASHW_B2, FLASHW_B2_LAST)
+            FLASHW_STEP(FLASHW_A3, FLASHW_A3_M, FLASHW_B3, FLASHW_B3_LAST)
+            FLASHW_STEP(FLASHW_A4, FLASHW_A4_M, FLASHW_B4, FLASHW_B4_LAST)
+            FLASHW_STEP(FLASHW_A5, FLASHW_A5_M, FLASHW_B5, FLASHW_B5_LAST)
+            FLASHW_STEP(FLASHW_A0, FLASHW_A0_M, FLASHW_B0, FLASHW_B0_LAST)
+          }
+        } while (false);
 #undef FLASHW_STEP
 #undef FLASHW_HALF_A
-      const int i = t % 6;                      // of the tile behind the last: its half A alone is left (O += V^T . P^T)
-      switch (i) {
-        case 0: FLASHW_ASM(FLASHW_PV0); break;
-        case 1: FLASHW_ASM(FLASHW_PV1); break;
-        case 2: FLASHW_ASM(FLASHW_PV2); break;
-        case 3: FLASHW_ASM(FLASHW_PV3); break;
-        case 4: FLASHW_ASM(FLASHW_PV4); break;
-        case 5: FLASHW_ASM(FLASHW_PV5); break;
+        const int i = t % 6;                      // of the tile behind the last: its half A alone is left (O += V^T . P^T)
+        switch (i) {
+          case 0: FLASHW_ASM(FLASHW_PV0); break;
+          case 1: FLASHW_ASM(FLASHW_PV1); break;
+          case 2: FLASHW_ASM(FLASHW_PV2); break;
+          case 3: FLASHW_ASM(FLASHW_PV3); break;
+          case 4: FLASHW_ASM(FLASHW_PV4); break;
+          case 5: FLASHW_ASM(FLASHW_PV5); break;
+        }
+        // nothing may still be writing LDS (the tiles requested past the block's end), and every wavefront must be
+        // done reading the rings, when the next block's tiles are requested (or the workgroup ends)
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
       }
-      // nothing may still be writing LDS (the tiles requested past the block's end), and every wavefront must be
-      // done reading the rings, when the next block's tiles are requested (or the workgroup ends)
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
     if (have_next) request_block(nxt);
 
     // ---- the finished block's output
-    FLASHW_ASM(FLASHW_DRAIN);
-    float m0, m1, lsum[2];
-    asm volatile(FLASHW_GET_ML : "=v"(m0), "=v"(m1), "=v"(lsum[0]), "=v"(lsum[1]));
-    int lane_e = lane;
-    asm volatile("" : "+v"(lane_e));
-    int64_t orow_e[2];
-    bool ok_e[2];
+    if (have) {
+      FLASHW_ASM(FLASHW_DRAIN);
+      float m0, m1, lsum[2];
+      asm volatile(FLASHW_GET_ML : "=v"(m0), "=v"(m1), "=v"(lsum[0]), "=v"(lsum[1]));
+      int lane_e = lane;
+      asm volatile("" : "+v"(lane_e));
+      int64_t orow_e[2];
+      bool ok_e[2];
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-      const int col = 32 * cb + (lane_e & 31);
-      const int tk = cur.t0 + wave * kTokPerWave + col / G;
-      ok_e[cb] = tk < cur.sq;
-      orow_e[cb] = ((int64_t)(cur.q_first + tk) * Hq + g * G + col % G) * kHeadDim + 8 * (lane_e >> 5);
-    }
-    // A lane holds dims 8 e4 + 4 half .. + 4 of each group of eight; the two halves of a wavefront trade one group
-    // of four per pair of groups (half-wave swap), after which a lane holds eight consecutive dims and stores 16 bytes
+      for (int cb = 0; cb < 2; ++cb) {
+        const int col = 32 * cb + (lane_e & 31);
+        const int tk = cur.t0 + wave * kTokPerWave + col / G;
+        ok_e[cb] = tk < cur.sq;
+        orow_e[cb] = ((int64_t)(cur.q_first + tk) * Hq + g * G + col % G) * kHeadDim + 8 * (lane_e >> 5);
+      }
+      // A lane holds dims 8 e4 + 4 half .. + 4 of each group of eight; the two halves of a wavefront trade one group
+      // of four per pair of groups (half-wave swap), after which a lane holds eight consecutive dims and stores 16 bytes
 #define FLASHW_STORE(CB, D)                                                                              \
-  {                                                                                                      \
-    float x[16];                                                                                         \
-    FLASHW_GETO(CB, D, x);                                                                               \
-    uint32_t w[8];                                                                                       \
-    _Pragma("unroll") for (int i = 0; i < 8; ++i) w[i] = pack_bf16x2(x[2 * i] * inv[CB], x[2 * i + 1] * inv[CB]); \
-    _Pragma("unroll") for (int pr = 0; pr < 2; ++pr) {                                                   \
-      const auto r0 = __builtin_amdgcn_permlane32_swap(w[4 * pr], w[4 * pr + 2], false, false);          \
-      const auto r1 = __builtin_amdgcn_permlane32_swap(w[4 * pr + 1], w[4 * pr + 3], false, false);      \
-      if (ok_e[CB])                                                                                      \
-        *reinterpret_cast<uint4*>(out + orow_e[CB] + 32 * D + 16 * pr) = make_uint4(r0[0], r1[0], r0[1], r1[1]); \
-    }                                                                                                    \
-  }
-    float inv[2];
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-      const int col = 32 * cb + (lane_e & 31);
-      inv[cb] = column_factor(opt, cb ? m1 : m0, half_wave_sum(lsum[cb]), g * G + col % G, cur.q_first + cur.t0 + wave * kTokPerWave + col / G,
-                              ok_e[cb]);
+    {                                                                                                      \
+      float x[16];                                                                                         \
+      FLASHW_GETO(CB, D, x);                                                                               \
+      uint32_t w[8];                                                                                       \
+      _Pragma("unroll") for (int i = 0; i < 8; ++i) w[i] = pack_bf16x2(x[2 * i] * inv[CB], x[2 * i + 1] * inv[CB]); \
+      _Pragma("unroll") for (int pr = 0; pr < 2; ++pr) {                                                   \
+        const auto r0 = __builtin_amdgcn_permlane32_swap(w[4 * pr], w[4 * pr + 2], false, false);          \
+        const auto r1 = __builtin_amdgcn_permlane32_swap(w[4 * pr + 1], w[4 * pr + 3], false, false);      \
+        if (ok_e[CB])                                                                                      \
+          *reinterpret_cast<uint4*>(out + orow_e[CB] + 32 * D + 16 * pr) = make_uint4(r0[0], r1[0], r0[1], r1[1]); \
+      }                                                                                                    \
     }
-    FLASHW_STORE(0, 0) FLASHW_STORE(0, 1) FLASHW_STORE(0, 2) FLASHW_STORE(0, 3)
-    FLASHW_STORE(1, 0) FLASHW_STORE(1, 1) FLASHW_STORE(1, 2) FLASHW_STORE(1, 3)
+      float inv[2];
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) {
+        const int col = 32 * cb + (lane_e & 31);
+        inv[cb] = column_factor(opt, cb ? m1 : m0, half_wave_sum(lsum[cb]), g * G + col % G, cur.q_first + cur.t0 + wave * kTokPerWave + col / G,
+                                ok_e[cb]);
+      }
+      FLASHW_STORE(0, 0) FLASHW_STORE(0, 1) FLASHW_STORE(0, 2) FLASHW_STORE(0, 3)
+      FLASHW_STORE(1, 0) FLASHW_STORE(1, 1) FLASHW_STORE(1, 2) FLASHW_STORE(1, 3)
 #undef FLASHW_STORE
+    }
+    if (!have_next) break;
     cur = nxt;
-    have = have_next;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #endif
@@ -782,7 +842,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVg
 template <int G>
 int flash_wide_launch_g(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                         const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
-                        int32_t causal, void* out, const RowOptions& opt, hipStream_t st) {
+                        int32_t causal, void* out, bool in_turn, const RowOptions& opt, hipStream_t st) {
   constexpr int kTokPerBlock = 4 * 64 / G;
   const int64_t blocks = ((int64_t)total_q + kTokPerBlock - 1) / kTokPerBlock + B;   // upper bound over ragged samples
   MSA_REQUIRE(blocks < (int64_t)1 << 30, "flash attention: too many query rows");
@@ -796,7 +856,7 @@ int flash_wide_launch_g(const void* q, const int32_t* cu_q, const void* k, const
   MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(kern), kWideLdsBytes));
   kern<<<dim3((unsigned)(per_head * Hkv)), 256, kWideLdsBytes, st>>>(
       static_cast<const bf16_t*>(q), cu_q, static_cast<const bf16_t*>(k), static_cast<const bf16_t*>(v), kv_off, kv_len,
-      B, Hq, Hkv, scale * kLog2e, causal, static_cast<bf16_t*>(out), (int32_t)blocks, opt);
+      B, Hq, Hkv, scale * kLog2e, causal, static_cast<bf16_t*>(out), in_turn, opt);
   MSA_LAUNCH_CHECK();
   return MSA_OK;
 }
@@ -849,12 +909,41 @@ int flash_launch(int G, Args... args) {
 }  // namespace
 
 namespace {
+// Where the wide form is ahead.  A workgroup of it has one block of 256 columns at a time and the launch ends with the last of them, where the
+// 32-column form has two workgroups a unit and smaller blocks: it wants long blocks and several of them a workgroup (rounds), or samples of
+// about one length in full blocks that fill an even number of rounds.  Few query heads to a key head share fewer of its rows, so with one or two the samples
+// have to be longer still.  us, 32-column form and wide, 32 heads over 8: 16 samples of 2048 to 4096 behind 291 keys 1503 and 1429, 8 773 and 733,
+// two of 4000 (7.8 rounds) 265 and 262, 20000 rows 3100 and 2918, 4096 148 and 140, 4000 159 and 149, 8 of 1024 102 and 98,
+// 2200 and 1780 92 and 89; but 3500 and 2160 (2.8
+// rounds) 149 and 161, three of 1500 to 3000 (3.6) 175 and 181, 5000 rows (2.5) 222 and 232, 16 of 1440 on average 475 and 473, of 1000 179 and 193, 12 of
+// 500 61 and 75, 1024 rows 26 and 36, documents of 256 to 2048 456 and 469; over 4: 12 of 4000 1077 and 1032, 3 of 3000 158 and 165; over 32: 20000 3127 and
+// 3022, 10000 833 and 834, 12 of 4000 1030 and 1109.
+enum Form { kColumns32, kWide, kWideInTurn };
+Form form_for(int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv) {
+  const int G = Hkv > 0 ? Hq / Hkv : 0;
+  if (G <= 0 || G > 8 || B <= 0 || (int64_t)total_q * G < 4096) return kColumns32;
+  const int64_t turn = std::max(1, device_compute_units() / Hkv);
+  const float rounds = (float)total_q * G / (256.f * turn), mean = (float)total_q / B;
+  int64_t blocks = 0;
+  if ((int64_t)max_sq * B == total_q) {
+    const int64_t columns = (int64_t)max_sq * G, each = (columns + 255) / 256;
+    if (each >= 4 && 16 * (256 * each - columns) <= columns) blocks = each * B;
+  } else if ((int64_t)max_sq * B <= (int64_t)total_q + total_q / 4 && mean * G >= 16 * 256.f) {
+    blocks = (int64_t)total_q * G / 256 + B / 2;
+  }
+  // (of more than three lengths back and forth comes out less even: 6 of 770 to 1540 172 and 161)
+  if (blocks > 0 && (blocks + turn / 8) % (2 * turn) <= turn / 8) return B <= 3 || (int64_t)max_sq * B == total_q ? kWideInTurn : kWide;
+  if (G >= 4 && mean >= 2000.f && rounds >= (mean >= 3000.f ? 3.25f : 7.f)) return kWide;
+  if (mean >= 12000.f && rounds >= 3.f) return kWide;
+  return kColumns32;
+}
+// What msa_flash_attn and msa_flash_attn_hint promise: the wide form from 4096 columns on, unless the batch is known to be ragged.
 bool wide_enough(int32_t total_q, int32_t Hq, int32_t Hkv) { return Hkv > 0 && (int64_t)total_q * (Hq / Hkv) >= 4096; }
 RowOptions dense_rows(int32_t Hq, int32_t D) { return {(int64_t)Hq * D, nullptr, nullptr, 0, nullptr}; }
 
 int flash_attn_entry(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                      const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D, float scale,
-                     int32_t causal, void* out, int32_t max_sq, bool enough, const RowOptions& opt, void* stream) {
+                     int32_t causal, void* out, Form wide, const RowOptions& opt, void* stream) {
   MSA_REQUIRE(q && k && v && kv_off && (kv_len || opt.kv_pos) && out, "msa_flash_attn: null pointer");
   MSA_REQUIRE(opt.q_stride >= (int64_t)Hq * D && opt.q_stride % 8 == 0 && (!opt.gate || opt.gate_stride >= Hq), "msa_flash_attn: strides");
   MSA_REQUIRE(D == kHeadDim, "msa_flash_attn: head dim %d unsupported (need %d)", D, kHeadDim);
@@ -866,14 +955,9 @@ int flash_attn_entry(const void* q, const int32_t* cu_q, const void* k, const vo
               "msa_flash_attn: q, k, v and out must be 16-byte aligned");
   const int G = Hq / Hkv;
   MSA_REQUIRE(G == 1 || G == 2 || G == 4 || G == 8, "msa_flash_attn: GQA group size %d unsupported (1, 2, 4, 8)", G);
-  // The wide form wants enough columns to fill its 256-column workgroups, and query blocks of about one length: its
-  // persistent launch deals the blocks out in a fixed order, which a batch of ragged samples unbalances (a packed
-  // block of 30 documents of 256 - 2048 tokens measured 6 % slower than with the 32-column form, whose workgroups
-  // the hardware hands out one by one)
   const int form = g_flash_form.load(std::memory_order_relaxed);
-  const bool ragged = max_sq > 0 && (int64_t)max_sq * B > (int64_t)total_q + total_q / 4;
-  if (form == 2 || (form == 0 && enough && !ragged))
-    return flash_wide_launch(G, q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, out, opt, as_stream(stream));
+  if (form == 2 || (form == 0 && wide != kColumns32))
+    return flash_wide_launch(G, q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, out, wide == kWideInTurn, opt, as_stream(stream));
   return flash_launch<false>(G, q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale,
                              causal, out, SplitPlan{1, 0}, (float*)nullptr, (float*)nullptr, opt, as_stream(stream));
 }
@@ -882,7 +966,7 @@ int flash_attn_entry(const void* q, const int32_t* cu_q, const void* k, const vo
 extern "C" int msa_flash_attn(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                               const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D,
                               float scale, int32_t causal, void* out, void* stream) {
-  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, 0, wide_enough(total_q, Hq, Hkv),
+  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, wide_enough(total_q, Hq, Hkv) ? kWide : kColumns32,
                           dense_rows(Hq, D), stream);
 }
 
@@ -890,7 +974,16 @@ extern "C" int msa_flash_attn_hint(const void* q, const int32_t* cu_q, const voi
                                    const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D,
                                    float scale, int32_t causal, void* out, int32_t max_sq, void* stream) {
   MSA_REQUIRE(max_sq > 0, "msa_flash_attn_hint: max_sq must be the longest query block of the batch");
-  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, max_sq, wide_enough(total_q, Hq, Hkv),
+  const bool ragged = (int64_t)max_sq * B > (int64_t)total_q + total_q / 4;
+  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, wide_enough(total_q, Hq, Hkv) && !ragged ? kWide : kColumns32,
+                          dense_rows(Hq, D), stream);
+}
+
+extern "C" int msa_flash_attn_fit(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
+                                  const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D,
+                                  float scale, int32_t causal, void* out, int32_t max_sq, void* stream) {
+  MSA_REQUIRE(max_sq > 0, "msa_flash_attn_fit: max_sq must be the longest query block of the batch");
+  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, form_for(B, total_q, max_sq, Hq, Hkv),
                           dense_rows(Hq, D), stream);
 }
 
@@ -899,18 +992,7 @@ extern "C" int msa_flash_attn_rows(const void* q, int64_t q_stride, const int32_
                                    float scale, const float* sink, const void* gate, int64_t gate_stride, void* out, void* stream) {
   MSA_REQUIRE(cu_q && kv_pos && max_sq > 0, "msa_flash_attn_rows: cu_q, kv_pos and max_sq are required");
   MSA_REQUIRE((int64_t)max_sq * q_stride < (int64_t)1 << 30, "msa_flash_attn_rows: query rows too far apart");
-  // The wide form's workgroups take its blocks of 256 columns in turn, back and forth, so their work is even where all samples are as
-  // long, in full blocks, and a head's blocks fill an even number of turns; elsewhere it waits for the longest of them.  us, 32-column form
-  // and wide, 16 heads: 8192 rows 254 and 240, four samples of 2048 92 and 78, eight of 1024 60 and 54; 32: 4096 134 and 129, 8192 500 and
-  // 475, four of 1024 behind 4000 keys 287 and 270; but 16 heads: 4096 rows 92 and 102, two of 3500 112 and 168, four of 2500 126 and 181; 32:
-  // 6001 283 and 300, three of 3000 over 8 key heads 230 and 249, ten of 600 65 and 90, eight of 800 79 and 94, of 512 43 and 45.
-  const int G = Hkv > 0 ? Hq / Hkv : 0;
-  bool even = false;
-  if (G > 0 && G <= 8 && (int64_t)max_sq * B == total_q) {
-    const int64_t columns = (int64_t)max_sq * G, blocks = (columns + 255) / 256, turn = std::max(1, device_compute_units() / Hkv);
-    even = blocks >= 4 && 16 * (256 * blocks - columns) <= columns && B * blocks % (2 * turn) == 0;
-  }
-  return flash_attn_entry(q, cu_q, k, v, kv_off, nullptr, B, total_q, Hq, Hkv, D, scale, 1, out, max_sq, even,
+  return flash_attn_entry(q, cu_q, k, v, kv_off, nullptr, B, total_q, Hq, Hkv, D, scale, 1, out, form_for(B, total_q, max_sq, Hq, Hkv),
                           {q_stride, sink, static_cast<const bf16_t*>(gate), gate_stride, kv_pos}, stream);
 }
 
