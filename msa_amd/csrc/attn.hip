@@ -810,7 +810,8 @@ int paired_splits(int32_t B, int32_t Hkv, int32_t Lcap) {
 extern "C" size_t msa_attn_workspace_bytes(int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D, int32_t max_kv) {
   if (total_q <= 0 || Hq <= 0 || Hkv <= 0 || D <= 0 || max_kv <= 0) return 0;
   // sized for whichever of the kernels has more partials
-  return partials_bytes(total_q, Hq, D, std::max(rows_splits(total_q, Hkv, max_kv), paired_splits(total_q, Hkv, max_kv)));
+  const int by_tiles = plan_splits_tiles(total_q, 1, Hq / Hkv, Hkv, max_kv).n_split;
+  return partials_bytes(total_q, Hq, D, std::max({rows_splits(total_q, Hkv, max_kv), paired_splits(total_q, Hkv, max_kv), by_tiles}));
 }
 
 extern "C" int msa_sparse_attn(const void* q, const int32_t* cu_q, const void* k, const void* v,
@@ -829,7 +830,9 @@ extern "C" int msa_sparse_attn(const void* q, const int32_t* cu_q, const void* k
               "msa_sparse_attn: q, k, v and out must be 16-byte aligned");
   MSA_REQUIRE((int64_t)total_q * Hq < (int64_t)1 << 31 && total_q < 65536 * 32, "msa_sparse_attn: too many rows");
   const bool mfma = dtype == MSA_BF16 && max_sq >= 8;
-  const SplitPlan plan = mfma ? plan_splits(total_q, Hkv, max_kv) : plan_splits_rows(total_q, Hkv, max_kv, dtype == MSA_BF16 && takes_ring(total_q, Hkv, max_kv, Hq / Hkv));
+  const SplitPlan tiles = plan_splits_tiles(total_q, B, Hq / Hkv, Hkv, max_kv);
+  const bool by_tiles = mfma && partials_bytes(total_q, Hq, D, tiles.n_split) <= workspace_bytes;
+  const SplitPlan plan = by_tiles ? tiles : mfma ? plan_splits(total_q, Hkv, max_kv) : plan_splits_rows(total_q, Hkv, max_kv, dtype == MSA_BF16 && takes_ring(total_q, Hkv, max_kv, Hq / Hkv));
   const int n_split = plan.n_split;
   MSA_REQUIRE(n_split <= 65535, "msa_sparse_attn: max_kv=%d too large", max_kv);
   const size_t need = partials_bytes(total_q, Hq, D, rows_splits(total_q, Hkv, max_kv));

@@ -25,6 +25,16 @@ static inline SplitPlan plan_splits_for(int64_t total_q, int32_t Hkv, int32_t ma
 static inline SplitPlan plan_splits(int64_t total_q, int32_t Hkv, int32_t max_kv) {
   return plan_splits_for(total_q, Hkv, max_kv, 1024);
 }
+// The same for blocks of query rows, by what the kernel makes workgroups of: tiles of 128 (token, head) columns, at least one a sample, and
+// two workgroups a compute unit.  By rows, as above, 128 rows of 8 KV heads were 1024 pairs and never split.  us, by rows and by tiles, 8 KV heads, groups of
+// four: one sample of 64 rows and 4096 keys 44.1 and 27.8, of 128 77.0 and 31.3, of 256 80.7 and 39.6, of 512 88.9 and 54.2, 4 of 64 79.0 and 43.3,
+// 8 of 64 83.9 and 59.0, 16 of 64 111 and 101; 2048 keys, one of 128 45.7 and 28.3.
+static inline SplitPlan plan_splits_tiles(int64_t total_q, int64_t samples, int G, int32_t Hkv, int32_t max_kv) {
+  const int64_t tiles = std::max(samples, (total_q * G + 127) / 128) * Hkv;
+  const int by_fill = (int)std::min<int64_t>(16, std::max<int64_t>(1, 512 / tiles)), by_size = std::max(1, (max_kv + kMinSplitKeys - 1) / kMinSplitKeys);
+  const int n = std::min(by_fill, by_size), keys = ((max_kv + n - 1) / n + 63) / 64 * 64;
+  return {(max_kv + keys - 1) / keys, keys};
+}
 // Single rows (decode): one workgroup per compute unit (fewer, longer key streams); the kernels divide each sample's own length
 // evenly over n_split.  The bf16 ring, of which two fit, is cut finer where that does not come out even and leaves 256 keys a split
 // or more (groups of four, us: 24 samples of 2200 to 4400 keys with 2 KV heads in 288 workgroups 28.2, in 528 23.6; but 16 of 256 to
