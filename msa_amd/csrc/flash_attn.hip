@@ -586,7 +586,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kWideCompilerVg
         block = causal ? nb - 1 - (pos - before) : pos - before;
         const int last_tok = min(sq_b, (block + 1) * kTokPerBlock) - 1;
         const int kmax = causal ? max(0, min(L, L - sq_b + last_tok + 1)) : L;
-        cost = 3 + min(kmax / (kKeysPerTile / 2), 1 << 20);        // (a block's start and end take as long as a tile and a half)
+        cost = 3 + min(max(0, kmax) / (kKeysPerTile / 2), 1 << 20);        // (a block's start and end take as long as a tile and a half)
         first_of = first;
         sq_of = sq_b;
         keys_of = L;

@@ -35,3 +35,11 @@ def test_against_the_oracle(lens, mem):
         want = cf.attention(q[cu[b]:cu[b + 1]], k[off[b]:off[b] + kv[b]], v[off[b]:off[b] + kv[b]], causal=True)
         for o in got:
             assert cf.rel_err(o[cu[b]:cu[b + 1]], want) < 1e-2
+
+
+def test_no_keys_are_refused():
+    from msa_amd import _lib, ops
+    q, k = torch.zeros((16, 32, 128), device="cuda").bfloat16(), torch.zeros((1, 8, 128), device="cuda").bfloat16()
+    cu = torch.tensor([0, 16]).int().cuda()
+    with pytest.raises(_lib.MsaError):
+        ops.sparse_attn(q, k, k, torch.zeros(1, dtype=torch.int64, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda"), 0, cu_q=cu, max_sq=16)
