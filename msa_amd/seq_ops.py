@@ -4,7 +4,6 @@ from __future__ import annotations
 
 import ctypes as C
 from dataclasses import dataclass
-from functools import lru_cache
 from typing import Optional, Sequence
 
 import numpy as np
@@ -339,7 +338,6 @@ def delta(qkv, a, b, gate, A_log, dt_bias, norm, eps: float, H: int, G: int, D: 
     return out
 
 
-@lru_cache(maxsize=None)
 def delta_step(qkv, a_low, g_low, w_low, n_a: int, b, A_log, dt_bias, norm, eps: float, H: int, G: int, D: int, E: int, state,
                batch: StepBatch) -> torch.Tensor:
     """:func:`delta` for one bf16 token a sequence, D and E up to 128, with ``a = a_low @ w_low[:H D].T`` and
