@@ -516,8 +516,8 @@ __device__ __forceinline__ int place_of(uint32_t key, bool all) {
 // 64 workgroups a head, several groups deal every second, third, .. position).  A round's lookup takes 0.8 us (code
 // that is cold each time) and 1.7 with rankings, a fixed order of back and forth 0.5, which however leaves the longest
 // of the workgroups 10 to 50 % behind the mean with ragged samples: 4 of 1000 to 2000 tokens 189 and 160 us, three of
-// 2700 to 3500 314 and 252, 16 of 2048 to 4096 1447 and 1405; two of 1780 and 2200, whose blocks fill two rounds, 84 and
-// 87: with `in_turn` the order is that one.
+// 2700 to 3500 314 and 252, 16 of 2048 to 4096 1447 and 1405; and even where one sample's
+// blocks, or those of samples of one length, fill pairs of rounds: with `in_turn` the order is that one (form_for).
 // Blocks are pipelined: once a block's last product is issued its LDS rings are free, so the next block's first tiles
 // and its query rows (into 16 KB of LDS per wavefront behind the rings) are requested before the finished block's
 // output is scaled and stored, and the block after that is looked up while those loads are awaited.
@@ -922,26 +922,30 @@ namespace {
 // 32-column form has two workgroups a unit and smaller blocks: it wants long blocks and several of them a workgroup (rounds), or samples of
 // about one length in full blocks that fill an even number of rounds.  Few query heads to a key head share fewer of its rows, so with one or two the samples
 // have to be longer still.  us, 32-column form and wide, 32 heads over 8: 16 samples of 2048 to 4096 behind 291 keys 1503 and 1429, 8 773 and 733,
-// two of 4000 (7.8 rounds) 265 and 262, 20000 rows 3100 and 2918, 4096 148 and 140, 4000 159 and 149, 8 of 1024 102 and 98,
-// 2200 and 1780 92 and 89; but 3500 and 2160 (2.8
-// rounds) 149 and 161, three of 1500 to 3000 (3.6) 175 and 181, 5000 rows (2.5) 222 and 232, 16 of 1440 on average 475 and 473, of 1000 179 and 193, 12 of
+// two of 4000 (7.8 rounds) 258 and 253, 20000 rows 3100 and 2918, 4096 148 and 140, 4000 159 and 149, 8 of 1024 102 and 98,
+// 2100 and 1900 80 and 77, 2200 and 1780 80 and 82; but 3500 and 2160 (2.8 rounds) 149 and 161, three of 1500 to 3000 (3.6) 175 and 181, 5000 rows (2.5) 222 and 232, 16 of 1440 on average 475 and 473, of 1000 179 and 193, 12 of
 // 500 61 and 75, 1024 rows 26 and 36, documents of 256 to 2048 456 and 469; over 4: 12 of 4000 1077 and 1032, 3 of 3000 158 and 165; over 32: 20000 3127 and
 // 3022, 10000 833 and 834, 12 of 4000 1030 and 1109.
+// Blocks in turn, back and forth, come out even for one sample, and for samples of one length whose blocks and the workgroups of a head divide one
+// another (1.0 to 1.1 times the mean).  Elsewhere the longest blocks of two samples meet: 3000 and then 5000 rows of 16 heads over 4 took 213 us in turn
+// and take 152 dealt by length, 1780 and then 2200 of 32 over 8 114 and 82, two of 3950 of 16 over 4 209
+// and 143 (32-column form 147).
 enum Form { kColumns32, kWide, kWideInTurn };
-Form form_for(int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv) {
+Form form_for(int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv, int units) {
   const int G = Hkv > 0 ? Hq / Hkv : 0;
   if (G <= 0 || G > 8 || B <= 0 || (int64_t)total_q * G < 4096) return kColumns32;
-  const int64_t turn = std::max(1, device_compute_units() / Hkv);
+  const int64_t turn = std::max(1, units / Hkv);
   const float rounds = (float)total_q * G / (256.f * turn), mean = (float)total_q / B;
+  const bool equal = (int64_t)max_sq * B == total_q;
+  const int64_t columns = (int64_t)max_sq * G, each = (columns + 255) / 256;
   int64_t blocks = 0;
-  if ((int64_t)max_sq * B == total_q) {
-    const int64_t columns = (int64_t)max_sq * G, each = (columns + 255) / 256;
+  if (equal) {
     if (each >= 4 && 16 * (256 * each - columns) <= columns) blocks = each * B;
   } else if ((int64_t)max_sq * B <= (int64_t)total_q + total_q / 4 && mean * G >= 16 * 256.f) {
     blocks = (int64_t)total_q * G / 256 + B / 2;
   }
-  // (of more than three lengths back and forth comes out less even: 6 of 770 to 1540 172 and 161)
-  if (blocks > 0 && (blocks + turn / 8) % (2 * turn) <= turn / 8) return B <= 3 || (int64_t)max_sq * B == total_q ? kWideInTurn : kWide;
+  if (blocks > 0 && (blocks + turn / 8) % (2 * turn) <= turn / 8)
+    return equal && (B == 1 || turn % each == 0 || each % turn == 0) ? kWideInTurn : kWide;
   if (G >= 4 && mean >= 2000.f && rounds >= (mean >= 3000.f ? 3.25f : 7.f)) return kWide;
   if (mean >= 12000.f && rounds >= 3.f) return kWide;
   return kColumns32;
@@ -992,16 +996,23 @@ extern "C" int msa_flash_attn_fit(const void* q, const int32_t* cu_q, const void
                                   const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D,
                                   float scale, int32_t causal, void* out, int32_t max_sq, void* stream) {
   MSA_REQUIRE(max_sq > 0, "msa_flash_attn_fit: max_sq must be the longest query block of the batch");
-  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, form_for(B, total_q, max_sq, Hq, Hkv),
+  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, form_for(B, total_q, max_sq, Hq, Hkv, device_compute_units()),
                           dense_rows(Hq, D), stream);
 }
 
+extern "C" int msa_diag_flash_form(int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv, int32_t compute_units) {
+  return form_for(B, total_q, max_sq, Hq, Hkv, compute_units);
+}
+
+// us before this rule (the wide form for samples of one length in whole pairs of rounds) and with it: 16 heads 4096 rows 95 and 88, 3000 73 and 69,
+// two of 1503 behind 300 keys 52 and 46, 8192 249 and 246, 7000 210 both; 16 over 4: three of 2650 113 and 99, 3000 and 5000 155 and 153; 32 over 8: 4096
+// 135 and 131, three of 1344 64 and 59, two of 1950 77 and 80; 32: 6001 295 and 293, 10000 768 and 767.
 extern "C" int msa_flash_attn_rows(const void* q, int64_t q_stride, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                                    const int64_t* kv_pos, int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv, int32_t D,
                                    float scale, const float* sink, const void* gate, int64_t gate_stride, void* out, void* stream) {
   MSA_REQUIRE(cu_q && kv_pos && max_sq > 0, "msa_flash_attn_rows: cu_q, kv_pos and max_sq are required");
   MSA_REQUIRE((int64_t)max_sq * q_stride < (int64_t)1 << 30, "msa_flash_attn_rows: query rows too far apart");
-  return flash_attn_entry(q, cu_q, k, v, kv_off, nullptr, B, total_q, Hq, Hkv, D, scale, 1, out, form_for(B, total_q, max_sq, Hq, Hkv),
+  return flash_attn_entry(q, cu_q, k, v, kv_off, nullptr, B, total_q, Hq, Hkv, D, scale, 1, out, form_for(B, total_q, max_sq, Hq, Hkv, device_compute_units()),
                           {q_stride, sink, static_cast<const bf16_t*>(gate), gate_stride, kv_pos}, stream);
 }
 
