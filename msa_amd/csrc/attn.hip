@@ -712,6 +712,7 @@ int launch_combine(const float* part_ml, const float* part_acc, int64_t rows, in
 // of 2000 19.3 / 26.8 / 32.8.
 int spread_heads(int64_t head_splits, int G, int n_split) {
   constexpr int kUnits = 256;
+  if (G != 1 && G != 2 && G != 4 && G != 8) return 0;       // (two heads of a group of three would be of two groups; launch_attn refuses these)
   if (head_splits <= kUnits && n_split <= 2) return 1;
   return G >= 2 && head_splits <= 2 * kUnits ? 2 : 0;
 }
