@@ -62,6 +62,8 @@ def _compile(src: str) -> str:
 #  * rows_ring_kernel (rows_ring.h), attn_ring_kernel and attn_decode_fused_kernel (attn.hip): likewise, they count what
 #    their rings have in flight.  What the first requests into LDS in front of its loop is read by asm statements, for
 #    which the compiler does not wait: the first request has to be waited for in front of the first LDS read.
+#  * delta_step_kernel (seq_delta.hip): loads past the end of what it reads rely on the range check of the buffer, which compares
+#    the vector offset alone.  No scalar offsets.
 # ---------------------------------------------------------------------------------------------------------------
 CONTRACTS = {
     "route_score.hip": [("score_scan4_kernel", {"max_compiler_vgpr": 127, "no_agpr": True})],
@@ -70,6 +72,7 @@ CONTRACTS = {
     "linear.hip": [("rows_ring_kernel", {})],
     "seq_rows.hip": [("rows_ring_kernel", {})],
     "attn.hip": [("attn_ring_kernel", {}), ("attn_decode_fused_kernel", {})],
+    "seq_delta.hip": [("delta_step_kernel", {"no_scalar_offset": True})],
 }
 LDS_WAITS = {"linear.hip": "rows_ring_kernel", "seq_rows.hip": "rows_ring_kernel"}
 
@@ -81,10 +84,10 @@ def _device_asm(src: str, extra=()) -> str:
     return r.stdout
 
 
-def check_kernel_contracts(asm: str, kernel_substring: str, max_compiler_vgpr=None, no_agpr=False):
+def check_kernel_contracts(asm: str, kernel_substring: str, max_compiler_vgpr=None, no_agpr=False, no_scalar_offset=False):
     """Returns the list of violations found in the device assembly `asm` for every kernel whose symbol contains
     `kernel_substring`: scratch use or spills (always), and, outside inline-asm regions, vector registers above
-    `max_compiler_vgpr` / any accumulation register."""
+    `max_compiler_vgpr` / any accumulation register / any buffer access with a scalar offset."""
     problems = []
     lines = asm.split("\n")
     # function bodies: from "<symbol>:" to s_endpgm
@@ -115,6 +118,8 @@ def check_kernel_contracts(asm: str, kernel_substring: str, max_compiler_vgpr=No
                 problems.append(f"{name}: scratch access: {code}")
             if no_agpr and re.search(r"\ba\d+\b|\ba\[\d+|accvgpr", code):
                 problems.append(f"{name}: compiler-generated code touches an accumulation register: {code}")
+            if no_scalar_offset and re.match(r"buffer_(load|store)\w* .*\bs\[\d+:\d+\], (?!0\b)", code):
+                problems.append(f"{name}: buffer access with a scalar offset: {code}")
             if max_compiler_vgpr is not None:
                 for mm in re.finditer(r"\bv(\d+)\b|\bv\[(\d+):(\d+)\]", code):
                     hi = int(mm.group(1) or mm.group(3))

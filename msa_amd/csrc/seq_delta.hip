@@ -231,7 +231,8 @@ __global__ __launch_bounds__(RW * CW * 64) void delta_step_kernel(msa_delta_args
   const bool dense = b.rows == b.n_seq;
   const int row = dense ? s : b.cu[s], kvh = head / (a.H / a.G);
   if (!dense && b.cu[s + 1] == row) return;
-  float* const st = a.state + ((int64_t)b.slot[s] * a.H + head) * a.D * a.E;
+  const int slot = b.slot[s];
+  float* const st = a.state + ((int64_t)slot * a.H + head) * a.D * a.E;
   const bf16_t* const qkv = static_cast<const bf16_t*>(a.qkv) + row * a.qkv_stride;
 
   const __amdgpu_buffer_rsrc_t rs_w = bytes_rsrc(static_cast<const bf16_t*>(low.w) + (int64_t)head * a.D * low.rank, a.D * low.rank * 2);
@@ -240,15 +241,18 @@ __global__ __launch_bounds__(RW * CW * 64) void delta_step_kernel(msa_delta_args
   const __amdgpu_buffer_rsrc_t rs_xg = bytes_rsrc(static_cast<const bf16_t*>(low.g_low) + row * low.g_stride, low.rank * 2);
   u32x4_t wa[kTurnsA], wg[kTurnsG], xa, xg;
   auto fetch_low = [&](int unit) {
-    const int at = (tid >> 4) * low.rank * 2 + unit * 16, end = unit * 8 < low.rank ? 0 : kOutside;        // (a row's end, not the next row)
+    // (a row's end, not the next row; rows behind the head's own by the vector offset, which is what the range check compares)
+    const int at = unit * 8 < low.rank ? (tid >> 4) * low.rank * 2 + unit * 16 : kOutside, turn = kRows * low.rank * 2;
     xa = __builtin_amdgcn_raw_buffer_load_b128(rs_xa, unit * 16, 0, 0);
     xg = __builtin_amdgcn_raw_buffer_load_b128(rs_xg, unit * 16, 0, 0);
 #pragma unroll
-    for (int i = 0; i < kTurnsA; ++i) wa[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, at + end, i * kRows * low.rank * 2, 0);
+    for (int i = 0; i < kTurnsA; ++i) wa[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_w, at + i * turn, 0, 0);
 #pragma unroll
-    for (int i = 0; i < kTurnsG; ++i) wg[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_g, at + end, i * kRows * low.rank * 2, 0);
+    for (int i = 0; i < kTurnsG; ++i) wg[i] = __builtin_amdgcn_raw_buffer_load_b128(rs_g, at + i * turn, 0, 0);
   };
-  // ---- everything is requested
+  // ---- everything is requested, once the slot and all arguments are there (else they are waits in between)
+  asm volatile("" ::"s"(slot));
+  __builtin_amdgcn_sched_barrier(0);
   float k[kEach], q[kEach], bias = 0.f;
   const __amdgpu_buffer_rsrc_t rs_q = bytes_rsrc(qkv + (int64_t)kvh * a.D, a.D * 2), rs_k = bytes_rsrc(qkv + (int64_t)(a.G + kvh) * a.D, a.D * 2);
 #pragma unroll
