@@ -38,17 +38,21 @@ constexpr int kSchedCounterWords = 32;
 constexpr int kSchedMaxWorkgroups = 1024;
 constexpr size_t kSchedBytes = (size_t)(kSchedCounterWords + kSchedMaxWorkgroups) * sizeof(uint32_t);
 
-// Eight fp32 values as three bf16 operands whose sum they are: the first cut off (infinities stay, a NaN's remainder is one), the others
-// rounded, 8 + 9 + 8 bits or more together.
+// Eight fp32 values as three bf16 operands whose sum they are, each the rest rounded: up to 2^-8 and 2^-17 of the value behind the first.
+// kInfinite: a first part that would round to an infinity is cut off instead, and nothing is left of an infinity; without it either leaves a NaN.
 template <bool kInfinite>
 __device__ __forceinline__ void split_three(const float (&x)[8], uint4 (&part)[3]) {
   uint32_t w[3][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t a = __float_as_uint(x[2 * i]), b = __float_as_uint(x[2 * i + 1]);
-    const float a1 = __uint_as_float(a & 0xffff0000u), b1 = __uint_as_float(b & 0xffff0000u);
-    const float ra = kInfinite && x[2 * i] == a1 ? 0.f : x[2 * i] - a1, rb = kInfinite && x[2 * i + 1] == b1 ? 0.f : x[2 * i + 1] - b1;
-    w[0][i] = __builtin_amdgcn_perm(b, a, 0x07060302);
+    const float a = x[2 * i], b = x[2 * i + 1];
+    w[0][i] = pack_bf16x2(a, b);
+    if constexpr (kInfinite) {
+      if ((w[0][i] & 0x7f80u) == 0x7f80u) w[0][i] = (w[0][i] & 0xffff0000u) | __float_as_uint(a) >> 16;
+      if ((w[0][i] & 0x7f800000u) == 0x7f800000u) w[0][i] = (w[0][i] & 0xffffu) | (__float_as_uint(b) & 0xffff0000u);
+    }
+    const float a1 = bf16lo(w[0][i]), b1 = bf16hi(w[0][i]);
+    const float ra = kInfinite && a == a1 ? 0.f : a - a1, rb = kInfinite && b == b1 ? 0.f : b - b1;
     w[1][i] = pack_bf16x2(ra, rb);
     w[2][i] = pack_bf16x2(ra - bf16lo(w[1][i]), rb - bf16hi(w[1][i]));
   }
@@ -1313,8 +1317,10 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void score_split_kernel(const 
 
 // ------------------------------------------------------------------------------------------
 // fp32 banks of up to 32 chunks a compute unit: the same split of the work, the products on the bf16 matrix cores.  An fp32 value is
-// three bf16 ones exactly, and of the nine products of two values the six largest carry 24 bits (what is left out is below 2^-24 of
-// the product): 192 cycles where the fp32 form takes 512.  Errors of 8000 chunks x 64 rows against float64, all scores: 5.8e-8 of
+// three bf16 ones exactly, and of the nine products of two values the six largest are formed: 192 cycles where the fp32 form takes 512.  What
+// is left out is up to 2^-24 of a product (the second parts times the third ones), 2^-27 in the mean: with its own rounding a product is within
+// 2^-23 where the fp32 instruction gives 2^-24.  (First parts cut off instead of rounded: 2^-21.8.  Eight products, 2^-24: 8192 chunks x 1024
+// rows 127 -> 141 us, 1000 x 64 16.6 -> 17.1.)  Values below 2^-109 lose their last parts.  Errors of 8000 chunks x 64 rows against float64, all scores: 5.8e-8 of
 // their norm, 1.7e-7 there.  Eight wavefronts hold an eighth of K each, of their 32 chunks in three parts in 96 registers; the
 // queries come as operands from the prologue (part_at), a kilobyte a load, four steps of K ahead.  The first parts' products and the
 // others' have sums of their own, so that small ones are not rounded away one by one.  What bounds it: K_r from memory with few rows
@@ -1447,7 +1453,7 @@ __global__ __launch_bounds__(kPartsWaves * 64) void score_parts_kernel(const cha
           const char* qp = qs + part_at(32 * blk + row, x, kSplitK);
           for (int e = 0; e < 8; ++e) {
             auto piece = [&](int n) { return bf16_to_f32(reinterpret_cast<const bf16_t*>(qp + n * kPartBytes)[e]); };
-            v += ((piece(0) + piece(1)) + piece(2)) * kr[(int64_t)(n0 + l32) * kSplitK + x + e];
+            v += (piece(0) + (piece(1) + piece(2))) * kr[(int64_t)(n0 + l32) * kSplitK + x + e];
           }
         }
       }
