@@ -59,14 +59,14 @@ def _compile(src: str) -> str:
 #  * flash_wide_kernel (flash_attn.hip): likewise, its statements own v56-v255 and all accumulation registers.
 #  * flash_attn_kernel (flash_attn.hip): its direct-to-LDS loads are asm statements the compiler does not order
 #    against LDS reads; a spill would add vector-memory waits in the middle of that ring.  No scratch, no spills.
-#  * rows_ring_kernel (rows_ring.h), attn_ring_kernel and attn_decode_fused_kernel (attn.hip): likewise, they count what
+#  * score_parts_kernel (route_score.hip), rows_ring_kernel (rows_ring.h), attn_ring_kernel and attn_decode_fused_kernel (attn.hip): likewise, they count what
 #    their rings have in flight.  What the first requests into LDS in front of its loop is read by asm statements, for
 #    which the compiler does not wait: the first request has to be waited for in front of the first LDS read.
 #  * delta_step_kernel (seq_delta.hip): loads past the end of what it reads rely on the range check of the buffer, which compares
 #    the vector offset alone.  No scalar offsets.
 # ---------------------------------------------------------------------------------------------------------------
 CONTRACTS = {
-    "route_score.hip": [("score_scan4_kernel", {"max_compiler_vgpr": 127, "no_agpr": True})],
+    "route_score.hip": [("score_scan4_kernel", {"max_compiler_vgpr": 127, "no_agpr": True}), ("score_parts_kernel", {})],
     "gemm.hip": [("tile_gemm_kernel", {"max_compiler_vgpr": 127, "no_agpr": True}), ("tile_flow_kernel", {"max_compiler_vgpr": 23, "no_agpr": True})],
     "flash_attn.hip": [("flash_attn_kernel", {}), ("flash_wide_kernel", {"max_compiler_vgpr": 55, "no_agpr": True})],
     "linear.hip": [("rows_ring_kernel", {})],
