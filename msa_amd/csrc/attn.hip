@@ -547,55 +547,79 @@ struct NormRope {
   }
 };
 
-// kPaired (up to 64 samples): the pieces of samples of different lengths dealt so that two beside one another are about as long as any two.
+// kPaired (up to 64 samples): the pieces of samples of different lengths dealt so that two beside one another are about as long as any two.  The
+// host knows the caches' capacity only: where no sample has `worth` keys the pieces are `few`, in the launch's own order, as without kPaired, and
+// the other workgroups leave empty sums.  us, 8 KV heads, both launches, without kPaired, always paired and so: 16 samples of 100 keys in caches of 4388
+// 8.4, 10.0 and 8.7, of 1000 17.6, 17.8 and 17.9, 8 of 1000 in 4160 12.3, 14.3 and 12.7, 32 of 300 in 2048 13.1, 14.7 and 13.3.
 constexpr int kDecodeUnits = 256;
+struct Pairing {
+  int32_t worth, few;
+};
 template <bool kPaired>
 __global__ __launch_bounds__(kRingWaves * 64) void attn_decode_fused_kernel(
     const bf16_t* __restrict__ qkv, int64_t row_stride, int32_t Hq, int32_t Hkv, const int64_t* __restrict__ pos,
     const bf16_t* __restrict__ qw, const bf16_t* __restrict__ kw, float eps, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, int32_t rope_rows, bf16_t* __restrict__ kcache, bf16_t* __restrict__ vcache,
     int32_t Lcap, const int32_t* __restrict__ kv_len, float scale_log2e, int32_t n_split,
-    float* __restrict__ part_ml, float* __restrict__ part_acc) {
+    float* __restrict__ part_ml, float* __restrict__ part_acc, Pairing pairing) {
   extern __shared__ __align__(16) char lds[];
   HeadSums& new_token = sums_of(lds, kRingWaves);
   uint4* sm_q = reinterpret_cast<uint4*>(lds + kRingLds + sizeof(HeadSums));        // [G][16]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), G = Hq / Hkv;
-  int b = blockIdx.x, g = blockIdx.y, split = blockIdx.z, L_old;
+  int b = blockIdx.x, g = blockIdx.y, split = blockIdx.z, pieces = n_split, L_old;
   int64_t position;
+  const int j = lane & 15, hq = tid >> 4;                  // 16 lanes a head: the group's q heads, and behind them the new key
+  NormRope head;
+  uint4 v_new;
+  auto load_row = [&]() {
+    const bf16_t* row = qkv + (int64_t)b * row_stride + 8 * j;
+    head.load(row + (int64_t)(hq < G ? g * G + hq : Hq + g) * kHeadDim, (hq < G ? qw : kw) + 8 * j);
+    v_new = *reinterpret_cast<const uint4*>(row + (int64_t)(Hq + Hkv + g) * kHeadDim);
+  };
   if constexpr (kPaired) {
     // Units in the order of the workgroups, the longest samples first in each of their rounds, the second round (of those a compute unit has
     // two places for) backwards: whoever has a long piece gets a short one beside it.
     const int B = gridDim.x, total = B * Hkv * n_split, second = min(2 * kDecodeUnits, total);
     const int len = lane < B ? kv_len[lane] : 0;
     const int64_t at = lane < B ? pos[lane] : 0;
-    int unit = b + B * (g + Hkv * split);
-    if (unit >= kDecodeUnits && unit < second) unit = kDecodeUnits + second - 1 - unit;
-    const int row_of = unit / B, place = unit - row_of * B;
-    split = row_of / Hkv;
-    g = row_of - split * Hkv;
-    // a sample's place by length; no two keys are equal, and those of absent lanes come last
-    const uint32_t key = (uint32_t)min(max(len, 0), (1 << 25) - 1) * 64 + (63 - lane);
-    int rank = 0;
-    for (int i0 = 0; i0 < B; i0 += 16)
+    load_row();                                            // (of the launch's own order, under the lengths' way here)
+    if (__any(len >= pairing.worth)) {
+      int unit = b + B * (g + Hkv * split);
+      if (unit >= kDecodeUnits && unit < second) unit = kDecodeUnits + second - 1 - unit;
+      const int row_of = unit / B, place = unit - row_of * B;
+      split = row_of / Hkv;
+      g = row_of - split * Hkv;
+      // a sample's place by length; no two keys are equal, and those of absent lanes come last
+      const uint32_t key = (uint32_t)min(max(len, 0), (1 << 25) - 1) * 64 + (63 - lane);
+      int rank = 0;
+      for (int i0 = 0; i0 < B; i0 += 16)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) rank += (uint32_t)__builtin_amdgcn_readlane((int)key, i0 + i) > key;
-    b = __builtin_ctzll(__ballot(rank == place));
+        for (int i = 0; i < 16; ++i) rank += (uint32_t)__builtin_amdgcn_readlane((int)key, i0 + i) > key;
+      b = __builtin_ctzll(__ballot(rank == place));
+      load_row();
+    } else {
+      pieces = pairing.few;
+      if (split >= pieces) {
+        for (int idx = tid; idx < G * kHeadDim; idx += kRingWaves * 64) {
+          const int64_t o = ((int64_t)b * Hq + g * G + idx / kHeadDim) * n_split + split;
+          part_acc[o * kHeadDim + idx % kHeadDim] = 0.f;
+          if (idx % kHeadDim == 0) { part_ml[o * 2] = -INFINITY; part_ml[o * 2 + 1] = 0.f; }
+        }
+        return;
+      }
+    }
     L_old = __builtin_amdgcn_readlane(len, b);
     position = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)((uint64_t)at >> 32), b) << 32 | (uint32_t)__builtin_amdgcn_readlane((int)at, b));
   } else {
     L_old = kv_len[b];
     position = pos[b];
+    load_row();
   }
-  const int j = lane & 15, hq = tid >> 4;                  // 16 lanes a head: the group's q heads, and behind them the new key
-  const bf16_t* row = qkv + (int64_t)b * row_stride + 8 * j;
-  NormRope head;
-  head.load(row + (int64_t)(hq < G ? g * G + hq : Hq + g) * kHeadDim, (hq < G ? qw : kw) + 8 * j);
-  const uint4 v_new = *reinterpret_cast<const uint4*>(row + (int64_t)(Hq + Hkv + g) * kHeadDim);
   const int64_t p = min((int64_t)max((int64_t)0, position), (int64_t)rope_rows - 1);
   head.load_rotary(cos_t + p * 64, sin_t + p * 64, j);
 
   const bool has_new = L_old < Lcap;
-  const int per_split = (L_old + n_split - 1) / n_split, key0 = split * per_split, key1 = min(L_old, key0 + per_split);
+  const int per_split = (L_old + pieces - 1) / pieces, key0 = split * per_split, key1 = min(L_old, key0 + per_split);
   const int64_t column = ((int64_t)b * Lcap * Hkv + g) * kHeadDim;
   const Ring ring(kcache + column, vcache + column, Hkv * kRowBytes, key0, key1, wave, lane, lds);
   asm volatile("" ::: "memory");                           // (the requests above stay above: loads return in order)
@@ -604,7 +628,7 @@ __global__ __launch_bounds__(kRingWaves * 64) void attn_decode_fused_kernel(
   const uint4 prepared = head.result(eps, j);
   if (hq < G) lds_write16(sm_q + hq * 16 + j, prepared);
   // the new token: the first 16 lanes of the last wavefront of the last split
-  const bool takes_new = has_new && split == n_split - 1, owner = takes_new && wave == kRingWaves - 1 && lane < 16;
+  const bool takes_new = has_new && split == pieces - 1, owner = takes_new && wave == kRingWaves - 1 && lane < 16;
   if (owner) {
     const int64_t at = (((int64_t)b * Lcap + L_old) * Hkv + g) * kHeadDim + 8 * j;
     *reinterpret_cast<uint4*>(kcache + at) = prepared;
@@ -652,7 +676,7 @@ __global__ __launch_bounds__(kRingWaves * 64) void attn_decode_fused_kernel(
 }
 
 // One workgroup of 128 threads per (query row, head): merges the row's partials and normalises.  The partials are requested sixteen
-// at a time (one after the other, each waited for the one before: 32 of them took 16 us), four at a time where there are no more.  With `kv_len` (decode: rows = samples)
+// at a time (one after the other, each waited for the one before: 32 of them took 16 us), four or eight at a time where there are no more.  With `kv_len` (decode: rows = samples)
 // the workgroup of head 0 also advances the sample's cache length, unless the cache was full and the new row was dropped.
 template <typename T, int kBatch>
 __global__ __launch_bounds__(kHeadDim) void attn_combine_kernel(const float* __restrict__ part_ml,
@@ -698,7 +722,7 @@ __global__ __launch_bounds__(kHeadDim) void attn_combine_kernel(const float* __r
 template <typename T>
 int launch_combine(const float* part_ml, const float* part_acc, int64_t rows, int32_t n_split, void* out, hipStream_t st,
                    int32_t* kv_len = nullptr, int32_t Lcap = 0, int32_t Hq = 1) {
-  const auto kernel = n_split <= 4 ? attn_combine_kernel<T, 4> : attn_combine_kernel<T, 16>;
+  const auto kernel = n_split <= 4 ? attn_combine_kernel<T, 4> : n_split <= 8 ? attn_combine_kernel<T, 8> : attn_combine_kernel<T, 16>;
   kernel<<<(unsigned)rows, kHeadDim, 0, st>>>(part_ml, part_acc, n_split, static_cast<T*>(out), kv_len, Lcap, Hq);
   MSA_LAUNCH_CHECK();
   return MSA_OK;
@@ -805,6 +829,9 @@ int paired_splits(int32_t B, int32_t Hkv, int32_t Lcap) {
   if (n * pairs < 400) return 0;                           // (too few places taken: 24 samples of 2000 43.3 -> 44.0)
   return Lcap >= n * (kDecodeUnits % pairs == 0 ? 500 : 160) ? n : 0;
 }
+// From how many keys of the longest sample on the pieces are dealt in pairs, in a launch that has the workgroups for it: fewer than the capacity's
+// line above, where the choice is between these and half as many pieces in the same launch.
+Pairing pairing_of(int64_t pairs, int n, int even) { return {n * (n == 1 || kDecodeUnits % pairs == 0 ? 300 : 50), std::min(even, n)}; }
 
 }  // namespace
 
@@ -881,7 +908,7 @@ extern "C" int msa_decode_attn_fused(const void* qkv, int64_t row_stride, const 
     msa_set_error("msa_decode_attn_fused: workspace of %zu bytes, need %zu", workspace_bytes, need);
     return MSA_ESIZE;
   }
-  const int n_split = pairs ? paired : plan_splits_rows(B, Hkv, Lcap, true).n_split;
+  const int even = plan_splits_rows(B, Hkv, Lcap, true).n_split, n_split = pairs ? paired : even;
   const size_t n = (size_t)B * Hq * n_split;
   float* part_ml = static_cast<float*>(workspace);
   float* part_acc = reinterpret_cast<float*>(static_cast<char*>(workspace) + align_up(n * 2 * sizeof(float), 256));
@@ -892,7 +919,8 @@ extern "C" int msa_decode_attn_fused(const void* qkv, int64_t row_stride, const 
   kernel<<<dim3((unsigned)B, (unsigned)Hkv, (unsigned)n_split), kRingWaves * 64, kFusedLds, st>>>(
       static_cast<const bf16_t*>(qkv), row_stride, Hq, Hkv, positions, static_cast<const bf16_t*>(q_norm_w),
       static_cast<const bf16_t*>(k_norm_w), eps, rope_cos, rope_sin, rope_rows, static_cast<bf16_t*>(kcache),
-      static_cast<bf16_t*>(vcache), Lcap, kv_len, scale * 1.4426950408889634f, n_split, part_ml, part_acc);
+      static_cast<bf16_t*>(vcache), Lcap, kv_len, scale * 1.4426950408889634f, n_split, part_ml, part_acc,
+      pairs ? pairing_of((int64_t)B * Hkv, n_split, even) : Pairing{});
   MSA_LAUNCH_CHECK();
   return launch_combine<bf16_t>(part_ml, part_acc, (int64_t)B * Hq, n_split, out, st, kv_len, Lcap, Hq);
 }
