@@ -382,7 +382,9 @@ def sparse_attn(q, k, v, kv_off, kv_len, max_kv: int, cu_q=None, max_sq: int = 1
     # workgroups 400 keys, 16 550, 32 700, 64 1200, 128 1900, 256 5000 (us, flash and split: 128 rows of 32 heads over 8 and 640 keys 18.5 and 18.1,
     # 1152 26.7 and 20.3; 512 rows and 1024 keys 25.5 and 31.7, 2560 48.5 and 40.8; 4 samples of 500 rows and keys 26.2 and 47.5)
     tiles = Hkv * max(B, -(-total_q * (Hq // max(1, Hkv)) // 128))
-    if q.dtype == torch.bfloat16 and max_sq >= FLASH_MIN_ROWS and (tiles > 128 or 0 < max_kv <= 300 + 16 * tiles):
+    # (without keys: zeros from as many rows as fill the chip, refused below)
+    one_pass = tiles > 128 or max_kv <= 300 + 16 * tiles if max_kv > 0 else total_q * Hkv >= 32 * 512
+    if q.dtype == torch.bfloat16 and max_sq >= FLASH_MIN_ROWS and one_pass:
         out = torch.empty_like(q)
         check(lib.msa_flash_attn_fit(ptr(q), ptr(cu_q), ptr(k), ptr(v), ptr(kv_off), ptr(kv_len), B, total_q, Hq, Hkv, D,
                                      sc, int(causal), ptr(out), int(max_sq), _stream()), "msa_flash_attn")
