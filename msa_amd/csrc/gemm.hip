@@ -650,12 +650,13 @@ bool flows(const TileArgs& a, int mode) {
 }
 
 // The columns that fill whole rounds, where the others are better off in block_gemm.hip's smaller tiles (N: none).  A few tiles behind the
-// last whole round take a launch most of another one, whole or in pieces: `last`, fitted to 16 to 128 such tiles, 1024 and 2560 deep (less: not measured).  us,
+// last whole round take a launch most of another one, whole or in pieces: `last`, fitted to 16 to 128 such tiles, 1024 and 2560 deep (less: not measured;
+// more: level, 8192 x 3072 x 6176 233 and 234, x 4096 x 6176 301 and 302, 6001 x 9728 x 4608 384 and 380).  us,
 // rows x K x N, all tiles and split: 8192 x 1024 x 6176 (32 columns' tiles a fourth round) 98 and 87, x 2304 52 and 42, 6001 x 1024 x 3072 50
 // and 43, 8192 x 2560 x 4608 165 and 153, x 12368 442 and 431; level or behind, and not split: 8192 x 1024 x 3072 54 and 58, 6001 x 1024 x
 // 6176 74 and 76, x 2560 x 8480 204 and 205, 1700 x 2560 x 19456 glu 143 and 147.  The ends round their sums alike in both kernels where the tiles' end flows.
 int whole_columns(const TileArgs& a, int mode) {
-  if ((mode != kStore && mode != kGelu && mode != kGlu) || (mode != kStore && !flows(a, mode)) || a.K < 1024) return a.N;
+  if ((mode != kStore && mode != kGelu && mode != kGlu) || (mode != kStore && !flows(a, mode)) || a.K < 1024 || a.K > 2560) return a.N;
   const int tiles_t = (a.T + kTile - 1) / kTile, tiles_n = (a.N + kTile - 1) / kTile;
   const int units = std::max(kXcds * 2, device_compute_units() / kXcds * kXcds), rounds = (int)((int64_t)tiles_t * tiles_n / units);
   const int columns = (int)((int64_t)rounds * units / tiles_t), behind = (int)((int64_t)tiles_t * tiles_n - (int64_t)rounds * units);
