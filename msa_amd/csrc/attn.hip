@@ -733,10 +733,12 @@ int launch_combine(const float* part_ml, const float* part_acc, int64_t rows, in
 // (`head_splits`: with one head each; twice as many with two).  More than two splits are short already.  us, 8 KV heads of four, groups
 // / two heads / one: one row of 192 keys 11.4 / 9.0 / 8.1, 8 rows 12.5 / 8.6 / 7.3, 16 rows 13.5 / 9.5 / 12.2, 32 rows 15.3 / 15.4 /
 // 21.9; 2 rows of 400 keys in two splits 14.5 / 11.3 / 11.2, of 1000 in four 15.2 / 12.2 / 14.8, of 2000 in eight 16.2 / 15.6 / 25.3; 4 rows
-// of 2000 19.3 / 26.8 / 32.8.
-int spread_heads(int64_t head_splits, int G, int n_split) {
+// of 2000 19.3 / 26.8 / 32.8.  Groups of one and two are in four wavefronts then, which is as many as few keys keep busy (eight, so and now: one head,
+// 16 rows of 100 keys 7.1 / 6.1, 25 of 43 6.2 / 4.3; two, 4 rows of 82 6.4 / 4.7, one of 100 6.2 / 5.1, but 8 of 110 6.6 / 7.5).
+int spread_heads(int64_t head_splits, int G, int n_split, int max_kv) {
   constexpr int kUnits = 256;
   if (G != 1 && G != 2 && G != 4 && G != 8) return 0;       // (two heads of a group of three would be of two groups; launch_attn refuses these)
+  if ((G == 1 && max_kv <= 128) || (G == 2 && max_kv <= 104)) return 0;
   if (head_splits <= kUnits && n_split <= 2) return 1;
   return G >= 2 && head_splits <= 2 * kUnits ? 2 : 0;
 }
@@ -744,9 +746,8 @@ int spread_heads(int64_t head_splits, int G, int n_split) {
 template <typename T>
 int launch_attn(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                     const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, float scale,
-                    int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st) {
+                    int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st, int spread = 0) {
   const int n_split = plan.n_split;
-  const int spread = sizeof(T) == 4 ? spread_heads((int64_t)total_q * Hq * n_split, Hq / Hkv, n_split) : 0;
   const int G = spread ? spread : Hq / Hkv;
   dim3 grid((unsigned)total_q, (unsigned)(Hq / G), (unsigned)n_split);
   const float sl2 = scale * 1.4426950408889634f;
@@ -805,7 +806,9 @@ int launch_attn_bf16(const void* q, const int32_t* cu_q, const void* k, const vo
                      const int32_t* kv_len, int32_t B, int32_t total_q, int32_t max_kv, int32_t Hq, int32_t Hkv, float scale,
                      int32_t causal, SplitPlan plan, void* out, float* part_ml, float* part_acc, hipStream_t st) {
   const int G = Hq / Hkv;
-  const auto launch = !takes_ring(total_q, Hkv, max_kv, G) ? launch_attn<bf16_t> : G <= 2 ? launch_attn_ring<3> : launch_attn_ring<2>;
+  if (!takes_ring(total_q, Hkv, max_kv, G))
+    return launch_attn<bf16_t>(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml, part_acc, st);
+  const auto launch = G <= 2 ? launch_attn_ring<3> : launch_attn_ring<2>;
   return launch(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml, part_acc, st);
 }
 
@@ -883,8 +886,8 @@ extern "C" int msa_sparse_attn(const void* q, const int32_t* cu_q, const void* k
   if (dtype == MSA_BF16)
     return launch_attn_bf16(q, cu_q, k, v, kv_off, kv_len, B, total_q, max_kv, Hq, Hkv, scale, causal, plan, out, part_ml,
                             part_acc, st);
-  return launch_attn<float>(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml,
-                            part_acc, st);
+  return launch_attn<float>(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, scale, causal, plan, out, part_ml, part_acc, st,
+                            spread_heads((int64_t)total_q * Hq * n_split, Hq / Hkv, n_split, max_kv));
 }
 
 extern "C" int msa_decode_attn_fused(const void* qkv, int64_t row_stride, const int64_t* positions, const void* q_norm_w,
