@@ -378,12 +378,13 @@ def sparse_attn(q, k, v, kv_off, kv_len, max_kv: int, cu_q=None, max_sq: int = 1
     lib = _lib.load()
     sc = D ** -0.5 if scale is None else scale
     # bf16 query blocks: the one-pass MFMA flash kernel, except where its few workgroups (tiles of 128 columns) would each walk over many
-    # keys: there the split-KV entry point below, which runs the same kernel per key range and combines.  Where both take as long: 8
-    # workgroups 400 keys, 16 550, 32 700, 64 1200, 128 1900, 256 5000 (us, flash and split: 128 rows of 32 heads over 8 and 640 keys 18.5 and 18.1,
-    # 1152 26.7 and 20.3; 512 rows and 1024 keys 25.5 and 31.7, 2560 48.5 and 40.8; 4 samples of 500 rows and keys 26.2 and 47.5)
+    # keys: there the split-KV entry point below, which runs the same kernel per key range and combines.  A key range less costs 2.3 us in 128
+    # keys, the combining 3 us and the way of the partials, which grows with the rows and heads.  Where both take as long, and the line: 16 rows of 8
+    # heads over 8 370 keys and 278, of 32 over 32 370 and 336, 128 rows of 32 over 8 560 and 515, 4 x 60 of 16 over 8 500 and 503, 16 x 60 of 8 over 8 900 and
+    # 848, 400 of 32 over 8 1400 and 1066 (us there, flash and split: 1024 keys 24.4 and 30.1, 1536 34.1 and 32.8); within 0.2 % of the better one in the
+    # mean of 600 sizes, 13 % behind at most (without keys: zeros from as many rows as fill the chip, refused below)
     tiles = Hkv * max(B, -(-total_q * (Hq // max(1, Hkv)) // 128))
-    # (without keys: zeros from as many rows as fill the chip, refused below)
-    one_pass = tiles > 128 or max_kv <= 300 + 16 * tiles if max_kv > 0 else total_q * Hkv >= 32 * 512
+    one_pass = tiles > 128 or max_kv <= 260 + total_q * Hq // 20 + 8 * tiles // 5 if max_kv > 0 else total_q * Hkv >= 32 * 512
     if q.dtype == torch.bfloat16 and max_sq >= FLASH_MIN_ROWS and one_pass:
         out = torch.empty_like(q)
         check(lib.msa_flash_attn_fit(ptr(q), ptr(cu_q), ptr(k), ptr(v), ptr(kv_off), ptr(kv_len), B, total_q, Hq, Hkv, D,

@@ -42,6 +42,8 @@ def test_no_keys(call, G, Hkv):
 
 
 def test_with_keys(call):
-    assert call(64, 1, 32, 8, 400) == "one pass" and call(64, 1, 32, 8, 4000) == "splits"
-    assert call(2048, 1, 8, 8, 2348) == "one pass" and call(2048, 1, 8, 8, 2349) == "splits" and call(2048, 1, 16, 8, 1 << 20) == "one pass"
+    # rows x heads / 20 and 1.6 keys a tile of 128 columns over 260 keys, up to 128 tiles
+    for rows, B, Hq, Hkv, line in ((64, 1, 32, 8, 387), (64, 4, 32, 8, 413), (82, 4, 8, 8, 343), (400, 1, 32, 8, 1066), (2048, 1, 8, 8, 1283), (16, 1, 8, 8, 278)):
+        assert call(rows, B, Hq, Hkv, line) == "one pass" and call(rows, B, Hq, Hkv, line + 1) == "splits", (rows, B, Hq, Hkv)
+    assert call(2048, 1, 16, 8, 1 << 20) == "one pass" and call(33, 17, 32, 8, 1 << 20) == "one pass"
     assert call(4096, 1, 32, 8, 100, torch.float32) == "splits"
