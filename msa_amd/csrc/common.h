@@ -112,6 +112,14 @@ __device__ __forceinline__ float row16_sum(float v) {   // all-reduce over the 1
   v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x121, 0xf, 0xf, false));
   return v;
 }
+// The sum over the lanes 16, 32 and 48 away, in the order (own + 16) + (32 + 48).
+__device__ __forceinline__ float lanes_sum(float v) {
+  uint32_t u = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  u = __float_as_uint(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+  const auto t = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+}
 __device__ __forceinline__ float row16_ror8(float v) {  // value of the lane 8 places away in the row
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false));
 }

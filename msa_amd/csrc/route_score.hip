@@ -1328,8 +1328,8 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void score_split_kernel(const 
 // the operands' way from the L2 with many, 196 KB a block, which takes twice the 1.4 us that the products do (half of it would want
 // 64 chunks a workgroup, whose parts the registers do not hold).  An infinity among the values makes NaN where parts of different
 // sign meet, so a sum that is NaN is formed again value by value, by a whole wavefront: once a NaN chunk or query row, which end there, once a
-// row for a chunk with an infinity.  Calls of 8000 chunks x 64 rows, one chunk with a NaN, with an infinity, all queries NaN: 28, 41 and 50 us, 26 without
-// (a lane for each sum, value after value: 187, 199 and 328).
+// row for a chunk with an infinity.  Calls of 8000 chunks x 64 rows, one chunk with a NaN, with an infinity, all queries NaN: 28, 40 and 49 us, 26 without
+// (a lane for each sum, value after value: 206, 212 and 328).
 // ------------------------------------------------------------------------------------------
 constexpr int kPartsWaves = 8, kPartsSlabs = 4, kPartsMaxRows = 1024;
 constexpr int kPartsLds = kPartsWaves * kPartsSlabs * kSplitSlab + kSplitMaxBlocks * kSplitCols * 4;
@@ -1357,12 +1357,6 @@ struct ValuesDot {
         sum += x * y;
       }
     }
-  }
-  __device__ __forceinline__ float wave_sum() const {
-    float v = sum;
-#pragma unroll
-    for (int x = 32; x > 0; x >>= 1) v += __shfl_xor(v, x);
-    return v;
   }
 };
 
@@ -1484,7 +1478,7 @@ __global__ __launch_bounds__(kPartsWaves * 64) void score_parts_kernel(const cha
       for (uint64_t again = __ballot(v != v && n0 + l32 < C && (nan_columns >> l32 & 1) == 0); again != 0;) {
         const int at = __builtin_ctzll(again);             // the lane whose sum is formed
         const ValuesDot dot(qs + part_at(32 * blk + wave * 4 + (at >> 5) * 2 + r, lane * 16, kSplitK), kr + (int64_t)(n0 + (at & 31)) * kSplitK + lane * 16);
-        const float sum = dot.wave_sum();
+        const float sum = lanes_sum(row16_sum(dot.sum));
         v = lane == at ? sum : v;
         again &= again - 1;
         if (__any(dot.query_nan)) again &= at < 32 ? ~0ull << 32 : 0ull;           // none of the row's sums is a number

@@ -71,15 +71,6 @@ __device__ __forceinline__ float quad_xor(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kPerm, 0xf, 0xf, false));
 }
 
-// The sum over the lanes 16, 32 and 48 away, in the order (own + 16) + (32 + 48).
-__device__ __forceinline__ float lanes_sum(float v) {
-  uint32_t u = __float_as_uint(v);
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  u = __float_as_uint(__uint_as_float(r[0]) + __uint_as_float(r[1]));
-  const auto t = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __uint_as_float(t[0]) + __uint_as_float(t[1]);
-}
-
 __device__ __forceinline__ uint32_t lds_offset(const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
 __device__ __forceinline__ u32x4_t lds_read16(uint32_t at) {
   u32x4_t v;

@@ -195,13 +195,7 @@ __device__ __forceinline__ float add_moved(float v) {
 }
 // The sum over sixteen lanes, and over a wavefront, in every lane.
 __device__ __forceinline__ float row_sum(float v) { return add_moved<0x140>(add_moved<0x141>(add_moved<0x4E>(add_moved<0xB1>(v)))); }
-__device__ __forceinline__ float wave_sum(float v) {
-  uint32_t u = __float_as_uint(row_sum(v));
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  u = __float_as_uint(__uint_as_float(r[0]) + __uint_as_float(r[1]));
-  const auto t = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __uint_as_float(t[0]) + __uint_as_float(t[1]);
-}
+__device__ __forceinline__ float wave_sum(float v) { return lanes_sum(row_sum(v)); }
 // One 16-byte chunk's products of a weight row and its operand.
 __device__ __forceinline__ float dot8(const u32x4_t& w, const u32x4_t& x, float s) {
 #pragma unroll
