@@ -311,9 +311,9 @@ int msa_flash_attn_fit(const void* q, const int32_t* cu_q, const void* k, const 
                        const int64_t* kv_off, const int32_t* kv_len, int32_t B, int32_t total_q,
                        int32_t Hq, int32_t Hkv, int32_t D, float scale, int32_t causal, void* out,
                        int32_t max_sq, void* stream);
-/* The form that msa_flash_attn_fit and msa_flash_attn_rows take: 0 32 columns a workgroup, 1 256 columns, blocks dealt by length, 2 256 columns in turn.
- * No device is asked. */
-int msa_diag_flash_form(int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv, int32_t compute_units);
+/* The form that msa_flash_attn_fit and msa_flash_attn_rows take, or with `promised` msa_flash_attn_hint and (max_sq 0) msa_flash_attn: 0 32 columns a
+ * wavefront, 1 256 columns a workgroup, blocks dealt by length, 2 256 columns in turn.  No device is asked. */
+int msa_diag_flash_form(int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv, int32_t compute_units, int32_t promised);
 /* Causal attention of rows as a decoder of mixed layers has them: query rows q_stride elements apart, sample b's keys end with its own rows
  * behind kv_pos[b] earlier ones.  sink [Hq] (or NULL): a member of every softmax of head h without a value; gate [rows, Hq] bf16, rows
  * gate_stride apart (or NULL): outputs times its sigmoid.  out [rows, Hq, D] dense. */

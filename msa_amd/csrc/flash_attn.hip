@@ -931,6 +931,11 @@ namespace {
 // and take 152 dealt by length, 1780 and then 2200 of 32 over 8 114 and 82, two of 3950 of 16 over 4 209
 // and 143 (32-column form 147).
 enum Form { kColumns32, kWide, kWideInTurn };
+Form order_of(int32_t B, int32_t total_q, int32_t max_sq, int G, int64_t turn) {
+  const int64_t each = ((int64_t)max_sq * G + 255) / 256;
+  if (B == 1 || (int64_t)total_q * G < 1024LL * B) return kWideInTurn;           // (short samples: the lookups are what counts)
+  return (int64_t)max_sq * B == total_q && (turn % each == 0 || each % turn == 0) ? kWideInTurn : kWide;
+}
 Form form_for(int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv, int units) {
   const int G = Hkv > 0 ? Hq / Hkv : 0;
   if (G <= 0 || G > 8 || B <= 0 || (int64_t)total_q * G < 4096) return kColumns32;
@@ -944,14 +949,18 @@ Form form_for(int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hk
   } else if ((int64_t)max_sq * B <= (int64_t)total_q + total_q / 4 && mean * G >= 16 * 256.f) {
     blocks = (int64_t)total_q * G / 256 + B / 2;
   }
-  if (blocks > 0 && (blocks + turn / 8) % (2 * turn) <= turn / 8)
-    return equal && (B == 1 || turn % each == 0 || each % turn == 0) ? kWideInTurn : kWide;
+  if (blocks > 0 && (blocks + turn / 8) % (2 * turn) <= turn / 8) return order_of(B, total_q, max_sq, G, turn);
   if (G >= 4 && mean >= 2000.f && rounds >= (mean >= 3000.f ? 3.25f : 7.f)) return kWide;
   if (mean >= 12000.f && rounds >= 3.f) return kWide;
   return kColumns32;
 }
-// What msa_flash_attn and msa_flash_attn_hint promise: the wide form from 4096 columns on, unless the batch is known to be ragged.
-bool wide_enough(int32_t total_q, int32_t Hq, int32_t Hkv) { return Hkv > 0 && (int64_t)total_q * (Hq / Hkv) >= 4096; }
+// What msa_flash_attn (max_sq 0) and msa_flash_attn_hint promise: the wide form from 4096 columns on, unless the batch is known to be ragged.  us, 32 heads
+// over 8, dealt by length and in turn: 200 samples of 64 131 and 111, 1000 of 16 494 and 460, 4 of 1024 50 and 48; three of 3000 241 and 257.
+Form promised_form(int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv, int units) {
+  const int G = Hkv > 0 ? Hq / Hkv : 0;
+  if ((int64_t)total_q * G < 4096 || B <= 0 || (max_sq > 0 && (int64_t)max_sq * B > (int64_t)total_q + total_q / 4)) return kColumns32;
+  return order_of(B, total_q, max_sq, G, std::max(1, units / Hkv));
+}
 RowOptions dense_rows(int32_t Hq, int32_t D) { return {(int64_t)Hq * D, nullptr, nullptr, 0, nullptr}; }
 
 int flash_attn_entry(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
@@ -979,7 +988,7 @@ int flash_attn_entry(const void* q, const int32_t* cu_q, const void* k, const vo
 extern "C" int msa_flash_attn(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
                               const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D,
                               float scale, int32_t causal, void* out, void* stream) {
-  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, wide_enough(total_q, Hq, Hkv) ? kWide : kColumns32,
+  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, promised_form(B, total_q, 0, Hq, Hkv, device_compute_units()),
                           dense_rows(Hq, D), stream);
 }
 
@@ -987,9 +996,8 @@ extern "C" int msa_flash_attn_hint(const void* q, const int32_t* cu_q, const voi
                                    const int32_t* kv_len, int32_t B, int32_t total_q, int32_t Hq, int32_t Hkv, int32_t D,
                                    float scale, int32_t causal, void* out, int32_t max_sq, void* stream) {
   MSA_REQUIRE(max_sq > 0, "msa_flash_attn_hint: max_sq must be the longest query block of the batch");
-  const bool ragged = (int64_t)max_sq * B > (int64_t)total_q + total_q / 4;
-  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out, wide_enough(total_q, Hq, Hkv) && !ragged ? kWide : kColumns32,
-                          dense_rows(Hq, D), stream);
+  return flash_attn_entry(q, cu_q, k, v, kv_off, kv_len, B, total_q, Hq, Hkv, D, scale, causal, out,
+                          promised_form(B, total_q, max_sq, Hq, Hkv, device_compute_units()), dense_rows(Hq, D), stream);
 }
 
 extern "C" int msa_flash_attn_fit(const void* q, const int32_t* cu_q, const void* k, const void* v, const int64_t* kv_off,
@@ -1000,8 +1008,8 @@ extern "C" int msa_flash_attn_fit(const void* q, const int32_t* cu_q, const void
                           dense_rows(Hq, D), stream);
 }
 
-extern "C" int msa_diag_flash_form(int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv, int32_t compute_units) {
-  return form_for(B, total_q, max_sq, Hq, Hkv, compute_units);
+extern "C" int msa_diag_flash_form(int32_t B, int32_t total_q, int32_t max_sq, int32_t Hq, int32_t Hkv, int32_t compute_units, int32_t promised) {
+  return promised ? promised_form(B, total_q, max_sq, Hq, Hkv, compute_units) : form_for(B, total_q, max_sq, Hq, Hkv, compute_units);
 }
 
 // us before this rule (the wide form for samples of one length in whole pairs of rounds) and with it: 16 heads 4096 rows 95 and 88, 3000 73 and 69,

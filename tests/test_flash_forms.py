@@ -21,7 +21,7 @@ def longest_share(lens, G, n):
 def test_in_turn_is_even(Hq, Hkv):
     from msa_amd import _lib
     lib, r, n = _lib.load(), random.Random(Hq + Hkv), 256 // Hkv
-    form = lambda lens: lib.msa_diag_flash_form(len(lens), sum(lens), max(lens), Hq, Hkv, 256)
+    form = lambda lens: lib.msa_diag_flash_form(len(lens), sum(lens), max(lens), Hq, Hkv, 256, 0)
     taken = 0
     for _ in range(6000):
         B = r.randint(1, 12)
@@ -38,4 +38,13 @@ def test_in_turn_is_even(Hq, Hkv):
                                               ([4000, 2500, 3000, 3500] * 4, 32, 8, DEALT), ([1000], 32, 8, COLUMNS32), ([3500, 2160], 32, 8, COLUMNS32)])
 def test_forms(lens, Hq, Hkv, form):
     from msa_amd import _lib
-    assert _lib.load().msa_diag_flash_form(len(lens), sum(lens), max(lens), Hq, Hkv, 256) == form
+    assert _lib.load().msa_diag_flash_form(len(lens), sum(lens), max(lens), Hq, Hkv, 256, 0) == form
+
+
+@pytest.mark.parametrize("lens,Hq,Hkv,hint,plain", [([4096], 32, 8, IN_TURN, IN_TURN), ([64] * 200, 32, 8, IN_TURN, IN_TURN), ([16] * 1000, 32, 8, IN_TURN, IN_TURN),
+                                                    ([1024] * 4, 32, 8, IN_TURN, DEALT), ([3000] * 3, 32, 8, DEALT, DEALT), ([3950] * 2, 16, 4, DEALT, DEALT),
+                                                    ([3000, 5000], 16, 4, DEALT, DEALT), ([3000, 1000], 32, 8, COLUMNS32, DEALT), ([1000], 32, 8, COLUMNS32, COLUMNS32)])
+def test_promised_forms(lens, Hq, Hkv, hint, plain):
+    from msa_amd import _lib
+    form = lambda top: _lib.load().msa_diag_flash_form(len(lens), sum(lens), top, Hq, Hkv, 256, 1)
+    assert form(max(lens)) == hint and form(0) == plain
