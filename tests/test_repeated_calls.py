@@ -77,16 +77,29 @@ def test_delta_steps_on_the_same_buffers(gpu, B, H, G, D, E, R):
         assert ((state - state2).norm() / state2.norm()).item() < 1e-5
 
 
-@pytest.mark.gpu
-def test_eager_steps_hold_no_memory(gpu, monkeypatch):
-    """Eager decode steps leave the allocator where it was, and a model and its cache that are dropped are given back."""
-    from msa_amd import seq_ops
+def _postnorm():
     from msa_amd.config import PostNormConfig
     from msa_amd.postnorm import PostNormForCausalLM
     from postnorm_models import ATTN, config, layer, random_weights, tensor_shapes
     cfg = config([layer("channel_delta", {"heads": 4, "kv_heads": 2, "dim": 64, "vdim": 128, "conv": 4}), layer("attention", ATTN)], width=256)
+    return lambda: PostNormForCausalLM.from_tensors(PostNormConfig.from_dict(cfg), random_weights(tensor_shapes(cfg, (64, 64))), torch.bfloat16, "cuda:0")
+
+
+def _hybrid():
+    from hybrid_models import CONFIGS
+    from msa_amd.config import HybridConfig
+    from msa_amd.hybrid import HybridForCausalLM
+    return lambda: HybridForCausalLM.random(HybridConfig.from_dict(CONFIGS["mixed"]), 0, torch.bfloat16, "cuda:0")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("make", [_postnorm, _hybrid])
+def test_eager_steps_hold_no_memory(gpu, monkeypatch, make):
+    """Eager decode steps leave the allocator where it was, and a model and its cache that are dropped are given back."""
+    from msa_amd import seq_ops
     taken, inner = [], seq_ops.delta_step
     monkeypatch.setattr(seq_ops, "delta_step", lambda *a: (taken.append(1), inner(*a))[1])
+    model = make()
 
     def held():
         gc.collect()
@@ -94,7 +107,7 @@ def test_eager_steps_hold_no_memory(gpu, monkeypatch):
         return torch.cuda.memory_allocated()
 
     def life():
-        m = PostNormForCausalLM.from_tensors(PostNormConfig.from_dict(cfg), random_weights(tensor_shapes(cfg, (64, 64))), torch.bfloat16, "cuda:0")
+        m = model()
         cache = m.create_cache(2, 64)
         sizes = []
         for i in range(12):
@@ -105,4 +118,4 @@ def test_eager_steps_hold_no_memory(gpu, monkeypatch):
     print("[repeated] second model", flush=True)
     before = held()
     life()
-    assert len(taken) == 24 and held() == before
+    assert len(taken) == (24 if make is _postnorm else 0) and held() == before
