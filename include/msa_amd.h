@@ -188,6 +188,11 @@ int msa_diag_read_stream(const void* src, int64_t bytes, void* dst, int32_t mode
 int msa_diag_scan_walk(int32_t tiles_m, int32_t tiles_n, int32_t grid, int32_t has_copy_workgroup, int32_t pool_n,
                        int32_t* visits);
 
+/* Test aid (no counterpart in the reference; runs on the host): how the rows of B bf16 queries of S tokens lie in the scan of
+ * C chunks by msa_route_topk: a query has a multiple of *unit rows (32, or 8 or 4 where queries share row blocks); *by_units: the large-tile
+ * scan takes them in units.  gathers: the scan is to carry a gather. */
+int msa_diag_row_packing(int32_t B, int32_t S, int64_t C, int32_t gathers, int32_t* unit, int32_t* by_units);
+
 /* Registers and bytes of scratch per lane of the loaded code object's asm-scheduled kernels (which = 0: the routing
  * scan score_scan4_kernel, 1: flash_wide_kernel).  Their statements keep state in physical registers across statements,
  * which only holds while the compiler spilled nothing: the library refuses to launch either with scratch (MSA_ESTATE),

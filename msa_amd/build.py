@@ -55,7 +55,8 @@ def _compile(src: str) -> str:
 #  * score_scan4_kernel (route_score.hip): its asm statements own v128-v255 and all accumulation registers across
 #    statements.  The code the compiler generates for that kernel must therefore stay below v128, touch no
 #    accumulation register (the compiler would only do so to spill), and use no scratch memory.
-#  * tile_gemm_kernel (gemm.hip): the same registers; tile_flow_kernel: v24-v255 and all accumulation registers.
+#    score_scan4_units_kernel: likewise below v96.
+#  * tile_gemm_kernel (gemm.hip): the registers of score_scan4_kernel; tile_flow_kernel: v24-v255 and all accumulation registers.
 #  * flash_wide_kernel (flash_attn.hip): likewise, its statements own v56-v255 and all accumulation registers.
 #  * flash_attn_kernel (flash_attn.hip): its direct-to-LDS loads are asm statements the compiler does not order
 #    against LDS reads; a spill would add vector-memory waits in the middle of that ring.  No scratch, no spills.
@@ -66,7 +67,8 @@ def _compile(src: str) -> str:
 #    the vector offset alone.  No scalar offsets.
 # ---------------------------------------------------------------------------------------------------------------
 CONTRACTS = {
-    "route_score.hip": [("score_scan4_kernel", {"max_compiler_vgpr": 127, "no_agpr": True}), ("score_parts_kernel", {})],
+    "route_score.hip": [("score_scan4_kernel", {"max_compiler_vgpr": 127, "no_agpr": True}),
+                        ("score_scan4_units_kernel", {"max_compiler_vgpr": 95, "no_agpr": True}), ("score_parts_kernel", {})],
     "gemm.hip": [("tile_gemm_kernel", {"max_compiler_vgpr": 127, "no_agpr": True}), ("tile_flow_kernel", {"max_compiler_vgpr": 23, "no_agpr": True})],
     "flash_attn.hip": [("flash_attn_kernel", {}), ("flash_wide_kernel", {"max_compiler_vgpr": 55, "no_agpr": True})],
     "linear.hip": [("rows_ring_kernel", {})],

@@ -22,12 +22,13 @@ passes an accumulator twice as often for the same products, and these loops run 
 LDS: two stages of the query tile at 0 / 0x8000, three of the K_r tile at 0x10000 / 0x18000 / 0x20000, rows of 128
 bytes whose 16-byte units are XOR-swizzled by (row >> 1) & 7.
 
-Registers the statements own (the kernel's compiler-allocated code stays below v128 and uses no accumulation
-registers): v128-v159 fragments A0-A7, v160-v191 B0-B7, v192-v197 LDS addresses of the step, v198-v201 per-lane LDS offsets of the
+Registers the statements own (the kernel's compiler-allocated code stays below v128, below v96 where queries lie in units, and uses
+no accumulation registers): v128-v159 fragments A0-A7, v160-v191 B0-B7, v192-v197 LDS addresses of the step, v198-v201 per-lane LDS offsets of the
 two sub-steps (A, then B), v208-v215 global offsets of the wavefront's eight 1 KB blocks, v216-v223 tile pool and prefetch values
 (see the kernel), v224-v231 the maxima of the tile just finished (row block of 32 rows i and column group of 64 columns p in
 v224 + 2 i + p, lane l column 64 p + l; in the folding form the maxima over all rows, column group p in v224 + p), v232-v239 their
-parts before the lanes are joined, v240-v247 scratch of the reduction and the fold, v248-v252 per-lane constants of the fold,
+parts before the lanes are joined, v96-v127 those of units of eight rows (unit u of row block i in v96 + 8 i + 4 p + u, lane l column
+64 p + l), v240-v247 scratch of the reduction and the fold, v248-v252 per-lane constants of the fold,
 s76-s95 scratch.
 
 The reduction of a finished tile (per lane the maximum of each block's four values, then of the blocks below it, then over the four
@@ -36,7 +37,9 @@ the next tile's first K step, a block in front of the MFMA that overwrites it: w
 under it.  When the wavefront's rows belong to one query and all count and the tile lies inside the bank, the fold of the
 column maxima over the chunks of a document (order-preserving key, segmented max-scan over the 64
 lanes by row moves, one atomic per document run) follows in the same statement, dealt out behind the MFMAs of
-the second sub-step; its atomics are issued behind the step's wait so that the wait does not count them.
+the second sub-step; its atomics are issued behind the step's wait so that the wait does not count them.  Short queries lie in units
+of eight rows, four units a row block, unit u in rows 4 u .. 4 u + 3 of either sixteen: a lane has a unit's maximum of its column
+without an exchange, and the joining becomes a transposition of (column block, unit), the same swaps without the maxima.
 
 In the products the A operand is the weights and the B operand the tokens; each has row offsets of its own (v208-v215 the eight blocks
 of the A tile, v216-v223 those of the B tile), neither is read non-temporal, and a finished tile's accumulators are read behind its
@@ -55,6 +58,7 @@ VOFF = 208
 VOFF_B = 216         # of the products' B operand
 VMAX = 224
 VPART = 232
+VUNIT = 96
 VRED = 240           # 8 scratch registers; the fold's temporaries: pair p in v(240 + 4 p) .. v(243 + 4 p)
 V_LOWMASK, V_DISTBASE, V_L32P1, V_IS31, V_L15 = 248, 249, 250, 251, 252
 VDOC = 220           # documents of the wavefront's columns: group p in v(220 + p)
@@ -107,10 +111,12 @@ def order(sub, q, tile=SCAN):
 class Reduction:
     """The maxima of a finished tile, a block at a time in the order of the first sub-step's quadrants."""
 
-    def __init__(self, joined):
-        self.joined, self.seen, self.flip = joined, set(), 0
+    def __init__(self, joined, units=False):
+        self.joined, self.units, self.seen, self.flip = joined, units, set(), 0
 
     def part(self, i, j):
+        if self.units:
+            return VUNIT + 4 * ((i >> 1) * 2 + (j >> 2)) + (j & 3)
         # joined: one row of parts per column group, over all rows; otherwise one per row block of 32 inside the quadrant
         return VPART + (4 * (j >> 2) if self.joined else 4 * ((i >> 1) & 1)) + (j & 3)
 
@@ -129,6 +135,11 @@ class Reduction:
     def after(self, q):
         """What a quadrant's parts allow: the lanes of a column group joined, lane l column l of the group."""
         ha, hb = QUADS[0][q]
+        if self.units:
+            firsts = [VUNIT + 4 * ((2 * ha + r) * 2 + hb) for r in range(2)]
+            return [f"{op} v{first + x}, v{first + y}" for op, x, y in (("v_permlane32_swap_b32", 0, 2), ("v_permlane32_swap_b32", 1, 3),
+                                                                        ("v_permlane16_swap_b32", 0, 1), ("v_permlane16_swap_b32", 2, 3))
+                    for first in firsts]
         if self.joined:
             groups = [(VPART + 4 * hb, VMAX + hb)] if q >= 2 else []
         else:
@@ -236,13 +247,13 @@ def kstep(fresh, reduce=None, tile=SCAN, voff_b=VOFF, nt=" nt", woff=("woff", "w
     """One K step.  Operands: [sa] / [sb] LDS stage of the step's A / B tile (advanced to the next step's),
     [ra] / [rb] resources the loads of this step read, [k] their byte offset inside a row, [woff] the wavefront's part of a stage.
     fresh: a tile's first step (the first sub-step multiplies into zero); reduce: it also reduces the accumulators the
-    previous tile left, "blocks" to one maximum per row block, "fold" on to the key plane ([okey]: the query's keys).
+    previous tile left, "blocks" to one maximum per row block, "units" per eight rows, "fold" on to the key plane ([okey]: the query's keys).
     fillers go behind the MFMAs, stores (of the tile before) behind the step's wait so that it does not count them;
     early_fillers: a list per block in front of the MFMA that overwrites it."""
     out = []
     e = out.append
     fillers, atomics, stores = list(fillers), [], list(stores)
-    red = Reduction(reduce == "fold") if reduce else None
+    red = Reduction(reduce == "fold", reduce == "units") if reduce else None
     if reduce == "fold":
         (a0, at0), (a1, at1) = fold_pair(0), fold_pair(1)
         fillers = interleave(a0, a1)
@@ -336,10 +347,10 @@ def kstep(fresh, reduce=None, tile=SCAN, voff_b=VOFF, nt=" nt", woff=("woff", "w
     return fix_lane_move_hazards(out)
 
 
-def reduction():
+def reduction(units=False):
     """The reduction by itself, behind a workgroup's last tile (an MFMA's result may be read 18 wait states after its
     issue at the earliest)."""
-    red, out = Reduction(False), ["s_nop 15", "s_nop 7"]
+    red, out = Reduction(False, units), ["s_nop 15", "s_nop 7"]
     for q in range(4):
         for i, j in order(0, q):
             out += red.block(i, j)
@@ -390,7 +401,10 @@ def scan_text():
         define("MSA_SCAN4_KSTEP_FRESH", kstep(True)),
         define("MSA_SCAN4_KSTEP_FRESH_REDUCE", kstep(True, "blocks")),
         define("MSA_SCAN4_KSTEP_FRESH_FOLD", kstep(True, "fold")),
+        define("MSA_SCAN4_KSTEP_FRESH_UNITS", kstep(True, "units")),
         define("MSA_SCAN4_REDUCE", reduction()),
+        define("MSA_SCAN4_REDUCE_UNITS", reduction(True)),
+        *(define(f"MSA_SCAN4_UNIT_READ_{i}", [f"v_mov_b32 %{x}, v{VUNIT + 8 * i + x}" for x in range(8)]) for i in range(4)),
         define("MSA_SCAN4_MAX_READ", [f"v_mov_b32 %{x}, v{VMAX + x}" for x in range(8)]),
         define("MSA_SCAN4_FRAGS0", frags0()),
         define("MSA_SCAN4_LOAD8", load8(VOFF)),
@@ -402,7 +416,8 @@ def scan_text():
             f"v_lshlrev_b32 v{V_LOWMASK}, %0, 2", f"v_add_u32 v{V_LOWMASK}, -1, v{V_LOWMASK}",      # (2 << l32) - 1
             f"v_add_u32 v{V_DISTBASE}, -31, %0", f"v_add_u32 v{V_L32P1}, 1, %0",
             f"v_cmp_eq_u32 vcc, 31, %0", f"v_cndmask_b32 v{V_IS31}, 0, 1, vcc", f"v_and_b32 v{V_L15}, 15, %0"]),
-        clobbers("MSA_SCAN4_CLOBBERS")])
+        clobbers("MSA_SCAN4_CLOBBERS"),
+        clobbers("MSA_SCAN4_UNITS_CLOBBERS", VUNIT)])
 
 
 # ---------------------------------------------------------------------------------------------------------------

@@ -21,8 +21,8 @@ struct GatherJob {
 };
 
 struct RouteWorkspace {
-  int32_t S_pad;        // query tokens padded to a multiple of 32 (one MFMA row block never spans two queries)
-  int32_t M_rows;       // B * S_pad
+  int32_t S_pad;        // query tokens padded to a multiple of 32 (one MFMA row block never spans two queries), or of a smaller unit
+  int32_t M_rows;       // B * S_pad, to a multiple of 32
   int32_t topk_blocks;  // candidate lists per query
   int32_t mask_words;   // words of the scored-row bitmask, padded to whole M tiles
   size_t off_qs;        // pre-summed queries [M_rows, Hkv * D] (with `parts` six bytes a value: three bf16 parts of fp32)
@@ -39,7 +39,7 @@ static inline int32_t topk_blocks_for(int64_t n_docs) {
 }
 
 RouteWorkspace route_workspace_layout(int32_t B, int32_t S, int32_t Hkv, int32_t D, int64_t plane_cols, int64_t n_docs,
-                                      int32_t dtype, bool parts = false);
+                                      int32_t dtype, bool parts = false, int32_t unit = 32);
 
 // query_reduce: MSA_QUERY_*; extra_plane_cols: words per query reserved behind the key plane (the per-document keys
 // of the chunk-mean reduction).

@@ -31,6 +31,8 @@ typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 // skipped and its keys stay 0.  The workgroup of every 32nd row writes the mask word of its 32 rows (all ones or
 // zero), workgroup 0 the zero words that pad the mask to whole M tiles, and all workgroups together clear the
 // `clear_words` key words the scoring kernel merges into with atomicMax.
+// Short queries of a batch share row blocks (RowPacking): then the word of a row block tells every row's own query, rows behind the last
+// query are zero, and the scan's large tiles have a block's rows in the order of its units (unit_row).
 // ------------------------------------------------------------------------------------------
 // Words behind the persistent scan's tile pool: the pool's counter, on a cache line of its own, then one word per
 // workgroup through which the wavefront that drew a tile tells the workgroup's others.
@@ -65,21 +67,39 @@ __device__ __forceinline__ int64_t part_at(int row, int k, int K) {
   return ((int64_t)(row >> 5) * (K / 16) + k / 16) * kPartStep + (row & 31) * 16 + (k & 8) * 64;
 }
 
+// Where the large-tile scan has row `row` of a block of four units of eight rows: unit u in rows 4 u .. 4 u + 3 of either sixteen.
+__device__ __forceinline__ int unit_row(int row) { return (row & ~31) | (row & 4) << 2 | (row & 24) >> 1 | (row & 3); }
+
 template <typename TIn, typename TOut, bool kParts = false>
 __global__ void presum_queries_kernel(const TIn* __restrict__ q, const uint8_t* __restrict__ qmask, int32_t B,
                                       int32_t S, int32_t S_pad, int32_t Hq, int32_t Hkv, int32_t normalize,
                                       TOut* __restrict__ qs, uint32_t* __restrict__ row_bits, int32_t mask_words,
-                                      uint32_t* __restrict__ key_plane, int64_t clear_words, uint32_t* __restrict__ sched) {
+                                      uint32_t* __restrict__ key_plane, int64_t clear_words, uint32_t* __restrict__ sched,
+                                      int32_t packed, int32_t by_units) {
   const int row = blockIdx.x;              // b * S_pad + s
   const int b = row / S_pad;
   int s = row % S_pad;
   const int G = Hq / Hkv;
   const int g = threadIdx.x >> 4, j = threadIdx.x & 15;
-  bool valid = s < S && (qmask == nullptr || qmask[(int64_t)b * S + s] != 0);
+  const bool behind = b >= B;              // (packed: the last block's rows behind the last query)
+  bool valid = !behind && s < S && (qmask == nullptr || qmask[(int64_t)b * S + s] != 0);
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < clear_words; i += (int64_t)gridDim.x * blockDim.x)
     key_plane[i] = 0u;
-  const bool writes_word = (row & 31) == 0;           // rows are padded per query to a multiple of 32
-  if (!valid || writes_word) {                        // (uniform over the workgroup)
+  const bool writes_word = (row & 31) == 0;           // rows are padded per query to a multiple of 32, or packed
+  if (packed && writes_word) {
+    __shared__ uint32_t scored_rows;
+    if (threadIdx.x == 0) scored_rows = 0u;
+    __syncthreads();
+    const int tokens = (min((row + 31) / S_pad, B - 1) - b + 1) * S;      // of the block's queries, which lie side by side
+    for (int i = (int)threadIdx.x; i < tokens; i += blockDim.x)
+      if (qmask == nullptr || qmask[(int64_t)b * S + i] != 0) {
+        const int first = (b + i / S) * S_pad - row, lo = max(first, 0), hi = min(first + S_pad, 32);
+        atomicOr(&scored_rows, (hi < 32 ? (1u << hi) - 1u : 0xffffffffu) & (0xffffffffu << lo));
+      }
+    __syncthreads();
+    if (threadIdx.x == 0) row_bits[row >> 5] = scored_rows;
+  }
+  if (!behind && (!valid || (writes_word && !packed))) {      // (uniform over the workgroup)
     // the query's first scored token, found by the workgroup's first wavefront
     __shared__ int first_scored;
     if (threadIdx.x < 64) {
@@ -93,7 +113,7 @@ __global__ void presum_queries_kernel(const TIn* __restrict__ q, const uint8_t* 
       }
       if (threadIdx.x == 0) {
         first_scored = found;
-        if (writes_word) row_bits[row >> 5] = found >= 0 ? 0xffffffffu : 0u;
+        if (writes_word && !packed) row_bits[row >> 5] = found >= 0 ? 0xffffffffu : 0u;
       }
     }
     __syncthreads();
@@ -151,7 +171,7 @@ __global__ void presum_queries_kernel(const TIn* __restrict__ q, const uint8_t* 
     for (int p = 0; p < 3; ++p) *reinterpret_cast<uint4*>(to + p * kPartBytes) = part[p];
     return;
   }
-  TOut* o = qs + ((int64_t)row * Hkv + g) * kHeadDim + 8 * j;
+  TOut* o = qs + ((int64_t)(by_units ? unit_row(row) : row) * Hkv + g) * kHeadDim + 8 * j;
   if constexpr (sizeof(TOut) == 2) {
     uint4 w;
     w.x = pack_bf16x2(acc[0], acc[1]); w.y = pack_bf16x2(acc[2], acc[3]);
@@ -310,6 +330,44 @@ struct Mma<float> {
 // 96 KB per compute unit in flight (returns are in order, so the query tile has to run as far ahead as the K_r tile for
 // the K_r tile's lead to count).
 constexpr int kDtlStreamLdsBytes = 3 * (128 + 256) * 128;
+
+// Chunks of a document are adjacent columns: a segmented max-scan over the 32 lanes of each half of a wavefront leaves a document's maximum
+// in the last lane of its run, which alone touches memory (about two atomics per 32 chunks instead of 32 stores, and no per-chunk plane
+// to read back).  What a lane may take in a step of the scan depends on the documents alone, so it is found once for all queries that are
+// folded over them: four shifts inside the rows of 16 lanes, then lane 15 of the lower row joins the runs that cross into the upper one.
+// Lanes that a shift cannot reach read 0, the identity of max over keys.
+struct DocRuns {
+  int doc;
+  uint32_t take[5];      // all ones where the lane's run reaches as far
+  bool last;             // the run's last lane, inside the bank
+};
+__device__ __forceinline__ DocRuns doc_runs(int doc, bool inside, int half, int l32) {
+  DocRuns r;
+  r.doc = doc;
+  const int prev = __builtin_amdgcn_update_dpp(doc, doc, 0x138, 0xF, 0xF, false);      // wave_shr:1
+  const uint64_t heads64 = __ballot(l32 == 0 || prev != doc);
+  const uint32_t heads = half ? (uint32_t)(heads64 >> 32) : (uint32_t)heads64;
+  const uint32_t upto = heads & ((2u << l32) - 1u);                  // heads at or below this lane (never empty)
+  const int dist = l32 - (31 - __builtin_clz(upto));                 // from the first lane of the run
+#pragma unroll
+  for (int k = 0; k < 4; ++k) r.take[k] = dist >= 1 << k ? 0xffffffffu : 0u;
+  r.take[4] = dist > (l32 & 15) ? 0xffffffffu : 0u;
+  r.last = inside && (l32 == 31 || ((heads >> (l32 + 1)) & 1u));
+  return r;
+}
+// The lanes' keys folded over the runs, into the query's row of the key plane.
+__device__ __forceinline__ void merge_runs(const DocRuns& r, float run, uint32_t* row, bool scored) {
+  uint32_t m = f32_to_key(run);
+#define MSA_SCAN_STEP(K, CTRL, ROWS) \
+  m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, CTRL, ROWS, 0xF, ROWS == 0xF) & r.take[K]);
+  MSA_SCAN_STEP(0, 0x111, 0xF)   // row_shr:1
+  MSA_SCAN_STEP(1, 0x112, 0xF)
+  MSA_SCAN_STEP(2, 0x114, 0xF)
+  MSA_SCAN_STEP(3, 0x118, 0xF)
+  MSA_SCAN_STEP(4, 0x142, 0xA)   // row_bcast:15 into rows 1, 3
+#undef MSA_SCAN_STEP
+  if (r.last && scored) atomicMax(row + r.doc, m);
+}
 template <typename T, int BM, int BN, int kSets, bool kStream>
 constexpr bool score_tile_is_direct_stream() {
   return sizeof(T) == 2 && BM == 128 && BN == 256 && kSets == 1 && kStream;
@@ -321,20 +379,23 @@ constexpr bool score_tile_is_direct_stream() {
 // more bytes in flight per compute unit than one tile holds.
 // kDocMax: keys are folded over the chunks of a document (chunk_doc) and merged into out_key[B, n_docs];
 // otherwise one key per (query, chunk) is merged into out_key[B, C].
+// kUnit: rows a query is a multiple of.  32: one that is scored counts whole.  8 and 4: short queries share a row block, whose word tells
+// the rows that count; a query of units of 4 is one unit.
 // kStream: one workgroup per compute-unit slot walks N tiles blockIdx.x, blockIdx.x + gridDim.x, ... (one M tile
 // only) with the load / store / multiply pipeline running across tile boundaries: the first K tiles of the next N
 // tile are already in flight while the last ones of the current tile are multiplied and its epilogue runs, so the
 // HBM stream never drains between tiles.  That is what the HBM-bound shapes need; the fp32 form keeps one
 // workgroup per tile.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int kSets, bool kDocMax, bool kStream>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int kSets, bool kDocMax, bool kStream, int kUnit = 32>
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void score_gemm_kernel(
     const T* __restrict__ qs,            // [M_rows, K]  pre-summed queries, M_rows = B * S_pad
     const T* __restrict__ kr,            // [C, K]
     const uint32_t* __restrict__ row_bits,  // [ceil(M_alloc / 32)] scored-row bitmask
     uint32_t* __restrict__ out_key,      // [B, n_docs] or [B, C], zeroed
     const int32_t* __restrict__ chunk_doc,  // [C] document of every chunk (kDocMax)
-    int32_t M_rows, int32_t C, int32_t K, int32_t blocks_per_query, int32_t tiles_m, int32_t tiles_n,
+    int32_t M_rows, int32_t C, int32_t K, int32_t units_per_query, int32_t tiles_m, int32_t tiles_n,
     int32_t m_group, int32_t n_docs) {
+  static_assert(kUnit == 32 || (kDocMax && (kUnit == 8 || kUnit == 4)), "packed queries are folded over documents");
   constexpr int kThreads = WAVES_M * WAVES_N * 64;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
   constexpr int TM = WM / 32, TN = WN / 32;
@@ -521,17 +582,17 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void score_gemm_kernel(
   // With one workgroup per compute unit nothing else runs while an epilogue waits, so it must not wait on memory:
   // the scored-row words of the wavefront's row blocks and the documents of its columns are requested ahead (before
   // the K loop / a tile ahead) and only consumed here, and the lane exchanges of the document fold are row moves.
-  const int n_queries = M_rows / (blocks_per_query * 32);
+  const int n_queries = M_rows / (units_per_query * kUnit);
   uint32_t rbits[TM];                                   // scored-row word of each row block (same in every lane)
-  // query of the wavefront's first row block and that block's place in the query: later blocks follow by counting
+  // query of the wavefront's first row block (unit) and its place in the query: later ones follow by counting
   // (one division per wavefront, under the first tile's load latency, instead of one per block in the epilogue)
   int q_first = 0, r_first = 0;
   auto fetch_rows = [&]() {
 #pragma unroll
     for (int i = 0; i < TM; ++i) rbits[i] = row_bits[(m0 + wm * WM + i * 32) >> 5];   // 0 past M_rows (buffer is padded)
-    const int blk0 = (m0 + wm * WM) >> 5;
-    q_first = blk0 / blocks_per_query;
-    r_first = blk0 - q_first * blocks_per_query;
+    const int blk0 = (m0 + wm * WM) / kUnit;
+    q_first = blk0 / units_per_query;
+    r_first = blk0 - q_first * units_per_query;
   };
   int cdoc[TN];                                         // document of each column; lanes past the bank never join a run
   auto fetch_docs = [&](int tile_n0) {
@@ -548,55 +609,76 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void score_gemm_kernel(
   // and the upper 32 lanes block 1's, so the segmented scan and the atomics below run once per query for the
   // wavefront's 64 columns instead of once per block with half the lanes idle.
   static_assert(TN == 2, "the epilogue pairs the two column blocks of a wavefront");
+  DocRuns runs[kUnit == 4 ? 2 : 1];      // of the wavefront's 64 columns, half a half; of either 32, in both halves, where a half has queries of its own
+  auto find_runs = [&](int tile_n0) {
+    if constexpr (kDocMax && kUnit == 4) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) runs[j] = doc_runs(cdoc[j], tile_n0 + wn * WN + j * 32 + l32 < C, half, l32);
+    } else if constexpr (kDocMax) {
+      runs[0] = doc_runs(half ? cdoc[1] : cdoc[0], tile_n0 + wn * WN + half * 32 + l32 < C, half, l32);
+    }
+  };
   auto emit = [&](int q, int tile_n0, const float (&run_half)[TN], bool any) {
     if (!any || q >= n_queries) return;
     const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(run_half[0]), __float_as_uint(run_half[1]), false, false);
     const float run = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-    const int n = tile_n0 + wn * WN + half * 32 + l32;
-    const int doc = kDocMax ? (half ? cdoc[1] : cdoc[0]) : 0;
-    const bool ok = n < C;
-    const uint32_t key = ok ? f32_to_key(run) : 0u;
     if constexpr (kDocMax) {
-      // Chunks of a document are adjacent columns: a segmented max-scan over the 32 lanes of each half leaves a
-      // document's maximum in the last lane of its run, which alone touches memory (about two atomics per 32
-      // chunks instead of 32 stores, and no per-chunk plane to read back).  `dist` is a lane's distance from the
-      // first lane of its run, from a ballot of the run heads; the scan itself moves keys only: four shifts inside
-      // the rows of 16 lanes, then lane 15 of the lower row joins the runs that cross into the upper one.  Lanes a
-      // shift cannot reach read 0, the identity of max over keys.
-      const int prev = __builtin_amdgcn_update_dpp(doc, doc, 0x138, 0xF, 0xF, false);      // wave_shr:1
-      const uint64_t heads64 = __ballot(l32 == 0 || prev != doc);
-      const uint32_t heads = half ? (uint32_t)(heads64 >> 32) : (uint32_t)heads64;
-      const uint32_t upto = heads & ((2u << l32) - 1u);                  // heads at or below this lane (never empty)
-      const int dist = l32 - (31 - __builtin_clz(upto));
-      const bool last = l32 == 31 || ((heads >> (l32 + 1)) & 1u);
-      int m = (int)key;
-#define MSA_SCAN_STEP(OFF, CTRL)                                                          \
-      {                                                                                   \
-        const int o = __builtin_amdgcn_update_dpp(0, m, CTRL, 0xF, 0xF, true);            \
-        if (dist >= OFF) m = (int)max((uint32_t)m, (uint32_t)o);                          \
-      }
-      MSA_SCAN_STEP(1, 0x111)   // row_shr:1
-      MSA_SCAN_STEP(2, 0x112)
-      MSA_SCAN_STEP(4, 0x114)
-      MSA_SCAN_STEP(8, 0x118)
-#undef MSA_SCAN_STEP
-      const int low = __builtin_amdgcn_update_dpp(0, m, 0x142, 0xA, 0xF, false);          // row_bcast:15 into rows 1, 3
-      if (dist > (l32 & 15)) m = (int)max((uint32_t)m, (uint32_t)low);
-      if (ok && last) atomicMax(&out_key[(int64_t)q * n_docs + doc], (uint32_t)m);
+      merge_runs(runs[0], run, out_key + (int64_t)q * n_docs, true);
     } else {
-      if (ok) atomicMax(&out_key[(int64_t)q * C + n], key);
+      const int n = tile_n0 + wn * WN + half * 32 + l32;
+      if (n < C) atomicMax(&out_key[(int64_t)q * C + n], f32_to_key(run));
     }
   };
+  auto four = [&](const floatx16_t& a, int g) { return fmaxf(fmaxf(a[4 * g], a[4 * g + 1]), fmaxf(a[4 * g + 2], a[4 * g + 3])); };
   auto epilogue = [&](int tile_n0) {
+    find_runs(tile_n0);
+    if constexpr (kUnit == 4) {
+      // registers 4 g .. 4 g + 3 of a block are rows of two queries, one a half of the wavefront: nothing to join
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const uint32_t bits = __builtin_amdgcn_readfirstlane(rbits[i]);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          if ((bits >> (8 * g) & 0xffu) == 0u) continue;
+          const bool scored = bits >> (8 * g + 4 * half) & 1u;
+          uint32_t* const row = out_key + (int64_t)(q_first + 8 * i + 2 * g + half) * n_docs;
+#pragma unroll
+          for (int j = 0; j < TN; ++j) merge_runs(runs[j], four(acc[i][j], g), row, scored);
+        }
+      }
+      return;
+    }
     float run[TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j) run[j] = -INFINITY;
     bool any = false;
     int run_q = q_first, r = r_first;                      // query of row block i, its block index inside the query
+    if constexpr (kUnit == 8) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const uint32_t bits = __builtin_amdgcn_readfirstlane(rbits[i]);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          if (r == units_per_query) {                      // the unit opens the next query
+            emit(run_q, tile_n0, run, any);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) run[j] = -INFINITY;
+            any = false; ++run_q; r = 0;
+          }
+          ++r;
+          if ((bits >> (8 * g) & 0xffu) == 0u) continue;
+#pragma unroll
+          for (int j = 0; j < TN; ++j) run[j] = fmaxf(run[j], four(acc[i][j], g));
+          any = true;
+        }
+      }
+      emit(run_q, tile_n0, run, any);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const uint32_t bits = __builtin_amdgcn_readfirstlane(rbits[i]);
-      if (r == blocks_per_query) {                         // row block i opens the next query
+      if (r == units_per_query) {                          // row block i opens the next query
         emit(run_q, tile_n0, run, any);
 #pragma unroll
         for (int j = 0; j < TN; ++j) run[j] = -INFINITY;
@@ -851,17 +933,21 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void score_gemm_kernel(
 #include "scan_walk.h"
 
 constexpr int kScan4CompilerVgprs = 128;     // the compiler's share of the vector registers in score_scan4_kernel
+constexpr int kScan4UnitsVgprs = 96;         // and in score_scan4_units_kernel, whose statements own v96 - v127 too
 constexpr int kScan4LdsBytes = 5 * 256 * 128;
 
-template <bool kDocMax>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerVgprs))) void score_scan4_kernel(
+// kUnits: short queries share row blocks in units of eight rows (RowPacking), up to four queries a block.  A block's word tells the units
+// that count, the reduction leaves a maximum per unit, and all of a tile's maxima are folded between two of the next tile's steps.
+template <bool kDocMax, bool kUnits>
+__device__ __forceinline__ void scan4_body(
     const bf16_t* __restrict__ qs,          // [M_rows, K]  pre-summed queries, M_rows = B * S_pad
     const bf16_t* __restrict__ kr,          // [C, K]
     const uint32_t* __restrict__ row_bits,  // [ceil(M_alloc / 32)] scored-row bitmask
     uint32_t* __restrict__ out_key,         // [B, n_docs] or [B, C], zeroed
     const int32_t* __restrict__ chunk_doc,  // [C] document of every chunk (kDocMax)
     int32_t M_rows, int32_t C, int32_t K, int32_t blocks_per_query, int32_t tiles_m, int32_t tiles_n, int32_t m_group,
-    int32_t n_docs, GatherJob job, uint32_t* __restrict__ sched, int32_t pool_n) {
+    int32_t n_docs, const GatherJob& job, uint32_t* __restrict__ sched, int32_t pool_n) {      // (kUnits: units per query)
+  [[maybe_unused]] constexpr int kUnit = kUnits ? 8 : 32;
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int kThreads = 256, BM = 256, BN = 256;
   extern __shared__ __align__(16) char lds[];
@@ -956,10 +1042,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
   const uint32_t zero_off = 0;
 
   // ---- epilogue state: see score_gemm_kernel's epilogue, of which this is the form with four row blocks ----
-  const int n_queries = M_rows / (blocks_per_query * 32);
+  const int n_queries = M_rows / (blocks_per_query * kUnit);
   typedef const __attribute__((address_space(4))) uint32_t* const_words_t;      // scalar loads
   const const_words_t row_bits_c = (const_words_t)row_bits;
-  // floor(2^32 / d) + 1 divides exactly while n * d < 2^32 (row blocks < 2^19, blocks per query <= 2^11)
+  // floor(2^32 / d) + 1 divides exactly while n * d < 2^32 (row blocks < 2^19, blocks per query <= 2^11; units < 2^21, a query's <= 2^7)
   const uint32_t bpq_magic = (uint32_t)(0x100000000ull / (uint32_t)blocks_per_query) + 1u;
   uint32_t rbits[4] = {0u, 0u, 0u, 0u};
   int q_first = 0, r_first = 0;
@@ -967,8 +1053,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
     const int blk0 = (m0 + wm * 128) >> 5;
 #pragma unroll
     for (int i = 0; i < 4; ++i) rbits[i] = row_bits_c[blk0 + i];          // 0 past M_rows (the buffer is padded)
-    q_first = blocks_per_query == 1 ? blk0 : (int)__umulhi((uint32_t)blk0, bpq_magic);     // blk0 / blocks_per_query
-    r_first = blk0 - q_first * blocks_per_query;
+    const int first = (m0 + wm * 128) / kUnit;
+    q_first = blocks_per_query == 1 ? first : (int)__umulhi((uint32_t)first, bpq_magic);     // first / blocks_per_query
+    r_first = first - q_first * blocks_per_query;
   };
   // the documents of the wavefront's 128 columns, 64 per load, into v220 / v221 (v216: their offsets): requested in
   // front of a K step (whose waits cover them), read when the tile's maxima are folded; columns past the bank read 0
@@ -981,38 +1068,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
                    ::"s"(rsrc_docs), "s"(first) : MSA_SCAN4_CLOBBERS);
     }
   };
-  // One group of 64 columns, a column a lane: the segmented scan leaves a document's maximum in the last lane of its
-  // run, which alone touches memory.
-  auto emit_group = [&](int q, int n_first, float run, int doc_raw) {
-    const int n = n_first + lane;
-    const bool ok = n < C;
-    const uint32_t key = ok ? f32_to_key(run) : 0u;
-    if constexpr (kDocMax) {
-      const int doc = ok ? doc_raw : -1 - l32;
-      const int prev = __builtin_amdgcn_update_dpp(doc, doc, 0x138, 0xF, 0xF, false);      // wave_shr:1
-      const uint64_t heads64 = __ballot(l32 == 0 || prev != doc);
-      const uint32_t heads = half ? (uint32_t)(heads64 >> 32) : (uint32_t)heads64;
-      const uint32_t upto = heads & ((2u << l32) - 1u);                  // heads at or below this lane (never empty)
-      const int dist = l32 - (31 - __builtin_clz(upto));
-      const bool last = l32 == 31 || ((heads >> (l32 + 1)) & 1u);
-      int m = (int)key;
-#define MSA_SCAN_STEP(OFF, CTRL)                                                          \
-      {                                                                                   \
-        const int o = __builtin_amdgcn_update_dpp(0, m, CTRL, 0xF, 0xF, true);            \
-        if (dist >= OFF) m = (int)max((uint32_t)m, (uint32_t)o);                          \
-      }
-      MSA_SCAN_STEP(1, 0x111)   // row_shr:1
-      MSA_SCAN_STEP(2, 0x112)
-      MSA_SCAN_STEP(4, 0x114)
-      MSA_SCAN_STEP(8, 0x118)
-#undef MSA_SCAN_STEP
-      const int low = __builtin_amdgcn_update_dpp(0, m, 0x142, 0xA, 0xF, false);          // row_bcast:15 into rows 1, 3
-      if (dist > (l32 & 15)) m = (int)max((uint32_t)m, (uint32_t)low);
-      if (ok && last) atomicMax(&out_key[(int64_t)q * n_docs + doc], (uint32_t)m);
-    } else {
-      if (ok) atomicMax(&out_key[(int64_t)q * C + n], key);
-    }
-  };
   // Folds the finished tile's block maxima (v224 - v239, left by the reduction that rides in the next tile's first K
   // step or by the stand-alone one): row blocks of one query are joined, and at a query's end the two pairs of column
   // blocks are merged into the key plane.  Every row of a scored block counts (the prologue kernel made unscored rows
@@ -1020,18 +1075,54 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
   // past M_rows and is skipped.
   auto fold_tile = [&](int n0) {
     float mx[8];
-    asm volatile(MSA_SCAN4_MAX_READ
-                 : "=v"(mx[0]), "=v"(mx[1]), "=v"(mx[2]), "=v"(mx[3]), "=v"(mx[4]), "=v"(mx[5]), "=v"(mx[6]), "=v"(mx[7]));
-    int doc0 = 0, doc1 = 0;
-    if constexpr (kDocMax) asm volatile("v_mov_b32 %0, v220\n\tv_mov_b32 %1, v221" : "=v"(doc0), "=v"(doc1));
+#define MSA_SCAN4_READ8(TEXT)                                                                                                     \
+    asm volatile(TEXT : "=v"(mx[0]), "=v"(mx[1]), "=v"(mx[2]), "=v"(mx[3]), "=v"(mx[4]), "=v"(mx[5]), "=v"(mx[6]), "=v"(mx[7]))
+    const int n_first = n0 + wn * 128 + lane;      // the lane's columns: this one and the 64th behind it
+    DocRuns runs[2];
+    if constexpr (kDocMax) {
+      int doc0, doc1;
+      asm volatile("v_mov_b32 %0, v220\n\tv_mov_b32 %1, v221" : "=v"(doc0), "=v"(doc1));
+      runs[0] = doc_runs(n_first < C ? doc0 : -1 - l32, n_first < C, half, l32);
+      runs[1] = doc_runs(n_first + 64 < C ? doc1 : -1 - l32, n_first + 64 < C, half, l32);
+    }
     float run[2] = {-INFINITY, -INFINITY};
     bool any = false;
     int run_q = q_first, r = r_first;
     auto emit = [&]() {
       if (!any || run_q >= n_queries) return;
-      emit_group(run_q, n0 + wn * 128, run[0], doc0);
-      emit_group(run_q, n0 + wn * 128 + 64, run[1], doc1);
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        if constexpr (kDocMax) merge_runs(runs[p], run[p], out_key + (int64_t)run_q * n_docs, true);
+        else if (n_first + 64 * p < C) atomicMax(&out_key[(int64_t)run_q * C + n_first + 64 * p], f32_to_key(run[p]));
+      }
     };
+    if constexpr (kUnits) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (i == 0) MSA_SCAN4_READ8(MSA_SCAN4_UNIT_READ_0);
+        if (i == 1) MSA_SCAN4_READ8(MSA_SCAN4_UNIT_READ_1);
+        if (i == 2) MSA_SCAN4_READ8(MSA_SCAN4_UNIT_READ_2);
+        if (i == 3) MSA_SCAN4_READ8(MSA_SCAN4_UNIT_READ_3);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (r == blocks_per_query) {                     // the unit opens the next query
+            emit();
+            run[0] = run[1] = -INFINITY;
+            any = false; ++run_q; r = 0;
+          }
+          ++r;
+          if (rbits[i] >> (8 * u) & 0xffu) {
+            any = true;
+            run[0] = fmaxf(run[0], mx[u]);
+            run[1] = fmaxf(run[1], mx[4 + u]);
+          }
+        }
+      }
+      emit();
+      return;
+    }
+    MSA_SCAN4_READ8(MSA_SCAN4_MAX_READ);
+#undef MSA_SCAN4_READ8
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (r == blocks_per_query) {                         // row block i opens the next query
@@ -1068,9 +1159,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
     // out so that between two of them the scalar unit has next to nothing to do (a wavefront that is alone on its SIMD
     // pays for every instruction between two MFMAs): the resources a step reads are fixed per loop, and the tile
     // pool's hops ride in front of four peeled steps.
-#define MSA_SCAN4_STEP(TEXT, RA, RB, KOFF)                                                                   \
+#define MSA_SCAN4_STEP_CLOBBERS(TEXT, RA, RB, KOFF, ...)                                                     \
     asm volatile(TEXT : [sa] "+s"(sa), [sb] "+s"(sb)                                                         \
-                 : [ra] "s"(RA), [rb] "s"(RB), [k] "s"(KOFF), [woff] "s"(woff) : MSA_SCAN4_CLOBBERS)
+                 : [ra] "s"(RA), [rb] "s"(RB), [k] "s"(KOFF), [woff] "s"(woff) : __VA_ARGS__)
+#define MSA_SCAN4_STEP(TEXT, RA, RB, KOFF) MSA_SCAN4_STEP_CLOBBERS(TEXT, RA, RB, KOFF, MSA_SCAN4_CLOBBERS)
     const bool pending = nxt_pending;      // the tile behind this one comes from the pool (k_tiles >= 6 then)
     if (pending && drawer && lane == 0)    // v217 = counter++
       asm volatile("s_nop 4\n\tglobal_atomic_add v217, %0, v223, %1 sc0" ::"v"(zero_off), "s"(pool_counter) : "memory");
@@ -1079,7 +1171,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
     // the tile lies inside the bank: then the step also folds the maxima into the key plane.  Otherwise it leaves one
     // maximum per block and fold_tile() does the rest; a wavefront whose rows are all padding has nothing to fold.
     const bool fold_any = have_prev && (rbits[0] | rbits[1] | rbits[2] | rbits[3]) != 0;
-    const bool fold_fast = kDocMax && fold_any && (blocks_per_query & 3) == 0 && rbits[0] != 0 && prev_n0 + BN <= C;
+    const bool fold_fast = kDocMax && !kUnits && fold_any && (blocks_per_query & 3) == 0 && rbits[0] != 0 && prev_n0 + BN <= C;
     if (fold_fast) {
       const uint32_t* okey = out_key + (int64_t)q_first * n_docs;
       if (k_tiles > 2)
@@ -1088,6 +1180,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
       else
         asm volatile(MSA_SCAN4_KSTEP_FRESH_FOLD : [sa] "+s"(sa), [sb] "+s"(sb)
                      : [ra] "s"(ra_n), [rb] "s"(rb_n), [k] "s"(0), [woff] "s"(woff), [okey] "s"(okey) : MSA_SCAN4_CLOBBERS);
+    } else if (kUnits && fold_any) {
+      if (k_tiles > 2) MSA_SCAN4_STEP_CLOBBERS(MSA_SCAN4_KSTEP_FRESH_UNITS, ra_c, rb_c, 2 * kRowBytes, MSA_SCAN4_UNITS_CLOBBERS);
+      else MSA_SCAN4_STEP_CLOBBERS(MSA_SCAN4_KSTEP_FRESH_UNITS, ra_n, rb_n, 0, MSA_SCAN4_UNITS_CLOBBERS);
+      fold_tile(prev_n0);
     } else if (fold_any) {
       if (k_tiles > 2) MSA_SCAN4_STEP(MSA_SCAN4_KSTEP_FRESH_REDUCE, ra_c, rb_c, 2 * kRowBytes);
       else MSA_SCAN4_STEP(MSA_SCAN4_KSTEP_FRESH_REDUCE, ra_n, rb_n, 0);
@@ -1120,6 +1216,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
     for (int k_l = (kt + 2) * kRowBytes; k_l < row_bytes; k_l += kRowBytes) MSA_SCAN4_STEP(MSA_SCAN4_KSTEP, ra_c, rb_c, k_l);
     for (int k_l = k_tiles > 2 ? 0 : kRowBytes; k_l < 2 * kRowBytes; k_l += kRowBytes) MSA_SCAN4_STEP(MSA_SCAN4_KSTEP, ra_n, rb_n, k_l);
 #undef MSA_SCAN4_STEP
+#undef MSA_SCAN4_STEP_CLOBBERS
     have_prev = true;
     prev_n0 = n0;
     if (!nxt_valid) break;
@@ -1127,11 +1224,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerV
     ra_c = ra_n; rb_c = rb_n;
     plan_next();
   }
-  asm volatile(MSA_SCAN4_REDUCE ::: MSA_SCAN4_CLOBBERS);
+  if constexpr (kUnits) asm volatile(MSA_SCAN4_REDUCE_UNITS ::: MSA_SCAN4_UNITS_CLOBBERS);
+  else asm volatile(MSA_SCAN4_REDUCE ::: MSA_SCAN4_CLOBBERS);
   fold_tile(prev_n0);
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 #endif
 }
+
+#define MSA_SCAN4_PARAMS                                                                                                          \
+  const bf16_t *__restrict__ qs, const bf16_t *__restrict__ kr, const uint32_t *__restrict__ row_bits, uint32_t *__restrict__ out_key, \
+      const int32_t *__restrict__ chunk_doc, int32_t M_rows, int32_t C, int32_t K, int32_t per_query, int32_t tiles_m, int32_t tiles_n, \
+      int32_t m_group, int32_t n_docs, GatherJob job, uint32_t *__restrict__ sched, int32_t pool_n
+template <bool kDocMax>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4CompilerVgprs))) void score_scan4_kernel(MSA_SCAN4_PARAMS) {
+  scan4_body<kDocMax, false>(qs, kr, row_bits, out_key, chunk_doc, M_rows, C, K, per_query, tiles_m, tiles_n, m_group, n_docs, job, sched, pool_n);
+}
+__global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(kScan4UnitsVgprs))) void score_scan4_units_kernel(MSA_SCAN4_PARAMS) {
+  scan4_body<true, true>(qs, kr, row_bits, out_key, chunk_doc, M_rows, C, K, per_query, tiles_m, tiles_n, m_group, n_docs, job, sched, pool_n);
+}
+#undef MSA_SCAN4_PARAMS
 
 // chunk_key -> fp32 scores (times scale / Hq); key 0 (query without a scored token) -> -inf.
 __global__ void decode_scores_kernel(const uint32_t* __restrict__ key, int64_t n, float mul,
@@ -1521,9 +1632,9 @@ int compute_units() {
   return n;
 }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int kSets, bool kDocMax, bool kStream>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int kSets, bool kDocMax, bool kStream, int kUnit = 32>
 int launch_gemm(const void* qs, const void* kr, const uint32_t* row_bits, uint32_t* out_key, const int32_t* chunk_doc,
-                int32_t M_rows, int32_t C, int32_t K, int32_t blocks_per_query, int32_t n_docs, hipStream_t st) {
+                int32_t M_rows, int32_t C, int32_t K, int32_t units_per_query, int32_t n_docs, hipStream_t st) {
   const size_t lds = score_tile_is_direct_stream<T, BM, BN, kSets, kStream>() ? (size_t)kDtlStreamLdsBytes
                                                                                : (size_t)2 * (BM + BN) * kRowStride;
   const int tiles_m = (M_rows + BM - 1) / BM;
@@ -1541,7 +1652,7 @@ int launch_gemm(const void* qs, const void* kr, const uint32_t* row_bits, uint32
     }
     grid = std::min(tiles_n, compute_units() * std::max<int>(1, (int)(kLdsPerCu / lds)));
   }
-  auto kern = score_gemm_kernel<T, BM, BN, WAVES_M, WAVES_N, kSets, kDocMax, kStream>;
+  auto kern = score_gemm_kernel<T, BM, BN, WAVES_M, WAVES_N, kSets, kDocMax, kStream, kUnit>;
   static std::atomic<int> lds_limit_raised{0};
   MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(kern), (int)lds));
   int slot = -1;
@@ -1551,7 +1662,7 @@ int launch_gemm(const void* qs, const void* kr, const uint32_t* row_bits, uint32
   }
   if (slot >= 0) MSA_HIP(hipEventRecord(g_timer.start[slot], st));
   kern<<<grid, WAVES_M * WAVES_N * 64, lds, st>>>(static_cast<const T*>(qs), static_cast<const T*>(kr), row_bits, out_key,
-                                                  chunk_doc, M_rows, C, K, blocks_per_query, tiles_m, tiles_n, m_group,
+                                                  chunk_doc, M_rows, C, K, units_per_query, tiles_m, tiles_n, m_group,
                                                   n_docs);
   MSA_LAUNCH_CHECK();
   if (slot >= 0) MSA_HIP(hipEventRecord(g_timer.stop[slot], st));
@@ -1641,7 +1752,7 @@ int launch_parts(const void* qs, const void* kr, const uint32_t* row_bits, uint3
 // Launch of the MFMA-bound form (score_scan4_kernel): one workgroup per compute unit, persistent.
 std::atomic<int> g_tile_pool_enabled{1};
 
-template <bool kDocMax>
+template <bool kDocMax, bool kUnits = false>
 int launch_scan4(const void* qs, const void* kr, const uint32_t* row_bits, uint32_t* out_key, const int32_t* chunk_doc,
                  int32_t M_rows, int32_t C, int32_t K, int32_t blocks_per_query, int32_t n_docs, hipStream_t st,
                  const GatherJob* job, bool* job_taken, uint32_t* sched) {
@@ -1674,8 +1785,9 @@ int launch_scan4(const void* qs, const void* kr, const uint32_t* row_bits, uint3
     if (job_taken) *job_taken = true;
   }
   auto kern = score_scan4_kernel<kDocMax>;
+  if constexpr (kUnits) kern = score_scan4_units_kernel;
   static std::atomic<int> lds_limit_raised{0}, resources_checked{0};
-  if (const int rc = check_asm_kernel_resources(resources_checked, reinterpret_cast<const void*>(kern), "score_scan4_kernel",
+  if (const int rc = check_asm_kernel_resources(resources_checked, reinterpret_cast<const void*>(kern), kUnits ? "score_scan4_units_kernel" : "score_scan4_kernel",
                                                 nullptr, nullptr))
     return rc;
   MSA_HIP(raise_dynamic_lds_limit(lds_limit_raised, reinterpret_cast<const void*>(kern), kScan4LdsBytes));
@@ -1703,7 +1815,18 @@ int launch_scan4(const void* qs, const void* kr, const uint32_t* row_bits, uint3
 template <bool kDocMax>
 int launch_gemm_for(int32_t dtype, const void* qs, const void* kr, const uint32_t* row_bits, uint32_t* out_key,
                     const int32_t* chunk_doc, int32_t M_rows, int32_t C, int32_t K, int32_t bpq, int32_t n_docs,
-                    hipStream_t st, const GatherJob* job, bool* job_taken, uint32_t* sched) {
+                    hipStream_t st, const GatherJob* job, bool* job_taken, uint32_t* sched, int unit, bool by_units) {
+  if constexpr (kDocMax) {
+    if (by_units) return launch_scan4<true, true>(qs, kr, row_bits, out_key, chunk_doc, M_rows, C, K, bpq, n_docs, st, job, job_taken, sched);
+    if (unit == 8 && M_rows <= 64)
+      return launch_gemm<bf16_t, 64, 128, 2, 2, 2, true, true, 8>(qs, kr, row_bits, out_key, chunk_doc, M_rows, C, K, bpq, n_docs, st);
+    if (unit == 8)
+      return launch_gemm<bf16_t, 128, 256, 2, 4, 1, true, true, 8>(qs, kr, row_bits, out_key, chunk_doc, M_rows, C, K, bpq, n_docs, st);
+    if (unit == 4 && M_rows <= 64)
+      return launch_gemm<bf16_t, 64, 128, 2, 2, 2, true, true, 4>(qs, kr, row_bits, out_key, chunk_doc, M_rows, C, K, bpq, n_docs, st);
+    if (unit == 4)
+      return launch_gemm<bf16_t, 128, 256, 2, 4, 1, true, true, 4>(qs, kr, row_bits, out_key, chunk_doc, M_rows, C, K, bpq, n_docs, st);
+  }
   // The line between the fp32 forms: above it the tiles' reuse of both operands is worth more than the even split (16384 chunks x
   // 128 rows: 61 us in the split form, 84 in tiles; x 256 rows 95 and 88; 65536 x 128: 190 and 151), except that the tiles pad up
   // to 64 rows to 128 (65536 x 64: 123 and 142).
@@ -1725,10 +1848,10 @@ int launch_gemm_for(int32_t dtype, const void* qs, const void* kr, const uint32_
 // ------------------------------------------------------------------------------------------
 
 RouteWorkspace route_workspace_layout(int32_t B, int32_t S, int32_t Hkv, int32_t D, int64_t plane_cols, int64_t n_docs,
-                                      int32_t dtype, bool parts) {
+                                      int32_t dtype, bool parts, int32_t unit) {
   RouteWorkspace w{};
-  w.S_pad = (S + 31) / 32 * 32;
-  w.M_rows = B * w.S_pad;
+  w.S_pad = (S + unit - 1) / unit * unit;
+  w.M_rows = (B * w.S_pad + 31) / 32 * 32;
   const int64_t m_alloc = ((int64_t)w.M_rows + 255) / 256 * 256;   // every M tile may read whole mask words
   w.mask_words = (int32_t)(m_alloc / 32);
   size_t off = 0;
@@ -1744,6 +1867,33 @@ RouteWorkspace route_workspace_layout(int32_t B, int32_t S, int32_t Hkv, int32_t
 }
 
 namespace {
+// How the rows of a batch of queries lie in the scan (bf16, maxima over tokens and chunks).  A query has row blocks of 32 of its own, or,
+// where that asks for a smaller form of the scan or fewer of its large tiles, queries are padded to units of 8 or 4 rows and share
+// blocks: the padding is multiplied like the rest, 4 tokens in 32 rows eight times over.  What it costs is a fold per query in place of
+// one per block, and in the large tiles a fold between two steps (16 queries of 104 rows 4129 -> 3930 us where one tile row in eight goes).
+// Whole calls, us, row blocks of their own and shared ones, 1.6M chunks: 28 queries x 2 tokens 2059 -> 597, 22 x 4 1550 -> 574, 10 x 3
+// 1118 -> 525, 7 x 5 599 -> 510, 16 x 8 1114 -> 580, 32 x 8 2078 -> 760 (one row of large tiles: every step waits for K_r), 6 x 37 1192 ->
+// 703, 32 x 37 4118 -> 2928, 5 x 20 613 -> 547; 160,000 chunks: 28 x 2 230 -> 86, 32 x 37 426 -> 326.  Where all tiles are one round
+// anyway the blocks stay apart (20,000 chunks, 9 x 37: 35.9 and 37.9).  A scan that carries a gather stays one that can.
+struct RowPacking {
+  int32_t unit;
+  bool by_units;      // the large tiles, rows in the order of their units
+};
+RowPacking row_packing(int32_t B, int32_t S, int64_t C, bool gathers) {
+  auto rows = [&](int unit) { return (int64_t)B * ((S + unit - 1) / unit * unit); };
+  const int64_t whole = rows(32);
+  if (!gathers || whole <= 128)
+    for (const int64_t most : {64, 128}) {
+      if (whole <= most) return {32, false};
+      if (rows(8) <= most) return {8, false};
+      if (S <= 4 && rows(4) <= most) return {4, false};
+    }
+  // rounds of tiles that the compute units have to multiply
+  auto rounds = [&](int64_t m) { return ((m + 255) / 256 * ((C + 255) / 256) + compute_units() - 1) / compute_units(); };
+  if (S <= 1024 && rounds(rows(8)) < rounds(whole)) return {8, true};
+  return {32, false};
+}
+
 // Whether some bank's fp32 queries of these sizes come in parts.
 bool may_take_parts(int32_t B, int32_t S, int32_t Hkv, int32_t D) { return (int64_t)B * ((S + 31) / 32 * 32) <= kPartsMaxRows && Hkv * D == kSplitK; }
 }  // namespace
@@ -1794,6 +1944,15 @@ extern "C" int msa_diag_scan_walk(int32_t tiles_m, int32_t tiles_n, int32_t grid
     }
     draws.swap(still);
   }
+  return MSA_OK;
+}
+
+// How route_scores_to_keys lays the rows of a call's queries (a test aid).
+extern "C" int msa_diag_row_packing(int32_t B, int32_t S, int64_t C, int32_t gathers, int32_t* unit, int32_t* by_units) {
+  MSA_REQUIRE(unit != nullptr && by_units != nullptr && B > 0 && S > 0 && C > 0, "msa_diag_row_packing: null output, or no rows");
+  const RowPacking p = row_packing(B, S, C, gathers != 0);
+  *unit = p.unit;
+  *by_units = p.by_units;
   return MSA_OK;
 }
 
@@ -1907,6 +2066,10 @@ int route_scores_to_keys(const msa_bank* bank, int32_t layer, const void* q, con
     msa_set_error("%s: workspace of %zu bytes, need %zu", who, workspace_bytes, w.bytes);
     return MSA_ESIZE;
   }
+  RowPacking packing{32, false};
+  if (bank->dtype == MSA_BF16 && doc_max && query_reduce == kQueryMax) packing = row_packing(B, S, bank->C, job != nullptr && job->active);
+  if (packing.unit != 32)      // (no more rows than whole blocks have: it fits where they do)
+    w = route_workspace_layout(B, S, bank->Hkv, bank->D, plane_cols + extra_plane_cols, bank->n_docs, bank->dtype, false, packing.unit);
   char* ws = static_cast<char*>(workspace);
   void* qs = ws + w.off_qs;
   uint32_t* row_bits = reinterpret_cast<uint32_t*>(ws + w.off_row_bits);
@@ -1936,28 +2099,28 @@ int route_scores_to_keys(const msa_bank* bank, int32_t layer, const void* q, con
   } else if (bank->dtype == MSA_BF16) {
     presum_queries_kernel<bf16_t, bf16_t><<<w.M_rows, pthreads, 0, st>>>(
         static_cast<const bf16_t*>(q), qmask_u8, B, S, w.S_pad, Hq, bank->Hkv, normalize, static_cast<bf16_t*>(qs),
-        row_bits, w.mask_words, key, clear_words, sched);
+        row_bits, w.mask_words, key, clear_words, sched, packing.unit != 32, packing.by_units);
   } else if (parts) {
     presum_queries_kernel<float, float, true><<<w.M_rows, pthreads, 0, st>>>(
         static_cast<const float*>(q), qmask_u8, B, S, w.S_pad, Hq, bank->Hkv, normalize, static_cast<float*>(qs),
-        row_bits, w.mask_words, key, clear_words, sched);
+        row_bits, w.mask_words, key, clear_words, sched, 0, 0);
   } else {
     presum_queries_kernel<float, float><<<w.M_rows, pthreads, 0, st>>>(
         static_cast<const float*>(q), qmask_u8, B, S, w.S_pad, Hq, bank->Hkv, normalize, static_cast<float*>(qs),
-        row_bits, w.mask_words, key, clear_words, sched);
+        row_bits, w.mask_words, key, clear_words, sched, 0, 0);
   }
   MSA_LAUNCH_CHECK();
 
   const int32_t K = bank->Hkv * bank->D;
-  const int32_t bpq = w.S_pad / 32;
+  const int32_t bpq = w.S_pad / packing.unit;      // row blocks (units) of a query
   const auto by_parts = doc_max ? launch_parts<true> : launch_parts<false>;
   const int rc = parts ? by_parts(qs, bank->kr_dev[layer], row_bits, key, doc_max ? bank->chunk_doc_dev : nullptr, w.M_rows, (int32_t)bank->C, bpq,
                                   (int32_t)bank->n_docs, st)
                  : doc_max ? launch_gemm_for<true>(bank->dtype, qs, bank->kr_dev[layer], row_bits, key, bank->chunk_doc_dev,
                                                  w.M_rows, (int32_t)bank->C, K, bpq, (int32_t)bank->n_docs, st, job,
-                                                 job_taken, sched)
+                                                 job_taken, sched, packing.unit, packing.by_units)
                          : launch_gemm_for<false>(bank->dtype, qs, bank->kr_dev[layer], row_bits, key, nullptr, w.M_rows,
-                                                  (int32_t)bank->C, K, bpq, (int32_t)bank->n_docs, st, job, job_taken, sched);
+                                                  (int32_t)bank->C, K, bpq, (int32_t)bank->n_docs, st, job, job_taken, sched, 32, false);
   if (rc != MSA_OK) return rc;
   *layout_out = w;
   *mul_out = sc / (float)Hq;
