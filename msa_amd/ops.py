@@ -492,6 +492,7 @@ def tile_linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
 
 TILE_MIN = 144 << 16    # outputs (144 tiles of 256 x 256) from which tile_linear with an end is at least the equal of the vendor's two launches
 TILE_PLAIN = 256 << 16  # without one, where the vendor's tiles fit the columns
+DEEP, DEEP_ROWS, DEEP_TILES = 8192, 448, (20, 110)
 TILE_ROWS = 256         # no matrix of the models has outputs enough for fewer rows
 
 
@@ -502,11 +503,14 @@ def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1, end: boo
     times the speed; without one and N no multiple of 256 1600 x 1024 x 6176 1.10, 900 x 2560 x 14944 1.17 times.  Where N is one, a single
     round of tiles is behind the vendor's smaller ones (6001 x 9728 x 2560 199 and 217, 6001 x 4096 x 2560 86 and 93, 10000 x 3072 x 1024 53 and
     63), and several are level or ahead (7000 x 2560 x 2560 1.14 times, 6001 x 4096 x 12288 1.28, but 4096 x 2560 x 6144 0.87).  Padding does not
-    count.  Depths under 1024 were not measured and stay where they were."""
+    count.  Deep products whose tiles are less than half a round, cut into pieces of K, are ahead as well (``DEEP``; weights not in the caches: 500 x 9728 x 2560 51.1 and 46.2,
+    769 76 and 58, 1492 89 and 78, 2340 189 and 116; a third of a round deeper or half as deep they are level or behind: 3200 x 9728 x 2560 130 and 150, 1492 x
+    4096 x 2560 42 and 47).  Depths under 1024 were not measured and stay where they were."""
     N = matrices * w.shape[0]
     K = x.shape[-1]
     if x.numel() * N < (TILE_MIN if end or N % 256 else TILE_PLAIN) * max(K, 1):   # (most calls end here: steps of few tokens wait for the host)
-        return False
+        if end or N % 256 or K < DEEP or x.numel() < DEEP_ROWS * K or not DEEP_TILES[0] <= -(-x.numel() // (256 * K)) * (N // 256) <= DEEP_TILES[1]:
+            return False
     T = x.numel() // K
     return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == K
             and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 21))
