@@ -51,6 +51,15 @@ const char* msa_last_error(void);
 int msa_abi_version(void);
 
 /* ---------------------------------------------------------------------------------------------
+ * Segments of a packed block [template (ids -2) | documents]: the template, if it has tokens, and every run of equal ids behind it
+ * (src/msa/memory_sparse_attention.py:137-163).  ids, mask (may be null) and pos (may be null): int64 [T].
+ * head (int32 [8]): tokens of the template, documents, whether some id behind the template is not positive, the largest position
+ * (clamped to int32), the low and high word of the mask's sum.  cu [T + 2]: first token of every segment and the end; start [T + 8] and
+ * len [T + 1]: the same as int64, and tokens of every segment.  What lies behind the segments has no meaning. */
+int msa_block_segments(const int64_t* ids, const int64_t* mask, const int64_t* pos, int64_t T, int32_t* head, int32_t* cu,
+                       int64_t* start, int32_t* len, void* stream);
+
+/* ---------------------------------------------------------------------------------------------
  * Chunk table of a packed block.  Replaces the nonzero / unique_consecutive / cumsum /
  * repeat_interleave chain of src/msa/memory_sparse_attention.py:138-163 and the per-document
  * ceil(len / P) of src/prefill.py:225.

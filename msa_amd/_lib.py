@@ -22,6 +22,7 @@ _vp, _i32, _i64, _f32, _sz = C.c_void_p, C.c_int32, C.c_int64, C.c_float, C.c_si
 SIGNATURES = {
     "msa_last_error": (C.c_char_p, []),
     "msa_abi_version": (C.c_int, []),
+    "msa_block_segments": (C.c_int, [_vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp]),
     "msa_chunk_table": (C.c_int, [_vp, _i32, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp]),
     "msa_pool_chunks": (C.c_int, [_vp, _vp, _vp, _i32, _i64, _i32, _i32, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i32,
                                   _i32, _i32, _vp, _vp, _vp, _vp]),

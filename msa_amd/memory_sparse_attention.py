@@ -249,16 +249,27 @@ class MemorySparseAttention(nn.Module):
         if B != 1:
             raise ValueError("stage 1 takes one packed block at a time (batch size 1)")
         Hq, Hkv, D, P = self.config.num_attention_heads, self.num_kv_heads, self.head_dim, self.pooling_kernel_size
-        ids = doc_ids[0]
-        n_template = int((ids == -2).sum())
-        vals, counts = torch.unique_consecutive(ids[n_template:], return_counts=True)
-        doc_lens = counts.tolist()
-        if (vals <= 0).any() or (attention_mask is not None and int(attention_mask.sum()) != T):
+        block = cache.meta.get("block_segments")                # of this forward pass, where the model has them found for all layers
+        if block is not None and (block.ids is not doc_ids or block.mask is not attention_mask):
+            block = None
+        if block is not None:
+            if not block.done:
+                block.read()
+                cache.meta["q_lens_host"] = [block.mask_sum]
+                self.check_positions(block.last_position)
+            n_template, doc_lens, bad = block.n_template, block.doc_lens, block.bad or block.mask_sum != T
+        else:
+            ids = doc_ids[0]
+            n_template = int((ids == -2).sum())
+            vals, counts = torch.unique_consecutive(ids[n_template:], return_counts=True)
+            doc_lens = counts.tolist()
+            bad = (vals <= 0).any() or (attention_mask is not None and int(attention_mask.sum()) != T)
+        if bad:
             raise ValueError("stage 1 expects [template (-2) | documents (ids > 0)] with no padding")
         kwargs = {"template_prefix_kcache": k[:, :n_template].transpose(1, 2),          # [1, Hkv, n, D] views
                   "template_prefix_vcache": v[:, :n_template].transpose(1, 2)}
         if self.is_router_layer:
-            table = ops.chunk_table(doc_lens, P, first_token=n_template, device=hidden_states.device)
+            table = block.table(P) if block is not None else ops.chunk_table(doc_lens, P, first_token=n_template, device=hidden_states.device)
             if not self.decouple_router:
                 rk = None
             elif router_k is not None:                       # came out of the fused projection
@@ -275,11 +286,13 @@ class MemorySparseAttention(nn.Module):
         cache.record_kwargs(self.layer_idx, kwargs)
 
         # every document (and the template head) attends causally within itself
-        seg = ([n_template] if n_template else []) + doc_lens
-        cu = torch.tensor([0] + seg, dtype=torch.int64).cumsum(0)
-        dev = hidden_states.device
-        out = ops.sparse_attn(q[0], k[0], v[0], cu[:-1].to(dev), torch.tensor(seg, dtype=torch.int32, device=dev),
-                              max(seg), cu_q=cu.to(torch.int32).to(dev), max_sq=max(seg), scale=self.scaling, causal=True)
+        if block is not None:
+            seg, cu, start, lens = block.lens, block.cu, block.start, block.len
+        else:
+            seg = ([n_template] if n_template else []) + doc_lens
+            cu, dev = torch.tensor([0] + seg, dtype=torch.int64).cumsum(0), hidden_states.device
+            cu, start, lens = cu.to(torch.int32).to(dev), cu[:-1].to(dev), torch.tensor(seg, dtype=torch.int32, device=dev)
+        out = ops.sparse_attn(q[0], k[0], v[0], start, lens, max(seg), cu_q=cu, max_sq=max(seg), scale=self.scaling, causal=True)
         return ops.linear(self.o_proj, out.view(1, T, Hq * D)), None
 
     # ------------------------------------------------------------------------------------------ stage 2

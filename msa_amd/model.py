@@ -16,6 +16,7 @@ from .config import MSAConfig
 from .generation import greedy_decode
 from .memory_sparse_attention import MemorySparseAttention, RMSNorm, rotary_embedding
 from .prefill import query_position_ids, source_block_position_ids
+from .seq_ops import upload
 
 
 class MLP(nn.Module):
@@ -133,6 +134,19 @@ class MSAModel(nn.Module):
             h = ops.embed_rows(e.weight, input_ids)
         else:
             h = e(input_ids)
+        block = self._block_segments(h, attention_mask, position_ids, past_key_values, doc_ids)
+        if block is not None:
+            # stage 1: the block's segments, positions and mask are read once, by the first layer, which has its projections enqueued by then
+            past_key_values.meta["block_segments"] = block
+            try:
+                for layer in self.layers:
+                    h = layer(h, doc_ids, attention_mask, None, past_key_values, position_ids=position_ids)
+            finally:
+                past_key_values.meta.pop("block_segments", None)
+            if not block.done:                         # (no layer of this class's has run)
+                past_key_values.meta["q_lens_host"] = [block.read().mask_sum]
+                self.layers[0].self_attn.check_positions(block.last_position)
+            return ops.rmsnorm(h, self.norm.weight, self.norm.variance_epsilon) if final_norm else h
         if past_key_values is not None and attention_mask is not None and input_ids.shape[1] > 1:
             past_key_values.meta["q_lens_host"] = attention_mask.sum(dim=1).tolist()   # one sync per forward, not per layer
             if h.is_cuda and position_ids is not None:
@@ -149,6 +163,18 @@ class MSAModel(nn.Module):
         for layer in self.layers:
             h = layer(h, doc_ids, attention_mask, pe, past_key_values)
         return self.norm(h)
+
+
+    def _block_segments(self, h, attention_mask, position_ids, cache, doc_ids):
+        """The segments of a packed block where every layer is to encode one (int64 operands as the kernel takes them), or None."""
+        if cache is None or not h.is_cuda or h.shape[0] != 1 or h.shape[1] < 2 or not len(self.layers):
+            return None
+        if any(cache.cache_kwargs.get(layer.self_attn.layer_idx, {}).get("stage") != "prefill_stage1" for layer in self.layers):
+            return None
+        if any(not torch.is_tensor(t) or t.dtype != torch.int64 or t.shape != h.shape[:2] or t.device != h.device or not t.is_contiguous()
+               for t in (doc_ids, attention_mask, position_ids)):
+            return None
+        return ops.BlockSegments(doc_ids, attention_mask, position_ids)
 
 
 class MSAForCausalLM(nn.Module):
@@ -326,7 +352,12 @@ def encode_block(model: MSAForCausalLM, block_input, device) -> CustomDynamicCac
     cache = create_cache()
     for i in range(model.config.num_hidden_layers):
         cache.record_kwargs(i, {"stage": "prefill_stage1"})
+    parts = (block_input.doc_input_ids, block_input.doc_attention_mask, block_input.position_ids, block_input.doc_ids)
+    if torch.device(device).type == "cuda" and all(t.device.type == "cpu" and t.dtype == torch.int64 for t in parts):
+        # one copy that the host does not wait for (the inputs are for this stream's work alone)
+        parts = [flat.view(t.shape) for flat, t in zip(upload(device, [t.reshape(-1).numpy() for t in parts], wait=False), parts)]
+    else:
+        parts = [t.to(device) for t in parts]
     with torch.no_grad():
-        model.model(block_input.doc_input_ids.to(device), block_input.doc_attention_mask.to(device),
-                    block_input.position_ids.to(device), cache, block_input.doc_ids.to(device))
+        model.model(parts[0], parts[1], parts[2], cache, parts[3])
     return cache

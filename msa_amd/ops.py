@@ -76,17 +76,20 @@ class ChunkTable:
         return self.chunk_start.numel()
 
 
-def chunk_table(doc_lens: Sequence[int], P: int, first_token: int = 0, device="cuda") -> ChunkTable:
+def chunk_table(doc_lens: Sequence[int], P: int, first_token: int = 0, device="cuda", doc_start: Optional[torch.Tensor] = None) -> ChunkTable:
     """Builds the chunk table on the device from host-side document lengths (the host only sizes
-    the outputs: ``C = sum(ceil(len / P))``, as src/prefill.py:225 does)."""
+    the outputs: ``C = sum(ceil(len / P))``, as src/prefill.py:225 does).  ``doc_start``: the documents' first tokens and the end
+    (int32) where the device has them already; without it they are copied there, which waits for the device."""
     lib = _lib.load()
     lens = [int(x) for x in doc_lens]
     if not lens or min(lens) <= 0:
         raise ValueError("every document needs at least one token")
     n_chunks = sum((n + P - 1) // P for n in lens)
-    starts = torch.tensor([first_token] + lens, dtype=torch.int64).cumsum(0).to(torch.int32)
-    doc_start = starts.to(device)
     n_docs = len(lens)
+    if doc_start is None:
+        doc_start = torch.tensor([first_token] + lens, dtype=torch.int64).cumsum(0).to(torch.int32).to(device)
+    elif doc_start.dtype != torch.int32 or doc_start.numel() != n_docs + 1 or not doc_start.is_contiguous() or not doc_start.is_cuda:
+        raise ValueError(f"doc_start: {n_docs + 1} contiguous int32 values on the device")
     i32 = dict(dtype=torch.int32, device=device)
     t = ChunkTable(doc_start, torch.empty(n_docs + 1, **i32), torch.empty(n_chunks, **i32),
                    torch.empty(n_chunks, **i32), torch.empty(n_chunks, **i32),
@@ -94,6 +97,52 @@ def chunk_table(doc_lens: Sequence[int], P: int, first_token: int = 0, device="c
     check(lib.msa_chunk_table(ptr(t.doc_start), n_docs, P, n_chunks, ptr(t.doc_chunk_off), ptr(t.chunk_start),
                               ptr(t.chunk_len), ptr(t.chunk_doc), ptr(t.n_chunks), _stream()), "msa_chunk_table")
     return t
+
+
+class BlockSegments:
+    """The segments of one packed block ``[template | documents]`` for all layers of a forward pass: found on the device in one launch,
+    read by the host once (``read``), behind work that has been enqueued meanwhile."""
+    HOST = 4096                      # documents in the first copy
+
+    def __init__(self, ids: torch.Tensor, mask: Optional[torch.Tensor], pos: Optional[torch.Tensor]):
+        """``ids [1, T]``, ``mask`` and ``pos`` (of that shape, or None): contiguous int64 on the device."""
+        self.ids, self.mask, self.T = ids, mask, ids.numel()
+        _need_cuda(ids, mask, pos)
+        if any(t is not None and (t.dtype != torch.int64 or t.shape != ids.shape) for t in (ids, mask, pos)) or ids.shape != (1, self.T):
+            raise ValueError("block segments: ids, mask and positions must be int64 [1, T]")
+        self._words = torch.empty(8 + self.T + 2, dtype=torch.int32, device=ids.device)      # head, cu
+        self._start = torch.empty(self.T + 8, dtype=torch.int64, device=ids.device)
+        self._len = torch.empty(self.T + 1, dtype=torch.int32, device=ids.device)
+        check(_lib.load().msa_block_segments(ptr(ids), ptr(mask), ptr(pos), self.T, ptr(self._words), ptr(self._words[8:]), ptr(self._start),
+                                             ptr(self._len), _stream()), "msa_block_segments")
+        n = min(8 + self.T + 2, 8 + self.HOST)
+        self._host = torch.empty(n, dtype=torch.int32, pin_memory=True)
+        self._host.copy_(self._words[:n], non_blocking=True)
+        self._copied = torch.cuda.Event()
+        self._copied.record()
+        self._tables = {}
+        self.done = False
+
+    def read(self) -> "BlockSegments":
+        if self.done:
+            return self
+        self._copied.synchronize()
+        n_template, n_docs, bad, last, low, high = self._host[:6].tolist()
+        n = n_docs + (n_template > 0)
+        words = self._host[8:9 + n] if 9 + n <= self._host.numel() else self._words[8:9 + n].cpu()
+        cu = words.tolist()
+        self.n_template, self.bad, self.last_position, self.mask_sum = n_template, bool(bad), last, (low & 0xffffffff) | high << 32
+        self.lens = [b - a for a, b in zip(cu, cu[1:])]                    # of all segments
+        self.doc_lens = self.lens[n_template > 0:]
+        self.cu, self.start, self.len = self._words[8:9 + n], self._start[:n], self._len[:n]
+        self.done = True
+        return self
+
+    def table(self, P: int) -> ChunkTable:
+        if P not in self._tables:
+            self._tables[P] = chunk_table(self.doc_lens, P, first_token=self.n_template, device=self.ids.device,
+                                          doc_start=self.cu[self.n_template > 0:])
+        return self._tables[P]
 
 
 # ------------------------------------------------------------------------------ pooling
