@@ -281,6 +281,20 @@ typedef struct {
   int32_t reserved;
 } msa_rows_post;
 int msa_rows_linear_post(const msa_rows_args* args, int32_t epilogue, const msa_rows_post* post, void* stream);
+/* The head of such a decoder, MSA_ROWS_F32 with the last residual step and the norm behind it in front: the operand is
+ * rms_norm(x_in + rms_norm(y) * w) * next_w in bf16, both norms with `eps`.  x_out may hold the sum afterwards (scratch, not x_in). */
+int msa_rows_linear_final(const msa_rows_args* args, const msa_rows_post* post, const float* next_w, void* stream);
+/* The same with an embedding lookup in front: the operand's row m is row tokens[m] (from the end where it is negative) of `table` (bf16
+ * [vocab, K]; args->x is not read), x_out [M, K] gets it in fp32.  In a launch of its own through `h` (bf16 [M, K]) where the epilogue
+ * is neither PLAIN nor MAMBA or the product is too small or long.  One operand, groups = 1. */
+typedef struct {
+  const int64_t* tokens;
+  const void* table;
+  int64_t vocab;
+  float* x_out;
+  void* h;
+} msa_rows_embed;
+int msa_rows_linear_embed(const msa_rows_args* args, int32_t epilogue, const msa_rows_embed* embed, void* stream);
 
 #ifdef __cplusplus
 }

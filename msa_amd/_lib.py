@@ -126,6 +126,11 @@ class RowsPost(C.Structure):
     _fields_ = [("x_in", _vp), ("x_out", _vp), ("w", _vp), ("h", _vp), ("eps", _f32), ("reserved", _i32)]
 
 
+class RowsEmbed(C.Structure):
+    """``msa_rows_embed``."""
+    _fields_ = [("tokens", _vp), ("table", _vp), ("vocab", _i64), ("x_out", _vp), ("h", _vp)]
+
+
 class QKRopeArgs(C.Structure):
     """``msa_qk_rope_args``."""
     _fields_ = [("q", _vp), ("k", _vp), ("v", _vp), ("q_stride", _i64), ("k_stride", _i64), ("v_stride", _i64), ("q_norm", _vp),
@@ -190,6 +195,8 @@ SEQ_SIGNATURES = {
     "msa_seq_clamped_glu": (C.c_int, [_vp, _i64, _i32, _i32, _i32, _f32, _f32, _f32, _vp, _vp]),
     "msa_rows_linear": (C.c_int, [C.POINTER(RowsArgs), _i32, _vp]),
     "msa_rows_linear_post": (C.c_int, [C.POINTER(RowsArgs), _i32, C.POINTER(RowsPost), _vp]),
+    "msa_rows_linear_embed": (C.c_int, [C.POINTER(RowsArgs), _i32, C.POINTER(RowsEmbed), _vp]),
+    "msa_rows_linear_final": (C.c_int, [C.POINTER(RowsArgs), C.POINTER(RowsPost), _vp, _vp]),
 }
 # entry points of include/msa_amd.h that libmsa_seq.so holds too (the error text is per library)
 SEQ_SHARED = ("msa_last_error", "msa_abi_version", "msa_greedy_sample", "msa_embed_rows")

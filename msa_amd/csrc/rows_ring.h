@@ -47,8 +47,9 @@ static inline int64_t busy_weights(int64_t N, int64_t K) {
 }
 constexpr int kFar = 0x7ff00000;                   // past every extent, whatever is added: reads zeros, touches no memory
 // What happens to the activations in front of the products: nothing, an RMSNorm, or a residual step with the norm of its own (one
-// launch less, but all workgroups read its fp32 operands: seq_rows.hip has the line).
-enum { kPlain, kNormed, kPost };
+// launch less, but all workgroups read its fp32 operands: seq_rows.hip has the line), or that and the norm behind it (the head);
+// or they are rows of an embedding table, found by their tokens.
+enum { kPlain, kNormed, kPost, kFinal, kEmbed };
 constexpr int kMaxPost = 3;                        // units per wavefront that the residual step takes: what its registers hold
 constexpr int slots(int pro) { return pro ? 3 : 2; }              // of a wavefront's ring
 // Rows too long for the registers (nu = 0): the activations' unit lies behind the weights' in its slot, and there is room for one plane
@@ -56,10 +57,11 @@ constexpr int slots(int pro) { return pro ? 3 : 2; }              // of a wavefr
 constexpr int planes(int nu) { return nu == 0 ? 1 : 2; }
 constexpr int slab(int nu) { return nu == 0 ? 2 * kUnitSlab : kUnitSlab; }
 constexpr int lds_bytes(int pro, int nu) {
-  return planes(nu) * kWaves * kPlane * 4 + kWaves * slots(pro) * slab(nu) + (pro ? kWaves * 16 * 4 + kWaves * 1024 : 0);
+  return planes(nu) * kWaves * kPlane * 4 + kWaves * slots(pro) * slab(nu) + (pro == kFinal ? 2 : pro == kPlain || pro == kEmbed ? 0 : 1) * kWaves * 16 * 4;
 }
 static_assert(kMaxPost * 2 * kUnitBytes <= 1024 && kMaxResident * kUnitBytes <= 1024, "one request for a wavefront's part of the norm's weights");
-static_assert(lds_bytes(kNormed, 1) <= 160 * 1024 && lds_bytes(kPlain, 0) <= 160 * 1024);
+static_assert(kPlane * 4 >= 1024 && kPlane % 4 == 0, "which lies where the wavefront's first partial sums will");
+static_assert(lds_bytes(kNormed, 1) <= 160 * 1024 && lds_bytes(kPlain, 0) <= 160 * 1024 && lds_bytes(kFinal, 1) <= 160 * 1024);
 constexpr int kNonTemporal = 2;                    // a step reads a weight once
 
 // vmcnt(n), the other counters not waited for
@@ -81,7 +83,10 @@ __device__ __forceinline__ u32x4_t lds_read16(uint32_t at) {
 struct Args {
   const char *w, *x, *x_b, *norm_w;
   const float *post_x, *post_w;                    // kPost: the operand is post_x + rms_norm(x) * post_w, which one workgroup
-  float* post_out;                                 // leaves in post_out (rows of K)
+  float* post_out;                                 // leaves in post_out (rows of K); kFinal: rms_norm(that) * post_next
+  const float* post_next;
+  const int64_t* tokens;                           // kEmbed: the operand's row m is row tokens[m] of x (vocab rows of row_bytes); also left in post_out
+  int64_t vocab;
   int64_t xs, xbs;                                 // bytes between activation rows
   int32_t M, N, n_b, row_bytes;                    // weight rows from n_b on multiply x_b
   int32_t wgs_a, granule, qa, ra, qb, rb;  // workgroup i < wgs_a: its share of the granules of the rows before n_b
@@ -94,7 +99,7 @@ struct Args {
 // for what it requests: loads return in order, so that would wait for the weights in front of it.
 template <class Epi, int NU, int kPro>
 __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename Epi::Args s) {
-  constexpr bool kResident = NU > 0, kNorm = kPro == kNormed;
+  constexpr bool kResident = NU > 0, kNorm = kPro == kNormed, kPosts = kPro == kPost || kPro == kFinal;
   constexpr int kSlots = slots(kPro), kPlanes = planes(NU), kSlab = slab(NU);
   extern __shared__ __align__(16) char lds[];
   float(*part)[kWaves][kPlane] = reinterpret_cast<float(*)[kWaves][kPlane]>(lds);
@@ -118,7 +123,7 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
   const int off0 = l_row * row_bytes + col, off1 = off0 + 8 * row_bytes;
   const int64_t xs = second ? a.xbs : a.xs;
   const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(second ? a.x_b : a.x), 0,
-                                                                        (int)((a.M - 1) * xs + row_bytes), 0x00020000);
+                                                                        (int)(kPro == kEmbed ? a.vocab * row_bytes : (a.M - 1) * xs + row_bytes), 0x00020000);
   const int xoff0 = l_row * (int)xs + col, xoff1 = xoff0 + 8 * (int)xs;      // of the activations, likewise
   int req_item = 0, slot_in = 0;
   __amdgpu_buffer_rsrc_t rs;
@@ -148,11 +153,12 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
     slot_in = slot_in + 1 == kSlots ? 0 : slot_in + 1;
   };
   const int x_col = wave * kUnitBytes + g * 16;
+  const int x_row = kPro == kEmbed ? (int)embed_row(a.tokens[min(n_l, a.M - 1)], a.vocab, true) * row_bytes : n_l * (int)xs;
   auto load_x = [&](u32x4_t (&x)[2], int u) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int so = u * (kUnitBytes * kWaves) + h * 64;
-      x[h] = __builtin_amdgcn_raw_buffer_load_b128(rs_x, x_col + so < row_bytes ? n_l * (int)xs + x_col : kFar, so, 0);
+      x[h] = __builtin_amdgcn_raw_buffer_load_b128(rs_x, x_col + so < row_bytes ? x_row + x_col : kFar, so, 0);
     }
   };
   const int rd0 = n_l * kUnitBytes + ((g ^ (n_l & 7)) * 16), rd1 = n_l * kUnitBytes + (((g + 4) ^ (n_l & 7)) * 16);
@@ -181,18 +187,22 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
     for (int u = 0; u < NU; ++u) load_x(xf[u], u);
   }
   // The norm's weights, alike for all rows, through LDS (in registers, five units of them spill: 2560 x 5120 with one row took 13.9
-  // us instead of 8.8)
-  char* norm_lds = lds + lds_bytes(kPro, NU) - (kWaves - wave) * 1024;
+  // us instead of 8.8): where the wavefront's own partial sums will lie, which it writes behind its reads
+  char *norm_lds = reinterpret_cast<char*>(part[0][wave]), *next_lds = reinterpret_cast<char*>(part[kPlanes - 1][wave]);
   if constexpr (kNorm) {
     const __amdgpu_buffer_rsrc_t rs_g = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.norm_w), 0, row_bytes, 0x00020000);
     MSA_LOAD_TO_LDS(rs_g, norm_lds, (lane >> 3) * (kUnitBytes * kWaves) + wave * kUnitBytes + (lane & 7) * 16, 0, 0);
   }
   // The residual step's other operands: the fp32 rows into registers, the weights likewise
-  u32x4_t px[kPro == kPost ? NU : 1][2][2];
-  if constexpr (kPro == kPost) {
+  u32x4_t px[kPosts ? NU : 1][2][2];
+  if constexpr (kPosts) {
     const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.post_w), 0, 2 * row_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rs_p = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.post_x), 0, a.M * 2 * row_bytes, 0x00020000);
     MSA_LOAD_TO_LDS(rs_w, norm_lds, (lane >> 4) * (2 * kUnitBytes * kWaves) + wave * 2 * kUnitBytes + (lane & 15) * 16, 0, 0);
+    if constexpr (kPro == kFinal) {
+      const __amdgpu_buffer_rsrc_t rs_n = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.post_next), 0, 2 * row_bytes, 0x00020000);
+      MSA_LOAD_TO_LDS(rs_n, next_lds, (lane >> 4) * (2 * kUnitBytes * kWaves) + wave * 2 * kUnitBytes + (lane & 15) * 16, 0, 0);
+    }
 #pragma unroll
     for (int u = 0; u < NU; ++u)
 #pragma unroll
@@ -202,7 +212,7 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
         for (int i = 0; i < 2; ++i) px[u][h][i] = __builtin_amdgcn_raw_buffer_load_b128(rs_p, at + 16 * i, 2 * so, 0);
       }
   }
-  constexpr bool kLate = kPro == kPost && NU == kMaxPost;    // (no registers for it in front of the residual step)
+  constexpr bool kLate = kPosts && NU == kMaxPost;    // (no registers for it in front of the residual step)
   if (!kLate) epi.load(s, m, r0 + nr, quarter == 0 && m < a.M && r0 + nr < r1, second, 0);
   asm volatile("" ::: "memory");                             // (not to be sunk behind the requests)
   point();
@@ -239,7 +249,20 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
     ssq = lanes_sum(ssq);
     if (g == 0) row_ssq[wave * 16 + n_l] = ssq;              // read behind the first barrier
   }
-  if constexpr (kPro == kPost) {
+  if constexpr (kPro == kEmbed) {                            // (each row by one workgroup)
+    const bool writes = n_l < a.M && n_l % gridDim.x == wg;
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int at = x_col + u * (kUnitBytes * kWaves) + h * 64;
+        if (!writes || at >= row_bytes) continue;
+        float4* to = reinterpret_cast<float4*>(a.post_out + (int64_t)n_l * (row_bytes / 2) + at / 2);
+        to[0] = make_float4(bf16lo(xf[u][h][0]), bf16hi(xf[u][h][0]), bf16lo(xf[u][h][1]), bf16hi(xf[u][h][1]));
+        to[1] = make_float4(bf16lo(xf[u][h][2]), bf16hi(xf[u][h][2]), bf16lo(xf[u][h][3]), bf16hi(xf[u][h][3]));
+      }
+  }
+  if constexpr (kPosts) {
     // x + rms_norm(y) * w as the operand, the sums as in the launch of its own
     float ssq = 0.f;
 #pragma unroll
@@ -253,18 +276,23 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
         }
     ssq = lanes_sum(ssq);
     const uint32_t row_at = lds_offset(row_ssq + n_l * 16);
-    asm volatile("ds_write_b32 %0, %1\n\ts_waitcnt vmcnt(%2) lgkmcnt(0)\n\ts_barrier" ::"v"(row_at + 4 * wave), "v"(ssq), "n"(2 * kSlots) : "memory");
-    u32x4_t p[4];
-    if constexpr (NU < kMaxPost)
-      asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:16\n\tds_read_b128 %2, %4 offset:32\n\tds_read_b128 %3, %4 offset:48\n\t"
-                   "s_waitcnt lgkmcnt(0)" : "=&v"(p[0]), "=&v"(p[1]), "=&v"(p[2]), "=&v"(p[3]) : "v"(row_at) : "memory");
-    float total = 0.f;
+    auto row_total = [&](uint32_t row_at) {
+      u32x4_t p[4];
+      if constexpr (NU < kMaxPost)
+        asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:16\n\tds_read_b128 %2, %4 offset:32\n\tds_read_b128 %3, %4 offset:48\n\t"
+                     "s_waitcnt lgkmcnt(0)" : "=&v"(p[0]), "=&v"(p[1]), "=&v"(p[2]), "=&v"(p[3]) : "v"(row_at) : "memory");
+      float total = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if constexpr (NU == kMaxPost) p[i] = lds_read16(row_at + 16 * i);                    // (no registers for all of them)
-      total += (__uint_as_float(p[i][0]) + __uint_as_float(p[i][1])) + (__uint_as_float(p[i][2]) + __uint_as_float(p[i][3]));
-    }
-    const float post_inv = 1.0f / sqrtf(total / (float)(row_bytes / 2) + a.eps);
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (NU == kMaxPost) p[i] = lds_read16(row_at + 16 * i);                  // (no registers for all of them)
+        total += (__uint_as_float(p[i][0]) + __uint_as_float(p[i][1])) + (__uint_as_float(p[i][2]) + __uint_as_float(p[i][3]));
+      }
+      return 1.0f / sqrtf(total / (float)(row_bytes / 2) + a.eps);
+    };
+    if constexpr (kPro == kFinal) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kSlots) : "memory");      // (the second weights' wait as well)
+    asm volatile("ds_write_b32 %0, %1\n\ts_waitcnt vmcnt(%2) lgkmcnt(0)\n\ts_barrier" ::"v"(row_at + 4 * wave), "v"(ssq), "n"(2 * kSlots) : "memory");
+    const float post_inv = row_total(row_at);
+    float next_ssq = 0.f;
 #pragma unroll
     for (int u = 0; u < NU; ++u)
 #pragma unroll
@@ -284,6 +312,14 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
             v[4 * i + c] = __uint_as_float(px[u][h][i][c]) + (c & 1 ? bf16hi(y) : bf16lo(y)) * post_inv * __uint_as_float(w[i][c]);
           }
         }
+        if constexpr (kPro == kFinal) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            next_ssq += v[e] * v[e];
+            px[u][h][e >> 2][e & 3] = __float_as_uint(v[e]);
+          }
+          continue;
+        }
         if (wg == 0 && n_l < a.M && x_col + so < row_bytes) {
           float4* to = reinterpret_cast<float4*>(a.post_out + (int64_t)n_l * (row_bytes / 2) + (x_col + so) / 2);
           to[0] = make_float4(v[0], v[1], v[2], v[3]);
@@ -292,6 +328,25 @@ __global__ __launch_bounds__(kWaves * 64) void rows_ring_kernel(Args a, typename
 #pragma unroll
         for (int c = 0; c < 4; ++c) xf[u][h][c] = pack_bf16x2(v[2 * c], v[2 * c + 1]);
       }
+    if constexpr (kPro == kFinal) {
+      next_ssq = lanes_sum(next_ssq);
+      const uint32_t next_at = row_at + kWaves * 16 * 4;
+      asm volatile("ds_write_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::"v"(next_at + 4 * wave), "v"(next_ssq) : "memory");
+      const float next_inv = row_total(next_at);
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const u32x4_t w = lds_read16(lds_offset(next_lds) + u * 2 * kUnitBytes + h * 128 + g * 32 + 16 * i);
+            float v[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = __uint_as_float(px[u][h][i][c]) * next_inv * __uint_as_float(w[c]);
+            xf[u][h][2 * i] = pack_bf16x2(v[0], v[1]);
+            xf[u][h][2 * i + 1] = pack_bf16x2(v[2], v[3]);
+          }
+    }
   }
 
   float inv = 1.f;
@@ -383,12 +438,12 @@ int launch(Args a, const typename Epi::Args& s, int granule, hipStream_t st) {
   if (units <= 1) return start<Epi, 1, kPro>(a, s, wgs, st);
   if (units <= 2) return start<Epi, 2, kPro>(a, s, wgs, st);
   if (units <= 3) return start<Epi, 3, kPro>(a, s, wgs, st);
-  if constexpr (kPro != kPost) {
+  if constexpr (kPro != kPost && kPro != kFinal) {
     if (units <= 4) return start<Epi, 4, kPro>(a, s, wgs, st);
     if (units <= kMaxResident) return start<Epi, kMaxResident, kPro>(a, s, wgs, st);
   }
   if constexpr (kPro != kPlain) {
-    msa_set_error("rows_ring: a folded norm takes rows of at most %d bytes, not %d", (kPro == kPost ? kMaxPost : kMaxResident) * kUnitBytes * kWaves, a.row_bytes);
+    msa_set_error("rows_ring: a folded norm takes rows of at most %d bytes, not %d", (kPro == kNormed || kPro == kEmbed ? kMaxResident : kMaxPost) * kUnitBytes * kWaves, a.row_bytes);
     return MSA_EINVAL;
   } else {
     return start<Epi, 0, kPlain>(a, s, wgs, st);

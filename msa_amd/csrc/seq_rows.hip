@@ -305,8 +305,15 @@ bool takes_ring(const msa_rows_args& a, int32_t epilogue) {
 }
 
 template <int EPI, int kPro = rows_ring::kPlain>
-int launch_ring(const msa_rows_args& a, hipStream_t st, const msa_rows_post* post = nullptr) {
+int launch_ring(const msa_rows_args& a, hipStream_t st, const msa_rows_post* post = nullptr, const float* next_w = nullptr,
+                const msa_rows_embed* embed = nullptr) {
   rows_ring::Args r{};
+  r.post_next = next_w;
+  if (embed) {
+    r.tokens = embed->tokens;
+    r.vocab = embed->vocab;
+    r.post_out = embed->x_out;
+  }
   if (post) {
     r.post_x = post->x_in;
     r.post_w = post->w;
@@ -336,7 +343,8 @@ int launch_rows(const msa_rows_args& a, int waves, int rows_per_wg, hipStream_t 
 }  // namespace
 
 namespace {
-int rows_entry(const msa_rows_args& a, int32_t epilogue, const msa_rows_post* post, void* stream) {
+int rows_entry(const msa_rows_args& a, int32_t epilogue, const msa_rows_post* post, void* stream, const float* next_w = nullptr,
+               const msa_rows_embed* embed = nullptr) {
   MSA_REQUIRE(a.x && a.w && a.M > 0 && a.M <= 16 && a.N > 0 && a.K > 0 && a.K % 8 == 0 && a.groups > 0 && a.groups <= 65535,
               "msa_rows_linear: M=%d (1..16) N=%d K=%d (a multiple of 8) groups=%d", a.M, a.N, a.K, a.groups);
   MSA_REQUIRE(a.x_stride >= (int64_t)a.K * a.groups && a.x_stride % 8 == 0 && a.x_stride * 32 < ((int64_t)1 << 30) &&
@@ -389,6 +397,9 @@ int rows_entry(const msa_rows_args& a, int32_t epilogue, const msa_rows_post* po
     if (units % cand == 0) { waves = cand; break; }
   hipStream_t st = as_stream(stream);
   if (takes_ring(a, epilogue)) {
+    if (embed && epilogue == MSA_ROWS_MAMBA) return launch_ring<MSA_ROWS_MAMBA, rows_ring::kEmbed>(a, st, nullptr, nullptr, embed);
+    if (embed) return launch_ring<MSA_ROWS_PLAIN, rows_ring::kEmbed>(a, st, nullptr, nullptr, embed);
+    if (post && next_w) return launch_ring<MSA_ROWS_F32, rows_ring::kFinal>(a, st, post, next_w);
     if (post) {
       switch (epilogue) {
         case MSA_ROWS_PLAIN: return launch_ring<MSA_ROWS_PLAIN, rows_ring::kPost>(a, st, post);
@@ -440,14 +451,50 @@ bool worth_folding(const msa_rows_args& a) {
   const int64_t elements = a.M * (int64_t)a.K;
   return a.K <= kPostRow ? elements <= kMaxPostElements : elements <= kMaxLongPostElements && (int64_t)a.N * a.K >= kMinLongPostWeights;
 }
+// What the residual step asks of its operands to be formed on the way.
+static bool post_fits(const msa_rows_args& a, const msa_rows_post* post) {
+  return a.K % 8 == 0 && a.K <= rows_ring::kMaxPost * rows_ring::kWaves * rows_ring::kUnitBytes / 2 &&
+         (((uintptr_t)post->x_in | (uintptr_t)post->x_out | (uintptr_t)post->w) & 15) == 0;
+}
+// Likewise in front of the head, in the same limits (steps of one, 4 and 8 rows of 1024: 180.3, 185.9 and 196.6 us separate, 179.2, 184.9
+// and 195.3 folded: of the launch's 5 us a second reduction, behind the first and while the whole ring waits, costs most).
+extern "C" int msa_rows_linear_final(const msa_rows_args* args, const msa_rows_post* post, const float* next_w, void* stream) {
+  MSA_REQUIRE(args && post && next_w && post->x_in && post->w && post->h && post->eps >= 0.f, "msa_rows_linear_final: null arguments");
+  msa_rows_args a = *args;
+  MSA_REQUIRE(a.x && a.M > 0 && a.M <= 16 && a.K > 0 && a.groups == 1 && a.x_stride >= a.K && a.n_b >= a.N,
+              "msa_rows_linear_final: M=%d (1..16) K=%d groups=%d n_b=%d", a.M, a.K, a.groups, a.n_b);
+  if (takes_ring(a, MSA_ROWS_F32) && worth_folding(a) && post_fits(a, post) && ((uintptr_t)next_w & 15) == 0) return rows_entry(a, MSA_ROWS_F32, post, stream, next_w);
+  MSA_REQUIRE(post->x_out, "msa_rows_linear_final: the separate launch needs x_out");
+  if (const int rc = msa_seq_rms_residual(post->x_in, a.x, a.x_stride, post->w, post->eps, post->x_out, next_w, post->h, MSA_BF16, a.M, a.K, stream); rc != MSA_OK) return rc;
+  a.x = post->h;
+  a.x_stride = a.K;
+  return rows_entry(a, MSA_ROWS_F32, nullptr, stream);
+}
+// The lookup is folded wherever the ring's registers hold the rows and 32-bit offsets reach the table: every workgroup reads the same bytes
+// as without, one latency (the tokens') later.  Whole decode steps of four layers, us, with the launch of its own and without: one row of
+// 1024 179.7 and 176.2, 4 rows 185.1 and 180.9, one of 2560 384.3 and 380.8, 16 of them 485.7 and 481.4.
+extern "C" int msa_rows_linear_embed(const msa_rows_args* args, int32_t epilogue, const msa_rows_embed* embed, void* stream) {
+  MSA_REQUIRE(args && embed && embed->tokens && embed->table && embed->x_out && embed->h, "msa_rows_linear_embed: null arguments");
+  msa_rows_args a = *args;
+  MSA_REQUIRE(a.M > 0 && a.M <= 16 && a.K > 0 && a.K % 8 == 0 && a.groups == 1 && a.n_b >= a.N && embed->vocab > 0 &&
+                  (((uintptr_t)embed->table | (uintptr_t)embed->x_out | (uintptr_t)embed->h) & 15) == 0,
+              "msa_rows_linear_embed: M=%d (1..16) K=%d groups=%d n_b=%d, 16-byte alignment", a.M, a.K, a.groups, a.n_b);
+  a.x = embed->table;
+  a.x_stride = a.K;
+  if ((epilogue == MSA_ROWS_PLAIN || epilogue == MSA_ROWS_MAMBA) && takes_ring(a, epilogue) && a.K <= rows_ring::kMaxResidentK &&
+      embed->vocab <= rows_ring::kFar / (a.K * 2))
+    return rows_entry(a, epilogue, nullptr, stream, nullptr, embed);
+  if (const int rc = msa_embed_rows(embed->tokens, a.M, embed->table, embed->vocab, 1, a.K, MSA_BF16, embed->h, embed->x_out, stream); rc != MSA_OK) return rc;
+  a.x = embed->h;
+  return rows_entry(a, epilogue, nullptr, stream);
+}
 extern "C" int msa_rows_linear_post(const msa_rows_args* args, int32_t epilogue, const msa_rows_post* post, void* stream) {
   MSA_REQUIRE(args && post && post->x_in && post->x_out && post->w && post->h && post->eps >= 0.f, "msa_rows_linear_post: null arguments");
   msa_rows_args a = *args;
   MSA_REQUIRE(a.x && a.M > 0 && a.M <= 16 && a.K > 0 && a.groups == 1 && a.x_stride >= a.K && a.n_b >= a.N,
               "msa_rows_linear_post: M=%d (1..16) K=%d groups=%d n_b=%d", a.M, a.K, a.groups, a.n_b);
-  const bool folds = (epilogue == MSA_ROWS_PLAIN || epilogue == MSA_ROWS_MAMBA || epilogue == MSA_ROWS_GLU) && takes_ring(a, epilogue) && worth_folding(a) && a.K % 8 == 0 &&
-                     a.K <= rows_ring::kMaxPost * rows_ring::kWaves * rows_ring::kUnitBytes / 2 && post->x_in != post->x_out &&
-                     (((uintptr_t)post->x_in | (uintptr_t)post->x_out | (uintptr_t)post->w) & 15) == 0;
+  const bool folds = (epilogue == MSA_ROWS_PLAIN || epilogue == MSA_ROWS_MAMBA || epilogue == MSA_ROWS_GLU) && takes_ring(a, epilogue) && worth_folding(a) && post_fits(a, post) &&
+                     post->x_in != post->x_out;
   if (folds) return rows_entry(a, epilogue, post, stream);
   if (const int rc = msa_seq_rms_residual(post->x_in, a.x, a.x_stride, post->w, post->eps, post->x_out, nullptr, post->h, MSA_BF16, a.M, a.K, stream); rc != MSA_OK) return rc;
   a.x = post->h;

@@ -3,7 +3,8 @@ clamped gated feed-forwards: the Sugizen architecture.
 
 The residual stream is fp32 and is itself (in the activations' type) what every sublayer reads.  Behind an output projection
 stands one fused step, residual + norm + the next operand (``seq_ops.rms_residual``).  The decode form folds it into the product
-that reads it (``seq_ops.PostRows``), the convolution into the mixer's input projection and the gated unit into the feed-forward's.
+that reads it (``seq_ops.PostRows``, ``seq_ops.FinalRows`` the last one and the final norm), the embedding lookup into the first one
+(``seq_ops.EmbedRows``), the convolution into the mixer's input projection and the gated unit into the feed-forward's.
 """
 from __future__ import annotations
 
@@ -63,7 +64,11 @@ class PostNormForCausalLM(StepDecoder):
         glu = lambda l, h: seq_ops.rows_glu(h, l.w_gate_up, l.mlp.limit)
         if trace is not None or not self.layers:
             return self._layers(tokens, trace, decode, seq_ops.rows_linear, glu)
-        x, h = self._start(tokens)
+        if self.embed.dtype == self.dtype != F32 and tokens.dim() == 1 and ops.embed_ok(self.embed, tokens):
+            h = seq_ops.EmbedRows(self.embed, tokens)        # (the first layer's product looks the rows up)
+            x = h.out
+        else:
+            x, h = self._start(tokens)
         y = w = None
         for r, layer in enumerate(self.layers):
             parts = [(lambda h: decode(r, layer, h), layer.w_o, layer.norm1)]
@@ -74,4 +79,4 @@ class PostNormForCausalLM(StepDecoder):
                     h = seq_ops.PostRows(x, y, w, self.config.norm_eps)
                     x = h.out
                 y, w = seq_ops.rows_linear(part(h), w_out), norm
-        return self._residual(x, y, w, True)[1]
+        return seq_ops.FinalRows(x, y, w, self.config.norm_eps, self.final_norm)

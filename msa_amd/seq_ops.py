@@ -545,10 +545,40 @@ class PostRows:
         self.c = _lib.RowsPost(ptr(x), ptr(self.out), ptr(w), ptr(self.keep[1]), eps, 0)
 
 
+class EmbedRows:
+    """The operand ``table[tokens]`` (bf16) for up to 16 tokens, which the product that takes it looks up itself; the rows in fp32 are
+    then in ``out``.  ``ops.embed_ok(table, tokens)`` has to hold."""
+
+    def __init__(self, table, tokens):
+        _dense(table, tokens)
+        if table.dtype != torch.bfloat16 or tokens.dtype != torch.int64 or tokens.dim() != 1:
+            raise ValueError("EmbedRows: bf16 table and int64 tokens [M]")
+        self.shape, self.device = (tokens.shape[0], table.shape[1]), table.device
+        self.table = table.detach()
+        self.out, h = torch.empty(self.shape, dtype=torch.float32, device=table.device), torch.empty(self.shape, dtype=table.dtype, device=table.device)
+        self.keep = (tokens, h)
+        self.c = _lib.RowsEmbed(ptr(tokens), ptr(table), table.shape[0], ptr(self.out), ptr(h))
+
+
+class FinalRows:
+    """The operand ``rms_norm(x + rms_norm(y) * w) * next_w`` of :func:`rms_residual` for up to 16 rows, which the head that takes it
+    (:func:`rows_linear_f32`) forms on the way where they are few."""
+
+    def __init__(self, x, y, w, eps: float, next_w):
+        _f32(x.shape[1], next_w)
+        self.post, self.next_w, self.args = PostRows(x, y, w, eps), next_w, (x, y, w, eps)
+        self.shape, self.device = y.shape, y.device
+
+    def rows(self) -> torch.Tensor:
+        """The operand itself."""
+        x, y, w, eps = self.args
+        return rms_residual(x, torch.bfloat16, y, w, eps, self.next_w)[1]
+
+
 def _rows_args(x, w, groups: int = 1, x_b=None, n_b: Optional[int] = None) -> _lib.RowsArgs:
-    post = x if isinstance(x, PostRows) else None
-    x = x if post is None else post.y
-    M = x.shape[0]
+    post = x if isinstance(x, (PostRows, EmbedRows)) else None
+    x = x if post is None else post.y if isinstance(post, PostRows) else post.table
+    M = x.shape[0] if post is None else post.shape[0]
     K = w.shape[1]
     N = w.shape[0] // groups
     _dense(w)
@@ -566,6 +596,9 @@ def _rows_args(x, w, groups: int = 1, x_b=None, n_b: Optional[int] = None) -> _l
 
 
 def _run_rows(a: _lib.RowsArgs, epilogue: int) -> None:
+    if isinstance(a.post, EmbedRows):
+        _check(_lib.load_seq().msa_rows_linear_embed(C.byref(a), epilogue, C.byref(a.post.c), _stream()), "msa_rows_linear_embed")
+        return
     if a.post is not None:
         _check(_lib.load_seq().msa_rows_linear_post(C.byref(a), epilogue, C.byref(a.post.c), _stream()), "msa_rows_linear_post")
         return
@@ -584,11 +617,15 @@ def rows_linear(x, w, groups: int = 1, x_b=None, n_b: Optional[int] = None, gelu
 
 def rows_linear_f32(x, w, cap: float = 0.0, add: Optional[torch.Tensor] = None) -> torch.Tensor:
     """fp32 products of up to 16 rows, softcapped, plus ``add [N]``."""
-    a = _rows_args(x, w)
+    final = x if isinstance(x, FinalRows) else None
+    a = _rows_args(x if final is None else final.post, w)
     out = torch.empty((x.shape[0], w.shape[0]), dtype=torch.float32, device=x.device)
     if add is not None:
         _f32(w.shape[0], add)
     a.out, a.out_stride, a.cap, a.add = ptr(out), out.shape[1], cap, ptr(add)
+    if final is not None:
+        _check(_lib.load_seq().msa_rows_linear_final(C.byref(a), C.byref(a.post.c), ptr(final.next_w), _stream()), "msa_rows_linear_final")
+        return out
     _run_rows(a, _lib.ROWS_F32)
     return out
 

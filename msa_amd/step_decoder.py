@@ -151,6 +151,7 @@ class StepDecoder:
         if not rows:
             return None
         if rows != list(range(batch.rows)):
+            h = h.rows() if isinstance(h, seq_ops.FinalRows) else h
             h = h[rows[0]:rows[0] + 1] if len(rows) == 1 else h[torch.tensor(rows, device=h.device) if index is None else index]
         cap = getattr(self.config, "logit_softcap", None) or 0.0
         if self.fused_decode and len(rows) <= seq_ops.MAX_ROWS:
