@@ -235,6 +235,16 @@ def load_seq() -> C.CDLL:
     return _libs.get(SEQ_LIB_PATH) or _open(SEQ_LIB_PATH, {**SEQ_SIGNATURES, **{n: SIGNATURES[n] for n in SEQ_SHARED}})
 
 
+def load_host():
+    """The extension module of the host's side (``csrc/host.cpp``), behind the library of the layers it launches."""
+    load_seq()
+    try:
+        from . import _host
+    except ImportError as e:
+        raise ImportError(f"{HERE}/_host.so: build it with `python -m msa_amd.build` ({e})") from e
+    return _host
+
+
 def check(code: int, where: str, lib: Optional[C.CDLL] = None) -> None:
     if code != 0:
         raise MsaError(code, where, (lib or load()).msa_last_error().decode("utf-8", "replace"))
@@ -245,10 +255,14 @@ def ptr(t) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+_dtype_codes = {}
+
+
 def dtype_code(torch_dtype) -> int:
-    import torch
-    if torch_dtype == torch.bfloat16:
-        return MSA_BF16
-    if torch_dtype == torch.float32:
-        return MSA_F32
+    if not _dtype_codes:
+        import torch
+        _dtype_codes.update({torch.bfloat16: MSA_BF16, torch.float32: MSA_F32})
+    code = _dtype_codes.get(torch_dtype)
+    if code is not None:
+        return code
     raise TypeError(f"unsupported dtype {torch_dtype}: the kernels take bfloat16 or float32")

@@ -1,7 +1,7 @@
 """Builds the C-ABI libraries from ``csrc/*.hip`` for gfx950 with hipcc: ``libmsa_amd.so`` (routing / sparse attention)
-and ``libmsa_seq.so`` (the layers of the decoders of mixed layers).
+and ``libmsa_seq.so`` (the layers of the decoders of mixed layers), and the extension module ``_host.so`` (``csrc/host.cpp``).
 
-``python -m msa_amd.build`` compiles both in-tree; the libraries then travel with the source tree.
+``python -m msa_amd.build`` compiles all in-tree; the libraries then travel with the source tree.
 """
 from __future__ import annotations
 
@@ -16,6 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmsa_amd.so")
 SEQ_LIB = os.path.join(HERE, "libmsa_seq.so")
+HOST_LIB = os.path.join(HERE, "_host.so")    # the extension module of csrc/host.cpp
 SHARED = ("status.hip", "glue.hip")          # linked into both libraries
 ARCH = "gfx950"
 # packed fp32 VALU ops are switched off for all device code of this library
@@ -183,6 +184,23 @@ def _link(objs, lib: str) -> str:
     return lib
 
 
+def build_host() -> str:
+    """Compiles the extension module of the host's side (C++ against PyTorch's headers, no device code)."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    torch_lib = os.path.join(os.path.dirname(cpp_extension.__file__), "..", "lib")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    include = [sysconfig.get_paths()["include"], *cpp_extension.include_paths(), os.path.join(rocm, "include")]
+    tmp = HOST_LIB + ".tmp"
+    r = subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", *("-I" + i for i in include),
+                        os.path.join(CSRC, "host.cpp"), "-o", tmp, "-L" + torch_lib, "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10",
+                        "-L" + os.path.join(rocm, "lib"), "-lamdhip64", "-ldl"], capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for host.cpp:\n{r.stderr}")
+    os.replace(tmp, HOST_LIB)
+    return HOST_LIB
+
+
 def build_seq(jobs: int = 8) -> str:
     """Compiles and links ``libmsa_seq.so`` alone."""
     with ThreadPoolExecutor(max_workers=jobs) as ex:
@@ -190,12 +208,14 @@ def build_seq(jobs: int = 8) -> str:
 
 
 def ensure_seq() -> str:
-    """``libmsa_seq.so``, compiled if it is missing (a fresh checkout); concurrent callers wait for the first."""
-    if not os.path.exists(SEQ_LIB):
+    """``libmsa_seq.so`` and the extension module, compiled if they are missing (a fresh checkout); concurrent callers wait for the first."""
+    if not (os.path.exists(SEQ_LIB) and os.path.exists(HOST_LIB)):
         with open(SEQ_LIB + ".lock", "w") as lock:
             fcntl.flock(lock, fcntl.LOCK_EX)
             if not os.path.exists(SEQ_LIB):
                 build_seq()
+            if not os.path.exists(HOST_LIB):
+                build_host()
     return SEQ_LIB
 
 
@@ -208,7 +228,7 @@ def build(jobs: int = 8) -> str:
             raise RuntimeError(f"csrc/{inc} is not what csrc/{gen} generates: run the generator")
     checked = [s for s in srcs if os.path.basename(s) in {**CONTRACTS, **LDS_WAITS}]
     with ThreadPoolExecutor(max_workers=min(jobs, len(srcs) + len(checked))) as ex:
-        checks = [ex.submit(_check_contracts, s) for s in checked]
+        checks = [ex.submit(_check_contracts, s) for s in checked] + [ex.submit(build_host)]
         objs = dict(zip(srcs, ex.map(_compile, srcs)))
         for c in checks:
             c.result()

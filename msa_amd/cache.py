@@ -9,6 +9,8 @@ from typing import Dict, Hashable, List, Optional, Sequence, Tuple
 
 import torch
 
+from . import ops
+
 
 class CustomDynamicCache:
     def __init__(self):
@@ -159,9 +161,11 @@ class SequenceStateCache:
             self._resize(2 * self.slots, self.capacity)
         slot = self._free.pop(0)
         # in one launch: a model's six to thirty states took 4 us each, several times what clearing them costs
-        fixed = [held[name][slot] for spec, held in zip(self.specs, self.tensors) for name, s in spec.items() if not s.per_token]
-        if fixed:
-            torch._foreach_zero_(fixed)
+        fixed = [held[name] for spec, held in zip(self.specs, self.tensors) for name, s in spec.items() if not s.per_token]
+        if fixed and all(t.is_cuda for t in fixed):
+            ops.host().clear(fixed, slot)
+        elif fixed:
+            torch._foreach_zero_([t[slot] for t in fixed])
         self.slot_of[key], self.length[key] = slot, 0
         return slot
 

@@ -1,0 +1,368 @@
+// The host's side of the calls a prompt makes most: operands checked, results allocated and the kernel launched without Python in
+// between.  A prompt of few tokens waits for the host, not for the kernels (122 tokens of four layers of 1024: 350 us of kernels, 610 to 650
+// us in all through the interpreter, 385 to 430 so), and a call through the interpreter costs 9 to 14 us, of which the launch is 3 (us a
+// call, in Python and here: a product 9.7 and 5.2, a residual step with norm and shift 14.3 and 6.4, an RMS residual 8.9 and 4.4, a
+// convolution 8.7 and 4.4, an opened sequence 23 and 13).
+//
+// Every function takes the operands as they come and answers None for whatever it does not take, without having launched anything: the
+// caller's own path in Python then decides, with the checks and errors it has.  A code other than MSA_OK of the library is handed back.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/GradMode.h>
+#include <c10/hip/HIPStream.h>
+#include <dlfcn.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
+
+#include "../../include/msa_amd.h"
+#include "../../include/msa_seq.h"
+
+namespace {
+
+decltype(&msa_block_linear) block_linear;
+decltype(&msa_block_linear_us) block_linear_us;
+decltype(&msa_seq_residual_norm) residual_norm_;
+decltype(&msa_seq_rms_residual) rms_residual_;
+decltype(&msa_seq_conv_silu) conv_silu_;
+decltype(&msa_seq_group_rmsnorm) group_rmsnorm_;
+decltype(&msa_seq_ssd_scan) ssd_scan;
+decltype(&msa_seq_ssd_chunked) ssd_chunked;
+decltype(&msa_seq_ssd_chunked_workspace_bytes) ssd_bytes;
+decltype(&msa_seq_delta_scan) delta_scan;
+decltype(&msa_seq_delta_chunked) delta_chunked;
+decltype(&msa_seq_delta_chunked_workspace_bytes) delta_bytes;
+
+// Lines of the products' dispatch, as the caller has them.
+struct Lines {
+  long long block_rows, block_depth, captured_rows, captured_depth;
+  double block_us, captured_us;
+} lines;
+
+bool is_none(PyObject* o) { return o == nullptr || o == Py_None; }
+const at::Tensor* tensor(PyObject* o) { return !is_none(o) && THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+void* at_(const at::Tensor* t) { return t ? t->data_ptr() : nullptr; }
+void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
+int dtype_of(const at::Tensor& t) { return t.scalar_type() == at::kBFloat16 ? MSA_BF16 : t.scalar_type() == at::kFloat ? MSA_F32 : -1; }
+bool dense(const at::Tensor* t) { return t && t->is_cuda() && t->is_contiguous(); }
+bool plain(const at::Tensor* t) { return !(t->requires_grad() && at::GradMode::is_enabled()); }
+bool floats(const at::Tensor* t, int64_t n) { return dense(t) && t->scalar_type() == at::kFloat && t->numel() == n; }
+// rows with unit column stride, and the stride between them
+bool rows(const at::Tensor* t) { return t && t->is_cuda() && t->dim() == 2 && (t->size(1) <= 1 || t->stride(1) == 1); }
+int64_t row_stride(const at::Tensor& t) { return t.size(0) > 1 ? t.stride(0) : std::max(t.stride(0), t.size(1)); }
+bool aligned(const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+
+template <class Launch>
+int run(Launch launch) {
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = launch();
+  Py_END_ALLOW_THREADS
+  return rc;
+}
+PyObject* none() { Py_RETURN_NONE; }
+PyObject* wrap(const at::Tensor& t) { return THPVariable_Wrap(t); }
+
+// block_ok(x, w, end): the caller's rule (block_linear_ok has it, with its reasons).
+PyObject* block_ok(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 3) return PyErr_Format(PyExc_TypeError, "block_ok takes 3 arguments");
+  const at::Tensor *x = tensor(args[0]), *w = tensor(args[1]);
+  if (!x || !w || !block_linear_us) return none();
+  const bool end = PyObject_IsTrue(args[2]);
+  if (x->dim() != 2 || w->dim() != 2) Py_RETURN_FALSE;
+  const int64_t T = x->size(0), K = x->size(1), N = w->size(0);
+  if (!(T > 0 && x->is_cuda() && x->scalar_type() == at::kBFloat16 && w->scalar_type() == at::kBFloat16 && w->is_contiguous() && w->size(1) == K &&
+        K % 64 == 0 && K >= 64 && K <= 32768 && N % 16 == 0 && N > 0 && N < 1 << 20 && T < 1 << 22 && (T <= lines.block_rows || K <= lines.block_depth)))
+    Py_RETURN_FALSE;
+  const double us = block_linear_us(T, (int32_t)K, (int32_t)N);
+  if (us > lines.block_us) Py_RETURN_FALSE;
+  if (!end && (us > lines.captured_us || T > lines.captured_rows || K > lines.captured_depth)) {
+    hipStreamCaptureStatus status;
+    if (hipStreamIsCapturing(c10::hip::getCurrentHIPStream().stream(), &status) != hipSuccess) return none();
+    if (status != hipStreamCaptureStatusNone) Py_RETURN_FALSE;
+  }
+  return PyBool_FromLong((x->is_contiguous() || (x->stride(1) == 1 && x->stride(0) % 8 == 0 && K <= x->stride(0) && x->stride(0) < 1 << 21)) && aligned(*x) &&
+                         aligned(*w) && w->device() == x->device() && plain(x) && plain(w));
+  END_HANDLE_TH_ERRORS
+}
+
+// linear(x, w, mode, gelu_n, limit, alpha, shift): msa_block_linear of operands that block_ok took
+PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 7) return PyErr_Format(PyExc_TypeError, "linear takes 7 arguments");
+  const at::Tensor *x = tensor(args[0]), *w = tensor(args[1]);
+  const long mode = PyLong_AsLong(args[2]), gelu_n = PyLong_AsLong(args[3]);
+  const msa_tile_end end{(int32_t)mode, (int32_t)gelu_n, (float)PyFloat_AsDouble(args[4]), (float)PyFloat_AsDouble(args[5]), (float)PyFloat_AsDouble(args[6])};
+  if (PyErr_Occurred()) return nullptr;
+  if (!x || !w || !block_linear || !x->is_cuda() || x->dim() != 2 || w->dim() != 2) return none();
+  const int64_t T = x->size(0), K = x->size(1), N = w->size(0);
+  at::Tensor out = at::empty({T, mode == MSA_TILE_GLU ? N / 2 : N}, x->options().requires_grad(false));
+  const auto st = stream();
+  const int rc = run([&] {
+    return block_linear(x->data_ptr(), T > 1 ? x->stride(0) : K, T, (int32_t)K, w->data_ptr(), (int32_t)N, &end, out.data_ptr(), out.size(1), st);
+  });
+  return rc == MSA_OK ? wrap(out) : PyLong_FromLong(rc);
+  END_HANDLE_TH_ERRORS
+}
+
+struct Batch {
+  const msa_seq_batch* c;
+  int64_t top;                 // its largest slot
+  bool get(PyObject* address, PyObject* slot) {
+    c = static_cast<const msa_seq_batch*>(PyLong_AsVoidPtr(address));
+    top = PyLong_AsLongLong(slot);
+    return c && !PyErr_Occurred();
+  }
+};
+
+// residual_norm(batch address, its largest slot, x, y, gate, gate_bias, norm_w, norm_b, alpha, shift, prev, want_h, dtype): (x', h, h_shift)
+PyObject* residual_norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 13) return PyErr_Format(PyExc_TypeError, "residual_norm takes 13 arguments");
+  Batch b;
+  if (!b.get(args[0], args[1])) return PyErr_Occurred() ? nullptr : none();
+  const at::Tensor *x = tensor(args[2]), *y = tensor(args[3]), *gate = tensor(args[4]), *gate_bias = tensor(args[5]), *nw = tensor(args[6]),
+                   *nb = tensor(args[7]), *shift = tensor(args[9]), *prev = tensor(args[10]);
+  const msa_dyn_tanh norm{nw ? static_cast<const float*>(nw->data_ptr()) : nullptr, nb ? static_cast<const float*>(nb->data_ptr()) : nullptr,
+                          (float)PyFloat_AsDouble(args[8]), 0};
+  const long want_h = PyLong_AsLong(args[11]), dtype = PyLong_AsLong(args[12]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!dense(x) || x->dim() != 2 || x->scalar_type() != at::kFloat || x->size(0) != b.c->rows || (!is_none(args[10]) && !dense(prev))) return none();
+  const int64_t T = x->size(0), W = x->size(1);
+  if ((!is_none(args[6]) || !is_none(args[7])) && !(floats(nw, W) && floats(nb, W))) return none();
+  if (!is_none(args[3])) {
+    if (!rows(y) || !rows(gate) || !floats(gate_bias, W) || y->sizes() != x->sizes() || gate->sizes() != x->sizes() || dtype_of(*y) != dtype || dtype_of(*gate) != dtype)
+      return none();
+  }
+  if (!is_none(args[9]) && !(floats(shift, W) && prev && prev->scalar_type() == at::kFloat && prev->dim() == 2 && prev->size(1) == W && prev->size(0) > b.top)) return none();
+  const auto f32 = x->options().requires_grad(false), act = f32.dtype(dtype == MSA_BF16 ? at::kBFloat16 : at::kFloat);
+  at::Tensor out, h, hs;
+  if (y) out = at::empty({T, W}, f32);
+  if (nw && want_h) h = at::empty({T, W}, act);
+  if (shift) hs = at::empty({T, W}, act);
+  const auto st = stream();
+  const int rc = run([&] {
+    return residual_norm_(static_cast<const float*>(x->data_ptr()), at_(y), y ? row_stride(*y) : 0, at_(gate), gate ? row_stride(*gate) : 0,
+                          static_cast<const float*>(at_(gate_bias)), y ? static_cast<float*>(out.data_ptr()) : nullptr, (int32_t)dtype, (int32_t)W, &norm,
+                          h.defined() ? h.data_ptr() : nullptr, static_cast<const float*>(at_(shift)), static_cast<float*>(at_(prev)),
+                          hs.defined() ? hs.data_ptr() : nullptr, b.c, st);
+  });
+  if (rc != MSA_OK) return PyLong_FromLong(rc);
+  PyObject* first = y ? wrap(out) : (Py_INCREF(args[2]), args[2]);
+  return Py_BuildValue("(NNN)", first, h.defined() ? wrap(h) : none(), hs.defined() ? wrap(hs) : none());
+  END_HANDLE_TH_ERRORS
+}
+
+// rms_residual(x, y, w, eps, next_w, out, want_h, dtype): (x', h)
+PyObject* rms_residual(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 8) return PyErr_Format(PyExc_TypeError, "rms_residual takes 8 arguments");
+  const at::Tensor *x = tensor(args[0]), *y = tensor(args[1]), *w = tensor(args[2]), *next_w = tensor(args[4]), *out = tensor(args[5]);
+  const double eps = PyFloat_AsDouble(args[3]);
+  const long want_h = PyLong_AsLong(args[6]), dtype = PyLong_AsLong(args[7]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!dense(x) || x->dim() != 2 || x->scalar_type() != at::kFloat || !y || !rows(y) || !floats(w, x->size(1)) || y->sizes() != x->sizes() || dtype_of(*y) != dtype ||
+      !out || !dense(out) || out->sizes() != x->sizes() || out->scalar_type() != at::kFloat || (!is_none(args[4]) && !floats(next_w, x->size(1))))
+    return none();
+  const int64_t T = x->size(0), W = x->size(1);
+  at::Tensor h;
+  if (want_h || next_w) h = at::empty({T, W}, x->options().requires_grad(false).dtype(dtype == MSA_BF16 ? at::kBFloat16 : at::kFloat));
+  const auto st = stream();
+  const int rc = run([&] {
+    return rms_residual_(static_cast<const float*>(x->data_ptr()), y->data_ptr(), row_stride(*y), static_cast<const float*>(w->data_ptr()), (float)eps,
+                         static_cast<float*>(out->data_ptr()), static_cast<const float*>(at_(next_w)), h.defined() ? h.data_ptr() : nullptr, (int32_t)dtype,
+                         (int32_t)T, (int32_t)W, st);
+  });
+  if (rc != MSA_OK) return PyLong_FromLong(rc);
+  Py_INCREF(args[5]);
+  return Py_BuildValue("(NN)", args[5], h.defined() ? wrap(h) : none());
+  END_HANDLE_TH_ERRORS
+}
+
+// conv_silu(batch address, its largest slot, x, taps, bias, state): the convolved rows
+PyObject* conv_silu(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 6) return PyErr_Format(PyExc_TypeError, "conv_silu takes 6 arguments");
+  Batch b;
+  if (!b.get(args[0], args[1])) return PyErr_Occurred() ? nullptr : none();
+  const at::Tensor *x = tensor(args[2]), *taps = tensor(args[3]), *bias = tensor(args[4]), *state = tensor(args[5]);
+  if (!rows(x) || dtype_of(*x) < 0 || !taps || taps->dim() != 2) return none();
+  const int64_t T = x->size(0), Cn = x->size(1), K = taps->size(1);
+  if (!floats(taps, Cn * K) || (!is_none(args[4]) && !floats(bias, Cn)) || !dense(state) || state->scalar_type() != at::kFloat || state->dim() != 3 ||
+      state->size(1) != K - 1 || state->size(2) != Cn || state->size(0) <= b.top || T != b.c->rows)
+    return none();
+  at::Tensor out = at::empty({T, Cn}, x->options().requires_grad(false));
+  const auto st = stream();
+  const int rc = run([&] {
+    return conv_silu_(x->data_ptr(), row_stride(*x), static_cast<const float*>(taps->data_ptr()), static_cast<const float*>(at_(bias)), dtype_of(*x), (int32_t)Cn,
+                      (int32_t)K, static_cast<float*>(state->data_ptr()), out.data_ptr(), Cn, b.c, st);
+  });
+  return rc == MSA_OK ? wrap(out) : PyLong_FromLong(rc);
+  END_HANDLE_TH_ERRORS
+}
+
+// group_rmsnorm(v, w, parts, eps)
+PyObject* group_rmsnorm(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 4) return PyErr_Format(PyExc_TypeError, "group_rmsnorm takes 4 arguments");
+  const at::Tensor *v = tensor(args[0]), *w = tensor(args[1]);
+  const long parts = PyLong_AsLong(args[2]);
+  const double eps = PyFloat_AsDouble(args[3]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!dense(v) || v->dim() != 2 || dtype_of(*v) < 0 || !floats(w, v->size(1))) return none();
+  at::Tensor out = at::empty({v->size(0), v->size(1)}, v->options().requires_grad(false));
+  const auto st = stream();
+  const int rc = run([&] {
+    return group_rmsnorm_(v->data_ptr(), dtype_of(*v), (int32_t)v->size(0), (int32_t)v->size(1), (int32_t)parts, static_cast<const float*>(w->data_ptr()), (float)eps,
+                          out.data_ptr(), st);
+  });
+  return rc == MSA_OK ? wrap(out) : PyLong_FromLong(rc);
+  END_HANDLE_TH_ERRORS
+}
+
+// [slots, a, b, c] fp32 states that reach the step's slots
+bool states(const at::Tensor* t, int64_t a, int64_t b, int64_t c, int64_t top) {
+  return dense(t) && t->scalar_type() == at::kFloat && t->dim() == 4 && t->size(1) == a && t->size(2) == b && t->size(3) == c && t->size(0) > top;
+}
+bool block(const at::Tensor* t, int64_t r, int64_t c, at::ScalarType type) { return rows(t) && t->size(0) == r && t->size(1) == c && t->scalar_type() == type; }
+
+// ssd(batch address, its largest slot, xbc, z, dt_raw, dt_bias, A_log, D, H, P, N, G, state, chunked): the gated output
+PyObject* ssd(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 14) return PyErr_Format(PyExc_TypeError, "ssd takes 14 arguments");
+  Batch b;
+  if (!b.get(args[0], args[1])) return PyErr_Occurred() ? nullptr : none();
+  const at::Tensor *xbc = tensor(args[2]), *z = tensor(args[3]), *dt = tensor(args[4]), *bias = tensor(args[5]), *a_log = tensor(args[6]), *d = tensor(args[7]),
+                   *state = tensor(args[12]);
+  const long H = PyLong_AsLong(args[8]), P = PyLong_AsLong(args[9]), N = PyLong_AsLong(args[10]), G = PyLong_AsLong(args[11]);
+  const bool chunked = PyObject_IsTrue(args[13]);
+  if (PyErr_Occurred()) return nullptr;
+  const int64_t T = b.c->rows;
+  if (!xbc || dtype_of(*xbc) < 0 || !floats(bias, H) || !floats(a_log, H) || !floats(d, H) || !states(state, H, N, P, b.top) ||
+      !block(xbc, T, H * P + 2 * G * N, xbc->scalar_type()) || !block(z, T, H * P, xbc->scalar_type()) || !block(dt, T, H, xbc->scalar_type()))
+    return none();
+  at::Tensor v = at::empty({T, H * P}, xbc->options().requires_grad(false)), ws;
+  const size_t need = chunked ? ssd_bytes(b.c->max_rows, b.c->n_seq, (int32_t)H, (int32_t)P, (int32_t)N) : 0;
+  if (need) ws = at::empty({(int64_t)need}, v.options().dtype(at::kByte));
+  const auto st = stream();
+  auto f = [](const at::Tensor* t) { return static_cast<float*>(t->data_ptr()); };
+  const int rc = run([&] {
+    auto call = [&](auto fn, auto... more) {
+      return fn(xbc->data_ptr(), row_stride(*xbc), z->data_ptr(), row_stride(*z), dt->data_ptr(), row_stride(*dt), f(bias), f(a_log), f(d), dtype_of(*xbc), (int32_t)H,
+                (int32_t)P, (int32_t)N, (int32_t)G, f(state), v.data_ptr(), b.c, more...);
+    };
+    return chunked ? call(ssd_chunked, need ? ws.data_ptr() : nullptr, need, st) : call(ssd_scan, st);
+  });
+  return rc == MSA_OK ? wrap(v) : PyLong_FromLong(rc);
+  END_HANDLE_TH_ERRORS
+}
+
+// delta(batch address, its largest slot, qkv, a, b, gate, A_log, dt_bias, norm, eps, H, G, D, E, state, chunked): normed and gated read-outs
+PyObject* delta(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 16) return PyErr_Format(PyExc_TypeError, "delta takes 16 arguments");
+  Batch b;
+  if (!b.get(args[0], args[1])) return PyErr_Occurred() ? nullptr : none();
+  const at::Tensor *qkv = tensor(args[2]), *a = tensor(args[3]), *beta = tensor(args[4]), *gate = tensor(args[5]), *a_log = tensor(args[6]), *bias = tensor(args[7]),
+                   *norm = tensor(args[8]), *state = tensor(args[14]);
+  const double eps = PyFloat_AsDouble(args[9]);
+  const long H = PyLong_AsLong(args[10]), G = PyLong_AsLong(args[11]), D = PyLong_AsLong(args[12]), E = PyLong_AsLong(args[13]);
+  const bool chunked = PyObject_IsTrue(args[15]);
+  if (PyErr_Occurred()) return nullptr;
+  const int64_t T = b.c->rows;
+  if (!qkv || dtype_of(*qkv) < 0 || !floats(a_log, H) || !floats(bias, H * D) || !floats(norm, E) || !states(state, H, D, E, b.top)) return none();
+  const auto type = qkv->scalar_type();
+  if (!block(qkv, T, 2 * G * D + H * E, type) || !block(a, T, H * D, type) || !block(beta, T, H, type) || !block(gate, T, H * E, type)) return none();
+  at::Tensor out = at::empty({T, H * E}, qkv->options().requires_grad(false)), ws;
+  auto f = [](const at::Tensor* t) { return static_cast<float*>(t->data_ptr()); };
+  msa_delta_args c{};
+  c.qkv = qkv->data_ptr(), c.a = a->data_ptr(), c.b = beta->data_ptr(), c.gate = gate->data_ptr();
+  c.qkv_stride = row_stride(*qkv), c.a_stride = row_stride(*a), c.b_stride = row_stride(*beta), c.gate_stride = row_stride(*gate);
+  c.A_log = f(a_log), c.dt_bias = f(bias), c.norm = f(norm), c.state = f(state), c.out = out.data_ptr();
+  c.H = (int32_t)H, c.G = (int32_t)G, c.D = (int32_t)D, c.E = (int32_t)E, c.eps = (float)eps;
+  const size_t need = chunked ? delta_bytes(&c, b.c->max_rows, b.c->n_seq) : 0;
+  if (need) ws = at::empty({(int64_t)need}, out.options().dtype(at::kByte));
+  const auto st = stream();
+  const int rc = run([&] {
+    return chunked ? delta_chunked(&c, b.c, need ? ws.data_ptr() : nullptr, need, st) : delta_scan(&c, dtype_of(*qkv), b.c, st);
+  });
+  return rc == MSA_OK ? wrap(out) : PyLong_FromLong(rc);
+  END_HANDLE_TH_ERRORS
+}
+
+// pieces(words, places): the parts of an int64 vector, (first word, elements, whether of 32 bits) each
+PyObject* pieces(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 2 || !PyList_Check(args[1])) return PyErr_Format(PyExc_TypeError, "pieces takes a tensor and a list");
+  const at::Tensor* words = tensor(args[0]);
+  if (!words || words->dim() != 1 || words->scalar_type() != at::kLong) return PyErr_Format(PyExc_TypeError, "pieces of an int64 vector");
+  const Py_ssize_t count = PyList_GET_SIZE(args[1]);
+  THPObjectPtr out(PyList_New(count));
+  if (!out) return nullptr;
+  const at::Tensor halves = words->view(at::kInt);
+  for (Py_ssize_t i = 0; i < count; ++i) {
+    long long at, len;
+    int small;
+    if (!PyArg_ParseTuple(PyList_GET_ITEM(args[1], i), "LLp", &at, &len, &small)) return nullptr;
+    PyObject* part = wrap(small ? halves.narrow(0, 2 * at, len) : words->narrow(0, at, len));
+    if (!part) return nullptr;
+    PyList_SET_ITEM(out.get(), i, part);
+  }
+  return out.release();
+  END_HANDLE_TH_ERRORS
+}
+
+// clear(tensors, slot): zeroes the tensors' rows of that slot, in one launch or a few
+PyObject* clear(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 2 || !PyList_Check(args[0])) return PyErr_Format(PyExc_TypeError, "clear takes a list and a slot");
+  const long slot = PyLong_AsLong(args[1]);
+  if (PyErr_Occurred()) return nullptr;
+  std::vector<at::Tensor> rows;
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[0]); ++i) {
+    const at::Tensor* t = tensor(PyList_GET_ITEM(args[0], i));
+    if (!t) return PyErr_Format(PyExc_TypeError, "clear: not a tensor");
+    rows.push_back(t->select(0, slot));
+  }
+  if (!rows.empty()) at::_foreach_zero_(rows);
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+template <class F>
+bool resolve(void* lib, const char* name, F& f) {
+  f = reinterpret_cast<F>(dlsym(lib, name));
+  if (!f) PyErr_Format(PyExc_ImportError, "%s is not in the library", name);
+  return f != nullptr;
+}
+// bind(libmsa_amd.so or None, libmsa_seq.so, (lines ...)): once, in front of everything else.  The libraries stay apart: both have some
+// names.  Without the first, which a checkout that only runs the decoders of mixed layers has not built, products are declined.
+PyObject* bind(PyObject*, PyObject* args) {
+  const char *amd, *seq;
+  Lines l;
+  if (!PyArg_ParseTuple(args, "zs(LLLLdd)", &amd, &seq, &l.block_rows, &l.block_depth, &l.captured_rows, &l.captured_depth, &l.block_us,
+                        &l.captured_us))
+    return nullptr;
+  void *a = amd ? dlopen(amd, RTLD_NOW | RTLD_LOCAL) : nullptr, *s = dlopen(seq, RTLD_NOW | RTLD_LOCAL);
+  if ((amd && !a) || !s) return PyErr_Format(PyExc_ImportError, "%s", dlerror());
+  if (a && (!resolve(a, "msa_block_linear", block_linear) || !resolve(a, "msa_block_linear_us", block_linear_us))) return nullptr;
+  if (!resolve(s, "msa_seq_residual_norm", residual_norm_) || !resolve(s, "msa_seq_rms_residual", rms_residual_) ||
+      !resolve(s, "msa_seq_conv_silu", conv_silu_) || !resolve(s, "msa_seq_group_rmsnorm", group_rmsnorm_) ||
+      !resolve(s, "msa_seq_ssd_scan", ssd_scan) || !resolve(s, "msa_seq_ssd_chunked", ssd_chunked) ||
+      !resolve(s, "msa_seq_ssd_chunked_workspace_bytes", ssd_bytes) || !resolve(s, "msa_seq_delta_scan", delta_scan) ||
+      !resolve(s, "msa_seq_delta_chunked", delta_chunked) || !resolve(s, "msa_seq_delta_chunked_workspace_bytes", delta_bytes))
+    return nullptr;
+  lines = l;
+  Py_RETURN_NONE;
+}
+
+#define MSA_FAST(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr}, MSA_FAST(block_ok), MSA_FAST(linear), MSA_FAST(residual_norm), MSA_FAST(rms_residual), MSA_FAST(conv_silu),
+                         MSA_FAST(group_rmsnorm), MSA_FAST(ssd), MSA_FAST(delta), MSA_FAST(pieces), MSA_FAST(clear), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host() { return PyModule_Create(&module); }

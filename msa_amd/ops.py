@@ -7,6 +7,7 @@ stream is given, and raise :class:`msa_amd._lib.MsaError` on any failure.
 from __future__ import annotations
 
 import ctypes as C
+import os
 from dataclasses import dataclass
 from typing import List, Optional, Sequence, Tuple
 
@@ -575,12 +576,14 @@ CAPTURED_US, CAPTURED_ROWS, CAPTURED_DEPTH = 12.5, 1024, 2048
 def block_linear_ok(x: torch.Tensor, w: torch.Tensor, end: bool = False) -> bool:
     """Whether ``x [T, K] @ w.T`` (with an ``end``: behind which the vendor's product needs another launch) is ``block_linear``'s: operands
     as it takes them, no gradients asked for, and about as fast there or faster.  The host takes about 21 us to hand a product to the
-    vendor's library and 7 to this, so up to ``BLOCK_ROWS`` rows, where a prompt waits for the host, products of about that length are here
+    vendor's library and 5 to this, so up to ``BLOCK_ROWS`` rows, where a prompt waits for the host, products of about that length are here
     also where the vendor's kernel alone is a little faster (us, the vendor's and here, rows x K x N: 64 x 1024 x 1024 6.6 and 5.0, 1000 x
     1024 x 6176 24.2 and 20.5, 2048 x 1024 x 4096 20.6 and 22; behind the line 300 x 2560 x 8192, 25.8 and 27.4).  Of more rows those of a depth up to ``BLOCK_DEPTH`` (6001 x 128 x 4096 25.9 and 18.5; 8192 x 256 x 2048 16.7 and 19.0).  A captured
     call pays for no host: there the kernels alone decide (17 x 1024 x 6176 9.0 and 5.7, 64 x 1024 x 1024 7.0 and 5.4, 1000 x 2048 x 1024 11.8
     and 11.0; behind the lines 32 x 2560 x 2560 7.7 and 9.9, 17 x 4096 x 2560 11.8 and 13.8, 1500 x 128 x 4096 9.0 and 10.4, 573 x 1024 x 8192
     16.4 and 21.0)."""
+    if x.is_cuda and (took := host().block_ok(x, w, end)) is not None:
+        return took
     (T, K), N = (x.shape if x.dim() == 2 else (0, 0)), w.shape[0]
     if not (T > 0 and w.dim() == 2 and x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] == K
             and K % 64 == 0 and 64 <= K <= 32768 and N % 16 == 0 and 0 < N < 1 << 20 and T < 1 << 22 and (T <= BLOCK_ROWS or K <= BLOCK_DEPTH)):
@@ -596,12 +599,26 @@ def block_linear_ok(x: torch.Tensor, w: torch.Tensor, end: bool = False) -> bool
 
 def block_linear(x: torch.Tensor, w: torch.Tensor, glu: Optional[Tuple[float, float, float]] = None, gelu_n: int = 0) -> torch.Tensor:
     """``tile_linear`` of few rows (``x`` and ``w`` as ``block_linear_ok`` has them), with ``glu``, ``gelu_n`` or neither."""
-    (T, K), N = x.shape, w.shape[0]
-    out = torch.empty((T, N if glu is None else N // 2), dtype=x.dtype, device=x.device)
-    end = _lib.TileEnd(_lib.TILE_GLU if glu is not None else _lib.TILE_GELU if gelu_n else _lib.TILE_STORE, gelu_n, *(glu or (0.0, 0.0, 0.0)))
-    check(_lib.load().msa_block_linear(x.data_ptr(), x.stride(0) if T > 1 else K, T, K, w.data_ptr(), N, C.byref(end), out.data_ptr(),
-                                       out.shape[1], _stream()), "msa_block_linear")
+    out = host().linear(x, w, _lib.TILE_GLU if glu is not None else _lib.TILE_GELU if gelu_n else _lib.TILE_STORE, gelu_n, *(glu or _NO_GLU))
+    if out is None:
+        raise ValueError("block_linear: x [T, K] and w [N, K] on the device")
+    if type(out) is int:
+        check(out, "msa_block_linear")
     return out
+
+
+_NO_GLU = (0.0, 0.0, 0.0)
+_host = None
+
+
+def host():
+    """The module of ``csrc/host.cpp``, bound to the libraries; raises if it is missing."""
+    global _host
+    if _host is None:
+        module = _lib.load_host()
+        module.bind(_lib.LIB_PATH if os.path.exists(_lib.LIB_PATH) else None, _lib.SEQ_LIB_PATH, (BLOCK_ROWS, BLOCK_DEPTH, CAPTURED_ROWS, CAPTURED_DEPTH, BLOCK_US, CAPTURED_US))
+        _host = module
+    return _host
 
 
 def plain_module(module: torch.nn.Module, base: type) -> bool:

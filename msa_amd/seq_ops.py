@@ -66,6 +66,8 @@ def upload(device, arrays, wait: bool = True) -> list:
     for a, at in zip(arrays, places):
         to[at:at + (a.nbytes + 7) // 8].view(a.dtype)[:len(a)] = a
     dev = host.to(device, non_blocking=not wait)
+    if dev.is_cuda:
+        return ops.host().pieces(dev, [(at, len(a), a.dtype == np.int32) for a, at in zip(arrays, places)])
     return [dev[at:at + (a.nbytes + 7) // 8].view(torch.int32 if a.dtype == np.int32 else torch.int64)[:len(a)]
             for a, at in zip(arrays, places)]
 
@@ -94,7 +96,7 @@ class StepBatch:
         self.row_seq = rest.pop(0) if many else zeros
         self.extra = rest
         self.c = _lib.SeqBatch(ptr(self.cu), ptr(self.row_seq), ptr(self.slot), ptr(self.pos), n, self.rows, self.max_rows, 0)
-        self.ref = C.byref(self.c)
+        self.ref, self.address, self.top = C.byref(self.c), C.addressof(self.c), max(slots)
         self.max_keys = max(p + c for p, c in zip(positions, counts))     # longest sequence at the end of the step
         self._row_at = {}
 
@@ -123,6 +125,13 @@ def residual_norm(x: torch.Tensor, batch: StepBatch, dtype: torch.dtype, y=None,
                   norm: Optional[DynTanhNorm] = None, shift=None, prev=None, want_h: bool = True):
     """``(x', h, h_shift)``: ``x' = x + sigmoid(gate + gate_bias) * y`` (``x`` itself without ``y``), ``h = norm(x')``
     and the token-shifted ``h`` (``prev [slots, W]`` holds every sequence's last ``h`` and is updated)."""
+    if x.is_cuda:
+        n = norm or _NO_NORM
+        got = ops.host().residual_norm(batch.address, batch.top, x, y, gate, gate_bias, n.w, n.b, n.alpha, shift, prev, want_h, dtype_code(dtype))
+        if type(got) is tuple:
+            return got
+        if got is not None:
+            _check(got, "msa_seq_residual_norm")
     _dense(x, prev)
     T, W = x.shape
     if x.dtype != torch.float32 or T != batch.rows:
@@ -169,6 +178,12 @@ def embed_norm(tokens: torch.Tensor, table: torch.Tensor, batch: StepBatch, norm
 def rms_residual(x: torch.Tensor, dtype: torch.dtype, y=None, w=None, eps: float = 0.0, next_w=None, out=None, want_h: bool = True):
     """``(x', h)``: ``x' = x + rms_norm(y) * w`` (``x`` itself without ``y``; into ``out``, which may be ``x``), and ``h = x'``, or
     ``rms_norm(x') * next_w``, in ``dtype``."""
+    if x.is_cuda and y is not None and out is not None:
+        got = ops.host().rms_residual(x, y, w, eps, next_w, out, want_h, dtype_code(dtype))
+        if type(got) is tuple:
+            return got
+        if got is not None:
+            _check(got, "msa_seq_rms_residual")
     _dense(x, out)
     T, W = x.shape
     if x.dtype != torch.float32 or (out is not None and (out.shape != x.shape or out.dtype != torch.float32)):
@@ -256,6 +271,12 @@ def join(x: torch.Tensor, x0: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
 
 def conv_silu(x: torch.Tensor, taps: torch.Tensor, bias: Optional[torch.Tensor], state: torch.Tensor, batch: StepBatch) -> torch.Tensor:
     """Causal per-channel convolution + silu of ``x [rows, C]``; ``state [slots, K - 1, C]`` is updated."""
+    if x.is_cuda:
+        got = ops.host().conv_silu(batch.address, batch.top, x, taps, bias, state)
+        if type(got) is int:
+            _check(got, "msa_seq_conv_silu")
+        if got is not None:
+            return got
     T, Cn = x.shape
     K = taps.shape[1]
     _f32(Cn * K, taps)
@@ -272,6 +293,12 @@ def conv_silu(x: torch.Tensor, taps: torch.Tensor, bias: Optional[torch.Tensor],
 def ssd(xbc, z, dt_raw, dt_bias, A_log, D, H: int, P: int, N: int, G: int, state, batch: StepBatch, chunked: bool = False):
     """Gated output ``[rows, H P]`` of the state-space recurrence; ``state [slots, H, N, P]`` fp32 is updated.  ``chunked``
     takes the matrix-core form (bf16)."""
+    if xbc.is_cuda:
+        got = ops.host().ssd(batch.address, batch.top, xbc, z, dt_raw, dt_bias, A_log, D, H, P, N, G, state, chunked)
+        if type(got) is int:
+            _check(got, "msa_seq_ssd")
+        if got is not None:
+            return got
     _f32(H, dt_bias, A_log, D)
     _dense(state)
     T = batch.rows
@@ -294,6 +321,12 @@ def ssd(xbc, z, dt_raw, dt_bias, A_log, D, H: int, P: int, N: int, G: int, state
 
 def group_rmsnorm(v: torch.Tensor, w: torch.Tensor, parts: int, eps: float) -> torch.Tensor:
     """RMS norm of ``v [rows, n]`` in ``parts`` equal parts, times ``w``."""
+    if v.is_cuda:
+        got = ops.host().group_rmsnorm(v, w, parts, eps)
+        if type(got) is int:
+            _check(got, "msa_seq_group_rmsnorm")
+        if got is not None:
+            return got
     _dense(v)
     T, n = v.shape
     _f32(n, w)
@@ -315,6 +348,12 @@ def delta(qkv, a, b, gate, A_log, dt_bias, norm, eps: float, H: int, G: int, D: 
     """Normed and gated read-outs ``[rows, H E]`` of the delta rule with a decay per key channel; ``qkv [rows, 2 G D + H E]``,
     ``a [rows, H D]``, ``b [rows, H]``, ``gate [rows, H E]``; ``state [slots, H, D, E]`` fp32 is updated.  ``chunked`` takes the
     matrix-core form (bf16)."""
+    if qkv.is_cuda:
+        got = ops.host().delta(batch.address, batch.top, qkv, a, b, gate, A_log, dt_bias, norm, eps, H, G, D, E, state, chunked)
+        if type(got) is int:
+            _check(got, "msa_seq_delta")
+        if got is not None:
+            return got
     T = batch.rows
     _f32(H, A_log)
     _f32(H * D, dt_bias)

@@ -123,7 +123,8 @@ class StepDecoder:
         for key, tokens, want in entries:
             if not len(tokens) or any(not 0 <= w < len(tokens) for w in want):
                 raise ValueError(f"sequence {key!r}: no tokens, or a wanted place outside them")
-            if not 0 <= int(tokens.min()) <= int(tokens.max()) < self.config.vocab:
+            ids = tokens.numpy()
+            if not 0 <= int(ids.min()) <= int(ids.max()) < self.config.vocab:
                 raise ValueError(f"sequence {key!r}: token outside the vocabulary")
         cache.reserve(max(cache.length.get(k, 0) + len(t) for k, t, _ in entries))
         for key, _, _ in entries:
