@@ -64,6 +64,8 @@ def _compile(src: str) -> str:
 #  * score_parts_kernel (route_score.hip), rows_ring_kernel (rows_ring.h), attn_ring_kernel and attn_decode_fused_kernel (attn.hip): likewise, they count what
 #    their rings have in flight.  What the first requests into LDS in front of its loop is read by asm statements, for
 #    which the compiler does not wait: the first request has to be waited for in front of the first LDS read.
+#  * flow_gemm_kernel (flow_gemm.hip): its products are asm statements whose latency the compiler does not know: between the first
+#    and the last of them nothing else may touch an accumulation register.  It counts what its ring has in flight.
 #  * delta_step_kernel (seq_delta.hip): loads past the end of what it reads rely on the range check of the buffer, which compares
 #    the vector offset alone.  No scalar offsets.
 # ---------------------------------------------------------------------------------------------------------------
@@ -73,11 +75,12 @@ CONTRACTS = {
     "gemm.hip": [("tile_gemm_kernel", {"max_compiler_vgpr": 127, "no_agpr": True}), ("tile_flow_kernel", {"max_compiler_vgpr": 23, "no_agpr": True})],
     "flash_attn.hip": [("flash_attn_kernel", {}), ("flash_wide_kernel", {"max_compiler_vgpr": 55, "no_agpr": True})],
     "linear.hip": [("rows_ring_kernel", {})],
+    "flow_gemm.hip": [("flow_gemm_kernel", {"fixed_products": True})],
     "seq_rows.hip": [("rows_ring_kernel", {})],
     "attn.hip": [("attn_ring_kernel", {}), ("attn_decode_fused_kernel", {})],
     "seq_delta.hip": [("delta_step_kernel", {"no_scalar_offset": True})],
 }
-LDS_WAITS = {"linear.hip": "rows_ring_kernel", "seq_rows.hip": "rows_ring_kernel"}
+LDS_WAITS = {"flow_gemm.hip": "flow_gemm_kernel", "linear.hip": "rows_ring_kernel", "seq_rows.hip": "rows_ring_kernel"}
 
 
 def _device_asm(src: str, extra=()) -> str:
@@ -87,10 +90,10 @@ def _device_asm(src: str, extra=()) -> str:
     return r.stdout
 
 
-def check_kernel_contracts(asm: str, kernel_substring: str, max_compiler_vgpr=None, no_agpr=False, no_scalar_offset=False):
+def check_kernel_contracts(asm: str, kernel_substring: str, max_compiler_vgpr=None, no_agpr=False, no_scalar_offset=False, fixed_products=False):
     """Returns the list of violations found in the device assembly `asm` for every kernel whose symbol contains
     `kernel_substring`: scratch use or spills (always), and, outside inline-asm regions, vector registers above
-    `max_compiler_vgpr` / any accumulation register / any buffer access with a scalar offset."""
+    `max_compiler_vgpr` / any accumulation register (with `fixed_products` between the products) / any buffer access with a scalar offset."""
     problems = []
     lines = asm.split("\n")
     # function bodies: from "<symbol>:" to s_endpgm
@@ -101,7 +104,7 @@ def check_kernel_contracts(asm: str, kernel_substring: str, max_compiler_vgpr=No
             i += 1
             continue
         name, found = m.group(1), found + 1
-        in_asm = False
+        in_asm, multiplied, between = False, False, []
         i += 1
         while i < len(lines) and "s_endpgm" not in lines[i]:
             line = lines[i]
@@ -116,7 +119,12 @@ def check_kernel_contracts(asm: str, kernel_substring: str, max_compiler_vgpr=No
             if not code or code.endswith(":") or code.startswith("."):
                 continue
             if in_asm:
+                if code.startswith("v_mfma"):
+                    problems += between
+                    multiplied, between = True, []
                 continue
+            if fixed_products and multiplied and re.search(r"\ba\d+\b|\ba\[\d+|accvgpr", code):
+                between.append(f"{name}: an accumulation register is touched between the products: {code}")
             if code.startswith("scratch_"):
                 problems.append(f"{name}: scratch access: {code}")
             if no_agpr and re.search(r"\ba\d+\b|\ba\[\d+|accvgpr", code):

@@ -23,6 +23,9 @@ namespace {
 
 decltype(&msa_block_linear) block_linear;
 decltype(&msa_block_linear_us) block_linear_us;
+decltype(&msa_flow_linear) flow_linear;
+decltype(&msa_flow_linear_us) flow_linear_us;
+decltype(&msa_flow_workspace_bytes) flow_bytes;
 decltype(&msa_seq_residual_norm) residual_norm_;
 decltype(&msa_seq_rms_residual) rms_residual_;
 decltype(&msa_seq_conv_silu) conv_silu_;
@@ -102,6 +105,33 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const auto st = stream();
   const int rc = run([&] {
     return block_linear(x->data_ptr(), T > 1 ? x->stride(0) : K, T, (int32_t)K, w->data_ptr(), (int32_t)N, &end, out.data_ptr(), out.size(1), st);
+  });
+  return rc == MSA_OK ? wrap(out) : PyLong_FromLong(rc);
+  END_HANDLE_TH_ERRORS
+}
+
+// flow(x, w, mode, gelu_n, limit, alpha, shift): msa_flow_linear where msa_flow_linear_us takes it, with no gradients asked for
+PyObject* flow(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 7) return PyErr_Format(PyExc_TypeError, "flow takes 7 arguments");
+  const at::Tensor *x = tensor(args[0]), *w = tensor(args[1]);
+  const long mode = PyLong_AsLong(args[2]), gelu_n = PyLong_AsLong(args[3]);
+  const msa_tile_end end{(int32_t)mode, (int32_t)gelu_n, (float)PyFloat_AsDouble(args[4]), (float)PyFloat_AsDouble(args[5]), (float)PyFloat_AsDouble(args[6])};
+  if (PyErr_Occurred()) return nullptr;
+  if (!x || !w || !flow_linear || !x->is_cuda() || x->dim() != 2 || w->dim() != 2) return none();
+  const int64_t T = x->size(0), K = x->size(1), N = w->size(0);
+  if (!(x->scalar_type() == at::kBFloat16 && w->scalar_type() == at::kBFloat16 && w->is_contiguous() && w->size(1) == K && K <= 32768 && N % 16 == 0 &&
+        N < 1 << 20 && (x->is_contiguous() || (x->stride(1) == 1 && x->stride(0) % 8 == 0 && K <= x->stride(0) && x->stride(0) < 1 << 21)) && aligned(*x) &&
+        aligned(*w) && w->device() == x->device() && plain(x) && plain(w) && gelu_n % 8 == 0 && gelu_n <= N &&
+        flow_linear_us(T, (int32_t)K, (int32_t)N) > 0.f))
+    return none();
+  at::Tensor out = at::empty({T, mode == MSA_TILE_GLU ? N / 2 : N}, x->options().requires_grad(false)), ws;
+  const size_t need = flow_bytes(T, (int32_t)K, (int32_t)N);
+  if (need) ws = at::empty({(int64_t)need}, x->options().requires_grad(false).dtype(at::kByte));
+  const auto st = stream();
+  const int rc = run([&] {
+    return flow_linear(x->data_ptr(), x->stride(0), T, (int32_t)K, w->data_ptr(), (int32_t)N, &end, out.data_ptr(), out.size(1),
+                       need ? ws.data_ptr() : nullptr, need, st);
   });
   return rc == MSA_OK ? wrap(out) : PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
@@ -347,7 +377,8 @@ PyObject* bind(PyObject*, PyObject* args) {
     return nullptr;
   void *a = amd ? dlopen(amd, RTLD_NOW | RTLD_LOCAL) : nullptr, *s = dlopen(seq, RTLD_NOW | RTLD_LOCAL);
   if ((amd && !a) || !s) return PyErr_Format(PyExc_ImportError, "%s", dlerror());
-  if (a && (!resolve(a, "msa_block_linear", block_linear) || !resolve(a, "msa_block_linear_us", block_linear_us))) return nullptr;
+  if (a && (!resolve(a, "msa_block_linear", block_linear) || !resolve(a, "msa_block_linear_us", block_linear_us) || !resolve(a, "msa_flow_linear", flow_linear) ||
+            !resolve(a, "msa_flow_linear_us", flow_linear_us) || !resolve(a, "msa_flow_workspace_bytes", flow_bytes))) return nullptr;
   if (!resolve(s, "msa_seq_residual_norm", residual_norm_) || !resolve(s, "msa_seq_rms_residual", rms_residual_) ||
       !resolve(s, "msa_seq_conv_silu", conv_silu_) || !resolve(s, "msa_seq_group_rmsnorm", group_rmsnorm_) ||
       !resolve(s, "msa_seq_ssd_scan", ssd_scan) || !resolve(s, "msa_seq_ssd_chunked", ssd_chunked) ||
@@ -359,7 +390,7 @@ PyObject* bind(PyObject*, PyObject* args) {
 }
 
 #define MSA_FAST(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr}, MSA_FAST(block_ok), MSA_FAST(linear), MSA_FAST(residual_norm), MSA_FAST(rms_residual), MSA_FAST(conv_silu),
+PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr}, MSA_FAST(block_ok), MSA_FAST(linear), MSA_FAST(flow), MSA_FAST(residual_norm), MSA_FAST(rms_residual), MSA_FAST(conv_silu),
                          MSA_FAST(group_rmsnorm), MSA_FAST(ssd), MSA_FAST(delta), MSA_FAST(pieces), MSA_FAST(clear), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

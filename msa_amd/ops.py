@@ -608,6 +608,20 @@ def block_linear(x: torch.Tensor, w: torch.Tensor, glu: Optional[Tuple[float, fl
 
 
 _NO_GLU = (0.0, 0.0, 0.0)
+FLOW_FIRST = 896        # rows up to which deep products are flow_linear's (weights from memory, there and here: 700 x 9728 x 2560 53 and 49 us, 1000 61.5 and 64)
+
+
+def flow_linear(x: torch.Tensor, w: torch.Tensor, glu: Optional[Tuple[float, float, float]] = None, gelu_n: int = 0) -> Optional[torch.Tensor]:
+    """``tile_linear`` of some hundred rows, ``x [T, K]`` and ``w [N, K]``, with ``glu``, ``gelu_n`` or neither, where one round of mid-sized
+    tiles fills the chip; None where another form is the better one or has to take the operands (gradients, strides, types)."""
+    if not x.is_cuda:
+        return None
+    out = host().flow(x, w, _lib.TILE_GLU if glu is not None else _lib.TILE_GELU if gelu_n else _lib.TILE_STORE, gelu_n, *(glu or _NO_GLU))
+    if type(out) is int:
+        check(out, "msa_flow_linear")
+    return out
+
+
 _host = None
 
 

@@ -219,8 +219,13 @@ def clamped_glu(gu: torch.Tensor, limit: float, alpha: float = GLU_ALPHA, shift:
 
 def product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x @ w.T`` of a step's rows."""
+    few = MAX_ROWS < x.shape[0] < ops.FLOW_FIRST
+    if few and (y := ops.flow_linear(x, w)) is not None:
+        return y
     if x.shape[0] >= ops.TILE_ROWS and ops.tile_linear_ok(x, w, end=False):
         return ops.tile_linear(x, w)
+    if not few and x.shape[0] > MAX_ROWS and (y := ops.flow_linear(x, w)) is not None:
+        return y
     return ops.block_linear(x, w) if ops.block_linear_ok(x, w) else F.linear(x, w)
 
 
@@ -228,6 +233,8 @@ def product_gelu(x: torch.Tensor, w: torch.Tensor, n: int) -> torch.Tensor:
     """``x @ w.T``, its first ``n`` columns through gelu."""
     if x.shape[0] >= ops.TILE_ROWS and n % 8 == 0 and ops.tile_linear_ok(x, w):
         return ops.tile_linear(x, w, gelu_n=n)
+    if n > 0 and x.shape[0] > MAX_ROWS and (y := ops.flow_linear(x, w, gelu_n=n)) is not None:
+        return y
     if n % 8 == 0 and ops.block_linear_ok(x, w, True):
         return ops.block_linear(x, w, gelu_n=n)
     y = F.linear(x, w)
@@ -239,6 +246,8 @@ def product_glu(x: torch.Tensor, w: torch.Tensor, limit: float, alpha: float = G
     """``clamped_glu(x @ w.T)``."""
     if x.shape[0] >= ops.TILE_ROWS and w.shape[0] % 16 == 0 and ops.tile_linear_ok(x, w):
         return ops.tile_linear(x, w, glu=(limit, alpha, shift))
+    if x.shape[0] > MAX_ROWS and (y := ops.flow_linear(x, w, glu=(limit, alpha, shift))) is not None:
+        return y
     if ops.block_linear_ok(x, w, True):
         return ops.block_linear(x, w, glu=(limit, alpha, shift))
     return clamped_glu(F.linear(x, w), limit, alpha, shift)
