@@ -83,6 +83,8 @@ int msa_seq_ssd_chunked(const void* xbc, int64_t xbc_stride, const void* z, int6
                         size_t workspace_bytes, void* stream);
 
 /* RMS norm of n columns in `parts` equal parts, times w: [rows, n] dense of `dtype`. */
+/* Zeroes row slots[s] of every tensor: base[t], rows of bytes[t] bytes behind one another.  All arguments on the host. */
+int msa_seq_clear(void* const* base, const int64_t* bytes, int32_t tensors, const int64_t* slots, int32_t n_slots, void* stream);
 int msa_seq_group_rmsnorm(const void* v, int32_t dtype, int32_t rows, int32_t n, int32_t parts, const float* w, float eps,
                           void* out, void* stream);
 

@@ -155,19 +155,25 @@ class SequenceStateCache:
 
     def open(self, key: Hashable) -> int:
         """Gives ``key`` a cleared slot."""
-        if key in self.slot_of:
-            raise KeyError(f"sequence {key!r} is already open")
-        if not self._free:
+        return self.open_all([key])[0]
+
+    def open_all(self, keys: Sequence[Hashable]) -> List[int]:
+        """Gives every one of ``keys`` a cleared slot."""
+        for i, key in enumerate(keys):
+            if key in self.slot_of or key in keys[:i]:
+                raise KeyError(f"sequence {key!r} is already open")
+        while len(self._free) < len(keys):
             self._resize(2 * self.slots, self.capacity)
-        slot = self._free.pop(0)
-        # in one launch: a model's six to thirty states took 4 us each, several times what clearing them costs
+        slots, self._free = self._free[:len(keys)], self._free[len(keys):]
+        # in one launch: a model's six to thirty states took 4 us each, several times what clearing them costs, and so did every sequence
         fixed = [held[name] for spec, held in zip(self.specs, self.tensors) for name, s in spec.items() if not s.per_token]
-        if fixed and all(t.is_cuda for t in fixed):
-            ops.host().clear(fixed, slot)
-        elif fixed:
-            torch._foreach_zero_([t[slot] for t in fixed])
-        self.slot_of[key], self.length[key] = slot, 0
-        return slot
+        if slots and fixed and all(t.is_cuda for t in fixed):
+            ops.host().clear(fixed, slots)
+        elif slots and fixed:
+            torch._foreach_zero_([t[slot] for t in fixed for slot in slots])
+        for key, slot in zip(keys, slots):
+            self.slot_of[key], self.length[key] = slot, 0
+        return slots
 
     def close(self, key: Hashable) -> None:
         """Gives the sequence's slot back."""

@@ -26,6 +26,7 @@ decltype(&msa_block_linear_us) block_linear_us;
 decltype(&msa_flow_linear) flow_linear;
 decltype(&msa_flow_linear_us) flow_linear_us;
 decltype(&msa_flow_workspace_bytes) flow_bytes;
+decltype(&msa_seq_clear) clear_;
 decltype(&msa_seq_residual_norm) residual_norm_;
 decltype(&msa_seq_rms_residual) rms_residual_;
 decltype(&msa_seq_conv_silu) conv_silu_;
@@ -344,17 +345,36 @@ PyObject* pieces(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// clear(tensors, slot): zeroes the tensors' rows of that slot, in one launch or a few
+// clear(tensors, slot): zeroes the tensors' rows of that slot, or of a list of slots, in one launch or a few
 PyObject* clear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 2 || !PyList_Check(args[0])) return PyErr_Format(PyExc_TypeError, "clear takes a list and a slot");
-  const long slot = PyLong_AsLong(args[1]);
+  std::vector<int64_t> slots;
+  const bool several = PyList_Check(args[1]);
+  for (Py_ssize_t i = 0; i < (several ? PyList_GET_SIZE(args[1]) : 1); ++i) slots.push_back(PyLong_AsLongLong(several ? PyList_GET_ITEM(args[1], i) : args[1]));
   if (PyErr_Occurred()) return nullptr;
   std::vector<at::Tensor> rows;
+  std::vector<void*> base;
+  std::vector<int64_t> bytes;
+  const at::Tensor* like = nullptr;
+  bool dense = clear_ != nullptr;
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[0]); ++i) {
     const at::Tensor* t = tensor(PyList_GET_ITEM(args[0], i));
     if (!t) return PyErr_Format(PyExc_TypeError, "clear: not a tensor");
-    rows.push_back(t->select(0, slot));
+    for (const int64_t slot : slots) {
+      rows.push_back(t->select(0, slot));
+      dense = dense && slot >= 0;
+    }
+    dense = dense && t->is_cuda() && t->is_contiguous() && plain(t) && (!like || t->device() == like->device());
+    if (!dense || t->numel() == 0) continue;
+    like = t;
+    base.push_back(t->data_ptr());
+    bytes.push_back((int64_t)t->nbytes() / t->size(0));
+  }
+  if (dense && like) {
+    const auto st = stream();
+    const int rc = run([&] { return clear_(base.data(), bytes.data(), (int32_t)base.size(), slots.data(), (int32_t)slots.size(), st); });
+    if (rc == MSA_OK) Py_RETURN_NONE;
   }
   if (!rows.empty()) at::_foreach_zero_(rows);
   Py_RETURN_NONE;
@@ -379,7 +399,7 @@ PyObject* bind(PyObject*, PyObject* args) {
   if ((amd && !a) || !s) return PyErr_Format(PyExc_ImportError, "%s", dlerror());
   if (a && (!resolve(a, "msa_block_linear", block_linear) || !resolve(a, "msa_block_linear_us", block_linear_us) || !resolve(a, "msa_flow_linear", flow_linear) ||
             !resolve(a, "msa_flow_linear_us", flow_linear_us) || !resolve(a, "msa_flow_workspace_bytes", flow_bytes))) return nullptr;
-  if (!resolve(s, "msa_seq_residual_norm", residual_norm_) || !resolve(s, "msa_seq_rms_residual", rms_residual_) ||
+  if (!resolve(s, "msa_seq_clear", clear_) || !resolve(s, "msa_seq_residual_norm", residual_norm_) || !resolve(s, "msa_seq_rms_residual", rms_residual_) ||
       !resolve(s, "msa_seq_conv_silu", conv_silu_) || !resolve(s, "msa_seq_group_rmsnorm", group_rmsnorm_) ||
       !resolve(s, "msa_seq_ssd_scan", ssd_scan) || !resolve(s, "msa_seq_ssd_chunked", ssd_chunked) ||
       !resolve(s, "msa_seq_ssd_chunked_workspace_bytes", ssd_bytes) || !resolve(s, "msa_seq_delta_scan", delta_scan) ||

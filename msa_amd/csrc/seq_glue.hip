@@ -508,6 +508,53 @@ extern "C" int msa_seq_join(const float* x, const float* x0, int32_t dtype, int3
   return MSA_OK;
 }
 
+namespace {
+// Rows of several tensors, by address and bytes of a row; up to as many of both as a launch's arguments hold.
+constexpr int kClearTensors = 24, kClearSlots = 16, kClearBytes = 16 << 10;      // bytes of a workgroup
+struct ClearArgs {
+  char* base[kClearTensors];
+  int64_t bytes[kClearTensors];
+  int32_t slot[kClearSlots];
+};
+__global__ __launch_bounds__(256) void clear_kernel(ClearArgs a) {
+  const int64_t bytes = a.bytes[blockIdx.y], from = (int64_t)blockIdx.x * kClearBytes;
+  if (from >= bytes) return;
+  char* row = a.base[blockIdx.y] + a.slot[blockIdx.z] * bytes;
+  const int64_t to = from + kClearBytes < bytes ? from + kClearBytes : bytes;
+  if ((((uintptr_t)row | (uintptr_t)bytes) & 15) == 0)
+    for (int64_t i = from + threadIdx.x * 16; i < to; i += 256 * 16) *reinterpret_cast<uint4*>(row + i) = make_uint4(0, 0, 0, 0);
+  else if ((((uintptr_t)row | (uintptr_t)bytes) & 3) == 0)
+    for (int64_t i = from + threadIdx.x * 4; i < to; i += 256 * 4) *reinterpret_cast<uint32_t*>(row + i) = 0;
+  else
+    for (int64_t i = from + threadIdx.x; i < to; i += 256) row[i] = 0;
+}
+}  // namespace
+
+// One launch for the states of all sequences that a step opens: 5.0 us for the six states of eight sequences of the 1b size, which took 4.6 a
+// sequence (prompts of 1000 tokens in eight sequences 583 and 559 us, of 300 in six 545 and 520).
+extern "C" int msa_seq_clear(void* const* base, const int64_t* bytes, int32_t tensors, const int64_t* slots, int32_t n_slots, void* stream) {
+  MSA_REQUIRE(tensors >= 0 && n_slots >= 0 && (tensors == 0 || (base && bytes)) && (n_slots == 0 || slots), "msa_seq_clear: null pointer");
+  for (int32_t t = 0; t < tensors; ++t)
+    MSA_REQUIRE((base[t] || bytes[t] == 0) && bytes[t] >= 0 && bytes[t] <= (int64_t)0x7fffffff * kClearBytes, "msa_seq_clear: tensor %d of %lld bytes a row", t, (long long)bytes[t]);
+  for (int32_t s = 0; s < n_slots; ++s) MSA_REQUIRE(slots[s] >= 0 && slots[s] <= 0x7fffffff, "msa_seq_clear: slot %lld", (long long)slots[s]);
+  for (int32_t t0 = 0; t0 < tensors; t0 += kClearTensors)
+    for (int32_t s0 = 0; s0 < n_slots; s0 += kClearSlots) {
+      ClearArgs a{};
+      const int nt = std::min(kClearTensors, tensors - t0), ns = std::min(kClearSlots, n_slots - s0);
+      int64_t most = 0;
+      for (int t = 0; t < nt; ++t) {
+        a.base[t] = static_cast<char*>(base[t0 + t]);
+        a.bytes[t] = bytes[t0 + t];
+        most = std::max(most, a.bytes[t]);
+      }
+      for (int s = 0; s < ns; ++s) a.slot[s] = (int32_t)slots[s0 + s];
+      if (most == 0) continue;
+      clear_kernel<<<dim3((unsigned)((most + kClearBytes - 1) / kClearBytes), nt, ns), 256, 0, as_stream(stream)>>>(a);
+      MSA_LAUNCH_CHECK();
+    }
+  return MSA_OK;
+}
+
 extern "C" int msa_seq_group_rmsnorm(const void* v, int32_t dtype, int32_t rows, int32_t n, int32_t parts, const float* w, float eps,
                                      void* out, void* stream) {
   MSA_REQUIRE(v && w && out && rows > 0 && n > 0 && parts > 0 && n % parts == 0 && parts <= 65535,

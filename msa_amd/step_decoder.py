@@ -127,9 +127,9 @@ class StepDecoder:
             if not 0 <= int(ids.min()) <= int(ids.max()) < self.config.vocab:
                 raise ValueError(f"sequence {key!r}: token outside the vocabulary")
         cache.reserve(max(cache.length.get(k, 0) + len(t) for k, t, _ in entries))
-        for key, _, _ in entries:
-            if key not in cache.slot_of:
-                cache.open(key)
+        new = [key for key in dict.fromkeys(k for k, _, _ in entries) if key not in cache.slot_of]
+        if new:
+            cache.open_all(new)
         counts, rows, at = [len(t) for _, t, _ in entries], [], 0
         for (_, ts, want) in entries:
             rows += [at + w for w in want]
