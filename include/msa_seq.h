@@ -82,9 +82,17 @@ int msa_seq_ssd_chunked(const void* xbc, int64_t xbc_stride, const void* z, int6
                         int32_t N, int32_t G, float* state, void* v, const msa_seq_batch* batch, void* workspace,
                         size_t workspace_bytes, void* stream);
 
-/* RMS norm of n columns in `parts` equal parts, times w: [rows, n] dense of `dtype`. */
+/* The same with msa_seq_group_rmsnorm of v behind it, in `parts` parts, where msa_seq_ssd_norm_folds is not 0. */
+int msa_seq_ssd_norm_folds(int32_t max_rows, int32_t n_seq, int32_t H, int32_t P, int32_t N, int32_t G, int32_t parts);
+int msa_seq_ssd_chunked_norm(const void* xbc, int64_t xbc_stride, const void* z, int64_t z_stride, const void* dt_raw, int64_t dt_stride,
+                             const float* dt_bias, const float* A_log, const float* D, int32_t dtype, int32_t H, int32_t P,
+                             int32_t N, int32_t G, float* state, void* v, const msa_seq_batch* batch, void* workspace,
+                             size_t workspace_bytes, const float* norm_w, int32_t parts, float eps, void* stream);
+
 /* Zeroes row slots[s] of every tensor: base[t], rows of bytes[t] bytes behind one another.  All arguments on the host. */
 int msa_seq_clear(void* const* base, const int64_t* bytes, int32_t tensors, const int64_t* slots, int32_t n_slots, void* stream);
+
+/* RMS norm of n columns in `parts` equal parts, times w: [rows, n] dense of `dtype`. */
 int msa_seq_group_rmsnorm(const void* v, int32_t dtype, int32_t rows, int32_t n, int32_t parts, const float* w, float eps,
                           void* out, void* stream);
 

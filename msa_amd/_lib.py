@@ -176,6 +176,9 @@ SEQ_SIGNATURES = {
     "msa_seq_ssd_chunked_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32]),
     "msa_seq_ssd_chunked": (C.c_int, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _batch,
                                       _vp, _sz, _vp]),
+    "msa_seq_ssd_norm_folds": (C.c_int, [_i32] * 7),
+    "msa_seq_ssd_chunked_norm": (C.c_int, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _batch,
+                                           _vp, _sz, _vp, _i32, _f32, _vp]),
     "msa_seq_clear": (C.c_int, [C.POINTER(_vp), C.POINTER(_i64), _i32, C.POINTER(_i64), _i32, _vp]),
     "msa_seq_group_rmsnorm": (C.c_int, [_vp, _i32, _i32, _i32, _i32, _vp, _f32, _vp, _vp]),
     "msa_seq_min_gru_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32]),

@@ -27,6 +27,8 @@ decltype(&msa_flow_linear) flow_linear;
 decltype(&msa_flow_linear_us) flow_linear_us;
 decltype(&msa_flow_workspace_bytes) flow_bytes;
 decltype(&msa_seq_clear) clear_;
+decltype(&msa_seq_ssd_chunked_norm) ssd_normed;
+decltype(&msa_seq_ssd_norm_folds) ssd_folds;
 decltype(&msa_seq_residual_norm) residual_norm_;
 decltype(&msa_seq_rms_residual) rms_residual_;
 decltype(&msa_seq_conv_silu) conv_silu_;
@@ -259,18 +261,25 @@ bool states(const at::Tensor* t, int64_t a, int64_t b, int64_t c, int64_t top) {
 }
 bool block(const at::Tensor* t, int64_t r, int64_t c, at::ScalarType type) { return rows(t) && t->size(0) == r && t->size(1) == c && t->scalar_type() == type; }
 
-// ssd(batch address, its largest slot, xbc, z, dt_raw, dt_bias, A_log, D, H, P, N, G, state, chunked): the gated output
+// ssd(batch address, its largest slot, xbc, z, dt_raw, dt_bias, A_log, D, H, P, N, G, state, chunked[, w, parts, eps]): the gated output, or its norm
+// where that is folded
 PyObject* ssd(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 14) return PyErr_Format(PyExc_TypeError, "ssd takes 14 arguments");
+  if (n != 14 && n != 17) return PyErr_Format(PyExc_TypeError, "ssd takes 14 or 17 arguments");
   Batch b;
   if (!b.get(args[0], args[1])) return PyErr_Occurred() ? nullptr : none();
   const at::Tensor *xbc = tensor(args[2]), *z = tensor(args[3]), *dt = tensor(args[4]), *bias = tensor(args[5]), *a_log = tensor(args[6]), *d = tensor(args[7]),
                    *state = tensor(args[12]);
   const long H = PyLong_AsLong(args[8]), P = PyLong_AsLong(args[9]), N = PyLong_AsLong(args[10]), G = PyLong_AsLong(args[11]);
   const bool chunked = PyObject_IsTrue(args[13]);
+  const at::Tensor* norm = n == 17 ? tensor(args[14]) : nullptr;
+  const long parts = n == 17 ? PyLong_AsLong(args[15]) : 0;
+  const double eps = n == 17 ? PyFloat_AsDouble(args[16]) : 0.0;
   if (PyErr_Occurred()) return nullptr;
   const int64_t T = b.c->rows;
+  if (n == 17 && (!chunked || !floats(norm, H * P) || !aligned(*norm) ||
+                  !ssd_folds(b.c->max_rows, b.c->n_seq, (int32_t)H, (int32_t)P, (int32_t)N, (int32_t)G, (int32_t)parts)))
+    return none();
   if (!xbc || dtype_of(*xbc) < 0 || !floats(bias, H) || !floats(a_log, H) || !floats(d, H) || !states(state, H, N, P, b.top) ||
       !block(xbc, T, H * P + 2 * G * N, xbc->scalar_type()) || !block(z, T, H * P, xbc->scalar_type()) || !block(dt, T, H, xbc->scalar_type()))
     return none();
@@ -284,6 +293,7 @@ PyObject* ssd(PyObject*, PyObject* const* args, Py_ssize_t n) {
       return fn(xbc->data_ptr(), row_stride(*xbc), z->data_ptr(), row_stride(*z), dt->data_ptr(), row_stride(*dt), f(bias), f(a_log), f(d), dtype_of(*xbc), (int32_t)H,
                 (int32_t)P, (int32_t)N, (int32_t)G, f(state), v.data_ptr(), b.c, more...);
     };
+    if (norm) return call(ssd_normed, need ? ws.data_ptr() : nullptr, need, f(norm), (int32_t)parts, (float)eps, st);
     return chunked ? call(ssd_chunked, need ? ws.data_ptr() : nullptr, need, st) : call(ssd_scan, st);
   });
   return rc == MSA_OK ? wrap(v) : PyLong_FromLong(rc);
@@ -401,7 +411,8 @@ PyObject* bind(PyObject*, PyObject* args) {
             !resolve(a, "msa_flow_linear_us", flow_linear_us) || !resolve(a, "msa_flow_workspace_bytes", flow_bytes))) return nullptr;
   if (!resolve(s, "msa_seq_clear", clear_) || !resolve(s, "msa_seq_residual_norm", residual_norm_) || !resolve(s, "msa_seq_rms_residual", rms_residual_) ||
       !resolve(s, "msa_seq_conv_silu", conv_silu_) || !resolve(s, "msa_seq_group_rmsnorm", group_rmsnorm_) ||
-      !resolve(s, "msa_seq_ssd_scan", ssd_scan) || !resolve(s, "msa_seq_ssd_chunked", ssd_chunked) ||
+      !resolve(s, "msa_seq_ssd_scan", ssd_scan) || !resolve(s, "msa_seq_ssd_chunked", ssd_chunked) || !resolve(s, "msa_seq_ssd_chunked_norm", ssd_normed) ||
+      !resolve(s, "msa_seq_ssd_norm_folds", ssd_folds) ||
       !resolve(s, "msa_seq_ssd_chunked_workspace_bytes", ssd_bytes) || !resolve(s, "msa_seq_delta_scan", delta_scan) ||
       !resolve(s, "msa_seq_delta_chunked", delta_chunked) || !resolve(s, "msa_seq_delta_chunked_workspace_bytes", delta_bytes))
     return nullptr;

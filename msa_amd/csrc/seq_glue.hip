@@ -531,7 +531,7 @@ __global__ __launch_bounds__(256) void clear_kernel(ClearArgs a) {
 }  // namespace
 
 // One launch for the states of all sequences that a step opens: 5.0 us for the six states of eight sequences of the 1b size, which took 4.6 a
-// sequence (prompts of 1000 tokens in eight sequences 583 and 559 us, of 300 in six 545 and 520).
+// sequence (steps of 1000 tokens in eight sequences 583 and 559 us).
 extern "C" int msa_seq_clear(void* const* base, const int64_t* bytes, int32_t tensors, const int64_t* slots, int32_t n_slots, void* stream) {
   MSA_REQUIRE(tensors >= 0 && n_slots >= 0 && (tensors == 0 || (base && bytes)) && (n_slots == 0 || slots), "msa_seq_clear: null pointer");
   for (int32_t t = 0; t < tensors; ++t)

@@ -40,9 +40,13 @@ struct ChunkArgs {
   float* acs;              // the running log-decay of the chunk (in powers of two)
   int64_t xbc_stride, z_stride, dt_stride;
   int32_t H, P, N, G, n_chunks, heads_per_wg;
+  const float* norm_w;     // RMS norm of a group's outputs, where it is folded
+  float norm_eps;
 };
 
 constexpr int kMaxHeads = 8;             // heads of a group per workgroup
+constexpr int kMaxNormHeads = 5;         // and with the norm of their outputs, which wait in LDS for it
+constexpr int kKeepStride = kMaxNormHeads * kPB + 8;
 
 // A wavefront per (chunk, head).  Tokens behind the sequence have dt = 0.
 template <int Q>
@@ -242,7 +246,7 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(ChunkArgs a, msa_seq_bat
   *keep = S;
 }
 
-template <int Q, int NP>
+template <int Q, int NP, bool kNorm>
 __global__ __launch_bounds__(4 * Q) void ssd_output_kernel(ChunkArgs a, msa_seq_batch b) {
   constexpr int kBS = NP + 8, kBlocks = Q / 32;
   constexpr int kBSt = Q * kBS > 2 * NP * kXS ? Q * kBS : 2 * NP * kXS;
@@ -255,6 +259,9 @@ __global__ __launch_bounds__(4 * Q) void ssd_output_kernel(ChunkArgs a, msa_seq_
   float* dts = reinterpret_cast<float*>(xs + Q * kXS);
   float* acs = dts + kMaxHeads * Q;
   float* wbs = acs + kMaxHeads * Q;                 // [heads][kBefore] weights of earlier blocks' tokens at a block's start
+  float* row_ssq = wbs + kMaxHeads * kBefore;       // [2][Q] the columns' halves' sums of squares
+  float* norm_w = row_ssq + 2 * Q;                  // [heads][kPB]
+  bf16_t* keep = reinterpret_cast<bf16_t*>(norm_w + kMaxNormHeads * kPB);        // [Q][kKeepStride] outputs
   Unit u;
   if (!unit_of<Q>(a, b, u)) return;
   const int inner = a.H * a.P;
@@ -296,6 +303,8 @@ __global__ __launch_bounds__(4 * Q) void ssd_output_kernel(ChunkArgs a, msa_seq_
     dts[i] = a.dts[u.chunk0 * Q + i];
     acs[i] = a.acs[u.chunk0 * Q + i];
   }
+  if constexpr (kNorm)
+    for (int i = threadIdx.x; i < u.heads * kPB; i += 4 * Q) norm_w[i] = i % kPB < a.P ? a.norm_w[(u.head0 + i / kPB) * a.P + i % kPB] : 0.f;
   tileB.store(Bs, kBS);
   __syncthreads();
   for (int i = threadIdx.x; i < u.heads * kBefore; i += 4 * Q) {
@@ -325,6 +334,7 @@ __global__ __launch_bounds__(4 * Q) void ssd_output_kernel(ChunkArgs a, msa_seq_
     z_at[q] = p < a.P ? zin : kOutside;
     v_at[q] = p < a.P ? vin : kOutside;
   }
+  float ssq = 0.f;                                  // of token t's outputs, this lane's
   for (int hh = 0; hh < u.heads; ++hh) {
     const int head = u.head0 + hh;
     __syncthreads();                                // the last reads of B or of the head before, and the weights
@@ -409,28 +419,53 @@ __global__ __launch_bounds__(4 * Q) void ssd_output_kernel(ChunkArgs a, msa_seq_
       const float zv[4] = {bf16lo(zw[q].x), bf16hi(zw[q].x), bf16lo(zw[q].y), bf16hi(zw[q].y)};
 #pragma unroll
       for (int x = 0; x < 4; ++x) y[x] = (acc[4 * q + x] + Dh * xv[x]) * silu_f(zv[x]);
-      __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])}, rs_v, v_at[q], head * a.P * 2, 0);
+      const u32x2_t o = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+      if constexpr (kNorm) {
+        ssq += (bf16lo(o.x) * bf16lo(o.x) + bf16hi(o.x) * bf16hi(o.x)) + (bf16lo(o.y) * bf16lo(o.y) + bf16hi(o.y) * bf16hi(o.y));
+        *reinterpret_cast<u32x2_t*>(keep + t * kKeepStride + hh * kPB + pb + 8 * q + 4 * half) = o;
+      } else {
+        __builtin_amdgcn_raw_buffer_store_b64(o, rs_v, v_at[q], head * a.P * 2, 0);
+      }
+    }
+  }
+  if constexpr (kNorm) {
+    ssq += __shfl_xor(ssq, 32);
+    if (half == 0) row_ssq[(pb >> 5) * Q + t] = ssq;
+    __syncthreads();
+    const int units = u.heads * (kPB / 8);           // of eight columns, whole rows behind one another
+    for (int i = threadIdx.x; i < Q * units; i += 4 * Q) {
+      const int row = i / units, at = (i - row * units) * 8, hh = at / kPB, p = at % kPB;
+      const float inv = 1.0f / sqrtf((row_ssq[row] + row_ssq[Q + row]) / (float)(u.heads * a.P) + a.norm_eps);
+      float y[8], w[8];
+      load_vec<bf16_t, 8>(keep + row * kKeepStride + at, y);
+      load_vec<float, 8>(norm_w + at, w);
+      uint32_t o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = pack_bf16x2(y[2 * e] * (inv * w[2 * e]), y[2 * e + 1] * (inv * w[2 * e + 1]));
+      __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{o[0], o[1], o[2], o[3]}, rs_v, p < a.P ? (row * inner + hh * a.P + p) * 2 : kOutside, u.head0 * a.P * 2, 0);
     }
   }
 }
 
 int chunk_tokens(int32_t N) { return N <= 128 ? 128 : 64; }
+constexpr int kNormRounds = 1;
 
 template <int Q, int NP>
 int launch_chunked(ChunkArgs a, const msa_seq_batch& b, hipStream_t st) {
   constexpr int tile = Q * (NP + 8), x = Q * kXS, state = 2 * NP * kXS;
   constexpr int lds2 = (tile > 2 * x ? tile : 2 * x) * 2 + kMaxHeads * Q * 4;
   constexpr int lds3 = ((tile > state ? tile : state) + x) * 2 + kMaxHeads * (2 * Q + (Q / 32) * (Q / 32 - 1) * 16) * 4;
-  static_assert(lds2 <= 160 * 1024 && lds3 <= 160 * 1024, "tiles of a chunk must fit LDS");
+  constexpr int lds_norm = lds3 + (2 * Q + kMaxNormHeads * kPB) * 4 + Q * kKeepStride * 2;
+  static_assert(lds2 <= 160 * 1024 && lds3 <= 160 * 1024 && (Q == 64 || lds_norm <= 160 * 1024), "tiles of a chunk must fit LDS");
   // as many heads per workgroup as leave a launch two workgroups per compute unit
   const int per_group = a.H / a.G, blocks = (a.P + kPB - 1) / kPB;
   auto sets = [&](int h) { return (per_group + h - 1) / h; };
   int heads = std::min(kMaxHeads, per_group);
   while (heads > 1 && (int64_t)a.n_chunks * b.n_seq * a.G * blocks * sets(heads) < 2 * device_compute_units()) --heads;
   a.heads_per_wg = (per_group + sets(heads) - 1) / sets(heads);
-  static std::atomic<int> raised2{0}, raised3{0};
+  static std::atomic<int> raised2{0}, raised3{0}, raised_norm{0};
   MSA_HIP(raise_dynamic_lds_limit(raised2, reinterpret_cast<const void*>(ssd_local_kernel<Q, NP>), lds2));
-  MSA_HIP(raise_dynamic_lds_limit(raised3, reinterpret_cast<const void*>(ssd_output_kernel<Q, NP>), lds3));
+  MSA_HIP(raise_dynamic_lds_limit(raised3, reinterpret_cast<const void*>(ssd_output_kernel<Q, NP, false>), lds3));
   ssd_decay_kernel<Q><<<dim3((a.H + 3) / 4, a.n_chunks, b.n_seq), 256, 0, st>>>(a, b);
   MSA_LAUNCH_CHECK();
   const dim3 grid((unsigned)(a.G * blocks * sets(a.heads_per_wg)), a.n_chunks, b.n_seq);
@@ -438,7 +473,16 @@ int launch_chunked(ChunkArgs a, const msa_seq_batch& b, hipStream_t st) {
   MSA_LAUNCH_CHECK();
   ssd_carry_kernel<Q><<<dim3((a.N * a.P / 4 + 255) / 256, a.H, b.n_seq), 256, 0, st>>>(a, b);
   MSA_LAUNCH_CHECK();
-  ssd_output_kernel<Q, NP><<<grid, 4 * Q, lds3, st>>>(a, b);
+  if constexpr (Q == 128) {
+    if (a.norm_w) {
+      MSA_HIP(raise_dynamic_lds_limit(raised_norm, reinterpret_cast<const void*>(ssd_output_kernel<Q, NP, true>), lds_norm));
+      a.heads_per_wg = per_group;
+      ssd_output_kernel<Q, NP, true><<<dim3((unsigned)a.G, a.n_chunks, b.n_seq), 4 * Q, lds_norm, st>>>(a, b);
+      MSA_LAUNCH_CHECK();
+      return MSA_OK;
+    }
+  }
+  ssd_output_kernel<Q, NP, false><<<grid, 4 * Q, lds3, st>>>(a, b);
   MSA_LAUNCH_CHECK();
   return MSA_OK;
 }
@@ -451,10 +495,16 @@ extern "C" size_t msa_seq_ssd_chunked_workspace_bytes(int32_t max_rows, int32_t 
   return (size_t)n_seq * ((max_rows + Q - 1) / Q) * H * ((size_t)N * P + 2 * Q) * sizeof(float);
 }
 
-extern "C" int msa_seq_ssd_chunked(const void* xbc, int64_t xbc_stride, const void* z, int64_t z_stride, const void* dt_raw,
+// The norm is folded where a workgroup per group and chunk fills the chip: it has all heads of a group then.
+extern "C" int msa_seq_ssd_norm_folds(int32_t max_rows, int32_t n_seq, int32_t H, int32_t P, int32_t N, int32_t G, int32_t parts) {
+  return max_rows > 0 && n_seq > 0 && H > 0 && G > 0 && H % G == 0 && parts == G && H / G <= kMaxNormHeads && P >= 8 && P <= kPB && P % 8 == 0 && N > 0 && N <= 128 &&
+         N % 8 == 0 && (int64_t)((max_rows + chunk_tokens(N) - 1) / chunk_tokens(N)) * n_seq * G >= kNormRounds * device_compute_units();
+}
+
+static int ssd_chunked(const void* xbc, int64_t xbc_stride, const void* z, int64_t z_stride, const void* dt_raw,
                                    int64_t dt_stride, const float* dt_bias, const float* A_log, const float* D, int32_t dtype, int32_t H,
                                    int32_t P, int32_t N, int32_t G, float* state, void* v, const msa_seq_batch* batch, void* workspace,
-                                   size_t workspace_bytes, void* stream) {
+                                   size_t workspace_bytes, void* stream, const float* norm_w, float norm_eps) {
   MSA_CHECK_BATCH(batch, "msa_seq_ssd_chunked");
   MSA_REQUIRE(dtype == MSA_BF16, "msa_seq_ssd_chunked: bf16 only");
   MSA_REQUIRE(xbc && z && dt_raw && dt_bias && A_log && D && state && v && workspace, "msa_seq_ssd_chunked: null pointer");
@@ -473,10 +523,26 @@ extern "C" int msa_seq_ssd_chunked(const void* xbc, int64_t xbc_stride, const vo
   uint32_t* states = static_cast<uint32_t*>(workspace);
   float* dts = reinterpret_cast<float*>(states + (int64_t)batch->n_seq * chunks * H * N * P);
   const ChunkArgs a{(const bf16_t*)xbc, (const bf16_t*)z, (const bf16_t*)dt_raw, dt_bias, A_log, D, state, (bf16_t*)v, states, dts,
-                    dts + (int64_t)batch->n_seq * chunks * H * Q, xbc_stride, z_stride, dt_stride, H, P, N, G, chunks, 1};
+                    dts + (int64_t)batch->n_seq * chunks * H * Q, xbc_stride, z_stride, dt_stride, H, P, N, G, chunks, 1, norm_w, norm_eps};
   hipStream_t st = as_stream(stream);
   if (N <= 32) return launch_chunked<128, 32>(a, *batch, st);
   if (N <= 64) return launch_chunked<128, 64>(a, *batch, st);
   if (N <= 128) return launch_chunked<128, 128>(a, *batch, st);
   return launch_chunked<64, 256>(a, *batch, st);
+}
+
+extern "C" int msa_seq_ssd_chunked(const void* xbc, int64_t xbc_stride, const void* z, int64_t z_stride, const void* dt_raw,
+                                   int64_t dt_stride, const float* dt_bias, const float* A_log, const float* D, int32_t dtype, int32_t H,
+                                   int32_t P, int32_t N, int32_t G, float* state, void* v, const msa_seq_batch* batch, void* workspace,
+                                   size_t workspace_bytes, void* stream) {
+  return ssd_chunked(xbc, xbc_stride, z, z_stride, dt_raw, dt_stride, dt_bias, A_log, D, dtype, H, P, N, G, state, v, batch, workspace, workspace_bytes, stream, nullptr, 0.f);
+}
+extern "C" int msa_seq_ssd_chunked_norm(const void* xbc, int64_t xbc_stride, const void* z, int64_t z_stride, const void* dt_raw,
+                                        int64_t dt_stride, const float* dt_bias, const float* A_log, const float* D, int32_t dtype, int32_t H,
+                                        int32_t P, int32_t N, int32_t G, float* state, void* v, const msa_seq_batch* batch, void* workspace,
+                                        size_t workspace_bytes, const float* norm_w, int32_t parts, float eps, void* stream) {
+  MSA_CHECK_BATCH(batch, "msa_seq_ssd_chunked_norm");
+  MSA_REQUIRE(norm_w && v && (((uintptr_t)norm_w | (uintptr_t)v) & 15) == 0 && msa_seq_ssd_norm_folds(batch->max_rows, batch->n_seq, H, P, N, G, parts),
+              "msa_seq_ssd_chunked_norm: H=%d P=%d N=%d G=%d in %d parts is not folded", H, P, N, G, parts);
+  return ssd_chunked(xbc, xbc_stride, z, z_stride, dt_raw, dt_stride, dt_bias, A_log, D, dtype, H, P, N, G, state, v, batch, workspace, workspace_bytes, stream, norm_w, eps);
 }

@@ -75,9 +75,8 @@ class Mamba2Mixer:
         c = self.c
         chunked = (xbc.dtype == torch.bfloat16 and batch.max_rows >= seq_ops.SSD_CHUNKED_ROWS and c.state % 8 == 0
                    and c.state <= 256 and c.vdim % 8 == 0)
-        v = seq_ops.ssd(xbc, z, dt, self.dt_bias, self.A_log, self.D, c.heads, c.vdim, c.state, c.groups, state["ssm"], batch,
-                        chunked=chunked)
-        return seq_ops.group_rmsnorm(v, self.norm, c.norm_groups, self.eps)
+        return seq_ops.ssd_norm(xbc, z, dt, self.dt_bias, self.A_log, self.D, c.heads, c.vdim, c.state, c.groups, state["ssm"], batch,
+                                chunked, self.norm, c.norm_groups, self.eps)
 
     def mix(self, proj, state, batch):
         z, xbc, dt = self._columns(proj)

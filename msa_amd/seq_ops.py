@@ -328,6 +328,20 @@ def ssd(xbc, z, dt_raw, dt_bias, A_log, D, H: int, P: int, N: int, G: int, state
     return v
 
 
+SSD_NORM_ROWS = 2048       # rows of a step below which no norm is folded
+
+
+def ssd_norm(xbc, z, dt_raw, dt_bias, A_log, D, H: int, P: int, N: int, G: int, state, batch: StepBatch, chunked: bool, w, parts: int, eps: float):
+    """:func:`group_rmsnorm` of :func:`ssd`, in the launch that makes the outputs where that folds it."""
+    if chunked and batch.rows >= SSD_NORM_ROWS and xbc.is_cuda:
+        got = ops.host().ssd(batch.address, batch.top, xbc, z, dt_raw, dt_bias, A_log, D, H, P, N, G, state, True, w, parts, eps)
+        if type(got) is int:
+            _check(got, "msa_seq_ssd_chunked_norm")
+        if got is not None:
+            return got
+    return group_rmsnorm(ssd(xbc, z, dt_raw, dt_bias, A_log, D, H, P, N, G, state, batch, chunked), w, parts, eps)
+
+
 def group_rmsnorm(v: torch.Tensor, w: torch.Tensor, parts: int, eps: float) -> torch.Tensor:
     """RMS norm of ``v [rows, n]`` in ``parts`` equal parts, times ``w``."""
     if v.is_cuda:
