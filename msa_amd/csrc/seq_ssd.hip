@@ -3,13 +3,13 @@
 // a_t = sum of the chunk's log-decays up to t, inside a chunk
 //   y_t = exp(a_t) S_in^T C_t + sum_{s <= t} exp(a_t - a_s) dt_s (B_s . C_t) x_s,   S_out = exp(a_end) S_in + S_loc,
 //   S_loc = sum_s exp(a_end - a_s) dt_s B_s x_s^T.
-//   (1) ssd_decay_kernel   dt and a_t of every token and head
-//   (2) ssd_local_kernel   every chunk's S_loc
-//   (3) ssd_carry_kernel   the chunk-to-chunk recurrence, element by element; leaves each chunk's S_in in its place
-//   (4) ssd_output_kernel  the outputs
-// A workgroup of (2) and (4) takes one chunk and several heads of one group, whose B, C and B . C^T are the same: those are read /
+//   (1) ssd_local_kernel   dt and a_t of every token and head, every chunk's S_loc
+//   (2) ssd_carry_kernel   the chunk-to-chunk recurrence, element by element; leaves each chunk's S_in in its place
+//   (3) ssd_output_kernel  the outputs
+// (dt and a_t in a launch of their own, in front, took 4 to 6 us; here they are formed while the first tiles are on their way)
+// A workgroup of (1) and (3) takes one chunk and several heads of one group, whose B, C and B . C^T are the same: those are read /
 // formed once and stay in registers; a head's x and S_in are fetched while the head before is multiplied.  (Walking over the chunks
-// with the state in accumulators instead of (2) and (3) moves fewer bytes but is a chain of latencies: faster only with several
+// with the state in accumulators instead of (1) and (2) moves fewer bytes but is a chain of latencies: faster only with several
 // hundred heads in the step, 1.7 times slower with 32.)
 // Operands that carry decays or states are fp32 values: they enter the bf16 products as a high and a low part (two products
 // with about 16 bits of mantissa), so only x, B and C, which are bf16 to begin with, set the precision.
@@ -47,31 +47,6 @@ struct ChunkArgs {
 constexpr int kMaxHeads = 8;             // heads of a group per workgroup
 constexpr int kMaxNormHeads = 5;         // and with the norm of their outputs, which wait in LDS for it
 constexpr int kKeepStride = kMaxNormHeads * kPB + 8;
-
-// A wavefront per (chunk, head).  Tokens behind the sequence have dt = 0.
-template <int Q>
-__global__ __launch_bounds__(256) void ssd_decay_kernel(ChunkArgs a, msa_seq_batch b) {
-  const int lane = threadIdx.x & 63, head = blockIdx.x * 4 + (threadIdx.x >> 6), s = blockIdx.z;
-  const int lo = b.cu[s], t0 = blockIdx.y * Q, rows = min(Q, b.cu[s + 1] - lo - t0);
-  if (head >= a.H || rows <= 0) return;
-  const float rate = -expf(a.A_log[head]) * kLog2e, bias = a.dt_bias[head];
-  const int64_t at = (((int64_t)s * a.n_chunks + blockIdx.y) * a.H + head) * Q;
-  float before = 0.f;
-#pragma unroll
-  for (int t = lane; t < Q; t += 64) {
-    const float dt = t < rows ? softplus_f(bf16_to_f32(a.dt_raw[(int64_t)(lo + t0 + t) * a.dt_stride + head]) + bias) : 0.f;
-    float ac = rate * dt;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const float up = __shfl_up(ac, o);
-      if (lane >= o) ac += up;
-    }
-    ac += before;
-    before = __shfl(ac, 63);
-    a.dts[at + t] = dt;
-    a.acs[at + t] = ac;
-  }
-}
 
 // All global accesses inside the loops below go through buffer resources whose extent is the valid rows: what lies outside
 // reads as zero and is not written, nothing is conditional, and the compiler can count the loads and stores in flight (behind a
@@ -117,7 +92,7 @@ __device__ __forceinline__ uint32_t pack_split(float v) {
   return hi | ((uint32_t)f32_to_bf16(v - bf16_to_f32((bf16_t)hi)) << 16);
 }
 
-// What a workgroup of kernels (2) and (4) works on.
+// What a workgroup of kernels (1) and (3) works on.
 struct Unit {
   int head0, heads, grp, p0, lo, t0, rows, row0;
   int64_t chunk0;          // chunk index of head0
@@ -152,18 +127,50 @@ __global__ __launch_bounds__(4 * Q) void ssd_local_kernel(ChunkArgs a, msa_seq_b
   if (!unit_of<Q>(a, b, u)) return;
   const int inner = a.H * a.P, stride = (int)a.xbc_stride;
   const bf16_t* src = a.xbc + (int64_t)u.row0 * a.xbc_stride;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, l16 = lane & 15;
+  constexpr int kTurns = (kMaxHeads + kWaves - 1) / kWaves, kPer = Q / 64;
+  bf16_t raw[kTurns][kPer];
+#pragma unroll
+  for (int k = 0; k < kTurns; ++k)
+#pragma unroll
+    for (int j = 0; j < kPer; ++j)
+      raw[k][j] = a.dt_raw[(int64_t)(u.row0 + min(lane + 64 * j, u.rows - 1)) * a.dt_stride + min(u.head0 + wave + k * kWaves, a.H - 1)];
   RowTile<Q, NP, 4 * Q> tb;
   RowTile<Q, kPB, 4 * Q> tx;
   const typename RowTile<Q, kPB, 4 * Q>::Offsets off_x(stride, a.P - u.p0);
   tb.load(typename RowTile<Q, NP, 4 * Q>::Offsets(stride, a.N), src + inner + u.grp * a.N, stride, u.rows, a.N);
   tx.load(off_x, src + u.head0 * a.P + u.p0, stride, u.rows, a.P - u.p0);
-  for (int i = threadIdx.x; i < u.heads * Q; i += 4 * Q) {      // weights of the tokens at the chunk's end
-    const float* ac = a.acs + u.chunk0 * Q;
-    ws[i] = a.dts[u.chunk0 * Q + i] * __builtin_amdgcn_exp2f(ac[i / Q * Q + Q - 1] - ac[i]);
+  // dt, the running log-decay and the tokens' weights at the chunk's end, a wavefront a head; tokens behind the sequence have dt = 0
+#pragma unroll
+  for (int k = 0; k < kTurns; ++k) {
+    const int hh = wave + k * kWaves, head = min(u.head0 + hh, a.H - 1);
+    const float rate = -expf(a.A_log[head]) * kLog2e, bias = a.dt_bias[head];
+    float dt[kPer], ac[kPer], before = 0.f;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      dt[j] = lane + 64 * j < u.rows ? softplus_f(bf16_to_f32(raw[k][j]) + bias) : 0.f;
+      ac[j] = rate * dt[j];
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const float up = __shfl_up(ac[j], o);
+        if (lane >= o) ac[j] += up;
+      }
+      ac[j] += before;
+      before = __shfl(ac[j], 63);
+    }
+    if (hh >= u.heads) continue;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int64_t at = (u.chunk0 + hh) * Q + lane + 64 * j;
+      if (u.p0 == 0) {
+        a.dts[at] = dt[j];
+        a.acs[at] = ac[j];
+      }
+      ws[hh * Q + lane + 64 * j] = dt[j] * __builtin_amdgcn_exp2f(before - ac[j]);
+    }
   }
   tb.store(Bs, kBS);
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, l16 = lane & 15;
   const int r = 8 * half + (l16 >> 2), c = (lane & 16) + (l16 & 3) * 4;
   bf16x8_t bf[kTiles][Q / 16];                      // B^T operands of this wavefront's tiles, for every head
   int out_at[kTiles];
@@ -466,8 +473,6 @@ int launch_chunked(ChunkArgs a, const msa_seq_batch& b, hipStream_t st) {
   static std::atomic<int> raised2{0}, raised3{0}, raised_norm{0};
   MSA_HIP(raise_dynamic_lds_limit(raised2, reinterpret_cast<const void*>(ssd_local_kernel<Q, NP>), lds2));
   MSA_HIP(raise_dynamic_lds_limit(raised3, reinterpret_cast<const void*>(ssd_output_kernel<Q, NP, false>), lds3));
-  ssd_decay_kernel<Q><<<dim3((a.H + 3) / 4, a.n_chunks, b.n_seq), 256, 0, st>>>(a, b);
-  MSA_LAUNCH_CHECK();
   const dim3 grid((unsigned)(a.G * blocks * sets(a.heads_per_wg)), a.n_chunks, b.n_seq);
   ssd_local_kernel<Q, NP><<<grid, 4 * Q, lds2, st>>>(a, b);
   MSA_LAUNCH_CHECK();
