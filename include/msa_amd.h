@@ -401,8 +401,8 @@ int msa_block_linear(const void* x, int64_t ldx, int64_t T, int32_t K, const voi
 /* The same where one round of larger tiles, or of pieces of K of them, fills the chip (some hundred tokens).  ws: msa_flow_workspace_bytes
  * bytes, or fewer or NULL, without which K stays whole.  msa_flow_linear_us: about what it takes, 0 where msa_block_linear, msa_tile_linear
  * or the vendor's product are the better form. */
-float msa_flow_linear_us(int64_t T, int32_t K, int32_t N);
-size_t msa_flow_workspace_bytes(int64_t T, int32_t K, int32_t N);
+float msa_flow_linear_us(int64_t T, int32_t K, int32_t N, int32_t mode);
+size_t msa_flow_workspace_bytes(int64_t T, int32_t K, int32_t N, int32_t mode);
 int msa_flow_linear(const void* x, int64_t ldx, int64_t T, int32_t K, const void* w, int32_t N, const msa_tile_end* end, void* out,
                     int64_t ldo, void* ws, size_t ws_bytes, void* stream);
 /* msa_qk_norm_rope for a decode step (one new token per sample, N = B) fused with msa_cache_append: the

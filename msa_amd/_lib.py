@@ -72,8 +72,8 @@ SIGNATURES = {
     "msa_tile_workspace_bytes": (_sz, [_i64, _i32, _i32]),
     "msa_block_linear_us": (C.c_float, [_i64, _i32, _i32]),
     "msa_block_linear": (C.c_int, [_vp, _i64, _i64, _i32, _vp, _i32, _vp, _vp, _i64, _vp]),
-    "msa_flow_linear_us": (C.c_float, [_i64, _i32, _i32]),
-    "msa_flow_workspace_bytes": (_sz, [_i64, _i32, _i32]),
+    "msa_flow_linear_us": (C.c_float, [_i64, _i32, _i32, _i32]),
+    "msa_flow_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32]),
     "msa_flow_linear": (C.c_int, [_vp, _i64, _i64, _i32, _vp, _i32, _vp, _vp, _i64, _vp, _sz, _vp]),
     "msa_tile_linear": (C.c_int, [_vp, _i64, _i64, _i32, _vp, _i32, _vp, _vp, _i64, _vp, _sz, _vp]),
     "msa_qk_norm_rope_append": (C.c_int, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _f32, _vp, _vp, _i32, _i32, _i32,

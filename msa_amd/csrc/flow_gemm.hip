@@ -227,8 +227,10 @@ constexpr Tile kTile[] = {{64, 32, .175f, .06f}, {64, 64, .208f, .83f}, {64, 96,
                           {128, 160, .534f, 3.23f}, {192, 128, .651f, 3.27f}, {192, 160, .71f, 3.91f}, {192, 192, .886f, 3.99f}, {256, 128, .848f, 3.77f}};
 
 struct Plan { int tile, pieces; float us; };
-// The cheapest tile and pieces of one round; none (us = 0) where there is none.
-Plan plan_of(int64_t T, int32_t K, int64_t N, bool whole) {
+// The cheapest tile and pieces of one round; none (us = 0) where there is none.  A gated unit or gelu costs kEnd for every output of a lane, of
+// which nothing is hidden where a compute unit has one tile (2000 x 1024 x 4096 in tiles of 256 x 128 21.5 us, with gelu 27.3).
+constexpr float kEnd = 0.04f;
+Plan plan_of(int64_t T, int32_t K, int64_t N, bool end, bool whole) {
   const int units = device_compute_units(), steps = K / kK;
   Plan best{0, 1, 0.f};
   for (int v = 0; v < (int)(sizeof(kTile) / sizeof(kTile[0])); ++v)
@@ -236,31 +238,35 @@ Plan plan_of(int64_t T, int32_t K, int64_t N, bool whole) {
       const int64_t wgs = ((T + kTile[v].t - 1) / kTile[v].t) * ((N + kTile[v].n - 1) / kTile[v].n) * p;
       if (wgs > units) break;
       const float bytes = ((float)(N + T) * (float)K + (float)T * (float)N) * 2.f;
-      float us = 2.8f + std::max((float)((steps + p - 1) / p) * kTile[v].step + kTile[v].end, bytes / 6.7e6f * (float)units / (float)wgs);
+      const float ends = end && p == 1 ? kEnd * (float)(kTile[v].n * kTile[v].t / kThreads) : 0.f;
+      float us = 2.8f + ends + std::max((float)((steps + p - 1) / p) * kTile[v].step + kTile[v].end, bytes / 6.7e6f * (float)units / (float)wgs);
       if (p > 1) us += 3.5f + (float)p * (float)T * (float)N * 8.f / 5.6e6f;
       if (best.us == 0.f || us < best.us) best = {v, p, us};
     }
   return best;
 }
 
-// Where this form is taken: one round, faster than block_gemm.hip's by its own measure.  With fewer tokens the weights' way is all there is,
+// Where this form is taken: one round, faster than block_gemm.hip's by its own measure up to the length that form is asked for (behind it the
+// vendor's product is the other choice: 700 x 4096 x 2560 25.0 and 22.7, 700 x 5120 x 2560 36.0 and 35.3).  With fewer tokens the weights' way is all there is,
 // which more workgroups of smaller tiles do better, except for long rows, which are cut (us, the faster other form and here: 100 x 2560 x 12288
 // 22.9 and 24.4, 48 x 2560 x 8480 16.2 and 18.3, but 48 x 9728 x 2560 20.4 and 17.1, 20 x 5120 x 2560 15.1 and 12.1).  More tokens and shorter rows
-// were not measured.
+// were not measured.  (Behind 2304 tokens full rounds are level with the vendor's, 4096 x 3072 x 1024 29.6 and 29.2, 8192 47.0 and 50.6; tiles of
+// 256 x 160 to 256 x 256 are behind it, 850 x 2560 x 12368 53.9 and 65.3.)
+constexpr float kBlockUs = 23.f;
 constexpr int64_t kLeastTokens = 17, kTokens = 160, kMostTokens = 2304;
 constexpr int32_t kLong = 3072, kShort = 1024;
 
 }  // namespace
 
-extern "C" float msa_flow_linear_us(int64_t T, int32_t K, int32_t N) {
+extern "C" float msa_flow_linear_us(int64_t T, int32_t K, int32_t N, int32_t mode) {
   if (T < kLeastTokens || T > kMostTokens || K < kShort || K > 32768 || K % kK != 0 || N < 16 || N >= (1 << 20) || (T < kTokens && K < kLong)) return 0.f;
-  const float us = plan_of(T, K, N, false).us;
-  return us < 0.99f * msa_block_linear_us(T, K, N) ? us : 0.f;
+  const float us = plan_of(T, K, N, mode != MSA_TILE_STORE, false).us, block = msa_block_linear_us(T, K, N);
+  return us < 0.99f * block || block > kBlockUs ? us : 0.f;
 }
 
-extern "C" size_t msa_flow_workspace_bytes(int64_t T, int32_t K, int32_t N) {
+extern "C" size_t msa_flow_workspace_bytes(int64_t T, int32_t K, int32_t N, int32_t mode) {
   if (T <= 0 || K < kK || N <= 0) return 0;
-  const Plan plan = plan_of(T, K, N, false);
+  const Plan plan = plan_of(T, K, N, mode != MSA_TILE_STORE, false);
   return plan.us > 0.f && plan.pieces > 1 ? (size_t)plan.pieces * (size_t)T * (size_t)N * sizeof(float) : 0;
 }
 
@@ -275,8 +281,9 @@ extern "C" int msa_flow_linear(const void* x, int64_t ldx, int64_t T, int32_t K,
               "msa_flow_linear: row strides %lld and %lld", (long long)ldx, (long long)ldo);
   MSA_REQUIRE(mode != MSA_TILE_GELU || (end->gelu_n >= 0 && end->gelu_n <= N && end->gelu_n % 8 == 0), "msa_flow_linear: gelu_n=%d", end->gelu_n);
   MSA_REQUIRE((((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)workspace) & 15) == 0, "msa_flow_linear: operands must be 16-byte aligned");
-  Plan plan = plan_of(T, K, N, false);
-  if (plan.pieces > 1 && (workspace == nullptr || workspace_bytes < msa_flow_workspace_bytes(T, K, N))) plan = plan_of(T, K, N, true);
+  const bool with_end = mode != MSA_TILE_STORE;
+  Plan plan = plan_of(T, K, N, with_end, false);
+  if (plan.pieces > 1 && (workspace == nullptr || workspace_bytes < msa_flow_workspace_bytes(T, K, N, mode))) plan = plan_of(T, K, N, with_end, true);
   if (plan.us == 0.f) return msa_block_linear(x, ldx, T, K, w, N, end, out, ldo, stream);      // (more than a round)
   const FlowArgs a{static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), static_cast<bf16_t*>(out), static_cast<float*>(workspace), ldx, ldo,
                    (int32_t)T, K, N, 0, 0, 1, plan.pieces, *end};

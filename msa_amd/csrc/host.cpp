@@ -126,10 +126,10 @@ PyObject* flow(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!(x->scalar_type() == at::kBFloat16 && w->scalar_type() == at::kBFloat16 && w->is_contiguous() && w->size(1) == K && K <= 32768 && N % 16 == 0 &&
         N < 1 << 20 && (x->is_contiguous() || (x->stride(1) == 1 && x->stride(0) % 8 == 0 && K <= x->stride(0) && x->stride(0) < 1 << 21)) && aligned(*x) &&
         aligned(*w) && w->device() == x->device() && plain(x) && plain(w) && gelu_n % 8 == 0 && gelu_n <= N &&
-        flow_linear_us(T, (int32_t)K, (int32_t)N) > 0.f))
+        flow_linear_us(T, (int32_t)K, (int32_t)N, (int32_t)mode) > 0.f))
     return none();
   at::Tensor out = at::empty({T, mode == MSA_TILE_GLU ? N / 2 : N}, x->options().requires_grad(false)), ws;
-  const size_t need = flow_bytes(T, (int32_t)K, (int32_t)N);
+  const size_t need = flow_bytes(T, (int32_t)K, (int32_t)N, (int32_t)mode);
   if (need) ws = at::empty({(int64_t)need}, x->options().requires_grad(false).dtype(at::kByte));
   const auto st = stream();
   const int rc = run([&] {

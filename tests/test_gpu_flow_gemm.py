@@ -30,7 +30,7 @@ def _flow(x, w, pieces=True, **end):
     glu, gelu_n = end.get("glu"), end.get("gelu_n", 0)
     mode = _lib.TILE_GLU if glu else _lib.TILE_GELU if gelu_n else _lib.TILE_STORE
     out = torch.full((T + 1, (N // 2 if glu else N) + 8), 7.0, device="cuda").bfloat16()
-    need = lib.msa_flow_workspace_bytes(T, K, N) if pieces else 0
+    need = lib.msa_flow_workspace_bytes(T, K, N, mode) if pieces else 0
     ws = torch.full((need + 64,), 9, dtype=torch.uint8, device="cuda")
     e = _lib.TileEnd(mode, gelu_n, *(glu or (0.0, 0.0, 0.0)))
     _lib.check(lib.msa_flow_linear(x.data_ptr(), x.stride(0), T, K, w.data_ptr(), N, C.byref(e), out.data_ptr(), out.shape[1], ws.data_ptr() if need else None, need,
@@ -76,7 +76,7 @@ def test_route(monkeypatch):
     from msa_amd import ops, seq_ops
     taken, inner = [], ops.flow_linear
     monkeypatch.setattr(ops, "flow_linear", lambda x, w, **k: (lambda y: (taken.append(y is not None), y)[1])(inner(x, w, **k)))
-    for T, K, N, here in ((450, 2560, 2560, True), (100, 9728, 2560, True), (700, 9728, 2560, True), (1000, 9728, 2560, False), (1000, 1024, 6144, True),
+    for T, K, N, here in ((450, 2560, 2560, True), (100, 9728, 2560, True), (700, 9728, 2560, True), (1000, 9728, 2560, False), (1000, 1024, 6144, True), (1500, 1024, 6144, True),
                           (16, 9728, 2560, False), (159, 2560, 12288, False), (2305, 1024, 3072, False), (64, 1024, 1024, False), (450, 2592, 2560, False)):
         print(f"[flow_gemm] route T={T} K={K} N={N}", flush=True)
         x, w, want = _operands(T, K, N, 3)
