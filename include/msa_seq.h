@@ -305,6 +305,18 @@ typedef struct {
   void* h;
 } msa_rows_embed;
 int msa_rows_linear_embed(const msa_rows_args* args, int32_t epilogue, const msa_rows_embed* embed, void* stream);
+/* MSA_ROWS_PLAIN beside msa_seq_latent_append of other rows (bf16), in one launch where neither has a form of its own. */
+typedef struct {
+  const void* in;
+  int64_t in_stride;
+  const float* w;
+  void* cache;
+  int64_t Lcap;
+  const msa_seq_batch* batch;
+  float eps;
+  int32_t rank;
+} msa_rows_append;
+int msa_rows_linear_append(const msa_rows_args* args, const msa_rows_append* append, void* stream);
 
 #ifdef __cplusplus
 }

@@ -134,6 +134,11 @@ class RowsEmbed(C.Structure):
     _fields_ = [("tokens", _vp), ("table", _vp), ("vocab", _i64), ("x_out", _vp), ("h", _vp)]
 
 
+class RowsAppend(C.Structure):
+    """``msa_rows_append``."""
+    _fields_ = [("in_", _vp), ("in_stride", _i64), ("w", _vp), ("cache", _vp), ("Lcap", _i64), ("batch", _vp), ("eps", _f32), ("rank", _i32)]
+
+
 class QKRopeArgs(C.Structure):
     """``msa_qk_rope_args``."""
     _fields_ = [("q", _vp), ("k", _vp), ("v", _vp), ("q_stride", _i64), ("k_stride", _i64), ("v_stride", _i64), ("q_norm", _vp),
@@ -203,6 +208,7 @@ SEQ_SIGNATURES = {
     "msa_rows_linear": (C.c_int, [C.POINTER(RowsArgs), _i32, _vp]),
     "msa_rows_linear_post": (C.c_int, [C.POINTER(RowsArgs), _i32, C.POINTER(RowsPost), _vp]),
     "msa_rows_linear_embed": (C.c_int, [C.POINTER(RowsArgs), _i32, C.POINTER(RowsEmbed), _vp]),
+    "msa_rows_linear_append": (C.c_int, [C.POINTER(RowsArgs), C.POINTER(RowsAppend), _vp]),
     "msa_rows_linear_final": (C.c_int, [C.POINTER(RowsArgs), C.POINTER(RowsPost), _vp, _vp]),
 }
 # entry points of include/msa_amd.h that libmsa_seq.so holds too (the error text is per library)

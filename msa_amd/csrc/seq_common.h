@@ -88,6 +88,35 @@ __device__ __forceinline__ void store_vec(T* p, const float (&v)[VEC]) {
   }
 }
 
+// A row's normed latent to its place in the cache, by a wavefront.
+template <typename T, int VEC>
+__device__ __forceinline__ void append_latent(const T* in, int64_t stride, const float* w, float eps, int32_t rank, T* cache, int64_t Lcap,
+                                              const msa_seq_batch& b, int row) {
+  const int lane = threadIdx.x & 63, s = b.row_seq[row];
+  const int64_t p = b.pos[s] + (row - b.cu[s]);
+  const T* src = in + row * stride;
+  T* dst = cache + ((int64_t)b.slot[s] * Lcap + p) * rank;
+  float ssq = 0.f;
+  for (int i = lane * VEC; i < rank; i += 64 * VEC) {
+    float x[VEC];
+    load_vec<T, VEC>(src + i, x);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) ssq += x[e] * x[e];
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) ssq += __shfl_xor(ssq, o);
+  if (p >= Lcap) return;
+  const float inv = 1.0f / sqrtf(ssq / (float)rank + eps);
+  for (int i = lane * VEC; i < rank; i += 64 * VEC) {
+    float x[VEC], g[VEC];
+    load_vec<T, VEC>(src + i, x);
+    load_vec<float, VEC>(w + i, g);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) x[e] *= inv * g[e];
+    store_vec<T, VEC>(dst + i, x);
+  }
+}
+
 // Host side: vectors are usable when every given address is 16-byte aligned and every stride a multiple of `n` elements.
 static inline bool vec_ok(int n, std::initializer_list<const void*> ps, std::initializer_list<int64_t> strides) {
   for (const void* p : ps)

@@ -197,36 +197,12 @@ __global__ __launch_bounds__(256) void group_rmsnorm_kernel(const T* __restrict_
   }
 }
 
-// One wavefront per row.
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void latent_append_kernel(const T* __restrict__ in, int64_t stride, const float* __restrict__ w,
                                                             float eps, int32_t rank, T* __restrict__ cache, int64_t Lcap,
                                                             msa_seq_batch b) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (row >= b.rows) return;
-  const int s = b.row_seq[row];
-  const int64_t p = b.pos[s] + (row - b.cu[s]);
-  const T* src = in + row * stride;
-  T* dst = cache + ((int64_t)b.slot[s] * Lcap + p) * rank;
-  float ssq = 0.f;
-  for (int i = lane * VEC; i < rank; i += 64 * VEC) {
-    float x[VEC];
-    load_vec<T, VEC>(src + i, x);
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) ssq += x[e] * x[e];
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) ssq += __shfl_xor(ssq, o);
-  if (p >= Lcap) return;
-  const float inv = 1.0f / sqrtf(ssq / (float)rank + eps);
-  for (int i = lane * VEC; i < rank; i += 64 * VEC) {
-    float x[VEC], g[VEC];
-    load_vec<T, VEC>(src + i, x);
-    load_vec<float, VEC>(w + i, g);
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) x[e] *= inv * g[e];
-    store_vec<T, VEC>(dst + i, x);
-  }
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row < b.rows) append_latent<T, VEC>(in, stride, w, eps, rank, cache, Lcap, b, row);
 }
 
 // A workgroup per row: x' = x + rms_norm(y) w, and the next sublayer's operand.  A row of up to 256 * kKeep vectors stays in

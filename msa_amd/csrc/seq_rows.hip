@@ -136,7 +136,7 @@ struct Finish<MSA_ROWS_GLU> {
 };
 
 template <int EPI, int R>
-__global__ __launch_bounds__(kMaxWaves * 64) void rows_linear_kernel(msa_rows_args a, int32_t rows_per_wg) {
+__device__ __forceinline__ void rows_linear(const msa_rows_args& a, int32_t rows_per_wg) {
   constexpr int J = kVectors<R>, kUnit = 32 * J;
   extern __shared__ __align__(16) float part[];   // [waves][R][64][4]
   const int tid = threadIdx.x, lane = tid & 63, waves = blockDim.x >> 6;
@@ -243,6 +243,20 @@ __global__ __launch_bounds__(kMaxWaves * 64) void rows_linear_kernel(msa_rows_ar
   }
 }
 
+template <int EPI, int R>
+__global__ __launch_bounds__(kMaxWaves * 64) void rows_linear_kernel(msa_rows_args a, int32_t rows_per_wg) {
+  rows_linear<EPI, R>(a, rows_per_wg);
+}
+
+// The same beside the appending of the rows' latents, which needs nothing of the products: the last column of workgroups does that.
+template <int R>
+__global__ __launch_bounds__(kMaxWaves * 64) void rows_append_kernel(msa_rows_args a, int32_t rows_per_wg, msa_rows_append p, msa_seq_batch b) {
+  if (blockIdx.x + 1 < gridDim.x) return rows_linear<MSA_ROWS_PLAIN, R>(a, rows_per_wg);
+  const int waves = blockDim.x >> 6;
+  for (int row = blockIdx.y * waves + (threadIdx.x >> 6); row < b.rows; row += gridDim.y * waves)
+    append_latent<bf16_t, 8>(static_cast<const bf16_t*>(p.in), p.in_stride, p.w, p.eps, p.rank, static_cast<bf16_t*>(p.cache), p.Lcap, b, row);
+}
+
 // What rows_ring.h's kernel does with a product: the same ends, and the minimal gated recurrence, whose three sums of a channel
 // are three consecutive items of a workgroup.
 template <int EPI>
@@ -333,9 +347,12 @@ int launch_ring(const msa_rows_args& a, hipStream_t st, const msa_rows_post* pos
 }
 
 template <int EPI, int R>
-int launch_rows(const msa_rows_args& a, int waves, int rows_per_wg, hipStream_t st) {
+int launch_rows(const msa_rows_args& a, int waves, int rows_per_wg, hipStream_t st, const msa_rows_append* append = nullptr) {
   const size_t lds = (size_t)waves * R * 256 * sizeof(float);       // at most 48 KB
-  rows_linear_kernel<EPI, R><<<dim3((a.N + rows_per_wg - 1) / rows_per_wg, a.groups), waves * 64, lds, st>>>(a, rows_per_wg);
+  if (EPI == MSA_ROWS_PLAIN && append)
+    rows_append_kernel<R><<<dim3((a.N + rows_per_wg - 1) / rows_per_wg + 1, a.groups), waves * 64, lds, st>>>(a, rows_per_wg, *append, *append->batch);
+  else
+    rows_linear_kernel<EPI, R><<<dim3((a.N + rows_per_wg - 1) / rows_per_wg, a.groups), waves * 64, lds, st>>>(a, rows_per_wg);
   MSA_LAUNCH_CHECK();
   return MSA_OK;
 }
@@ -344,7 +361,7 @@ int launch_rows(const msa_rows_args& a, int waves, int rows_per_wg, hipStream_t 
 
 namespace {
 int rows_entry(const msa_rows_args& a, int32_t epilogue, const msa_rows_post* post, void* stream, const float* next_w = nullptr,
-               const msa_rows_embed* embed = nullptr) {
+               const msa_rows_embed* embed = nullptr, const msa_rows_append* append = nullptr) {
   MSA_REQUIRE(a.x && a.w && a.M > 0 && a.M <= 16 && a.N > 0 && a.K > 0 && a.K % 8 == 0 && a.groups > 0 && a.groups <= 65535,
               "msa_rows_linear: M=%d (1..16) N=%d K=%d (a multiple of 8) groups=%d", a.M, a.N, a.K, a.groups);
   MSA_REQUIRE(a.x_stride >= (int64_t)a.K * a.groups && a.x_stride % 8 == 0 && a.x_stride * 32 < ((int64_t)1 << 30) &&
@@ -417,8 +434,8 @@ int rows_entry(const msa_rows_args& a, int32_t epilogue, const msa_rows_post* po
     }
   }
   switch (epilogue * 4 + R) {
-    case MSA_ROWS_PLAIN * 4 + 1: return launch_rows<MSA_ROWS_PLAIN, 1>(a, waves, rows_per_wg, st);
-    case MSA_ROWS_PLAIN * 4 + 2: return launch_rows<MSA_ROWS_PLAIN, 2>(a, waves, rows_per_wg, st);
+    case MSA_ROWS_PLAIN * 4 + 1: return launch_rows<MSA_ROWS_PLAIN, 1>(a, waves, rows_per_wg, st, append);
+    case MSA_ROWS_PLAIN * 4 + 2: return launch_rows<MSA_ROWS_PLAIN, 2>(a, waves, rows_per_wg, st, append);
     case MSA_ROWS_F32 * 4 + 1: return launch_rows<MSA_ROWS_F32, 1>(a, waves, rows_per_wg, st);
     case MSA_ROWS_F32 * 4 + 2: return launch_rows<MSA_ROWS_F32, 2>(a, waves, rows_per_wg, st);
     case MSA_ROWS_RESIDUAL * 4 + 1: return launch_rows<MSA_ROWS_RESIDUAL, 1>(a, waves, rows_per_wg, st);
@@ -437,6 +454,18 @@ int rows_entry(const msa_rows_args& a, int32_t epilogue, const msa_rows_post* po
 extern "C" int msa_rows_linear(const msa_rows_args* args, int32_t epilogue, void* stream) {
   MSA_REQUIRE(args != nullptr, "msa_rows_linear: null arguments");
   return rows_entry(*args, epilogue, nullptr, stream);
+}
+
+// One launch for the latents and the products of the queries with the heads' matrices, which follow one another in a step but need nothing
+// of each other (whole steps, us: one sequence of the 1b size 165.0 and 161.6, eight 183.4 and 180.3, sixteen of the 4b size 434 and 430).
+extern "C" int msa_rows_linear_append(const msa_rows_args* args, const msa_rows_append* append, void* stream) {
+  MSA_REQUIRE(args && append, "msa_rows_linear_append: null arguments");
+  const msa_rows_append& p = *append;
+  MSA_CHECK_BATCH(p.batch, "msa_rows_linear_append");
+  MSA_REQUIRE(p.in && p.w && p.cache && p.rank > 0 && p.in_stride >= p.rank && p.Lcap > 0, "msa_rows_linear_append: bad arguments");
+  if (!takes_ring(*args, MSA_ROWS_PLAIN) && vec_ok(8, {p.in, p.w, p.cache}, {p.in_stride, p.rank})) return rows_entry(*args, MSA_ROWS_PLAIN, nullptr, stream, nullptr, nullptr, append);
+  if (const int rc = msa_seq_latent_append(p.in, p.in_stride, p.w, p.eps, MSA_BF16, p.rank, p.cache, p.Lcap, p.batch, stream); rc != MSA_OK) return rc;
+  return rows_entry(*args, MSA_ROWS_PLAIN, nullptr, stream);
 }
 
 // The residual step is folded where its operands are few: every workgroup reads all of them, six bytes an element where the product

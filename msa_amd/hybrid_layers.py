@@ -152,18 +152,22 @@ class LatentAttention:
         c = self.c
         return c.dim % 8 == 0 and c.kv_rank % 8 == 0 and (c.heads * c.vdim) % 8 == 0
 
-    def _absorbed(self, q, cache, batch):
+    def _absorbed(self, q, latents, cache, batch):
         c = self.c
-        qa = head_linear(q, self.uk_t, c.heads)
+        if q.dtype == torch.bfloat16 and c.dim % 8 == 0 and q.stride(0) % 8 == 0 and batch.rows <= seq_ops.MAX_ROWS:
+            qa = seq_ops.rows_linear_append(q, self.uk_t, c.heads, latents, self.c_norm, self.eps, cache, batch)
+        else:
+            seq_ops.latent_append(latents, self.c_norm, self.eps, cache, batch)
+            qa = head_linear(q, self.uk_t, c.heads)
         ctx = seq_ops.latent_attn(qa.view(batch.rows, c.heads, c.kv_rank), cache, self.sink, c.scale, batch, batch.max_keys)
         return head_linear(ctx.view(batch.rows, -1), self.uv, c.heads)
 
     def mix(self, proj, state, batch):
         c, cache = self.c, state["latent"]
-        q = proj[:, :c.heads * c.dim]
-        seq_ops.latent_append(proj[:, self.c_at:self.c_at + c.kv_rank], self.c_norm, self.eps, cache, batch)
+        q, latents = proj[:, :c.heads * c.dim], proj[:, self.c_at:self.c_at + c.kv_rank]
         if batch.max_rows <= self.ABSORB_ROWS or not seq_ops.flash_ok(q.dtype, c.dim, c.vdim, c.scale) or proj.stride(0) % 8:
-            return self._absorbed(q, cache, batch)
+            return self._absorbed(q, latents, cache, batch)
+        seq_ops.latent_append(latents, self.c_norm, self.eps, cache, batch)
         ends = [p + n for p, n in zip(batch.positions, batch.counts)]
         lat = cache[batch.slots[0], :ends[0]] if batch.n_seq == 1 else torch.cat([cache[s, :e] for s, e in zip(batch.slots, ends)])
         return seq_ops.flash(q, seq_ops.product(lat, self.uk), seq_ops.product(lat, self.uv), batch.key_off, self.sink, c.scale, c.heads, batch)
@@ -171,8 +175,7 @@ class LatentAttention:
     def decode(self, w, hs, h, state, batch):
         c, n_b = self.c, self.w_in.shape[0]
         out = seq_ops.rows_linear(hs, w, x_b=h, n_b=n_b)
-        seq_ops.latent_append(out[:, self.c_at:self.c_at + c.kv_rank], self.c_norm, self.eps, state["latent"], batch)
-        return self._absorbed(out[:, :c.heads * c.dim], state["latent"], batch), out[:, n_b:]
+        return self._absorbed(out[:, :c.heads * c.dim], out[:, self.c_at:self.c_at + c.kv_rank], state["latent"], batch), out[:, n_b:]
 
 
 def _pad_cols(w: torch.Tensor, n: int) -> torch.Tensor:

@@ -458,13 +458,17 @@ def _latent_cache(cache: torch.Tensor, rank: int, dtype, batch: StepBatch) -> in
     return cache.shape[1]
 
 
-def latent_append(x: torch.Tensor, w: torch.Tensor, eps: float, cache: torch.Tensor, batch: StepBatch) -> None:
-    """RMS-normed rows of ``x [rows, rank]`` go to the latent cache at their positions."""
-    rank = x.shape[1]
-    _f32(rank, w)
-    Lcap = _latent_cache(cache, rank, x.dtype, batch)
+def _append_capacity(x, w, cache, batch: StepBatch) -> int:
+    _f32(x.shape[1], w)
+    Lcap = _latent_cache(cache, x.shape[1], x.dtype, batch)
     if batch.max_keys > Lcap:
         raise ValueError(f"latent cache of {Lcap} rows cannot take {batch.max_keys} tokens")
+    return Lcap
+
+
+def latent_append(x: torch.Tensor, w: torch.Tensor, eps: float, cache: torch.Tensor, batch: StepBatch) -> None:
+    """RMS-normed rows of ``x [rows, rank]`` go to the latent cache at their positions."""
+    rank, Lcap = x.shape[1], _append_capacity(x, w, cache, batch)
     _check(_lib.load_seq().msa_seq_latent_append(ptr(x), _rows(x), ptr(w), eps, dtype_code(x.dtype), rank, ptr(cache), Lcap, batch.ref,
                                                  _stream()), "msa_seq_latent_append")
 
@@ -674,6 +678,19 @@ def rows_linear(x, w, groups: int = 1, x_b=None, n_b: Optional[int] = None, gelu
     out = torch.empty((x.shape[0], w.shape[0]), dtype=torch.bfloat16, device=x.device)
     a.out, a.out_stride, a.gelu_n = ptr(out), out.shape[1], gelu_n
     _run_rows(a, _lib.ROWS_PLAIN)
+    return out
+
+
+def rows_linear_append(x, w, groups: int, latents, norm, eps: float, cache, batch: StepBatch) -> torch.Tensor:
+    """:func:`rows_linear` beside :func:`latent_append` of ``latents``."""
+    a = _rows_args(x, w, groups)
+    if latents.dtype != torch.bfloat16 or latents.shape[0] != batch.rows:
+        raise ValueError("rows_linear_append: bf16 latents [rows, rank]")
+    Lcap = _append_capacity(latents, norm, cache, batch)
+    out = torch.empty((x.shape[0], w.shape[0]), dtype=torch.bfloat16, device=x.device)
+    a.out, a.out_stride = ptr(out), out.shape[1]
+    p = _lib.RowsAppend(ptr(latents), _rows(latents), ptr(norm), ptr(cache), Lcap, batch.address, eps, latents.shape[1])
+    _check(_lib.load_seq().msa_rows_linear_append(C.byref(a), C.byref(p), _stream()), "msa_rows_linear_append")
     return out
 
 
