@@ -168,6 +168,10 @@ typedef struct {
 int msa_seq_kv_attn(const msa_kv_attn_args* args, int32_t dtype, const msa_seq_batch* batch, void* stream);
 size_t msa_seq_kv_decode_workspace_bytes(const msa_kv_attn_args* args, int32_t rows);
 int msa_seq_kv_decode(const msa_kv_attn_args* args, const msa_seq_batch* batch, void* workspace, size_t workspace_bytes, void* stream);
+/* msa_seq_qk_rope_append (bf16) with msa_seq_kv_decode of its queries behind it (args->q == rope->q_out, which may stay unwritten), in one
+ * launch less for single rows of heads of 128 that are rotated whole. */
+int msa_seq_kv_decode_rope(const msa_kv_attn_args* args, const msa_qk_rope_args* rope, const msa_seq_batch* batch, void* workspace,
+                           size_t workspace_bytes, void* stream);
 
 /* Delta rule with a decay per key channel.  qkv rows [q: G D | k: G D | v: H E] (after convolution and silu); per head h, with
  * q and k those of key head h G / H as unit vectors (1e-6 under the root), q times D^-1/2:

@@ -197,6 +197,7 @@ SEQ_SIGNATURES = {
     "msa_seq_qk_rope_append": (C.c_int, [C.POINTER(QKRopeArgs), _i32, _batch, _vp]),
     "msa_seq_kv_attn": (C.c_int, [C.POINTER(KVAttnArgs), _i32, _batch, _vp]),
     "msa_seq_kv_decode_workspace_bytes": (_sz, [C.POINTER(KVAttnArgs), _i32]),
+    "msa_seq_kv_decode_rope": (C.c_int, [C.POINTER(KVAttnArgs), C.POINTER(QKRopeArgs), _batch, _vp, _sz, _vp]),
     "msa_seq_kv_decode": (C.c_int, [C.POINTER(KVAttnArgs), _batch, _vp, _sz, _vp]),
     "msa_seq_delta_scan": (C.c_int, [C.POINTER(DeltaArgs), _i32, _batch, _vp]),
     "msa_seq_delta_step": (C.c_int, [C.POINTER(DeltaArgs), C.POINTER(DeltaLow), _batch, _vp]),

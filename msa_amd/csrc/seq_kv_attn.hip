@@ -1,7 +1,7 @@
 // Grouped-query attention over cached keys and values: what prepares queries, keys and values (norms, rotation, cache rows), and
 // the forms for decoding and short portions.  (Long bf16 portions go through flash_sink_kernel of seq_attn.hip, straight over
 // the caches.)
-//   qk_rope_append_kernel  a workgroup per row; L lanes per head, eight dimensions a lane (or a wavefront per head, any sizes)
+//   qk_rope_append_kernel  (single rows of heads of 128 do without) a workgroup per row; L lanes per head, eight dimensions a lane (or a wavefront per head, any sizes)
 //   kv_attn_kernel         any sizes and type: a workgroup per (row, head), fp32 arithmetic throughout
 //   kv_split_kernel        bf16: a workgroup per (row, key head, range of keys).  Its wavefronts take key ranges of their own and
 //                          work without a barrier: scores S^T = K Q^T straight from the rows in registers, whose accumulator
@@ -228,6 +228,7 @@ struct SplitArgs {
   float* part_ml;                        // [rows, n_split, H, 2]
   float scale_log2e;
   int32_t n_split;
+  msa_qk_rope_args rope;   // kRope: what prepares the queries
 };
 
 // DP / EP: D and E padded to 64, 128 or 256.
@@ -235,7 +236,10 @@ struct SplitArgs {
 // which leaves the caches to the keys, whose lines take two requests, where there are enough of both for that to matter (8 key heads
 // of 128, us without and with, none of it in a cache before: 16 sequences behind 2048 to 4096 tokens 52 / 45, 4 of them 21.2 / 19.1,
 // 32 behind 128 to 256, 33 MB, 9.7 / 9.0; but 16 of these 7.5 / 7.9, 4 behind 500 to 1000 11.0 / 11.6, one behind 256 6.5 / 6.9).
-template <int DP, int EP, bool kOnce>
+// kRope (D = DP, E = EP, D / 2 pairs, a row a sequence): the queries come as they are projected, and so do the row's own key and value.  A
+// lane's dimensions of a head hold both members of its pairs, so a wavefront norms and turns its queries itself while its first keys are
+// on their way; the one that has the range's last key takes that from the row instead of the cache, and appends it.
+template <int DP, int EP, bool kOnce, bool kRope>
 __global__ __launch_bounds__(256) void kv_split_kernel(SplitArgs p, msa_seq_batch b) {
   constexpr int kVS = EP + 8, kUnits = EP / 8, kVP = kStepKeys * kUnits / 64, kK = DP / 32, kC = EP / 16;
   constexpr int kOS = EP + 4;                                    // row stride of the sums at the end
@@ -280,9 +284,64 @@ __global__ __launch_bounds__(256) void kv_split_kernel(SplitArgs p, msa_seq_batc
 #pragma unroll
     for (int i = 0; i < kVP; ++i) r.v[i] = __builtin_amdgcn_raw_buffer_load_b128(rv, v_at[i], 0, kOnce ? 2 : 0);
   };
-  fetch(cur, first);
   bf16x8_t qf[kK];
-  {
+  u32x4_t own_k[kRope ? kK : 1], own_v = {0u, 0u, 0u, 0u};       // of the row's own key: like a fragment's rows, 16 bytes of lane % 16
+  const bool takes = kRope && p.rope.k && first < last && last == steps;
+  if constexpr (kRope) {
+    static_assert(DP == 128 && EP == 128, "lanes' shares of a row");
+    __shared__ float2 cs[DP / 2];
+    const msa_qk_rope_args& r = p.rope;
+    const bf16_t* q = static_cast<const bf16_t*>(r.q) + row * r.q_stride + (int64_t)(h0 + min(l16, heads - 1)) * DP + 8 * g;
+    const bf16_t* k = takes ? static_cast<const bf16_t*>(r.k) + row * r.k_stride + kvh * DP + 8 * g : q;
+    const float* kn = takes ? r.k_norm : r.q_norm;
+    float x[kK][8], y[kK][8], qw[kK][8], kw[kK][8];
+    const double freq = tid < DP / 2 ? r.freqs[tid] : 0.0;
+#pragma unroll
+    for (int kk = 0; kk < kK; ++kk) {
+      load_vec<bf16_t, 8>(q + 32 * kk, x[kk]);
+      load_vec<bf16_t, 8>(k + 32 * kk, y[kk]);
+      load_vec<float, 8>(r.q_norm + 32 * kk + 8 * g, qw[kk]);
+      load_vec<float, 8>(kn + 32 * kk + 8 * g, kw[kk]);
+    }
+    if (takes) own_v = *reinterpret_cast<const u32x4_t*>(static_cast<const bf16_t*>(r.v) + row * r.v_stride + kvh * EP + l16 * 8);
+    __builtin_amdgcn_sched_barrier(0);                           // (in front of the cache's rows: loads return in order)
+    fetch(cur, first);
+    if (tid < DP / 2) cs[tid] = cos_sin((double)pos * freq);
+    __syncthreads();
+    auto packed = [](const float (&x)[8]) { return u32x4_t{pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]), pack_bf16x2(x[4], x[5]), pack_bf16x2(x[6], x[7])}; };
+    auto norm_and_turn = [&](float (&x)[kK][8], const float (&w)[kK][8]) {
+      float ssq = 0.f;
+#pragma unroll
+      for (int kk = 0; kk < kK; ++kk)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ssq += x[kk][e] * x[kk][e];
+      const float inv = 1.0f / sqrtf(lanes_sum(ssq) / (float)DP + r.eps);
+#pragma unroll
+      for (int kk = 0; kk < kK / 2; ++kk)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float2 c = cs[32 * kk + 8 * g + e];
+          const float s = x[kk][e] * (inv * w[kk][e]), t = x[kk + kK / 2][e] * (inv * w[kk + kK / 2][e]);
+          x[kk][e] = s * c.x - t * c.y;
+          x[kk + kK / 2][e] = t * c.x + s * c.y;
+        }
+    };
+    norm_and_turn(x, qw);
+    norm_and_turn(y, kw);
+#pragma unroll
+    for (int kk = 0; kk < kK; ++kk) {
+      qf[kk] = __builtin_bit_cast(bf16x8_t, l16 < heads ? packed(x[kk]) : u32x4_t{0u, 0u, 0u, 0u});
+      own_k[kk] = packed(y[kk]);
+    }
+    if (takes && blockIdx.y % tiles == 0 && pos < a.Lcap) {
+      char* to_k = const_cast<char*>(kc) + (int64_t)(n_keys - 1) * krow + 16 * g;
+      if (l16 == 0)
+#pragma unroll
+        for (int kk = 0; kk < kK; ++kk) *reinterpret_cast<u32x4_t*>(to_k + 64 * kk) = own_k[kk];
+      if (g == 0) *reinterpret_cast<u32x4_t*>(const_cast<char*>(vc) + (int64_t)(n_keys - 1) * vrow + 16 * l16) = own_v;
+    }
+  } else {
+    fetch(cur, first);
     const bf16_t* q = static_cast<const bf16_t*>(a.q) + ((int64_t)row * a.H + h0 + l16) * a.D + 8 * g;
 #pragma unroll
     for (int kk = 0; kk < kK; ++kk) {
@@ -296,6 +355,16 @@ __global__ __launch_bounds__(256) void kv_split_kernel(SplitArgs p, msa_seq_batc
   float m = kNoScore, l = 0.f;           // of head l16: m the same in its four lanes, l each lane's own keys
   for (int step = first; step < last; ++step) {
     fetch(next, step + 1);
+    if constexpr (kRope)
+      if (takes && step + 1 == steps) {                          // (the cache's row is not there yet)
+        const int own = n_keys - 1 - step * kStepKeys;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int kk = 0; kk < kK; ++kk) cur.k[t][kk] = l16 + 16 * t == own ? own_k[kk] : cur.k[t][kk];
+#pragma unroll
+        for (int i = 0; i < kVP; ++i) cur.v[i] = 4 * i + g == own ? own_v : cur.v[i];
+      }
     floatx4_t sc[2] = {floatx4_t{0.f, 0.f, 0.f, 0.f}, floatx4_t{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int kk = 0; kk < kK; ++kk)
@@ -449,14 +518,14 @@ int kv_splits(const msa_kv_attn_args& a, int32_t rows) {
   return (int)std::min<int64_t>(std::min<int64_t>(kMaxSplits, (steps + 7) / 8), std::max<int64_t>(1, (2 * device_compute_units() + blocks - 1) / blocks));
 }
 
-template <int DP, int EP>
+template <int DP, int EP, bool kRope = false>
 int launch_split(const SplitArgs& p, const msa_seq_batch& b, hipStream_t st) {
   const msa_kv_attn_args& a = p.a;
   const int tiles = (a.H / a.G + kHeadTile - 1) / kHeadTile;
   const dim3 grid(p.n_split, a.G * tiles, b.rows);
   const int64_t bytes = kv_span(a) * b.rows * a.G * (a.D + a.E) * 2;
-  if (b.max_rows == 1 && tiles == 1 && bytes >= kOnceBytes) kv_split_kernel<DP, EP, true><<<grid, 256, 0, st>>>(p, b);
-  else kv_split_kernel<DP, EP, false><<<grid, 256, 0, st>>>(p, b);
+  if (b.max_rows == 1 && tiles == 1 && bytes >= kOnceBytes) kv_split_kernel<DP, EP, true, kRope><<<grid, 256, 0, st>>>(p, b);
+  else kv_split_kernel<DP, EP, false, kRope><<<grid, 256, 0, st>>>(p, b);
   MSA_LAUNCH_CHECK();
   if (p.n_split > 1) {
     const int64_t items = (int64_t)b.rows * a.H;
@@ -475,9 +544,7 @@ int check_kv(const msa_kv_attn_args* a, const char* who) {
 
 }  // namespace
 
-extern "C" int msa_seq_qk_rope_append(const msa_qk_rope_args* args, int32_t dtype, const msa_seq_batch* batch, void* stream) {
-  MSA_CHECK_BATCH(batch, "msa_seq_qk_rope_append");
-  MSA_CHECK_DTYPE(dtype, "msa_seq_qk_rope_append");
+static int check_rope(const msa_qk_rope_args* args) {
   MSA_REQUIRE(args && args->q && args->q_norm && args->q_out, "msa_seq_qk_rope_append: null pointer");
   const msa_qk_rope_args& a = *args;
   MSA_REQUIRE(a.H > 0 && a.G > 0 && a.D > 0 && a.D <= 512 && a.E > 0 && a.n_pairs >= 0 && 2 * a.n_pairs <= a.D && a.n_pairs <= kMaxPairs && (!a.n_pairs || a.freqs),
@@ -485,6 +552,14 @@ extern "C" int msa_seq_qk_rope_append(const msa_qk_rope_args* args, int32_t dtyp
   MSA_REQUIRE(a.q_stride >= (int64_t)a.H * a.D, "msa_seq_qk_rope_append: query stride");
   MSA_REQUIRE(!a.k || (a.v && a.k_norm && a.k_cache && a.v_cache && a.Lcap > 0 && a.k_stride >= (int64_t)a.G * a.D && a.v_stride >= (int64_t)a.G * a.E),
               "msa_seq_qk_rope_append: key and value arguments");
+  return MSA_OK;
+}
+
+extern "C" int msa_seq_qk_rope_append(const msa_qk_rope_args* args, int32_t dtype, const msa_seq_batch* batch, void* stream) {
+  MSA_CHECK_BATCH(batch, "msa_seq_qk_rope_append");
+  MSA_CHECK_DTYPE(dtype, "msa_seq_qk_rope_append");
+  if (const int rc = check_rope(args); rc != MSA_OK) return rc;
+  const msa_qk_rope_args& a = *args;
   return dtype == MSA_BF16 ? launch_prepare<bf16_t>(a, *batch, as_stream(stream)) : launch_prepare<float>(a, *batch, as_stream(stream));
 }
 
@@ -508,7 +583,7 @@ extern "C" size_t msa_seq_kv_decode_workspace_bytes(const msa_kv_attn_args* args
   return splits == 1 ? 0 : (size_t)rows * splits * args->H * (args->E + 2) * sizeof(float);
 }
 
-extern "C" int msa_seq_kv_decode(const msa_kv_attn_args* args, const msa_seq_batch* batch, void* workspace, size_t workspace_bytes, void* stream) {
+static int kv_decode(const msa_kv_attn_args* args, const msa_qk_rope_args* rope, const msa_seq_batch* batch, void* workspace, size_t workspace_bytes, void* stream) {
   MSA_CHECK_BATCH(batch, "msa_seq_kv_decode");
   const int rc = check_kv(args, "msa_seq_kv_decode");
   if (rc != MSA_OK) return rc;
@@ -526,10 +601,29 @@ extern "C" int msa_seq_kv_decode(const msa_kv_attn_args* args, const msa_seq_bat
   }
   const int splits = kv_splits(a, batch->rows);
   float* part_o = static_cast<float*>(workspace);
-  const SplitArgs p{a, part_o, splits == 1 ? nullptr : part_o + (int64_t)batch->rows * splits * a.H * a.E, a.scale * kLog2e, splits};
+  const SplitArgs p{a, part_o, splits == 1 ? nullptr : part_o + (int64_t)batch->rows * splits * a.H * a.E, a.scale * kLog2e, splits, rope ? *rope : msa_qk_rope_args{}};
   hipStream_t st = as_stream(stream);
+  if (rope) return launch_split<128, 128, true>(p, *batch, st);
   const int big = std::max(a.D, a.E);
   if (big <= 64) return launch_split<64, 64>(p, *batch, st);
   if (big <= 128) return launch_split<128, 128>(p, *batch, st);
   return launch_split<256, 256>(p, *batch, st);
+}
+
+extern "C" int msa_seq_kv_decode(const msa_kv_attn_args* args, const msa_seq_batch* batch, void* workspace, size_t workspace_bytes, void* stream) {
+  return kv_decode(args, nullptr, batch, workspace, workspace_bytes, stream);
+}
+
+extern "C" int msa_seq_kv_decode_rope(const msa_kv_attn_args* args, const msa_qk_rope_args* rope, const msa_seq_batch* batch, void* workspace, size_t workspace_bytes,
+                                      void* stream) {
+  MSA_CHECK_BATCH(batch, "msa_seq_kv_decode_rope");
+  if (const int rc = check_rope(rope); rc != MSA_OK) return rc;
+  const msa_qk_rope_args& r = *rope;
+  MSA_REQUIRE(args && r.H == args->H && r.G == args->G && r.D == args->D && r.E == args->E && r.q_out == args->q && (!r.k || (r.k_cache == args->k_cache && r.v_cache == args->v_cache && r.Lcap == args->Lcap)),
+              "msa_seq_kv_decode_rope: two different layers");
+  const bool folds = batch->max_rows == 1 && r.D == 128 && r.E == 128 && 2 * r.n_pairs == r.D && vec_ok(8, {r.q, r.q_norm}, {r.q_stride}) &&
+                     (!r.k || vec_ok(8, {r.k, r.v, r.k_norm}, {r.k_stride, r.v_stride}));
+  if (folds) return kv_decode(args, rope, batch, workspace, workspace_bytes, stream);
+  if (const int rc = msa_seq_qk_rope_append(rope, MSA_BF16, batch, stream); rc != MSA_OK) return rc;
+  return kv_decode(args, nullptr, batch, workspace, workspace_bytes, stream);
 }

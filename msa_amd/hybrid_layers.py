@@ -286,8 +286,10 @@ class RotaryAttention:
         c, kc, vc = self.c, state["k"], state["v"]
         cols = lambda i, n: proj[:, self.at[i]:self.at[i] + n]
         own = {} if self.kv_from is not None else {"k": cols(1, c.kv_heads * c.dim), "v": cols(2, c.kv_heads * c.vdim), "k_norm": self.k_norm}
-        q = seq_ops.qk_rope_append(cols(0, c.heads * c.dim), self.q_norm, self.freqs, self.eps, kc, vc, batch, **own)
         gate, chunk = cols(len(self.at) - 1, c.heads), c.mask.size if c.mask is not None else 0
+        if batch.max_rows == 1:
+            return seq_ops.rope_kv_attn(cols(0, c.heads * c.dim), self.q_norm, self.freqs, self.eps, kc, vc, c.scale, batch, chunk, gate, **own)
+        q = seq_ops.qk_rope_append(cols(0, c.heads * c.dim), self.q_norm, self.freqs, self.eps, kc, vc, batch, **own)
         if batch.max_rows > self.SPLIT_ROWS and seq_ops.flash_ok(q.dtype, c.dim, c.vdim, c.scale):
             rows = kc.shape[0] * kc.shape[1]
             return seq_ops.flash(q.view(batch.rows, -1), kc.view(rows, -1), vc.view(rows, -1), batch.cache_rows(kc.shape[1]), None, c.scale,

@@ -555,6 +555,13 @@ def _kv_caches(k_cache, v_cache, dtype, batch: StepBatch):
 def qk_rope_append(q, q_norm, freqs, eps: float, k_cache, v_cache, batch: StepBatch, k=None, v=None, k_norm=None) -> torch.Tensor:
     """Normed and rotated queries ``[rows, H, D]`` of ``q [rows, H D]``; with ``k [rows, G D]`` and ``v [rows, G E]`` the normed and
     rotated keys and the values go to the caches at their positions.  ``freqs`` (fp64): radians per position of each pair."""
+    c, out, _ = _rope_args(q, q_norm, freqs, eps, k_cache, v_cache, batch, k, v, k_norm)
+    _check(_lib.load_seq().msa_seq_qk_rope_append(C.byref(c), dtype_code(q.dtype), batch.ref, _stream()), "msa_seq_qk_rope_append")
+    return out
+
+
+def _rope_args(q, q_norm, freqs, eps, k_cache, v_cache, batch, k, v, k_norm):
+    """Arguments of :func:`qk_rope_append`, its queries, and what has to live as long."""
     Lcap, G, D, E = _kv_caches(k_cache, v_cache, q.dtype, batch)
     H = q.shape[1] // D
     _f32(D, q_norm)
@@ -567,12 +574,11 @@ def qk_rope_append(q, q_norm, freqs, eps: float, k_cache, v_cache, batch: StepBa
     out = torch.empty((batch.rows, H, D), dtype=q.dtype, device=q.device)
     c = _lib.QKRopeArgs(ptr(q), ptr(k), ptr(v), _rows(q), _rows(k) if k is not None else 0, _rows(v) if k is not None else 0, ptr(q_norm),
                         ptr(k_norm), ptr(freqs), ptr(out), ptr(k_cache), ptr(v_cache), Lcap, H, G, D, E, freqs.numel(), eps)
-    _check(_lib.load_seq().msa_seq_qk_rope_append(C.byref(c), dtype_code(q.dtype), batch.ref, _stream()), "msa_seq_qk_rope_append")
-    return out
+    return c, out, (q, k, v)
 
 
 def kv_attn(q: torch.Tensor, k_cache, v_cache, scale: float, batch: StepBatch, chunk: int = 0, gate: Optional[torch.Tensor] = None,
-            split: Optional[bool] = None) -> torch.Tensor:
+            split: Optional[bool] = None, rope=None) -> torch.Tensor:
     """Causal attention ``[rows, H E]`` of prepared queries ``q [rows, H, D]`` over the caches, a few rows a sequence, with the chunk
     mask and the gate of :func:`flash`.  bf16 of aligned sizes takes the split matrix-core kernel (``split`` chooses by hand)."""
     _dense(q)
@@ -591,10 +597,21 @@ def kv_attn(q: torch.Tensor, k_cache, v_cache, scale: float, batch: StepBatch, c
     if split:
         need = lib.msa_seq_kv_decode_workspace_bytes(C.byref(c), T)
         ws = ops.scratch(need, q.device)
-        _check(lib.msa_seq_kv_decode(C.byref(c), batch.ref, ptr(ws), need, _stream()), "msa_seq_kv_decode")
+        if rope is not None:
+            _check(lib.msa_seq_kv_decode_rope(C.byref(c), C.byref(rope), batch.ref, ptr(ws), need, _stream()), "msa_seq_kv_decode_rope")
+        else:
+            _check(lib.msa_seq_kv_decode(C.byref(c), batch.ref, ptr(ws), need, _stream()), "msa_seq_kv_decode")
     else:
+        if rope is not None:
+            _check(lib.msa_seq_qk_rope_append(C.byref(rope), dtype_code(q.dtype), batch.ref, _stream()), "msa_seq_qk_rope_append")
         _check(lib.msa_seq_kv_attn(C.byref(c), dtype_code(q.dtype), batch.ref, _stream()), "msa_seq_kv_attn")
     return out
+
+
+def rope_kv_attn(q, q_norm, freqs, eps: float, k_cache, v_cache, scale: float, batch: StepBatch, chunk: int = 0, gate=None, k=None, v=None, k_norm=None):
+    """:func:`kv_attn` of :func:`qk_rope_append`'s queries, which single rows' attention prepares itself."""
+    c, out, _ = _rope_args(q, q_norm, freqs, eps, k_cache, v_cache, batch, k, v, k_norm)
+    return kv_attn(out, k_cache, v_cache, scale, batch, chunk, gate, rope=c)
 
 
 class PostRows:
