@@ -238,7 +238,9 @@ struct SplitArgs {
 // 32 behind 128 to 256, 33 MB, 9.7 / 9.0; but 16 of these 7.5 / 7.9, 4 behind 500 to 1000 11.0 / 11.6, one behind 256 6.5 / 6.9).
 // kRope (D = DP, E = EP, D / 2 pairs, a row a sequence): the queries come as they are projected, and so do the row's own key and value.  A
 // lane's dimensions of a head hold both members of its pairs, so a wavefront norms and turns its queries itself while its first keys are
-// on their way; the one that has the range's last key takes that from the row instead of the cache, and appends it.
+// on their way; the one that has the range's last key takes that from the row instead of the cache, and appends it.  (Whole steps with the
+// preparation in a launch of its own and so, us: eight sequences of the 1b size 193.1 and 191.0, one 173.3 and 172.7, one of the 4b size behind
+// 8000 tokens 368.6 and 366.6: most of the launch's 3.3 us is the same chain of loads, in front of the first scores.)
 template <int DP, int EP, bool kOnce, bool kRope>
 __global__ __launch_bounds__(256) void kv_split_kernel(SplitArgs p, msa_seq_batch b) {
   constexpr int kVS = EP + 8, kUnits = EP / 8, kVP = kStepKeys * kUnits / 64, kK = DP / 32, kC = EP / 16;
