@@ -128,8 +128,11 @@ class StepDecoder:
                 raise ValueError(f"sequence {key!r}: token outside the vocabulary")
         cache.reserve(max(cache.length.get(k, 0) + len(t) for k, t, _ in entries))
         new = [key for key in dict.fromkeys(k for k, _, _ in entries) if key not in cache.slot_of]
-        if new:
+        if type(cache) is SequenceStateCache and "open" not in vars(cache):
             cache.open_all(new)
+        else:                                            # (a cache with an ``open`` of its own)
+            for key in new:
+                cache.open(key)
         counts, rows, at = [len(t) for _, t, _ in entries], [], 0
         for (_, ts, want) in entries:
             rows += [at + w for w in want]
