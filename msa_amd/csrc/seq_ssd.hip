@@ -266,8 +266,7 @@ __global__ __launch_bounds__(4 * Q) void ssd_output_kernel(ChunkArgs a, msa_seq_
   float* dts = reinterpret_cast<float*>(xs + Q * kXS);
   float* acs = dts + kMaxHeads * Q;
   float* wbs = acs + kMaxHeads * Q;                 // [heads][kBefore] weights of earlier blocks' tokens at a block's start
-  float* row_ssq = wbs + kMaxHeads * kBefore;       // [2][Q] the columns' halves' sums of squares
-  float* norm_w = row_ssq + 2 * Q;                  // [heads][kPB]
+  float* norm_w = wbs + kMaxHeads * kBefore;        // [heads][kPB]
   bf16_t* keep = reinterpret_cast<bf16_t*>(norm_w + kMaxNormHeads * kPB);        // [Q][kKeepStride] outputs
   Unit u;
   if (!unit_of<Q>(a, b, u)) return;
@@ -341,7 +340,6 @@ __global__ __launch_bounds__(4 * Q) void ssd_output_kernel(ChunkArgs a, msa_seq_
     z_at[q] = p < a.P ? zin : kOutside;
     v_at[q] = p < a.P ? vin : kOutside;
   }
-  float ssq = 0.f;                                  // of token t's outputs, this lane's
   for (int hh = 0; hh < u.heads; ++hh) {
     const int head = u.head0 + hh;
     __syncthreads();                                // the last reads of B or of the head before, and the weights
@@ -427,29 +425,35 @@ __global__ __launch_bounds__(4 * Q) void ssd_output_kernel(ChunkArgs a, msa_seq_
 #pragma unroll
       for (int x = 0; x < 4; ++x) y[x] = (acc[4 * q + x] + Dh * xv[x]) * silu_f(zv[x]);
       const u32x2_t o = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
-      if constexpr (kNorm) {
-        ssq += (bf16lo(o.x) * bf16lo(o.x) + bf16hi(o.x) * bf16hi(o.x)) + (bf16lo(o.y) * bf16lo(o.y) + bf16hi(o.y) * bf16hi(o.y));
-        *reinterpret_cast<u32x2_t*>(keep + t * kKeepStride + hh * kPB + pb + 8 * q + 4 * half) = o;
-      } else {
-        __builtin_amdgcn_raw_buffer_store_b64(o, rs_v, v_at[q], head * a.P * 2, 0);
-      }
+      if constexpr (kNorm) *reinterpret_cast<u32x2_t*>(keep + t * kKeepStride + hh * kPB + pb + 8 * q + 4 * half) = o;
+      else __builtin_amdgcn_raw_buffer_store_b64(o, rs_v, v_at[q], head * a.P * 2, 0);
     }
   }
   if constexpr (kNorm) {
-    ssq += __shfl_xor(ssq, 32);
-    if (half == 0) row_ssq[(pb >> 5) * Q + t] = ssq;
+    // A lane has eight columns, as in group_rmsnorm_kernel: its squares, then the lanes, are added in that kernel's order, so that a norm has the
+    // same bits folded and behind its own launch (a sum in another order moves a few results to the neighbouring bf16 value, and a decoder's
+    // logits with them).  Up to 256 columns are a half of a wavefront, whose other half has another row.
     __syncthreads();
-    const int units = u.heads * (kPB / 8);           // of eight columns, whole rows behind one another
-    for (int i = threadIdx.x; i < Q * units; i += 4 * Q) {
-      const int row = i / units, at = (i - row * units) * 8, hh = at / kPB, p = at % kPB;
-      const float inv = 1.0f / sqrtf((row_ssq[row] + row_ssq[Q + row]) / (float)(u.heads * a.P) + a.norm_eps);
-      float y[8], w[8];
+    const int per_head = a.P / 8, units = u.heads * per_head, seg = units <= 32 ? 32 : 64, j = lane & (seg - 1), hh = j / per_head, p = (j - hh * per_head) * 8;
+    const bool in = j < units;
+    const int at = in ? hh * kPB + p : 0;
+    float w[8];
+    load_vec<float, 8>(norm_w + at, w);
+#pragma unroll 4
+    for (int row = (wave * 64 + lane) / seg; row < Q; row += 4 * Q / seg) {
+      float y[8], ssq = 0.f;
       load_vec<bf16_t, 8>(keep + row * kKeepStride + at, y);
-      load_vec<float, 8>(norm_w + at, w);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ssq += y[e] * y[e];
+      ssq = in ? ssq : 0.f;
+      if (seg == 64) ssq += __shfl_xor(ssq, 32);
+#pragma unroll
+      for (int o = 16; o > 0; o >>= 1) ssq += __shfl_xor(ssq, o);
+      const float inv = 1.0f / sqrtf(ssq / (float)(u.heads * a.P) + a.norm_eps);
       uint32_t o[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = pack_bf16x2(y[2 * e] * (inv * w[2 * e]), y[2 * e + 1] * (inv * w[2 * e + 1]));
-      __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{o[0], o[1], o[2], o[3]}, rs_v, p < a.P ? (row * inner + hh * a.P + p) * 2 : kOutside, u.head0 * a.P * 2, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{o[0], o[1], o[2], o[3]}, rs_v, in ? (row * inner + hh * a.P + p) * 2 : kOutside, u.head0 * a.P * 2, 0);
     }
   }
 }
@@ -462,7 +466,7 @@ int launch_chunked(ChunkArgs a, const msa_seq_batch& b, hipStream_t st) {
   constexpr int tile = Q * (NP + 8), x = Q * kXS, state = 2 * NP * kXS;
   constexpr int lds2 = (tile > 2 * x ? tile : 2 * x) * 2 + kMaxHeads * Q * 4;
   constexpr int lds3 = ((tile > state ? tile : state) + x) * 2 + kMaxHeads * (2 * Q + (Q / 32) * (Q / 32 - 1) * 16) * 4;
-  constexpr int lds_norm = lds3 + (2 * Q + kMaxNormHeads * kPB) * 4 + Q * kKeepStride * 2;
+  constexpr int lds_norm = lds3 + kMaxNormHeads * kPB * 4 + Q * kKeepStride * 2;
   static_assert(lds2 <= 160 * 1024 && lds3 <= 160 * 1024 && (Q == 64 || lds_norm <= 160 * 1024), "tiles of a chunk must fit LDS");
   // as many heads per workgroup as leave a launch two workgroups per compute unit
   const int per_group = a.H / a.G, blocks = (a.P + kPB - 1) / kPB;
