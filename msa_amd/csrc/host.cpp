@@ -50,6 +50,13 @@ bool is_none(PyObject* o) { return o == nullptr || o == Py_None; }
 const at::Tensor* tensor(PyObject* o) { return !is_none(o) && THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
 void* at_(const at::Tensor* t) { return t ? t->data_ptr() : nullptr; }
 void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
+// The device that `stream` is of, or -1 without one.
+int device() {
+  int d = -1;
+  if (hipGetDevice(&d) == hipSuccess) return d;
+  (void)hipGetLastError();
+  return -1;
+}
 int dtype_of(const at::Tensor& t) { return t.scalar_type() == at::kBFloat16 ? MSA_BF16 : t.scalar_type() == at::kFloat ? MSA_F32 : -1; }
 bool dense(const at::Tensor* t) { return t && t->is_cuda() && t->is_contiguous(); }
 bool plain(const at::Tensor* t) { return !(t->requires_grad() && at::GradMode::is_enabled()); }
@@ -355,7 +362,8 @@ PyObject* pieces(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// clear(tensors, slot): zeroes the tensors' rows of that slot, or of a list of slots, in one launch or a few
+// clear(tensors, slot): zeroes the tensors' rows of that slot, or of a list of slots, in one launch or a few.  Tensors of another device than
+// the current one go to the library's call, which switches to theirs: a launch from here would be of the current device and its stream.
 PyObject* clear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 2 || !PyList_Check(args[0])) return PyErr_Format(PyExc_TypeError, "clear takes a list and a slot");
@@ -366,7 +374,7 @@ PyObject* clear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   std::vector<at::Tensor> rows;
   std::vector<void*> base;
   std::vector<int64_t> bytes;
-  const at::Tensor* like = nullptr;
+  const int here = device();
   bool dense = clear_ != nullptr;
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[0]); ++i) {
     const at::Tensor* t = tensor(PyList_GET_ITEM(args[0], i));
@@ -375,13 +383,12 @@ PyObject* clear(PyObject*, PyObject* const* args, Py_ssize_t n) {
       rows.push_back(t->select(0, slot));
       dense = dense && slot >= 0;
     }
-    dense = dense && t->is_cuda() && t->is_contiguous() && plain(t) && (!like || t->device() == like->device());
+    dense = dense && t->is_cuda() && t->device().index() == here && t->is_contiguous() && plain(t);
     if (!dense || t->numel() == 0) continue;
-    like = t;
     base.push_back(t->data_ptr());
     bytes.push_back((int64_t)t->nbytes() / t->size(0));
   }
-  if (dense && like) {
+  if (dense && !base.empty()) {
     const auto st = stream();
     const int rc = run([&] { return clear_(base.data(), bytes.data(), (int32_t)base.size(), slots.data(), (int32_t)slots.size(), st); });
     if (rc == MSA_OK) Py_RETURN_NONE;

@@ -2,6 +2,8 @@
 what that path refuses is refused with its errors."""
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from msa_amd import _lib, cache, ops, seq_ops
 
@@ -47,6 +49,24 @@ def test_an_opened_sequence_s_states_are_cleared(device):
     for t in c.tensors[0].values():
         t.fill_(1.0)
     assert c.open("a") == 0 and c.tensors[0]["s"].sum(1).tolist() == [0, 3] and c.tensors[0]["rows"].sum() == 20
+
+
+def test_states_of_another_device_are_cleared_there():
+    """A launch goes to the current device: tensors of another one are cleared by the call that switches to theirs.  (Fake tensors name a second
+    device without one; where no device is current, none is theirs.)"""
+    cleared = []
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, f, types, args=(), kwargs=None):
+            if f is torch.ops.aten._foreach_zero_.default:
+                cleared.extend((str(t.device), tuple(t.shape)) for t in args[0])
+            return f(*args, **(kwargs or {}))
+
+    with FakeTensorMode():
+        c = cache.SequenceStateCache([{"s": cache.StateSpec((3,), torch.float32), "c": cache.StateSpec((2, 2), torch.bfloat16)}], "cuda:1", 3, 5)
+        with Seen():
+            assert c.open_all(["a", "b"]) == [0, 1]
+    assert cleared == [("cuda:1", (3,))] * 2 + [("cuda:1", (2, 2))] * 2
 
 
 def same(a, b):
