@@ -51,6 +51,7 @@ def test_an_opened_sequence_s_states_are_cleared(device):
     assert c.open("a") == 0 and c.tensors[0]["s"].sum(1).tolist() == [0, 3] and c.tensors[0]["rows"].sum() == 20
 
 
+@pytest.mark.skipif(torch.cuda.device_count() == 1, reason="where there is a device, a fake tensor cannot name one that is not")
 def test_states_of_another_device_are_cleared_there():
     """A launch goes to the current device: tensors of another one are cleared by the call that switches to theirs.  (Fake tensors name a second
     device without one; where no device is current, none is theirs.)"""
