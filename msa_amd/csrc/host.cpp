@@ -66,14 +66,18 @@ bool rows(const at::Tensor* t) { return t && t->is_cuda() && t->dim() == 2 && (t
 int64_t row_stride(const at::Tensor& t) { return t.size(0) > 1 ? t.stride(0) : std::max(t.stride(0), t.size(1)); }
 bool aligned(const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
 
+// The launch with the interpreter's lock given back, which is taken again however it ends.  It gets addresses, not tensors: data_ptr() of a
+// tensor without storage (fake ones, wrappers of vmap) throws, and that has to be while the lock is held.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
 template <class Launch>
 int run(Launch launch) {
-  int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = launch();
-  Py_END_ALLOW_THREADS
-  return rc;
+  const Unlocked unlocked;
+  return launch();
 }
+float* f32(const at::Tensor* t) { return static_cast<float*>(at_(t)); }
 PyObject* none() { Py_RETURN_NONE; }
 PyObject* wrap(const at::Tensor& t) { return THPVariable_Wrap(t); }
 
@@ -110,12 +114,12 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const msa_tile_end end{(int32_t)mode, (int32_t)gelu_n, (float)PyFloat_AsDouble(args[4]), (float)PyFloat_AsDouble(args[5]), (float)PyFloat_AsDouble(args[6])};
   if (PyErr_Occurred()) return nullptr;
   if (!x || !w || !block_linear || !x->is_cuda() || x->dim() != 2 || w->dim() != 2) return none();
-  const int64_t T = x->size(0), K = x->size(1), N = w->size(0);
+  const int64_t T = x->size(0), K = x->size(1), N = w->size(0), ldx = T > 1 ? x->stride(0) : K;
+  void *xp = at_(x), *wp = at_(w);
   at::Tensor out = at::empty({T, mode == MSA_TILE_GLU ? N / 2 : N}, x->options().requires_grad(false));
-  const auto st = stream();
-  const int rc = run([&] {
-    return block_linear(x->data_ptr(), T > 1 ? x->stride(0) : K, T, (int32_t)K, w->data_ptr(), (int32_t)N, &end, out.data_ptr(), out.size(1), st);
-  });
+  void *to = out.data_ptr(), *st = stream();
+  const int64_t ldo = out.size(1);
+  const int rc = run([&] { return block_linear(xp, ldx, T, (int32_t)K, wp, (int32_t)N, &end, to, ldo, st); });
   return rc == MSA_OK ? wrap(out) : PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
 }
@@ -138,11 +142,9 @@ PyObject* flow(PyObject*, PyObject* const* args, Py_ssize_t n) {
   at::Tensor out = at::empty({T, mode == MSA_TILE_GLU ? N / 2 : N}, x->options().requires_grad(false)), ws;
   const size_t need = flow_bytes(T, (int32_t)K, (int32_t)N, (int32_t)mode);
   if (need) ws = at::empty({(int64_t)need}, x->options().requires_grad(false).dtype(at::kByte));
-  const auto st = stream();
-  const int rc = run([&] {
-    return flow_linear(x->data_ptr(), x->stride(0), T, (int32_t)K, w->data_ptr(), (int32_t)N, &end, out.data_ptr(), out.size(1),
-                       need ? ws.data_ptr() : nullptr, need, st);
-  });
+  void *xp = at_(x), *wp = at_(w), *to = out.data_ptr(), *scratch = need ? ws.data_ptr() : nullptr, *st = stream();
+  const int64_t ldx = x->stride(0), ldo = out.size(1);
+  const int rc = run([&] { return flow_linear(xp, ldx, T, (int32_t)K, wp, (int32_t)N, &end, to, ldo, scratch, need, st); });
   return rc == MSA_OK ? wrap(out) : PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
 }
@@ -177,18 +179,18 @@ PyObject* residual_norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
       return none();
   }
   if (!is_none(args[9]) && !(floats(shift, W) && prev && prev->scalar_type() == at::kFloat && prev->dim() == 2 && prev->size(1) == W && prev->size(0) > b.top)) return none();
-  const auto f32 = x->options().requires_grad(false), act = f32.dtype(dtype == MSA_BF16 ? at::kBFloat16 : at::kFloat);
+  const auto wide = x->options().requires_grad(false), act = wide.dtype(dtype == MSA_BF16 ? at::kBFloat16 : at::kFloat);
+  const float *xp = f32(x), *bias = f32(gate_bias), *shifts = f32(shift);
+  float* before = f32(prev);
+  void *yp = at_(y), *gp = at_(gate);
+  const int64_t ldy = y ? row_stride(*y) : 0, ldg = gate ? row_stride(*gate) : 0;
   at::Tensor out, h, hs;
-  if (y) out = at::empty({T, W}, f32);
+  if (y) out = at::empty({T, W}, wide);
   if (nw && want_h) h = at::empty({T, W}, act);
   if (shift) hs = at::empty({T, W}, act);
-  const auto st = stream();
-  const int rc = run([&] {
-    return residual_norm_(static_cast<const float*>(x->data_ptr()), at_(y), y ? row_stride(*y) : 0, at_(gate), gate ? row_stride(*gate) : 0,
-                          static_cast<const float*>(at_(gate_bias)), y ? static_cast<float*>(out.data_ptr()) : nullptr, (int32_t)dtype, (int32_t)W, &norm,
-                          h.defined() ? h.data_ptr() : nullptr, static_cast<const float*>(at_(shift)), static_cast<float*>(at_(prev)),
-                          hs.defined() ? hs.data_ptr() : nullptr, b.c, st);
-  });
+  float* sum = y ? f32(&out) : nullptr;
+  void *hp = h.defined() ? h.data_ptr() : nullptr, *hsp = hs.defined() ? hs.data_ptr() : nullptr, *st = stream();
+  const int rc = run([&] { return residual_norm_(xp, yp, ldy, gp, ldg, bias, sum, (int32_t)dtype, (int32_t)W, &norm, hp, shifts, before, hsp, b.c, st); });
   if (rc != MSA_OK) return PyLong_FromLong(rc);
   PyObject* first = y ? wrap(out) : (Py_INCREF(args[2]), args[2]);
   return Py_BuildValue("(NNN)", first, h.defined() ? wrap(h) : none(), hs.defined() ? wrap(hs) : none());
@@ -207,14 +209,14 @@ PyObject* rms_residual(PyObject*, PyObject* const* args, Py_ssize_t n) {
       !out || !dense(out) || out->sizes() != x->sizes() || out->scalar_type() != at::kFloat || (!is_none(args[4]) && !floats(next_w, x->size(1))))
     return none();
   const int64_t T = x->size(0), W = x->size(1);
+  const float *xp = f32(x), *wp = f32(w), *next = f32(next_w);
+  float* to = f32(out);
+  void* yp = at_(y);
+  const int64_t ldy = row_stride(*y);
   at::Tensor h;
   if (want_h || next_w) h = at::empty({T, W}, x->options().requires_grad(false).dtype(dtype == MSA_BF16 ? at::kBFloat16 : at::kFloat));
-  const auto st = stream();
-  const int rc = run([&] {
-    return rms_residual_(static_cast<const float*>(x->data_ptr()), y->data_ptr(), row_stride(*y), static_cast<const float*>(w->data_ptr()), (float)eps,
-                         static_cast<float*>(out->data_ptr()), static_cast<const float*>(at_(next_w)), h.defined() ? h.data_ptr() : nullptr, (int32_t)dtype,
-                         (int32_t)T, (int32_t)W, st);
-  });
+  void *hp = h.defined() ? h.data_ptr() : nullptr, *st = stream();
+  const int rc = run([&] { return rms_residual_(xp, yp, ldy, wp, (float)eps, to, next, hp, (int32_t)dtype, (int32_t)T, (int32_t)W, st); });
   if (rc != MSA_OK) return PyLong_FromLong(rc);
   Py_INCREF(args[5]);
   return Py_BuildValue("(NN)", args[5], h.defined() ? wrap(h) : none());
@@ -233,12 +235,14 @@ PyObject* conv_silu(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!floats(taps, Cn * K) || (!is_none(args[4]) && !floats(bias, Cn)) || !dense(state) || state->scalar_type() != at::kFloat || state->dim() != 3 ||
       state->size(1) != K - 1 || state->size(2) != Cn || state->size(0) <= b.top || T != b.c->rows)
     return none();
+  const void* xp = at_(x);
+  const float *tp = f32(taps), *bp = f32(bias);
+  float* sp = f32(state);
+  const int64_t ldx = row_stride(*x);
+  const int dtype = dtype_of(*x);
   at::Tensor out = at::empty({T, Cn}, x->options().requires_grad(false));
-  const auto st = stream();
-  const int rc = run([&] {
-    return conv_silu_(x->data_ptr(), row_stride(*x), static_cast<const float*>(taps->data_ptr()), static_cast<const float*>(at_(bias)), dtype_of(*x), (int32_t)Cn,
-                      (int32_t)K, static_cast<float*>(state->data_ptr()), out.data_ptr(), Cn, b.c, st);
-  });
+  void *to = out.data_ptr(), *st = stream();
+  const int rc = run([&] { return conv_silu_(xp, ldx, tp, bp, dtype, (int32_t)Cn, (int32_t)K, sp, to, Cn, b.c, st); });
   return rc == MSA_OK ? wrap(out) : PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
 }
@@ -252,12 +256,13 @@ PyObject* group_rmsnorm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const double eps = PyFloat_AsDouble(args[3]);
   if (PyErr_Occurred()) return nullptr;
   if (!dense(v) || v->dim() != 2 || dtype_of(*v) < 0 || !floats(w, v->size(1))) return none();
-  at::Tensor out = at::empty({v->size(0), v->size(1)}, v->options().requires_grad(false));
-  const auto st = stream();
-  const int rc = run([&] {
-    return group_rmsnorm_(v->data_ptr(), dtype_of(*v), (int32_t)v->size(0), (int32_t)v->size(1), (int32_t)parts, static_cast<const float*>(w->data_ptr()), (float)eps,
-                          out.data_ptr(), st);
-  });
+  const int64_t T = v->size(0), W = v->size(1);
+  const void* vp = at_(v);
+  const float* wp = f32(w);
+  const int dtype = dtype_of(*v);
+  at::Tensor out = at::empty({T, W}, v->options().requires_grad(false));
+  void *to = out.data_ptr(), *st = stream();
+  const int rc = run([&] { return group_rmsnorm_(vp, dtype, (int32_t)T, (int32_t)W, (int32_t)parts, wp, (float)eps, to, st); });
   return rc == MSA_OK ? wrap(out) : PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
 }
@@ -290,18 +295,21 @@ PyObject* ssd(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!xbc || dtype_of(*xbc) < 0 || !floats(bias, H) || !floats(a_log, H) || !floats(d, H) || !states(state, H, N, P, b.top) ||
       !block(xbc, T, H * P + 2 * G * N, xbc->scalar_type()) || !block(z, T, H * P, xbc->scalar_type()) || !block(dt, T, H, xbc->scalar_type()))
     return none();
+  const void *xp = at_(xbc), *zp = at_(z), *dp = at_(dt);
+  const float *bp = f32(bias), *ap = f32(a_log), *skip = f32(d), *wp = f32(norm);
+  float* sp = f32(state);
+  const int64_t ldx = row_stride(*xbc), ldz = row_stride(*z), ldd = row_stride(*dt);
+  const int dtype = dtype_of(*xbc);
   at::Tensor v = at::empty({T, H * P}, xbc->options().requires_grad(false)), ws;
   const size_t need = chunked ? ssd_bytes(b.c->max_rows, b.c->n_seq, (int32_t)H, (int32_t)P, (int32_t)N) : 0;
   if (need) ws = at::empty({(int64_t)need}, v.options().dtype(at::kByte));
-  const auto st = stream();
-  auto f = [](const at::Tensor* t) { return static_cast<float*>(t->data_ptr()); };
+  void *to = v.data_ptr(), *scratch = need ? ws.data_ptr() : nullptr, *st = stream();
   const int rc = run([&] {
     auto call = [&](auto fn, auto... more) {
-      return fn(xbc->data_ptr(), row_stride(*xbc), z->data_ptr(), row_stride(*z), dt->data_ptr(), row_stride(*dt), f(bias), f(a_log), f(d), dtype_of(*xbc), (int32_t)H,
-                (int32_t)P, (int32_t)N, (int32_t)G, f(state), v.data_ptr(), b.c, more...);
+      return fn(xp, ldx, zp, ldz, dp, ldd, bp, ap, skip, dtype, (int32_t)H, (int32_t)P, (int32_t)N, (int32_t)G, sp, to, b.c, more...);
     };
-    if (norm) return call(ssd_normed, need ? ws.data_ptr() : nullptr, need, f(norm), (int32_t)parts, (float)eps, st);
-    return chunked ? call(ssd_chunked, need ? ws.data_ptr() : nullptr, need, st) : call(ssd_scan, st);
+    if (norm) return call(ssd_normed, scratch, need, wp, (int32_t)parts, (float)eps, st);
+    return chunked ? call(ssd_chunked, scratch, need, st) : call(ssd_scan, st);
   });
   return rc == MSA_OK ? wrap(v) : PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
@@ -324,18 +332,16 @@ PyObject* delta(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const auto type = qkv->scalar_type();
   if (!block(qkv, T, 2 * G * D + H * E, type) || !block(a, T, H * D, type) || !block(beta, T, H, type) || !block(gate, T, H * E, type)) return none();
   at::Tensor out = at::empty({T, H * E}, qkv->options().requires_grad(false)), ws;
-  auto f = [](const at::Tensor* t) { return static_cast<float*>(t->data_ptr()); };
   msa_delta_args c{};
   c.qkv = qkv->data_ptr(), c.a = a->data_ptr(), c.b = beta->data_ptr(), c.gate = gate->data_ptr();
   c.qkv_stride = row_stride(*qkv), c.a_stride = row_stride(*a), c.b_stride = row_stride(*beta), c.gate_stride = row_stride(*gate);
-  c.A_log = f(a_log), c.dt_bias = f(bias), c.norm = f(norm), c.state = f(state), c.out = out.data_ptr();
+  c.A_log = f32(a_log), c.dt_bias = f32(bias), c.norm = f32(norm), c.state = f32(state), c.out = out.data_ptr();
   c.H = (int32_t)H, c.G = (int32_t)G, c.D = (int32_t)D, c.E = (int32_t)E, c.eps = (float)eps;
   const size_t need = chunked ? delta_bytes(&c, b.c->max_rows, b.c->n_seq) : 0;
   if (need) ws = at::empty({(int64_t)need}, out.options().dtype(at::kByte));
-  const auto st = stream();
-  const int rc = run([&] {
-    return chunked ? delta_chunked(&c, b.c, need ? ws.data_ptr() : nullptr, need, st) : delta_scan(&c, dtype_of(*qkv), b.c, st);
-  });
+  void *scratch = need ? ws.data_ptr() : nullptr, *st = stream();
+  const int dtype = dtype_of(*qkv);
+  const int rc = run([&] { return chunked ? delta_chunked(&c, b.c, scratch, need, st) : delta_scan(&c, dtype, b.c, st); });
   return rc == MSA_OK ? wrap(out) : PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
 }
@@ -389,7 +395,7 @@ PyObject* clear(PyObject*, PyObject* const* args, Py_ssize_t n) {
     bytes.push_back((int64_t)t->nbytes() / t->size(0));
   }
   if (dense && !base.empty()) {
-    const auto st = stream();
+    void* st = stream();
     const int rc = run([&] { return clear_(base.data(), bytes.data(), (int32_t)base.size(), slots.data(), (int32_t)slots.size(), st); });
     if (rc == MSA_OK) Py_RETURN_NONE;
   }

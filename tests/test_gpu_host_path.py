@@ -70,6 +70,28 @@ def test_states_of_another_device_are_cleared_there():
     assert cleared == [("cuda:1", (3,))] * 2 + [("cuda:1", (2, 2))] * 2
 
 
+@pytest.mark.parametrize("name", ["linear", "residual_norm", "rms_residual", "conv_silu", "group_rmsnorm", "ssd", "delta"])
+def test_operands_without_an_address_raise(name):
+    """A wrapper of vmap passes for a tensor of the device and has no storage: the error of asking it for an address comes back as one, in front of
+    any launch."""
+    host, bf, batch = ops.host(), torch.bfloat16, seq_ops.StepBatch([4], [0], [0], "cpu")
+    with FakeTensorMode():
+        r = lambda *s, t=torch.float32: torch.empty(s, dtype=t, device="cuda:0")
+        b = (batch.address, batch.top)
+        calls = {
+            "linear": ((4, 64), lambda x: host.linear(x, r(16, 64, t=bf), _lib.TILE_STORE, 0, 0.0, 0.0, 0.0)),
+            "residual_norm": ((4, 8), lambda y: host.residual_norm(*b, r(4, 8), y, y, r(8), r(8), r(8), 1.0, None, None, True, _lib.MSA_BF16)),
+            "rms_residual": ((4, 8), lambda y: host.rms_residual(r(4, 8), y, r(8), 1e-5, None, r(4, 8), True, _lib.MSA_BF16)),
+            "conv_silu": ((4, 8), lambda x: host.conv_silu(*b, x, r(8, 4), None, r(1, 3, 8))),
+            "group_rmsnorm": ((4, 8), lambda v: host.group_rmsnorm(v, r(8), 1, 1e-5)),
+            "ssd": ((4, 32), lambda x: host.ssd(*b, x, r(4, 16, t=bf), r(4, 2, t=bf), r(2), r(2), r(2), 2, 8, 8, 1, r(1, 2, 8, 8), False)),
+            "delta": ((4, 32), lambda x: host.delta(*b, x, r(4, 16, t=bf), r(4, 2, t=bf), r(4, 16, t=bf), r(2), r(16), r(8), 1e-5, 2, 1, 8, 8, r(1, 2, 8, 8), False)),
+        }
+        shape, call = calls[name]
+        with pytest.raises(RuntimeError, match="data pointer"):
+            torch.vmap(call)(r(3, *shape, t=bf))
+
+
 def same(a, b):
     return all((x is None) == (y is None) and (x is None or (x.dtype == y.dtype and x.shape == y.shape and torch.equal(x, y))) for x, y in zip(a, b))
 
