@@ -10,6 +10,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 #include <torch/csrc/Exceptions.h>
@@ -59,7 +60,15 @@ int device() {
 }
 int dtype_of(const at::Tensor& t) { return t.scalar_type() == at::kBFloat16 ? MSA_BF16 : t.scalar_type() == at::kFloat ? MSA_F32 : -1; }
 bool dense(const at::Tensor* t) { return t && t->is_cuda() && t->is_contiguous(); }
-bool plain(const at::Tensor* t) { return !(t->requires_grad() && at::GradMode::is_enabled()); }
+// Whether nothing but the values is asked of a tensor: no gradient in either direction, no batch of vmap, no trace, no dispatch of a class
+// or a mode of its own.  A launch would pass all of these by, without a word: what is not plain goes to torch's own call.
+bool plain(PyObject* o, const at::Tensor* t) {
+  using K = c10::DispatchKey;
+  static const c10::DispatchKeySet of_tensor({K::Python, K::Functionalize, K::FuncTorchBatched, K::FuncTorchGradWrapper});
+  static const c10::DispatchKeySet of_thread({K::Python, K::PythonDispatcher, K::Functionalize, K::Tracer, K::FuncTorchDynamicLayerFrontMode});
+  return THPVariable_CheckExact(o) && !(t->requires_grad() && at::GradMode::is_enabled()) && !t->key_set().has_any(of_tensor) &&
+         !c10::impl::tls_local_dispatch_key_set().included_.has_any(of_thread) && !t->_fw_grad(0).defined();
+}
 bool floats(const at::Tensor* t, int64_t n) { return dense(t) && t->scalar_type() == at::kFloat && t->numel() == n; }
 // rows with unit column stride, and the stride between them
 bool rows(const at::Tensor* t) { return t && t->is_cuda() && t->dim() == 2 && (t->size(1) <= 1 || t->stride(1) == 1); }
@@ -81,6 +90,17 @@ float* f32(const at::Tensor* t) { return static_cast<float*>(at_(t)); }
 PyObject* none() { Py_RETURN_NONE; }
 PyObject* wrap(const at::Tensor& t) { return THPVariable_Wrap(t); }
 
+// ordinary(operands ...): whether all tensors among them are plain
+PyObject* ordinary(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const at::Tensor* t = tensor(args[i]);
+    if (t && !plain(args[i], t)) Py_RETURN_FALSE;
+  }
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
 // block_ok(x, w, end): the caller's rule (block_linear_ok has it, with its reasons).
 PyObject* block_ok(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -88,7 +108,7 @@ PyObject* block_ok(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const at::Tensor *x = tensor(args[0]), *w = tensor(args[1]);
   if (!x || !w || !block_linear_us) return none();
   const bool end = PyObject_IsTrue(args[2]);
-  if (x->dim() != 2 || w->dim() != 2) Py_RETURN_FALSE;
+  if (x->dim() != 2 || w->dim() != 2 || !plain(args[0], x) || !plain(args[1], w)) Py_RETURN_FALSE;
   const int64_t T = x->size(0), K = x->size(1), N = w->size(0);
   if (!(T > 0 && x->is_cuda() && x->scalar_type() == at::kBFloat16 && w->scalar_type() == at::kBFloat16 && w->is_contiguous() && w->size(1) == K &&
         K % 64 == 0 && K >= 64 && K <= 32768 && N % 16 == 0 && N > 0 && N < 1 << 20 && T < 1 << 22 && (T <= lines.block_rows || K <= lines.block_depth)))
@@ -101,7 +121,7 @@ PyObject* block_ok(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (status != hipStreamCaptureStatusNone) Py_RETURN_FALSE;
   }
   return PyBool_FromLong((x->is_contiguous() || (x->stride(1) == 1 && x->stride(0) % 8 == 0 && K <= x->stride(0) && x->stride(0) < 1 << 21)) && aligned(*x) &&
-                         aligned(*w) && w->device() == x->device() && plain(x) && plain(w));
+                         aligned(*w) && w->device() == x->device());
   END_HANDLE_TH_ERRORS
 }
 
@@ -124,7 +144,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// flow(x, w, mode, gelu_n, limit, alpha, shift): msa_flow_linear where msa_flow_linear_us takes it, with no gradients asked for
+// flow(x, w, mode, gelu_n, limit, alpha, shift): msa_flow_linear where msa_flow_linear_us takes it, of plain operands
 PyObject* flow(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 7) return PyErr_Format(PyExc_TypeError, "flow takes 7 arguments");
@@ -134,9 +154,10 @@ PyObject* flow(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (PyErr_Occurred()) return nullptr;
   if (!x || !w || !flow_linear || !x->is_cuda() || x->dim() != 2 || w->dim() != 2) return none();
   const int64_t T = x->size(0), K = x->size(1), N = w->size(0);
-  if (!(x->scalar_type() == at::kBFloat16 && w->scalar_type() == at::kBFloat16 && w->is_contiguous() && w->size(1) == K && K <= 32768 && N % 16 == 0 &&
+  if (!(plain(args[0], x) && plain(args[1], w) &&
+        x->scalar_type() == at::kBFloat16 && w->scalar_type() == at::kBFloat16 && w->is_contiguous() && w->size(1) == K && K <= 32768 && N % 16 == 0 &&
         N < 1 << 20 && (x->is_contiguous() || (x->stride(1) == 1 && x->stride(0) % 8 == 0 && K <= x->stride(0) && x->stride(0) < 1 << 21)) && aligned(*x) &&
-        aligned(*w) && w->device() == x->device() && plain(x) && plain(w) && gelu_n % 8 == 0 && gelu_n <= N &&
+        aligned(*w) && w->device() == x->device() && gelu_n % 8 == 0 && gelu_n <= N &&
         flow_linear_us(T, (int32_t)K, (int32_t)N, (int32_t)mode) > 0.f))
     return none();
   at::Tensor out = at::empty({T, mode == MSA_TILE_GLU ? N / 2 : N}, x->options().requires_grad(false)), ws;
@@ -389,7 +410,7 @@ PyObject* clear(PyObject*, PyObject* const* args, Py_ssize_t n) {
       rows.push_back(t->select(0, slot));
       dense = dense && slot >= 0;
     }
-    dense = dense && t->is_cuda() && t->device().index() == here && t->is_contiguous() && plain(t);
+    dense = dense && t->is_cuda() && t->device().index() == here && t->is_contiguous() && plain(PyList_GET_ITEM(args[0], i), t);
     if (!dense || t->numel() == 0) continue;
     base.push_back(t->data_ptr());
     bytes.push_back((int64_t)t->nbytes() / t->size(0));
@@ -434,7 +455,7 @@ PyObject* bind(PyObject*, PyObject* args) {
 }
 
 #define MSA_FAST(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr}, MSA_FAST(block_ok), MSA_FAST(linear), MSA_FAST(flow), MSA_FAST(residual_norm), MSA_FAST(rms_residual), MSA_FAST(conv_silu),
+PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr}, MSA_FAST(ordinary), MSA_FAST(block_ok), MSA_FAST(linear), MSA_FAST(flow), MSA_FAST(residual_norm), MSA_FAST(rms_residual), MSA_FAST(conv_silu),
                          MSA_FAST(group_rmsnorm), MSA_FAST(ssd), MSA_FAST(delta), MSA_FAST(pieces), MSA_FAST(clear), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

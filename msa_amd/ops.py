@@ -548,7 +548,7 @@ TILE_ROWS = 256         # no matrix of the models has outputs enough for fewer r
 
 def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1, end: bool = True) -> bool:
     """Whether ``x [..., K] @ w.T`` (``matrices`` of w's shape in one; with an ``end`` besides the store) is ``tile_linear``'s: operands as it
-    takes them, no gradients asked for, and outputs enough to fill the compute units.  us in a loop of 60 ms, the vendor's (and its second
+    takes them, nothing but their values asked for (no gradients in either direction, no vmap or trace), and outputs enough to fill the compute units.  us in a loop of 60 ms, the vendor's (and its second
     launch) and here, rows x K x N: with an end 573 x 2560 x 19456 glu and 1600 x 1024 x 6144 glu level, 900 x 2560 x 19456 1.06 times, 6001 1.26
     times the speed; without one and N no multiple of 256 1600 x 1024 x 6176 1.10, 900 x 2560 x 14944 1.17 times.  Where N is one, a single
     round of tiles is behind the vendor's smaller ones (6001 x 9728 x 2560 199 and 217, 6001 x 4096 x 2560 86 and 93, 10000 x 3072 x 1024 53 and
@@ -562,7 +562,7 @@ def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1, end: boo
         if end or N % 256 or K < DEEP or x.numel() < DEEP_ROWS * K or not DEEP_TILES[0] <= -(-x.numel() // (256 * K)) * (N // 256) <= DEEP_TILES[1]:
             return False
     T = x.numel() // K
-    return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.shape[1] == K
+    return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and host().ordinary(x, w) and w.dim() == 2 and w.is_contiguous() and w.shape[1] == K
             and (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 21))
             and K % 64 == 0 and 1024 <= K <= 32768 and N % 8 == 0 and N < 1 << 20 and T < 1 << 22
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.device == x.device

@@ -97,6 +97,41 @@ def test_route(monkeypatch):
     assert ops.flow_linear(x.cpu(), w) is None
 
 
+@pytest.mark.parametrize("T,K,N", [(64, 1024, 1024), (450, 2560, 2560), (1536, 8192, 2560)])      # block_linear's, flow_linear's and tile_linear's
+def test_more_than_values(T, K, N):
+    """A tangent, a batch of vmap, and what a class or a mode sees of a call are torch's own product's."""
+    import torch.autograd.forward_ad as fwd
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from msa_amd import seq_ops
+    x, w, want = _operands(T, K, N, 6)
+    t = torch.randn(x.shape, device="cuda").bfloat16()
+    turned = t.float() @ w.float().t()
+    with fwd.dual_level():
+        for a in (fwd.make_dual(x, t), fwd.make_dual(x[:, :], t)):
+            y, tangent = fwd.unpack_dual(seq_ops.product(a, w))
+            assert _err(y, want) < TOL and tangent is not None and _err(tangent, turned) < TOL
+    y, tangent = torch.func.jvp(lambda x: seq_ops.product(x, w), (x,), (t,))
+    assert _err(y, want) < TOL and _err(tangent, turned) < TOL
+    both = torch.vmap(lambda x: seq_ops.product(x, w))(torch.stack([x, t]))
+    assert _err(both[0], want) < TOL and _err(both[1], turned) < TOL
+
+    class Own(torch.Tensor):
+        pass
+
+    class Seen(TorchDispatchMode):
+        calls = 0
+
+        def __torch_dispatch__(self, f, types, args=(), kwargs=None):
+            Seen.calls += 1
+            return f(*args, **(kwargs or {}))
+
+    assert type(seq_ops.product(x.as_subclass(Own), w)) is Own
+    with Seen():
+        seq_ops.product(x, w)
+    assert Seen.calls
+    assert _err(seq_ops.product(x, torch.nn.Parameter(w, requires_grad=False)), want) < TOL
+
+
 @pytest.mark.parametrize("T,K,N", [(450, 2560, 2560), (300, 9728, 2560)])
 def test_captured(T, K, N):
     from msa_amd import ops
