@@ -169,7 +169,8 @@ class MSAModel(nn.Module):
         """The segments of a packed block where every layer is to encode one (int64 operands as the kernel takes them), or None."""
         if cache is None or not h.is_cuda or h.shape[0] != 1 or h.shape[1] < 2 or not len(self.layers):
             return None
-        if any(cache.cache_kwargs.get(layer.self_attn.layer_idx, {}).get("stage") != "prefill_stage1" for layer in self.layers):
+        attention = [getattr(layer, "self_attn", None) for layer in self.layers]
+        if any(not isinstance(a, MemorySparseAttention) or cache.cache_kwargs.get(a.layer_idx, {}).get("stage") != "prefill_stage1" for a in attention):
             return None
         if any(not torch.is_tensor(t) or t.dtype != torch.int64 or t.shape != h.shape[:2] or t.device != h.device or not t.is_contiguous()
                for t in (doc_ids, attention_mask, position_ids)):

@@ -249,3 +249,18 @@ def test_bench_refuses_more_than_one_gpu():
                        capture_output=True, text=True, timeout=300)
     assert r.returncode != 0
     assert "one GPU" in (r.stdout + r.stderr)
+
+
+def test_layers_of_another_kind_are_asked_for_nothing():
+    """Whether a block's segments are found once for all layers is told without an attribute that a layer of another kind may not have."""
+    from types import SimpleNamespace
+
+    from msa_amd.model import MSAModel
+    cfg = mconfig.MSAConfig(num_hidden_layers=3, hidden_size=64, intermediate_size=128, vocab_size=50, num_attention_heads=2, num_key_value_heads=2)
+    model, h = MSAModel(cfg), SimpleNamespace(is_cuda=True, shape=(1, 9))
+    model.layers[1] = torch.nn.Identity()
+    for stages in (["prefill_stage1"] * 3, ["prefill_stage2"] * 3):
+        cache = mcache.create_cache()
+        for i, stage in enumerate(stages):
+            cache.record_kwargs(i, {"stage": stage})
+        assert model._block_segments(h, None, None, cache, None) is None
