@@ -8,6 +8,8 @@
 // caller's own path in Python then decides, with the checks and errors it has.  A code other than MSA_OK of the library is handed back.
 #include <Python.h>
 
+#include <algorithm>
+
 #include <ATen/ATen.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -398,19 +400,19 @@ PyObject* clear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const bool several = PyList_Check(args[1]);
   for (Py_ssize_t i = 0; i < (several ? PyList_GET_SIZE(args[1]) : 1); ++i) slots.push_back(PyLong_AsLongLong(several ? PyList_GET_ITEM(args[1], i) : args[1]));
   if (PyErr_Occurred()) return nullptr;
-  std::vector<at::Tensor> rows;
+  std::vector<const at::Tensor*> tensors;
   std::vector<void*> base;
   std::vector<int64_t> bytes;
   const int here = device();
+  const auto [least, most] = std::minmax_element(slots.begin(), slots.end());
   bool dense = clear_ != nullptr;
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[0]); ++i) {
-    const at::Tensor* t = tensor(PyList_GET_ITEM(args[0], i));
+    PyObject* o = PyList_GET_ITEM(args[0], i);
+    const at::Tensor* t = tensor(o);
     if (!t) return PyErr_Format(PyExc_TypeError, "clear: not a tensor");
-    for (const int64_t slot : slots) {
-      rows.push_back(t->select(0, slot));
-      dense = dense && slot >= 0;
-    }
-    dense = dense && t->is_cuda() && t->device().index() == here && t->is_contiguous() && plain(PyList_GET_ITEM(args[0], i), t);
+    tensors.push_back(t);
+    dense = dense && t->is_cuda() && t->device().index() == here && t->is_contiguous() && plain(o, t) && t->dim() > 0 &&
+            (slots.empty() || (*least >= 0 && *most < t->size(0)));
     if (!dense || t->numel() == 0) continue;
     base.push_back(t->data_ptr());
     bytes.push_back((int64_t)t->nbytes() / t->size(0));
@@ -420,6 +422,10 @@ PyObject* clear(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int rc = run([&] { return clear_(base.data(), bytes.data(), (int32_t)base.size(), slots.data(), (int32_t)slots.size(), st); });
     if (rc == MSA_OK) Py_RETURN_NONE;
   }
+  // (a view a tensor and slot costs as much as a launch where there are some of both: only here)
+  std::vector<at::Tensor> rows;
+  for (const at::Tensor* t : tensors)
+    for (const int64_t slot : slots) rows.push_back(t->select(0, slot));
   if (!rows.empty()) at::_foreach_zero_(rows);
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS

@@ -26,6 +26,16 @@ def test_rows_of_many_tensors(slots):
             ops.host().clear(ts, bad)
 
 
+@pytest.mark.gpu
+def test_one_launch_makes_no_views():
+    """Of six states and eight slots, forty-eight views would take the host as long as several launches."""
+    ts = [torch.ones((9, 4 + i), device="cuda") for i in range(6)]
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as p:
+        ops.host().clear(ts, list(range(8)))
+    assert all(t[:8].sum() == 0 and t[8].sum() == t.shape[1] for t in ts)
+    assert not [e.key for e in p.key_averages() if e.key.startswith("aten::")]
+
+
 @pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
 def test_opening_several(device):
     c = cache.SequenceStateCache([{"s": cache.StateSpec((3,), torch.float32), "rows": cache.StateSpec((2,), torch.bfloat16, per_token=True)}], device, 2, 5)
