@@ -159,9 +159,11 @@ class SequenceStateCache:
 
     def open_all(self, keys: Sequence[Hashable]) -> List[int]:
         """Gives every one of ``keys`` a cleared slot."""
-        for i, key in enumerate(keys):
-            if key in self.slot_of or key in keys[:i]:
+        seen = set()
+        for key in keys:
+            if key in self.slot_of or key in seen:
                 raise KeyError(f"sequence {key!r} is already open")
+            seen.add(key)
         while len(self._free) < len(keys):
             self._resize(2 * self.slots, self.capacity)
         slots, self._free = self._free[:len(keys)], self._free[len(keys):]

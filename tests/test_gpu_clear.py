@@ -50,3 +50,21 @@ def test_opening_several(device):
     assert "e" not in c.slot_of and c.open_all([]) == []
     c.close("b")
     assert c.open("e") == 1
+
+
+def test_opening_several_compares_no_two_of_them():
+    class Key:
+        compared = 0
+
+        def __init__(self, n):
+            self.n = n
+
+        def __hash__(self):
+            return self.n
+
+        def __eq__(self, other):
+            Key.compared += 1
+            return self.n == other.n
+
+    c = cache.SequenceStateCache([{"s": cache.StateSpec((3,), torch.float32)}], "cpu", 300, 5)
+    assert len(c.open_all([Key(n) for n in range(300)])) == 300 and Key.compared < 300
