@@ -555,7 +555,7 @@ def tile_linear_ok(x: torch.Tensor, w: torch.Tensor, matrices: int = 1, end: boo
     63), and several are level or ahead (7000 x 2560 x 2560 1.14 times, 6001 x 4096 x 12288 1.28, but 4096 x 2560 x 6144 0.87).  Padding does not
     count.  Deep products whose tiles are less than half a round, cut into pieces of K, are ahead as well (``DEEP``; weights not in the caches: 500 x 9728 x 2560 51.1 and 46.2,
     769 76 and 58, 1492 89 and 78, 2340 189 and 116; a third of a round deeper or half as deep they are level or behind: 3200 x 9728 x 2560 130 and 150, 1492 x
-    4096 x 2560 42 and 47).  Depths under 1024 were not measured and stay where they were."""
+    4096 x 2560 42 and 47).  A step's products ask ``flow_linear`` first up to ``FLOW_FIRST`` rows, modules (``linear``) come here from ``DEEP_ROWS`` on.  Depths under 1024 were not measured and stay where they were."""
     N = matrices * w.shape[0]
     K = x.shape[-1]
     if x.numel() * N < (TILE_MIN if end or N % 256 else TILE_PLAIN) * max(K, 1):   # (most calls end here: steps of few tokens wait for the host)

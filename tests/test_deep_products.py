@@ -36,5 +36,11 @@ def test_products(T, K, N):
     x = torch.randn((T, K + 32), generator=g, device="cuda").bfloat16()[:, 8:K + 8]
     w = (torch.randn((N, K), generator=g, device="cuda") * K ** -0.5).bfloat16()
     assert ops.tile_linear_ok(x, w, end=False)
-    want = x.float() @ w.float().t()
-    assert ((seq_ops.product(x, w).float() - want).norm() / want.norm()).item() < 3e-3
+    want, got = x.float() @ w.float().t(), ops.tile_linear(x, w)
+    assert ((got.float() - want).norm() / want.norm()).item() < 3e-3
+    # a step's products of fewer rows have another form in front of this one
+    assert torch.equal(seq_ops.product(x, w), got if T >= ops.FLOW_FIRST else ops.flow_linear(x, w))
+    lin = torch.nn.Linear(K, N, bias=False, device="cuda", dtype=torch.bfloat16)
+    lin.weight.data.copy_(w)
+    with torch.no_grad():
+        assert torch.equal(ops.linear(lin, x.contiguous()), got)
