@@ -184,7 +184,8 @@ struct Finish {
     }
   }
 
-  // the token's row of the rotary tables
+  // the token's row of the rotary tables, inside them whatever its position: a block's first layer runs before the host has heard that one
+  // is refused
   __device__ int table_row(int token) const {
     return token < a.T ? (int)min(max((int64_t)0, a.pos[token]), (int64_t)a.rope_rows - 1) : 0;
   }

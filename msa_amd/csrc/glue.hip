@@ -76,6 +76,7 @@ __global__ void qk_norm_rope_kernel(const T* __restrict__ q, const T* __restrict
 #pragma unroll
   for (int i = 0; i < 8; ++i) ssq += x[i] * x[i];
   const float inv = rsqrtf(row16_sum(ssq) * (1.0f / kHeadDim) + eps);
+  // (clamped: a block's first layer runs before the host has heard that a position is refused)
   const int64_t p = min((int64_t)max((int64_t)0, pos[n]), (int64_t)rope_rows - 1);
   const int f = 8 * (j & 7);                    // frequency index of this lane's first element
   // lanes j and j ^ 8 need the same eight cosines and sines: the lower lane fetches the cosines, the upper one the

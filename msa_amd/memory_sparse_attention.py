@@ -173,8 +173,8 @@ class MemorySparseAttention(nn.Module):
         return w[lo:lo + (Hq + 2 * Hkv) * D]
 
     def _rope_tables(self, device):
-        # one row per position the configuration allows; positions beyond it are refused where they are made
-        # (check_positions), not clamped in the kernels
+        # one row per position the configuration allows; positions beyond it are refused (check_positions).  The kernels clamp
+        # them to the tables, and stage 1 relies on that: the host hears of a block's positions behind the first layer's projections
         rows = int(self.config.max_position_embeddings)
         key = (device, rows, float(self.config.rope_theta))
         if key not in _ROPE_TABLES:
@@ -256,7 +256,7 @@ class MemorySparseAttention(nn.Module):
             if not block.done:
                 block.read()
                 cache.meta["q_lens_host"] = [block.mask_sum]
-                self.check_positions(block.last_position)
+                self.check_positions(block.last_position)       # (behind this layer's rotation, whose kernels clamp)
             n_template, doc_lens, bad = block.n_template, block.doc_lens, block.bad or block.mask_sum != T
         else:
             ids = doc_ids[0]
