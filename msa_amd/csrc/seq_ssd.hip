@@ -504,7 +504,8 @@ extern "C" size_t msa_seq_ssd_chunked_workspace_bytes(int32_t max_rows, int32_t 
   return (size_t)n_seq * ((max_rows + Q - 1) / Q) * H * ((size_t)N * P + 2 * Q) * sizeof(float);
 }
 
-// The norm is folded where a workgroup per group and chunk fills the chip: it has all heads of a group then.
+// Where the norm can be folded and a workgroup per group and chunk, which then has all heads of the group, fills the chip: groups of at most five
+// heads (the 1b size's four, not the 4b size's ten), whose outputs LDS holds.  The caller has a line of its own for steps of few rows.
 extern "C" int msa_seq_ssd_norm_folds(int32_t max_rows, int32_t n_seq, int32_t H, int32_t P, int32_t N, int32_t G, int32_t parts) {
   return max_rows > 0 && n_seq > 0 && H > 0 && G > 0 && H % G == 0 && parts == G && H / G <= kMaxNormHeads && P >= 8 && P <= kPB && P % 8 == 0 && N > 0 && N <= 128 &&
          N % 8 == 0 && (int64_t)((max_rows + chunk_tokens(N) - 1) / chunk_tokens(N)) * n_seq * G >= kNormRounds * device_compute_units();

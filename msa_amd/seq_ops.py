@@ -328,7 +328,10 @@ def ssd(xbc, z, dt_raw, dt_bias, A_log, D, H: int, P: int, N: int, G: int, state
     return v
 
 
-SSD_NORM_ROWS = 2048       # rows of a step below which no norm is folded
+# Rows of a step below which no norm is folded, whatever msa_seq_ssd_norm_folds says of its chunks: those are then of many short sequences, mostly
+# padding, and more than a round of them costs more than the launch (heads of the 1b size, recurrence and norm, us, folded and apart: 34
+# sequences of 60 90.4 and 85.7, 40 of 30 92.0 and 84.4, but 32 of 64 66.5 and 72.9, 64 of 64 115.8 and 117.7, one of 4096 62.7 and 75.6).
+SSD_NORM_ROWS = 2048
 
 
 def ssd_norm(xbc, z, dt_raw, dt_bias, A_log, D, H: int, P: int, N: int, G: int, state, batch: StepBatch, chunked: bool, w, parts: int, eps: float):
