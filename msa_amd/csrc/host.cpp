@@ -1,8 +1,9 @@
 // The host's side of the calls a prompt makes most: operands checked, results allocated and the kernel launched without Python in
 // between.  A prompt of few tokens waits for the host, not for the kernels (122 tokens of four layers of 1024: 350 us of kernels, 610 to 650
 // us in all through the interpreter, 385 to 430 so), and a call through the interpreter costs 9 to 14 us, of which the launch is 3 (us a
-// call, in Python and here: a product 9.7 and 5.2, a residual step with norm and shift 14.3 and 6.4, an RMS residual 8.9 and 4.4, a
-// convolution 8.7 and 4.4, an opened sequence 23 and 13).
+// call, in Python and here: a product 9.7 and 5.4, 0.2 of it for what is asked of its operands besides, a residual step with norm and shift
+// 14.3 and 6.4, an RMS residual 8.9 and 4.4, a convolution 8.7 and 4.4, an opened sequence 23 and 6; eight of them together 7, and 26 with
+// a view of every state's every row).
 //
 // Every function takes the operands as they come and answers None for whatever it does not take, without having launched anything: the
 // caller's own path in Python then decides, with the checks and errors it has.  A code other than MSA_OK of the library is handed back.
