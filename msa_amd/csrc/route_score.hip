@@ -633,7 +633,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void score_gemm_kernel(
   auto epilogue = [&](int tile_n0) {
     find_runs(tile_n0);
     if constexpr (kUnit == 4) {
-      // registers 4 g .. 4 g + 3 of a block are rows of two queries, one a half of the wavefront: nothing to join
+      // registers 4 g .. 4 g + 3 of a block are rows of two queries, one a half of the wavefront: nothing to join.  A maximum of what is no
+      // number counts for nothing, as in the forms that join some with -inf: its key would be in front of every score's.
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         const uint32_t bits = __builtin_amdgcn_readfirstlane(rbits[i]);
@@ -643,7 +644,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void score_gemm_kernel(
           const bool scored = bits >> (8 * g + 4 * half) & 1u;
           uint32_t* const row = out_key + (int64_t)(q_first + 8 * i + 2 * g + half) * n_docs;
 #pragma unroll
-          for (int j = 0; j < TN; ++j) merge_runs(runs[j], four(acc[i][j], g), row, scored);
+          for (int j = 0; j < TN; ++j) merge_runs(runs[j], fmaxf(-INFINITY, four(acc[i][j], g)), row, scored);
         }
       }
       return;

@@ -59,6 +59,25 @@ def test_packed_queries(form, B, S, Hkv):
         assert (alone.cpu()[0] - s[b]).abs().max() <= SUMS
 
 
+@pytest.mark.parametrize("form,B,S", [((4, False), 10, 3), ((4, False), 28, 2), ((8, False), 7, 5), ((8, True), 300, 2)])
+def test_no_numbers(form, B, S):
+    """What is no number counts for nothing in a maximum: a chunk of them, a document of such chunks and a query are what they are where a
+    query has row blocks of its own."""
+    print(f"[case] no numbers B={B} S={S}", flush=True)
+    chunks = [20, 1, 32, 8, 44, 12, 4, 160] * 8
+    ops, bank, kr, dco, q, _ = _case(B, S, 2, chunks, 5 + B)
+    assert _form(B, S, kr.shape[0]) == form
+    kr[2] = kr[20] = kr[700, 1, 7] = float("nan")               # one of a document's chunks, a document's only one, a value of one
+    bank.set_layer(0, kr)
+    q[1], q[2, 0], q[3, S - 1, 5] = float("nan"), float("nan"), float("nan")      # a query, a token, a head
+    s, d, _ = ops.route_topk(bank, 0, q, None, "cosine", 1.0, 64)
+    assert (s[1] == -torch.inf).all() and (s[0].isfinite().sum(), s[2].isfinite().sum()) == (len(chunks) - 1,) * 2
+    assert (s.gather(1, (d == 1).long().argmax(1, keepdim=True)) == -torch.inf).all()                        # (all 64 documents come back)
+    for b in range(min(B, 6)):
+        alone, _, _ = ops.route_topk(bank, 0, q[b:b + 1], None, "cosine", 1.0, 64)
+        assert torch.allclose(alone[0], s[b], rtol=0, atol=SUMS)
+
+
 def _large(B, S, seed):
     """A bank of 300 tiles of chunks, the last one ragged, and what a call over it gives: (layers' bank, kr, queries, mask, the best 64 scores, all)."""
     r = np.random.default_rng(seed)
