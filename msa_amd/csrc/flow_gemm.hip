@@ -222,9 +222,14 @@ int launch(FlowArgs a, hipStream_t st) {
 // The tiles, and what a K tile of them and storing them cost, us.  A launch costs 2.8 more; the operands come at 6.7 TB/s, at a share of
 // that where compute units are left without a tile; pieces cost another launch of 3.5 and their sums' way at 5.6 TB/s, to and fro.  Fitted to
 // the times of 14 matrices of the models by 10 numbers of tokens from 20 to 2200 (9 % off them, the best tile's time 2 % below the chosen one's).
-struct Tile { int n, t; float step, end; };
-constexpr Tile kTile[] = {{64, 32, .175f, .06f}, {64, 64, .208f, .83f}, {64, 96, .247f, .78f}, {64, 128, .331f, .72f}, {128, 96, .405f, 2.03f}, {128, 128, .485f, 2.25f},
-                          {128, 160, .534f, 3.23f}, {192, 128, .651f, 3.27f}, {192, 160, .71f, 3.91f}, {192, 192, .886f, 3.99f}, {256, 128, .848f, 3.77f}};
+// `behind`: with whole K behind the vendor's product.  That has tiles of its own for every size, whose times follow no measure of ours, so it is told
+// tile by tile (288 products of 22 matrices and 41 numbers of tokens of 17 to 2304, weights from memory, their time over the vendor's: in pieces of K
+// 0.43 to 0.98, 64 x 96 0.81 to 0.98, 128 x 160 0.81 to 0.99, 192 x 192 0.75 to 0.97, 128 x 128 0.84 to 1.03; half of them under 0.92, 0.96 and 0.97:
+// 192 x 160 0.86 to 1.11, 128 x 96 0.82 to 1.10, 192 x 128 0.92 to 1.04; but 64 x 128 0.97 to 1.07, 256 x 128 1.02 to 1.09).
+struct Tile { int n, t; float step, end; bool behind; };
+constexpr Tile kTile[] = {{64, 32, .175f, .06f, false},   {64, 64, .208f, .83f, false},   {64, 96, .247f, .78f, false},   {64, 128, .331f, .72f, true},
+                          {128, 96, .405f, 2.03f, false}, {128, 128, .485f, 2.25f, false}, {128, 160, .534f, 3.23f, false}, {192, 128, .651f, 3.27f, false},
+                          {192, 160, .71f, 3.91f, false}, {192, 192, .886f, 3.99f, false}, {256, 128, .848f, 3.77f, true}};
 
 struct Plan { int tile, pieces; float us; };
 // The cheapest tile and pieces of one round; none (us = 0) where there is none.  A gated unit or gelu costs kEnd for every output of a lane, of
@@ -246,13 +251,15 @@ Plan plan_of(int64_t T, int32_t K, int64_t N, bool end, bool whole) {
   return best;
 }
 
-// Where this form is taken: one round, faster than block_gemm.hip's by its own measure up to the length that form is asked for (behind it the
-// vendor's product is the other choice: 700 x 4096 x 2560 25.0 and 22.7, 700 x 5120 x 2560 36.0 and 35.3).  With fewer tokens the weights' way is all there is,
-// which more workgroups of smaller tiles do better, except for long rows, which are cut (us, the faster other form and here: 100 x 2560 x 12288
+// Where this form is taken: one round.  Up to the length that block_gemm.hip's is asked for it has to be faster than that by its own measure,
+// plain products by a little more (177 of them, their time over block_gemm.hip's: of the eleven whose measures are within 1 to 4 % 0.88 to 1.11).
+// Behind it the vendor's product is the other choice, of plain products in tiles that are not behind it (us, weights from memory, here and the vendor's:
+// 573 x 2560 x 12384 47.8 and 44.7, 640 x 4096 x 2560 29.1 and 27.1); an end saves the launch that it needs besides.  With fewer tokens the weights' way
+// is all there is, which more workgroups of smaller tiles do better, except for long rows, which are cut (us, the faster other form and here: 100 x 2560 x 12288
 // 22.9 and 24.4, 48 x 2560 x 8480 16.2 and 18.3, but 48 x 9728 x 2560 20.4 and 17.1, 20 x 5120 x 2560 15.1 and 12.1).  More tokens and shorter rows
 // were not measured.  (Behind 2304 tokens full rounds are level with the vendor's, 4096 x 3072 x 1024 29.6 and 29.2, 8192 47.0 and 50.6; tiles of
 // 256 x 160 to 256 x 256 are behind it, 850 x 2560 x 12368 53.9 and 65.3.)
-constexpr float kBlockUs = 23.f;
+constexpr float kBlockUs = 23.f, kSure = 0.96f, kSooner = 0.99f;
 constexpr int64_t kLeastTokens = 17, kTokens = 160, kMostTokens = 2304;
 constexpr int32_t kLong = 3072, kShort = 1024;
 
@@ -260,8 +267,11 @@ constexpr int32_t kLong = 3072, kShort = 1024;
 
 extern "C" float msa_flow_linear_us(int64_t T, int32_t K, int32_t N, int32_t mode) {
   if (T < kLeastTokens || T > kMostTokens || K < kShort || K > 32768 || K % kK != 0 || N < 16 || N >= (1 << 20) || (T < kTokens && K < kLong)) return 0.f;
-  const float us = plan_of(T, K, N, mode != MSA_TILE_STORE, false).us, block = msa_block_linear_us(T, K, N);
-  return us < 0.99f * block || block > kBlockUs ? us : 0.f;
+  const bool end = mode != MSA_TILE_STORE;
+  const Plan plan = plan_of(T, K, N, end, false);
+  const float block = msa_block_linear_us(T, K, N);
+  const bool taken = block <= kBlockUs ? plan.us < (end ? kSooner : kSure) * block : end || plan.pieces > 1 || !kTile[plan.tile].behind;
+  return taken ? plan.us : 0.f;
 }
 
 extern "C" size_t msa_flow_workspace_bytes(int64_t T, int32_t K, int32_t N, int32_t mode) {

@@ -172,6 +172,19 @@ def test_products_of_no_depth(rows):
     assert seq_ops.product(x, w).shape == (rows, 5)
 
 
+@pytest.mark.parametrize("T,K,N,taken", [(450, 2560, 2560, True), (769, 9728, 2560, True), (48, 9728, 2560, True), (640, 2560, 7680, True), (1200, 2560, 2560, True),
+                                         (1119, 1024, 4256, True), (33, 3072, 1024, True), (769, 2560, 2560, True), (573, 2560, 12384, False), (1000, 2560, 7680, False),
+                                         (1793, 4096, 4096, False), (640, 4096, 2560, False), (400, 4096, 4096, False), (257, 4096, 2560, False), (300, 5120, 2560, False)])
+def test_products_that_another_form_makes_sooner(T, K, N, taken):
+    """Plain products of one round of mid-sized tiles: those that are behind the vendor's or the smaller tiles go there.  With an end, which costs
+    the vendor's another launch, they stay where the smaller tiles are not asked for."""
+    from msa_amd import _lib
+    lib = _lib.load()
+    assert (lib.msa_flow_linear_us(T, K, N, _lib.TILE_STORE) > 0) == taken
+    if lib.msa_block_linear_us(T, K, N) > 23:
+        assert lib.msa_flow_linear_us(T, K, N, _lib.TILE_GELU) > 0
+
+
 def _err(got, want):
     return ((got.float() - want).norm() / want.norm()).item()
 
